@@ -2,7 +2,9 @@
 // for activations A (M rows, K contiguous) and nn.Linear weights W (N, K) — the dense contractions of the prompt pass
 // (c_attn / c_proj flash_stu/modules/attention.py:74,101; gate / up / down flash_stu/modules/swiglu.py:22-29;
 // x @ M_inputs flash_stu/modules/stu.py:87), with the element-wise work that follows them as epilogues:
-//   mode 0  C = T(acc)
+//   mode 0  C = T(acc), any feature count and row stride: the tied head's 50257 features go through here too (on the
+//           general kernel of fstu_gemm_any.hip they took longer than all layers: logits of 4 x 4096 positions at 2048-d,
+//           8 layers 103.7 -> 42.9 ms, of 3 x 777 positions at 768-d, 12 layers 6.06 -> 2.97 ms for the whole pass)
 //   mode 1  GLU: C[m, i] = T( T(gelu_tanh(T(acc_gate))) * T(acc_up) ) from two weight matrices (swiglu.py:23-26),
 //           so the gate and up activations never travel through HBM
 //   mode 2  C = T( R + T(acc) ): the residual add behind c_proj / down_proj (attention_layer.py:57,62, stu_layer.py:96)
@@ -85,6 +87,23 @@ __device__ __forceinline__ void lds_wait(u32x4_t (&f)[N]) {
     asm volatile("s_waitcnt lgkmcnt(%8)"
                  : "+v"(f[0]), "+v"(f[1]), "+v"(f[2]), "+v"(f[3]), "+v"(f[4]), "+v"(f[5]), "+v"(f[6]), "+v"(f[7])
                  : "n"(LEFT));
+}
+
+// 4 consecutive features of one row.  RAGGED: any row stride and feature count, so the address may be only 2-byte aligned
+// (a global store takes any alignment) and the last group of a row may hold fewer than 4 features.
+typedef unsigned u32x2_any_t __attribute__((ext_vector_type(2), aligned(2)));
+template <bool RAGGED>
+__device__ __forceinline__ void store_feat4(bf16_t* p, int left, unsigned lo, unsigned hi) {
+  if constexpr (!RAGGED) {
+    *(uint2*)p = make_uint2(lo, hi);
+  } else if (left >= 4) {
+    u32x2_any_t v = {lo, hi};
+    *(u32x2_any_t*)p = v;
+  } else {
+    p[0] = (bf16_t)lo;
+    if (left > 1) p[1] = (bf16_t)(lo >> 16);
+    if (left > 2) p[2] = (bf16_t)hi;
+  }
 }
 
 template <int WFN_, int WTN_, int FI_, int TJ_, int BK_, int NS_>
@@ -286,7 +305,7 @@ gemm_bf16_kernel(const bf16_t* __restrict__ A, long long lda, const bf16_t* __re
             v[2] = __uint_as_float(rv.y << 16) + rnd_bf16(v[2]);
             v[3] = __uint_as_float(rv.y & 0xffff0000u) + rnd_bf16(v[3]);
           }
-          *(uint2*)(C + (size_t)m * ldc + f) = make_uint2(pack2_bf16(v[0], v[1]), pack2_bf16(v[2], v[3]));
+          store_feat4<MODE == 0>(C + (size_t)m * ldc + f, N - f, pack2_bf16(v[0], v[1]), pack2_bf16(v[2], v[3]));
         }
     }
   }
@@ -590,12 +609,12 @@ extern "C" int fstu_gemm_bf16(const void* A, int64_t lda, const void* W, const v
   FSTU_REQUIRE(A && W && C, FSTU_ENULL, "fstu_gemm_bf16: null pointer");
   FSTU_REQUIRE(mode >= 0 && mode <= 2, FSTU_EARG, "fstu_gemm_bf16: mode %d", mode);
   FSTU_REQUIRE((mode != 1 || W2) && (mode != 2 || R), FSTU_ENULL, "fstu_gemm_bf16: mode %d needs its second operand", mode);
-  FSTU_REQUIRE(M >= 1 && N >= 4 && N % 4 == 0 && K >= 32 && K % 32 == 0, FSTU_ESHAPE,
-               "fstu_gemm_bf16: need K %% 32 == 0 and N %% 4 == 0 (M=%d N=%d K=%d)", M, N, K);
-  FSTU_REQUIRE(lda >= K && lda % 8 == 0 && ldc >= N && ldc % 4 == 0 && (mode != 2 || (ldr >= N && ldr % 4 == 0)), FSTU_ESHAPE,
+  FSTU_REQUIRE(M >= 1 && N >= 1 && (mode == 0 || N % 4 == 0) && K >= 32 && K % 32 == 0, FSTU_ESHAPE,
+               "fstu_gemm_bf16: need K %% 32 == 0 and, in modes 1 and 2, N %% 4 == 0 (M=%d N=%d K=%d)", M, N, K);
+  FSTU_REQUIRE(lda >= K && lda % 8 == 0 && ldc >= N && (mode == 0 || ldc % 4 == 0) && (mode != 2 || (ldr >= N && ldr % 4 == 0)), FSTU_ESHAPE,
                "fstu_gemm_bf16: row strides (lda=%lld ldc=%lld ldr=%lld)", (long long)lda, (long long)ldc, (long long)ldr);
-  FSTU_REQUIRE(fstu_aligned(A, 16) && fstu_aligned(W, 16) && fstu_aligned(W2, 16) && fstu_aligned(C, 8) && fstu_aligned(R, 8),
-               FSTU_EALIGN, "fstu_gemm_bf16: pointers must be 16-byte aligned (C, R: 8)");
+  FSTU_REQUIRE(fstu_aligned(A, 16) && fstu_aligned(W, 16) && fstu_aligned(W2, 16) && fstu_aligned(C, mode == 0 ? 2 : 8) && fstu_aligned(R, 8),
+               FSTU_EALIGN, "fstu_gemm_bf16: pointers must be 16-byte aligned (C, R: 8; C in mode 0: 2)");
   FSTU_REQUIRE(lda < GM_MAX_LD && K < GM_MAX_LD, FSTU_ESHAPE, "fstu_gemm_bf16: lda=%lld / K=%d beyond the 32-bit tile offsets",
                (long long)lda, K);
   int rc;

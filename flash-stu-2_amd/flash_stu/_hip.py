@@ -276,11 +276,12 @@ def bias_act(y: torch.Tensor, bias: Optional[torch.Tensor], silu: bool = False) 
     return y
 
 
-def gemm_supported(x2: torch.Tensor, weight: torch.Tensor) -> bool:
-    """Shapes the matrix-core prompt GEMM takes: bf16, K a multiple of 32, N a multiple of 4, rows 16-byte aligned."""
+def gemm_supported(x2: torch.Tensor, weight: torch.Tensor, plain: bool = False) -> bool:
+    """Shapes the matrix-core prompt GEMM takes: bf16, K a multiple of 32, N a multiple of 4 (plain: any N, for a product
+    without the gate or the residual as its epilogue), rows 16-byte aligned."""
     K = x2.shape[-1]
     return (x2.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x2.dim() == 2 and K % 32 == 0 and
-            weight.shape[0] % 4 == 0 and weight.is_contiguous() and x2.stride(1) == 1 and x2.stride(0) % 8 == 0 and
+            (plain or weight.shape[0] % 4 == 0) and weight.is_contiguous() and x2.stride(1) == 1 and x2.stride(0) % 8 == 0 and
             x2.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0)
 
 
@@ -292,7 +293,7 @@ def gemm(x2: torch.Tensor, weight: torch.Tensor, up_weight: Optional[torch.Tenso
     for t in (x2, residual, out):          # rows may be strided
         if t is not None and not t.is_cuda:
             raise FlashSTUHipError("tensor is not on the GPU: the HIP path has no CPU fallback")
-    if not gemm_supported(x2, weight):
+    if not gemm_supported(x2, weight, plain=up_weight is None and residual is None):
         raise FlashSTUHipError(f"gemm: unsupported operands {tuple(x2.shape)} {x2.dtype} x {tuple(weight.shape)} {weight.dtype}")
     if up_weight is not None and residual is not None:
         raise FlashSTUHipError("gemm: the gated pair and the residual epilogue do not combine")
@@ -394,7 +395,7 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] =
         y = linear_decode(x2.contiguous(), weight)
         if bias is not None:
             bias_act(y, bias)
-    elif gemm_supported(x2, weight):
+    elif gemm_supported(x2, weight, plain=True):
         y = gemm(x2, weight)
         if bias is not None:
             bias_act(y, bias)

@@ -391,7 +391,8 @@ int fstu_head_argmax_static(const void* x, int ldx, const void* W, void* logits,
  *   mode 2  C = T(R + T(acc))                            c_proj / down_proj and the residual add
  *                                                        (flash_stu/layers/attention_layer.py:57,62)
  * A (M,K) with row stride lda, W and W2 (N,K) contiguous, R / C (M,N) with row strides ldr / ldc (elements).
- * K % 64 == 0, N % 4 == 0, lda % 8 == 0; A, W, W2 16-byte aligned.  C may alias R. */
+ * K % 32 == 0, lda % 8 == 0; modes 1 and 2: N, ldc and ldr multiples of 4 (mode 0 takes any N and ldc: the vocabulary of
+ * the tied head, model.py:176, is odd); A, W, W2 16-byte aligned.  C may alias R. */
 int fstu_gemm_bf16(const void* A, int64_t lda, const void* W, const void* W2, const void* R, int64_t ldr, void* C,
                    int64_t ldc, int M, int N, int K, int mode, void* stream);
 /* The same contraction cut into ksplit slices of K, for a long K with few output tiles (down_proj of a decode step over

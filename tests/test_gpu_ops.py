@@ -247,6 +247,22 @@ def test_gemm_bf16_splitk_feeds_the_residual_norm(hip, M, N, K, ks):
     check(h, O.rms_norm(xd.cpu(), nw, O.RMS_EPS_DEFAULT), torch.bfloat16, frac=0.05)
 
 
+@pytest.mark.parametrize("M,N,K", [(17, 1, 32), (31, 259, 128), (33, 130, 64), (130, 1031, 1056), (700, 515, 1024), (4100, 10003, 1024)])
+def test_gemm_bf16_plain_any_feature_count(hip, M, N, K):
+    """Mode 0 with N % 4 != 0 and an odd row stride (the vocabulary of the tied head), every tile shape: one bf16 ulp
+    against F.linear in fp32 rounded once, and nothing written beside the (M, N) block."""
+    g = gen(65)
+    x = torch.randn(M, K, generator=g).bfloat16()
+    W = (torch.randn(N, K, generator=g) / math.sqrt(K)).bfloat16()
+    ref = F.linear(x.float(), W.float()).bfloat16()
+    big = torch.full((M + 2, N + 3), -7.0, dtype=torch.bfloat16, device="cuda")
+    hip.gemm(dev(x), dev(W), out=big[1:M + 1, 1:N + 1])
+    check(big[1:M + 1, 1:N + 1].cpu(), ref, torch.bfloat16)
+    big[1:M + 1, 1:N + 1] = -7.0
+    assert bool((big == -7.0).all())
+    check(hip.linear(dev(x), dev(W)), ref, torch.bfloat16)
+
+
 def test_gemm_bf16_strided_operands_and_errors(hip):
     g = gen(63)
     big = torch.randn(200, 3, 128, generator=g).bfloat16()
