@@ -20,12 +20,14 @@
 // wave's feature tiles are half gate, half up rows of the same features.  Workgroup ids are dealt round-robin to the
 // 8 XCDs; each XCD works through its own contiguous share of the tiles in panels of 8 feature tiles, so the workgroups
 // resident on an XCD share a few weight and activation tiles in its L2.
+#include <algorithm>
 #include "fstu_common.h"
 
 namespace {
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float floatx16_t __attribute__((ext_vector_type(16)));
+typedef float floatx4_t __attribute__((ext_vector_type(4)));
 typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
 
 #define GM_PANEL 8     // feature tiles per panel of the tile order
@@ -76,8 +78,10 @@ __device__ __forceinline__ void lds_read_rows(u32x4_t* f, unsigned addr) {   // 
 // that nothing that uses them is placed ahead of the wait.
 template <int LEFT, int N>
 __device__ __forceinline__ void lds_wait(u32x4_t (&f)[N]) {
-  static_assert(N == 3 || N == 4 || N == 6 || N == 8, "fragment group");
-  if constexpr (N == 3)
+  static_assert(N == 2 || N == 3 || N == 4 || N == 6 || N == 8, "fragment group");
+  if constexpr (N == 2)
+    asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(f[0]), "+v"(f[1]) : "n"(LEFT));
+  else if constexpr (N == 3)
     asm volatile("s_waitcnt lgkmcnt(%3)" : "+v"(f[0]), "+v"(f[1]), "+v"(f[2]) : "n"(LEFT));
   else if constexpr (N == 4)
     asm volatile("s_waitcnt lgkmcnt(%4)" : "+v"(f[0]), "+v"(f[1]), "+v"(f[2]), "+v"(f[3]) : "n"(LEFT));
@@ -104,6 +108,16 @@ __device__ __forceinline__ void store_feat4(bf16_t* p, int left, unsigned lo, un
     if (left > 1) p[1] = (bf16_t)(lo >> 16);
     if (left > 2) p[2] = (bf16_t)hi;
   }
+}
+
+int gemm_cus() {
+  static int cus = [] {
+    int dev = 0;
+    hipDeviceProp_t p;
+    if (hipGetDevice(&dev) != hipSuccess || hipGetDeviceProperties(&p, dev) != hipSuccess) return 256;
+    return p.multiProcessorCount;
+  }();
+  return cus;
 }
 
 template <int WFN_, int WTN_, int FI_, int TJ_, int BK_, int NS_>
@@ -325,6 +339,247 @@ int gemm_launch_tile(const void* A, long long lda, const void* W, const void* W2
   return 0;
 }
 
+// ---------------------------------------------------------------- 256 x 256 tiles in two alternating wave groups
+// Large contractions.  A workgroup of 8 waves owns 256 features x 256 rows (mode 1: 128 features, gate and up), K in tiles
+// of 64 through two LDS stages.  Waves 0-3 and 4-7 (one of each on every SIMD) run the same program half a phase apart:
+// while one group multiplies, the other reads its next fragments and requests the tiles to come, so a SIMD's matrix core
+// always has one of its two waves to work for, and neither barriers nor LDS reads show.
+// The halves of the weight tile (W0, W1: 128 features) and of the activation tile (X0, X1: 128 rows) are parts of 16 KB;
+// a wave owns 32 features of each W half and 64 rows of each X half, and a k tile is two phases of 32
+// v_mfma_f32_16x16x32_bf16 (512 cycles) each:
+//   phase  fragments read      multiplied      parts requested
+//   0      W0, W1, X0 of kt    (W0, W1) X0     X1 of kt + 1
+//   1      X1 of kt            (W0, W1) X1     W0, W1, X0 of kt + 2
+// A part is requested in the first phase after its last readers have left it (their reads are complete before the barrier
+// that ends a memory phase) and waited for three phases later: vmcnt(8) at the end of a memory phase leaves the two
+// youngest requests in flight, at 512 cycles a phase and group that is longer than a trip to the memory-side cache.
+// The grid is one workgroup per compute unit, each walks its share of the tiles: the first k tiles of the next output tile
+// are requested before this one is stored.  The epilogue passes 32 rows at a time through LDS beside the stages, so that
+// rows leave in 16-byte pieces, whole lines per instruction; straight from the accumulators a store instruction covers 16
+// rows of 32 bytes.
+// What bounds it: the power the matrix cores draw.  A loop of nothing but v_mfma on random bf16 operands runs at 1.77
+// PFLOP/s in the 32x32x16 form and 2.03 in the 16x16x32 form on this card (2.42 on zeros): hence the smaller instruction,
+// although it reads the same operands twice as often (1.30 -> 1.33-1.42 PFLOP/s).  Measured against the kernel above
+// (256 x 256 tile) and hipBLASLt, us: 16384 x 2048 x 24576 with the residual 1127 / 1395 / 1366 (1.46 PFLOP/s), 16384 x 6144
+// x 2048 291 / 384 / 294, 16384 x 50257 x 2048 2550 / 3339 / 2500; gate+up 16384 x 2 x 24576 x 2048 2487 / 3148, 4096 x
+// 2 x 9216 x 768 109 / 121.  What keeps K = 2048 below K = 24576: the epilogue (in mode 1 the GELU's 70 cycles per element).
+#define PP_STAGE 65536u
+#define PP_PART 16384u
+#define PP_LDS (2 * PP_STAGE + 32768u)   // + what the epilogue passes the rows through
+typedef unsigned u32x4_any_t __attribute__((ext_vector_type(4), aligned(2)));
+typedef unsigned u32x2_t __attribute__((ext_vector_type(2)));
+
+// 8 consecutive features of one row (the last group of a row may hold fewer), any 2-byte alignment; MODE 2: the residual
+// row's 8 features are added first
+template <int MODE>
+__device__ __forceinline__ void store_feat8(u32x4_t v, const bf16_t* rp, bf16_t* cp, int left) {
+  if (left >= 8) {
+    if (MODE == 2) {
+      const u32x4_any_t rv = *(const u32x4_any_t*)rp;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        v[e] = pack2_bf16(__uint_as_float(rv[e] << 16) + __uint_as_float(v[e] << 16),
+                          __uint_as_float(rv[e] & 0xffff0000u) + __uint_as_float(v[e] & 0xffff0000u));
+    }
+    *(u32x4_any_t*)cp = v;
+    return;
+  }
+  for (int e = 0; e < left; ++e) {
+    bf16_t h = (bf16_t)(v[e >> 1] >> (16 * (e & 1)));
+    if (MODE == 2) h = f32_to_bf16(bf16_to_f32(rp[e]) + bf16_to_f32(h));
+    cp[e] = h;
+  }
+}
+
+template <int MODE>
+__global__ void __launch_bounds__(512)
+gemm_pp_bf16_kernel(const bf16_t* __restrict__ A, long long lda, const bf16_t* __restrict__ W, const bf16_t* __restrict__ W2,
+                    const bf16_t* __restrict__ R, long long ldr, bf16_t* __restrict__ C, long long ldc, int M, int N, int K,
+                    int mt, int nt, int share) {
+  constexpr int NF = MODE == 1 ? 128 : 256;
+  extern __shared__ __align__(16) unsigned char gm_smem[];   // stage: W0 | W1 | X0 | X1
+  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int per_panel = mt * GM_PANEL, xcd = (int)(blockIdx.x & 7) * share, tiles = mt * nt;
+  int idx = (int)(blockIdx.x >> 3);                    // this workgroup's next tile in its XCD's share
+  if (idx >= share || xcd + idx >= tiles) return;
+  int m0, n0;
+  size_t wbytes, abytes;
+  const bf16_t *wb, *wb2, *ab;
+#define PP_OPEN_TILE                                                                     \
+  {                                                                                      \
+    const int o_ = xcd + idx;                                                            \
+    const int panel_ = o_ / per_panel, in_panel_ = o_ - panel_ * per_panel;              \
+    const int pw_ = min(GM_PANEL, nt - panel_ * GM_PANEL);                               \
+    m0 = in_panel_ / pw_ * 256;                                                          \
+    n0 = (panel_ * GM_PANEL + in_panel_ % pw_) * NF;                                     \
+    wbytes = (size_t)min(NF, N - n0) * K * 2;                                            \
+    abytes = ((size_t)(min(256, M - m0) - 1) * lda + K) * 2;                             \
+    wb = W + (size_t)n0 * K;                                                             \
+    wb2 = MODE == 1 ? W2 + (size_t)n0 * K : wb;                                          \
+    ab = A + (size_t)m0 * lda;                                                           \
+  }
+  const int wn = wv & 3, wm = wv >> 2;                 // 32-feature slice and 64-row slice of every half
+  // ---- fills: part = 128 rows x 128 bytes; a wave fills rows 16 wv .. 16 wv + 15 of it with two instructions
+  unsigned wvoff[2], avoff[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int row = wv * 16 + j * 8 + (lane >> 3), ch = (lane & 7) ^ ((row >> 1) & 7);
+    wvoff[j] = (unsigned)row * (unsigned)K * 2u + (unsigned)ch * 16u;
+    avoff[j] = (unsigned)row * (unsigned)lda * 2u + (unsigned)ch * 16u;
+  }
+  const unsigned w1off = MODE == 1 ? 0u : 128u * (unsigned)K * 2u, x1off = 128u * (unsigned)lda * 2u;
+  const int nkt = K >> 6;
+  unsigned char* fill0 = gm_smem + (unsigned)wv * 2048u;
+  // requests part P (0 W0, 1 X0, 2 W1, 3 X1) of k tile kt_; beyond the last tile the descriptor is empty: nothing is fetched
+#define PP_FETCH(P, kt_, stage_)                                                                                           \
+  {                                                                                                                        \
+    const bool in_ = (kt_) < nkt;                                                                                          \
+    const unsigned so_ = (unsigned)(kt_) * 128u;                                                                           \
+    unsigned char* l_ = fill0 + (stage_) * PP_STAGE + ((P) == 0 ? 0u : (P) == 2 ? PP_PART : (P) == 1 ? 2 * PP_PART : 3 * PP_PART); \
+    const rsrc_t rs_ = ((P) & 1) ? make_rsrc(ab, in_ ? abytes : 0) : make_rsrc((P) == 2 ? wb2 : wb, in_ ? wbytes : 0);     \
+    _Pragma("unroll") for (int j = 0; j < 2; ++j)                                                                          \
+      buf_load16_to_lds(rs_, (((P) & 1) ? avoff[j] : wvoff[j]) + ((P) == 2 ? w1off : (P) == 3 ? x1off : 0u), so_, l_ + j * 1024); \
+  }
+  const int l16 = lane & 15, lq = lane >> 4;
+  unsigned fw_off[2], fx_off[2];                       // fragment addresses of the two k steps inside a part
+#pragma unroll
+  for (int kk = 0; kk < 2; ++kk) {
+    const int rw = wn * 32 + l16, rx = wm * 64 + l16, c = kk * 4 + lq;
+    fw_off[kk] = (unsigned)rw * 128u + (unsigned)((c ^ ((rw >> 1) & 7)) << 4);
+    fx_off[kk] = 2 * PP_PART + (unsigned)rx * 128u + (unsigned)((c ^ ((rx >> 1) & 7)) << 4);
+  }
+  const unsigned smem0 = lds_addr(gm_smem);
+  u32x4_t wa[8], xf[8];                                // fragments: W (k step, half, feature tile), X (k step, row tile)
+  floatx4_t acc[2][2][2][4];                           // [W half][feature tile][X half][row tile]
+#define PP_READ_W(stage_)                                                                              \
+  _Pragma("unroll") for (int kk = 0; kk < 2; ++kk) {                                                   \
+    wa[4 * kk] = lds_read16<0>(smem0 + (stage_) * PP_STAGE + fw_off[kk]);                              \
+    wa[4 * kk + 1] = lds_read16<2048>(smem0 + (stage_) * PP_STAGE + fw_off[kk]);                       \
+    wa[4 * kk + 2] = lds_read16<16384>(smem0 + (stage_) * PP_STAGE + fw_off[kk]);                      \
+    wa[4 * kk + 3] = lds_read16<16384 + 2048>(smem0 + (stage_) * PP_STAGE + fw_off[kk]);               \
+  }
+#define PP_READ_X(stage_, H)                                                                           \
+  _Pragma("unroll") for (int kk = 0; kk < 2; ++kk)                                                     \
+    lds_read_rows<4, 2048>(xf + 4 * kk, smem0 + (stage_) * PP_STAGE + (H) * 16384u + fx_off[kk]);
+  // end of a memory phase: this wave's reads are complete, its share of the parts that the next phase reads has landed
+#define PP_MEM_END                                                                                     \
+  asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)"                                                         \
+               : "+v"(xf[0]), "+v"(xf[1]), "+v"(xf[2]), "+v"(xf[3]), "+v"(xf[4]), "+v"(xf[5]), "+v"(xf[6]), "+v"(xf[7]), \
+                 "+v"(wa[0]), "+v"(wa[1]), "+v"(wa[2]), "+v"(wa[3]), "+v"(wa[4]), "+v"(wa[5]), "+v"(wa[6]), "+v"(wa[7])::"memory"); \
+  __builtin_amdgcn_s_barrier();                                                                        \
+  __builtin_amdgcn_sched_barrier(0);
+#define PP_MUL(HX)                                                                                     \
+  __builtin_amdgcn_s_setprio(1);                                                                       \
+  _Pragma("unroll") for (int kk = 0; kk < 2; ++kk)                                                     \
+    _Pragma("unroll") for (int i = 0; i < 4; ++i)                                                      \
+      _Pragma("unroll") for (int j = 0; j < 4; ++j)                                                    \
+        acc[i >> 1][i & 1][HX][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, wa[4 * kk + i]), \
+                                                                            __builtin_bit_cast(bf16x8_t, xf[4 * kk + j]), \
+                                                                            acc[i >> 1][i & 1][HX][j], 0, 0, 0); \
+  __builtin_amdgcn_s_setprio(0);                                                                       \
+  __builtin_amdgcn_sched_barrier(0);                                                                   \
+  __builtin_amdgcn_s_barrier();                                                                        \
+  __builtin_amdgcn_sched_barrier(0);
+#define PP_TILE(S_)                                                                                    \
+  PP_READ_W(S_) PP_READ_X(S_, 0) PP_FETCH(3, kt + 1, 1 - (S_)) PP_MEM_END PP_MUL(0)                    \
+  PP_READ_X(S_, 1) PP_FETCH(0, kt + 2, S_) PP_FETCH(2, kt + 2, S_) PP_FETCH(1, kt + 2, S_) PP_MEM_END PP_MUL(1)
+#define PP_FIRST                                                         \
+  PP_FETCH(0, 0, 0) PP_FETCH(2, 0, 0) PP_FETCH(1, 0, 0) PP_FETCH(3, 0, 0) \
+  PP_FETCH(0, 1, 1) PP_FETCH(2, 1, 1) PP_FETCH(1, 1, 1)
+  // epilogue addresses: a group passes 32 rows at a time through 16 KB of its own, chunks XOR-ed with the row
+  constexpr int CH = NF / 8, RBY = NF * 2, NST = 32 * CH / 256;      // 16-byte chunks per row, row bytes, chunks per lane
+  const unsigned scratch = smem0 + 2 * PP_STAGE + (unsigned)wm * 16384u;
+  const int gl = tid & 255;
+  PP_OPEN_TILE
+  PP_FIRST
+  for (;;) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[i >> 2][(i >> 1) & 1][i & 1][j] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+    asm volatile("s_waitcnt vmcnt(8)" ::: "memory");   // W0, W1 and X0 of k tile 0
+    __builtin_amdgcn_s_barrier();
+    if (wm) __builtin_amdgcn_s_barrier();              // the second group runs half a phase later
+    __builtin_amdgcn_sched_barrier(0);
+    for (int kt = 0;; ++kt) {
+      PP_TILE(0)
+      if (++kt >= nkt) break;
+      PP_TILE(1)
+      if (kt + 1 >= nkt) break;
+    }
+    if (!wm) __builtin_amdgcn_s_barrier();
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the empty fills behind the last k tile
+    __builtin_amdgcn_s_barrier();
+    // every wave has left the stages: the next tile's first k tiles are on their way while this one is stored
+    const int em0 = m0, en0 = n0;
+    idx += (int)(gridDim.x >> 3);
+    const bool more = idx < share && xcd + idx < tiles;
+    if (more) {
+      PP_OPEN_TILE
+      PP_FIRST
+    }
+    // D of a 16x16 tile: lane l holds row l % 16 and features 4*(l/16) + e
+#pragma unroll
+    for (int hx = 0; hx < 2; ++hx)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+#pragma unroll
+        for (int hw = 0; hw < (MODE == 1 ? 1 : 2); ++hw)
+#pragma unroll
+          for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+              const int c = hw * 16 + wn * 4 + i * 2 + (lq >> 1), r = t * 16 + l16;
+              float v[4];
+#pragma unroll
+              for (int e = 0; e < 4; ++e)
+                v[e] = MODE == 1 ? rnd_bf16(gelu_tanh_fast(rnd_bf16(acc[0][i][hx][2 * j + t][e]))) * rnd_bf16(acc[1][i][hx][2 * j + t][e])
+                                 : acc[hw][i][hx][2 * j + t][e];
+              const u32x2_t p = {pack2_bf16(v[0], v[1]), pack2_bf16(v[2], v[3])};
+              asm volatile("ds_write_b64 %0, %1" ::"v"(scratch + (unsigned)(r * RBY + ((c ^ (r & (CH - 1))) << 4) + (lq & 1) * 8)), "v"(p) : "memory");
+            }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        u32x4_t o[NST];
+#pragma unroll
+        for (int i = 0; i < NST; ++i) {
+          const int r = (i * 256 + gl) / CH, c = gl % CH;
+          o[i] = lds_read16<0>(scratch + (unsigned)(r * RBY + ((c ^ (r & (CH - 1))) << 4)));
+        }
+        lds_wait<0>(o);
+        __builtin_amdgcn_s_barrier();
+#pragma unroll
+        for (int i = 0; i < NST; ++i) {
+          const int r = (i * 256 + gl) / CH, c = gl % CH;
+          const int m = em0 + hx * 128 + wm * 64 + j * 32 + r, f = en0 + c * 8;
+          if (m < M && f < N) store_feat8<MODE>(o[i], MODE == 2 ? R + (size_t)m * ldr + f : nullptr, C + (size_t)m * ldc + f, N - f);
+        }
+      }
+    if (!more) break;
+  }
+#undef PP_OPEN_TILE
+#undef PP_FIRST
+#undef PP_FETCH
+#undef PP_READ_W
+#undef PP_READ_X
+#undef PP_MEM_END
+#undef PP_MUL
+#undef PP_TILE
+}
+
+template <int MODE>
+int gemm_pp_launch(const void* A, long long lda, const void* W, const void* W2, const void* R, long long ldr, void* C,
+                   long long ldc, int M, int N, int K, hipStream_t s) {
+  constexpr int NF = MODE == 1 ? 128 : 256;
+  static hipError_t attr_err = hipFuncSetAttribute((const void*)gemm_pp_bf16_kernel<MODE>, hipFuncAttributeMaxDynamicSharedMemorySize, PP_LDS);
+  if (attr_err != hipSuccess) { fstu_set_error("fstu_gemm_bf16: hipFuncSetAttribute: %s", hipGetErrorString(attr_err)); return (int)attr_err; }
+  const int mt = (M + 255) / 256, nt = (N + NF - 1) / NF;
+  const int share = (int)(((long long)mt * nt + 7) / 8);
+  hipLaunchKernelGGL((gemm_pp_bf16_kernel<MODE>), dim3(8u * (unsigned)std::min(share, gemm_cus() / 8)), dim3(512), PP_LDS, s, (const bf16_t*)A, lda,
+                     (const bf16_t*)W, (const bf16_t*)W2, (const bf16_t*)R, ldr, (bf16_t*)C, ldc, M, N, K, mt, nt, share);
+  return 0;
+}
+
 // ---------------------------------------------------------------- transposed activations
 // C[b][m, n] = sum_k A[b][k, m] W[n, k]: the activations come as a slab with the REDUCTION index slowest (k rows of
 // lda elements, m contiguous) — the time-major U+- of the exact-mode STU operator (flash_stu/modules/stu.py:107-120:
@@ -335,7 +590,6 @@ int gemm_launch_tile(const void* A, long long lda, const void* W, const void* W2
 // (ds_read_b64_tr_b16: in a block of 16 lanes, lane i supplies the address of 4 consecutive m of row i/4 starting at
 // column 4*(i%4), and receives column i of the 4 rows).  The 64-byte column groups of a row are XOR-ed with the row's
 // low two bits, so the four rows of a read fall into different banks.  `nbatch` slabs run as one grid.
-typedef unsigned u32x2_t __attribute__((ext_vector_type(2)));
 template <int OFF>
 __device__ __forceinline__ u32x2_t lds_read_tr8(unsigned addr) {
   u32x2_t v;
@@ -538,18 +792,9 @@ int gemm_ta_launch_tile(const void* A, long long lda, long long sa, const void* 
   return 0;
 }
 
-int gemm_cus() {
-  static int cus = [] {
-    int dev = 0;
-    hipDeviceProp_t p;
-    if (hipGetDevice(&dev) != hipSuccess || hipGetDeviceProperties(&p, dev) != hipSuccess) return 256;
-    return p.multiProcessorCount;
-  }();
-  return cus;
-}
 
 //                     waves  tiles  BK  stages
-using TileBig = GemmTile<4, 2, 2, 4, 64, 2>;     // 256 x 256, 8 waves, 128 KB of LDS
+using TileBig = GemmTile<4, 2, 2, 4, 64, 2>;     // 256 x 256, 8 waves, 128 KB of LDS (transposed activations)
 using TileSmall = GemmTile<2, 2, 2, 2, 64, 2>;   // 128 x 128, 4 waves, 64 KB: two workgroups per compute unit
 using TileDeep = GemmTile<2, 2, 2, 2, 64, 4>;    // 128 x 128, 4 waves, 3 tiles in flight: one workgroup per compute unit
 using TileRows32 = GemmTile<2, 1, 2, 1, 64, 4>;  // 128 features x 32 rows, 2 waves, 80 KB: weight streaming, two workgroups per compute unit
@@ -561,14 +806,18 @@ int gemm_launch(const void* A, long long lda, const void* W, const void* W2, con
                 int M, int N, int K, hipStream_t s) {
   if (K % 64 != 0) return gemm_launch_tile<TileK32, MODE>(A, lda, W, W2, R, ldr, C, ldc, M, N, K, s);
   if (M <= 32) return gemm_launch_tile<TileRows32, MODE>(A, lda, W, W2, R, ldr, C, ldc, M, N, K, s);
-  // Measured choices (MI355X, bf16): the large tile halves the fill traffic per flop and pays once K amortises its
-  // start-up and the grid still covers the chip twice (M=32768, K >= 2048: 1.01-1.18 PFLOP/s against 0.89-0.99;
-  // M=4096, N=9216, K=768: 92 us against 80 us).  A grid that leaves one workgroup per compute unit anyway gains from
-  // the deeper pipeline when K is long (M=4096, N=768, K=9216: 83 us against 93 us).
   const int nf = MODE == 1 ? 2 : 1;
-  const long long big = (long long)((M + 255) / 256) * ((N * nf + 255) / 256);
-  const long long small = (long long)((M + 127) / 128) * ((N * nf + 127) / 128);
-  if (K >= 1024 && big >= 2 * gemm_cus()) return gemm_launch_tile<TileBig, MODE>(A, lda, W, W2, R, ldr, C, ldc, M, N, K, s);
+  const long long big = (long long)((M + 255) / 256) * (((long long)N * nf + 255) / 256);
+  const long long small = (long long)((M + 127) / 128) * (((long long)N * nf + 127) / 128);
+  // A round of 256 x 256 tiles (one per compute unit) in the alternating-group kernel takes as long as 2.25 rounds of 128 x
+  // 128 tiles (K = 2048: 40 us against 18 us), so the large tile wins where its last round is not too empty.  Both sides
+  // of the line, us (large / small): 2048 x 4096 x 2048 (128 large tiles) 39.8 / 37.6, 2331 x 4096 x 2048 (160) 40.0 / 54.1;
+  // 3072 x 2304 x 768 (108) 20.9 / 19.0, 4096 x 2304 x 768 (144) 21.5 / 27.9; 777 x 2 x 9216 x 768 (288) 41 / 28,
+  // 1536 x 2 x 9216 x 768 (432) 43 / 51; 384 x 50257 x 768 (394) 38.5 / 45.6.
+  if (9 * ((big + gemm_cus() - 1) / gemm_cus()) * gemm_cus() < 4 * small)
+    return gemm_pp_launch<MODE>(A, lda, W, W2, R, ldr, C, ldc, M, N, K, s);
+  // A grid that leaves one workgroup per compute unit anyway gains from the deeper pipeline when K is long (M=4096, N=768,
+  // K=9216: 83 us against 93 us).
   if constexpr (MODE != 1) {
     // A feature count that is a whole number of 96-wide tiles but leaves compute units idle (or nearly idle in a last
     // round) with 128-wide ones: the time follows the rounds a compute unit runs times the area of a tile

@@ -247,7 +247,31 @@ def test_gemm_bf16_splitk_feeds_the_residual_norm(hip, M, N, K, ks):
     check(h, O.rms_norm(xd.cpu(), nw, O.RMS_EPS_DEFAULT), torch.bfloat16, frac=0.05)
 
 
-@pytest.mark.parametrize("M,N,K", [(17, 1, 32), (31, 259, 128), (33, 130, 64), (130, 1031, 1056), (700, 515, 1024), (4100, 10003, 1024)])
+@pytest.mark.parametrize("M,N,K", [(1030, 16388, 64), (1030, 16388, 192), (2100, 8200, 320)])
+def test_gemm_bf16_alternating_groups(hip, M, N, K):
+    """The 256 x 256 kernel (grids of more than 2.25 rounds of 128 x 128 tiles) at its edges: one k tile and odd numbers of
+    them, ragged last rows and features, several tiles per workgroup; the three modes against fp32 rounded where the
+    reference rounds, bounds as for the other tiles."""
+    g = gen(66)
+    x = torch.randn(M, K, generator=g).bfloat16()
+    W = (torch.randn(N, K, generator=g) / math.sqrt(K)).bfloat16()
+    res = torch.randn(M, N, generator=g).bfloat16()
+    ref = F.linear(x.float(), W.float()).bfloat16()
+    xd, Wd = dev(x), dev(W)
+    check(hip.gemm(xd, Wd), ref, torch.bfloat16)
+    rd = dev(res.clone())
+    hip.gemm(xd, Wd, residual=rd, out=rd)
+    check(rd, (res.float() + ref.float()).bfloat16(), torch.bfloat16, frac=0.05, atol=2.0 ** -7 * float(ref.float().abs().max()))
+    n2 = N // 2 - N // 2 % 4
+    act = hip.gemm(xd, Wd[:n2].contiguous(), up_weight=Wd[n2:2 * n2].contiguous()).float().cpu()
+    gate, up = ref[:, :n2].float(), ref[:, n2:2 * n2].float()
+    want = (F.gelu(ref[:, :n2], approximate="tanh") * ref[:, n2:2 * n2]).float()
+    tol = want.abs() * 2.0 ** -6 + 1.2 * 2.0 ** -7 * (gate * up).abs() + 1e-3 * 2.0 ** -7 * float(want.abs().max())   # as below
+    assert bool(((act - want).abs() <= tol).all())
+    assert float(((act - want).abs() > 0).float().mean()) <= 0.05
+
+
+@pytest.mark.parametrize("M,N,K", [(1283, 15001, 128), (17, 1, 32), (31, 259, 128), (33, 130, 64), (130, 1031, 1056), (700, 515, 1024), (4100, 10003, 1024)])
 def test_gemm_bf16_plain_any_feature_count(hip, M, N, K):
     """Mode 0 with N % 4 != 0 and an odd row stride (the vocabulary of the tied head), every tile shape: one bf16 ulp
     against F.linear in fp32 rounded once, and nothing written beside the (M, N) block."""
