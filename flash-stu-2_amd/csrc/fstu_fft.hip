@@ -1,548 +1,734 @@
-// Spectral convolution of the STU prefill as the reference computes it (rfft -> product -> irfft,
-// flash_stu/utils/stu_utils.py:195-246), as in-LDS complex FFTs on gfx950.
+// Spectral convolution of the STU prefill (flash_stu/utils/stu_utils.py:195-246: rfft -> product -> irfft, both sign
+// branches), as in-LDS complex FFTs on gfx950, on the two parities of the sequence at once.
 //
-// One workgroup transforms `cols` whole columns (one (batch, channel) signal each) that live in LDS from the
-// first load to the last store: forward decimation-in-frequency passes (natural order in, digit-reversed order
-// out), a pointwise product with a filter spectrum stored in that same digit-reversed order, and the mirrored
-// decimation-in-time passes back to natural order.  No bit-reversal pass is ever needed.  A pass is a radix-16
-// (first pass: 2, 4, 8 or 16) butterfly held in registers, so a length-4096 transform touches LDS three times.
+// With E and O the even- and odd-lag parts of the causal convolution of x with a filter f, the two branches are
+// plus = E + O and minus = E - O.  Lags of one parity connect positions of fixed parities only, so with
+//     z[m] = x[2m] + i x[2m+1],   fe[j] = f[2j],   fo[j] = f[2j+1]
+// the convolution of the complex sequence z with the REAL filter fe holds E of both parities, E[2m] + i E[2m+1], and its
+// convolution with fo holds Re[m] = O[2m+1] and Im[m] = O[2m+2].  One forward transform of z and one inverse per part
+// replace a forward and an inverse transform of twice the length: for approx mode three transforms of n/2 points instead
+// of two of n, for a bank of K filters 1 + 2K of n/2 instead of 1 + K of n, each one level shorter and in half the LDS,
+// so that two workgroups share a compute unit where one filled it.
 //
-// Both sign branches come out of ONE inverse transform: with F the filter's spectrum, the minus branch
-// conv(x, (-1)^s f) has spectrum F[k + n/2], so the product X * (F[k] + i F[k + n/2]) inverts to
-// plus + i*minus (both real).  k + n/2 sits at digit-reversed position p ^ 8 because the last pass has radix 16.
+// A transform of N = n/2 points belongs to N/16 threads, 16 points each.  Forward: radix-2 stages grouped by four in
+// registers, natural order in, bit-reversed out (twiddles depend on the block); the last group stays in registers, where
+// the spectrum is multiplied; inverse: bit-reversed in, natural out (twiddles depend on the position).  Both directions
+// multiply BEFORE they add, so a butterfly with its twiddle is six fused multiply-adds (u = a + w b, v = 2a - u) and a
+// group of 16 points 192 instructions and 8 twiddles; a radix-16 butterfly followed by 15 twiddles took 228, and 44 more
+// for the powers.  The upper half of z is zero and only the lower half of the results is wanted: the first stage copies
+// and the last produces half.  The two innermost groups exchange among 16 threads of one wave, without a barrier.
+//
+// What bounds it: vector-ALU issue.  The exact-mode bank of 4 x 8192 x 1024 positions and channels and 24 filters issues 1.6 k
+// instructions per thread and filter, 4.9 M cycles of every compute unit's four SIMDs, and takes 2.73 ms = 5.6 M cycles
+// (4.66 ms on transforms of 16384 points in 139 KB of LDS, one workgroup per compute unit; 3.77 ms while spectra and
+// twiddles lay in position order, so that every load of a wave touched up to 64 lines).  bf16, before -> now, us: 8 x 512 x
+// 768 24.5 -> 17.4, 32 x 300 x 2048 188 -> 105, 4 x 4096 x 2048 296 -> 218, one time-major sequence of 4096 x 2048 95 -> 50.
 #include "fstu_common.h"
 
 namespace {
 
 typedef float2 cpx;
 
-__device__ __forceinline__ cpx cadd(cpx a, cpx b) { return make_float2(a.x + b.x, a.y + b.y); }
-__device__ __forceinline__ cpx csub(cpx a, cpx b) { return make_float2(a.x - b.x, a.y - b.y); }
-__device__ __forceinline__ cpx cmul(cpx a, cpx b) {
-  return make_float2(fmaf(a.x, b.x, -a.y * b.y), fmaf(a.x, b.y, a.y * b.x));
-}
-// a * conj(b)
-__device__ __forceinline__ cpx cmulc(cpx a, cpx b) {
-  return make_float2(fmaf(a.x, b.x, a.y * b.y), fmaf(a.y, b.x, -a.x * b.y));
-}
-__device__ __forceinline__ cpx cconj(cpx a) { return make_float2(a.x, -a.y); }
-
-// LDS index of element i of a column: one pad slot every 16 elements keeps the stride-16 accesses of the
-// last pass (and every other power-of-two stride) off a single bank.
+// LDS index of element i of a column: one pad slot every 16 elements keeps the stride-16 accesses of the stride-1 group
+// (and every other power-of-two stride) off a single bank.
 __device__ __forceinline__ int phys(int i) { return i + (i >> 4); }
 
-// z * exp(-2 pi i k / 16), k = 0..7, k known at compile time after unrolling
-__device__ __forceinline__ cpx mul_root16(cpx z, int k) {
-  const float s = 0.70710678118654752f, c1 = 0.92387953251128674f, s1 = 0.38268343236508977f;
-  switch (k) {
-    case 0: return z;
-    case 1: return make_float2(fmaf(c1, z.x, s1 * z.y), fmaf(c1, z.y, -s1 * z.x));
-    case 2: return make_float2((z.x + z.y) * s, (z.y - z.x) * s);
-    case 3: return make_float2(fmaf(s1, z.x, c1 * z.y), fmaf(s1, z.y, -c1 * z.x));
-    case 4: return make_float2(z.y, -z.x);
-    case 5: return make_float2(fmaf(-s1, z.x, c1 * z.y), fmaf(-s1, z.y, -c1 * z.x));
-    case 6: return make_float2((z.y - z.x) * s, -(z.x + z.y) * s);
-    default: return make_float2(fmaf(-c1, z.x, s1 * z.y), fmaf(-c1, z.y, -s1 * z.x));
-  }
+// ---------------------------------------------------------------- butterflies
+// (a, b) <- (a + w r b, a - w r b), r = 1 or (ROT) the quarter turn of the direction (-i forward, +i inverse)
+template <bool INV, bool ROT>
+__device__ __forceinline__ cpx turn(cpx b) {
+  if constexpr (!ROT) return b;
+  return INV ? make_float2(-b.y, b.x) : make_float2(b.y, -b.x);
 }
+template <bool INV, bool ROT>
+__device__ __forceinline__ void bfly1(cpx& a, cpx& b) {
+  const cpx t = turn<INV, ROT>(b);
+  b = make_float2(a.x - t.x, a.y - t.y);
+  a = make_float2(a.x + t.x, a.y + t.y);
+}
+template <bool INV, bool ROT>
+__device__ __forceinline__ void bfly(cpx& a, cpx& b, cpx w) {
+  const cpx t = turn<INV, ROT>(b);
+  const cpx u = make_float2(fmaf(-w.y, t.y, fmaf(w.x, t.x, a.x)), fmaf(w.y, t.x, fmaf(w.x, t.y, a.y)));
+  b = make_float2(fmaf(2.f, a.x, -u.x), fmaf(2.f, a.y, -u.y));
+  a = u;
+}
+// a + w r b alone
+template <bool INV, bool ROT>
+__device__ __forceinline__ cpx bsum(cpx a, cpx b, cpx w) {
+  const cpx t = turn<INV, ROT>(b);
+  return make_float2(fmaf(-w.y, t.y, fmaf(w.x, t.x, a.x)), fmaf(w.y, t.x, fmaf(w.x, t.y, a.y)));
+}
+__device__ __forceinline__ cpx cmul(cpx a, cpx b) { return make_float2(fmaf(a.x, b.x, -a.y * b.y), fmaf(a.x, b.y, a.y * b.x)); }
 
-template <int R> __device__ __forceinline__ constexpr int brev(int k) {
+// ---------------------------------------------------------------- groups of 2^G points in registers
+// cos / sin of k/32 turns, k = 0 .. 7
+__device__ __forceinline__ constexpr float cos32(int k) {
+  constexpr float c[8] = {1.f, 0.98078528040323044f, 0.92387953251128674f, 0.83146961230254524f, 0.70710678118654752f, 0.55557023301960222f, 0.38268343236508977f, 0.19509032201612827f};
+  return c[k];
+}
+__device__ __forceinline__ constexpr float sin32(int k) { return k == 0 ? 0.f : cos32(8 - k); }
+// e^(+-2 pi i k / 32), k = 0 .. 7
+template <bool INV> __device__ __forceinline__ cpx root32(int k) { return make_float2(cos32(k), INV ? sin32(k) : -sin32(k)); }
+template <bool INV> __device__ __forceinline__ cpx turn32(cpx z, int k) {
+  if (k == 0) return z;
+  if (k == 4) return INV ? make_float2((z.x - z.y) * cos32(4), (z.x + z.y) * cos32(4)) : make_float2((z.x + z.y) * cos32(4), (z.y - z.x) * cos32(4));
+  const float c = cos32(k), s = INV ? sin32(k) : -sin32(k);
+  return make_float2(fmaf(c, z.x, -s * z.y), fmaf(c, z.y, s * z.x));
+}
+__host__ __device__ constexpr int brev_bits(int v, int bits) {
   int r = 0;
-  for (int b = 1; b < R; b <<= 1) {
-    r = (r << 1) | (k & 1);
-    k >>= 1;
-  }
+  for (int i = 0; i < bits; ++i) r |= ((v >> i) & 1) << (bits - 1 - i);
   return r;
 }
+template <int G> struct Powers { cpx w[G]; };     // w^(2^i)
 
-// In-register DFT of R points (R = 2, 4, 8, 16): input v[m] in natural order, output k left in v[brev(k)].
-template <int R> __device__ __forceinline__ void dft_inreg(cpx (&v)[R]) {
+// G forward stages on 2^G points a fixed distance apart, natural order in, bit-reversed out.  TW: times the block's
+// twiddles t; HALF0: the upper half of the inputs is zero.
+template <int G, bool TW, bool HALF0>
+__device__ __forceinline__ void fwd_stages(cpx* v, const Powers<G>& t) {
 #pragma unroll
-  for (int h = R / 2; h >= 1; h >>= 1) {
+  for (int s = 0; s < G; ++s) {
+    const int dist = 1 << (G - 1 - s);
 #pragma unroll
-    for (int b0 = 0; b0 < R; b0 += 2 * h) {
+    for (int b = 0; b < (1 << s); ++b) {
+      const int k = brev_bits(b, s), quarter = s > 0 ? 1 << (s - 1) : 1;
+      const bool rot = s > 0 && k >= quarter;
+      const int kr = (rot ? k - quarter : k) << (4 - s);            // in 1/32 turns
 #pragma unroll
-      for (int j = 0; j < h; ++j) {
-        cpx a = v[b0 + j], b = v[b0 + j + h];
-        v[b0 + j] = cadd(a, b);
-        v[b0 + j + h] = mul_root16(csub(a, b), j * (8 / h));
+      for (int j = 0; j < dist; ++j) {
+        cpx &x = v[b * 2 * dist + j], &y = v[b * 2 * dist + j + dist];
+        if (s == 0 && HALF0) { y = x; continue; }
+        if (!TW && kr == 0) {
+          if (rot) bfly1<false, true>(x, y); else bfly1<false, false>(x, y);
+        } else {
+          const cpx w = TW ? turn32<false>(t.w[G - 1 - s], kr) : root32<false>(kr);
+          if (rot) bfly<false, true>(x, y, w); else bfly<false, false>(x, y, w);
+        }
+      }
+    }
+  }
+}
+// G inverse stages, bit-reversed in, natural out; t holds the conjugate twiddles of the position.  LOWER: only the lower
+// half of the results is produced.
+template <int G, bool TW, bool LOWER>
+__device__ __forceinline__ void inv_stages(cpx* v, const Powers<G>& t) {
+#pragma unroll
+  for (int s = 0; s < G; ++s) {
+    const int dist = 1 << s;
+#pragma unroll
+    for (int b = 0; b < (1 << s); ++b) {
+      const int quarter = s > 0 ? 1 << (s - 1) : 1;
+      const bool rot = s > 0 && b >= quarter;
+      const int kr = (rot ? b - quarter : b) << (4 - s);
+#pragma unroll
+      for (int g = 0; g < (1 << G); g += 2 * dist) {
+        cpx &x = v[g + b], &y = v[g + b + dist];
+        const cpx w = TW ? turn32<true>(t.w[G - 1 - s], kr) : root32<true>(kr);
+        if (LOWER && s == G - 1) {
+          if (rot) x = bsum<true, true>(x, y, w); else x = bsum<true, false>(x, y, w);
+        } else if (!TW && kr == 0) {
+          if (rot) bfly1<true, true>(x, y); else bfly1<true, false>(x, y);
+        } else {
+          if (rot) bfly<true, true>(x, y, w); else bfly<true, false>(x, y, w);
+        }
       }
     }
   }
 }
 
-// a * exp(-2 pi i k / 16) for a real a (the values mul_root16 gives for z = (a, 0))
-__device__ __forceinline__ cpx mul_root16_real(float a, int k) {
-  const float s = 0.70710678118654752f, c1 = 0.92387953251128674f, s1 = 0.38268343236508977f;
-  switch (k) {
-    case 0: return make_float2(a, 0.f);
-    case 1: return make_float2(c1 * a, -s1 * a);
-    case 2: return make_float2(a * s, -a * s);
-    case 3: return make_float2(s1 * a, -c1 * a);
-    case 4: return make_float2(0.f, -a);
-    case 5: return make_float2(-s1 * a, -c1 * a);
-    case 6: return make_float2(-a * s, -a * s);
-    default: return make_float2(-c1 * a, -s1 * a);
-  }
+// ---------------------------------------------------------------- a transform on N/16 threads, 16 points each
+// Groups of stages from the inside out: four at stride 1 (16 neighbours), four at stride 16 (16 neighbouring threads
+// exchange: one wave), four at stride 256, and the LOGN mod 4 remaining ones outermost.  Natural order is held by the
+// threads of the outermost group, in registers: point r + Q*m with r = u + i*G (i < NI), m < R; of the zero-padded input
+// and of the results only the lower half, m < R/2, 8 points per thread.
+template <int LOGN> struct Half {
+  static constexpr int N = 1 << LOGN, G = N / 16, STRIDE = N + N / 16, REM = LOGN & 3, NF = LOGN / 4;
+  static constexpr int GL = REM ? REM : 4, R = 1 << GL, Q = N / R, NI = 16 / R, H = R / 2;   // the outermost group
+  static constexpr int MID = REM ? NF - 1 : NF - 2;                                        // groups between it and stride 1
+  static constexpr bool ONE_WAVE = G <= 64;                                                // a column's threads are in one wave
+};
+
+// the exchange through LDS behind a group: among the threads of one wave, or of the workgroup
+__device__ __forceinline__ void wave_sync() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_sched_barrier(0);   // the next group starts with its own registers
+}
+template <int LOGN> __device__ __forceinline__ void col_sync() {
+  if constexpr (Half<LOGN>::ONE_WAVE) wave_sync();
+  else __syncthreads();
 }
 
-// The R-point DFT of a real input whose upper half is zero (a zero-padded signal in the first pass of its transform):
-// the first stage adds and subtracts nothing, v[j + R/2] = x[j] W_R^j, and the other stages run as always.
-// in: x[0 .. R/2) ; out: as dft_inreg.
-template <int R> __device__ __forceinline__ void dft_inreg_real_half(const float (&x)[R / 2], cpx (&v)[R]) {
-#pragma unroll
-  for (int j = 0; j < R / 2; ++j) {
-    v[j] = make_float2(x[j], 0.f);
-    v[j + R / 2] = mul_root16_real(x[j], j * (16 / R));
-  }
-#pragma unroll
-  for (int h = R / 4; h >= 1; h >>= 1) {
-#pragma unroll
-    for (int b0 = 0; b0 < R; b0 += 2 * h) {
-#pragma unroll
-      for (int j = 0; j < h; ++j) {
-        cpx a = v[b0 + j], b = v[b0 + j + h];
-        v[b0 + j] = cadd(a, b);
-        v[b0 + j + h] = mul_root16(csub(a, b), j * (8 / h));
-      }
-    }
-  }
-}
-
-// powers 1..R-1 of w = tw[r*ts] : the binary powers come from the table, the rest are products of two of them
-template <int R> __device__ __forceinline__ void twiddle_powers(cpx (&pw)[R], const cpx* __restrict__ tw, int e) {
-  pw[0] = make_float2(1.f, 0.f);
-  pw[1] = tw[e];
-  if (R >= 4) {
-    pw[2] = tw[2 * e];
-    pw[3] = cmul(pw[1], pw[2]);
-  }
-  if (R >= 8) {
-    pw[4] = tw[4 * e];
-    pw[5] = cmul(pw[4], pw[1]);
-    pw[6] = cmul(pw[4], pw[2]);
-    pw[7] = cmul(pw[4], pw[3]);
-  }
-  if (R >= 16) {
-    pw[8] = tw[8 * e];
-#pragma unroll
-    for (int k = 1; k < 8; ++k) pw[8 + k] = cmul(pw[8], pw[k]);
-  }
-}
-
-template <int R> __host__ __device__ constexpr int lg_radix() { return R == 16 ? 4 : R == 8 ? 3 : R == 4 ? 2 : 1; }
-
-// One radix-R butterfly of a pass over blocks of Nb = R*q elements (q = 1 << LQ).  Forward: decimation in
-// frequency, y[k] = w^(r k) * sum_m x[m] W_R^(m k) written where x was read.  Inverse: the exact mirror.
-// The transform length and the stride are compile-time constants: the R points of a butterfly sit a fixed distance
-// apart in the padded column (q + q/16 slots; q = 1 only occurs with R = 16 on blocks that start at a multiple of
-// 16), so their addresses are one base and immediate offsets.
-// HALF 1 (forward, first pass of a transform): the inputs are real and the upper half of the column is zero (a signal
-// of at most n/2 samples): only the lower half's real parts are read.  HALF 2 (inverse, last pass): only the lower
-// half of the column is wanted afterwards, the other outputs are neither stored nor (their last stage) computed.
-template <int R, bool INV, int LQ, int LOGN, int HALF = 0>
-__device__ __forceinline__ void butterfly(cpx* __restrict__ col, const cpx* __restrict__ tw, int u) {
-  static_assert(HALF == 0 || (HALF == 1 && !INV) || (HALF == 2 && INV), "half-column passes: forward first, inverse last");
-  static_assert(HALF == 0 || LQ + lg_radix<R>() == LOGN, "half-column passes span the whole column");
-  constexpr int LR = lg_radix<R>();
-  constexpr int q = 1 << LQ;
-  constexpr int TS = 1 << (LOGN - LQ - LR);   // table stride: w_Nb = tw[TS]
-  constexpr int ST = (LQ >= 4) ? (q + (q >> 4)) : 1;
-  static_assert(LQ == 0 || LQ >= 4, "strides between 2 and 8 would cross a pad slot");
-  const int r = u & (q - 1);
-  const int base = ((u >> LQ) << (LQ + LR)) + r;
-  cpx* __restrict__ p = col + phys(base);
-  cpx v[R], pw[R];
-  constexpr bool twid = LQ > 0;
-  if (twid) twiddle_powers<R>(pw, tw, r * TS);
-  if (!INV) {
-    if constexpr (HALF == 1) {
-      float xr[R / 2];
-#pragma unroll
-      for (int m = 0; m < R / 2; ++m) xr[m] = p[m * ST].x;
-      dft_inreg_real_half<R>(xr, v);
-    } else {
-#pragma unroll
-      for (int m = 0; m < R; ++m) v[m] = p[m * ST];
-      dft_inreg<R>(v);
-    }
-#pragma unroll
-    for (int k = 0; k < R; ++k) {
-      cpx o = v[brev<R>(k)];
-      if (twid && k > 0) o = cmul(o, pw[k]);
-      p[k * ST] = o;
-    }
+// The twiddle table: for every group the powers 1, 2, 4, 8 of the twiddles of its positions (inverse, conjugated) or
+// blocks (forward, in block order), as planes of two powers each, so that the lanes of a wave read whole lines and a
+// group's twiddles are at most two loads.  All of it fits the n entries of exp(-2 pi i j / n).
+template <int LOGN> struct Table {
+  using W = Half<LOGN>;
+  static constexpr int planes(int stages) { return stages == 1 ? 1 : stages == 2 ? 2 : 4; }    // entries per position
+  static constexpr int INV1 = 0;                                                   // stride 16: 16 positions
+  static constexpr int INV2 = INV1 + (W::MID >= 1 ? 16 * 4 : 0);                   // stride 256
+  static constexpr int OUTER = INV2 + (W::MID >= 2 ? 256 * 4 : 0);                 // outermost group: Q positions
+  static constexpr int FWD2 = OUTER + W::Q * planes(W::GL);
+  static constexpr int FWD1 = FWD2 + (W::MID >= 2 ? (W::N >> 12) * 4 : 0);         // stride 16: N / 256 blocks
+  static constexpr int FWD0 = FWD1 + (W::MID >= 1 ? (W::N >> 8) * 4 : 0);          // stride 1: N / 16 blocks
+  static constexpr int END = FWD0 + (W::N >> 4) * 4;
+  static_assert(END <= 2 * W::N, "the table fits n entries");
+};
+// GS powers of entry i of a part of the table that has `count` entries
+template <int GS> __device__ __forceinline__ Powers<GS> powers(const cpx* __restrict__ part, int count, int i) {
+  Powers<GS> t;
+  if constexpr (GS == 1) {
+    t.w[0] = part[i];
   } else {
-#pragma unroll
-    for (int k = 0; k < R; ++k) {
-      cpx o = p[k * ST];
-      if (twid && k > 0) o = cmulc(o, pw[k]);
-      v[k] = cconj(o);
+    const float4 a = ((const float4*)part)[i];
+    t.w[0] = make_float2(a.x, a.y);
+    t.w[1] = make_float2(a.z, a.w);
+    if constexpr (GS > 2) {
+      const float4 c = ((const float4*)part)[count + i];
+      t.w[2] = make_float2(c.x, c.y);
+      if constexpr (GS > 3) t.w[3] = make_float2(c.z, c.w);
     }
-    dft_inreg<R>(v);
-#pragma unroll
-    for (int m = 0; m < (HALF == 2 ? R / 2 : R); ++m) p[m * ST] = cconj(v[brev<R>(m)]);
   }
+  return t;
+}
+// position of the thread's k-th natural-order point (k < 8)
+template <int LOGN> __device__ __forceinline__ int point(int u, int k) {
+  using W = Half<LOGN>;
+  return u + (k / W::H) * W::G + (k % W::H) * W::Q;
 }
 
-template <int LOGN> __host__ __device__ constexpr int col_stride() { return (1 << LOGN) + (1 << (LOGN - 4)); }
-
-template <int R, bool INV, int LQ, int LOGN, int NT, int HALF = 0>
-__device__ __forceinline__ void run_pass(cpx* lds, const cpx* __restrict__ tw, int cols) {
-  constexpr int LPER = LOGN - lg_radix<R>();   // log2 of butterflies per column
-  const int total = cols << LPER;
-  for (int w = threadIdx.x; w < total; w += NT)
-    butterfly<R, INV, LQ, LOGN, HALF>(lds + (size_t)(w >> LPER) * col_stride<LOGN>(), tw, w & ((1 << LPER) - 1));
-  __syncthreads();
+// LDS index of the thread's i-th butterfly of the outermost group
+template <int LOGN> __device__ __forceinline__ int butterfly_at(int u, int i) {
+  using W = Half<LOGN>;
+  if constexpr (W::G >= 16) return phys(u) + i * (W::G + W::G / 16);
+  return phys(u + i * W::G);
 }
 
-// LOGN = 4*a + rem: the first forward pass has radix 2^rem (if rem > 0), every other pass radix 16.  The last forward
-// pass and the first inverse pass work on the same 16 neighbours of a column (stride 1): callers that multiply by a
-// spectrum in between skip both here and do the three steps in registers (fft_middle).
-// HALF_COL: the columns hold real signals of at most n/2 samples (forward: the pass that spans the whole column reads
-// only those; inverse: only the lower half of the result is produced).
-// NO_R2 (lengths with a radix-2 pass): the caller performs that pass itself while it writes the column (forward) or
-// collects the results (inverse).
-template <int LOGN, int NT, bool SKIP_LAST, bool HALF_COL = false, bool NO_R2 = false>
-__device__ __forceinline__ void fft_forward(cpx* lds, const cpx* __restrict__ tw, int cols) {
-  constexpr int REM = LOGN & 3, TOP = LOGN - REM;
-  constexpr int H = HALF_COL ? 1 : 0;
-  constexpr int H16A = (REM == 0 && TOP == 12) ? H : 0, H16B = (REM == 0 && TOP == 8) ? H : 0;
-  if constexpr (REM == 1 && !NO_R2) run_pass<2, false, LOGN - 1, LOGN, NT, H>(lds, tw, cols);
-  if constexpr (REM == 2) run_pass<4, false, LOGN - 2, LOGN, NT, H>(lds, tw, cols);
-  if constexpr (REM == 3) run_pass<8, false, LOGN - 3, LOGN, NT, H>(lds, tw, cols);
-  if constexpr (TOP >= 12) run_pass<16, false, 8, LOGN, NT, H16A>(lds, tw, cols);
-  if constexpr (TOP >= 8) run_pass<16, false, 4, LOGN, NT, H16B>(lds, tw, cols);
-  if constexpr (!SKIP_LAST) run_pass<16, false, 0, LOGN, NT>(lds, tw, cols);
-}
-
-template <int LOGN, int NT, bool SKIP_FIRST, bool HALF_COL = false, bool NO_R2 = false>
-__device__ __forceinline__ void fft_inverse(cpx* lds, const cpx* __restrict__ tw, int cols) {
-  constexpr int REM = LOGN & 3, TOP = LOGN - REM;
-  constexpr int H = HALF_COL ? 2 : 0;
-  constexpr int H16A = (REM == 0 && TOP == 12) ? H : 0, H16B = (REM == 0 && TOP == 8) ? H : 0;
-  if constexpr (!SKIP_FIRST) run_pass<16, true, 0, LOGN, NT>(lds, tw, cols);
-  if constexpr (TOP >= 8) run_pass<16, true, 4, LOGN, NT, H16B>(lds, tw, cols);
-  if constexpr (TOP >= 12) run_pass<16, true, 8, LOGN, NT, H16A>(lds, tw, cols);
-  if constexpr (REM == 1 && !NO_R2) run_pass<2, true, LOGN - 1, LOGN, NT, H>(lds, tw, cols);
-  if constexpr (REM == 2) run_pass<4, true, LOGN - 2, LOGN, NT, H>(lds, tw, cols);
-  if constexpr (REM == 3) run_pass<8, true, LOGN - 3, LOGN, NT, H>(lds, tw, cols);
-}
-
-// 16 spectrum values of 16 neighbouring positions (128 contiguous bytes)
-__device__ __forceinline__ void load_spec16(const cpx* __restrict__ sp, cpx (&s)[16]) {
-#pragma unroll
-  for (int k = 0; k < 16; k += 2) {
-    const float4 t = *(const float4*)(sp + k);
-    s[k] = make_float2(t.x, t.y);
-    s[k + 1] = make_float2(t.z, t.w);
-  }
-}
-
-// forward stride-1 butterfly of 16 neighbours, left in registers in position order (x[k] belongs to position base + k)
-__device__ __forceinline__ void forward16(const cpx* __restrict__ p, cpx (&x)[16]) {
+// four stages at stride 16^LEVEL, in place
+template <int LOGN, int LEVEL>
+__device__ __forceinline__ void fwd_mid(cpx* __restrict__ col, const cpx* __restrict__ tw, int u) {
+  constexpr int LQ = 4 * LEVEL, S = LOGN - 4 - LQ, ST = (1 << LQ) + (1 << LQ) / 16;
+  const int blk = u >> LQ;
+  const Powers<4> t = powers<4>(tw + (LEVEL == 1 ? Table<LOGN>::FWD1 : Table<LOGN>::FWD2), 1 << S, blk);
+  cpx* p = col + phys((blk << (LQ + 4)) + (u & ((1 << LQ) - 1)));
   cpx v[16];
 #pragma unroll
-  for (int m = 0; m < 16; ++m) v[m] = p[m];
-  dft_inreg<16>(v);
+  for (int m = 0; m < 16; ++m) v[m] = p[m * ST];
+  fwd_stages<4, true, false>(v, t);
 #pragma unroll
-  for (int k = 0; k < 16; ++k) x[k] = v[brev<16>(k)];
+  for (int m = 0; m < 16; ++m) p[m * ST] = v[m];
 }
-
-// x[k] * s[k] through the inverse stride-1 butterfly, written to the 16 neighbours
-__device__ __forceinline__ void product_inverse16(cpx* __restrict__ p, const cpx (&x)[16], const cpx (&s)[16]) {
+template <int LOGN, int LEVEL>
+__device__ __forceinline__ void inv_mid(cpx* __restrict__ col, const cpx* __restrict__ tw, int u) {
+  constexpr int LQ = 4 * LEVEL, ST = (1 << LQ) + (1 << LQ) / 16;
+  const int r = u & ((1 << LQ) - 1);
+  const Powers<4> t = powers<4>(tw + (LEVEL == 1 ? Table<LOGN>::INV1 : Table<LOGN>::INV2), 1 << LQ, r);
+  cpx* p = col + phys(((u >> LQ) << (LQ + 4)) + r);
   cpx v[16];
 #pragma unroll
-  for (int k = 0; k < 16; ++k) v[k] = cconj(cmul(x[k], s[k]));
-  dft_inreg<16>(v);
+  for (int m = 0; m < 16; ++m) v[m] = p[m * ST];
+  inv_stages<4, true, false>(v, t);
 #pragma unroll
-  for (int m = 0; m < 16; ++m) p[m] = cconj(v[brev<16>(m)]);
+  for (int m = 0; m < 16; ++m) p[m * ST] = v[m];
 }
 
-// last forward pass, product with the per-column spectra spec[(c0 + col) * n + position], first inverse pass
-template <int LOGN, int NT>
-__device__ __forceinline__ void fft_middle(cpx* lds, const cpx* __restrict__ spec, int c0, int ncol) {
-  constexpr int LPER = LOGN - 4;
-  const int total = ncol << LPER;
-  for (int w = threadIdx.x; w < total; w += NT) {
-    const int colid = w >> LPER, u = w & ((1 << LPER) - 1);
-    cpx* p = lds + (size_t)colid * col_stride<LOGN>() + 17 * u;   // phys(16 u)
-    cpx s[16], x[16];
-    load_spec16(spec + ((size_t)(c0 + colid) << LOGN) + 16 * u, s);
-    forward16(p, x);
-    product_inverse16(p, x, s);
+// z: the thread's 8 points of the lower half -> xs: spectrum of positions 16u .. 16u+15 (bit-reversed order).  When it
+// returns, a thread may overwrite its own 16 positions of the column.
+template <int LOGN>
+__device__ __forceinline__ void fft_forward(cpx* __restrict__ col, const cpx* __restrict__ tw, int u, const cpx (&z)[8], cpx (&xs)[16]) {
+  using W = Half<LOGN>;
+#pragma unroll
+  for (int i = 0; i < W::NI; ++i) {
+    cpx v[W::R];
+#pragma unroll
+    for (int m = 0; m < W::H; ++m) v[m] = z[i * W::H + m];
+    fwd_stages<W::GL, false, true>(v, Powers<W::GL>{});
+    cpx* p = col + butterfly_at<LOGN>(u, i);
+#pragma unroll
+    for (int m = 0; m < W::R; ++m) p[m * (W::Q + W::Q / 16)] = v[m];
   }
-  __syncthreads();
+  if constexpr (W::MID >= 2) { col_sync<LOGN>(); fwd_mid<LOGN, 2>(col, tw, u); }
+  if constexpr (W::MID >= 1) { col_sync<LOGN>(); fwd_mid<LOGN, 1>(col, tw, u); }
+  if constexpr (W::MID == 0) col_sync<LOGN>();
+  else wave_sync();
+  const Powers<4> t = powers<4>(tw + Table<LOGN>::FWD0, W::G, u);
+#pragma unroll
+  for (int m = 0; m < 16; ++m) xs[m] = col[17 * u + m];
+  fwd_stages<4, true, false>(xs, t);
+}
+
+// v: spectrum of positions 16u .. 16u+15 -> r: the thread's 8 points of the lower half of the result.  The thread's own 16
+// positions of the column must be free; when it returns, other threads may still read the column.
+template <int LOGN>
+__device__ __forceinline__ void fft_inverse(cpx* __restrict__ col, const cpx* __restrict__ tw, int u, cpx (&v)[16], cpx (&r)[8]) {
+  using W = Half<LOGN>;
+  inv_stages<4, false, false>(v, Powers<4>{});
+#pragma unroll
+  for (int m = 0; m < 16; ++m) col[17 * u + m] = v[m];
+  if constexpr (W::MID == 0) col_sync<LOGN>();
+  else wave_sync();
+  if constexpr (W::MID >= 1) { inv_mid<LOGN, 1>(col, tw, u); col_sync<LOGN>(); }
+  if constexpr (W::MID >= 2) { inv_mid<LOGN, 2>(col, tw, u); col_sync<LOGN>(); }
+#pragma unroll
+  for (int i = 0; i < W::NI; ++i) {
+    const int rr = u + i * W::G;
+    const Powers<W::GL> t = powers<W::GL>(tw + Table<LOGN>::OUTER, W::Q, rr);
+    const cpx* p = col + butterfly_at<LOGN>(u, i);
+    cpx x[W::R];
+#pragma unroll
+    for (int m = 0; m < W::R; ++m) x[m] = p[m * (W::Q + W::Q / 16)];
+    inv_stages<W::GL, true, true>(x, t);
+#pragma unroll
+    for (int m = 0; m < W::H; ++m) r[i * W::H + m] = x[m];
+  }
+}
+
+// Im of the result one position earlier (0 in front of the first) for each of a thread's 8 results: the neighbouring
+// lane's, and across the ends of the waves through rec, 8 floats per wave (or column, where a wave holds several) of the
+// workgroup.  Contains the barrier behind which the column is free.
+template <int LOGN>
+__device__ __forceinline__ void earlier_im(const cpx (&r)[8], float (&prev)[8], float* rec, int u) {
+  using W = Half<LOGN>;
+  constexpr int SEG = W::G < 64 ? W::G : 64;           // threads of a column in one wave
+  const int seg = threadIdx.x / SEG, in = u % SEG;
+  if (in == SEG - 1) {
+#pragma unroll
+    for (int k = 0; k < 8; ++k) rec[seg * 8 + k] = r[k].y;
+  }
+  col_sync<LOGN>();
+#pragma unroll
+  for (int k = 0; k < 8; ++k) prev[k] = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(r[k].y), 0x138, 0xf, 0xf, true));   // lane - 1
+  if (in == 0) {
+    // u > 0: the last thread of the wave in front; u == 0: the column's last thread, one butterfly (or, for the first of
+    // them, one step of Q) earlier
+    const float* q = rec + (u > 0 ? seg - 1 : seg + W::G / SEG - 1) * 8;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const int wrap = k >= W::H ? k - W::H : (W::NI - 1) * W::H + k - 1;
+      prev[k] = u > 0 ? q[k] : (k > 0 ? q[wrap] : 0.f);
+    }
+  }
+}
+
+// The thread's 16 spectrum values times x.  A spectrum lies in memory as the transform's threads hold it: the values of
+// positions 16u + 2k and 16u + 2k + 1 at float4 k*G + u, so that the lanes of a load read whole lines (in position order
+// every load of a wave would touch 64 of them, and the eight loads together more than the L1 holds).
+template <int LOGN>
+__device__ __forceinline__ void product16(const cpx* __restrict__ sp, const cpx (&x)[16], cpx (&v)[16]) {
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const float4 s = ((const float4*)sp)[k * Half<LOGN>::G];
+    v[2 * k] = cmul(x[2 * k], make_float2(s.x, s.y));
+    v[2 * k + 1] = cmul(x[2 * k + 1], make_float2(s.z, s.w));
+  }
+}
+
+// Inside a loop over filters or channels the twiddles and addresses of a transform are the same every time round; hoisted
+// out of the loop they would not fit the registers.  Passing the table pointer and the thread's index through here keeps
+// their loads and arithmetic where they are used.
+__device__ __forceinline__ const cpx* here(const cpx* p) {
+  asm volatile("" : "+s"(p));
+  return p;
+}
+__device__ __forceinline__ int here(int i) {
+  asm volatile("" : "+v"(i));
+  return i;
+}
+
+// the outputs of pair m from the even-lag result e = E[2m] + i E[2m+1] and the odd-lag results O[2m] = Im[m-1], O[2m+1] = Re[m]
+// (SUM: both branches rounded and added, else the plus branch)
+template <typename T, bool SUM>
+__device__ __forceinline__ float branch_sum(float e, float o) {
+  return SUM ? DT<T>::rnd(e + o) + DT<T>::rnd(e - o) : e + o;
+}
+template <typename T>
+__device__ __forceinline__ float branch_sum(float e, float o, int mode) {
+  return mode == 0 ? branch_sum<T, true>(e, o) : branch_sum<T, false>(e, o);
 }
 
 // ---------------------------------------------------------------- twiddle table
-__global__ void fft_twiddle_kernel(cpx* __restrict__ tw, int n) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= n) return;
+template <int LOGN>
+__global__ void __launch_bounds__(256) fft_twiddle_kernel(cpx* __restrict__ tw) {
+  using W = Half<LOGN>;
+  using B = Table<LOGN>;
+  const int j = blockIdx.x * 256 + threadIdx.x;
+  if (j >= 2 * W::N) return;
+  // entry j: its part, its index there, its power and its angle in turns
+  struct Part { int begin, count, entries, shift; bool fwd; };
+  const Part parts[6] = {{B::INV1, 16, W::MID >= 1 ? 4 : 0, 8, false},
+                         {B::INV2, 256, W::MID >= 2 ? 4 : 0, 12, false},
+                         {B::OUTER, W::Q, B::planes(W::GL), LOGN, false},
+                         {B::FWD2, W::N >> 12, W::MID >= 2 ? 4 : 0, 0, true},
+                         {B::FWD1, W::N >> 8, W::MID >= 1 ? 4 : 0, 0, true},
+                         {B::FWD0, W::N >> 4, 4, 0, true}};
+  double turns = 0.0;
+  for (int q = 0; q < 6; ++q) {
+    const Part& p = parts[q];
+    const int o = j - p.begin;
+    if (p.entries == 0 || o < 0 || o >= p.count * p.entries) continue;
+    int i = o, power = 0;
+    if (p.entries > 1) {
+      i = (o >> 1) % p.count;
+      power = 2 * ((o >> 1) / p.count) + (o & 1);
+    }
+    if (p.fwd) {
+      int lg = 0;
+      while ((1 << lg) < p.count) ++lg;
+      const double f = lg ? (double)(__brev((unsigned)i) >> (32 - lg)) : 0.0;
+      turns = -f * (double)(1 << power) / (double)(p.count * 16);
+    } else {
+      turns = (double)i * (double)(1 << power) / (double)(1 << p.shift);
+    }
+  }
   double s, c;
-  sincospi(-2.0 * (double)j / (double)n, &s, &c);
+  sincospi(2.0 * turns, &s, &c);
   tw[j] = make_float2((float)c, (float)s);
 }
 
+// Columns a workgroup transforms at a time: 512 threads (70 KB of LDS, two workgroups per compute unit) for the long
+// transforms, at most 16 (32 at N = 32) columns for the short ones; a thread may hold 128 registers.
+template <int LOGN> __host__ __device__ constexpr int fft_lcols() { return LOGN >= 13 ? 0 : LOGN == 12 ? 1 : LOGN == 11 ? 2 : LOGN >= 9 ? 3 : LOGN >= 6 ? 4 : 5; }
+template <int LOGN> __host__ __device__ constexpr int fft_threads() { return (1 << (LOGN + fft_lcols<LOGN>())) / 16; }
+template <int LOGN, int NT> __host__ __device__ constexpr size_t fft_lds_bytes() {      // columns, and earlier_im's record
+  return (size_t)(NT / Half<LOGN>::G) * Half<LOGN>::STRIDE * sizeof(cpx) + (size_t)(NT / (Half<LOGN>::G < 64 ? Half<LOGN>::G : 64)) * 32;
+}
+
+// ---------------------------------------------------------------- pairs of positions
+// Two consecutive positions of a channel as they lie in memory when time is contiguous, and staged in LDS.
+template <typename T> struct Pair;
+template <> struct Pair<bf16_t> {
+  typedef unsigned type;
+  typedef unsigned mem __attribute__((aligned(2)));    // at any element's address
+  static __device__ __forceinline__ cpx get(type v) { return make_float2(__uint_as_float(v << 16), __uint_as_float(v & 0xffff0000u)); }
+  static __device__ __forceinline__ type put(float a, float b) { return pack2_bf16(a, b); }
+};
+template <> struct Pair<float> {
+  typedef float type __attribute__((ext_vector_type(2)));
+  typedef float mem __attribute__((ext_vector_type(2), aligned(4)));
+  static __device__ __forceinline__ cpx get(type v) { return make_float2(v[0], v[1]); }
+  static __device__ __forceinline__ type put(float a, float b) { return type{a, b}; }
+};
+
 // ---------------------------------------------------------------- filter spectra
-// Column j of the filter matrix (element (s, j) at filt[s*f_ls + j*f_cs], taps s < taps) -> spec[j*n + p] =
-// (F[p] + i F[p^8]) / n (both branches) or F[p] / n, p running over the digit-reversed positions.
-template <typename T, int LOGN, int NT>
-__global__ void __launch_bounds__(NT)
-fft_filter_kernel(const T* __restrict__ filt, size_t f_ls, size_t f_cs, cpx* __restrict__ spec,
-                  const cpx* __restrict__ tw, int taps, int ncol_total, int lcols, int both) {
+// Column j of the filter matrix (element (s, j) at filt[s*f_ls + j*f_cs], taps s < taps) -> Fe / N in spec[j*n ..] and
+// Fo / N in spec[j*n + N ..], in the order of product16.  One transform of fe + i fo gives both: with G its
+// spectrum, Fe[k] = (G[k] + conj G[-k]) / 2 and Fo[k] = (G[k] - conj G[-k]) / 2i.  Channel-contiguous filters go through
+// LDS so that the lanes of a load run along the channels.
+template <typename T, int LOGN>
+__global__ void __launch_bounds__(fft_threads<LOGN>())
+fft_filter_kernel(const T* __restrict__ filt, size_t f_ls, size_t f_cs, cpx* __restrict__ spec, const cpx* __restrict__ tw,
+                  int taps, int ncol_total) {
   extern __shared__ cpx fft_lds[];
-  constexpr int n = 1 << LOGN, colstride = col_stride<LOGN>();
-  const int cols = 1 << lcols;
-  const int c0 = blockIdx.x * cols;
-  for (int idx = threadIdx.x; idx < (cols << LOGN); idx += NT) {
-    const int colid = idx & (cols - 1), s = idx >> lcols;
-    float v = 0.f;
-    if (s < taps && c0 + colid < ncol_total) v = DT<T>::ld(filt + (size_t)s * f_ls + (size_t)(c0 + colid) * f_cs);
-    fft_lds[(size_t)colid * colstride + phys(s)] = make_float2(v, 0.f);
+  using H = Half<LOGN>;
+  constexpr int N = H::N, LC = fft_lcols<LOGN>(), COLS = 1 << LC, NT = fft_threads<LOGN>();
+  const int c0 = blockIdx.x * COLS;
+  for (int idx = threadIdx.x; idx < COLS * (N / 2); idx += NT) {
+    const int colid = idx & (COLS - 1), m = idx >> LC;
+    const T* f = filt + (size_t)(2 * m) * f_ls + (size_t)(c0 + colid) * f_cs;
+    cpx g = make_float2(0.f, 0.f);
+    if (c0 + colid < ncol_total) {
+      if (2 * m < taps) g.x = DT<T>::ld(f);
+      if (2 * m + 1 < taps) g.y = DT<T>::ld(f + f_ls);
+    }
+    fft_lds[(size_t)colid * H::STRIDE + phys(m)] = g;
   }
   __syncthreads();
-  fft_forward<LOGN, NT, false>(fft_lds, tw, cols);
-  const float inv_n = 1.0f / (float)n;
-  for (int idx = threadIdx.x; idx < (cols << LOGN); idx += NT) {
-    const int colid = idx >> LOGN, p = idx & (n - 1);
-    if (c0 + colid >= ncol_total) continue;
-    const cpx* col = fft_lds + (size_t)colid * colstride;
-    cpx f = col[phys(p)];
-    if (both) {
-      const cpx g = col[phys(p ^ 8)];
-      f = make_float2(f.x - g.y, f.y + g.x);
+  const int colid = threadIdx.x / H::G, u = threadIdx.x % H::G;
+  cpx* col = fft_lds + (size_t)colid * H::STRIDE;
+  cpx z[8], v[16];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) z[k] = col[phys(point<LOGN>(u, k))];
+  __syncthreads();
+  fft_forward<LOGN>(col, tw, u, z, v);
+#pragma unroll
+  for (int m = 0; m < 16; ++m) col[17 * u + m] = v[m];
+  __syncthreads();
+  if (c0 + colid >= ncol_total) return;
+  const float sc = 0.5f / (float)N;
+  float4* out = (float4*)(spec + (size_t)(c0 + colid) * (2 * N)) + u;
+#pragma unroll
+  for (int m = 0; m < 16; m += 2) {
+    cpx h[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const unsigned k = __brev((unsigned)(16 * u + m + i)) >> (32 - LOGN), km = (N - k) & (N - 1);
+      h[i] = col[phys((int)(__brev(km) >> (32 - LOGN)))];
     }
-    spec[(size_t)(c0 + colid) * n + p] = make_float2(f.x * inv_n, f.y * inv_n);
+    out[(m / 2) * H::G] = make_float4((v[m].x + h[0].x) * sc, (v[m].y - h[0].y) * sc, (v[m + 1].x + h[1].x) * sc, (v[m + 1].y - h[1].y) * sc);
+    out[N / 2 + (m / 2) * H::G] = make_float4((v[m].y + h[0].y) * sc, (h[0].x - v[m].x) * sc, (v[m + 1].y + h[1].y) * sc, (h[1].x - v[m + 1].x) * sc);
   }
 }
 
-// ---------------------------------------------------------------- convolution
-// x element (b, t, c) at x[b*x_sb + t*x_st + c*x_sc]; the K outputs of channel c (K = 1: per-channel spectra
-// spec[c]; K > 1: a shared bank spec[k]) go to y[b*y_sb + t*y_st + k*y_sk + c*y_sc] (and y2 likewise).
-// mode 0: y = T(T(re) + T(im));  mode 1: y = T(re);  mode 2: y = T(re), y2 = T(im).
-template <typename T, int LOGN, int NT>
-__global__ void __launch_bounds__(NT)
+// ---------------------------------------------------------------- convolution of time-major slabs, one filter or a bank
+// Positions lie next to each other (the transposed activations of a few long sequences, the U+- slabs of the filter bank):
+// neighbouring threads hold neighbouring pairs, which are read from and written to memory straight from registers.
+// Channel c of x at x[b*x_sb + c*x_sc]; the K outputs of a channel (K = 1: per-channel spectra spec[c]; K > 1: a shared
+// bank spec[k]) at y[b*y_sb + k*y_sk + c*y_sc] (and y2 likewise).
+// mode 0: y = T(T(plus) + T(minus));  mode 1: y = T(plus);  mode 2: y = T(plus), y2 = T(minus).
+// NT threads: as many columns as fill the longest transforms' workgroup or, for small grids, one wave or column.
+template <typename T, int LOGN, int NT, bool SUM>
+__global__ void __launch_bounds__(NT, 4)
+fft_slab_kernel(const T* __restrict__ x, size_t x_sb, size_t x_sc, const cpx* __restrict__ spec, T* __restrict__ y,
+                T* __restrict__ y2, size_t y_sb, size_t y_sk, size_t y_sc, const cpx* __restrict__ tw, int Tn, int d, int K,
+                int xcd_remap) {
+  extern __shared__ cpx fft_lds[];
+  using W = Half<LOGN>;
+  constexpr int N = W::N, COLS = NT / W::G;
+  int bx = blockIdx.x;
+  if (xcd_remap) bx = (bx & 7) * (gridDim.x >> 3) + (bx >> 3);
+  const int b = blockIdx.y, mycol = threadIdx.x / W::G, u = threadIdx.x % W::G, c = bx * COLS + mycol;
+  const bool live = c < d;
+  cpx* col = fft_lds + (size_t)mycol * W::STRIDE;
+  float* rec = (float*)(fft_lds + (size_t)COLS * W::STRIDE);
+  const T* xp = x + (size_t)b * x_sb + (size_t)min(c, d - 1) * x_sc;
+  cpx z[8], xs[16];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const int t = 2 * point<LOGN>(u, k);
+    z[k] = make_float2(0.f, 0.f);
+    if (t + 1 < Tn) z[k] = Pair<T>::get(*(const typename Pair<T>::mem*)(xp + t));
+    else if (t < Tn) z[k].x = DT<T>::ld(xp + t);
+  }
+  fft_forward<LOGN>(col, tw, u, z, xs);
+  const cpx* sp = spec + (K == 1 ? (size_t)min(c, d - 1) * (2 * N) : 0) + 2 * u;
+  T* yp = y + (size_t)b * y_sb + (size_t)c * y_sc;
+  T* yp2 = y2 + (size_t)b * y_sb + (size_t)c * y_sc;
+  for (int k = 0; k < K; ++k, sp += 2 * N, yp += y_sk, yp2 += y_sk) {
+    cpx v[16], e[8], o[8];
+    float prev[8];
+    product16<LOGN>(sp, xs, v);
+    fft_inverse<LOGN>(col, here(tw), here(u), v, e);
+    col_sync<LOGN>();
+    product16<LOGN>(sp + N, xs, v);
+    fft_inverse<LOGN>(col, here(tw), here(u), v, o);
+    earlier_im<LOGN>(o, prev, rec, u);
+    const int uo = here(u), tmax = live ? Tn - 1 : 0;  // pairs t, t + 1 <= tmax are stored
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int t = 2 * point<LOGN>(uo, i);
+      if (t < tmax) *(typename Pair<T>::mem*)(yp + t) = Pair<T>::put(branch_sum<T, SUM>(e[i].x, prev[i]), branch_sum<T, SUM>(e[i].y, o[i].x));
+    }
+    if (!SUM && y2) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int t = 2 * point<LOGN>(uo, i);
+        if (t < tmax) *(typename Pair<T>::mem*)(yp2 + t) = Pair<T>::put(e[i].x - prev[i], e[i].y - o[i].x);
+      }
+    }
+    if (live && (Tn & 1)) {                            // an odd length's last position
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        if (2 * point<LOGN>(uo, i) == Tn - 1) {
+          DT<T>::st(yp + Tn - 1, branch_sum<T, SUM>(e[i].x, prev[i]));
+          if (!SUM && y2) DT<T>::st(yp2 + Tn - 1, e[i].x - prev[i]);
+        }
+    }
+  }
+}
+
+// ---------------------------------------------------------------- any strides
+// The same for operands of any strides: element (b, t, c) of x at x[b*x_sb + t*x_st + c*x_sc], of the k-th output at
+// y[b*y_sb + t*y_st + k*y_sk + c*y_sc].  Pairs pass through the columns' LDS so that the lanes of a memory access run
+// along the channels.
+template <typename T, int LOGN>
+__global__ void __launch_bounds__(fft_threads<LOGN>(), 4)
 fft_conv_kernel(const T* __restrict__ x, size_t x_sb, size_t x_st, size_t x_sc, const cpx* __restrict__ spec,
                 T* __restrict__ y, T* __restrict__ y2, size_t y_sb, size_t y_st, size_t y_sk, size_t y_sc,
-                const cpx* __restrict__ tw, int Tn, int d, int K, int lcols, int mode, int xcd_remap) {
+                const cpx* __restrict__ tw, int Tn, int d, int K, int mode, int xcd_remap) {
   extern __shared__ cpx fft_lds[];
-  constexpr int n = 1 << LOGN, colstride = col_stride<LOGN>();
-  const int cols = 1 << lcols;
+  using W = Half<LOGN>;
+  constexpr int N = W::N, LC = fft_lcols<LOGN>(), COLS = 1 << LC, NT = fft_threads<LOGN>();
   int bx = blockIdx.x;
   if (xcd_remap) bx = (bx & 7) * (gridDim.x >> 3) + (bx >> 3);   // consecutive channel groups share an XCD
-  const int c0 = bx * cols;
-  const int b = blockIdx.y;
-  const int ncol = min(cols, d - c0);
+  const int c0 = bx * COLS, b = blockIdx.y, ncol = min(COLS, d - c0);
+  float* rec = (float*)(fft_lds + (size_t)COLS * W::STRIDE);
   const T* xb = x + (size_t)b * x_sb + (size_t)c0 * x_sc;
-  const bool t_fast = x_st == 1;   // time-major input: walk t with the lanes
-
-  for (int idx = threadIdx.x; idx < (cols << LOGN); idx += NT) {
-    int colid, t;
-    if (t_fast) { colid = idx >> LOGN; t = idx & (n - 1); } else { colid = idx & (cols - 1); t = idx >> lcols; }
-    float v = 0.f;
-    if (t < Tn && colid < ncol) v = DT<T>::ld(xb + (size_t)t * x_st + (size_t)colid * x_sc);
-    fft_lds[(size_t)colid * colstride + phys(t)] = make_float2(v, 0.f);
+  for (int idx = threadIdx.x; idx < COLS * (N / 2); idx += NT) {
+    const int colid = idx & (COLS - 1), m = idx >> LC;
+    cpx z = make_float2(0.f, 0.f);
+    if (colid < ncol) {
+      const T* p = xb + (size_t)(2 * m) * x_st + (size_t)colid * x_sc;
+      if (2 * m < Tn) z.x = DT<T>::ld(p);
+      if (2 * m + 1 < Tn) z.y = DT<T>::ld(p + x_st);
+    }
+    fft_lds[(size_t)colid * W::STRIDE + phys(m)] = z;
   }
   __syncthreads();
-  fft_forward<LOGN, NT, true>(fft_lds, tw, cols);
-
-  const bool yt_fast = y_st == 1;
-  if (K == 1) {
-    fft_middle<LOGN, NT>(fft_lds, spec, c0, ncol);
-    fft_inverse<LOGN, NT, true, true>(fft_lds, tw, cols);   // outputs t < Tn <= n/2 only
-    T* yb = y + (size_t)b * y_sb + (size_t)c0 * y_sc;
-    T* yb2 = (mode == 2) ? y2 + (size_t)b * y_sb + (size_t)c0 * y_sc : nullptr;
-    for (int idx = threadIdx.x; idx < cols * Tn; idx += NT) {
-      int colid, t;
-      if (yt_fast) { colid = idx / Tn; t = idx - colid * Tn; } else { colid = idx & (cols - 1); t = idx >> lcols; }
-      if (colid >= ncol) continue;
-      const cpx z = fft_lds[(size_t)colid * colstride + phys(t)];
-      const size_t o = (size_t)t * y_st + (size_t)colid * y_sc;
-      if (mode == 0) DT<T>::st(yb + o, DT<T>::rnd(z.x) + DT<T>::rnd(z.y));
-      else {
-        DT<T>::st(yb + o, z.x);
-        if (mode == 2) DT<T>::st(yb2 + o, z.y);
-      }
-    }
-    return;
-  }
-
-  // filter bank (one column per workgroup): the thread keeps the spectrum of its groups of 16 neighbouring positions
-  // in registers and runs, per filter, the product and the first inverse pass from them
-  constexpr int NB = ((n >> 4) + NT - 1) / NT;     // groups of 16 per thread
-  cpx xs[NB][16];
+  const int mycol = threadIdx.x / W::G, u = threadIdx.x % W::G;
+  cpx* col = fft_lds + (size_t)mycol * W::STRIDE;
+  cpx z[8], xs[16];
 #pragma unroll
-  for (int i = 0; i < NB; ++i) {
-    const int u = threadIdx.x + i * NT;
-    if (u < (n >> 4)) forward16(fft_lds + 17 * u, xs[i]);
-  }
+  for (int k = 0; k < 8; ++k) z[k] = col[phys(point<LOGN>(u, k))];
   __syncthreads();
-  for (int k = 0; k < K; ++k) {
+  fft_forward<LOGN>(col, tw, u, z, xs);
+  const cpx* sp = spec + (K == 1 ? (size_t)min(c0 + mycol, d - 1) * (2 * N) : 0) + 2 * u;
+  for (int k = 0; k < K; ++k, sp += 2 * N) {
+    cpx v[16], e[8], o[8];
+    float prev[8];
+    product16<LOGN>(sp, xs, v);
+    fft_inverse<LOGN>(col, here(tw), here(u), v, e);
+    col_sync<LOGN>();
+    product16<LOGN>(sp + N, xs, v);
+    fft_inverse<LOGN>(col, here(tw), here(u), v, o);
+    earlier_im<LOGN>(o, prev, rec, u);
+    for (int br = 0; br < (mode == 2 ? 2 : 1); ++br) {
+      __syncthreads();
 #pragma unroll
-    for (int i = 0; i < NB; ++i) {
-      const int u = threadIdx.x + i * NT;
-      if (u < (n >> 4)) {
-        cpx s[16];
-        load_spec16(spec + ((size_t)k << LOGN) + 16 * u, s);
-        product_inverse16(fft_lds + 17 * u, xs[i], s);
-      }
-    }
-    __syncthreads();
-    fft_inverse<LOGN, NT, true, true>(fft_lds, tw, 1);      // outputs t < Tn <= n/2 only
-    T* yb = y + (size_t)b * y_sb + (size_t)c0 * y_sc + (size_t)k * y_sk;
-    T* yb2 = (mode == 2) ? y2 + (size_t)b * y_sb + (size_t)c0 * y_sc + (size_t)k * y_sk : nullptr;
-    for (int t = threadIdx.x; t < Tn; t += NT) {
-      const cpx z = fft_lds[phys(t)];
-      const size_t o = (size_t)t * y_st;
-      if (mode == 0) DT<T>::st(yb + o, DT<T>::rnd(z.x) + DT<T>::rnd(z.y));
-      else {
-        DT<T>::st(yb + o, z.x);
-        if (mode == 2) DT<T>::st(yb2 + o, z.y);
+      for (int i = 0; i < 8; ++i)
+        col[phys(point<LOGN>(here(u), i))] = br ? make_float2(e[i].x - prev[i], e[i].y - o[i].x)
+                                               : make_float2(branch_sum<T>(e[i].x, prev[i], mode), branch_sum<T>(e[i].y, o[i].x, mode));
+      __syncthreads();
+      T* yb = (br ? y2 : y) + (size_t)b * y_sb + (size_t)k * y_sk + (size_t)c0 * y_sc;
+      for (int idx = threadIdx.x; idx < COLS * (N / 2); idx += NT) {
+        const int colid = idx & (COLS - 1), m = idx >> LC;
+        if (colid >= ncol || 2 * m >= Tn) continue;
+        const cpx r = fft_lds[(size_t)colid * W::STRIDE + phys(m)];
+        T* q = yb + (size_t)(2 * m) * y_st + (size_t)colid * y_sc;
+        DT<T>::st(q, r.x);
+        if (2 * m + 1 < Tn) DT<T>::st(q + y_st, r.y);
       }
     }
     __syncthreads();
   }
 }
 
-// ---------------------------------------------------------------- convolution, whole 16-byte row pieces per lane
-// The same computation for channel-contiguous (B, T, d) operands with d a multiple of the workgroup's channel count:
-// a workgroup owns CHW = max(COLS, 16 bytes' worth) neighbouring channels, reads them as 16-byte pieces of the rows
-// (all loads in flight at once, kept in registers), transforms COLS of them at a time in LDS, collects the results in
-// registers and writes 16-byte pieces of the output rows.  Global accesses are 8 (bf16) or 4 (fp32) channels wide
-// instead of COLS; for the long transforms (COLS = 1) that is the difference between 2-byte and 16-byte accesses.
+// ---------------------------------------------------------------- whole 16-byte row pieces per lane
+// The same for channel-contiguous (B, T, d) operands with d a multiple of the workgroup's channel count: a workgroup owns
+// CHW = max(COLS, 16 bytes' worth) neighbouring channels, reads pairs of rows as 16-byte pieces (all loads in flight at
+// once, kept in registers), passes the pairs of COLS channels at a time through LDS to the threads of their transforms and
+// the finished pairs back, and writes 16-byte pieces of the output rows.  A group takes the first COLS channels of the
+// pieces and puts its results behind the last ones, so the loop over the groups is one copy of the code and every index
+// into the registers is a constant.
 template <typename T> struct RowVec;
 template <> struct RowVec<bf16_t> {
   static constexpr int CH = 8;
-  template <int E> static __device__ __forceinline__ float get(const unsigned (&w)[4]) {
-    return __uint_as_float((E & 1) ? (w[E >> 1] & 0xffff0000u) : (w[E >> 1] << 16));
+  // channel e of two consecutive rows
+  static __device__ __forceinline__ unsigned pair(const unsigned (&a)[4], const unsigned (&b)[4], int e) {
+    return (e & 1) ? __builtin_amdgcn_perm(b[e >> 1], a[e >> 1], 0x07060302) : __builtin_amdgcn_perm(b[e >> 1], a[e >> 1], 0x05040100);
   }
-  template <int E> static __device__ __forceinline__ void put(unsigned (&w)[4], float v) {
-    const unsigned h = f32_to_bf16(v);
-    w[E >> 1] = (E & 1) ? ((w[E >> 1] & 0x0000ffffu) | (h << 16)) : ((w[E >> 1] & 0xffff0000u) | h);
+  // the pairs r[0..NE) of the first NE channels go behind the others
+  template <int NE> static __device__ __forceinline__ void rotate_in(unsigned (&a)[4], unsigned (&b)[4], const unsigned (&r)[NE]) {
+    if constexpr (NE == 1) {
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        a[i] = __builtin_amdgcn_alignbit(a[i + 1], a[i], 16);
+        b[i] = __builtin_amdgcn_alignbit(b[i + 1], b[i], 16);
+      }
+      a[3] = __builtin_amdgcn_alignbit(r[0], a[3], 16);
+      b[3] = __builtin_amdgcn_alignbit(r[0] >> 16, b[3], 16);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4 - NE / 2; ++i) { a[i] = a[i + NE / 2]; b[i] = b[i + NE / 2]; }
+#pragma unroll
+      for (int i = 0; i < NE / 2; ++i) {
+        a[4 - NE / 2 + i] = __builtin_amdgcn_perm(r[2 * i + 1], r[2 * i], 0x05040100);
+        b[4 - NE / 2 + i] = __builtin_amdgcn_perm(r[2 * i + 1], r[2 * i], 0x07060302);
+      }
+    }
   }
+  static __device__ __forceinline__ unsigned cut(unsigned p, bool first, bool second) { return (first ? p & 0xffffu : 0u) | (second ? p & 0xffff0000u : 0u); }
 };
 template <> struct RowVec<float> {
   static constexpr int CH = 4;
-  template <int E> static __device__ __forceinline__ float get(const unsigned (&w)[4]) { return __uint_as_float(w[E]); }
-  template <int E> static __device__ __forceinline__ void put(unsigned (&w)[4], float v) { w[E] = __float_as_uint(v); }
+  typedef Pair<float>::type pair_t;
+  static __device__ __forceinline__ pair_t pair(const unsigned (&a)[4], const unsigned (&b)[4], int e) { return pair_t{__uint_as_float(a[e]), __uint_as_float(b[e])}; }
+  template <int NE> static __device__ __forceinline__ void rotate_in(unsigned (&a)[4], unsigned (&b)[4], const pair_t (&r)[NE]) {
+#pragma unroll
+    for (int i = 0; i < 4 - NE; ++i) { a[i] = a[i + NE]; b[i] = b[i + NE]; }
+#pragma unroll
+    for (int i = 0; i < NE; ++i) { a[4 - NE + i] = __float_as_uint(r[i][0]); b[4 - NE + i] = __float_as_uint(r[i][1]); }
+  }
+  static __device__ __forceinline__ pair_t cut(pair_t p, bool first, bool second) { return pair_t{first ? p[0] : 0.f, second ? p[1] : 0.f}; }
 };
 
-// columns in LDS at a time: as many as 34 KB hold (at most 16); n = 4096 takes two with twice the threads (measured
-// 14 % faster than one), n = 8192 one (two with 1024 threads spill registers and were 12 % slower)
-template <int LOGN> __host__ __device__ constexpr int fft_lcols() { return LOGN >= 13 ? 0 : LOGN == 12 ? 1 : (12 - LOGN > 4 ? 4 : 12 - LOGN); }
+template <typename T, int LOGN> struct RowCut {
+  static constexpr int COLS = 1 << fft_lcols<LOGN>(), CH = RowVec<T>::CH, CHW = COLS > CH ? COLS : CH;
+  static constexpr int VR = CHW / CH, NG = CHW / COLS, NE = COLS < CH ? COLS : CH;   // pieces per row, groups, channels per piece and group
+  static constexpr int NT = fft_threads<LOGN>(), NV = (Half<LOGN>::N / 2) * VR / NT;
+};
 
-// R2: the radix-2 first pass of the forward transform happens here.  Its butterfly pairs sample t with the zero at
-// t + n/2, so position t keeps x and position t + n/2 receives x * w^t (wt = tw[t]): the same values the pass would
-// leave, without its trip through LDS and its barrier.
-template <typename T, int LOGN, int NT, int G, int E, bool R2 = false>
-__device__ __forceinline__ void rows_scatter(cpx* lds, const unsigned (&w)[4], int t, int part, cpx wt = make_float2(1.f, 0.f)) {
-  constexpr int COLS = 1 << fft_lcols<LOGN>(), CH = RowVec<T>::CH, VR = (COLS > CH ? COLS : CH) / CH;
-  constexpr int n = 1 << LOGN;
-  if constexpr (E < CH) {
-    // VR == 1: the column is known at compile time; VR > 1 (one group): it follows the row piece
-    constexpr int col_ct = E - G * COLS;
-    if constexpr (VR > 1 || (col_ct >= 0 && col_ct < COLS)) {
-      const int col = VR > 1 ? part * CH + E : col_ct;
-      const float xv = RowVec<T>::template get<E>(w);
-      cpx* c = lds + (size_t)col * col_stride<LOGN>();
-      c[phys(t)] = make_float2(xv, 0.f);
-      if constexpr (R2) c[phys(t + n / 2)] = make_float2(xv * wt.x, xv * wt.y);
-    }
-    rows_scatter<T, LOGN, NT, G, E + 1, R2>(lds, w, t, part, wt);
-  }
-}
-
-// R2: the radix-2 last pass of the inverse transform happens here, for the wanted lower half only:
-// y[t] = u[t] + u[t + n/2] * conj(w^t).
-template <typename T, int LOGN, int NT, int G, int E, bool R2 = false>
-__device__ __forceinline__ void rows_gather(const cpx* lds, unsigned (&w)[4], int t, int part, int mode, cpx wt = make_float2(1.f, 0.f)) {
-  constexpr int COLS = 1 << fft_lcols<LOGN>(), CH = RowVec<T>::CH, VR = (COLS > CH ? COLS : CH) / CH;
-  constexpr int n = 1 << LOGN;
-  if constexpr (E < CH) {
-    constexpr int col_ct = E - G * COLS;
-    if constexpr (VR > 1 || (col_ct >= 0 && col_ct < COLS)) {
-      const int col = VR > 1 ? part * CH + E : col_ct;
-      const cpx* c = lds + (size_t)col * col_stride<LOGN>();
-      cpx z = c[phys(t)];
-      if constexpr (R2) z = cadd(z, cmulc(c[phys(t + n / 2)], wt));
-      RowVec<T>::template put<E>(w, mode == 0 ? DT<T>::rnd(z.x) + DT<T>::rnd(z.y) : z.x);
-    }
-    rows_gather<T, LOGN, NT, G, E + 1, R2>(lds, w, t, part, mode, wt);
-  }
-}
-
-template <typename T, int LOGN, int NT, int NV, int G>
-__device__ __forceinline__ void rows_groups(cpx* lds, const cpx* __restrict__ spec, const cpx* __restrict__ tw,
-                                            unsigned (&io)[NV][4], int Tn, int c0, int mode) {
-  constexpr int n = 1 << LOGN, COLS = 1 << fft_lcols<LOGN>(), CH = RowVec<T>::CH, CHW = COLS > CH ? COLS : CH;
-  constexpr int VR = CHW / CH, NG = CHW / COLS;
-  if constexpr (G < NG) {
-    if (G > 0) __syncthreads();   // the previous group's results have been collected
-    constexpr bool R2 = (LOGN & 3) == 1;   // the radix-2 pass of these lengths rides on the scatter and the gather
-#pragma unroll
-    for (int r = 0; r < NV; ++r) {
-      const int q = threadIdx.x + r * NT, t = q / VR, part = q % VR;
-      if (t < Tn) {
-        if constexpr (R2) rows_scatter<T, LOGN, NT, G, 0, true>(lds, io[r], t, part, tw[t]);
-        else rows_scatter<T, LOGN, NT, G, 0>(lds, io[r], t, part);
-      }
-    }
-    // zero padding behind the sequence, up to half the column: the first forward pass knows that the upper half of a
-    // column is zero and the inputs real and reads neither, the last inverse pass produces the lower half only.
-    // (At 512 and 8192 points those passes have radix 2: they are not run at all, the scatter above and the gather
-    // below do their work on the way.)
-    constexpr bool HF = !R2, HI = !R2;
-    constexpr int pad_to = n / 2;
-    for (int idx = threadIdx.x; idx < COLS * (pad_to - Tn); idx += NT) {
-      const int col = idx / (pad_to - Tn), t = Tn + idx - col * (pad_to - Tn);
-      cpx* c = lds + (size_t)col * col_stride<LOGN>();
-      c[phys(t)] = make_float2(0.f, 0.f);
-      if constexpr (R2) c[phys(t + n / 2)] = make_float2(0.f, 0.f);   // what the radix-2 pass makes of a zero pair
-    }
-    __syncthreads();
-    fft_forward<LOGN, NT, true, HF, R2>(lds, tw, COLS);
-    fft_middle<LOGN, NT>(lds, spec, c0 + G * COLS, COLS);
-    fft_inverse<LOGN, NT, true, HI, R2>(lds, tw, COLS);
-#pragma unroll
-    for (int r = 0; r < NV; ++r) {
-      const int q = threadIdx.x + r * NT, t = q / VR, part = q % VR;
-      if (t < Tn) {                                   // over the inputs this group consumed
-        if constexpr (R2) rows_gather<T, LOGN, NT, G, 0, true>(lds, io[r], t, part, mode, tw[t]);
-        else rows_gather<T, LOGN, NT, G, 0>(lds, io[r], t, part, mode);
-      }
-    }
-    rows_groups<T, LOGN, NT, NV, G + 1>(lds, spec, tw, io, Tn, c0, mode);
-  }
-}
-
-// (8192 points: two workgroups of 512 threads share a compute unit, 70 KB of LDS each, so a thread may hold 128 registers)
-template <typename T, int LOGN, int NT>
-__global__ void __launch_bounds__(NT, LOGN == 13 ? 4 : 1)
+template <typename T, int LOGN>
+__global__ void __launch_bounds__(fft_threads<LOGN>(), LOGN == 13 ? 2 : 4)
 fft_conv_rows_kernel(const T* __restrict__ x, size_t x_sb, size_t x_st, const cpx* __restrict__ spec, T* __restrict__ y,
                      size_t y_sb, size_t y_st, const cpx* __restrict__ tw, int Tn, int mode, int xcd_remap) {
   extern __shared__ cpx fft_lds[];
-  constexpr int n = 1 << LOGN, COLS = 1 << fft_lcols<LOGN>(), CH = RowVec<T>::CH, CHW = COLS > CH ? COLS : CH;
-  constexpr int VR = CHW / CH, NV = ((n / 2) * VR + NT - 1) / NT;
+  using W = Half<LOGN>;
+  using R = RowCut<T, LOGN>;
+  typedef typename Pair<T>::type pair_t;
+  constexpr int N = W::N, COLS = R::COLS, CH = R::CH, CHW = R::CHW, VR = R::VR, NV = R::NV, NE = R::NE, NT = R::NT;
+  constexpr int PST = N / 2 + 1;                       // staged pairs of a column (odd: neighbouring channels in different banks)
+  static_assert(NV * NT == (N / 2) * VR && (size_t)PST * sizeof(pair_t) <= (size_t)W::STRIDE * sizeof(cpx), "whole pairs per thread");
   int bx = blockIdx.x;
   if (xcd_remap) bx = (bx & 7) * (gridDim.x >> 3) + (bx >> 3);   // consecutive channel groups share an XCD
   const int c0 = bx * CHW, b = blockIdx.y;
   const T* xb = x + (size_t)b * x_sb + c0;
-  // the row pieces: inputs at first, each channel's result written over its input once its group is through
-  unsigned io[NV][4];
+  unsigned io[NV][2][4];
 #pragma unroll
   for (int r = 0; r < NV; ++r) {
-    const int q = threadIdx.x + r * NT, t = q / VR, part = q % VR;
-    // rows behind the sequence re-read its last row (no branch around the load) and are never used
-    const uint4 v = *(const uint4*)(xb + (size_t)min(t, Tn - 1) * x_st + part * CH);
-    io[r][0] = v.x; io[r][1] = v.y; io[r][2] = v.z; io[r][3] = v.w;
+    const int q = threadIdx.x + r * NT, m = q / VR, part = q % VR;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      // rows behind the sequence re-read its last row (no branch around the load) and are replaced by zeros below
+      const uint4 v = *(const uint4*)(xb + (size_t)min(2 * m + h, Tn - 1) * x_st + part * CH);
+      io[r][h][0] = v.x; io[r][h][1] = v.y; io[r][h][2] = v.z; io[r][h][3] = v.w;
+    }
   }
-  rows_groups<T, LOGN, NT, NV, 0>(fft_lds, spec, tw, io, Tn, c0, mode);
+  const int mycol = threadIdx.x / W::G, u = threadIdx.x % W::G;
+  cpx* col = fft_lds + (size_t)mycol * W::STRIDE;
+  float* rec = (float*)(fft_lds + (size_t)COLS * W::STRIDE);
+  pair_t* stage = (pair_t*)fft_lds;                    // [column][pair], in the columns' place
+  const cpx* sp = spec + (size_t)(c0 + mycol) * (2 * N) + 2 * u;
+  for (int g = 0; g < R::NG; ++g, sp += (size_t)COLS * (2 * N)) {
+    if (g > 0) __syncthreads();                        // the previous group's results have been collected
+    const int tid = here((int)threadIdx.x), ug = here(u);
+    const cpx* twg = here(tw);
+#pragma unroll
+    for (int r = 0; r < NV; ++r) {
+      const int q = tid + r * NT, m = q / VR, part = q % VR;
+#pragma unroll
+      for (int e = 0; e < NE; ++e)
+        stage[(VR > 1 ? part * CH + e : e) * PST + m] = RowVec<T>::cut(RowVec<T>::pair(io[r][0], io[r][1], e), 2 * m < Tn, 2 * m + 1 < Tn);
+    }
+    __syncthreads();
+    cpx xs[16], v[16], e[8], o[8];
+    float prev[8];
+    {
+      cpx z[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) z[k] = Pair<T>::get(stage[mycol * PST + point<LOGN>(ug, k)]);
+      __syncthreads();
+      fft_forward<LOGN>(col, twg, ug, z, xs);
+    }
+    product16<LOGN>(sp, xs, v);
+    fft_inverse<LOGN>(col, here(tw), ug, v, e);
+    col_sync<LOGN>();
+    product16<LOGN>(sp + N, xs, v);
+    fft_inverse<LOGN>(col, here(tw), ug, v, o);
+    earlier_im<LOGN>(o, prev, rec, ug);
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      stage[mycol * PST + point<LOGN>(ug, i)] = Pair<T>::put(branch_sum<T>(e[i].x, prev[i], mode), branch_sum<T>(e[i].y, o[i].x, mode));
+    __syncthreads();
+    const int tid_o = here((int)threadIdx.x);
+#pragma unroll
+    for (int r = 0; r < NV; ++r) {
+      const int q = tid_o + r * NT, m = q / VR, part = q % VR;
+      pair_t p[NE];
+#pragma unroll
+      for (int k = 0; k < NE; ++k) p[k] = stage[(VR > 1 ? part * CH + k : k) * PST + m];
+      RowVec<T>::template rotate_in<NE>(io[r][0], io[r][1], p);
+    }
+  }
   T* yb = y + (size_t)b * y_sb + c0;
 #pragma unroll
   for (int r = 0; r < NV; ++r) {
-    const int q = threadIdx.x + r * NT, t = q / VR, part = q % VR;
-    if (t < Tn) *(uint4*)(yb + (size_t)t * y_st + part * CH) = make_uint4(io[r][0], io[r][1], io[r][2], io[r][3]);
+    const int q = threadIdx.x + r * NT, m = q / VR, part = q % VR;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      if (2 * m + h < Tn)
+        *(uint4*)(yb + (size_t)(2 * m + h) * y_st + part * CH) = make_uint4(io[r][h][0], io[r][h][1], io[r][h][2], io[r][h][3]);
   }
 }
 
@@ -551,18 +737,6 @@ int ilog2_exact(int n) {
   while ((1 << l) < n) ++l;
   return ((1 << l) == n) ? l : -1;
 }
-
-// columns per workgroup and threads per workgroup for a transform length
-void fft_shape(int logn, int ncol_total, int* lcols, int* nt) {
-  int lc = 12 - logn;           // cols * n = 4096 complex elements = 34 KB of LDS
-  if (lc < 0) lc = 0;
-  if (lc > 4) lc = 4;
-  while (lc > 0 && (1 << lc) > ncol_total) --lc;
-  *lcols = lc;
-  *nt = (logn >= 14) ? 1024 : (logn == 13 ? 512 : 256);
-}
-
-size_t fft_lds_bytes(int n, int lcols) { return (size_t)(n + (n >> 4)) * sizeof(cpx) << lcols; }
 
 template <typename K> int allow_lds(K kernel, size_t bytes, const char* name) {
   if (bytes <= 48 * 1024) return 0;
@@ -575,6 +749,8 @@ template <typename K> int allow_lds(K kernel, size_t bytes, const char* name) {
   return 0;
 }
 
+int fft_cols(int half_logn) { return half_logn >= 13 ? 1 : half_logn == 12 ? 2 : half_logn == 11 ? 4 : half_logn >= 9 ? 8 : half_logn >= 6 ? 16 : 32; }
+
 }  // namespace
 
 extern "C" int fstu_fft_length(int T_) {
@@ -583,56 +759,57 @@ extern "C" int fstu_fft_length(int T_) {
   return (n >= 2 * T_) ? n : 0;
 }
 
+// KERNEL: one of the launchers below, given LOGN of the half-length transform
+#define FFT_GO(KERNEL, THREADS, SHM, GRID, NAME, ...)                                                  \
+  do {                                                                                                 \
+    static int rc__ = allow_lds(KERNEL, SHM, NAME);                                                    \
+    if (rc__) return rc__;                                                                             \
+    hipLaunchKernelGGL(KERNEL, GRID, dim3(THREADS), SHM, (hipStream_t)stream, __VA_ARGS__);            \
+  } while (0)
+#define FFT_TABLE(L, GRID, NAME, ...) FFT_GO((fft_twiddle_kernel<L>), 256, 0, GRID, NAME, __VA_ARGS__)
+#define FFT_FILTER(L, GRID, NAME, ...) \
+  FFT_GO((fft_filter_kernel<T, L>), fft_threads<L>(), (fft_lds_bytes<L, fft_threads<L>()>()), GRID, NAME, __VA_ARGS__)
+#define FFT_PLAIN(L, GRID, NAME, ...) \
+  FFT_GO((fft_conv_kernel<T, L>), fft_threads<L>(), (fft_lds_bytes<L, fft_threads<L>()>()), GRID, NAME, __VA_ARGS__)
+#define FFT_ROWS(L, GRID, NAME, ...) \
+  FFT_GO((fft_conv_rows_kernel<T, L>), fft_threads<L>(), (fft_lds_bytes<L, fft_threads<L>()>()), GRID, NAME, __VA_ARGS__)
+#define FFT_SLAB(L, GRID, NAME, ...)                                                                                        \
+  do {                                                                                                                      \
+    constexpr int few__ = Half<L>::G > 64 ? Half<L>::G : 64;                                                                \
+    if (narrow && mode == 0)                                                                                                \
+      FFT_GO((fft_slab_kernel<T, L, few__, true>), few__, (fft_lds_bytes<L, few__>()), GRID, NAME, __VA_ARGS__);            \
+    else if (narrow)                                                                                                        \
+      FFT_GO((fft_slab_kernel<T, L, few__, false>), few__, (fft_lds_bytes<L, few__>()), GRID, NAME, __VA_ARGS__);           \
+    else if (mode == 0)                                                                                                     \
+      FFT_GO((fft_slab_kernel<T, L, 512, true>), 512, (fft_lds_bytes<L, 512>()), GRID, NAME, __VA_ARGS__);                  \
+    else                                                                                                                    \
+      FFT_GO((fft_slab_kernel<T, L, 512, false>), 512, (fft_lds_bytes<L, 512>()), GRID, NAME, __VA_ARGS__);                 \
+  } while (0)
+
+#define FFT_LAUNCH(LOGN, KERNEL, GRID, NAME, ...)             \
+  do {                                                        \
+    switch (LOGN) {                                           \
+      case 5: KERNEL(5, GRID, NAME, __VA_ARGS__); break;      \
+      case 6: KERNEL(6, GRID, NAME, __VA_ARGS__); break;      \
+      case 7: KERNEL(7, GRID, NAME, __VA_ARGS__); break;      \
+      case 8: KERNEL(8, GRID, NAME, __VA_ARGS__); break;      \
+      case 9: KERNEL(9, GRID, NAME, __VA_ARGS__); break;      \
+      case 10: KERNEL(10, GRID, NAME, __VA_ARGS__); break;    \
+      case 11: KERNEL(11, GRID, NAME, __VA_ARGS__); break;    \
+      case 12: KERNEL(12, GRID, NAME, __VA_ARGS__); break;    \
+      default: KERNEL(13, GRID, NAME, __VA_ARGS__); break;    \
+    }                                                         \
+  } while (0)
+
 extern "C" int fstu_fft_twiddles(float* tw, int n, void* stream) {
   FSTU_REQUIRE(tw, FSTU_ENULL, "fstu_fft_twiddles: null pointer");
   const int logn = ilog2_exact(n);
   FSTU_REQUIRE(logn >= 6 && logn <= 14, FSTU_ESHAPE, "fstu_fft_twiddles: n=%d is not a power of two in 64..16384", n);
-  hipLaunchKernelGGL(fft_twiddle_kernel, dim3((n + 255) / 256), dim3(256), 0, (hipStream_t)stream, (cpx*)tw, n);
+  FSTU_REQUIRE(fstu_aligned(tw, 16), FSTU_EALIGN, "fstu_fft_twiddles: tw must be 16-byte aligned");
+  FFT_LAUNCH(logn - 1, FFT_TABLE, dim3((n + 255) / 256), "fstu_fft_twiddles", (cpx*)tw);
   FSTU_CHECK_LAUNCH("fstu_fft_twiddles");
   return FSTU_OK;
 }
-
-// threads per workgroup follow the transform length: one radix-16 butterfly per thread and pass for n = 4096 and
-// 8192, two at 16384 (1024 threads leave 128 registers each, which the bank form's resident spectrum overflows)
-#ifndef FFT_NT14
-#define FFT_NT14 512
-#endif
-#define FFT_LAUNCH_ONE(LOGNV, NTV, KERNEL, GRID, SHM, NAME, ...)                                              \
-  do {                                                                                                        \
-    int rc__ = allow_lds(KERNEL<T, LOGNV, NTV>, SHM, NAME);                                                   \
-    if (rc__) return rc__;                                                                                    \
-    hipLaunchKernelGGL((KERNEL<T, LOGNV, NTV>), GRID, dim3(NTV), SHM, (hipStream_t)stream, __VA_ARGS__);      \
-  } while (0)
-
-#define FFT_LAUNCH(LOGN, KERNEL, GRID, SHM, NAME, ...)                                  \
-  do {                                                                                  \
-    switch (LOGN) {                                                                     \
-      case 6: FFT_LAUNCH_ONE(6, 256, KERNEL, GRID, SHM, NAME, __VA_ARGS__); break;      \
-      case 7: FFT_LAUNCH_ONE(7, 256, KERNEL, GRID, SHM, NAME, __VA_ARGS__); break;      \
-      case 8: FFT_LAUNCH_ONE(8, 256, KERNEL, GRID, SHM, NAME, __VA_ARGS__); break;      \
-      case 9: FFT_LAUNCH_ONE(9, 256, KERNEL, GRID, SHM, NAME, __VA_ARGS__); break;      \
-      case 10: FFT_LAUNCH_ONE(10, 256, KERNEL, GRID, SHM, NAME, __VA_ARGS__); break;    \
-      case 11: FFT_LAUNCH_ONE(11, 256, KERNEL, GRID, SHM, NAME, __VA_ARGS__); break;    \
-      case 12: FFT_LAUNCH_ONE(12, 256, KERNEL, GRID, SHM, NAME, __VA_ARGS__); break;    \
-      case 13: FFT_LAUNCH_ONE(13, 512, KERNEL, GRID, SHM, NAME, __VA_ARGS__); break;    \
-      default: FFT_LAUNCH_ONE(14, FFT_NT14, KERNEL, GRID, SHM, NAME, __VA_ARGS__); break;   \
-    }                                                                                   \
-  } while (0)
-
-#define FFT_LAUNCH_ROWS(LOGN, KERNEL, GRID, SHM, NAME, ...)                              \
-  do {                                                                                  \
-    switch (LOGN) {                                                                     \
-      case 6: FFT_LAUNCH_ONE(6, 256, KERNEL, GRID, SHM, NAME, __VA_ARGS__); break;      \
-      case 7: FFT_LAUNCH_ONE(7, 256, KERNEL, GRID, SHM, NAME, __VA_ARGS__); break;      \
-      case 8: FFT_LAUNCH_ONE(8, 256, KERNEL, GRID, SHM, NAME, __VA_ARGS__); break;      \
-      case 9: FFT_LAUNCH_ONE(9, 256, KERNEL, GRID, SHM, NAME, __VA_ARGS__); break;      \
-      case 10: FFT_LAUNCH_ONE(10, 256, KERNEL, GRID, SHM, NAME, __VA_ARGS__); break;    \
-      case 11: FFT_LAUNCH_ONE(11, 256, KERNEL, GRID, SHM, NAME, __VA_ARGS__); break;    \
-      case 12: FFT_LAUNCH_ONE(12, 512, KERNEL, GRID, SHM, NAME, __VA_ARGS__); break;    \
-      case 13: FFT_LAUNCH_ONE(13, 512, KERNEL, GRID, SHM, NAME, __VA_ARGS__); break;    \
-      default: FFT_LAUNCH_ONE(14, 512, KERNEL, GRID, SHM, NAME, __VA_ARGS__); break;    \
-    }                                                                                   \
-  } while (0)
 
 extern "C" int fstu_stu_fft_filter(const void* filt, int64_t f_ls, int64_t f_cs, float* spec, const float* tw, int taps,
                                    int ncols, int n, int single_branch, int dtype, void* stream) {
@@ -641,14 +818,13 @@ extern "C" int fstu_stu_fft_filter(const void* filt, int64_t f_ls, int64_t f_cs,
   FSTU_REQUIRE(logn >= 6 && logn <= 14, FSTU_ESHAPE, "fstu_stu_fft_filter: n=%d is not a power of two in 64..16384", n);
   FSTU_REQUIRE(taps >= 1 && 2 * taps <= n && ncols >= 1, FSTU_ESHAPE,
                "fstu_stu_fft_filter: taps=%d must satisfy 1 <= taps <= n/2=%d (ncols=%d)", taps, n / 2, ncols);
-  FSTU_REQUIRE(fstu_aligned(spec, 8) && fstu_aligned(tw, 8), FSTU_EALIGN, "fstu_stu_fft_filter: spec/tw must be 8-byte aligned");
-  int lcols, nt;
-  fft_shape(logn, ncols, &lcols, &nt);
-  const size_t shm = fft_lds_bytes(n, lcols);
-  dim3 grid((ncols + (1 << lcols) - 1) >> lcols);
+  FSTU_REQUIRE(fstu_aligned(spec, 16) && fstu_aligned(tw, 16), FSTU_EALIGN, "fstu_stu_fft_filter: spec and tw must be 16-byte aligned");
+  (void)single_branch;      // both parts of the spectrum serve both forms of the convolution
+  const int cols = fft_cols(logn - 1);
+  dim3 grid((ncols + cols - 1) / cols);
   FSTU_DISPATCH_DTYPE(dtype, "fstu_stu_fft_filter",
-                      FFT_LAUNCH(logn, fft_filter_kernel, grid, shm, "fstu_stu_fft_filter", (const T*)filt, (size_t)f_ls,
-                                 (size_t)f_cs, (cpx*)spec, (const cpx*)tw, taps, ncols, lcols, single_branch ? 0 : 1));
+                      FFT_LAUNCH(logn - 1, FFT_FILTER, grid, "fstu_stu_fft_filter", (const T*)filt, (size_t)f_ls,
+                                 (size_t)f_cs, (cpx*)spec, (const cpx*)tw, taps, ncols));
   FSTU_CHECK_LAUNCH("fstu_stu_fft_filter");
   return FSTU_OK;
 }
@@ -660,40 +836,44 @@ static int conv_fft_launch(const char* name, const void* x, int64_t x_sb, int64_
   FSTU_REQUIRE(logn >= 6 && logn <= 14, FSTU_ESHAPE, "%s: n=%d is not a power of two in 64..16384", name, n);
   FSTU_REQUIRE(B >= 1 && B <= 65535 && T_ >= 1 && d >= 1 && K >= 1 && 2 * T_ <= n, FSTU_ESHAPE,
                "%s: bad shape B=%d T=%d d=%d K=%d n=%d (n >= 2T required)", name, B, T_, d, K, n);
-  FSTU_REQUIRE(fstu_aligned(spec, 8) && fstu_aligned(tw, 8), FSTU_EALIGN, "%s: spec/tw must be 8-byte aligned", name);
-  int lcols, nt;
-  fft_shape(logn, d, &lcols, &nt);
-  if (K > 1) lcols = 0;
-  {
-    // channel-contiguous operands whose rows split into whole 16-byte pieces per workgroup: the row-piece kernel
-    const int rows_lcols = logn >= 13 ? 0 : logn == 12 ? 1 : (12 - logn > 4 ? 4 : 12 - logn);
-    const int esz = dtype == FSTU_BF16 ? 2 : 4, ch = 16 / esz, cols_full = 1 << rows_lcols;
-    const int chw = cols_full > ch ? cols_full : ch;
-    // (the long transforms take a workgroup's channels one after the other: with fewer than two workgroups per compute
-    // unit the one-column kernel, eight times the workgroups, is the faster one)
-    const bool enough = logn < 13 || (long long)(d / chw) * B >= 512;
-    if (K == 1 && mode != 2 && enough && x_sc == 1 && y_sc == 1 && d % chw == 0 && x_st % ch == 0 && y_st % ch == 0 &&
-        x_sb % ch == 0 && y_sb % ch == 0 && fstu_aligned(x, 16) && fstu_aligned(y, 16)) {
-      const size_t shm = fft_lds_bytes(n, rows_lcols);
-      const int gx = d / chw;
-      dim3 grid(gx, B);
-      const int remap = (gx % 8 == 0) ? 1 : 0;
-      FSTU_DISPATCH_DTYPE(dtype, name,
-                          FFT_LAUNCH_ROWS(logn, fft_conv_rows_kernel, grid, shm, name, (const T*)x, (size_t)x_sb, (size_t)x_st,
-                                          (const cpx*)spec, (T*)y, (size_t)y_sb, (size_t)y_st, (const cpx*)tw, T_, mode, remap));
-      FSTU_CHECK_LAUNCH(name);
-      return FSTU_OK;
-    }
+  FSTU_REQUIRE(fstu_aligned(spec, 16) && fstu_aligned(tw, 16), FSTU_EALIGN, "%s: spec and tw must be 16-byte aligned", name);
+  const int cols = fft_cols(logn - 1), esz = dtype == FSTU_BF16 ? 2 : 4, ch = 16 / esz, chw = cols > ch ? cols : ch;
+  // Channel-contiguous operands whose rows split into whole 16-byte pieces per workgroup: the row-piece kernel.  The long
+  // transforms take a workgroup's channels one after the other: with fewer than two workgroups per compute unit the
+  // one-column kernel, eight times the workgroups, is the faster one.
+  const bool enough = logn < 13 || (long long)(d / chw) * B >= 512;
+  if (K == 1 && mode != 2 && enough && x_sc == 1 && y_sc == 1 && d % chw == 0 && x_st % ch == 0 && y_st % ch == 0 &&
+      x_sb % ch == 0 && y_sb % ch == 0 && fstu_aligned(x, 16) && fstu_aligned(y, 16)) {
+    const int gx = d / chw;
+    dim3 grid(gx, B);
+    const int remap = (gx % 8 == 0) ? 1 : 0;
+    FSTU_DISPATCH_DTYPE(dtype, name,
+                        FFT_LAUNCH(logn - 1, FFT_ROWS, grid, name, (const T*)x, (size_t)x_sb, (size_t)x_st,
+                                   (const cpx*)spec, (T*)y, (size_t)y_sb, (size_t)y_st, (const cpx*)tw, T_, mode, remap));
+    FSTU_CHECK_LAUNCH(name);
+    return FSTU_OK;
   }
-  (void)nt;   // n <= 16 * threads holds for every length: the bank form keeps 16 positions per thread
-  const size_t shm = fft_lds_bytes(n, lcols);
-  const int gx = (d + (1 << lcols) - 1) >> lcols;
+  if (x_st == 1 && y_st == 1) {
+    // as many columns per workgroup as fill 512 threads, or, where that leaves compute units idle, one wave (or column)
+    const int g = n / 32, many = g >= 512 ? 1 : 512 / g, few = g >= 64 ? 1 : 64 / g;
+    const bool narrow = (long long)((d + many - 1) / many) * B < 512;
+    const int gx = narrow ? (d + few - 1) / few : (d + many - 1) / many;
+    dim3 grid(gx, B);
+    const int remap = (gx % 8 == 0) ? 1 : 0;
+    FSTU_DISPATCH_DTYPE(dtype, name,
+                        FFT_LAUNCH(logn - 1, FFT_SLAB, grid, name, (const T*)x, (size_t)x_sb, (size_t)x_sc, (const cpx*)spec, (T*)y,
+                                   mode == 2 ? (T*)y2 : (T*)nullptr, (size_t)y_sb, (size_t)y_sk, (size_t)y_sc, (const cpx*)tw, T_,
+                                   d, K, remap));
+    FSTU_CHECK_LAUNCH(name);
+    return FSTU_OK;
+  }
+  const int gx = (d + cols - 1) / cols;
   dim3 grid(gx, B);
   const int remap = (gx % 8 == 0) ? 1 : 0;
   FSTU_DISPATCH_DTYPE(dtype, name,
-                      FFT_LAUNCH(logn, fft_conv_kernel, grid, shm, name, (const T*)x, (size_t)x_sb, (size_t)x_st,
+                      FFT_LAUNCH(logn - 1, FFT_PLAIN, grid, name, (const T*)x, (size_t)x_sb, (size_t)x_st,
                                  (size_t)x_sc, (const cpx*)spec, (T*)y, (T*)y2, (size_t)y_sb, (size_t)y_st, (size_t)y_sk,
-                                 (size_t)y_sc, (const cpx*)tw, T_, d, K, lcols, mode, remap));
+                                 (size_t)y_sc, (const cpx*)tw, T_, d, K, mode, remap));
   FSTU_CHECK_LAUNCH(name);
   return FSTU_OK;
 }

@@ -243,15 +243,16 @@ int fstu_stu_conv_bank(const void* x, const void* phi, void* u_plus, void* u_min
  * Here n is any power of two in 64..16384 with n >= 2T (fstu_fft_length gives the
  * smallest; a circular convolution of that length never wraps into the first T
  * outputs, so the result equals the reference's n = 2^ceil(log2(2L-1))), filters
- * are cut to their first min(L, n/2) taps, and both sign branches come out of one
- * complex inverse transform per channel.
+ * are cut to their first min(L, n/2) taps.  The transforms run on n/2 complex points:
+ * one forward transform of the two parities of the sequence, one inverse each for
+ * the even- and the odd-lag part, whose sum and difference are the sign branches.
  *
- * fstu_fft_twiddles fills tw (n complex fp32 = 2n floats) with exp(-2 pi i j / n).
+ * fstu_fft_twiddles fills tw (n complex fp32 = 2n floats, 16-byte aligned) with the
+ *   twiddle tables of the transform, in its own order.
  * fstu_stu_fft_filter transforms ncols filter columns (element (s, j) at
  *   filt[s*f_ls + j*f_cs], taps s < taps <= n/2) into spec (ncols, n) complex fp32,
- *   scaled by 1/n, in the transform's internal frequency order; with
- *   single_branch == 0 the spectrum of the (-1)^s branch is folded in as the
- *   imaginary companion.  Approx mode: columns = channels of phi_proj (f_ls = d,
+ *   (16-byte aligned): the spectra of the even and of the odd taps, scaled by 2/n, in
+ *   the transform's internal order (single_branch changes nothing in them).  Approx mode: columns = channels of phi_proj (f_ls = d,
  *   f_cs = 1); exact mode: columns = the K filters of phi (f_ls = K, f_cs = 1).
  *   Replaces the rfft of v at stu_utils.py:213-214 / the cached phi_fft of
  *   flash_stu/modules/stu.py:43-53.
@@ -270,8 +271,8 @@ int fstu_stu_fft_filter(const void* filt, int64_t f_ls, int64_t f_cs, float* spe
 int fstu_stu_conv_fft(const void* xp, const float* spec, void* y, const float* tw, int B, int T, int d, int n,
                       int single_branch, int dtype, void* stream);
 /* The same on strided operands: element (b,t,c) of xp at x_strides[0]*b + x_strides[1]*t + x_strides[2]*c (elements), y
- * likewise.  With a time stride of 1 (time-major slabs (B,d,T)) every load and store of the one-column kernel is
- * coalesced: the form for a few long sequences (transform length 8192 or 16384 and fewer than 512 groups of 8
+ * likewise.  With time strides of 1 (time-major slabs (B,d,T)) pairs of positions are read and written straight from
+ * registers, coalesced: the form for a few long sequences (transform length 8192 or 16384 and fewer than 512 groups of 8
  * channels x batch rows), where the channel-contiguous kernel leaves compute units idle. */
 int fstu_stu_conv_fft_strided(const void* xp, const int64_t* x_strides, const float* spec, void* y, const int64_t* y_strides,
                               const float* tw, int B, int T, int d, int n, int single_branch, int dtype, void* stream);

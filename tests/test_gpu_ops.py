@@ -376,6 +376,35 @@ def test_stu_conv_fft_equals_direct_fp32(hip):
     assert float(yf[1, :3].abs().max()) <= 5e-6 * float(filt.abs().max())
 
 
+@pytest.mark.parametrize("T", [32, 33, 64, 65, 127, 129, 255, 256, 511, 513, 1025, 2047, 2049, 4096, 4097, 8191])
+@pytest.mark.parametrize("B,d", [(2, 5), (64, 520)])
+def test_stu_conv_fft_every_length_and_layout(hip, T, B, d):
+    """Every transform length at its shortest and longest sequence: the slab kernel (one column or wave per workgroup, and,
+    on the large grid of short lengths, 512 threads), the row-piece kernel and the kernel for any strides give the same
+    bits, and in fp32 the time-domain kernel's values: a sum of T products collects sqrt(T) roundings of half an ulp on
+    the one side, a transform pair 2 log2 n stages of two roundings each on the other, all on the scale of the largest
+    output."""
+    if B * T * d > 4_000_000:
+        B, d = 1, 24
+    g = gen(91)
+    x = dev(torch.randn(B, T, d, generator=g))
+    f = dev(torch.randn(T, d, generator=g) / math.sqrt(T))
+    spec = hip.stu_fft_filter(f, hip.fft_length(T))
+    for single in (True, False):
+        want = hip.stu_conv_direct(x, f, single_branch=single)
+        y = torch.empty_like(x)
+        hip.stu_conv_fft_strided(x, spec, y, single_branch=single)            # channel-contiguous: row pieces or any strides
+        tol = 2.0 ** -24 * (math.sqrt(T) + 4 * math.log2(2 * T))
+        assert float((y - want).abs().max()) <= tol * float(want.abs().max())
+        xt = x.transpose(1, 2).contiguous()
+        yt = torch.full_like(xt, 9.0)
+        hip.stu_conv_fft_strided(xt.transpose(1, 2), spec, yt.transpose(1, 2), single_branch=single)
+        assert torch.equal(yt.transpose(1, 2), y)
+        z = torch.full((B, T, d + 1), 9.0, device="cuda")
+        hip.stu_conv_fft_strided(x, spec, z[:, :, :d], single_branch=single)    # an odd row stride: any strides
+        assert torch.equal(z[:, :, :d], y) and bool((z[:, :, d] == 9.0).all())
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("B,T,d,L,K", [(2, 100, 24, 128, 5), (1, 600, 6, 1024, 24), (1, 5000, 2, 8192, 3)])
 def test_stu_conv_bank_fft(hip, dtype, B, T, d, L, K):
