@@ -2,64 +2,238 @@
 // not take: fp32 (the bit-parity path of the reference's fp32 configuration, flash_stu/model.py:108-205 with
 // torch_dtype float32), bf16 shapes with K % 32 != 0 or unaligned rows, and operands with any pair of strides (the
 // (K*d, T) slabs of the exact-mode operator in fp32, flash_stu/modules/stu.py:107-120; phi @ M_filters, stu.py:88).
-// Accumulation in fp32 on the fp32 matrix instruction (v_mfma_f32_32x32x2_f32; bf16 inputs widen exactly), one
-// rounding to the output dtype.  A workgroup of 4 waves owns 64 rows x 64 features, a wave 32 x 32; K runs in tiles
-// of 32 through LDS.  Every global access is bounds-checked, so any M, N, K >= 1 works.
+// Accumulation in fp32 on the fp32 matrix instructions (bf16 inputs widen exactly), one rounding to the output dtype.
+// Every global access is bounds-checked, so any M, N, K >= 1 works.  Which kernel runs, and so the order of the sums,
+// depends on M, N and K alone: strides and alignment only choose how a tile is read.
 #include "fstu_common.h"
 
 namespace {
 
 typedef float floatx16_t __attribute__((ext_vector_type(16)));
-#define GA_BM 64
-#define GA_BN 64
-#define GA_BK 32
-#define GA_LD (GA_BK + 1)
+typedef float floatx4_t __attribute__((ext_vector_type(4)));
 
-// rows x GA_BK tile of a strided matrix into LDS as fp32, zero beyond the edges; threads run along the index whose
-// stride is 1 so that the loads coalesce either way
-template <typename T>
-__device__ __forceinline__ void ga_load_tile(float (*dst)[GA_LD], const T* __restrict__ src, long long srow, long long sk,
-                                             int row0, int nrows, int k0, int K) {
+// Elements k..k+3 of a row, zero from K on.  VEC: k runs with stride 1, rows start on 4-element boundaries and K % 4 == 0.
+// The loads are unconditional (an address beyond K is replaced by the row's start), so several stay in flight.
+template <typename T, bool VEC>
+__device__ __forceinline__ floatx4_t ga_load4(const T* __restrict__ row, long long sk, int k, int K) {
+  floatx4_t v;
+  if constexpr (VEC) {
+    const T* p = row + (k < K ? k : 0);
+    if constexpr (sizeof(T) == 4) {
+      v = *reinterpret_cast<const floatx4_t*>(p);
+    } else {
+      const uint2 u = *reinterpret_cast<const uint2*>(p);
+      v = floatx4_t{__uint_as_float(u.x << 16), __uint_as_float(u.x & 0xffff0000u), __uint_as_float(u.y << 16),
+                    __uint_as_float(u.y & 0xffff0000u)};
+    }
+    if (k >= K) v = floatx4_t{0.f, 0.f, 0.f, 0.f};
+  } else {
 #pragma unroll
-  for (int i = 0; i < GA_BM * GA_BK / 256; ++i) {
-    const int idx = threadIdx.x + 256 * i;
-    int r, k;
-    if (sk == 1) { k = idx % GA_BK; r = idx / GA_BK; }
-    else { r = idx % GA_BM; k = idx / GA_BM; }
-    const bool ok = row0 + r < nrows && k0 + k < K;
-    dst[r][k] = ok ? DT<T>::ld(src + (size_t)(row0 + r) * srow + (size_t)(k0 + k) * sk) : 0.f;
+    for (int e = 0; e < 4; ++e) {
+      const float x = DT<T>::ld(row + (size_t)(k + e < K ? k + e : 0) * sk);
+      v[e] = k + e < K ? x : 0.f;
+    }
+  }
+  return v;
+}
+
+// Few output tiles: the NW waves of a workgroup share one tile of 16*TM rows x 16*TN features and take every NW-th group of
+// 16 k, reading the fragments of v_mfma_f32_16x16x4_f32 from global memory (a lane holds 4 consecutive k, one matrix
+// instruction per element); the NW partial tiles are added in wave order through LDS.  Bound by one or two trips to
+// memory: a workgroup's k loop is K / (16 NW) trips where a tile of the staged kernel below takes K / 16 of them, one
+// behind the other.
+template <typename T, bool VEC, int TM, int TN, int NW, int U>
+__global__ void __launch_bounds__(64 * NW)
+gemm_any_split_kernel(const T* __restrict__ A, long long sam, long long sak, const T* __restrict__ W, long long swn, long long swk,
+                      T* __restrict__ C, long long ldc, int M, int N, int K) {
+  __shared__ float red[NW][TM * TN][256];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int r = lane & 15, g = lane >> 4;
+  const int m0 = blockIdx.x * 16 * TM, n0 = blockIdx.y * 16 * TN;
+  const T *ar[TM], *wr[TN];
+#pragma unroll
+  for (int j = 0; j < TM; ++j) ar[j] = A + (size_t)min(m0 + 16 * j + r, M - 1) * sam;
+#pragma unroll
+  for (int i = 0; i < TN; ++i) wr[i] = W + (size_t)min(n0 + 16 * i + r, N - 1) * swn;
+  floatx4_t acc[TN][TM];
+#pragma unroll
+  for (int i = 0; i < TN; ++i)
+#pragma unroll
+    for (int j = 0; j < TM; ++j) acc[i][j] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+  for (int k0 = 16 * w; k0 < K; k0 += 16 * NW * U) {
+    floatx4_t av[U][TM], wv[U][TN];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int k = k0 + 16 * NW * u;
+      if (k >= K) break;
+#pragma unroll
+      for (int i = 0; i < TN; ++i) wv[u][i] = ga_load4<T, VEC>(wr[i], swk, k + 4 * g, K);
+#pragma unroll
+      for (int j = 0; j < TM; ++j) av[u][j] = ga_load4<T, VEC>(ar[j], sak, k + 4 * g, K);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (k0 + 16 * NW * u >= K) break;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int i = 0; i < TN; ++i)
+#pragma unroll
+          for (int j = 0; j < TM; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[u][i][e], av[u][j][e], acc[i][j], 0, 0, 0);
+    }
+  }
+  // D: lane l holds row l % 16 and features 4*(l/16) + e of a 16 x 16 tile
+#pragma unroll
+  for (int i = 0; i < TN; ++i)
+#pragma unroll
+    for (int j = 0; j < TM; ++j) *reinterpret_cast<floatx4_t*>(&red[w][i * TM + j][4 * lane]) = acc[i][j];
+  __syncthreads();
+  for (int idx = threadIdx.x; idx < TM * TN * 256; idx += 64 * NW) {
+    const int f = idx % (16 * TN), mm = idx / (16 * TN);
+    const int tile = (f >> 4) * TM + (mm >> 4), off = ((((f & 15) >> 2) << 4) + (mm & 15)) * 4 + (f & 3);
+    float s = 0.f;
+#pragma unroll
+    for (int q = 0; q < NW; ++q) s += red[q][tile][off];
+    if (m0 + mm < M && n0 + f < N) DT<T>::st(C + (size_t)(m0 + mm) * ldc + n0 + f, s);
   }
 }
 
-template <typename T>
-__global__ void __launch_bounds__(256)
-gemm_any_kernel(const T* __restrict__ A, long long sam, long long sak, const T* __restrict__ W, long long swn, long long swk,
-                T* __restrict__ C, long long ldc, int M, int N, int K) {
-  __shared__ float xs[GA_BM][GA_LD], ws[GA_BN][GA_LD];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int wm = w & 1, wn = w >> 1;
-  const int m0 = blockIdx.x * GA_BM, n0 = blockIdx.y * GA_BN;
-  const int l32 = lane & 31, lh = lane >> 5;
-  floatx16_t acc;
+// Many output tiles: a workgroup of 4 waves owns 128 rows x 128 features, a wave 64 x 64 on v_mfma_f32_32x32x2_f32; K runs
+// in tiles of 16 through two LDS buffers, the next tile's loads in flight while this one is multiplied.  A k step of a
+// wave is 4 LDS reads for 4 matrix instructions of 64 cycles.  Bound by the fp32 matrix rate.
+#define GA_B 128
+#define GA_BK 16
+#define GA_LD (GA_BK + 1)
+
+// a thread's share (8 elements) of a 128 x 16 tile; threads run along the index whose stride is 1, so loads coalesce
+template <typename T, bool VEC>
+__device__ __forceinline__ void ga_fetch(float (&v)[8], const T* __restrict__ src, long long srow, long long sk, int row0,
+                                         int nrows, int k0, int K) {
+  if constexpr (VEC) {
 #pragma unroll
-  for (int e = 0; e < 16; ++e) acc[e] = 0.f;
-  for (int k0 = 0; k0 < K; k0 += GA_BK) {
-    ga_load_tile<T>(xs, A, sam, sak, m0, M, k0, K);
-    ga_load_tile<T>(ws, W, swn, swk, n0, N, k0, K);
-    __syncthreads();
+    for (int i = 0; i < 2; ++i) {
+      const int r = (threadIdx.x >> 2) + 64 * i, k = k0 + 4 * (threadIdx.x & 3);
+      const floatx4_t t = ga_load4<T, true>(src + (size_t)min(row0 + r, nrows - 1) * srow, 1, k, K);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[4 * i + e] = t[e];
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int idx = threadIdx.x + 256 * i;
+      const int r = sk == 1 ? idx / GA_BK : idx % GA_B, k = k0 + (sk == 1 ? idx % GA_BK : idx / GA_B);
+      const float x = DT<T>::ld(src + (size_t)min(row0 + r, nrows - 1) * srow + (size_t)(k < K ? k : 0) * sk);
+      v[i] = k < K ? x : 0.f;
+    }
+  }
+}
+
+template <bool VEC>
+__device__ __forceinline__ void ga_put(float (*dst)[GA_LD], const float (&v)[8], long long sk) {
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    if constexpr (VEC) {
+      dst[(threadIdx.x >> 2) + 64 * (i >> 2)][4 * (threadIdx.x & 3) + (i & 3)] = v[i];
+    } else {
+      const int idx = threadIdx.x + 256 * i;
+      if (sk == 1) dst[idx / GA_BK][idx % GA_BK] = v[i];
+      else dst[idx % GA_B][idx / GA_B] = v[i];
+    }
+  }
+}
+
+template <typename T, bool VEC>
+__global__ void __launch_bounds__(256)
+gemm_any_tile_kernel(const T* __restrict__ A, long long sam, long long sak, const T* __restrict__ W, long long swn, long long swk,
+                     T* __restrict__ C, long long ldc, int M, int N, int K) {
+  __shared__ float xs[2][GA_B][GA_LD], ws[2][GA_B][GA_LD];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int wm = 64 * (w & 1), wn = 64 * (w >> 1);
+  const int m0 = blockIdx.x * GA_B, n0 = blockIdx.y * GA_B;
+  const int l32 = lane & 31, lh = lane >> 5;
+  floatx16_t acc[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+  float av[8], wv[8];
+  ga_fetch<T, VEC>(av, A, sam, sak, m0, M, 0, K);
+  ga_fetch<T, VEC>(wv, W, swn, swk, n0, N, 0, K);
+  ga_put<VEC>(xs[0], av, sak);
+  ga_put<VEC>(ws[0], wv, swk);
+  __syncthreads();
+  for (int k0 = 0, b = 0; k0 < K; k0 += GA_BK, b ^= 1) {
+    const bool more = k0 + GA_BK < K;
+    if (more) {
+      ga_fetch<T, VEC>(av, A, sam, sak, m0, M, k0 + GA_BK, K);
+      ga_fetch<T, VEC>(wv, W, swn, swk, n0, N, k0 + GA_BK, K);
+    }
     // weights as the A operand (lane: feature l % 32, k = l / 32), activations as the B operand (lane: row l % 32)
 #pragma unroll
-    for (int kk = 0; kk < GA_BK; kk += 2)
-      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(ws[32 * wn + l32][kk + lh], xs[32 * wm + l32][kk + lh], acc, 0, 0, 0);
+    for (int kk = 0; kk < GA_BK; kk += 2) {
+      float x[2], y[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        x[i] = xs[b][wm + 32 * i + l32][kk + lh];
+        y[i] = ws[b][wn + 32 * i + l32][kk + lh];
+      }
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(y[i], x[j], acc[i][j], 0, 0, 0);
+    }
+    if (more) {      // the other buffer was last read before the barrier that ended the previous tile
+      ga_put<VEC>(xs[b ^ 1], av, sak);
+      ga_put<VEC>(ws[b ^ 1], wv, swk);
+    }
     __syncthreads();
   }
-  // D: lane l holds row l % 32 and features 8*(e/4) + 4*(l/32) + e%4 of the wave's 32 x 32 tile
-  const int m = m0 + 32 * wm + l32;
-  if (m >= M) return;
+  // D: lane l holds row l % 32 and features 8*(e/4) + 4*(l/32) + e%4 of a 32 x 32 tile
 #pragma unroll
-  for (int e = 0; e < 16; ++e) {
-    const int f = n0 + 32 * wn + 8 * (e >> 2) + 4 * lh + (e & 3);
-    if (f < N) DT<T>::st(C + (size_t)m * ldc + f, acc[e]);
+  for (int j = 0; j < 2; ++j) {
+    const int m = m0 + wm + 32 * j + l32;
+    if (m >= M) continue;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int f = n0 + wn + 32 * i + 8 * (e >> 2) + 4 * lh + (e & 3);
+        if (f < N) DT<T>::st(C + (size_t)m * ldc + f, acc[i][j][e]);
+      }
+  }
+}
+
+// 0: 16 x 16 tiles, 16 waves along K; 1: 32 x 32 tiles, 8 waves along K; 2: 128 x 128 tiles.  The large tile needs more
+// than one workgroup per compute unit before its matrix rate counts (192 tiles: 2000 x 1536 x 1536 141 us on 1, 158 on 2;
+// 512 tiles: 4096 x 2048 x 24 40 us on 1, 33 on 2; 1024: 16384 x 2048 x 2048 1885 on 1, 1153 on 2), the 32 x 32 tile half
+// the chip (16 tiles: 64 x 256 x 3072 13 us on 0, 27 on 1; 80: 300 x 256 x 3072 25 and 30; 256: 1000 x 256 x 3072 49 and 31).
+// One kernel of 64 x 64 tiles with no loads ahead took 228, 525, 500 us for the last three, 283 and 2860 for the first and
+// third, 23 us for 200 x 256 x 256 (now 8), and its sums in one chain were 2.5 to 4 times further from float64 than those
+// of the split kernels.
+static int ga_pick(int M, int N) {
+  const long long t128 = (long long)((M + 127) / 128) * ((N + 127) / 128);
+  const long long t32 = (long long)((M + 31) / 32) * ((N + 31) / 32);
+  return t128 > 256 ? 2 : t32 >= 128 ? 1 : 0;
+}
+
+template <typename T, bool VEC>
+static void ga_launch(const T* A, long long sam, long long sak, const T* W, long long swn, long long swk, T* C, long long ldc,
+                      int M, int N, int K, hipStream_t s) {
+  switch (ga_pick(M, N)) {
+    case 0:
+      hipLaunchKernelGGL((gemm_any_split_kernel<T, VEC, 1, 1, 16, 4>), dim3((M + 15) / 16, (N + 15) / 16), dim3(1024), 0, s, A, sam,
+                         sak, W, swn, swk, C, ldc, M, N, K);
+      break;
+    case 1:
+      hipLaunchKernelGGL((gemm_any_split_kernel<T, VEC, 2, 2, 8, 2>), dim3((M + 31) / 32, (N + 31) / 32), dim3(512), 0, s, A, sam,
+                         sak, W, swn, swk, C, ldc, M, N, K);
+      break;
+    default:
+      hipLaunchKernelGGL((gemm_any_tile_kernel<T, VEC>), dim3((M + 127) / 128, (N + 127) / 128), dim3(256), 0, s, A, sam, sak, W,
+                         swn, swk, C, ldc, M, N, K);
   }
 }
 
@@ -75,12 +249,14 @@ extern "C" int fstu_gemm_any(const void* A, int64_t sam, int64_t sak, const void
                    (swk > 0 || K == 1),
                FSTU_ESHAPE, "fstu_gemm_any: strides must be positive (sam=%lld sak=%lld swn=%lld swk=%lld)", (long long)sam,
                (long long)sak, (long long)swn, (long long)swk);
-  const unsigned gx = (unsigned)((M + GA_BM - 1) / GA_BM), gy = (unsigned)((N + GA_BN - 1) / GA_BN);
-  FSTU_REQUIRE(gy <= 65535u, FSTU_ESHAPE, "fstu_gemm_any: N=%d too large", N);
+  FSTU_REQUIRE(N <= 65535 * GA_B, FSTU_ESHAPE, "fstu_gemm_any: N=%d too large", N);
+  // four elements per load: k contiguous, rows on 4-element boundaries, K a whole number of fours
+  const size_t quad = dtype == FSTU_BF16 ? 8 : 16;
+  const bool vec = (sak == 1 || K == 1) && (swk == 1 || K == 1) && K % 4 == 0 && sam % 4 == 0 && swn % 4 == 0 && fstu_aligned(A, quad) &&
+                   fstu_aligned(W, quad);
   FSTU_DISPATCH_DTYPE(dtype, "fstu_gemm_any",
-                      hipLaunchKernelGGL((gemm_any_kernel<T>), dim3(gx, gy), dim3(256), 0, (hipStream_t)stream, (const T*)A,
-                                         (long long)sam, (long long)sak, (const T*)W, (long long)swn, (long long)swk, (T*)C,
-                                         (long long)ldc, M, N, K));
+                      if (vec) ga_launch<T, true>((const T*)A, sam, sak, (const T*)W, swn, swk, (T*)C, ldc, M, N, K, (hipStream_t)stream);
+                      else ga_launch<T, false>((const T*)A, sam, sak, (const T*)W, swn, swk, (T*)C, ldc, M, N, K, (hipStream_t)stream));
   FSTU_CHECK_LAUNCH("fstu_gemm_any");
   return FSTU_OK;
 }

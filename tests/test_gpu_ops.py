@@ -174,6 +174,29 @@ def test_gemm_any_against_float64(hip, dtype, M, N, K):
               atol=2.0 ** -7 * float(ref.float().abs().max()))
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("M,N,K", [(1, 50, 4), (17, 33, 64), (64, 256, 3072), (31, 4065, 20), (128, 1024, 1028),
+                                   (129, 992, 257), (2049, 2049, 40), (2050, 2052, 15)])
+def test_gemm_any_tiles(hip, dtype, M, N, K):
+    """Edges of the three tile sizes of fstu_gemm_any (16 x 16 and 32 x 32 with the waves along K, 128 x 128 staged):
+    ragged rows and features, K of less than one group of 16 and of many trips, a k tail.  fp32 within twice K rounding
+    errors of the sums of magnitudes (each product and each addition rounds once), bf16 within its own rounding more;
+    k-slow and unaligned views give the same values; what lies outside the result stays as it was."""
+    g = gen(65)
+    x, W = torch.randn(M, K, generator=g).to(dtype), torch.randn(N, K, generator=g).to(dtype)
+    xd, Wd = dev(x), dev(W)
+    out = torch.full((M + 1, N + 3), float("nan"), dtype=dtype, device="cuda")
+    got = hip.gemm_any(xd, Wd, out=out[:M, :N])
+    ref, mag = xd.double() @ Wd.double().t(), xd.double().abs() @ Wd.double().abs().t()
+    bound = 2 * K * 2.0 ** -24 * mag + (2.0 ** -8 * ref.abs() if dtype == torch.bfloat16 else 0.0)
+    assert bool(((got.double() - ref).abs() <= bound).all())
+    assert bool(torch.isnan(out[M:]).all()) and bool(torch.isnan(out[:, N:]).all())
+    assert torch.equal(hip.gemm_any(xd.t().contiguous().t(), Wd), got)
+    odd = torch.empty(M * K + 1, dtype=dtype, device="cuda")[1:].view(M, K)
+    odd.copy_(xd)
+    assert torch.equal(hip.gemm_any(odd, Wd), got)
+
+
 @pytest.mark.parametrize("nb,M,N,K", [(1, 128, 64, 64), (3, 256, 132, 192), (2, 1024, 1024, 1536), (4, 512, 260, 2048),
                                       (1, 4096, 768, 3072)])
 def test_gemm_bf16_transposed_activations(hip, nb, M, N, K):
