@@ -25,6 +25,8 @@
 // 768 24.5 -> 17.4, 32 x 300 x 2048 188 -> 105, 4 x 4096 x 2048 296 -> 218, one time-major sequence of 4096 x 2048 95 -> 50.
 #include "fstu_common.h"
 
+#include <type_traits>
+
 namespace {
 
 typedef float2 cpx;
@@ -732,6 +734,229 @@ fft_conv_rows_kernel(const T* __restrict__ x, size_t x_sb, size_t x_st, const cp
   }
 }
 
+// ---------------------------------------------------------------- gradients of the convolution
+// With gE = g+ + g- and gO = g+ - g- (the gradients that reach the even- and the odd-lag part; g- = g+ where the branches
+// are only ever added, then gO vanishes and so do all odd lags), zE[m] = gE[2m] + i gE[2m+1] and the shifted
+// zS[m] = gO[2m+1] + i gO[2m+2]:
+//   gradient of the input, both parities at once:  sum_j zE[m+j] fe[j] + zS[m+j] fo[j]      -> one inverse transform of
+//                                                  ZE conj(Fe) + ZS conj(Fo)
+//   gradient of the filter, one batch row's part:  gfe[j] = Re sum_m zE[m+j] conj z[m],  gfo[j] = Re sum_m zS[m+j] conj z[m]
+// so that a column costs four transforms of n/2 points (six with odd lags) and its operands are read once.  Composed of
+// the forward kernel on time-reversed fp32 copies the same took 18 n/2-point transforms per column, one launch and one
+// filter transform per batch row, and flips, sums and casts in between.  Rows' parts of the filter gradient go to memory in
+// fp32 and are added by fft_corr_finish_kernel in the order of the rows (no atomics: the same bits every time).
+// Vector-ALU issue bounds it as it does the convolution.  bf16, 8 x 2048 x 768: 120 us and 10 us for the sum over the rows,
+// where the composed form took 0.95 ms; a training step at that size 1.34 -> 0.37 ms.
+// A workgroup owns the COLS neighbouring channels that its threads transform and reads them as pieces of a row.
+template <typename T, int LOGN> struct CorrCut {
+  static constexpr int COLS = 1 << fft_lcols<LOGN>(), NE = COLS < RowVec<T>::CH ? COLS : RowVec<T>::CH, VR = COLS / NE;
+  static constexpr int NT = fft_threads<LOGN>(), NV = (Half<LOGN>::N / 2) * VR / NT, PST = Half<LOGN>::N / 2 + 1;
+};
+template <typename E, int NE> struct alignas(NE * sizeof(E)) Piece { E e[NE]; };
+// channels c .. c+NE-1 of a row: one access where rows and channels are whole pieces (vec), else element by element
+template <typename T, int NE>
+__device__ __forceinline__ void load_piece(const T* p, int c, int d, bool vec, float (&f)[NE]) {
+  if (vec) {
+    Piece<T, NE> v = {};
+    if (c < d) v = *(const Piece<T, NE>*)p;
+#pragma unroll
+    for (int k = 0; k < NE; ++k) f[k] = DT<T>::ld(&v.e[k]);
+  } else {
+#pragma unroll
+    for (int k = 0; k < NE; ++k) f[k] = c + k < d ? DT<T>::ld(p + k) : 0.f;
+  }
+}
+template <typename T, int NE>
+__device__ __forceinline__ void store_piece(T* p, int c, int d, bool vec, const float (&f)[NE]) {
+  if (vec) {
+    Piece<T, NE> v;
+#pragma unroll
+    for (int k = 0; k < NE; ++k) DT<T>::st(&v.e[k], f[k]);
+    if (c < d) *(Piece<T, NE>*)p = v;
+  } else {
+#pragma unroll
+    for (int k = 0; k < NE; ++k)
+      if (c + k < d) DT<T>::st(p + k, f[k]);
+  }
+}
+template <int LOGN>
+__device__ __forceinline__ void conj_product16(const cpx* __restrict__ sp, const cpx (&x)[16], cpx (&v)[16], bool add) {
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const float4 s = ((const float4*)sp)[k * Half<LOGN>::G];
+    const cpx a = cmul(x[2 * k], make_float2(s.x, -s.y)), b = cmul(x[2 * k + 1], make_float2(s.z, -s.w));
+    v[2 * k] = add ? make_float2(v[2 * k].x + a.x, v[2 * k].y + a.y) : a;
+    v[2 * k + 1] = add ? make_float2(v[2 * k + 1].x + b.x, v[2 * k + 1].y + b.y) : b;
+  }
+}
+
+template <typename T, int LOGN, bool ODD>
+__global__ void __launch_bounds__(fft_threads<LOGN>(), ODD ? 2 : 4)
+fft_corr_kernel(const T* __restrict__ g1, const T* __restrict__ g2, const T* __restrict__ x, const cpx* __restrict__ spec,
+                T* __restrict__ gx, float* __restrict__ part, const cpx* __restrict__ tw, int Tn, int d, int lags, int vec,
+                int xcd_remap) {
+  extern __shared__ cpx fft_lds[];
+  using W = Half<LOGN>;
+  using R = CorrCut<T, LOGN>;
+  constexpr int N = W::N, COLS = R::COLS, NE = R::NE, VR = R::VR, NV = R::NV, NT = R::NT, PST = R::PST;
+  static_assert(NV * NT == (N / 2) * VR && PST <= W::STRIDE, "whole pieces per thread");
+  int bx = blockIdx.x;
+  if (xcd_remap) bx = (bx & 7) * (gridDim.x >> 3) + (bx >> 3);   // consecutive channel groups share an XCD
+  const int c0 = bx * COLS, b = blockIdx.y;
+  const size_t row0 = (size_t)b * Tn;
+  const int mycol = threadIdx.x / W::G, u = threadIdx.x % W::G, c = min(c0 + mycol, d - 1);
+  cpx* col = fft_lds + (size_t)mycol * W::STRIDE;
+  cpx* stage = fft_lds;                                // [column][pair], in the columns' place
+  // pairs of rows of one tensor (WHICH 0: x, 1: gE, 2: gO) -> stage
+  auto put_stage = [&](auto which) {
+    constexpr int WHICH = decltype(which)::value;
+#pragma unroll
+    for (int r = 0; r < NV; ++r) {
+      const int q = threadIdx.x + r * NT, m = q / VR, cp = (q % VR) * NE;
+      float f[2][NE];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int t = 2 * m + h;
+#pragma unroll
+        for (int k = 0; k < NE; ++k) f[h][k] = 0.f;
+        if (t < Tn) {
+          const size_t at = (row0 + t) * (size_t)d + c0 + cp;
+          if constexpr (WHICH == 0) {
+            load_piece<T, NE>(x + at, c0 + cp, d, vec, f[h]);
+          } else {
+            load_piece<T, NE>(g1 + at, c0 + cp, d, vec, f[h]);
+            if constexpr (!ODD) {
+#pragma unroll
+              for (int k = 0; k < NE; ++k) f[h][k] *= 2.f;
+            } else if (g2) {
+              float s[NE];
+              load_piece<T, NE>(g2 + at, c0 + cp, d, vec, s);
+#pragma unroll
+              for (int k = 0; k < NE; ++k) f[h][k] = WHICH == 1 ? f[h][k] + s[k] : f[h][k] - s[k];
+            }
+          }
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < NE; ++k) stage[(cp + k) * PST + m] = make_float2(f[0][k], f[1][k]);
+    }
+    if (ODD && threadIdx.x < COLS) stage[threadIdx.x * PST + N / 2] = make_float2(0.f, 0.f);
+  };
+  auto take = [&](cpx (&z)[8]) {
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 8; ++k) z[k] = stage[mycol * PST + point<LOGN>(u, k)];
+    __syncthreads();
+  };
+  // real parts of a correlation: lags 2j + ODDLAG of this row's part of the filter gradient
+  auto put_part = [&](const cpx (&r)[8], int odd_lag) {
+    __syncthreads();
+    float* st = (float*)stage;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) st[mycol * PST + point<LOGN>(u, k)] = r[k].x * (1.f / (float)N);
+    __syncthreads();
+    const int rows = ODD ? lags : (lags + 1) / 2;
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      const int q = threadIdx.x + v * NT, m = q / VR, cp = (q % VR) * NE;
+      if (2 * m + odd_lag >= lags) continue;
+      float f[NE];
+#pragma unroll
+      for (int k = 0; k < NE; ++k) f[k] = st[(cp + k) * PST + m];
+      const int row = ODD ? 2 * m + odd_lag : m;
+      store_piece<float, NE>(part + ((size_t)b * rows + row) * d + c0 + cp, c0 + cp, d, vec, f);
+    }
+    __syncthreads();
+  };
+  const cpx* sp = spec + (size_t)c * (2 * N) + 2 * u;
+  cpx zx[8], z[8], xe[16], w[16], r8[8];
+  if (part) {
+    put_stage(std::integral_constant<int, 0>{});
+    take(zx);
+  }
+  put_stage(std::integral_constant<int, 1>{});
+  take(z);
+  fft_forward<LOGN>(col, tw, u, z, xe);
+  if (gx) conj_product16<LOGN>(sp, xe, w, false);
+  if constexpr (ODD) {
+    cpx xx[16];
+    if (part) {
+      __syncthreads();
+      fft_forward<LOGN>(col, here(tw), here(u), zx, xx);
+#pragma unroll
+      for (int k = 0; k < 16; ++k) xe[k] = cmul(xe[k], make_float2(xx[k].x, -xx[k].y));
+      fft_inverse<LOGN>(col, here(tw), here(u), xe, r8);
+      put_part(r8, 0);
+    } else {
+      __syncthreads();
+    }
+    put_stage(std::integral_constant<int, 2>{});
+    __syncthreads();
+    {
+      const float* st = (const float*)(stage + mycol * PST);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        const int m = point<LOGN>(u, k);
+        z[k] = make_float2(st[2 * m + 1], st[2 * m + 2]);
+      }
+    }
+    __syncthreads();
+    fft_forward<LOGN>(col, here(tw), here(u), z, xe);
+    if (gx) conj_product16<LOGN>(sp + N, xe, w, true);
+    if (part) {
+#pragma unroll
+      for (int k = 0; k < 16; ++k) xe[k] = cmul(xe[k], make_float2(xx[k].x, -xx[k].y));
+      fft_inverse<LOGN>(col, here(tw), here(u), xe, r8);
+      put_part(r8, 1);
+    }
+  }
+  if (gx) {
+    if (ODD) __syncthreads();
+    fft_inverse<LOGN>(col, here(tw), here(u), w, r8);
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 8; ++k) stage[mycol * PST + point<LOGN>(here(u), k)] = r8[k];
+    __syncthreads();
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      const int q = here((int)threadIdx.x) + v * NT, m = q / VR, cp = (q % VR) * NE;
+      float f[2][NE];
+#pragma unroll
+      for (int k = 0; k < NE; ++k) {
+        const cpx s = stage[(cp + k) * PST + m];
+        f[0][k] = s.x;
+        f[1][k] = s.y;
+      }
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        if (2 * m + h < Tn) store_piece<T, NE>(gx + (row0 + 2 * m + h) * (size_t)d + c0 + cp, c0 + cp, d, vec, f[h]);
+    }
+  }
+  if constexpr (!ODD) {
+    if (part) {
+      cpx xx[16];
+      __syncthreads();
+      fft_forward<LOGN>(col, here(tw), here(u), zx, xx);
+#pragma unroll
+      for (int k = 0; k < 16; ++k) xe[k] = cmul(xe[k], make_float2(xx[k].x, -xx[k].y));
+      fft_inverse<LOGN>(col, here(tw), here(u), xe, r8);
+      put_part(r8, 0);
+    }
+  }
+}
+
+// filter gradient (L, d): the rows' parts (B, rows, d) added in order; lags that have none are zero
+template <typename T, bool ODD>
+__global__ void __launch_bounds__(256) fft_corr_finish_kernel(const float* __restrict__ part, T* __restrict__ gf, int B, int lags, int L, int d) {
+  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= (size_t)L * d) return;
+  const int s = (int)(i / d), c = (int)(i - (size_t)s * d), rows = ODD ? lags : (lags + 1) / 2;
+  float a = 0.f;
+  if (s < lags && (ODD || !(s & 1)))
+    for (int b = 0; b < B; ++b) a += part[((size_t)b * rows + (ODD ? s : s >> 1)) * d + c];
+  DT<T>::st(gf + i, a);
+}
+
 int ilog2_exact(int n) {
   int l = 0;
   while ((1 << l) < n) ++l;
@@ -773,6 +998,10 @@ extern "C" int fstu_fft_length(int T_) {
   FFT_GO((fft_conv_kernel<T, L>), fft_threads<L>(), (fft_lds_bytes<L, fft_threads<L>()>()), GRID, NAME, __VA_ARGS__)
 #define FFT_ROWS(L, GRID, NAME, ...) \
   FFT_GO((fft_conv_rows_kernel<T, L>), fft_threads<L>(), (fft_lds_bytes<L, fft_threads<L>()>()), GRID, NAME, __VA_ARGS__)
+#define FFT_CORR_SUM(L, GRID, NAME, ...) \
+  FFT_GO((fft_corr_kernel<T, L, false>), fft_threads<L>(), (fft_lds_bytes<L, fft_threads<L>()>()), GRID, NAME, __VA_ARGS__)
+#define FFT_CORR_ALL(L, GRID, NAME, ...) \
+  FFT_GO((fft_corr_kernel<T, L, true>), fft_threads<L>(), (fft_lds_bytes<L, fft_threads<L>()>()), GRID, NAME, __VA_ARGS__)
 #define FFT_SLAB(L, GRID, NAME, ...)                                                                                        \
   do {                                                                                                                      \
     constexpr int few__ = Half<L>::G > 64 ? Half<L>::G : 64;                                                                \
@@ -904,4 +1133,53 @@ extern "C" int fstu_stu_conv_bank_fft(const void* x, const int64_t* x_strides, c
   return conv_fft_launch("fstu_stu_conv_bank_fft", x, x_strides[0], x_strides[1], x_strides[2], spec, u_plus, u_minus,
                          u_strides[0], u_strides[1], u_strides[2], u_strides[3], tw, B, T_, d, K, n, u_minus ? 2 : 1,
                          dtype, stream);
+}
+
+// Gradients of the convolution above.  g1, g2 (B, T, d): the gradients of the plus and the minus branch, or with
+// branches = 0 (sum) g1 alone for y = plus + minus, with branches = 1 g1 alone for the plus branch.  gx (B, T, d) and
+// gf (L, d) may each be null; part: fp32 scratch of fstu_stu_conv_fft_grad_ws(...) elements, needed for gf.
+extern "C" int64_t fstu_stu_conv_fft_grad_ws(int B, int T_, int d, int L, int branches) {
+  const int64_t lags = L < T_ ? L : T_;
+  return (int64_t)B * (branches == 0 ? (lags + 1) / 2 : lags) * d;
+}
+extern "C" int fstu_stu_conv_fft_grad(const void* g1, const void* g2, const void* x, const float* spec, void* gx, void* gf,
+                                      float* part, const float* tw, int B, int T_, int d, int L, int n, int branches,
+                                      int dtype, void* stream) {
+  FSTU_REQUIRE(g1 && spec && tw && (gx || gf), FSTU_ENULL, "fstu_stu_conv_fft_grad: null pointer");
+  FSTU_REQUIRE(!gf || (x && part), FSTU_ENULL, "fstu_stu_conv_fft_grad: gf needs x and part");
+  FSTU_REQUIRE(branches >= 0 && branches <= 2 && (branches == 2) == (g2 != nullptr), FSTU_EARG,
+               "fstu_stu_conv_fft_grad: branches=%d (0 sum, 1 plus, 2 both; g2 belongs to 2 alone)", branches);
+  const int logn = ilog2_exact(n);
+  FSTU_REQUIRE(logn >= 6 && logn <= 14, FSTU_ESHAPE, "fstu_stu_conv_fft_grad: n=%d is not a power of two in 64..16384", n);
+  FSTU_REQUIRE(B >= 1 && B <= 65535 && T_ >= 1 && d >= 1 && L >= 1 && 2 * T_ <= n, FSTU_ESHAPE,
+               "fstu_stu_conv_fft_grad: bad shape B=%d T=%d d=%d L=%d n=%d (n >= 2T required)", B, T_, d, L, n);
+  FSTU_REQUIRE(fstu_aligned(spec, 16) && fstu_aligned(tw, 16), FSTU_EALIGN, "fstu_stu_conv_fft_grad: spec and tw must be 16-byte aligned");
+  const int cols = fft_cols(logn - 1), esz = dtype == FSTU_BF16 ? 2 : 4, ch = 16 / esz, ne = cols < ch ? cols : ch;
+  // rows of whole pieces: every piece of every tensor lies on its own size (the fp32 parts are pieces of ne * 4 bytes)
+  const size_t al = (size_t)ne * esz;
+  const int vec = d % ne == 0 && fstu_aligned(g1, al) && (!g2 || fstu_aligned(g2, al)) && (!x || fstu_aligned(x, al)) &&
+                  (!gx || fstu_aligned(gx, al)) && (!gf || fstu_aligned(part, (size_t)ne * 4));
+  const int gxb = (d + cols - 1) / cols, lags = L < T_ ? L : T_;
+  dim3 grid(gxb, B);
+  const int remap = (gxb % 8 == 0) ? 1 : 0;
+  float* pt = gf ? part : nullptr;
+  if (branches == 0) {
+    FSTU_DISPATCH_DTYPE(dtype, "fstu_stu_conv_fft_grad",
+                        FFT_LAUNCH(logn - 1, FFT_CORR_SUM, grid, "fstu_stu_conv_fft_grad", (const T*)g1, (const T*)nullptr, (const T*)x,
+                                   (const cpx*)spec, (T*)gx, pt, (const cpx*)tw, T_, d, lags, vec, remap));
+  } else {
+    FSTU_DISPATCH_DTYPE(dtype, "fstu_stu_conv_fft_grad",
+                        FFT_LAUNCH(logn - 1, FFT_CORR_ALL, grid, "fstu_stu_conv_fft_grad", (const T*)g1, (const T*)g2, (const T*)x,
+                                   (const cpx*)spec, (T*)gx, pt, (const cpx*)tw, T_, d, lags, vec, remap));
+  }
+  FSTU_CHECK_LAUNCH("fstu_stu_conv_fft_grad");
+  if (!gf) return FSTU_OK;
+  const dim3 fg((unsigned)(((size_t)L * d + 255) / 256));
+  FSTU_DISPATCH_DTYPE(dtype, "fstu_stu_conv_fft_grad", if (branches == 0) {
+    hipLaunchKernelGGL((fft_corr_finish_kernel<T, false>), fg, dim3(256), 0, (hipStream_t)stream, part, (T*)gf, B, lags, L, d);
+  } else {
+    hipLaunchKernelGGL((fft_corr_finish_kernel<T, true>), fg, dim3(256), 0, (hipStream_t)stream, part, (T*)gf, B, lags, L, d);
+  });
+  FSTU_CHECK_LAUNCH("fstu_stu_conv_fft_grad");
+  return FSTU_OK;
 }

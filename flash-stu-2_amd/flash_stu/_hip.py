@@ -54,6 +54,8 @@ SIGNATURES = {
     "fstu_stu_conv_fft": [_vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _vp],
     "fstu_stu_conv_fft_strided": [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _vp],
     "fstu_transpose": [_vp, _vp, _i, _i, _i, _i, _vp],
+    "fstu_stu_conv_fft_grad_ws": [_i, _i, _i, _i, _i],
+    "fstu_stu_conv_fft_grad": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _vp],
     "fstu_stu_conv_bank_fft": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _vp],
     "fstu_kv_append": [_vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _vp],
     "fstu_kv_fill": [_vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _vp],
@@ -124,6 +126,7 @@ def load(path: Optional[str] = None):
     lib.fstu_sample_ws_bytes.restype = ctypes.c_int64
     lib.fstu_swa_prefill_ws_elems.restype = ctypes.c_int64
     lib.fstu_lds_sequence_ws_floats.restype = ctypes.c_size_t
+    lib.fstu_stu_conv_fft_grad_ws.restype = ctypes.c_int64
     if path is None:
         _lib = lib
     return lib
@@ -683,6 +686,30 @@ def stu_conv_fft_strided(xp: torch.Tensor, spec: torch.Tensor, out: torch.Tensor
     _check(load().fstu_stu_conv_fft_strided(_p(xp), xs, _p(spec), _p(out), ys, _p(fft_twiddles(n, xp.device)), B, T, d, n,
                                             int(single_branch), _dt(xp), _stream()), "fstu_stu_conv_fft_strided")
     return out
+
+
+def stu_conv_fft_grad(g1: torch.Tensor, g2: Optional[torch.Tensor], x: torch.Tensor, spec: torch.Tensor, taps: int,
+                      branches: int, want_x: bool = True, want_filter: bool = True):
+    """Gradients of the convolution of x (B,T,d) with a (taps,d) filter of spectra spec: branches 0: g1 is the gradient of
+    plus + minus, 1: of plus alone, 2: g1 and g2 those of plus and minus.  Returns (gx or None, (taps,d) gradient or None)."""
+    _dev(g1, g2, x, spec)
+    B, T, d = x.shape
+    n = spec.shape[1]
+    if spec.shape != (d, n, 2) or spec.dtype != torch.float32:
+        raise FlashSTUHipError(f"spec must be ({d}, n, 2) float32, got {tuple(spec.shape)} {spec.dtype}")
+    for g in (g1,) if g2 is None else (g1, g2):
+        if g.shape != x.shape or g.dtype != x.dtype:
+            raise FlashSTUHipError("gradients must have x's shape and dtype")
+    gx = torch.empty_like(x) if want_x else None
+    gf = part = None
+    if want_filter:
+        gf = torch.empty(taps, d, dtype=x.dtype, device=x.device)
+        part = torch.empty(int(load().fstu_stu_conv_fft_grad_ws(B, T, d, taps, branches)), dtype=torch.float32, device=x.device)
+    if want_x or want_filter:
+        _check(load().fstu_stu_conv_fft_grad(_p(g1), _p(g2), _p(x), _p(spec), _p(gx), _p(gf), _p(part),
+                                             _p(fft_twiddles(n, x.device)), B, T, d, taps, n, branches, _dt(x), _stream()),
+               "fstu_stu_conv_fft_grad")
+    return gx, gf
 
 
 def stu_conv_bank_fft(x: torch.Tensor, spec: torch.Tensor, u_plus: torch.Tensor, u_minus: Optional[torch.Tensor]):

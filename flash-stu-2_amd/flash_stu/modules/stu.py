@@ -320,7 +320,7 @@ class STU(nn.Module):
         """Training-side forward of the approx-mode STU (stu.py:81-98,120) under autograd: the two projections are
         library GEMMs, the convolution between them is the HIP kernel with its own backward
         (flash_stu.utils.stu_utils.convolve), so gradients reach x, M_inputs and M_filters.  No decode state."""
-        from ..utils.stu_utils import convolve, nearest_power_of_two
+        from ..utils.stu_utils import ApproxConvolveSum, convolve, nearest_power_of_two
         if not self.use_approx:
             raise NotImplementedError("forward_differentiable covers use_approx=True")
         if self.tile_size < self.d_in:
@@ -328,8 +328,10 @@ class STU(nn.Module):
         x_proj = x @ self.M_inputs
         phi_proj = self.phi @ self.M_filters
         n = nearest_power_of_two(2 * self.phi.shape[0] - 1, round_up=True)
-        plus, minus = convolve(x_proj, phi_proj, n, use_approx=True, return_both=not self.use_hankel_L)
-        return plus if self.use_hankel_L else plus + minus
+        if self.use_hankel_L or x_proj.dim() != 3 or not x_proj.is_cuda or n < 2 * x_proj.shape[1] - 1:
+            plus, minus = convolve(x_proj, phi_proj, n, use_approx=True, return_both=not self.use_hankel_L)
+            return plus if self.use_hankel_L else plus + minus
+        return ApproxConvolveSum.apply(x_proj, phi_proj.to(x_proj.dtype))
 
     @torch.no_grad()
     def forward(self, x: torch.Tensor, past_state=None, use_cache: bool = False):

@@ -72,65 +72,105 @@ def _alt_sign(L: int, like: torch.Tensor) -> torch.Tensor:
     return s
 
 
-def _causal_conv(u: torch.Tensor, v: torch.Tensor) -> torch.Tensor:
-    """u (B,T,d) with the per-channel filter v (L,d): out[b,t,c] = T(sum_{s<=t} v[s,c] u[b,t-s,c]), one branch.
-    FFT kernel from 32 positions on (as far as the in-LDS transform reaches), time-domain kernel otherwise."""
+def _conv_length(T: int) -> int:
+    """Transform length of the FFT kernels for T positions; 0 where the time-domain kernel runs instead (fewer than 32
+    positions, or more than the in-LDS transform reaches)."""
     from .. import _hip
-    T = u.shape[1]
-    n = _hip.fft_length(T) if T >= 32 else 0
+    return _hip.fft_length(T) if T >= 32 else 0
+
+
+def _causal_conv(u: torch.Tensor, v: torch.Tensor) -> torch.Tensor:
+    """u (B,T,d) with the per-channel filter v (L,d): out[b,t,c] = T(sum_{s<=t} v[s,c] u[b,t-s,c]), one branch."""
+    from .. import _hip
+    n = _conv_length(u.shape[1])
     if n == 0:
         return _hip.stu_conv_direct(u.contiguous(), v.contiguous(), single_branch=True)
     return _hip.stu_conv_fft(u.contiguous(), _hip.stu_fft_filter(v.contiguous(), n, single_branch=True), single_branch=True)
 
 
-class _ApproxConvolve(torch.autograd.Function):
-    """Both sign branches of the approx-mode convolution with their gradients.  The minus branch
-    sgn * conv(sgn * u, v) equals conv(u, v * (-1)^s), so every piece of forward and backward is the one causal
-    convolution kernel:
+def _convolve_grads(ctx, u, v, spec, gp, gm, branches):
+    """Gradients of the convolution in u and v, formed in fp32 whatever the input dtype (the reference differentiates
+    through an fp32 FFT, stu_utils.py:226-228) and rounded once at the end.  branches 0: gp is the gradient of
+    plus + minus; 1: of plus alone; 2: gp and gm are those of plus and minus.  With the forward's spectra one launch of
+    the gradient kernel; without (the lengths of the time-domain kernel) as convolutions: the minus branch
+    sgn * conv(sgn * u, v) equals conv(u, v * (-1)^s), and
       d/du: correlation with the filter     = time-reversed convolution of the time-reversed gradient
       d/dv: correlation of gradient and u   = per batch row, convolution of the time-reversed gradient with that
-            row's input as the filter, read backwards; summed over the batch in fp32
-    The backward runs in fp32 whatever the input dtype (the reference differentiates through an fp32 FFT,
-    stu_utils.py:226-228) and rounds the two gradients once at the end."""
+            row's input as the filter, read backwards; summed over the batch in fp32."""
+    from .. import _hip
+    want_u, want_v = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
+    if spec is not None:
+        return _hip.stu_conv_fft_grad(gp.contiguous(), gm.contiguous() if branches == 2 else None, u.contiguous(), spec,
+                                      v.shape[0], branches, want_u, want_v)
+    both = branches != 1
+    gm = gp if branches == 0 else gm
+    B, T, d = u.shape
+    L = v.shape[0]
+    uf, vf = u.float(), v.float()
+    gpf = gp.float().flip(1).contiguous()
+    gmf = gm.float().flip(1).contiguous() if both else None
+    gu = gv = None
+    if want_u:
+        gu = _causal_conv(gpf, vf)
+        if both:
+            gu = gu + _causal_conv(gmf, vf * _alt_sign(L, vf))
+        gu = gu.flip(1).to(u.dtype)
+    if want_v:
+        taps = min(L, T)
+        acc_p = torch.zeros(T, d, dtype=torch.float32, device=u.device)
+        acc_m = torch.zeros_like(acc_p) if both else None
+        for b in range(B):
+            ub = uf[b].contiguous()                              # (T,d): this row's input as the filter
+            acc_p += _causal_conv(gpf[b:b + 1], ub)[0]
+            if both:
+                acc_m += _causal_conv(gmf[b:b + 1], ub)[0]
+        gv = torch.zeros(L, d, dtype=torch.float32, device=u.device)
+        gv[:taps] = acc_p.flip(0)[:taps]                         # lag s sits at position T-1-s
+        if both:
+            gv[:taps] += acc_m.flip(0)[:taps] * _alt_sign(taps, acc_m)
+        gv = gv.to(v.dtype)
+    return gu, gv
+
+
+class _ApproxConvolve(torch.autograd.Function):
+    """Both sign branches of the approx-mode convolution with their gradients."""
 
     @staticmethod
     def forward(ctx, u, v, both):
-        ctx.save_for_backward(u, v)
+        from .. import _hip
         ctx.both = both
-        up = _causal_conv(u, v)
+        n = _conv_length(u.shape[1])
+        spec = _hip.stu_fft_filter(v.contiguous(), n) if n else None
+        ctx.save_for_backward(u, v, spec)
+        up = _hip.stu_conv_fft(u.contiguous(), spec, single_branch=True) if n else _causal_conv(u, v)
         if not both:
             return up, torch.zeros(0, dtype=u.dtype, device=u.device)
         return up, _causal_conv(u, v * _alt_sign(v.shape[0], v))
 
     @staticmethod
     def backward(ctx, gp, gm):
-        u, v = ctx.saved_tensors
-        B, T, d = u.shape
-        L = v.shape[0]
-        uf, vf = u.float(), v.float()
-        gpf = gp.float().flip(1).contiguous()
-        gmf = gm.float().flip(1).contiguous() if ctx.both else None
-        gu = gv = None
-        if ctx.needs_input_grad[0]:
-            gu = _causal_conv(gpf, vf)
-            if ctx.both:
-                gu = gu + _causal_conv(gmf, vf * _alt_sign(L, vf))
-            gu = gu.flip(1).to(u.dtype)
-        if ctx.needs_input_grad[1]:
-            taps = min(L, T)
-            acc_p = torch.zeros(T, d, dtype=torch.float32, device=u.device)
-            acc_m = torch.zeros_like(acc_p) if ctx.both else None
-            for b in range(B):
-                ub = uf[b].contiguous()                              # (T,d): this row's input as the filter
-                acc_p += _causal_conv(gpf[b:b + 1], ub)[0]
-                if ctx.both:
-                    acc_m += _causal_conv(gmf[b:b + 1], ub)[0]
-            gv = torch.zeros(L, d, dtype=torch.float32, device=u.device)
-            gv[:taps] = acc_p.flip(0)[:taps]                         # lag s sits at position T-1-s
-            if ctx.both:
-                gv[:taps] += acc_m.flip(0)[:taps] * _alt_sign(taps, acc_m)
-            gv = gv.to(v.dtype)
-        return gu, gv, None
+        u, v, spec = ctx.saved_tensors
+        return (*_convolve_grads(ctx, u, v, spec, gp, gm, 2 if ctx.both else 1), None)
+
+
+class ApproxConvolveSum(torch.autograd.Function):
+    """y = T(T(plus) + T(minus)) of the approx-mode convolution, as the STU adds its branches (stu.py:120), with its
+    gradients.  The odd lags cancel between the branches but for rounding, so they get none."""
+
+    @staticmethod
+    def forward(ctx, u, v):
+        from .. import _hip
+        n = _conv_length(u.shape[1])
+        spec = _hip.stu_fft_filter(v.contiguous(), n) if n else None
+        ctx.save_for_backward(u, v, spec)
+        if n:
+            return _hip.stu_conv_fft(u.contiguous(), spec)
+        return _hip.stu_conv_direct(u.contiguous(), v.contiguous())
+
+    @staticmethod
+    def backward(ctx, gy):
+        u, v, spec = ctx.saved_tensors
+        return _convolve_grads(ctx, u, v, spec, gy, None, 0)
 
 
 def convolve(u: torch.Tensor, v: torch.Tensor, n: int, use_approx: bool = True, return_both: bool = True,

@@ -276,6 +276,13 @@ int fstu_stu_conv_fft(const void* xp, const float* spec, void* y, const float* t
  * channels x batch rows), where the channel-contiguous kernel leaves compute units idle. */
 int fstu_stu_conv_fft_strided(const void* xp, const int64_t* x_strides, const float* spec, void* y, const int64_t* y_strides,
                               const float* tw, int B, int T, int d, int n, int single_branch, int dtype, void* stream);
+/* Gradients of the convolution: g1, g2 (B,T,d) those of the plus and minus branch (branches = 2), g1 alone that of the plus
+ * branch (branches = 1) or that of y = plus + minus (branches = 0), x (B,T,d) the forward input, spec (d, n) the filters'
+ * spectra.  Writes gx (B,T,d) and gf (L,d), each in dtype and skipped where null; gf needs x and part, fp32 scratch of
+ * fstu_stu_conv_fft_grad_ws elements.  Sums in fp32, one rounding at the end, the same bits every time. */
+int64_t fstu_stu_conv_fft_grad_ws(int B, int T, int d, int L, int branches);
+int fstu_stu_conv_fft_grad(const void* g1, const void* g2, const void* x, const float* spec, void* gx, void* gf, float* part,
+                           const float* tw, int B, int T, int d, int L, int n, int branches, int dtype, void* stream);
 /* out[b][c][r] = in[b][r][c] for (B,R,C) tensors in either dtype (out must not be in): the copy that hands (B,L,d)
  * activations to fstu_stu_conv_fft_strided as time-major slabs and takes the result back. */
 int fstu_transpose(const void* in, void* out, int B, int R, int C, int dtype, void* stream);

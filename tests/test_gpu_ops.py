@@ -521,6 +521,39 @@ def test_convolve_operator_gradients(hip, B, T, d, L, both):
         convolve(ud, dev(torch.randn(L, 4)), n, use_approx=False)
 
 
+@pytest.mark.parametrize("branches", [0, 1, 2])
+@pytest.mark.parametrize("dtype,B,T,d,L", [(torch.float32, 2, 32, 5, 40), (torch.bfloat16, 1, 33, 32, 20), (torch.bfloat16, 3, 101, 24, 128),
+                                           (torch.float32, 2, 200, 12, 199), (torch.bfloat16, 2, 511, 16, 512), (torch.float32, 1, 1000, 6, 1024),
+                                           (torch.bfloat16, 2, 2047, 12, 2048), (torch.bfloat16, 1, 4095, 5, 4096),
+                                           (torch.float32, 1, 4097, 4, 8192)])
+def test_convolution_gradient_kernel(hip, dtype, B, T, d, L, branches):
+    """Input and filter gradients at every transform length, whole and ragged channel pieces, filters shorter and longer
+    than the input, against float64 sums.  The operands are exact; the sums are fp32 transforms (some 1e-6 of the result's
+    scale) and each result is rounded once to the dtype: bf16 has 8 significant bits, half a unit is at most 2^-8 of it."""
+    g = gen(T + branches)
+    x, g1, g2 = (torch.randn(B, T, d, generator=g).to(dtype) for _ in range(3))
+    f = (torch.randn(L, d, generator=g) / L ** 0.5).to(dtype)
+    xd, a, b, fd = x.double(), g1.double(), g2.double(), f.double()
+    even, odd = (2 * a, 0 * a) if branches == 0 else (a, a) if branches == 1 else (a + b, a - b)
+    n = 2 * max(T, L)
+    sgn = (torch.arange(L) % 2 == 0).double()[:, None]
+
+    def corr(p, q):                       # sum_t p[t + s] q[t] for s >= 0
+        return torch.fft.irfft(torch.fft.rfft(p, 2 * n, 1) * torch.fft.rfft(q, 2 * n, 1).conj(), 2 * n, 1)
+    gx = (corr(even, (fd * sgn)[None]) + corr(odd, (fd * (1 - sgn))[None]))[:, :T]
+    gf = (corr(even, xd)[:, :L] * sgn + corr(odd, xd)[:, :L] * (1 - sgn)).sum(0)
+    spec = hip.stu_fft_filter(dev(f), hip.fft_length(T))
+    run = lambda *w: hip.stu_conv_fft_grad(dev(g1), dev(g2) if branches == 2 else None, dev(x), spec, L, branches, *w)
+    gxd, gfd = run()
+    half_ulp = 2.0 ** -8 if dtype == torch.bfloat16 else 0.0
+    for got, want in ((gxd, gx), (gfd, gf)):
+        bound = half_ulp * want.abs() + 1e-5 * float(want.abs().max())
+        assert bool(((got.cpu().double() - want).abs() <= bound).all())
+    only_x, none_f = run(True, False)
+    none_x, only_f = run(False, True)
+    assert none_f is None and none_x is None and torch.equal(only_x, gxd) and torch.equal(only_f, gfd)
+
+
 def _fit_lds(filt_even, S):
     """ridge fit of the even-lag filter by S real poles (host-side helper of the product)."""
     from flash_stu.utils.lds_fit import fit_even_lag_lds
