@@ -444,4 +444,4 @@ class STU(nn.Module):
 def _hist_nsplit(nlags: int) -> int:
     """Lag ranges per (batch) for the history kernel: enough workgroups to pull
     bandwidth without making the partial-sum traffic comparable to the history."""
-    return max(1, min(16, nlags // 64))
+    return max(1, min(16, nlags // 16))

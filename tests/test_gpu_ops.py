@@ -554,6 +554,36 @@ def test_convolution_gradient_kernel(hip, dtype, B, T, d, L, branches):
     assert none_f is None and none_x is None and torch.equal(only_x, gxd) and torch.equal(only_f, gfd)
 
 
+@pytest.mark.parametrize("rows", [1, 2, 3, 5, 8, 9, 16])
+@pytest.mark.parametrize("N,K", [(1, 4), (7, 252), (258, 256), (130, 260), (33, 1028), (16389, 264)])
+def test_linear_fp32_rows(hip, rows, N, K):
+    """The fp32 skinny kernels (plain, gate/up, split K, greedy head) on both sides of their chunk and row-count edges.  A sum
+    of K products of fp32 operands in any order is within K * 2^-24 of its absolute sum; 4 units more for the roundings of the
+    epilogue, whose derivatives stay below 2."""
+    g = gen(rows * 1000 + N)
+    x, W, U = (torch.randn(*s, generator=g) for s in ((rows, K), (N, K), (N, K)))
+    xd, Wd, Ud = dev(x), dev(W), dev(U)
+    ref, refu = x.double() @ W.double().t(), x.double() @ U.double().t()
+    tol, tolu = ((K + 4) * 2.0 ** -24 * (x.abs().double() @ M.abs().double().t()) for M in (W, U))
+    y = hip.linear_decode(xd, Wd).cpu().double()
+    assert bool(((y - ref).abs() <= tol).all())
+    act = hip.glu_decode(xd, Wd, Ud).cpu().double()
+    ge = torch.nn.functional.gelu(ref, approximate="tanh")
+    assert bool(((act - ge * refu).abs() <= 2 * tol * refu.abs() + tolu * ge.abs() + 2 * tol * tolu + 1e-6 * (1 + ge.abs() * refu.abs())).all())
+    for ks in (1, 3, min(K, 8)):
+        part = torch.full((ks, rows, N), float("nan"), device="cuda")
+        hip._check(hip.load().fstu_linear_decode_splitk(xd.data_ptr(), K, Wd.data_ptr(), part.data_ptr(), rows, N, K, ks,
+                                                        hip.FSTU_F32, hip._stream()), "splitk")
+        assert bool(((part.double().sum(0).cpu() - ref).abs() <= tol).all())
+    for temperature in (1.0, 0.7):
+        ws, toks = torch.zeros(rows * 64, dtype=torch.int64, device="cuda"), torch.zeros(rows, 2, dtype=torch.int64, device="cuda")
+        W2 = torch.cat([Wd, Wd[:1]])                                  # the last row repeats the first: the lower index wins
+        logits = hip.head_argmax(xd, W2, toks[:, 1], ws, temperature)
+        assert torch.equal(logits[:, :N].cpu().double(), y) and torch.equal(logits[:, N], logits[:, 0])
+        t = (logits / temperature).clamp(-1e4, 1e4)
+        assert torch.equal(toks[:, 1].cpu(), (t == t.max(1, keepdim=True).values).int().argmax(1).cpu()) and int(ws.abs().max()) == 0
+
+
 def _fit_lds(filt_even, S):
     """ridge fit of the even-lag filter by S real poles (host-side helper of the product)."""
     from flash_stu.utils.lds_fit import fit_even_lag_lds
