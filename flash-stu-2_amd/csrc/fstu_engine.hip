@@ -260,8 +260,8 @@ static int decode_step_wide(const fstu_model_desc* m, const int64_t* tok_in, int
 // kernel reads {pos, step} from that device int[2]; tok_in/tok_out are then the bases of token columns 0 and 1.
 static int decode_step_impl(const fstu_model_desc* m, const int64_t* tok_in, int64_t* tok_out, int64_t tok_stride,
                             int pos, float temperature, int top_k, float top_p, int do_sample, uint64_t seed,
-                            int step, int* dyn, void* stream) {
-  FSTU_REQUIRE(m && tok_in && tok_out, FSTU_ENULL, "fstu_decode_step: null pointer");
+                            int step, int* dyn, void* stream, bool logits_only = false) {
+  FSTU_REQUIRE(m && tok_in && (tok_out || logits_only), FSTU_ENULL, "fstu_decode_step: null pointer");
   FSTU_REQUIRE(dyn == nullptr || m->stu_mode == 1, FSTU_EARG, "fstu_decode_step: graph replay needs the recurrence (lds) STU state");
   FSTU_REQUIRE(m->layers && m->emb && m->final_norm_w && m->x && m->h && m->act && m->partial && m->logits,
                FSTU_ENULL, "fstu_decode_step: incomplete model descriptor");
@@ -383,6 +383,10 @@ static int decode_step_impl(const fstu_model_desc* m, const int64_t* tok_in, int
     }
     TIMED(PC_NORM, fstu_add_rmsnorm(xc, m->partial, 1, nsl, 0, next_w, m->h, B, d, m->eps, dt, stream));
   }
+  if (logits_only) {
+    TIMED(PC_HEAD, fstu_linear_decode(m->h, d, m->emb, m->logits, m->V, B, m->V, d, dt, stream));
+    return FSTU_OK;
+  }
   // the head over the packed copy of the embedding where the model holds one: a workgroup keeps the activations in
   // registers for its whole share of the vocabulary and issues one atomic per row (768-d, 8 rows: 14.2 us against
   // 17.4 us for the row-major kernel, whose workgroups own 16 vocabulary rows each)
@@ -414,6 +418,13 @@ extern "C" int fstu_decode_step(const fstu_model_desc* m, const int64_t* tok_in,
                                 int step, void* stream) {
   return decode_step_impl(m, tok_in, tok_out, tok_stride, pos, temperature, top_k, top_p, do_sample, seed, step, nullptr,
                           stream);
+}
+
+// The step without the pick, for callers that choose their tokens themselves.  A layer at a time from the host the same
+// step was 94 launches at the host's pace (768-d, 12 layers, 4 rows: 1.33 ms per position of which the GPU worked 0.53).
+extern "C" int fstu_decode_logits(const fstu_model_desc* m, const int64_t* tok_in, int64_t tok_stride, int pos, void* stream) {
+  FSTU_REQUIRE(m && m->B <= FSTU_MAX_DECODE_ROWS, FSTU_ESHAPE, "fstu_decode_logits: 1..%d rows", FSTU_MAX_DECODE_ROWS);
+  return decode_step_impl(m, tok_in, nullptr, tok_stride, pos, 1.f, 0, 0.f, 1, 0, 0, nullptr, stream, true);
 }
 
 // ---------------------------------------------------------------- one step as a replayable HIP graph

@@ -21,6 +21,10 @@ import torch
 from . import _hip
 from .layers.attention_layer import AttentionLayer
 from .layers.stu_layer import STULayer
+from .modules.attention import Attention
+from .modules.norm import RMSNorm
+from .modules.stu import STU
+from .modules.swiglu import MLP
 
 _vp, _i, _f = ctypes.c_void_p, ctypes.c_int, ctypes.c_float
 
@@ -53,6 +57,127 @@ def pick_ksplit_down(I: int) -> int:
         if I % (ks * 64) == 0:
             return ks
     return 1
+
+
+def _as_written(m, cls) -> bool:
+    """The module is of this class and calling it runs this class's forward and nothing else."""
+    return type(m) is cls and not m._forward_hooks and not m._forward_pre_hooks and "forward" not in m.__dict__
+
+
+@torch.no_grad()
+def step_on_caches(model, ids: torch.Tensor, past):
+    """One position of each row, ids (B,1), against the caches that model(..., use_cache=True) returned: (logits (B,1,V),
+    caches one position on) through the one-call step, the state in the caches advanced in place, or None where a row
+    count, a configuration, a cache or a module is not what that step takes (the layers' own forward calls then run).
+
+    Everything is read from the model and the caches of this call: no pointer or check outlives it, and the weights are
+    the parameters themselves, not packed copies."""
+    cfg = model.config
+    mod = torch.nn.modules.module
+    if not (ids.dim() == 2 and ids.shape[1] == 1 and 1 <= ids.shape[0] <= _hip.MAX_DECODE_ROWS and ids.dtype == torch.int64
+            and DecodeEngine.supports(cfg) and isinstance(past, (tuple, list)) and len(past) == len(model.layers) > 0
+            and not mod._global_forward_hooks and not mod._global_forward_pre_hooks and _as_written(model.norm, RMSNorm)):
+        return None
+    emb = model.lm_head.weight
+    dt, dev, B, (V, d) = emb.dtype, emb.device, ids.shape[0], emb.shape
+    H, W, eps, cap0 = cfg.n_heads, cfg.window_left, cfg.rms_norm_eps, float(cfg.softcap or 0.0)
+    n, lds = len(model.layers), cfg.resolved_stu_decode_mode() == "lds"
+    if (dt not in (torch.bfloat16, torch.float32) or not emb.is_cuda or ids.device != dev or model.tok_emb.weight is not emb
+            or model.lm_head.bias is not None or d != cfg.n_embd or d % H != 0 or model.norm.eps != eps):
+        return None
+    I, hd = d * cfg.mlp_scale, d // H
+    good = True
+
+    def ptr(t, *shape, dtype=dt):
+        nonlocal good
+        good = good and t is not None and t.dtype == dtype and t.device == dev and t.shape == shape and t.is_contiguous()
+        return t.data_ptr() if good else None
+    arr = (LayerDesc * n)()
+    keep, out = [], []
+    pos = hist_cap = fir_taps = None
+    S = 0
+    for layer, ld, entry in zip(model.layers, arr, past):
+        stu_layer = type(layer) is STULayer
+        if not _as_written(layer, STULayer if stu_layer else AttentionLayer) or not isinstance(entry, tuple) or len(entry) != 3:
+            return None
+        op, norm1 = (layer.stu, layer.stu_norm) if stu_layer else (layer.attn, layer.attn_norm)
+        mlp, norm2 = layer.mlp, layer.mlp_norm
+        if not (_as_written(op, STU if stu_layer else Attention) and _as_written(norm1, RMSNorm) and type(norm2) is RMSNorm
+                and _as_written(mlp, MLP) and norm1.eps == eps and norm2.eps == eps and mlp.gate_proj.bias is None):
+            return None
+        a0, a1, pos_t = entry
+        if pos_t.is_cuda or pos_t.dim() != 1 or pos_t.numel() < 1:
+            return None
+        p = int(pos_t[0])
+        if pos is not None and p != pos:
+            return None
+        pos = p
+        ld.norm1_w, ld.mlp_norm_w = ptr(norm1.weight, d), ptr(norm2.weight, d)
+        ld.w_gate, ld.w_up, ld.w_down = ptr(mlp.gate_proj.weight, I, d), ptr(mlp.up_proj.weight, I, d), ptr(mlp.down_proj.weight, d, I)
+        if not stu_layer:
+            ld.kind = 1
+            if op.n_heads != H or op.window_size != W or op.softcap != cap0 or op.c_attn.bias is not None or op.c_proj.bias is not None:
+                return None
+            ld.w_qkv, ld.w_proj = ptr(op.c_attn.weight, 3 * d, d), ptr(op.c_proj.weight, d, d)
+            ld.kring, ld.vring = ptr(a0, B, H, W + 1, hd), ptr(a1, B, H, W + 1, hd)
+            ld.slopes = ptr(op.alibi_slopes, H, dtype=torch.float32)
+        else:
+            if op.M_inputs.device != dev or op.d_in != d or op.config is not cfg:
+                return None
+            mit = op.m_inputs_t()
+            keep.append(mit)
+            ld.m_inputs_t = ptr(mit, d, d)
+            if lds:
+                a, ce, co = op.lds_params()
+                fir = op.lds_fir()
+                taps = fir.shape[0] if fir is not None and a0.shape[1] == fir.shape[0] else 0
+                if fir_taps not in (None, taps) or S not in (0, a.numel()) or (taps == 0 and a0.numel() != 0):
+                    return None
+                fir_taps, S = taps, a.numel()
+                keep += [a, ce, co, fir]
+                ld.lds_a, ld.lds_ce, ld.lds_co = (ptr(a, S, dtype=torch.float32), ptr(ce, S, d, dtype=torch.float32),
+                                                  ptr(co, S, d, dtype=torch.float32))
+                ld.lds_state = ptr(a1, B, 2, S, d, dtype=torch.float32)
+                if taps:
+                    ld.lds_ring, ld.lds_fir = ptr(a0, B, taps, d), ptr(fir, taps, d, dtype=torch.float32)
+            else:
+                filt = op.effective_filter()
+                if a0.dim() != 3 or hist_cap not in (None, a0.shape[1]) or a1.numel() != 0 or pos >= a0.shape[1] or pos >= filt.shape[0]:
+                    return None
+                hist_cap = a0.shape[1]
+                keep.append(filt)
+                ld.filt, ld.hist = ptr(filt, filt.shape[0], d), ptr(a0, B, hist_cap, d)
+                S = filt.shape[0]
+        if not good:
+            return None
+        out.append((a0, a1, pos_t))
+    m = ModelDesc()
+    m.dtype = _hip.FSTU_BF16 if dt == torch.bfloat16 else _hip.FSTU_F32
+    m.B, m.d, m.I, m.V, m.n_layers = B, d, I, V, n
+    m.n_heads, m.head_dim, m.window, m.kv_cap = H, hd, W, W + 1
+    m.L, m.hist_cap, m.stu_mode, m.lds_S = (cfg.seq_len if lds else S), hist_cap or 0, int(lds), (S if lds else 0)
+    m.lds_fir_taps, m.single_branch = fir_taps or 0, int(cfg.use_hankel_L)
+    m.ksplit_down = pick_ksplit_down(I) if dt == torch.bfloat16 else min(8, max(1, I // 512))
+    m.hist_nsplit_max = DecodeEngine.HIST_NSPLIT_MAX
+    m.eps, m.softcap = float(eps), cap0
+    m.emb, m.final_norm_w = ptr(emb, V, d), ptr(model.norm.weight, d)
+    if not good or pos < 0:
+        return None
+    m.layers = ctypes.cast(arr, ctypes.POINTER(LayerDesc))
+    logits = torch.empty(B, 1, V, dtype=dt, device=dev)
+    m.logits = logits.data_ptr()
+    esz = emb.element_size()
+    sizes = dict(x=B * d * esz, h=B * d * esz, y=B * d * esz, xp=B * d * esz, attn=B * d * esz, qkv=3 * B * d * esz,
+                 act=B * I * esz, partial=max(m.ksplit_down, 16) * B * d * 4,
+                 eo=0 if lds else DecodeEngine.HIST_NSPLIT_MAX * 2 * B * d * 4)
+    ws = torch.empty(sum((v + 255) // 256 * 256 for v in sizes.values()), dtype=torch.uint8, device=dev)
+    at = ws.data_ptr()
+    for name, size in sizes.items():
+        setattr(m, name, at)
+        at += (size + 255) // 256 * 256
+    _hip._check(_hip.load().fstu_decode_logits(ctypes.byref(m), ids.data_ptr(), ids.stride(0), pos, _hip._stream()),
+                "fstu_decode_logits")
+    return logits, tuple((a0, a1, pos_t + 1) for a0, a1, pos_t in out)
 
 
 class _Chunk:

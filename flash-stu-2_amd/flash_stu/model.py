@@ -156,7 +156,16 @@ class FlashSTU(nn.Module):
         if not input_ids.is_cuda:
             raise _hip.FlashSTUHipError("input_ids must be on the GPU: this model has no CPU path")
         hidden = [] if output_hidden_states else None
-        if past_key_values is not None and input_ids.shape[1] > 1:
+        logits = None
+        if past_key_values is not None and hidden is None and input_ids.dim() == 2 and input_ids.shape[1] == 1:
+            from .engine import step_on_caches
+            done = step_on_caches(self, input_ids, past_key_values)
+            if done is not None:
+                logits, cache = done
+                cache = cache if use_cache else None
+        if logits is not None:
+            pass
+        elif past_key_values is not None and input_ids.shape[1] > 1:
             outs = []
             cache = past_key_values
             for t in range(input_ids.shape[1]):
@@ -171,9 +180,10 @@ class FlashSTU(nn.Module):
                 hidden.append(x.clone())
             x, cache = self._run_layers(x, past_key_values, use_cache, hidden)
             xn = self.norm(x)
-        if kwargs.get("last_only"):        # generate() needs the newest position only (the reference computes all)
-            xn = xn[:, -1:, :].contiguous()
-        logits = self._head(xn)
+        if logits is None:
+            if kwargs.get("last_only"):        # generate() needs the newest position only (the reference computes all)
+                xn = xn[:, -1:, :].contiguous()
+            logits = self._head(xn)
         loss = None
         if labels is not None:
             sl = logits[..., :-1, :].contiguous()

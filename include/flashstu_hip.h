@@ -598,6 +598,8 @@ typedef struct {
 int fstu_decode_step(const fstu_model_desc* m, const int64_t* tok_in, int64_t* tok_out, int64_t tok_stride,
                      int pos, float temperature, int top_k, float top_p, int do_sample, uint64_t seed,
                      int step, void* stream);
+/* The same step without the pick: the state advances and m->logits holds the (B,V) logits; 1..16 rows. */
+int fstu_decode_logits(const fstu_model_desc* m, const int64_t* tok_in, int64_t tok_stride, int pos, void* stream);
 
 /* One decode step captured as a HIP graph that can be replayed for every position:
  * the position-dependent kernels read {position, sampling step} from `dyn`, a

@@ -326,6 +326,46 @@ def test_forward_full_sequence_and_stepwise_cache(dtype):
     assert torch.equal(re[1][0][0], cache[1][0][1])
 
 
+@pytest.mark.parametrize("rows", [1, 3, 16])
+@pytest.mark.parametrize("dtype,extra", [(torch.float32, dict(n_embd=96, n_heads=3)), (torch.float32, dict(use_hankel_L=True)),
+                                         (torch.bfloat16, dict(n_embd=256)), (torch.bfloat16, dict(n_embd=96, n_heads=3)),
+                                         (torch.bfloat16, dict(stu_lds_fir_taps=0, softcap=0.0)), (torch.bfloat16, dict(use_attn=False)),
+                                         (torch.bfloat16, dict(stu_decode_mode="history"))])
+def test_one_call_step_equals_the_layers_own_calls(dtype, extra, rows):
+    """forward() with caches for one position: the one-call step against the layers' forward calls (a hook that does nothing
+    keeps those in use), logits and caches, over the edges of the prompt's fill of rings and of the row range."""
+    from flash_stu import engine
+    kw = dict(mlp_scale=2, n_embd=128, n_layers=4, n_heads=2, window_size=8, num_eigh=8, seq_len=64, vocab_size=777)
+    _, _, model = make_pair(seed=5, init="healthy", dtype=dtype, **{**kw, **extra})
+    ids = prompt(rows, 14, 777, 6).cuda()
+    caches = {}
+    for how in ("one", "layers"):
+        hook = model.norm.register_forward_hook(lambda *a: None) if how == "layers" else None
+        out = model(ids[:, :6], use_cache=True)
+        logits, past = [out.logits[:, -1:]], out.past_key_values
+        assert (engine.step_on_caches(model, ids[:, 6:7], tuple(tuple(t.clone() for t in c) for c in past)) is None) == (how == "layers")
+        for t in range(6, 14):
+            out = model(ids[:, t:t + 1], past_key_values=past, use_cache=True)
+            assert out.logits.shape == (rows, 1, 777)
+            logits.append(out.logits)
+            past = out.past_key_values
+        caches[how] = (torch.cat(logits, 1), past)
+        if hook is not None:
+            hook.remove()
+    # sums in another order: fp32 as the forward tests hold it; bf16 a few roundings of 2^-8 that pass through four layers
+    tol = 1e-4 if dtype == torch.float32 else 2e-2
+    (la, ca), (lb, cb) = caches["one"], caches["layers"]
+    assert float((la.float() - lb.float()).abs().max()) <= tol * float(lb.float().abs().max())
+    for i, (ea, eb) in enumerate(zip(ca, cb)):
+        attn = len(ea) == 3 and ea[0].dim() == 4
+        for a, b in zip(ea, eb):
+            if attn and a.dim() == 4:                            # slots beyond the last position are not written
+                a, b = a[:, :, :min(14, 9)], b[:, :, :min(14, 9)]
+            assert a.shape == b.shape and a.dtype == b.dtype
+            if a.numel():
+                assert float((a.float() - b.float()).abs().max()) <= tol * max(float(b.float().abs().max()), 1e-6)
+
+
 def test_forward_accepts_reference_style_kv_cache():
     from flash_stu import Attention, FlashSTUConfig
     cfg = FlashSTUConfig(n_embd=128, n_heads=2, n_layers=2, seq_len=64, window_size=6, vocab_size=11, mlp_scale=2,
