@@ -391,11 +391,25 @@ __device__ __forceinline__ void store_feat8(u32x4_t v, const bf16_t* rp, bf16_t*
   }
 }
 
-template <int MODE>
+// (transposing read: in a block of 16 lanes, lane i supplies the address of 4 consecutive columns of row i/4 starting at column
+// 4*(i%4), and receives column i of the 4 rows)
+template <int OFF>
+__device__ __forceinline__ u32x2_t lds_read_tr8(unsigned addr) {
+  u32x2_t v;
+  asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(OFF));
+  return v;
+}
+struct Frag8 { u32x2_t lo, hi; };
+
+// TA: the activations are slabs with the reduction index slowest (see gemm_ta_bf16_kernel), M a multiple of 256.  Rows of an
+// X part are then 64 k of 128 columns, filled 16 bytes = 8 columns per lane and read with transposing reads, k and k + 4 of a
+// fragment's half; the 32-byte pieces of a row are XOR-ed with bits 0, 1 and 3 of k so that the eight rows that two blocks of
+// lanes read together lie in different banks.  `mts` row tiles per slab, slabs sa / sc / sr elements apart.
+template <int MODE, bool TA = false>
 __global__ void __launch_bounds__(512)
 gemm_pp_bf16_kernel(const bf16_t* __restrict__ A, long long lda, const bf16_t* __restrict__ W, const bf16_t* __restrict__ W2,
                     const bf16_t* __restrict__ R, long long ldr, bf16_t* __restrict__ C, long long ldc, int M, int N, int K,
-                    int mt, int nt, int share) {
+                    int mt, int nt, int share, int mts, long long sa, long long sc, long long sr) {
   constexpr int NF = MODE == 1 ? 128 : 256;
   extern __shared__ __align__(16) unsigned char gm_smem[];   // stage: W0 | W1 | X0 | X1
   const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -404,19 +418,29 @@ gemm_pp_bf16_kernel(const bf16_t* __restrict__ A, long long lda, const bf16_t* _
   if (idx >= share || xcd + idx >= tiles) return;
   int m0, n0;
   size_t wbytes, abytes;
-  const bf16_t *wb, *wb2, *ab;
+  const bf16_t *wb, *wb2, *ab, *rb = R;
+  bf16_t* cb = C;
 #define PP_OPEN_TILE                                                                     \
   {                                                                                      \
     const int o_ = xcd + idx;                                                            \
     const int panel_ = o_ / per_panel, in_panel_ = o_ - panel_ * per_panel;              \
     const int pw_ = min(GM_PANEL, nt - panel_ * GM_PANEL);                               \
-    m0 = in_panel_ / pw_ * 256;                                                          \
+    int bm_ = in_panel_ / pw_;                                                           \
+    ab = A;                                                                              \
+    if constexpr (TA) {                                                                  \
+      const int slab_ = bm_ / mts;                                                       \
+      bm_ -= slab_ * mts;                                                                \
+      ab += (size_t)slab_ * sa;                                                          \
+      cb = C + (size_t)slab_ * sc;                                                       \
+      if (MODE == 2) rb = R + (size_t)slab_ * sr;                                        \
+    }                                                                                    \
+    m0 = bm_ * 256;                                                                      \
     n0 = (panel_ * GM_PANEL + in_panel_ % pw_) * NF;                                     \
     wbytes = (size_t)min(NF, N - n0) * K * 2;                                            \
-    abytes = ((size_t)(min(256, M - m0) - 1) * lda + K) * 2;                             \
+    abytes = TA ? ((size_t)(K - 1) * lda + 256) * 2 : ((size_t)(min(256, M - m0) - 1) * lda + K) * 2; \
     wb = W + (size_t)n0 * K;                                                             \
     wb2 = MODE == 1 ? W2 + (size_t)n0 * K : wb;                                          \
-    ab = A + (size_t)m0 * lda;                                                           \
+    ab += TA ? (size_t)m0 : (size_t)m0 * lda;                                            \
   }
   const int wn = wv & 3, wm = wv >> 2;                 // 32-feature slice and 64-row slice of every half
   // ---- fills: part = 128 rows x 128 bytes; a wave fills rows 16 wv .. 16 wv + 15 of it with two instructions
@@ -425,16 +449,21 @@ gemm_pp_bf16_kernel(const bf16_t* __restrict__ A, long long lda, const bf16_t* _
   for (int j = 0; j < 2; ++j) {
     const int row = wv * 16 + j * 8 + (lane >> 3), ch = (lane & 7) ^ ((row >> 1) & 7);
     wvoff[j] = (unsigned)row * (unsigned)K * 2u + (unsigned)ch * 16u;
-    avoff[j] = (unsigned)row * (unsigned)lda * 2u + (unsigned)ch * 16u;
+    if constexpr (TA) {
+      const int kr = wv * 8 + j * 4 + (lane >> 4);
+      avoff[j] = (unsigned)kr * (unsigned)lda * 2u + (unsigned)((lane & 15) ^ (4 * (kr & 3)) ^ (2 * ((kr >> 3) & 1))) * 16u;
+    } else {
+      avoff[j] = (unsigned)row * (unsigned)lda * 2u + (unsigned)ch * 16u;
+    }
   }
-  const unsigned w1off = MODE == 1 ? 0u : 128u * (unsigned)K * 2u, x1off = 128u * (unsigned)lda * 2u;
+  const unsigned w1off = MODE == 1 ? 0u : 128u * (unsigned)K * 2u, x1off = TA ? 256u : 128u * (unsigned)lda * 2u;
   const int nkt = K >> 6;
   unsigned char* fill0 = gm_smem + (unsigned)wv * 2048u;
   // requests part P (0 W0, 1 X0, 2 W1, 3 X1) of k tile kt_; beyond the last tile the descriptor is empty: nothing is fetched
 #define PP_FETCH(P, kt_, stage_)                                                                                           \
   {                                                                                                                        \
     const bool in_ = (kt_) < nkt;                                                                                          \
-    const unsigned so_ = (unsigned)(kt_) * 128u;                                                                           \
+    const unsigned so_ = (unsigned)(kt_) * (TA && ((P) & 1) ? 128u * (unsigned)lda : 128u);                                 \
     unsigned char* l_ = fill0 + (stage_) * PP_STAGE + ((P) == 0 ? 0u : (P) == 2 ? PP_PART : (P) == 1 ? 2 * PP_PART : 3 * PP_PART); \
     const rsrc_t rs_ = ((P) & 1) ? make_rsrc(ab, in_ ? abytes : 0) : make_rsrc((P) == 2 ? wb2 : wb, in_ ? wbytes : 0);     \
     _Pragma("unroll") for (int j = 0; j < 2; ++j)                                                                          \
@@ -449,6 +478,15 @@ gemm_pp_bf16_kernel(const bf16_t* __restrict__ A, long long lda, const bf16_t* _
     fx_off[kk] = 2 * PP_PART + (unsigned)rx * 128u + (unsigned)((c ^ ((rx >> 1) & 7)) << 4);
   }
   const unsigned smem0 = lds_addr(gm_smem);
+  unsigned ta[4];                                      // TA: this lane's address of row tile t in an X part
+  if constexpr (TA) {
+    const int key = l16 >> 2;
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+      ta[t] = 2 * PP_PART + (unsigned)(8 * lq + key) * 256u + (unsigned)((wm * 8 + t * 2 + ((l16 & 3) >> 1)) ^ (4 * key) ^ (2 * (lq & 1))) * 16u +
+              (unsigned)(l16 & 1) * 8u;
+  }
+  u32x2_t xt[16];                                      // TA: the halves of X fragments (k step, row tile, half)
   u32x4_t wa[8], xf[8];                                // fragments: W (k step, half, feature tile), X (k step, row tile)
   floatx4_t acc[2][2][2][4];                           // [W half][feature tile][X half][row tile]
 #define PP_READ_W(stage_)                                                                              \
@@ -459,11 +497,27 @@ gemm_pp_bf16_kernel(const bf16_t* __restrict__ A, long long lda, const bf16_t* _
     wa[4 * kk + 3] = lds_read16<16384 + 2048>(smem0 + (stage_) * PP_STAGE + fw_off[kk]);               \
   }
 #define PP_READ_X(stage_, H)                                                                           \
-  _Pragma("unroll") for (int kk = 0; kk < 2; ++kk)                                                     \
-    lds_read_rows<4, 2048>(xf + 4 * kk, smem0 + (stage_) * PP_STAGE + (H) * 16384u + fx_off[kk]);
+  if constexpr (TA) {                                                                                  \
+    _Pragma("unroll") for (int t = 0; t < 4; ++t) {                                                    \
+      const unsigned a_ = smem0 + (stage_) * PP_STAGE + (H) * 16384u + ta[t];                          \
+      xt[2 * t] = lds_read_tr8<0>(a_);                                                                 \
+      xt[2 * t + 1] = lds_read_tr8<1024>(a_);                                                          \
+      xt[8 + 2 * t] = lds_read_tr8<8192>(a_);                                                          \
+      xt[8 + 2 * t + 1] = lds_read_tr8<8192 + 1024>(a_);                                               \
+    }                                                                                                  \
+  } else {                                                                                             \
+    _Pragma("unroll") for (int kk = 0; kk < 2; ++kk)                                                   \
+      lds_read_rows<4, 2048>(xf + 4 * kk, smem0 + (stage_) * PP_STAGE + (H) * 16384u + fx_off[kk]);    \
+  }
   // end of a memory phase: this wave's reads are complete, its share of the parts that the next phase reads has landed
 #define PP_MEM_END                                                                                     \
-  asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)"                                                         \
+  if constexpr (TA)                                                                                    \
+    asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)"                                                       \
+               : "+v"(xt[0]), "+v"(xt[1]), "+v"(xt[2]), "+v"(xt[3]), "+v"(xt[4]), "+v"(xt[5]), "+v"(xt[6]), "+v"(xt[7]), \
+                 "+v"(xt[8]), "+v"(xt[9]), "+v"(xt[10]), "+v"(xt[11]), "+v"(xt[12]), "+v"(xt[13]), "+v"(xt[14]), "+v"(xt[15]), \
+                 "+v"(wa[0]), "+v"(wa[1]), "+v"(wa[2]), "+v"(wa[3]), "+v"(wa[4]), "+v"(wa[5]), "+v"(wa[6]), "+v"(wa[7])::"memory"); \
+  else                                                                                                 \
+    asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)"                                                       \
                : "+v"(xf[0]), "+v"(xf[1]), "+v"(xf[2]), "+v"(xf[3]), "+v"(xf[4]), "+v"(xf[5]), "+v"(xf[6]), "+v"(xf[7]), \
                  "+v"(wa[0]), "+v"(wa[1]), "+v"(wa[2]), "+v"(wa[3]), "+v"(wa[4]), "+v"(wa[5]), "+v"(wa[6]), "+v"(wa[7])::"memory"); \
   __builtin_amdgcn_s_barrier();                                                                        \
@@ -474,7 +528,8 @@ gemm_pp_bf16_kernel(const bf16_t* __restrict__ A, long long lda, const bf16_t* _
     _Pragma("unroll") for (int i = 0; i < 4; ++i)                                                      \
       _Pragma("unroll") for (int j = 0; j < 4; ++j)                                                    \
         acc[i >> 1][i & 1][HX][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, wa[4 * kk + i]), \
-                                                                            __builtin_bit_cast(bf16x8_t, xf[4 * kk + j]), \
+                                                                            TA ? __builtin_bit_cast(bf16x8_t, Frag8{xt[8 * kk + 2 * j], xt[8 * kk + 2 * j + 1]}) \
+                                                                               : __builtin_bit_cast(bf16x8_t, xf[4 * kk + j]), \
                                                                             acc[i >> 1][i & 1][HX][j], 0, 0, 0); \
   __builtin_amdgcn_s_setprio(0);                                                                       \
   __builtin_amdgcn_sched_barrier(0);                                                                   \
@@ -512,6 +567,8 @@ gemm_pp_bf16_kernel(const bf16_t* __restrict__ A, long long lda, const bf16_t* _
     __builtin_amdgcn_s_barrier();
     // every wave has left the stages: the next tile's first k tiles are on their way while this one is stored
     const int em0 = m0, en0 = n0;
+    bf16_t* const ec = TA ? cb : C;
+    const bf16_t* const er = TA ? rb : R;
     idx += (int)(gridDim.x >> 3);
     const bool more = idx < share && xcd + idx < tiles;
     if (more) {
@@ -552,7 +609,7 @@ gemm_pp_bf16_kernel(const bf16_t* __restrict__ A, long long lda, const bf16_t* _
         for (int i = 0; i < NST; ++i) {
           const int r = (i * 256 + gl) / CH, c = gl % CH;
           const int m = em0 + hx * 128 + wm * 64 + j * 32 + r, f = en0 + c * 8;
-          if (m < M && f < N) store_feat8<MODE>(o[i], MODE == 2 ? R + (size_t)m * ldr + f : nullptr, C + (size_t)m * ldc + f, N - f);
+          if (m < M && f < N) store_feat8<MODE>(o[i], MODE == 2 ? er + (size_t)m * ldr + f : nullptr, ec + (size_t)m * ldc + f, N - f);
         }
       }
     if (!more) break;
@@ -567,16 +624,16 @@ gemm_pp_bf16_kernel(const bf16_t* __restrict__ A, long long lda, const bf16_t* _
 #undef PP_TILE
 }
 
-template <int MODE>
+template <int MODE, bool TA = false>
 int gemm_pp_launch(const void* A, long long lda, const void* W, const void* W2, const void* R, long long ldr, void* C,
-                   long long ldc, int M, int N, int K, hipStream_t s) {
+                   long long ldc, int M, int N, int K, hipStream_t s, int nbatch = 1, long long sa = 0, long long sc = 0, long long sr = 0) {
   constexpr int NF = MODE == 1 ? 128 : 256;
-  static hipError_t attr_err = hipFuncSetAttribute((const void*)gemm_pp_bf16_kernel<MODE>, hipFuncAttributeMaxDynamicSharedMemorySize, PP_LDS);
+  static hipError_t attr_err = hipFuncSetAttribute((const void*)gemm_pp_bf16_kernel<MODE, TA>, hipFuncAttributeMaxDynamicSharedMemorySize, PP_LDS);
   if (attr_err != hipSuccess) { fstu_set_error("fstu_gemm_bf16: hipFuncSetAttribute: %s", hipGetErrorString(attr_err)); return (int)attr_err; }
-  const int mt = (M + 255) / 256, nt = (N + NF - 1) / NF;
+  const int mts = (M + 255) / 256, mt = mts * nbatch, nt = (N + NF - 1) / NF;
   const int share = (int)(((long long)mt * nt + 7) / 8);
-  hipLaunchKernelGGL((gemm_pp_bf16_kernel<MODE>), dim3(8u * (unsigned)std::min(share, gemm_cus() / 8)), dim3(512), PP_LDS, s, (const bf16_t*)A, lda,
-                     (const bf16_t*)W, (const bf16_t*)W2, (const bf16_t*)R, ldr, (bf16_t*)C, ldc, M, N, K, mt, nt, share);
+  hipLaunchKernelGGL((gemm_pp_bf16_kernel<MODE, TA>), dim3(8u * (unsigned)std::min(share, gemm_cus() / 8)), dim3(512), PP_LDS, s, (const bf16_t*)A, lda,
+                     (const bf16_t*)W, (const bf16_t*)W2, (const bf16_t*)R, ldr, (bf16_t*)C, ldc, M, N, K, mt, nt, share, mts, sa, sc, sr);
   return 0;
 }
 
@@ -590,12 +647,6 @@ int gemm_pp_launch(const void* A, long long lda, const void* W, const void* W2, 
 // (ds_read_b64_tr_b16: in a block of 16 lanes, lane i supplies the address of 4 consecutive m of row i/4 starting at
 // column 4*(i%4), and receives column i of the 4 rows).  The 64-byte column groups of a row are XOR-ed with the row's
 // low two bits, so the four rows of a read fall into different banks.  `nbatch` slabs run as one grid.
-template <int OFF>
-__device__ __forceinline__ u32x2_t lds_read_tr8(unsigned addr) {
-  u32x2_t v;
-  asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(OFF));
-  return v;
-}
 template <int N, int STEP, int I = 0>
 __device__ __forceinline__ void lds_read_tr_cols(u32x2_t* f, const unsigned* addr) {   // N column tiles, rows k..k+3 and k+4..k+7
   if constexpr (I < N) {
@@ -667,7 +718,6 @@ gemm_ta_bf16_kernel(const bf16_t* __restrict__ A, long long lda, long long sa, c
     _Pragma("unroll") for (int j = 0; j < WL; ++j) buf_load16_to_lds(rs_w, wvoff[j], sw_, st_ + wslot + j * 1024); \
     _Pragma("unroll") for (int j = 0; j < AL; ++j) buf_load16_to_lds(rs_a, avoff[j], sa_, st_ + aslot + j * 1024); \
   }
-  struct Frag8 { u32x2_t lo, hi; };
 #define GT_MFMAS(fw_, fx_)                                                                                   \
   _Pragma("unroll") for (int i = 0; i < FI; ++i)                                                             \
     _Pragma("unroll") for (int j = 0; j < TJ; ++j) {                                                         \
@@ -794,7 +844,6 @@ int gemm_ta_launch_tile(const void* A, long long lda, long long sa, const void* 
 
 
 //                     waves  tiles  BK  stages
-using TileBig = GemmTile<4, 2, 2, 4, 64, 2>;     // 256 x 256, 8 waves, 128 KB of LDS (transposed activations)
 using TileSmall = GemmTile<2, 2, 2, 2, 64, 2>;   // 128 x 128, 4 waves, 64 KB: two workgroups per compute unit
 using TileDeep = GemmTile<2, 2, 2, 2, 64, 4>;    // 128 x 128, 4 waves, 3 tiles in flight: one workgroup per compute unit
 using TileRows32 = GemmTile<2, 1, 2, 1, 64, 4>;  // 128 features x 32 rows, 2 waves, 80 KB: weight streaming, two workgroups per compute unit
@@ -904,7 +953,14 @@ extern "C" int fstu_gemm_bf16_ta(const void* A, int64_t lda, int64_t batch_strid
                                             nbatch, s)                                                                           \
              : gemm_ta_launch_tile<TILE, 2>(A, lda, batch_stride_a, W, R, ldr, batch_stride_r, C, ldc, batch_stride_c, M, N, K,  \
                                             nbatch, s))
-  if (M % 256 == 0 && K >= 1024 && big >= 2 * gemm_cus()) rc = TA_GO(TileBig);
+  // The line between the tiles is gemm_launch's (a round of large tiles against 2.25 of small ones).  Large / 128 x 128 tiles
+  // (or 256 x 256 tiles all in step, the form before), us, K = 24 N: 4 x 8192 x 1024 (512 large tiles) 1155 / 1475, 2 x 8192 x
+  // 1024 (256) 547 / 833, 4 x 8192 x 768 (384) 758 / 880, 4 x 8192 x 512 (256) 295 / 458, 4 x 2048 x 1024 (128) 432 / 453,
+  // 1 x 8192 x 1024 (128) 443 / 440, 1 x 4096 x 768 (48) 176 / 179.
+  const long long small = (long long)(M / 128) * ((N + 127) / 128) * nbatch;
+  if (M % 256 == 0 && 9 * ((big + gemm_cus() - 1) / gemm_cus()) * gemm_cus() < 4 * small)
+    rc = mode == 0 ? gemm_pp_launch<0, true>(A, lda, W, nullptr, R, ldr, C, ldc, M, N, K, s, nbatch, batch_stride_a, batch_stride_c, batch_stride_r)
+                   : gemm_pp_launch<2, true>(A, lda, W, nullptr, R, ldr, C, ldc, M, N, K, s, nbatch, batch_stride_a, batch_stride_c, batch_stride_r);
   else rc = TA_GO(TileSmall);
 #undef TA_GO
   if (rc) return rc;

@@ -229,6 +229,25 @@ def test_gemm_bf16_transposed_activations(hip, nb, M, N, K):
         hip.gemm_ta(Ad.transpose(1, 2), Wd)  # M not the contiguous index
 
 
+@pytest.mark.parametrize("nb,M,N,K", [(1, 4096, 2308, 128), (3, 2048, 1540, 64), (1, 4096, 2304, 320)])
+def test_gemm_bf16_transposed_activations_large_tiles(hip, nb, M, N, K):
+    """The 256 x 256 tiles over slabs: one k tile, an even and an odd number of them, several slabs and tiles per workgroup, a
+    ragged last feature tile, rows in a wider buffer.  fp32 sums of exact products in any order stay within K * 2^-24 of the
+    absolute sum; one rounding to bf16 (2^-8 of the value), a second one with the residual."""
+    g = gen(K)
+    A, W = dev(torch.randn(nb, K, M, generator=g).bfloat16()), dev(torch.randn(N, K, generator=g).bfloat16())
+    R = dev(torch.randn(nb, M, N, generator=g).bfloat16())
+    ref = torch.stack([A[b].double().t() @ W.double().t() for b in range(nb)])
+    mag = torch.stack([A[b].double().abs().t() @ W.double().abs().t() for b in range(nb)])
+    bound = K * 2.0 ** -24 * mag + 2.0 ** -8 * ref.abs()
+    got = hip.gemm_ta(A, W)
+    assert bool(((got.double() - ref).abs() <= bound).all())
+    assert torch.equal(hip.gemm_ta(A, W, residual=R), (R.float() + got.float()).bfloat16())
+    wide = torch.full((nb, K, M + 64), float("nan"), dtype=torch.bfloat16, device="cuda")
+    wide[:, :, :M] = A
+    assert torch.equal(hip.gemm_ta(wide[:, :, :M], W), got)
+
+
 @pytest.mark.parametrize("M,d,I", [(4096, 768, 3072), (300, 256, 1000), (2048, 1024, 8192), (100, 96, 132)])
 def test_gemm_bf16_gated_pair(hip, M, d, I):
     """Mode 1: T(T(gelu_tanh(T(x Wg^T))) * T(x Wu^T)) in one kernel equals the three-step bf16 chain of the reference
