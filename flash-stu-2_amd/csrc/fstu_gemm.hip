@@ -670,32 +670,34 @@ template <class G, int MODE>
 __global__ void __launch_bounds__(G::THREADS)
 gemm_ta_bf16_kernel(const bf16_t* __restrict__ A, long long lda, long long sa, const bf16_t* __restrict__ W,
                     const bf16_t* __restrict__ R, long long ldr, long long sr, bf16_t* __restrict__ C, long long ldc,
-                    long long sc, int M, int N, int K, int mt, int nt, int share, int nbatch) {
+                    long long sc, int M, int N, int K, int mt, int nt, int share, int nbatch, int ksplit) {
   constexpr int FI = G::FI, TJ = G::TJ, BF = G::BF, BT = G::BT, WL = G::WL, AL = G::AL, NS = G::NS, KK = G::KK;
   constexpr unsigned STAGE = G::STAGE;
   constexpr int RBT = BT * 2, CPRT = BT / 8;              // bytes and 16-byte chunks of an activation row (one k)
   constexpr int NRD = FI + 2 * TJ;                        // LDS reads per k step
   static_assert(G::BK == 64 && BT >= 128, "k tile of 64, at least 128 columns");
-  static_assert((MODE == 0 || MODE == 2), "plain or residual epilogue");
+  static_assert((MODE == 0 || MODE == 2 || MODE == 3), "plain, residual or split-K epilogue");
   extern __shared__ __align__(16) unsigned char gm_smem[];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int wf = w % G::WFN, wt = w / G::WFN;
   int o = (int)(blockIdx.x & 7) * share + (int)(blockIdx.x >> 3);
-  if ((int)(blockIdx.x >> 3) >= share || o >= mt * nt * nbatch) return;
-  const int batch = o / (mt * nt);
-  o -= batch * (mt * nt);
+  if ((int)(blockIdx.x >> 3) >= share || o >= mt * nt * nbatch * ksplit) return;
+  const int bs = o / (mt * nt), slice = bs / nbatch, batch = bs - slice * nbatch;    // MODE 3: slices of K outermost
+  o -= bs * (mt * nt);
+  const int KS = MODE == 3 ? K / ksplit : K;           // this workgroup's share of K
   const int per_panel = mt * GM_PANEL;
   const int panel = o / per_panel, in_panel = o - panel * per_panel;
   const int pw = min(GM_PANEL, nt - panel * GM_PANEL);
   const int bt = in_panel / pw, bf = panel * GM_PANEL + in_panel % pw;
   const int m0 = bt * BT, n0 = bf * BF;
-  A += (size_t)batch * sa;
+  A += (size_t)batch * sa + (MODE == 3 ? (size_t)slice * KS * lda : 0);
+  if (MODE == 3) W += (size_t)slice * KS;
   C += (size_t)batch * sc;
   if (MODE == 2) R += (size_t)batch * sr;
   const int wv = __builtin_amdgcn_readfirstlane(w);
   const int rows_w = min(BF, N - n0);
-  const rsrc_t rs_w = make_rsrc(W + (size_t)n0 * K, (size_t)rows_w * K * 2);
-  const rsrc_t rs_a = make_rsrc(A + m0, ((size_t)(K - 1) * lda + BT) * 2);     // M % BT == 0: whole rows of BT columns
+  const rsrc_t rs_w = make_rsrc(W + (size_t)n0 * K, ((size_t)(rows_w - 1) * K + KS) * 2);
+  const rsrc_t rs_a = make_rsrc(A + m0, ((size_t)(KS - 1) * lda + BT) * 2);    // M % BT == 0: whole rows of BT columns
   unsigned wvoff[WL], avoff[AL];
 #pragma unroll
   for (int j = 0; j < WL; ++j) {
@@ -743,7 +745,7 @@ gemm_ta_bf16_kernel(const bf16_t* __restrict__ A, long long lda, long long sa, c
     for (int j = 0; j < TJ; ++j)
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
-  const int nkt = K / G::BK;
+  const int nkt = KS / G::BK;
   constexpr int LPT = WL + AL;
 #pragma unroll
   for (int t = 0; t < NS - 1; ++t)
@@ -817,6 +819,10 @@ gemm_ta_bf16_kernel(const bf16_t* __restrict__ A, long long lda, long long sa, c
         float v[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) v[e] = acc[i][j][q * 4 + e];
+        if (MODE == 3) {
+          *(float4*)((float*)R + (((size_t)slice * nbatch + batch) * M + m) * N + f) = make_float4(v[0], v[1], v[2], v[3]);
+          continue;
+        }
         if (MODE == 2) {
           const uint2 rv = *(const uint2*)(R + (size_t)m * ldr + f);
           v[0] = __uint_as_float(rv.x << 16) + rnd_bf16(v[0]);
@@ -831,14 +837,14 @@ gemm_ta_bf16_kernel(const bf16_t* __restrict__ A, long long lda, long long sa, c
 
 template <class G, int MODE>
 int gemm_ta_launch_tile(const void* A, long long lda, long long sa, const void* W, const void* R, long long ldr, long long sr,
-                        void* C, long long ldc, long long sc, int M, int N, int K, int nbatch, hipStream_t s) {
+                        void* C, long long ldc, long long sc, int M, int N, int K, int nbatch, hipStream_t s, int ksplit = 1) {
   static hipError_t attr_err = hipFuncSetAttribute((const void*)gemm_ta_bf16_kernel<G, MODE>, hipFuncAttributeMaxDynamicSharedMemorySize, G::LDS);
   if (attr_err != hipSuccess) { fstu_set_error("fstu_gemm_bf16_ta: hipFuncSetAttribute: %s", hipGetErrorString(attr_err)); return (int)attr_err; }
   const int mt = M / G::BT, nt = (N + G::BF - 1) / G::BF;
-  const long long tiles = (long long)mt * nt * nbatch;
+  const long long tiles = (long long)mt * nt * nbatch * ksplit;
   const int share = (int)((tiles + 7) / 8);
   hipLaunchKernelGGL((gemm_ta_bf16_kernel<G, MODE>), dim3((unsigned)share * 8u), dim3(G::THREADS), G::LDS, s, (const bf16_t*)A, lda, sa,
-                     (const bf16_t*)W, (const bf16_t*)R, ldr, sr, (bf16_t*)C, ldc, sc, M, N, K, mt, nt, share, nbatch);
+                     (const bf16_t*)W, (const bf16_t*)R, ldr, sr, (bf16_t*)C, ldc, sc, M, N, K, mt, nt, share, nbatch, ksplit);
   return 0;
 }
 
@@ -902,8 +908,68 @@ extern "C" int fstu_gemm_bf16_splitk(const void* A, int64_t lda, const void* W, 
   return FSTU_OK;
 }
 
+// fp32 slices (ns, nb, M, N) added in order -> C[b] = T(sum), or T(R[b] + T(sum)): bound by the slices' bytes
+__global__ void __launch_bounds__(256)
+join_slices_kernel(const float* __restrict__ part, int ns, const bf16_t* R, long long ldr, long long sr, bf16_t* C, long long ldc,
+                   long long sc, int M, int n4, unsigned groups) {
+  const unsigned i = blockIdx.x * 256u + threadIdx.x;
+  if (i >= groups) return;
+  const unsigned row = i / (unsigned)n4, c = (i - row * (unsigned)n4) * 4, b = row / (unsigned)M, m = row - b * (unsigned)M;
+  const float4* p = (const float4*)part + i;
+  uint2 rv = make_uint2(0, 0);
+  if (R) rv = *(const uint2*)(R + (size_t)b * sr + (size_t)m * ldr + c);
+  float4 t = p[0];
+#pragma unroll 4
+  for (int s = 1; s < ns; ++s) {
+    const float4 v = p[(size_t)s * groups];
+    t.x += v.x; t.y += v.y; t.z += v.z; t.w += v.w;
+  }
+  if (R) {
+    t.x = __uint_as_float(rv.x << 16) + rnd_bf16(t.x);
+    t.y = __uint_as_float(rv.x & 0xffff0000u) + rnd_bf16(t.y);
+    t.z = __uint_as_float(rv.y << 16) + rnd_bf16(t.z);
+    t.w = __uint_as_float(rv.y & 0xffff0000u) + rnd_bf16(t.w);
+  }
+  *(uint2*)(C + (size_t)b * sc + (size_t)m * ldc + c) = make_uint2(pack2_bf16(t.x, t.y), pack2_bf16(t.z, t.w));
+}
+static int fstu_join_slices(const float* part, int ns, const void* R, long long ldr, long long sr, void* C, long long ldc, long long sc,
+                            int nb, int M, int N, void* stream) {
+  const long long groups = (long long)nb * M * (N / 4);
+  FSTU_REQUIRE(groups < (1ll << 31), FSTU_ESHAPE, "fstu_gemm: %lld groups of slices", groups);
+  hipLaunchKernelGGL(join_slices_kernel, dim3((unsigned)((groups + 255) / 256)), dim3(256), 0, (hipStream_t)stream, part, ns, (const bf16_t*)R,
+                     ldr, sr, (bf16_t*)C, ldc, sc, M, N / 4, (unsigned)groups);
+  FSTU_CHECK_LAUNCH("fstu_gemm: slices");
+  return FSTU_OK;
+}
+
+// Slices of K for a product of few output tiles (1: none).  Without slices a workgroup walks all of K alone, 0.41 us per k tile
+// of 64 whatever the grid; two to a compute unit 0.62 us each; joining costs a launch and the slices' bytes out and back at
+// 4 TB/s.  The estimate only has to rank: us without / with the slices it picks, rows x features x K: 37 x 768 x 9216 58.8 /
+// 11.7 (18), 300 x 768 x 9216 60 / 19.3 (12), 1400 x 768 x 9216 64 / 41 (3), 2331 x 768 x 9216 65 / 47 (4), 3000 x 768 x 9216
+// 67 / 57 (3), 700 x 2048 x 24576 187 / 87 (4), 1500 x 2048 x 24576 198 / 165 (2), 300 x 2048 x 2048 22.5 / 14.8 (4); slabs 1 x
+// 1024 x 1024 x 24576 219 / 63 (8), 1 x 128 x 256 x 6144 50 / 12 (12).  Where it picks none, without / with two: 4096 x 768 x
+// 9216 70.7 / 73.3, 1000 x 2048 x 2048 23.9 / 23.4, 300 x 6144 x 2048 20.5 / 23.8, 1000 x 768 x 768 10.5 / 12.7.
+extern "C" int fstu_gemm_bf16_slices(int M, int N, int K, int nbatch) {
+  if (M <= 32 || N % 4 != 0 || K % 64 != 0) return 1;
+  const long long cus = gemm_cus(), tiles = (long long)((M + 127) / 128) * ((N + 127) / 128) * nbatch;
+  const int nkt = K / 64;
+  double least = 0.41 * nkt;
+  int best = 1;
+  for (int s = 2; s <= 32 && K / s >= 512 && tiles * s <= 2 * cus; ++s) {
+    if (nkt % s != 0) continue;
+    const double us = nkt / s * (tiles * s <= cus ? 0.41 : 0.62) + 4.0 + 8e-6 / 4.0 * s * nbatch * (double)M * N;
+    if (us < least) { least = us; best = s; }
+  }
+  return best;
+}
+
 extern "C" int fstu_gemm_bf16(const void* A, int64_t lda, const void* W, const void* W2, const void* R, int64_t ldr, void* C,
                               int64_t ldc, int M, int N, int K, int mode, void* stream) {
+  return fstu_gemm_bf16_ws(A, lda, W, W2, R, ldr, C, ldc, M, N, K, mode, nullptr, 1, stream);
+}
+// modes 0 and 2 with K in ksplit slices (partial: ksplit * M * N fp32), which a second launch adds
+extern "C" int fstu_gemm_bf16_ws(const void* A, int64_t lda, const void* W, const void* W2, const void* R, int64_t ldr, void* C,
+                                 int64_t ldc, int M, int N, int K, int mode, float* partial, int ksplit, void* stream) {
   FSTU_REQUIRE(A && W && C, FSTU_ENULL, "fstu_gemm_bf16: null pointer");
   FSTU_REQUIRE(mode >= 0 && mode <= 2, FSTU_EARG, "fstu_gemm_bf16: mode %d", mode);
   FSTU_REQUIRE((mode != 1 || W2) && (mode != 2 || R), FSTU_ENULL, "fstu_gemm_bf16: mode %d needs its second operand", mode);
@@ -916,6 +982,12 @@ extern "C" int fstu_gemm_bf16(const void* A, int64_t lda, const void* W, const v
   FSTU_REQUIRE(lda < GM_MAX_LD && K < GM_MAX_LD, FSTU_ESHAPE, "fstu_gemm_bf16: lda=%lld / K=%d beyond the 32-bit tile offsets",
                (long long)lda, K);
   int rc;
+  if (ksplit > 1) {
+    FSTU_REQUIRE(mode != 1 && ldc % 4 == 0 && fstu_aligned(C, 8), FSTU_ESHAPE, "fstu_gemm_bf16_ws: slices in modes 0 and 2, ldc %% 4 == 0");
+    rc = fstu_gemm_bf16_splitk(A, lda, W, partial, M, N, K, ksplit, stream);
+    if (rc) return rc;
+    return fstu_join_slices(partial, ksplit, mode == 2 ? R : nullptr, ldr, 0, C, ldc, 0, 1, M, N, stream);
+  }
   if (mode == 0) rc = gemm_launch<0>(A, lda, W, W2, R, ldr, C, ldc, M, N, K, (hipStream_t)stream);
   else if (mode == 1) rc = gemm_launch<1>(A, lda, W, W2, R, ldr, C, ldc, M, N, K, (hipStream_t)stream);
   else rc = gemm_launch<2>(A, lda, W, W2, R, ldr, C, ldc, M, N, K, (hipStream_t)stream);
@@ -924,11 +996,25 @@ extern "C" int fstu_gemm_bf16(const void* A, int64_t lda, const void* W, const v
   return FSTU_OK;
 }
 
+static int split_check(const char* name, int N, int K, int ksplit, const void* partial) {
+  FSTU_REQUIRE(partial && fstu_aligned(partial, 16), FSTU_EALIGN, "%s: partial must be 16-byte aligned", name);
+  FSTU_REQUIRE(ksplit >= 1 && ksplit <= 64 && K % (64 * ksplit) == 0 && N % 4 == 0, FSTU_ESHAPE,
+               "%s: K=%d must be a multiple of 64*ksplit (ksplit=%d, 1..64), N=%d of 4", name, K, ksplit, N);
+  return FSTU_OK;
+}
+
 // C[b] = T(A[b]^T W^T) (mode 0) or T(R[b] + T(A[b]^T W^T)) (mode 2) for nbatch slabs A[b] of shape (K, M) with row
 // stride lda (elements; the reduction index slowest, M contiguous), W (N, K) row-major.  M must be a multiple of 128.
 extern "C" int fstu_gemm_bf16_ta(const void* A, int64_t lda, int64_t batch_stride_a, const void* W, const void* R, int64_t ldr,
                                  int64_t batch_stride_r, void* C, int64_t ldc, int64_t batch_stride_c, int M, int N, int K,
                                  int nbatch, int mode, void* stream) {
+  return fstu_gemm_bf16_ta_ws(A, lda, batch_stride_a, W, R, ldr, batch_stride_r, C, ldc, batch_stride_c, M, N, K, nbatch, mode, nullptr, 1,
+                              stream);
+}
+// the same with K in ksplit slices (partial: ksplit * nbatch * M * N fp32), which a second launch adds
+extern "C" int fstu_gemm_bf16_ta_ws(const void* A, int64_t lda, int64_t batch_stride_a, const void* W, const void* R, int64_t ldr,
+                                    int64_t batch_stride_r, void* C, int64_t ldc, int64_t batch_stride_c, int M, int N, int K,
+                                    int nbatch, int mode, float* partial, int ksplit, void* stream) {
   FSTU_REQUIRE(A && W && C, FSTU_ENULL, "fstu_gemm_bf16_ta: null pointer");
   FSTU_REQUIRE(mode == 0 || mode == 2, FSTU_EARG, "fstu_gemm_bf16_ta: mode %d (0: plain, 2: residual add)", mode);
   FSTU_REQUIRE(mode != 2 || R, FSTU_ENULL, "fstu_gemm_bf16_ta: mode 2 needs R");
@@ -948,6 +1034,13 @@ extern "C" int fstu_gemm_bf16_ta(const void* A, int64_t lda, int64_t batch_strid
   hipStream_t s = (hipStream_t)stream;
   const long long big = (long long)(M / 256) * ((N + 255) / 256) * nbatch;
   int rc;
+  if (ksplit > 1) {
+    if ((rc = split_check("fstu_gemm_bf16_ta_ws", N, K, ksplit, partial))) return rc;
+    rc = gemm_ta_launch_tile<TileSmall, 3>(A, lda, batch_stride_a, W, partial, 0, 0, C, 0, 0, M, N, K, nbatch, s, ksplit);
+    if (rc) return rc;
+    FSTU_CHECK_LAUNCH("fstu_gemm_bf16_ta_ws");
+    return fstu_join_slices(partial, ksplit, mode == 2 ? R : nullptr, ldr, batch_stride_r, C, ldc, batch_stride_c, nbatch, M, N, stream);
+  }
 #define TA_GO(TILE)                                                                                                              \
   (mode == 0 ? gemm_ta_launch_tile<TILE, 0>(A, lda, batch_stride_a, W, R, ldr, batch_stride_r, C, ldc, batch_stride_c, M, N, K,  \
                                             nbatch, s)                                                                           \

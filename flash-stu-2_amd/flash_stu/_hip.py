@@ -94,6 +94,9 @@ SIGNATURES = {
     "fstu_gemm_bf16": [_vp, _i64, _vp, _vp, _vp, _i64, _vp, _i64, _i, _i, _i, _i, _vp],
     "fstu_gemm_bf16_splitk": [_vp, _i64, _vp, _vp, _i, _i, _i, _i, _vp],
     "fstu_gemm_any": [_vp, _i64, _i64, _vp, _i64, _i64, _vp, _i64, _i, _i, _i, _i, _vp],
+    "fstu_gemm_bf16_slices": [_i, _i, _i, _i],
+    "fstu_gemm_bf16_ws": [_vp, _i64, _vp, _vp, _vp, _i64, _vp, _i64, _i, _i, _i, _i, _vp, _i, _vp],
+    "fstu_gemm_bf16_ta_ws": [_vp, _i64, _i64, _vp, _vp, _i64, _i64, _vp, _i64, _i64, _i, _i, _i, _i, _i, _vp, _i, _vp],
     "fstu_gemm_bf16_ta": [_vp, _i64, _i64, _vp, _vp, _i64, _i64, _vp, _i64, _i64, _i, _i, _i, _i, _i, _vp],
     "fstu_lds_sequence_ws_floats": [_i, _i, _i],
     "fstu_lds_sequence_status": [_vp, _vp],
@@ -317,8 +320,13 @@ def gemm(x2: torch.Tensor, weight: torch.Tensor, up_weight: Optional[torch.Tenso
         if residual.shape != (M, N) or residual.stride(1) != 1 or residual.dtype != x2.dtype:
             raise FlashSTUHipError("gemm: residual must be (M,N) with contiguous rows")
         mode, ldr = 2, residual.stride(0)
-    _check(load().fstu_gemm_bf16(_p(x2), x2.stride(0), _p(weight), _p(up_weight), _p(residual), ldr, _p(out), out.stride(0),
-                                 M, N, K, mode, _stream()), "fstu_gemm_bf16")
+    slices, partial = 1, None
+    if mode != 1 and out.stride(0) % 4 == 0 and out.data_ptr() % 8 == 0:
+        slices = load().fstu_gemm_bf16_slices(M, N, K, 1)
+        if slices > 1:
+            partial = torch.empty(slices, M, N, dtype=torch.float32, device=x2.device)
+    _check(load().fstu_gemm_bf16_ws(_p(x2), x2.stride(0), _p(weight), _p(up_weight), _p(residual), ldr, _p(out), out.stride(0),
+                                    M, N, K, mode, _p(partial), slices, _stream()), "fstu_gemm_bf16")
     return out
 
 
@@ -365,10 +373,13 @@ def gemm_ta(slabs: torch.Tensor, weight: torch.Tensor, residual: Optional[torch.
         if t is not None and (t.shape != (nb, M, N) or t.stride(2) != 1 or t.dtype != slabs.dtype):
             raise FlashSTUHipError(f"gemm_ta: {name} must be (nb, M, N) with contiguous rows")
     mode = 2 if residual is not None else 0
-    _check(load().fstu_gemm_bf16_ta(_p(slabs), slabs.stride(1), slabs.stride(0) if nb > 1 else 0, _p(weight), _p(residual),
-                                    residual.stride(1) if residual is not None else 0,
-                                    residual.stride(0) if residual is not None and nb > 1 else 0, _p(out), out.stride(1),
-                                    out.stride(0) if nb > 1 else 0, M, N, K, nb, mode, _stream()), "fstu_gemm_bf16_ta")
+    slices = load().fstu_gemm_bf16_slices(M, N, K, nb)
+    partial = torch.empty(slices, nb, M, N, dtype=torch.float32, device=slabs.device) if slices > 1 else None
+    _check(load().fstu_gemm_bf16_ta_ws(_p(slabs), slabs.stride(1), slabs.stride(0) if nb > 1 else 0, _p(weight), _p(residual),
+                                       residual.stride(1) if residual is not None else 0,
+                                       residual.stride(0) if residual is not None and nb > 1 else 0, _p(out), out.stride(1),
+                                       out.stride(0) if nb > 1 else 0, M, N, K, nb, mode, _p(partial), slices, _stream()),
+           "fstu_gemm_bf16_ta")
     return out
 
 

@@ -429,6 +429,15 @@ int fstu_gemm_any(const void* A, int64_t sam, int64_t sak, const void* W, int64_
 int fstu_gemm_bf16_ta(const void* A, int64_t lda, int64_t batch_stride_a, const void* W, const void* R, int64_t ldr,
                       int64_t batch_stride_r, void* C, int64_t ldc, int64_t batch_stride_c, int M, int N, int K, int nbatch,
                       int mode, void* stream);
+/* Few output tiles and a long K: the same with K in ksplit slices (K % (64*ksplit) == 0, N % 4 == 0, modes 0 and 2), which a
+ * second launch adds in order.  fstu_gemm_bf16_slices says how many pay (1: none; nbatch = 1 for fstu_gemm_bf16_ws); partial
+ * holds ksplit * nbatch * M * N floats, 16-byte aligned. */
+int fstu_gemm_bf16_slices(int M, int N, int K, int nbatch);
+int fstu_gemm_bf16_ws(const void* A, int64_t lda, const void* W, const void* W2, const void* R, int64_t ldr, void* C,
+                      int64_t ldc, int M, int N, int K, int mode, float* partial, int ksplit, void* stream);
+int fstu_gemm_bf16_ta_ws(const void* A, int64_t lda, int64_t batch_stride_a, const void* W, const void* R, int64_t ldr,
+                         int64_t batch_stride_r, void* C, int64_t ldc, int64_t batch_stride_c, int M, int N, int K,
+                         int nbatch, int mode, float* partial, int ksplit, void* stream);
 
 /* ---- dense LDS (mini_stu/lds.py:95-101) ------------------------------------
  * T_steps consecutive steps with the fp32 state h (Bt,S) carried in place:

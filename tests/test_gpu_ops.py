@@ -229,6 +229,33 @@ def test_gemm_bf16_transposed_activations(hip, nb, M, N, K):
         hip.gemm_ta(Ad.transpose(1, 2), Wd)  # M not the contiguous index
 
 
+@pytest.mark.parametrize("nb,M,N,K,slices", [(1, 128, 132, 4096, 8), (3, 256, 260, 6144, 12), (1, 384, 1024, 3072, 6)])
+def test_gemm_bf16_in_slices(hip, nb, M, N, K, slices):
+    """Few output tiles and a long K: both prompt GEMMs in slices of K, plain and with the residual, ragged tiles and strided
+    rows.  fp32 sums of exact products in any order stay within (K + slices) * 2^-24 of the absolute sum; one rounding to bf16
+    (2^-8 of the value), with the residual a second."""
+    g = gen(M + K)
+    A, W = dev(torch.randn(nb, K, M, generator=g).bfloat16()), dev(torch.randn(N, K, generator=g).bfloat16())
+    R = dev(torch.randn(nb, M, N, generator=g).bfloat16())
+    assert hip.load().fstu_gemm_bf16_slices(M, N, K, nb) == slices and hip.load().fstu_gemm_bf16_slices(M, N + 1, K, nb) == 1
+    ref = torch.stack([A[b].double().t() @ W.double().t() for b in range(nb)])
+    mag = torch.stack([A[b].double().abs().t() @ W.double().abs().t() for b in range(nb)])
+    bound = (K + slices) * 2.0 ** -24 * mag + 2.0 ** -8 * ref.abs()
+    got = hip.gemm_ta(A, W)
+    assert bool(((got.double() - ref).abs() <= bound).all())
+    assert torch.equal(hip.gemm_ta(A, W, residual=R), (R.float() + got.float()).bfloat16())
+    for b, rows in ((0, M), (nb - 1, M - 3)):
+        wide = torch.full((rows + 1, K + 8), float("nan"), dtype=torch.bfloat16, device="cuda")
+        wide[:rows, :K] = A[b].t()[:rows]
+        out = torch.full((rows + 1, N + 4), float("nan"), dtype=torch.bfloat16, device="cuda")
+        assert hip.load().fstu_gemm_bf16_slices(rows, N, K, 1) > 1
+        y = hip.gemm(wide[:rows, :K], W, out=out[:rows, :N])
+        assert bool(((y.double() - ref[b, :rows]).abs() <= bound[b, :rows]).all())
+        assert bool(out[rows:].isnan().all()) and bool(out[:, N:].isnan().all())
+        z = hip.gemm(wide[:rows, :K], W, residual=R[b, :rows], out=R[b, :rows].clone())
+        assert torch.equal(z, (R[b, :rows].float() + y.float()).bfloat16())
+
+
 @pytest.mark.parametrize("nb,M,N,K", [(1, 4096, 2308, 128), (3, 2048, 1540, 64), (1, 4096, 2304, 320)])
 def test_gemm_bf16_transposed_activations_large_tiles(hip, nb, M, N, K):
     """The 256 x 256 tiles over slabs: one k tile, an even and an odd number of them, several slabs and tiles per workgroup, a
