@@ -173,6 +173,45 @@ class ApproxConvolveSum(torch.autograd.Function):
         return _convolve_grads(ctx, u, v, spec, gy, None, 0)
 
 
+class ProjectInputs(torch.autograd.Function):
+    """x (B,T,d_in) @ m (d_in,d_out) in bf16 with its gradients on the matrix-core kernels.  The gradient of m sums over all
+    B*T positions: x is the contraction's slab as it lies (reduction index slowest), the output gradient is transposed once,
+    and the long sum is taken in slices (8 x 2048 positions of 768: 60 us with the transpose, the library product 97)."""
+
+    @staticmethod
+    def takes(x, m) -> bool:
+        if x.dim() != 3 or not x.is_cuda or x.dtype != torch.bfloat16 or m.dtype != torch.bfloat16 or m.device != x.device:
+            return False
+        rows, d_in, d_out = x.shape[0] * x.shape[1], m.shape[0], m.shape[1]
+        return (x.shape[2] == d_in and rows >= 128 and rows % 64 == 0 and d_in % 128 == 0 and d_out % 128 == 0 and m.is_contiguous()
+                and m.data_ptr() % 16 == 0 and rows * d_in < 1 << 30 and rows * d_out < 1 << 30)
+
+    @staticmethod
+    def forward(ctx, x, m):
+        from .. import _hip
+        ctx.save_for_backward(x, m)
+        x2 = _aligned(x.reshape(-1, x.shape[2]))
+        return _hip.gemm(x2, _hip.transpose(m[None])[0]).view(*x.shape[:2], m.shape[1])
+
+    @staticmethod
+    def backward(ctx, g):
+        from .. import _hip
+        x, m = ctx.saved_tensors
+        g2 = _aligned(g.reshape(-1, g.shape[2]))
+        gx = _hip.gemm(g2, m).view_as(x) if ctx.needs_input_grad[0] else None
+        gm = None
+        if ctx.needs_input_grad[1]:
+            x2 = _aligned(x.reshape(-1, x.shape[2]))
+            gm = _hip.gemm_ta(x2[None], _hip.transpose(g2[None])[0])[0]
+        return gx, gm
+
+
+def _aligned(t: torch.Tensor) -> torch.Tensor:
+    """t with dense rows at a 16-byte address, as the matrix-core kernels read it."""
+    t = t.contiguous()
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
 def convolve(u: torch.Tensor, v: torch.Tensor, n: int, use_approx: bool = True, return_both: bool = True,
              sgn: Optional[torch.Tensor] = None, v_fft: Optional[torch.Tensor] = None):
     """The reference's causal convolution (flash_stu/utils/stu_utils.py:195-246), same arguments and results:
@@ -205,6 +244,6 @@ def convolve(u: torch.Tensor, v: torch.Tensor, n: int, use_approx: bool = True, 
         _hip.stu_conv_bank(u.contiguous(), v.contiguous(), up, um)
     else:
         spec = _hip.stu_fft_filter(v.contiguous(), nn_, single_branch=not return_both)
-        ut = u.transpose(1, 2).contiguous().transpose(1, 2)        # time-major copy: coalesced column loads
+        ut = _hip.transpose(u.contiguous()).transpose(1, 2)        # time-major copy: coalesced column loads
         _hip.stu_conv_bank_fft(ut, spec, up, um)
     return up, um

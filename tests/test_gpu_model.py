@@ -163,6 +163,32 @@ def test_stu_forward_differentiable_gradients(hankel):
         assert float((got.cpu() - want).abs().max()) <= 2e-4 * float(want.abs().max())
 
 
+@pytest.mark.parametrize("B,T,d", [(1, 128, 128), (3, 320, 256), (2, 97, 128)])
+def test_input_projection_gradients(B, T, d):
+    """x @ M_inputs and its gradients on the matrix-core kernels (and, for rows they do not take, the library's product)
+    against float64: fp32 sums of exact products, one rounding to bf16 (2^-8 of the value) each; x expanded, shifted off its
+    alignment and frozen."""
+    from flash_stu.utils.stu_utils import ProjectInputs
+    g = torch.Generator().manual_seed(B * T)
+    x, m, w = (torch.randn(*s, generator=g).bfloat16().cuda() for s in ((B, T, d), (d, 2 * d), (B, T, 2 * d)))
+    assert ProjectInputs.takes(x, m) == (B * T % 64 == 0)
+    if not ProjectInputs.takes(x, m):
+        return
+    shifted = torch.empty(B * T * d + 1, dtype=torch.bfloat16, device="cuda")[1:].view(B, T, d).copy_(x)
+    for xi in (x, shifted, x[:1].expand(B, T, d)):
+        xi, mi = xi.detach().requires_grad_(True), m.clone().requires_grad_(True)
+        y = ProjectInputs.apply(xi, mi)
+        y.backward(w)
+        xd, md, wd = xi.detach().double().reshape(-1, d), m.double(), w.double().reshape(-1, 2 * d)
+        for got, a, b in ((y.detach(), xd, md), (xi.grad, wd, md.t()), (mi.grad, xd.t(), wd)):
+            ref, mag = a @ b, a.abs() @ b.abs()
+            err = (got.double().reshape(ref.shape) - ref).abs()
+            assert bool((err <= 2.0 ** -8 * ref.abs() + a.shape[1] * 2.0 ** -23 * mag).all())
+    xi = x.clone().requires_grad_(True)
+    ProjectInputs.apply(xi, m).backward(w)             # m needs no gradient
+    assert xi.grad.shape == x.shape and m.grad is None
+
+
 def _teacher_forced(w, ocfg, tokens, P):
     logits, _ = O.model_forward(w, ocfg, tokens[:, :-1])
     return logits[:, P - 1:, :]          # predictions for positions P..end
