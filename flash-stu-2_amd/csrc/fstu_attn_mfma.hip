@@ -7,7 +7,7 @@
 //                                     the 16 rows of key tile t are the keys 8*(i>>2) + 4*t + (i&3) of the block, so
 //                                     that after both tiles lane (g, c) holds the scores of query c against the 8
 //                                     CONSECUTIVE keys 8g..8g+7: exactly its B-operand fragment of the second product
-//   O^T (dims x queries) = V^T P^T   V^T read from a transposed copy (B,H,hd,Tp) made by swa_vt_kernel, 16 bytes per
+//   O^T (dims x queries) = V^T P^T   V^T read from a transposed copy (B,H,hd,Tp) made in front, 16 bytes per
 //                                     lane; P is split into a bf16 head and a bf16 remainder (two MFMAs), which
 //                                     keeps the product at fp32-P accuracy.
 // Both products leave query c in lane c of every 16-lane group, so the online-softmax state (max, sum) is per lane
@@ -20,27 +20,6 @@ typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float floatx4_t __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ bf16x8_t as_bf16x8(uint4 v) { return __builtin_bit_cast(bf16x8_t, v); }
-
-// V^T copy: vt[b][h][i][t] = v[b][t][h][i], zero for T <= t < Tp
-__global__ void __launch_bounds__(256)
-swa_vt_kernel(const bf16_t* __restrict__ qkv, bf16_t* __restrict__ vt, int Tn, int Tp, int H, int HD) {
-  // a workgroup transposes a 64 (t) x 64 (dims) tile through LDS
-  __shared__ bf16_t tile[64][66];
-  const int d = H * HD;
-  const int t0 = blockIdx.x * 64, i0 = blockIdx.y * 64;   // i over H*HD
-  const int b = blockIdx.z;
-  for (int e = threadIdx.x; e < 64 * 64; e += 256) {
-    const int tt = e >> 6, ii = e & 63;
-    bf16_t v = 0;
-    if (t0 + tt < Tn && i0 + ii < d) v = qkv[((size_t)b * Tn + t0 + tt) * 3 * d + 2 * d + i0 + ii];
-    tile[tt][ii] = v;
-  }
-  __syncthreads();
-  for (int e = threadIdx.x; e < 64 * 64; e += 256) {
-    const int ii = e >> 6, tt = e & 63;
-    if (t0 + tt < Tp && i0 + ii < d) vt[((size_t)b * d + i0 + ii) * Tp + t0 + tt] = tile[tt][ii];
-  }
-}
 
 template <int HD, int NW>
 __global__ void __launch_bounds__(NW * 64)
@@ -215,7 +194,9 @@ extern "C" int fstu_swa_prefill_mfma(const void* qkv, void* vt_ws, void* out, co
   const int Tp = (T_ + 63) / 64 * 64;
   const int d = H * hd;
   hipStream_t s = (hipStream_t)stream;
-  hipLaunchKernelGGL(swa_vt_kernel, dim3(Tp / 64, (d + 63) / 64, B), dim3(256), 0, s, (const bf16_t*)qkv, (bf16_t*)vt_ws, T_, Tp, H, hd);
+  // V^T copy: vt[b][h][i][t] = v[b][t][h][i], zero for T <= t < Tp
+  const int rc = fstu_transpose16_launch((const bf16_t*)qkv + 2 * d, (size_t)T_ * 3 * d, (size_t)3 * d, vt_ws, (size_t)d * Tp, Tp, B, T_, Tp, d, stream);
+  if (rc) return rc;
   // queries per workgroup (waves sharing one K / V^T tile): 64 at head dim 64, 256 at head dim 128 (measured at
   // 4x1024 tokens, 16 heads of 128, window 1024: 200 us with 4 waves, 130 with 8, 109 with 16; at head dim 64
   // 4 waves were the fastest)

@@ -860,6 +860,19 @@ def test_stu_step_lds_pair_with_the_odd_lag_sum_handed_on(hip, dtype, S, R, T0):
     assert torch.equal(st_c, st_p) and (not R or torch.equal(ring_c, ring_p))
 
 
+@pytest.mark.parametrize("B,R,C", [(1, 8, 8), (2, 72, 136), (3, 64, 200), (1, 520, 64), (2, 8, 1032)])
+def test_transpose_in_whole_pieces(hip, B, R, C):
+    """bf16 rows and columns of whole 16-byte pieces (ragged against the 64 x 64 tiles), and the same off its alignment."""
+    x = dev(torch.randn(B, R, C, generator=gen(96)).bfloat16())
+    want = x.transpose(1, 2).contiguous()
+    assert torch.equal(hip.transpose(x), want)
+    shifted = torch.empty(B * R * C + 1, dtype=torch.bfloat16, device="cuda")[1:].view(B, R, C).copy_(x)
+    guard = torch.full((B * R * C + 16,), float("nan"), dtype=torch.bfloat16, device="cuda")
+    out = guard[8:-8].view(B, C, R)
+    assert torch.equal(hip.transpose(shifted, out), want) and torch.equal(hip.transpose(x, out), want)
+    assert bool(guard[:8].isnan().all()) and bool(guard[-8:].isnan().all())
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("B,R,C", [(1, 4096, 2048), (3, 100, 70), (2, 64, 64), (1, 1, 5), (2, 129, 1)])
 def test_transpose(hip, dtype, B, R, C):
