@@ -176,11 +176,12 @@ class ApproxConvolveSum(torch.autograd.Function):
 class ProjectInputs(torch.autograd.Function):
     """x (B,T,d_in) @ m (d_in,d_out) in bf16 with its gradients on the matrix-core kernels.  The gradient of m sums over all
     B*T positions: x is the contraction's slab as it lies (reduction index slowest), the output gradient is transposed once,
-    and the long sum is taken in slices (8 x 2048 positions of 768: 60 us with the transpose, the library product 97)."""
+    and the long sum is taken in slices (8 x 2048 positions of 768: 60 us with the transpose, the library product 97).
+    Where the gradients are to be differentiated themselves (create_graph=True) they are plain products."""
 
     @staticmethod
     def takes(x, m) -> bool:
-        if x.dim() != 3 or not x.is_cuda or x.dtype != torch.bfloat16 or m.dtype != torch.bfloat16 or m.device != x.device:
+        if x.dim() != 3 or not x.is_cuda or x.dtype != torch.bfloat16 or m.dtype != torch.bfloat16 or m.device != x.device or torch.is_autocast_enabled():
             return False
         rows, d_in, d_out = x.shape[0] * x.shape[1], m.shape[0], m.shape[1]
         return (x.shape[2] == d_in and rows >= 128 and rows % 64 == 0 and d_in % 128 == 0 and d_out % 128 == 0 and m.is_contiguous()
@@ -197,6 +198,9 @@ class ProjectInputs(torch.autograd.Function):
     def backward(ctx, g):
         from .. import _hip
         x, m = ctx.saved_tensors
+        if torch.is_grad_enabled():
+            return (g @ m.T if ctx.needs_input_grad[0] else None,
+                    x.reshape(-1, x.shape[2]).T @ g.reshape(-1, g.shape[2]) if ctx.needs_input_grad[1] else None)
         g2 = _aligned(g.reshape(-1, g.shape[2]))
         gx = _hip.gemm(g2, m).view_as(x) if ctx.needs_input_grad[0] else None
         gm = None

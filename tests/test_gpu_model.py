@@ -189,6 +189,22 @@ def test_input_projection_gradients(B, T, d):
     assert xi.grad.shape == x.shape and m.grad is None
 
 
+def test_input_projection_gradients_of_gradients():
+    """create_graph=True: the gradients of x @ m carry their own graph, as those of the plain product do.  Same bf16 products in
+    both: two roundings (2^-8 each) of sums of the same terms."""
+    from flash_stu.utils.stu_utils import ProjectInputs
+    g = torch.Generator().manual_seed(3)
+    x0, m0, w = (torch.randn(*s, generator=g).bfloat16().cuda() for s in ((2, 64, 128), (128, 128), (2, 64, 128)))
+    seconds = []
+    for f in (ProjectInputs.apply, torch.matmul):
+        x, m = x0.clone().requires_grad_(True), m0.clone().requires_grad_(True)
+        gx, gm = torch.autograd.grad(f(x, m), (x, m), w, create_graph=True)
+        assert gx.requires_grad and gm.requires_grad
+        seconds.append(torch.autograd.grad(gx.float().square().sum() + gm.float().square().sum(), (x, m)))
+    for got, ref in zip(*seconds):
+        assert float((got.float() - ref.float()).norm()) <= 2.0 ** -7 * float(ref.float().norm())
+
+
 def _teacher_forced(w, ocfg, tokens, P):
     logits, _ = O.model_forward(w, ocfg, tokens[:, :-1])
     return logits[:, P - 1:, :]          # predictions for positions P..end
