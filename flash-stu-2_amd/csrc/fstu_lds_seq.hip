@@ -43,7 +43,25 @@ __device__ __forceinline__ uint4 buf_load16(rsrc_t rs, unsigned off) {
 #define LSQ_SPIN_LIMIT (1 << 18)   // polls of one batch of published states before the wait gives up
 #define LSQ_LOOK 8                 // published states requested at a time
 
-template <int NT>
+// the 16 bytes of lane r ^ 8 of the same 16 lanes (a rotation of 16 lanes by 8)
+__device__ __forceinline__ uint4 swap8(uint4 v) {
+  v.x = __builtin_amdgcn_mov_dpp(v.x, 0x128, 0xf, 0xf, false);
+  v.y = __builtin_amdgcn_mov_dpp(v.y, 0x128, 0xf, 0xf, false);
+  v.z = __builtin_amdgcn_mov_dpp(v.z, 0x128, 0xf, 0xf, false);
+  v.w = __builtin_amdgcn_mov_dpp(v.w, 0x128, 0xf, 0xf, false);
+  return v;
+}
+typedef unsigned uintx4_t __attribute__((ext_vector_type(4)));
+typedef uintx4_t uintx4_a8_t __attribute__((aligned(8)));
+// outputs are 8-byte aligned
+__device__ __forceinline__ void store16_past(bf16_t* p, uint4 v) { __builtin_nontemporal_store(__builtin_bit_cast(uintx4_t, v), (uintx4_a8_t*)p); }
+
+// PAST: the outputs leave in whole lines and past the L2s, where they are more than those hold (32 MB): what they would push
+// out are the weights that every workgroup fetches again, and the next kernel would not find them there.  us, through the L2s
+// from the accumulators / past them: 64 x 4096 x 1024, state 160, 407 / 389 (whole lines through the L2s 404), 51 x 3262 x 256
+// 121 / 111; 2 x 776 x 512 54.2 / 54.9, 2 x 437 x 256 39.0 / 39.5.
+
+template <int NT, bool PAST>
 __global__ void __launch_bounds__(256, NT <= 10 ? 2 : 1)   // beyond S = 160 one workgroup fills the LDS anyway
 lds_seq_kernel(const bf16_t* __restrict__ x, const float* __restrict__ A, const bf16_t* __restrict__ BmT,
                const bf16_t* __restrict__ CmT, bf16_t* __restrict__ y, const float* __restrict__ h0,
@@ -246,13 +264,22 @@ lds_seq_kernel(const bf16_t* __restrict__ x, const float* __restrict__ A, const 
         }
       }
     }
+    // PAST: a lane stores 16 bytes, the eight lanes of a line next to each other in one instruction (straight from the
+    // accumulators an instruction covers 32 bytes of 16 rows): the rows of the
+    // two tiles of 32 features are dealt so that lane (r, g) ends up with features 8g .. 8g+7 of position r, and lanes r and
+    // r ^ 8 swap pieces, so that lanes r and r ^ 8 hold the two halves of a line of 64 features.
+    const int trow = t0 + 32 * w + (r & 7), fcol = 32 * (r >> 3) + 8 * g;
+    bf16_t* yr[4];                                           // position trow + 8 q
+#pragma unroll
+    for (int q = 0; q < 4; ++q) yr[q] = y + ((size_t)min(trow + 8 * q, T - 1) * Bt + b) * d_out + fcol;
     const int tA = t0 + 32 * w + r, tB = tA + 16;
     bf16_t* yA = y + ((size_t)min(tA, T - 1) * Bt + b) * d_out + 4 * g;
     bf16_t* yB = y + ((size_t)min(tB, T - 1) * Bt + b) * d_out + 4 * g;
     const int nto = d_out >> 4;
     // C^T travels through LDS like B^T above, 64 output features (4 tiles) at a time, double-buffered in the space of
     // U now that every wave holds its H fragments in registers.  Rows are S * 2 + 16 bytes: an odd number of 16-byte
-    // slots, so the 16 rows of a fragment read fall into 16 different slots.
+    // slots, so the 16 rows of a fragment read fall into 16 different slots.  With PAST feature 32p + 8g + 4h + i lies
+    // in row 32p + 16h + 4g + i.
     __syncthreads();
     unsigned char* cst = (unsigned char*)Us;
     const unsigned RS = (unsigned)S * 2u + 16u, cstage = 64u * RS;
@@ -269,7 +296,8 @@ lds_seq_kernel(const bf16_t* __restrict__ x, const float* __restrict__ A, const 
 #pragma unroll
       for (int i = 0; i < CPT; ++i) {
         const int q = tid + i * 256, row = q / ppr, c = q - row * ppr;
-        if (q < npc) *(uint4*)(cst + stage * cstage + row * RS + c * 16) = v[i];
+        const int at = !PAST ? row : (row & 0x23) | ((row & 0x18) >> 1) | ((row & 4) << 2);
+        if (q < npc) *(uint4*)(cst + stage * cstage + at * RS + c * 16) = v[i];
       }
     };
     uint4 cv0[CPT], cv1[CPT];     // the next two groups of output features
@@ -281,6 +309,7 @@ lds_seq_kernel(const bf16_t* __restrict__ x, const float* __restrict__ A, const 
 #define LSQ_OUT(NXT)                                                                                          \
     {                                                                                                         \
       const unsigned char* cs = cst + cur * cstage;                                                           \
+      if constexpr (!PAST) {                                                                                  \
       _Pragma("unroll") for (int j = 0; j < 4; ++j) {                                                         \
         const int ot = (o0 >> 4) + j;                                                                         \
         if (ot < nto) {                                                                                       \
@@ -297,6 +326,40 @@ lds_seq_kernel(const bf16_t* __restrict__ x, const float* __restrict__ A, const 
           if (tA < T) *(uint2*)(yA + ot * 16) = make_uint2(pack2_bf16(a0[0], a0[1]), pack2_bf16(a0[2], a0[3])); \
           if (tB < T) *(uint2*)(yB + ot * 16) = make_uint2(pack2_bf16(a1[0], a1[1]), pack2_bf16(a1[2], a1[3])); \
         }                                                                                                     \
+      }                                                                                                       \
+      } else {                                                                                                \
+      uint4 pc[2][2];                                                                                         \
+      _Pragma("unroll") for (int p = 0; p < 2; ++p) {                                                         \
+        if (o0 + 32 * p < d_out) {                                                                            \
+          floatx4_t acc[2][2];                                                                                \
+          _Pragma("unroll") for (int h = 0; h < 2; ++h) {                                                     \
+            floatx4_t a0 = {0.f, 0.f, 0.f, 0.f}, a1 = {0.f, 0.f, 0.f, 0.f};                                   \
+            _Pragma("unroll") for (int k = 0; k < KS; ++k) {                                                  \
+              if (k < ks2) {                                                                                  \
+                const uint4 wc = *(const uint4*)(cs + (32 * p + 16 * h + r) * RS + (32 * k + 8 * g) * 2);     \
+                a0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(wc), as_bf16x8(hb[0][k]), a0, 0, 0, 0);\
+                a0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(wc), as_bf16x8(lb[0][k]), a0, 0, 0, 0);\
+                a1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(wc), as_bf16x8(hb[1][k]), a1, 0, 0, 0);\
+                a1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(wc), as_bf16x8(lb[1][k]), a1, 0, 0, 0);\
+              }                                                                                               \
+            }                                                                                                 \
+            acc[0][h] = a0;                                                                                   \
+            acc[1][h] = a1;                                                                                   \
+          }                                                                                                   \
+          _Pragma("unroll") for (int m = 0; m < 2; ++m)                                                       \
+            pc[m][p] = make_uint4(pack2_bf16(acc[m][0][0], acc[m][0][1]), pack2_bf16(acc[m][0][2], acc[m][0][3]),\
+                                  pack2_bf16(acc[m][1][0], acc[m][1][1]), pack2_bf16(acc[m][1][2], acc[m][1][3]));\
+        } else {                                                                                              \
+          pc[0][p] = pc[1][p] = make_uint4(0, 0, 0, 0);                                                       \
+        }                                                                                                     \
+      }                                                                                                       \
+      _Pragma("unroll") for (int m = 0; m < 2; ++m) {                                                         \
+        const uint4 other = swap8(r < 8 ? pc[m][1] : pc[m][0]);                                               \
+        if (o0 + fcol < d_out) {                                                                              \
+          if (trow + 16 * m < T) store16_past(yr[2 * m] + o0, r < 8 ? pc[m][0] : other);                     \
+          if (trow + 16 * m + 8 < T) store16_past(yr[2 * m + 1] + o0, r < 8 ? other : pc[m][1]);             \
+        }                                                                                                     \
+      }                                                                                                       \
       }                                                                                                       \
       if (o0 + 64 < d_out) cstore(cur ^ 1, NXT);                                                              \
       cload(o0 + 192, NXT);                                                                                   \
@@ -354,24 +417,33 @@ extern "C" int fstu_lds_sequence(float* h, const void* x, const float* A, const 
   const size_t nwords = (size_t)nblk * BtS;
   unsigned cgrid = (unsigned)((nwords + 255) / 256);
   if (cgrid > 1024u) cgrid = 1024u;
-#define LSQ_RUN(NTV)                                                                                                      \
-  do {                                                                                                                    \
-    static const hipError_t e1 = hipFuncSetAttribute((const void*)lds_seq_kernel<NTV>,                                    \
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024);            \
-    if (e1 != hipSuccess) {                                                                                               \
-      fstu_set_error("fstu_lds_sequence: hipFuncSetAttribute: %s", hipGetErrorString(e1));                                \
-      return (int)e1;                                                                                                     \
-    }                                                                                                                     \
-    hipLaunchKernelGGL(lds_seq_clear_kernel, dim3(cgrid), dim3(256), 0, s, etag, nwords, status);                         \
-    hipLaunchKernelGGL((lds_seq_kernel<NTV>), grid, dim3(256), shm, s, (const bf16_t*)x, A, (const bf16_t*)BmT,           \
-                       (const bf16_t*)CmT, (bf16_t*)y, (const float*)h, hnew, etag, status, 1u, T, Bt, d_in, S, d_out);   \
-    hipLaunchKernelGGL(lds_seq_finish_kernel, dim3((unsigned)((BtS + 255) / 256)), dim3(256), 0, s, h, (const float*)hnew, \
-                       (int)BtS);                                                                                         \
+#define LSQ_RUN2(NTV, PASTV)                                                                                          \
+  do {                                                                                                        \
+    static const hipError_t e1 = hipFuncSetAttribute((const void*)lds_seq_kernel<NTV, PASTV>,                        \
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024); \
+    if (e1 != hipSuccess) {                                                                                   \
+      fstu_set_error("fstu_lds_sequence: hipFuncSetAttribute: %s", hipGetErrorString(e1));                    \
+      return (int)e1;                                                                                         \
+    }                                                                                                         \
+    hipLaunchKernelGGL(lds_seq_clear_kernel, dim3(cgrid), dim3(256), 0, s, etag, nwords, status);             \
+    hipLaunchKernelGGL((lds_seq_kernel<NTV, PASTV>), grid, dim3(256), shm, s, (const bf16_t*)x, A, (const bf16_t*)BmT,\
+                       (const bf16_t*)CmT, (bf16_t*)y, (const float*)h, hnew, etag, status, 1u, T, Bt, d_in, S, d_out);\
+    hipLaunchKernelGGL(lds_seq_finish_kernel, dim3((unsigned)((BtS + 255) / 256)), dim3(256), 0, s, h, (const float*)hnew,\
+                       (int)BtS);                                                                             \
   } while (0)
+#define LSQ_RUN(NTV)            \
+  do {                          \
+    if (past)                   \
+      LSQ_RUN2(NTV, true);      \
+    else                        \
+      LSQ_RUN2(NTV, false);     \
+  } while (0)
+  const bool past = (size_t)T * Bt * d_out * sizeof(bf16_t) > (size_t)32 << 20;
   if (S <= 64) LSQ_RUN(4);
   else if (S <= 160) LSQ_RUN(10);
   else LSQ_RUN(16);
 #undef LSQ_RUN
+#undef LSQ_RUN2
   FSTU_CHECK_LAUNCH("fstu_lds_sequence");
   return FSTU_OK;
 }

@@ -1356,6 +1356,30 @@ def test_sample_topk_spread_plateaus_and_errors(hip):
         hip.sample_topk(logits[:, :512].contiguous(), best, ws, out, 40)
 
 
+@pytest.mark.parametrize("T,Bt,d_in,S,d_out", [(1, 1, 32, 32, 16), (9, 3, 64, 64, 32), (23, 1, 96, 160, 80), (129, 2, 32, 96, 112),
+                                               (257, 1, 64, 256, 48), (1171, 129, 32, 64, 112), (1637, 129, 32, 32, 80)])
+def test_lds_sequence_edges_of_its_stores(hip, T, Bt, d_in, S, d_out):
+    """Outputs whose last line of 64 features is cut, whose last rows are missing, at an address of 8 mod 16, against float64:
+    fp32 sums of d_in, T and S terms, the state split into two bf16 parts (2^-16), one rounding to bf16 (2^-8); nothing is
+    written beside them.  The two largest are the outputs of more than 32 MB that are written past the caches."""
+    g = torch.Generator().manual_seed(T + d_out)
+    A = 0.9 + 0.099 * torch.rand(S, generator=g)
+    Bm, Cm, x = ((torch.randn(*s, generator=g) / s[0] ** 0.5).bfloat16() for s in ((d_in, S), (S, d_out), (T, Bt, d_in)))
+    around = torch.full((T * Bt * d_out + 8,), 7.0, dtype=torch.bfloat16, device="cuda")
+    y = around[4:-4].view(T, Bt, d_out)
+    h = torch.zeros(Bt, S, device="cuda")
+    hip.lds_steps(h, x.cuda(), A.cuda(), Bm.cuda(), Cm.cuda(), out=y, check_status=True)
+    assert bool((around[:4] == 7).all()) and bool((around[-4:] == 7).all())
+    state, size = torch.zeros(2, Bt, S, dtype=torch.float64)
+    for t in range(T):
+        state = A.double() * state + x[t].double() @ Bm.double()
+        size = A.double() * size + x[t].double().abs() @ Bm.double().abs()
+        ref, mag = state @ Cm.double(), size @ Cm.double().abs()
+        bound = 2.0 ** -8 * ref.abs() + ((d_in + 2 * T + S) * 2.0 ** -23 + 2.0 ** -16) * mag
+        assert bool(((y[t].double().cpu() - ref).abs() <= bound).all()), t
+    assert bool(((h.double().cpu() - state).abs() <= (d_in + 2 * T) * 2.0 ** -23 * size).all())
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_lds_steps_dense(hip, dtype):
     g = gen(13)
