@@ -182,7 +182,8 @@ def glu_roofline(eng, cfg, B, K, lib, torch, _hip):
         packed = bool(lib.fstu_mlp_packed_rows32_supported(rows, d, I))
         if packed:
             # as the step launches it: mlp_norm of the summed residual stream formed in the launch's own fragments
-            ops = [(eng._pack(l.mlp.gate_proj.weight), eng._pack(l.mlp.up_proj.weight), l.mlp_norm.weight) for l in eng.model.layers]
+            ops = [(eng._pack(l.mlp.gate_proj.weight, (i, "gate")), eng._pack(l.mlp.up_proj.weight, (i, "up")), l.mlp_norm.weight)
+                   for i, l in enumerate(eng.model.layers)]
             launch = lambda o: _hip.glu_packed_norm(h, None, o[2], cfg.rms_norm_eps, o[0], o[1], I, out=act)
             name = ("glu_balanced_kernel<two row tiles, norm in the fragments> (mlp_norm + gate/up projection + gelu*up over "
                     "all rows, packed weights, one workgroup per compute unit)")

@@ -220,13 +220,14 @@ class DecodeEngine:
         self._gstreams = []
 
     # ------------------------------------------------------------------
-    def _pack(self, w: torch.Tensor) -> torch.Tensor:
-        """MFMA-fragment-ordered copy of an (N,K) bf16 weight, rebuilt only when the weight changes."""
-        key = w.data_ptr()
-        hit = self._packed.get(key)
-        if hit is None or hit[0] != w._version:
-            hit = (w._version, _hip.pack_rows(w))
-            self._packed[key] = hit
+    def _pack(self, w: torch.Tensor, place) -> torch.Tensor:
+        """MFMA-fragment-ordered copy of the (N,K) bf16 weight at `place` in the model, rebuilt only when the weight changes.
+        The entry holds the storage that it was made from: while it is there no other tensor can come to lie at the address
+        it is recognised by."""
+        hit = self._packed.get(place)
+        if hit is None or hit[0] != (w._version, w.data_ptr()):
+            hit = ((w._version, w.data_ptr()), _hip.pack_rows(w), w.detach())
+            self._packed[place] = hit
             self._unfinished = True
         return hit[1]
 
@@ -372,12 +373,12 @@ class DecodeEngine:
         if dt == torch.bfloat16 and self.lib.fstu_glu_packed_supported(B, d, I):
             # gate/up projection over packed weights, one workgroup per CU with equal bytes each
             for i, layer in enumerate(model.layers):
-                arr[i].wp_gate = self._pack(layer.mlp.gate_proj.weight).data_ptr()
-                arr[i].wp_up = self._pack(layer.mlp.up_proj.weight).data_ptr()
+                arr[i].wp_gate = self._pack(layer.mlp.gate_proj.weight, (i, "gate")).data_ptr()
+                arr[i].wp_up = self._pack(layer.mlp.up_proj.weight, (i, "up")).data_ptr()
             m.glu_packed = 1
             if I % 512 == 0 and d % 16 == 0:
                 for i, layer in enumerate(model.layers):
-                    arr[i].wp_down = self._pack(layer.mlp.down_proj.weight).data_ptr()
+                    arr[i].wp_down = self._pack(layer.mlp.down_proj.weight, (i, "down")).data_ptr()
                 m.down_packed = 1
             if B * (d + 8) * 2 <= 96 * 1024:
                 m.x2 = buf(B, d).data_ptr()     # second residual buffer: the MLP norm runs as the gate/up prologue
@@ -386,21 +387,21 @@ class DecodeEngine:
                     # (the down projection leaves 4 split-K slices for it): one launch less per layer
                     for i, layer in enumerate(model.layers):
                         if isinstance(layer, AttentionLayer):
-                            arr[i].wp_qkv = self._pack(layer.attn.c_attn.weight).data_ptr()
+                            arr[i].wp_qkv = self._pack(layer.attn.c_attn.weight, (i, "qkv")).data_ptr()
                     m.merge_norm = 1
         if dt == torch.bfloat16 and self.lib.fstu_mlp_packed_rows32_supported(B, d, I):
             # 17..32 rows: the MLP streams packed weights as two row tiles per weight fragment
             for i, layer in enumerate(model.layers):
-                arr[i].wp_gate = self._pack(layer.mlp.gate_proj.weight).data_ptr()
-                arr[i].wp_up = self._pack(layer.mlp.up_proj.weight).data_ptr()
-                arr[i].wp_down = self._pack(layer.mlp.down_proj.weight).data_ptr()
+                arr[i].wp_gate = self._pack(layer.mlp.gate_proj.weight, (i, "gate")).data_ptr()
+                arr[i].wp_up = self._pack(layer.mlp.up_proj.weight, (i, "up")).data_ptr()
+                arr[i].wp_down = self._pack(layer.mlp.down_proj.weight, (i, "down")).data_ptr()
                 if isinstance(layer, AttentionLayer):
-                    arr[i].wp_qkv = self._pack(layer.attn.c_attn.weight).data_ptr()
-                    arr[i].wp_proj = self._pack(layer.attn.c_proj.weight).data_ptr()
+                    arr[i].wp_qkv = self._pack(layer.attn.c_attn.weight, (i, "qkv")).data_ptr()
+                    arr[i].wp_proj = self._pack(layer.attn.c_proj.weight, (i, "proj")).data_ptr()
                 elif mode == "lds":
-                    arr[i].wp_m_inputs = self._pack(layer.stu.m_inputs_t()).data_ptr()
+                    arr[i].wp_m_inputs = self._pack(layer.stu.m_inputs_t(), (i, "m_inputs")).data_ptr()
         if dt == torch.bfloat16 and self.lib.fstu_glu_packed_supported(min(B, _hip.MAX_DECODE_ROWS), d, V):
-            m.wp_emb = self._pack(model.lm_head.weight).data_ptr()      # the head streams a packed copy of the embedding
+            m.wp_emb = self._pack(model.lm_head.weight, "emb").data_ptr()      # the head streams a packed copy of the embedding
         ch.arr, ch.desc = arr, m
         if B > _hip.MAX_DECODE_ROWS:
             # first use of the tiled kernels outside any graph capture (their launch set-up raises an LDS limit once)

@@ -54,12 +54,14 @@ class STU(nn.Module):
             raise NotImplementedError("Tiling only supported for use_approx=True")
         self._derived = {}
 
-    # ---- tensors derived from the parameters, rebuilt when a parameter changes
+    # ---- tensors derived from the parameters, rebuilt when a parameter changes; an entry holds the storage that it was
+    # made from, so that no other tensor can come to lie at the address it is recognised by (a parametrized weight is a
+    # new tensor on every access)
     def _cached(self, key, params, build):
         ver = tuple((p._version, p.data_ptr()) for p in params)
         hit = self._derived.get(key)
         if hit is None or hit[0] != ver:
-            hit = (ver, build())
+            hit = (ver, build(), [p.detach() for p in params])
             self._derived[key] = hit
         return hit[1]
 

@@ -238,3 +238,38 @@ def test_lm_head_follows_config_bias():
     m = FlashSTU(FlashSTUConfig(bias=True, **kw))
     assert m.lm_head.bias is not None and "lm_head.bias" in m.state_dict()
     assert float(m.lm_head.bias.abs().max()) == 0.0
+
+
+class _Doubled(torch.nn.Module):
+    def forward(self, w):
+        return w * 2.0
+
+
+def test_derived_copies_follow_weights_that_are_new_tensors_every_time(monkeypatch):
+    """A parametrized weight, or a copy that was formed again, may lie where an older one lay: what was derived from the
+    older one must not be taken for it."""
+    from torch.nn.utils import parametrize
+    from flash_stu import STU, FlashSTUConfig, _hip
+    from flash_stu.engine import DecodeEngine
+    cfg = FlashSTUConfig(n_embd=64, n_heads=2, n_layers=2, seq_len=32, num_eigh=4, vocab_size=64, torch_dtype=torch.float32)
+    stu = STU(cfg, torch.randn(32, 4), 64)
+    for p in stu.parameters():
+        torch.nn.init.normal_(p)
+    for name in ("M_inputs", "M_filters"):
+        parametrize.register_parametrization(stu, name, _Doubled())
+    with torch.no_grad():
+        for _ in range(20):
+            assert torch.equal(stu.m_inputs_t(), stu.parametrizations.M_inputs.original.t() * 2.0)
+            assert torch.allclose(stu.effective_filter(), stu.phi @ (stu.parametrizations.M_filters.original * 2.0))
+            for p in stu.parameters():
+                p.add_(1.0)
+    monkeypatch.setattr(_hip, "pack_rows", torch.clone)
+    engine = DecodeEngine.__new__(DecodeEngine)
+    engine._packed, engine._unfinished = {}, False
+    places = set()
+    for i in range(20):
+        w = torch.full((64, 64), float(i), dtype=torch.bfloat16)
+        places.add(w.data_ptr())
+        assert torch.equal(engine._pack(w, (0, "m_inputs")), w)
+        del w
+    assert len(places) > 1 and len(engine._packed) == 1
