@@ -71,7 +71,8 @@ def step_on_caches(model, ids: torch.Tensor, past):
     count, a configuration, a cache or a module is not what that step takes (the layers' own forward calls then run).
 
     Everything is read from the model and the caches of this call: no pointer or check outlives it, and the weights are
-    the parameters themselves, not packed copies."""
+    the parameters themselves, not packed copies.  Every tensor whose address is taken is held until the launches are
+    enqueued: a parametrized weight is a temporary that its module forms on each access."""
     cfg = model.config
     mod = torch.nn.modules.module
     if not (ids.dim() == 2 and ids.shape[1] == 1 and 1 <= ids.shape[0] <= _hip.MAX_DECODE_ROWS and ids.dtype == torch.int64
@@ -87,13 +88,15 @@ def step_on_caches(model, ids: torch.Tensor, past):
         return None
     I, hd = d * cfg.mlp_scale, d // H
     good = True
+    keep = []
 
     def ptr(t, *shape, dtype=dt):
         nonlocal good
+        keep.append(t)
         good = good and t is not None and t.dtype == dtype and t.device == dev and t.shape == shape and t.is_contiguous()
         return t.data_ptr() if good else None
     arr = (LayerDesc * n)()
-    keep, out = [], []
+    out = []
     pos = hist_cap = fir_taps = None
     S = 0
     for layer, ld, entry in zip(model.layers, arr, past):
@@ -124,9 +127,7 @@ def step_on_caches(model, ids: torch.Tensor, past):
         else:
             if op.M_inputs.device != dev or op.d_in != d or op.config is not cfg:
                 return None
-            mit = op.m_inputs_t()
-            keep.append(mit)
-            ld.m_inputs_t = ptr(mit, d, d)
+            ld.m_inputs_t = ptr(op.m_inputs_t(), d, d)
             if lds:
                 a, ce, co = op.lds_params()
                 fir = op.lds_fir()
@@ -134,7 +135,6 @@ def step_on_caches(model, ids: torch.Tensor, past):
                 if fir_taps not in (None, taps) or S not in (0, a.numel()) or (taps == 0 and a0.numel() != 0):
                     return None
                 fir_taps, S = taps, a.numel()
-                keep += [a, ce, co, fir]
                 ld.lds_a, ld.lds_ce, ld.lds_co = (ptr(a, S, dtype=torch.float32), ptr(ce, S, d, dtype=torch.float32),
                                                   ptr(co, S, d, dtype=torch.float32))
                 ld.lds_state = ptr(a1, B, 2, S, d, dtype=torch.float32)
@@ -145,7 +145,6 @@ def step_on_caches(model, ids: torch.Tensor, past):
                 if a0.dim() != 3 or hist_cap not in (None, a0.shape[1]) or a1.numel() != 0 or pos >= a0.shape[1] or pos >= filt.shape[0]:
                     return None
                 hist_cap = a0.shape[1]
-                keep.append(filt)
                 ld.filt, ld.hist = ptr(filt, filt.shape[0], d), ptr(a0, B, hist_cap, d)
                 S = filt.shape[0]
         if not good:
@@ -281,23 +280,30 @@ class DecodeEngine:
         mode = cfg.resolved_stu_decode_mode()
         b0, b1 = ch.b0, ch.b1
         B = b1 - b0
-        keep = ch.keep.append
         n = len(model.layers)
+
+        def keep(t):
+            ch.keep.append(t)
+            return t
+
+        def ptr(t):      # held as long as the descriptor: a parametrized weight is a temporary of this access
+            return keep(t).data_ptr()
         arr = (LayerDesc * n)()
         hist_cap = 0
         fir_taps = 0
+        weights = []        # the projections of each layer, read once
         for i, layer in enumerate(model.layers):
             ld = arr[i]
-            ld.w_gate = layer.mlp.gate_proj.weight.data_ptr()
-            ld.w_up = layer.mlp.up_proj.weight.data_ptr()
-            ld.w_down = layer.mlp.down_proj.weight.data_ptr()
-            ld.mlp_norm_w = layer.mlp_norm.weight.data_ptr()
+            gate, up, down = (keep(p.weight) for p in (layer.mlp.gate_proj, layer.mlp.up_proj, layer.mlp.down_proj))
+            weights.append(dict(gate=gate, up=up, down=down))
+            ld.w_gate, ld.w_up, ld.w_down = gate.data_ptr(), up.data_ptr(), down.data_ptr()
+            ld.mlp_norm_w = ptr(layer.mlp_norm.weight)
             if isinstance(layer, STULayer):
                 stu = layer.stu
                 ld.kind = 0
-                ld.norm1_w = layer.stu_norm.weight.data_ptr()
-                mit = stu.m_inputs_t()
-                keep(mit)
+                ld.norm1_w = ptr(layer.stu_norm.weight)
+                mit = keep(stu.m_inputs_t())
+                weights[i]["m_inputs"] = mit
                 ld.m_inputs_t = mit.data_ptr()
                 hist, state, pos = caches[i]
                 if mode == "lds":
@@ -329,14 +335,15 @@ class DecodeEngine:
             elif isinstance(layer, AttentionLayer):
                 att = layer.attn
                 ld.kind = 1
-                ld.norm1_w = layer.attn_norm.weight.data_ptr()
-                ld.w_qkv = att.c_attn.weight.data_ptr()
-                ld.w_proj = att.c_proj.weight.data_ptr()
+                ld.norm1_w = ptr(layer.attn_norm.weight)
+                qkv, proj = keep(att.c_attn.weight), keep(att.c_proj.weight)
+                weights[i].update(qkv=qkv, proj=proj)
+                ld.w_qkv, ld.w_proj = qkv.data_ptr(), proj.data_ptr()
                 kr, vr, pos = caches[i]
                 kr, vr = kr[b0:b1], vr[b0:b1]
                 keep(kr), keep(vr)
                 ld.kring, ld.vring = kr.data_ptr(), vr.data_ptr()
-                ld.slopes = att.alibi_slopes.data_ptr()
+                ld.slopes = ptr(att.alibi_slopes)
             else:
                 raise TypeError(type(layer))
         m = ModelDesc()
@@ -353,8 +360,8 @@ class DecodeEngine:
         m.hist_nsplit_max = self.HIST_NSPLIT_MAX
         m.row0 = b0
         m.eps, m.softcap = float(cfg.rms_norm_eps), float(cfg.softcap or 0.0)
-        m.emb = model.lm_head.weight.data_ptr()
-        m.final_norm_w = model.norm.weight.data_ptr()
+        emb = keep(model.lm_head.weight)
+        m.emb, m.final_norm_w = emb.data_ptr(), ptr(model.norm.weight)
         m.layers = ctypes.cast(arr, ctypes.POINTER(LayerDesc))
 
         def buf(*shape, dtype=dt):
@@ -372,36 +379,32 @@ class DecodeEngine:
         m.samp_ws = buf((int(self.lib.fstu_sample_ws_bytes()) + 7) // 8, dtype=torch.int64).data_ptr()
         if dt == torch.bfloat16 and self.lib.fstu_glu_packed_supported(B, d, I):
             # gate/up projection over packed weights, one workgroup per CU with equal bytes each
-            for i, layer in enumerate(model.layers):
-                arr[i].wp_gate = self._pack(layer.mlp.gate_proj.weight, (i, "gate")).data_ptr()
-                arr[i].wp_up = self._pack(layer.mlp.up_proj.weight, (i, "up")).data_ptr()
+            for i, (ld, w) in enumerate(zip(arr, weights)):
+                ld.wp_gate, ld.wp_up = ptr(self._pack(w["gate"], (i, "gate"))), ptr(self._pack(w["up"], (i, "up")))
             m.glu_packed = 1
             if I % 512 == 0 and d % 16 == 0:
-                for i, layer in enumerate(model.layers):
-                    arr[i].wp_down = self._pack(layer.mlp.down_proj.weight, (i, "down")).data_ptr()
+                for i, (ld, w) in enumerate(zip(arr, weights)):
+                    ld.wp_down = ptr(self._pack(w["down"], (i, "down")))
                 m.down_packed = 1
             if B * (d + 8) * 2 <= 96 * 1024:
                 m.x2 = buf(B, d).data_ptr()     # second residual buffer: the MLP norm runs as the gate/up prologue
                 if mode == "lds" and d % 256 == 0 and m.down_packed and B * (d // 8) <= 1024 and I % 128 == 0:
                     # the add+norm between two layers runs as the prologue of the next layer's first projection
                     # (the down projection leaves 4 split-K slices for it): one launch less per layer
-                    for i, layer in enumerate(model.layers):
-                        if isinstance(layer, AttentionLayer):
-                            arr[i].wp_qkv = self._pack(layer.attn.c_attn.weight, (i, "qkv")).data_ptr()
+                    for i, (ld, w) in enumerate(zip(arr, weights)):
+                        if "qkv" in w:
+                            ld.wp_qkv = ptr(self._pack(w["qkv"], (i, "qkv")))
                     m.merge_norm = 1
         if dt == torch.bfloat16 and self.lib.fstu_mlp_packed_rows32_supported(B, d, I):
             # 17..32 rows: the MLP streams packed weights as two row tiles per weight fragment
-            for i, layer in enumerate(model.layers):
-                arr[i].wp_gate = self._pack(layer.mlp.gate_proj.weight, (i, "gate")).data_ptr()
-                arr[i].wp_up = self._pack(layer.mlp.up_proj.weight, (i, "up")).data_ptr()
-                arr[i].wp_down = self._pack(layer.mlp.down_proj.weight, (i, "down")).data_ptr()
-                if isinstance(layer, AttentionLayer):
-                    arr[i].wp_qkv = self._pack(layer.attn.c_attn.weight, (i, "qkv")).data_ptr()
-                    arr[i].wp_proj = self._pack(layer.attn.c_proj.weight, (i, "proj")).data_ptr()
+            for i, (ld, w) in enumerate(zip(arr, weights)):
+                ld.wp_gate, ld.wp_up, ld.wp_down = (ptr(self._pack(w[k], (i, k))) for k in ("gate", "up", "down"))
+                if "qkv" in w:
+                    ld.wp_qkv, ld.wp_proj = ptr(self._pack(w["qkv"], (i, "qkv"))), ptr(self._pack(w["proj"], (i, "proj")))
                 elif mode == "lds":
-                    arr[i].wp_m_inputs = self._pack(layer.stu.m_inputs_t(), (i, "m_inputs")).data_ptr()
+                    ld.wp_m_inputs = ptr(self._pack(w["m_inputs"], (i, "m_inputs")))
         if dt == torch.bfloat16 and self.lib.fstu_glu_packed_supported(min(B, _hip.MAX_DECODE_ROWS), d, V):
-            m.wp_emb = self._pack(model.lm_head.weight, "emb").data_ptr()      # the head streams a packed copy of the embedding
+            m.wp_emb = ptr(self._pack(emb, "emb"))      # the head streams a packed copy of the embedding
         ch.arr, ch.desc = arr, m
         if B > _hip.MAX_DECODE_ROWS:
             # first use of the tiled kernels outside any graph capture (their launch set-up raises an LDS limit once)

@@ -408,6 +408,41 @@ def test_one_call_step_equals_the_layers_own_calls(dtype, extra, rows):
                 assert float((a.float() - b.float()).abs().max()) <= tol * max(float(b.float().abs().max()), 1e-6)
 
 
+class _Scaled(torch.nn.Module):
+    def forward(self, w):
+        return w * 0.5
+
+
+@pytest.mark.parametrize("dtype,d", [(torch.bfloat16, 256), (torch.float32, 128)])
+def test_parametrized_projections_are_held_until_they_are_read(dtype, d):
+    """A parametrized weight is a new tensor on every access.  Scaling by 0.5 is exact, so the caches' one-call step and
+    generate() give the bits of a model whose weights were scaled beforehand."""
+    from torch.nn.utils import parametrize
+    kw = dict(seed=5, init="healthy", dtype=dtype, mlp_scale=2, n_embd=d, n_layers=4, n_heads=2, window_size=8, num_eigh=8,
+              seq_len=64, vocab_size=777)
+    _, _, plain = make_pair(**kw)
+    _, _, model = make_pair(**kw)
+    for scaled, layer in zip(plain.layers, model.layers):
+        names = ["mlp.gate_proj", "mlp.up_proj", "mlp.down_proj"] + (["attn.c_attn", "attn.c_proj"] if hasattr(layer, "attn") else [])
+        for name in names:
+            with torch.no_grad():
+                scaled.get_submodule(name).weight.mul_(0.5)
+            parametrize.register_parametrization(layer.get_submodule(name), "weight", _Scaled())
+    for rows in (3, 16, 20):
+        ids = prompt(rows, 10, 777, rows).cuda()
+        if rows <= 16:
+            outs = []
+            for m in (plain, model):
+                past, logits = m(ids[:, :6], use_cache=True).past_key_values, []
+                for t in range(6, 10):
+                    out = m(ids[:, t:t + 1], past_key_values=past, use_cache=True)
+                    past = out.past_key_values
+                    logits.append(out.logits)
+                outs.append(torch.cat(logits, 1))
+            assert torch.equal(*outs)
+        assert torch.equal(model.generate(ids, max_length=20, do_sample=False), plain.generate(ids, max_length=20, do_sample=False))
+
+
 def test_forward_accepts_reference_style_kv_cache():
     from flash_stu import Attention, FlashSTUConfig
     cfg = FlashSTUConfig(n_embd=128, n_heads=2, n_layers=2, seq_len=64, window_size=6, vocab_size=11, mlp_scale=2,
