@@ -174,7 +174,8 @@ def step_on_caches(model, ids: torch.Tensor, past):
     for name, size in sizes.items():
         setattr(m, name, at)
         at += (size + 255) // 256 * 256
-    _hip._check(_hip.load().fstu_decode_logits(ctypes.byref(m), ids.data_ptr(), ids.stride(0), pos, _hip._stream()),
+    ids = ids.contiguous()       # one token expanded over the rows has a row stride of 0
+    _hip._check(_hip.load().fstu_decode_logits(ctypes.byref(m), ids.data_ptr(), 1, pos, _hip._stream()),
                 "fstu_decode_logits")
     return logits, tuple((a0, a1, pos_t + 1) for a0, a1, pos_t in out)
 

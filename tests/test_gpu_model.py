@@ -443,6 +443,21 @@ def test_parametrized_projections_are_held_until_they_are_read(dtype, d):
         assert torch.equal(model.generate(ids, max_length=20, do_sample=False), plain.generate(ids, max_length=20, do_sample=False))
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_step_on_caches_takes_expanded_ids(dtype):
+    """One token for all rows as an expanded view, or as a column of a longer buffer: the logits of a dense column."""
+    _, _, model = make_pair(seed=5, init="healthy", dtype=dtype, mlp_scale=2, n_embd=256, n_layers=4, n_heads=2, window_size=8,
+                            num_eigh=8, seq_len=64, vocab_size=777)
+    for rows in (1, 3):
+        ids = prompt(rows, 6, 777, rows).cuda()
+        past = model(ids, use_cache=True).past_key_values
+        token = ids[0, 2]
+        step = lambda column: model(column, past_key_values=tuple(tuple(t.clone() for t in c) for c in past), use_cache=True).logits
+        want = step(token.repeat(rows, 1))
+        for column in (token.expand(rows, 1), token.reshape(1, 1).expand(rows, 4)[:, 2:3], token.repeat(rows, 5)[:, 3:4]):
+            assert torch.equal(step(column), want)
+
+
 def test_forward_accepts_reference_style_kv_cache():
     from flash_stu import Attention, FlashSTUConfig
     cfg = FlashSTUConfig(n_embd=128, n_heads=2, n_layers=2, seq_len=64, window_size=6, vocab_size=11, mlp_scale=2,
