@@ -59,9 +59,17 @@ def pick_ksplit_down(I: int) -> int:
     return 1
 
 
+# What the layers' own calls run, as defined when the package was imported
+_AS_DEFINED = [(cls, name, cls.__dict__[name]) for cls, names in (
+    (torch.nn.Module, ("__call__", "_call_impl")), (RMSNorm, ("forward", "add_then_norm")), (MLP, ("forward",)),
+    (Attention, ("forward",)), (STU, ("forward", "_step")), (STULayer, ("forward",)), (AttentionLayer, ("forward",)))
+    for name in names]
+_OWN_NAMES = {name for _, name, _ in _AS_DEFINED}
+
+
 def _as_written(m, cls) -> bool:
-    """The module is of this class and calling it runs this class's forward and nothing else."""
-    return type(m) is cls and not m._forward_hooks and not m._forward_pre_hooks and "forward" not in m.__dict__
+    """The module is of this class and calling it runs this class's methods and nothing else."""
+    return type(m) is cls and not m._forward_hooks and not m._forward_pre_hooks and _OWN_NAMES.isdisjoint(m.__dict__)
 
 
 @torch.no_grad()
@@ -77,7 +85,8 @@ def step_on_caches(model, ids: torch.Tensor, past):
     mod = torch.nn.modules.module
     if not (ids.dim() == 2 and ids.shape[1] == 1 and 1 <= ids.shape[0] <= _hip.MAX_DECODE_ROWS and ids.dtype == torch.int64
             and DecodeEngine.supports(cfg) and isinstance(past, (tuple, list)) and len(past) == len(model.layers) > 0
-            and not mod._global_forward_hooks and not mod._global_forward_pre_hooks and _as_written(model.norm, RMSNorm)):
+            and not mod._global_forward_hooks and not mod._global_forward_pre_hooks and _as_written(model.norm, RMSNorm)
+            and all(cls.__dict__.get(name) is f for cls, name, f in _AS_DEFINED)):
         return None
     emb = model.lm_head.weight
     dt, dev, B, (V, d) = emb.dtype, emb.device, ids.shape[0], emb.shape
@@ -106,6 +115,7 @@ def step_on_caches(model, ids: torch.Tensor, past):
         op, norm1 = (layer.stu, layer.stu_norm) if stu_layer else (layer.attn, layer.attn_norm)
         mlp, norm2 = layer.mlp, layer.mlp_norm
         if not (_as_written(op, STU if stu_layer else Attention) and _as_written(norm1, RMSNorm) and type(norm2) is RMSNorm
+                and _OWN_NAMES.isdisjoint(norm2.__dict__)
                 and _as_written(mlp, MLP) and norm1.eps == eps and norm2.eps == eps and mlp.gate_proj.bias is None):
             return None
         a0, a1, pos_t = entry

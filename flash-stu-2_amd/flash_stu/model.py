@@ -20,6 +20,7 @@ import torch.nn.functional as F
 
 from . import _hip
 from .config import FlashSTUConfig
+from .engine import DecodeEngine, step_on_caches
 from .layers.attention_layer import AttentionLayer
 from .layers.stu_layer import STULayer
 from .modules.attention import Attention
@@ -157,8 +158,8 @@ class FlashSTU(nn.Module):
             raise _hip.FlashSTUHipError("input_ids must be on the GPU: this model has no CPU path")
         hidden = [] if output_hidden_states else None
         logits = None
-        if past_key_values is not None and hidden is None and input_ids.dim() == 2 and input_ids.shape[1] == 1:
-            from .engine import step_on_caches
+        if (past_key_values is not None and hidden is None and input_ids.dim() == 2 and input_ids.shape[1] == 1
+                and all(getattr(type(self), n) is f and n not in self.__dict__ for n, f in _STEP_PARTS.items())):
             done = step_on_caches(self, input_ids, past_key_values)
             if done is not None:
                 logits, cache = done
@@ -200,7 +201,6 @@ class FlashSTU(nn.Module):
 
     # ------------------------------------------------------------ generate
     def decode_engine(self):
-        from .engine import DecodeEngine
         if self._engine is None:
             self._engine = DecodeEngine(self)
         return self._engine
@@ -218,7 +218,6 @@ class FlashSTU(nn.Module):
         n_new = max_length - P
         if n_new <= 0:
             return input_ids
-        from .engine import DecodeEngine
         # Sequences that outgrow seq_len leave the stateful paths: the filters end at lag seq_len, so the reference
         # re-runs the last seq_len tokens without a cache from there on (model.py:250-255), and so does the loop below.
         if use_cache and max_length <= self.config.seq_len and DecodeEngine.supports(self.config):
@@ -348,3 +347,7 @@ class FlashSTU(nn.Module):
             if isinstance(layer, STULayer):
                 layer.stu.phi.copy_(model.phi)
         return model
+
+
+# the pieces of forward() that the one-call step stands for
+_STEP_PARTS = {n: FlashSTU.__dict__[n] for n in ("_embed", "_run_layers", "_head")}

@@ -458,6 +458,41 @@ def test_step_on_caches_takes_expanded_ids(dtype):
             assert torch.equal(step(column), want)
 
 
+@pytest.mark.parametrize("what", ["MLP.forward", "RMSNorm.add_then_norm", "STU._step", "instance", "subclass", "model"])
+def test_replaced_methods_run_in_a_step_on_caches(what, monkeypatch):
+    """A method replaced on a class, an instance or in a subclass is called for one position on caches too."""
+    from flash_stu import FlashSTU
+    from flash_stu.modules.norm import RMSNorm
+    from flash_stu.modules.stu import STU
+    from flash_stu.modules.swiglu import MLP
+    _, _, model = make_pair(seed=5, init="healthy", dtype=torch.bfloat16, mlp_scale=2, n_embd=128, n_layers=4, n_heads=2,
+                            window_size=8, num_eigh=8, seq_len=64, vocab_size=777)
+    ids = prompt(2, 7, 777, 1).cuda()
+    past = model(ids[:, :6], use_cache=True).past_key_values
+    calls = []
+
+    def counted(f):
+        def g(*a, **k):
+            calls.append(1)
+            return f(*a, **k)
+        return g
+    layer = model.layers[0]
+    if what == "instance":
+        monkeypatch.setattr(layer.mlp_norm, "add_then_norm", counted(layer.mlp_norm.add_then_norm))
+    elif what == "model":
+        monkeypatch.setattr(model, "_head", counted(model._head))
+    elif what == "subclass":
+        class Other(FlashSTU):
+            _run_layers = counted(FlashSTU._run_layers)
+        model.__class__ = Other
+    else:
+        cls, name = what.split(".")
+        cls = {"MLP": MLP, "RMSNorm": RMSNorm, "STU": STU}[cls]
+        monkeypatch.setattr(cls, name, counted(getattr(cls, name)))
+    model(ids[:, 6:7], past_key_values=past, use_cache=True)
+    assert len(calls) == {"MLP.forward": 4, "RMSNorm.add_then_norm": 4, "STU._step": 2}.get(what, 1)
+
+
 def test_forward_accepts_reference_style_kv_cache():
     from flash_stu import Attention, FlashSTUConfig
     cfg = FlashSTUConfig(n_embd=128, n_heads=2, n_layers=2, seq_len=64, window_size=6, vocab_size=11, mlp_scale=2,
