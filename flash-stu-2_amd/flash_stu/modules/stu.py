@@ -28,6 +28,28 @@ from ..utils.lds_fit import check_lds_fit, fit_even_lag_lds
 FFT_MIN_T = 32     # shorter inputs take the time-domain kernel (a 64-point transform would be mostly padding)
 
 
+def _end_of_stream(device):
+    """What the current stream has been given so far, for a tensor that outlives the call: (event, stream), or None."""
+    if device.type != "cuda" or torch.cuda.is_current_stream_capturing():
+        return None
+    stream, event = torch.cuda.current_stream(device), torch.cuda.Event()
+    event.record(stream)
+    return event, stream
+
+
+def _stay_behind(made):
+    """Orders the current stream behind `made`; returns None once that has been reached."""
+    if torch.cuda.is_current_stream_capturing():
+        return made
+    event, stream = made
+    if event.query():
+        return None
+    now = torch.cuda.current_stream(stream.device)
+    if now != stream:
+        now.wait_event(event)
+    return made
+
+
 class STU(nn.Module):
     def __init__(self, config, phi: torch.Tensor, n: int, feature_dim: Optional[int] = None) -> None:
         super().__init__()
@@ -56,13 +78,15 @@ class STU(nn.Module):
 
     # ---- tensors derived from the parameters, rebuilt when a parameter changes; an entry holds the storage that it was
     # made from, so that no other tensor can come to lie at the address it is recognised by (a parametrized weight is a
-    # new tensor on every access)
+    # new tensor on every access).  A call on another stream than the one that launched the copy waits for it.
     def _cached(self, key, params, build):
         ver = tuple((p._version, p.data_ptr()) for p in params)
         hit = self._derived.get(key)
         if hit is None or hit[0] != ver:
-            hit = (ver, build(), [p.detach() for p in params])
+            hit = [ver, build(), [p.detach() for p in params], _end_of_stream(params[0].device)]
             self._derived[key] = hit
+        elif hit[3] is not None:
+            hit[3] = _stay_behind(hit[3])
         return hit[1]
 
     def decode_mode(self) -> str:

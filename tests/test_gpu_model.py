@@ -493,6 +493,35 @@ def test_replaced_methods_run_in_a_step_on_caches(what, monkeypatch):
     assert len(calls) == {"MLP.forward": 4, "RMSNorm.add_then_norm": 4, "STU._step": 2}.get(what, 1)
 
 
+def test_derived_tensors_are_complete_on_every_stream():
+    """Transposed weights and filter spectra that one stream has only just been given, read by the next call on another: the
+    values of a model that nothing else runs beside."""
+    from flash_stu import STU, FlashSTUConfig
+    cfg = FlashSTUConfig(n_embd=256, n_heads=4, n_layers=2, seq_len=512, num_eigh=8, vocab_size=64, torch_dtype=torch.bfloat16)
+    g = torch.Generator().manual_seed(2)
+    phi, x = torch.randn(512, 8, generator=g).bfloat16(), torch.randn(2, 300, 256, generator=g).bfloat16().cuda()
+    stu = STU(cfg, phi, 1024).cuda()
+    other, big = torch.cuda.Stream(), torch.randn(4096, 4096, device="cuda")
+    for turn in range(3):
+        with torch.no_grad():
+            for p in stu.parameters():
+                p.copy_(torch.randn(p.shape, generator=g))
+        fresh = STU(cfg, phi, 1024).cuda()
+        fresh.load_state_dict(stu.state_dict())
+        want = fresh(x)
+        torch.cuda.synchronize()
+        with torch.cuda.stream(other):
+            for _ in range(8):                  # some milliseconds in front of the copies
+                big @ big
+            there = stu(x)
+        here = stu(x)
+        assert torch.equal(here, want)
+        torch.cuda.current_stream().wait_stream(other)
+        assert torch.equal(there, want)
+        torch.cuda.synchronize()
+        assert torch.equal(stu(x), want) and stu._derived["mit"][3] is None
+
+
 def test_forward_accepts_reference_style_kv_cache():
     from flash_stu import Attention, FlashSTUConfig
     cfg = FlashSTUConfig(n_embd=128, n_heads=2, n_layers=2, seq_len=64, window_size=6, vocab_size=11, mlp_scale=2,
