@@ -92,14 +92,16 @@ def _convolve_grads(ctx, u, v, spec, gp, gm, branches):
     """Gradients of the convolution in u and v, formed in fp32 whatever the input dtype (the reference differentiates
     through an fp32 FFT, stu_utils.py:226-228) and rounded once at the end.  branches 0: gp is the gradient of
     plus + minus; 1: of plus alone; 2: gp and gm are those of plus and minus.  With the forward's spectra one launch of
-    the gradient kernel; without (the lengths of the time-domain kernel) as convolutions: the minus branch
+    the gradient kernel; without (the lengths of the time-domain kernel), and where the gradients are to be differentiated
+    themselves (create_graph=True: the composition carries its graph), as convolutions: the minus branch
     sgn * conv(sgn * u, v) equals conv(u, v * (-1)^s), and
       d/du: correlation with the filter     = time-reversed convolution of the time-reversed gradient
       d/dv: correlation of gradient and u   = per batch row, convolution of the time-reversed gradient with that
             row's input as the filter, read backwards; summed over the batch in fp32."""
     from .. import _hip
     want_u, want_v = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
-    if spec is not None:
+    graph = torch.is_grad_enabled()
+    if spec is not None and not graph:
         return _hip.stu_conv_fft_grad(gp.contiguous(), gm.contiguous() if branches == 2 else None, u.contiguous(), spec,
                                       v.shape[0], branches, want_u, want_v)
     both = branches != 1
@@ -107,13 +109,16 @@ def _convolve_grads(ctx, u, v, spec, gp, gm, branches):
     B, T, d = u.shape
     L = v.shape[0]
     uf, vf = u.float(), v.float()
+
+    def conv(a, f):
+        return _ApproxConvolve.apply(a, f, False)[0] if graph else _causal_conv(a, f)
     gpf = gp.float().flip(1).contiguous()
     gmf = gm.float().flip(1).contiguous() if both else None
     gu = gv = None
     if want_u:
-        gu = _causal_conv(gpf, vf)
+        gu = conv(gpf, vf)
         if both:
-            gu = gu + _causal_conv(gmf, vf * _alt_sign(L, vf))
+            gu = gu + conv(gmf, vf * _alt_sign(L, vf))
         gu = gu.flip(1).to(u.dtype)
     if want_v:
         taps = min(L, T)
@@ -121,9 +126,9 @@ def _convolve_grads(ctx, u, v, spec, gp, gm, branches):
         acc_m = torch.zeros_like(acc_p) if both else None
         for b in range(B):
             ub = uf[b].contiguous()                              # (T,d): this row's input as the filter
-            acc_p += _causal_conv(gpf[b:b + 1], ub)[0]
+            acc_p += conv(gpf[b:b + 1], ub)[0]
             if both:
-                acc_m += _causal_conv(gmf[b:b + 1], ub)[0]
+                acc_m += conv(gmf[b:b + 1], ub)[0]
         gv = torch.zeros(L, d, dtype=torch.float32, device=u.device)
         gv[:taps] = acc_p.flip(0)[:taps]                         # lag s sits at position T-1-s
         if both:

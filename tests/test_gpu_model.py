@@ -163,6 +163,35 @@ def test_stu_forward_differentiable_gradients(hankel):
         assert float((got.cpu() - want).abs().max()) <= 2e-4 * float(want.abs().max())
 
 
+@pytest.mark.parametrize("hankel", [False, True])
+@pytest.mark.parametrize("T", [20, 50])
+def test_stu_forward_differentiable_second_order(hankel, T):
+    """create_graph=True through the whole operator, at a length of the time-domain kernel and one of the transforms: gradients
+    of a penalty on the gradients against autograd through the oracle.  Each order of differentiation is one more pass of
+    fp32 convolutions and products: five times the bound of the first-order test."""
+    from flash_stu import STU, FlashSTUConfig
+    L, K, d, B = 64, 8, 32, 2
+    cfg = FlashSTUConfig(n_embd=d, n_heads=2, n_layers=2, seq_len=L, num_eigh=K, vocab_size=11, torch_dtype=torch.float32,
+                         use_hankel_L=hankel)
+    phi = torch.tensor(O.get_spectral_filters_f64(L, K, hankel)).float()
+    n = O.nearest_power_of_two(2 * L - 1, True)
+    g = torch.Generator().manual_seed(18)
+    Mi, Mf = torch.randn(d, d, generator=g) / d ** 0.5, torch.randn(K, d, generator=g) / K ** 0.5
+    x, wgt = torch.randn(B, T, d, generator=g), torch.randn(B, T, d, generator=g)
+    stu = STU(cfg, phi.cuda(), n).cuda()
+    with torch.no_grad():
+        stu.M_inputs.copy_(Mi)
+        stu.M_filters.copy_(Mf)
+    p = {"M_inputs": Mi.clone().requires_grad_(True), "M_filters": Mf.clone().requires_grad_(True)}
+    seconds = []
+    for leaves, y, w in (((x.cuda().requires_grad_(True), stu.M_inputs, stu.M_filters), stu.forward_differentiable, wgt.cuda()),
+                         ((x.clone().requires_grad_(True), *p.values()), lambda t: O.stu_forward(t, phi, p, n, use_approx=True, use_hankel_L=hankel), wgt)):
+        first = torch.autograd.grad((y(leaves[0]).square() * w).sum(), leaves, create_graph=True)
+        seconds.append(torch.autograd.grad(sum(t.square().sum() / t.detach().square().sum() for t in first), leaves))
+    for got, want in zip(*seconds):
+        assert float((got.cpu() - want).abs().max()) <= 1e-3 * float(want.abs().max())
+
+
 @pytest.mark.parametrize("B,T,d", [(1, 128, 128), (3, 320, 256), (2, 97, 128)])
 def test_input_projection_gradients(B, T, d):
     """x @ M_inputs and its gradients on the matrix-core kernels (and, for rows they do not take, the library's product)
