@@ -344,7 +344,8 @@ def gemm_any(a: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = Non
         out = torch.empty(M, N, dtype=a.dtype, device=a.device)
     if out.shape != (M, N) or out.stride(1) != 1 or out.dtype != a.dtype:
         raise FlashSTUHipError("gemm_any: out must be (M,N) with contiguous rows")
-    # a size-1 dimension may carry any stride: give it a positive one
+    # a size-1 dimension may carry any stride: give it a positive one; an expanded one is laid out
+    a, w = (t.contiguous() if any(n > 1 and st == 0 for n, st in zip(t.shape, t.stride())) else t for t in (a, w))
     sam, sak = max(a.stride(0), 1), max(a.stride(1), 1)
     swn, swk = max(w.stride(0), 1), max(w.stride(1), 1)
     _check(load().fstu_gemm_any(_p(a), sam, sak, _p(w), swn, swk, _p(out), out.stride(0), M, N, K, _dt(a), _stream()),

@@ -229,6 +229,17 @@ def test_gemm_bf16_transposed_activations(hip, nb, M, N, K):
         hip.gemm_ta(Ad.transpose(1, 2), Wd)  # M not the contiguous index
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_gemm_any_expanded_operands(hip, dtype):
+    """Rows, features or a reduction index that are one value repeated: the bits of the same operands laid out."""
+    g = gen(97)
+    x, W = dev(torch.randn(40, 36, generator=g).to(dtype)), dev(torch.randn(50, 36, generator=g).to(dtype))
+    for a, w in ((x[:1].expand(40, 36), W), (x, W[:1].expand(50, 36)), (x[:, :1].expand(40, 36), W), (x, W[:, :1].expand(50, 36)),
+                 (x[:1, :1].expand(40, 36), W.t().contiguous().t())):
+        assert torch.equal(hip.gemm_any(a, w), hip.gemm_any(a.contiguous(), w.contiguous()))
+        assert torch.equal(hip.linear(a, w.contiguous()), hip.linear(a.contiguous(), w.contiguous()))
+
+
 @pytest.mark.parametrize("nb,M,N,K,slices", [(1, 128, 132, 4096, 8), (3, 256, 260, 6144, 12), (1, 384, 1024, 3072, 6)])
 def test_gemm_bf16_in_slices(hip, nb, M, N, K, slices):
     """Few output tiles and a long K: both prompt GEMMs in slices of K, plain and with the residual, ragged tiles and strided
