@@ -18,6 +18,7 @@ LIB_PATH = os.path.join(os.path.dirname(_HERE), "csrc", "libflashstu_hip.so")
 
 FSTU_F32, FSTU_BF16 = 0, 1
 MAX_DECODE_ROWS = 16
+GEMM_MAX_STRIDE = 1 << 22     # elements between rows that the matrix-core GEMM's 32-bit offsets cover
 
 _lib = None
 
@@ -285,11 +286,12 @@ def bias_act(y: torch.Tensor, bias: Optional[torch.Tensor], silu: bool = False) 
 
 def gemm_supported(x2: torch.Tensor, weight: torch.Tensor, plain: bool = False) -> bool:
     """Shapes the matrix-core prompt GEMM takes: bf16, K a multiple of 32, N a multiple of 4 (plain: any N, for a product
-    without the gate or the residual as its epilogue), rows 16-byte aligned."""
+    without the gate or the residual as its epilogue), rows 16-byte aligned, not overlapping and within the kernel's 32-bit
+    tile offsets."""
     K = x2.shape[-1]
     return (x2.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x2.dim() == 2 and K % 32 == 0 and
             (plain or weight.shape[0] % 4 == 0) and weight.is_contiguous() and x2.stride(1) == 1 and x2.stride(0) % 8 == 0 and
-            x2.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0)
+            K <= x2.stride(0) < GEMM_MAX_STRIDE and x2.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0)
 
 
 def gemm(x2: torch.Tensor, weight: torch.Tensor, up_weight: Optional[torch.Tensor] = None,

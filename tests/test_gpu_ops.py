@@ -240,6 +240,21 @@ def test_gemm_any_expanded_operands(hip, dtype):
         assert torch.equal(hip.linear(a, w.contiguous()), hip.linear(a.contiguous(), w.contiguous()))
 
 
+@pytest.mark.parametrize("N", [50, 52])
+def test_linear_rows_of_any_stride(hip, N):
+    """Rows that overlap or lie further apart than the matrix-core GEMM's offsets reach go to the general kernel, whatever the
+    feature count: within its bound of the same rows laid out (K = 64 exact products summed in fp32, one rounding of 2^-8)."""
+    g = gen(98)
+    W = dev(torch.randn(N, 64, generator=g).bfloat16())
+    base = dev(torch.randn(40 * 8 + 64, generator=g).bfloat16())
+    far = torch.empty(17 * (1 << 22) + 64, dtype=torch.bfloat16, device="cuda").as_strided((18, 64), (1 << 22, 1))
+    far.copy_(torch.randn(18, 64, generator=g).bfloat16())
+    for x in (base.as_strided((40, 64), (8, 1)), base[:64].expand(40, 64), far):
+        ref = x.double() @ W.double().t()
+        bound = 2.0 ** -8 * ref.abs() + 64 * 2.0 ** -23 * (x.double().abs() @ W.double().abs().t())
+        assert bool(((hip.linear(x, W).double() - ref).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("nb,M,N,K,slices", [(1, 128, 132, 4096, 8), (3, 256, 260, 6144, 12), (1, 384, 1024, 3072, 6)])
 def test_gemm_bf16_in_slices(hip, nb, M, N, K, slices):
     """Few output tiles and a long K: both prompt GEMMs in slices of K, plain and with the residual, ragged tiles and strided
