@@ -92,6 +92,27 @@ def test_graph_replay_equals_eager_steps(do_sample):
     del junk
 
 
+@pytest.mark.parametrize("do_sample", [False, True])
+@pytest.mark.parametrize("rows,d", [(33, 256), (40, 128)])
+def test_several_chunks_replay_graphs(rows, d, do_sample, monkeypatch):
+    """More rows than one chunk holds (a wide one of 32 rows and one of 1; three of up to 16): runs of single-step graphs, of
+    8-step graphs alone and of both give the tokens of the steps launched one by one, and are runs of graphs."""
+    from flash_stu.engine import DecodeEngine
+    _, _, model = make_pair(seed=7, init="healthy", dtype=torch.bfloat16, mlp_scale=2, n_embd=d, n_layers=4, n_heads=2,
+                            window_size=8, num_eigh=8, seq_len=64, vocab_size=1001)
+    ids = prompt(rows, 5, 1001, 9).cuda()
+    launches = []
+    step = DecodeEngine.graph_step
+    monkeypatch.setattr(DecodeEngine, "graph_step", lambda self, *a: (launches.append(self.graph_steps), step(self, *a)))
+    for todo, graphs in ((2, [1] * 2), (9, [1] * 9), (31, [1] * 31), (32, [8] * 4), (37, [8] * 4 + [1] * 5)):
+        kw = dict(max_length=5 + 1 + todo, do_sample=do_sample, temperature=0.9, top_k=20, seed=5)
+        want = model.generate(ids, use_graph=False, **kw)
+        assert not launches
+        assert torch.equal(model.generate(ids, **kw), want)
+        assert len(model.decode_engine().chunks) == (2 if d == 256 else 3) and launches == graphs
+        launches.clear()
+
+
 @pytest.mark.parametrize("dtype,mode", [(torch.bfloat16, "lds"), (torch.float32, "lds"), (torch.float32, "history")])
 def test_scan_prefill_against_oracle_and_fft_prefill(dtype, mode):
     """stu_prefill_mode='scan' (the distilled recurrence over the prompt instead of the FFT convolution): prompt logits
