@@ -400,10 +400,16 @@ template <int MODE, int RB, int NF>
 static void launch_f32_u(const LinArgs& a, int ksplit, hipStream_t s) {
   constexpr int NWV = f32_waves<MODE, RB>();
   dim3 grid((a.N + NWV * NF - 1) / (NWV * NF), ksplit);
-  if (a.kw <= 256)
-    hipLaunchKernelGGL((linear_f32_kernel<MODE, RB, NF, 1>), grid, dim3(NWV * 64), 0, s, (const float*)a.x, (const float*)a.W, (const float*)a.W2, (float*)a.y, a.best, a.ldx, a.ldy, a.rows, a.N, a.K, a.kw, a.temperature);
-  else
-    hipLaunchKernelGGL((linear_f32_kernel<MODE, RB, NF, 2>), grid, dim3(NWV * 64), 0, s, (const float*)a.x, (const float*)a.W, (const float*)a.W2, (float*)a.y, a.best, a.ldx, a.ldy, a.rows, a.N, a.K, a.kw, a.temperature);
+  // The head's large workgroups leave a thread 128 registers: two chunks ahead fit them up to two rows (four rows and more
+  // spilled; 50257 features, K = 1024, us with two chunks / one: 4 rows 207 / 44, 8 rows 553 / 65, 16 rows 296 / 150;
+  // K = 512, 8 rows 263 / 42).
+  if constexpr (MODE != LIN_ARGMAX || RB <= 2) {
+    if (a.kw > 256) {
+      hipLaunchKernelGGL((linear_f32_kernel<MODE, RB, NF, 2>), grid, dim3(NWV * 64), 0, s, (const float*)a.x, (const float*)a.W, (const float*)a.W2, (float*)a.y, a.best, a.ldx, a.ldy, a.rows, a.N, a.K, a.kw, a.temperature);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((linear_f32_kernel<MODE, RB, NF, 1>), grid, dim3(NWV * 64), 0, s, (const float*)a.x, (const float*)a.W, (const float*)a.W2, (float*)a.y, a.best, a.ldx, a.ldy, a.rows, a.N, a.K, a.kw, a.temperature);
 }
 // Features per wave: one where the features are few (more waves), else as many as the sums of all rows leave registers for
 template <int MODE, int RB>
