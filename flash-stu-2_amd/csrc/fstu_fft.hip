@@ -532,18 +532,22 @@ fft_slab_kernel(const T* __restrict__ x, size_t x_sb, size_t x_sc, const cpx* __
 // ---------------------------------------------------------------- any strides
 // The same for operands of any strides: element (b, t, c) of x at x[b*x_sb + t*x_st + c*x_sc], of the k-th output at
 // y[b*y_sb + t*y_st + k*y_sk + c*y_sc].  Pairs pass through the columns' LDS so that the lanes of a memory access run
-// along the channels.
+// along the channels.  A workgroup takes the filters of its slice of the bank, kper of them: few channels and rows alone
+// are too few workgroups for the chip, and a slice more costs one forward transform beside the two inverse ones of each
+// of its filters.  24 filters into (B, T, K, d), both branches, us with the whole bank per workgroup / in slices (the call's
+// host side is 38): fp32 1 x 64 x 256 132 / 38, 2 x 100 x 256 140 / 38, 1 x 1000 x 256 226 / 53, 1 x 2048 x 256 247 / 84.
 template <typename T, int LOGN>
 __global__ void __launch_bounds__(fft_threads<LOGN>(), 4)
 fft_conv_kernel(const T* __restrict__ x, size_t x_sb, size_t x_st, size_t x_sc, const cpx* __restrict__ spec,
                 T* __restrict__ y, T* __restrict__ y2, size_t y_sb, size_t y_st, size_t y_sk, size_t y_sc,
-                const cpx* __restrict__ tw, int Tn, int d, int K, int mode, int xcd_remap) {
+                const cpx* __restrict__ tw, int Tn, int d, int K, int kper, int mode, int xcd_remap) {
   extern __shared__ cpx fft_lds[];
   using W = Half<LOGN>;
   constexpr int N = W::N, LC = fft_lcols<LOGN>(), COLS = 1 << LC, NT = fft_threads<LOGN>();
   int bx = blockIdx.x;
   if (xcd_remap) bx = (bx & 7) * (gridDim.x >> 3) + (bx >> 3);   // consecutive channel groups share an XCD
   const int c0 = bx * COLS, b = blockIdx.y, ncol = min(COLS, d - c0);
+  const int k0 = blockIdx.z * kper, k1 = min(K, k0 + kper);
   float* rec = (float*)(fft_lds + (size_t)COLS * W::STRIDE);
   const T* xb = x + (size_t)b * x_sb + (size_t)c0 * x_sc;
   for (int idx = threadIdx.x; idx < COLS * (N / 2); idx += NT) {
@@ -564,8 +568,8 @@ fft_conv_kernel(const T* __restrict__ x, size_t x_sb, size_t x_st, size_t x_sc, 
   for (int k = 0; k < 8; ++k) z[k] = col[phys(point<LOGN>(u, k))];
   __syncthreads();
   fft_forward<LOGN>(col, tw, u, z, xs);
-  const cpx* sp = spec + (K == 1 ? (size_t)min(c0 + mycol, d - 1) * (2 * N) : 0) + 2 * u;
-  for (int k = 0; k < K; ++k, sp += 2 * N) {
+  const cpx* sp = spec + (size_t)(K == 1 ? min(c0 + mycol, d - 1) : k0) * (2 * N) + 2 * u;
+  for (int k = k0; k < k1; ++k, sp += 2 * N) {
     cpx v[16], e[8], o[8];
     float prev[8];
     product16<LOGN>(sp, xs, v);
@@ -1096,13 +1100,17 @@ static int conv_fft_launch(const char* name, const void* x, int64_t x_sb, int64_
     FSTU_CHECK_LAUNCH(name);
     return FSTU_OK;
   }
+  // slices of the bank up to two workgroups per compute unit, where there is not one (fp32, 24 filters, both branches, us
+  // one / two slices: 4 x 1000 x 768, 384 workgroups, 396 / 409, 1 x 4096 x 512, 256 workgroups, 413 / 529)
   const int gx = (d + cols - 1) / cols;
-  dim3 grid(gx, B);
+  const long long groups = (long long)gx * B;
+  const int slices = groups >= 256 ? 1 : (int)(512 / groups), kper = slices >= K ? 1 : (K + slices - 1) / slices;
+  dim3 grid(gx, B, (K + kper - 1) / kper);
   const int remap = (gx % 8 == 0) ? 1 : 0;
   FSTU_DISPATCH_DTYPE(dtype, name,
                       FFT_LAUNCH(logn - 1, FFT_PLAIN, grid, name, (const T*)x, (size_t)x_sb, (size_t)x_st,
                                  (size_t)x_sc, (const cpx*)spec, (T*)y, (T*)y2, (size_t)y_sb, (size_t)y_st, (size_t)y_sk,
-                                 (size_t)y_sc, (const cpx*)tw, T_, d, K, mode, remap));
+                                 (size_t)y_sc, (const cpx*)tw, T_, d, K, kper, mode, remap));
   FSTU_CHECK_LAUNCH(name);
   return FSTU_OK;
 }

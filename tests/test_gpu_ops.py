@@ -454,6 +454,24 @@ def test_stu_conv_fft(hip, dtype, B, T, d, L):
     check(hip.stu_conv_fft(dev(xp), spec1, single_branch=True), plus, dtype, frac=0.05)
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("B,T,d,K", [(1, 40, 3, 2), (1, 64, 256, 24), (2, 100, 72, 7), (3, 300, 200, 24), (1, 1000, 256, 24), (40, 33, 256, 5)])
+def test_stu_conv_bank_in_slices(hip, dtype, B, T, d, K):
+    """The filter bank into (B,T,K,d): one filter, several and all of them per workgroup, both branches and one, the same bits
+    as the slab kernel's, which runs through the bank in one go; nothing is written beside."""
+    g = gen(T + K)
+    x, phi = dev(torch.randn(B, T, d, generator=g).to(dtype)), dev((torch.randn(T, K, generator=g) / math.sqrt(T)).to(dtype))
+    spec = hip.stu_fft_filter(phi, hip.fft_length(T))
+    xt = x.transpose(1, 2).contiguous().transpose(1, 2)
+    for both in (True, False):
+        u = [torch.full((B, T, K, d + 1), 9.0, dtype=dtype, device="cuda") for _ in range(2 if both else 1)]
+        hip.stu_conv_bank_fft(xt, spec, u[0][..., :d], u[1][..., :d] if both else None)
+        slab = [torch.empty(B, K, d, T, dtype=dtype, device="cuda") for _ in u]
+        hip.stu_conv_bank_fft(xt, spec, slab[0].permute(0, 3, 1, 2), slab[1].permute(0, 3, 1, 2) if both else None)
+        for a, b in zip(u, slab):
+            assert torch.equal(a[..., :d], b.permute(0, 3, 1, 2)) and bool((a[..., d] == 9.0).all())
+
+
 def test_stu_conv_fft_equals_direct_fp32(hip):
     """Both forms of the library on the same input: equal to fp32 round-off, and a delta returns the filter."""
     g = gen(21)
