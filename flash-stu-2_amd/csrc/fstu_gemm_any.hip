@@ -5,6 +5,7 @@
 // Accumulation in fp32 on the fp32 matrix instructions (bf16 inputs widen exactly), one rounding to the output dtype.
 // Every global access is bounds-checked, so any M, N, K >= 1 works.  Which kernel runs, and so the order of the sums,
 // depends on M, N and K alone: strides and alignment only choose how a tile is read.
+#include <algorithm>
 #include "fstu_common.h"
 
 namespace {
@@ -12,7 +13,8 @@ namespace {
 typedef float floatx16_t __attribute__((ext_vector_type(16)));
 typedef float floatx4_t __attribute__((ext_vector_type(4)));
 
-// Elements k..k+3 of a row, zero from K on.  VEC: k runs with stride 1, rows start on 4-element boundaries and K % 4 == 0.
+// Elements k..k+3 of a row, zero from K on.  VEC: k runs with stride 1, rows start on 4-element boundaries and K % 4 == 0;
+// each operand for itself (with W alone transposed 4096 x 768 x 768 takes 67 us; 138 where both were read one by one).
 // The loads are unconditional (an address beyond K is replaced by the row's start), so several stay in flight.
 template <typename T, bool VEC>
 __device__ __forceinline__ floatx4_t ga_load4(const T* __restrict__ row, long long sk, int k, int K) {
@@ -42,7 +44,7 @@ __device__ __forceinline__ floatx4_t ga_load4(const T* __restrict__ row, long lo
 // instruction per element); the NW partial tiles are added in wave order through LDS.  Bound by one or two trips to
 // memory: a workgroup's k loop is K / (16 NW) trips where a tile of the staged kernel below takes K / 16 of them, one
 // behind the other.
-template <typename T, bool VEC, int TM, int TN, int NW, int U>
+template <typename T, bool VA, bool VW, int TM, int TN, int NW, int U>
 __global__ void __launch_bounds__(64 * NW)
 gemm_any_split_kernel(const T* __restrict__ A, long long sam, long long sak, const T* __restrict__ W, long long swn, long long swk,
                       T* __restrict__ C, long long ldc, int M, int N, int K) {
@@ -67,9 +69,9 @@ gemm_any_split_kernel(const T* __restrict__ A, long long sam, long long sak, con
       const int k = k0 + 16 * NW * u;
       if (k >= K) break;
 #pragma unroll
-      for (int i = 0; i < TN; ++i) wv[u][i] = ga_load4<T, VEC>(wr[i], swk, k + 4 * g, K);
+      for (int i = 0; i < TN; ++i) wv[u][i] = ga_load4<T, VW>(wr[i], swk, k + 4 * g, K);
 #pragma unroll
-      for (int j = 0; j < TM; ++j) av[u][j] = ga_load4<T, VEC>(ar[j], sak, k + 4 * g, K);
+      for (int j = 0; j < TM; ++j) av[u][j] = ga_load4<T, VA>(ar[j], sak, k + 4 * g, K);
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -143,7 +145,7 @@ __device__ __forceinline__ void ga_put(float (*dst)[GA_LD], const float (&v)[8],
   }
 }
 
-template <typename T, bool VEC>
+template <typename T, bool VA, bool VW>
 __global__ void __launch_bounds__(256)
 gemm_any_tile_kernel(const T* __restrict__ A, long long sam, long long sak, const T* __restrict__ W, long long swn, long long swk,
                      T* __restrict__ C, long long ldc, int M, int N, int K) {
@@ -160,16 +162,16 @@ gemm_any_tile_kernel(const T* __restrict__ A, long long sam, long long sak, cons
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
   float av[8], wv[8];
-  ga_fetch<T, VEC>(av, A, sam, sak, m0, M, 0, K);
-  ga_fetch<T, VEC>(wv, W, swn, swk, n0, N, 0, K);
-  ga_put<VEC>(xs[0], av, sak);
-  ga_put<VEC>(ws[0], wv, swk);
+  ga_fetch<T, VA>(av, A, sam, sak, m0, M, 0, K);
+  ga_fetch<T, VW>(wv, W, swn, swk, n0, N, 0, K);
+  ga_put<VA>(xs[0], av, sak);
+  ga_put<VW>(ws[0], wv, swk);
   __syncthreads();
   for (int k0 = 0, b = 0; k0 < K; k0 += GA_BK, b ^= 1) {
     const bool more = k0 + GA_BK < K;
     if (more) {
-      ga_fetch<T, VEC>(av, A, sam, sak, m0, M, k0 + GA_BK, K);
-      ga_fetch<T, VEC>(wv, W, swn, swk, n0, N, k0 + GA_BK, K);
+      ga_fetch<T, VA>(av, A, sam, sak, m0, M, k0 + GA_BK, K);
+      ga_fetch<T, VW>(wv, W, swn, swk, n0, N, k0 + GA_BK, K);
     }
     // weights as the A operand (lane: feature l % 32, k = l / 32), activations as the B operand (lane: row l % 32)
 #pragma unroll
@@ -186,8 +188,8 @@ gemm_any_tile_kernel(const T* __restrict__ A, long long sam, long long sak, cons
         for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(y[i], x[j], acc[i][j], 0, 0, 0);
     }
     if (more) {      // the other buffer was last read before the barrier that ended the previous tile
-      ga_put<VEC>(xs[b ^ 1], av, sak);
-      ga_put<VEC>(ws[b ^ 1], wv, swk);
+      ga_put<VA>(xs[b ^ 1], av, sak);
+      ga_put<VW>(ws[b ^ 1], wv, swk);
     }
     __syncthreads();
   }
@@ -206,7 +208,9 @@ gemm_any_tile_kernel(const T* __restrict__ A, long long sam, long long sak, cons
   }
 }
 
-// 0: 16 x 16 tiles, 16 waves along K; 1: 32 x 32 tiles, 8 waves along K; 2: 128 x 128 tiles.  The large tile needs more
+// 0: 16 x 16 tiles, 16 waves along K; 1: 32 x 32 tiles, 8 waves along K; 2: 128 x 128 tiles.  Rows or features that fill at
+// most half of a large tile stay on 1 (bf16, us on 1 / 2: 17 x 50257 x 256 17 / 41, 64 x 50257 x 256 31 / 46, 100000 x 16 x 768
+// 68 / 227, 100000 x 64 x 256 54 / 89; 100 x 50257 x 768 143 / 128).  The large tile needs more
 // than one workgroup per compute unit before its matrix rate counts (192 tiles: 2000 x 1536 x 1536 141 us on 1, 158 on 2;
 // 512 tiles: 4096 x 2048 x 24 40 us on 1, 33 on 2; 1024: 16384 x 2048 x 2048 1885 on 1, 1153 on 2), the 32 x 32 tile half
 // the chip (16 tiles: 64 x 256 x 3072 13 us on 0, 27 on 1; 80: 300 x 256 x 3072 25 and 30; 256: 1000 x 256 x 3072 49 and 31).
@@ -216,23 +220,24 @@ gemm_any_tile_kernel(const T* __restrict__ A, long long sam, long long sak, cons
 static int ga_pick(int M, int N) {
   const long long t128 = (long long)((M + 127) / 128) * ((N + 127) / 128);
   const long long t32 = (long long)((M + 31) / 32) * ((N + 31) / 32);
-  return t128 > 256 ? 2 : t32 >= 128 ? 1 : 0;
+  if (t32 < 128) return 0;
+  return t128 > 256 && (std::min(M, N) > 64 || N > 65535 * 32) ? 2 : 1;
 }
 
-template <typename T, bool VEC>
+template <typename T, bool VA, bool VW>
 static void ga_launch(const T* A, long long sam, long long sak, const T* W, long long swn, long long swk, T* C, long long ldc,
                       int M, int N, int K, hipStream_t s) {
   switch (ga_pick(M, N)) {
     case 0:
-      hipLaunchKernelGGL((gemm_any_split_kernel<T, VEC, 1, 1, 16, 4>), dim3((M + 15) / 16, (N + 15) / 16), dim3(1024), 0, s, A, sam,
+      hipLaunchKernelGGL((gemm_any_split_kernel<T, VA, VW, 1, 1, 16, 4>), dim3((M + 15) / 16, (N + 15) / 16), dim3(1024), 0, s, A, sam,
                          sak, W, swn, swk, C, ldc, M, N, K);
       break;
     case 1:
-      hipLaunchKernelGGL((gemm_any_split_kernel<T, VEC, 2, 2, 8, 2>), dim3((M + 31) / 32, (N + 31) / 32), dim3(512), 0, s, A, sam,
+      hipLaunchKernelGGL((gemm_any_split_kernel<T, VA, VW, 2, 2, 8, 2>), dim3((M + 31) / 32, (N + 31) / 32), dim3(512), 0, s, A, sam,
                          sak, W, swn, swk, C, ldc, M, N, K);
       break;
     default:
-      hipLaunchKernelGGL((gemm_any_tile_kernel<T, VEC>), dim3((M + 127) / 128, (N + 127) / 128), dim3(256), 0, s, A, sam, sak, W,
+      hipLaunchKernelGGL((gemm_any_tile_kernel<T, VA, VW>), dim3((M + 127) / 128, (N + 127) / 128), dim3(256), 0, s, A, sam, sak, W,
                          swn, swk, C, ldc, M, N, K);
   }
 }
@@ -252,11 +257,12 @@ extern "C" int fstu_gemm_any(const void* A, int64_t sam, int64_t sak, const void
   FSTU_REQUIRE(N <= 65535 * GA_B, FSTU_ESHAPE, "fstu_gemm_any: N=%d too large", N);
   // four elements per load: k contiguous, rows on 4-element boundaries, K a whole number of fours
   const size_t quad = dtype == FSTU_BF16 ? 8 : 16;
-  const bool vec = (sak == 1 || K == 1) && (swk == 1 || K == 1) && K % 4 == 0 && sam % 4 == 0 && swn % 4 == 0 && fstu_aligned(A, quad) &&
-                   fstu_aligned(W, quad);
+  const bool va = sak == 1 && K % 4 == 0 && (sam % 4 == 0 || M == 1) && fstu_aligned(A, quad);
+  const bool vw = swk == 1 && K % 4 == 0 && (swn % 4 == 0 || N == 1) && fstu_aligned(W, quad);
+#define GA_GO(VA, VW) ga_launch<T, VA, VW>((const T*)A, sam, sak, (const T*)W, swn, swk, (T*)C, ldc, M, N, K, (hipStream_t)stream)
   FSTU_DISPATCH_DTYPE(dtype, "fstu_gemm_any",
-                      if (vec) ga_launch<T, true>((const T*)A, sam, sak, (const T*)W, swn, swk, (T*)C, ldc, M, N, K, (hipStream_t)stream);
-                      else ga_launch<T, false>((const T*)A, sam, sak, (const T*)W, swn, swk, (T*)C, ldc, M, N, K, (hipStream_t)stream));
+                      if (va && vw) GA_GO(true, true); else if (va) GA_GO(true, false); else if (vw) GA_GO(false, true); else GA_GO(false, false));
+#undef GA_GO
   FSTU_CHECK_LAUNCH("fstu_gemm_any");
   return FSTU_OK;
 }

@@ -230,6 +230,25 @@ def test_gemm_bf16_transposed_activations(hip, nb, M, N, K):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("M,N,K", [(17, 40000, 36), (64, 33000, 20), (65, 33000, 20), (33000, 64, 36), (40001, 3, 12), (300, 700, 132)])
+def test_gemm_any_narrow_shapes_and_mixed_layouts(hip, dtype, M, N, K):
+    """Few rows or few features of a large product, and each operand with its reduction index contiguous, transposed or off its
+    alignment: the bound of the test above, and the same bits in every layout."""
+    g = gen(M + N)
+    x, W = dev(torch.randn(M, K, generator=g).to(dtype)), dev(torch.randn(N, K, generator=g).to(dtype))
+    def layouts(t):
+        odd = torch.empty(t.numel() + 1, dtype=dtype, device="cuda")[1:].view(t.shape).copy_(t)
+        return t, t.t().contiguous().t(), odd
+    got = hip.gemm_any(x, W)
+    ref, mag = x.double() @ W.double().t(), x.double().abs() @ W.double().abs().t()
+    bound = 2 * K * 2.0 ** -24 * mag + (2.0 ** -8 * ref.abs() if dtype == torch.bfloat16 else 0.0)
+    assert bool(((got.double() - ref).abs() <= bound).all())
+    for a in layouts(x):
+        for w in layouts(W):
+            assert torch.equal(hip.gemm_any(a, w), got)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 def test_gemm_any_expanded_operands(hip, dtype):
     """Rows, features or a reduction index that are one value repeated: the bits of the same operands laid out."""
     g = gen(97)
