@@ -869,7 +869,14 @@ int gemm_launch(const void* A, long long lda, const void* W, const void* W2, con
   // of the line, us (large / small): 2048 x 4096 x 2048 (128 large tiles) 39.8 / 37.6, 2331 x 4096 x 2048 (160) 40.0 / 54.1;
   // 3072 x 2304 x 768 (108) 20.9 / 19.0, 4096 x 2304 x 768 (144) 21.5 / 27.9; 777 x 2 x 9216 x 768 (288) 41 / 28,
   // 1536 x 2 x 9216 x 768 (432) 43 / 51; 384 x 50257 x 768 (394) 38.5 / 45.6.
-  if (9 * ((big + gemm_cus() - 1) / gemm_cus()) * gemm_cus() < 4 * small)
+  // In mode 1 a round ends in the GELU of its whole tile, beside which a short K hides little, while two small tiles on a
+  // compute unit cover each other's: us, large / small tiles, 20000 x 2 x 512 (two rounds, 2.44 small tiles per place in them)
+  // K = 64 20.5 / 15.4, 256 25.8 / 21.4, 512 33.6 / 30.4, 768 42.2 / 39.8; 8192 x 2 x 2304 (three rounds, 3) 28.6 / 24.8, 39.8 /
+  // 36.1, 53.6 / 51.5, 68.7 / 69.3; 4096 x 2 x 1536 (one round, 3) K = 256 14.8 / 14.0, 512 18.7 / 20.5; 6000 x 2 x 2304 (two,
+  // 3.3) K = 64 20.6 / 20.0, 256 27.1 / 29.2.
+  const long long rounds = (big + gemm_cus() - 1) / gemm_cus();
+  const int quarters = MODE != 1 || K >= 1024 ? 9 : K < 256 ? 14 : K < 512 ? 13 : rounds == 1 ? 9 : 11;
+  if (quarters * rounds * gemm_cus() < 4 * small)
     return gemm_pp_launch<MODE>(A, lda, W, W2, R, ldr, C, ldc, M, N, K, s);
   // A grid that leaves one workgroup per compute unit anyway gains from the deeper pipeline when K is long (M=4096, N=768,
   // K=9216: 83 us against 93 us).

@@ -385,6 +385,22 @@ def test_gemm_bf16_alternating_groups(hip, M, N, K):
     assert float(((act - want).abs() > 0).float().mean()) <= 0.05
 
 
+@pytest.mark.parametrize("M,N,K", [(4093, 8188, 64), (4093, 8188, 320), (4093, 8188, 576), (2049, 4100, 1088), (3000, 1028, 192)])
+def test_gemm_bf16_gated_pair_on_both_tiles(hip, M, N, K):
+    """The gated pair on either side of the line between the tiles, ragged in rows and features, one k tile and odd numbers of
+    them: T(T(gelu(T(g))) T(u)) against the same from fp32 products.  A gate or up value on a rounding border moves by one bf16
+    ulp (2^-8 of it, gelu's slope stays below 1.13), each of the two roundings behind it by half of one more."""
+    g = gen(67)
+    x = dev(torch.randn(M, K, generator=g).bfloat16())
+    Wg, Wu = (dev((torch.randn(N, K, generator=g) / math.sqrt(K)).bfloat16()) for _ in range(2))
+    gate, up = (x.float() @ W.float().t() for W in (Wg, Wu))
+    want = (F.gelu(gate.bfloat16(), approximate="tanh") * up.bfloat16()).float()
+    act = hip.gemm(x, Wg, up_weight=Wu).float()
+    tol = want.abs() * 2.0 ** -6 + 1.2 * 2.0 ** -7 * (gate * up).abs() + 1e-3 * 2.0 ** -7 * float(want.abs().max())
+    assert bool(((act - want).abs() <= tol).all())
+    assert float(((act - want).abs() > 0).float().mean()) <= 0.05
+
+
 @pytest.mark.parametrize("M,N,K", [(1283, 15001, 128), (17, 1, 32), (31, 259, 128), (33, 130, 64), (130, 1031, 1056), (700, 515, 1024), (4100, 10003, 1024)])
 def test_gemm_bf16_plain_any_feature_count(hip, M, N, K):
     """Mode 0 with N % 4 != 0 and an odd row stride (the vocabulary of the tied head), every tile shape: one bf16 ulp
