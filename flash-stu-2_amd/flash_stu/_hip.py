@@ -18,6 +18,7 @@ LIB_PATH = os.path.join(os.path.dirname(_HERE), "csrc", "libflashstu_hip.so")
 
 FSTU_F32, FSTU_BF16 = 0, 1
 MAX_DECODE_ROWS = 16
+GEMM_MIN_SLICED_K = 1024      # fstu_gemm_bf16_slices takes slices of at least 512
 GEMM_MAX_STRIDE = 1 << 22     # elements between rows that the matrix-core GEMM's 32-bit offsets cover
 
 _lib = None
@@ -323,7 +324,7 @@ def gemm(x2: torch.Tensor, weight: torch.Tensor, up_weight: Optional[torch.Tenso
             raise FlashSTUHipError("gemm: residual must be (M,N) with contiguous rows")
         mode, ldr = 2, residual.stride(0)
     slices, partial = 1, None
-    if mode != 1 and out.stride(0) % 4 == 0 and out.data_ptr() % 8 == 0:
+    if K >= GEMM_MIN_SLICED_K and mode != 1 and out.stride(0) % 4 == 0 and out.data_ptr() % 8 == 0:
         slices = load().fstu_gemm_bf16_slices(M, N, K, 1)
         if slices > 1:
             partial = torch.empty(slices, M, N, dtype=torch.float32, device=x2.device)
@@ -376,7 +377,7 @@ def gemm_ta(slabs: torch.Tensor, weight: torch.Tensor, residual: Optional[torch.
         if t is not None and (t.shape != (nb, M, N) or t.stride(2) != 1 or t.dtype != slabs.dtype):
             raise FlashSTUHipError(f"gemm_ta: {name} must be (nb, M, N) with contiguous rows")
     mode = 2 if residual is not None else 0
-    slices = load().fstu_gemm_bf16_slices(M, N, K, nb)
+    slices = load().fstu_gemm_bf16_slices(M, N, K, nb) if K >= GEMM_MIN_SLICED_K else 1
     partial = torch.empty(slices, nb, M, N, dtype=torch.float32, device=slabs.device) if slices > 1 else None
     _check(load().fstu_gemm_bf16_ta_ws(_p(slabs), slabs.stride(1), slabs.stride(0) if nb > 1 else 0, _p(weight), _p(residual),
                                        residual.stride(1) if residual is not None else 0,
