@@ -248,7 +248,7 @@ def test_c5_shape_bf16_sampling_spread_over_the_chip(hip, rows):
     """Config 5's sampling (top-k 40, temperature 0.8) in bf16 through the one-call step, where the head leaves its
     packed maxima and the sampler spreads every row over the chip: every generated id is the oracle's draw (and the
     one-workgroup-per-row kernel's) from the logits the step produced, eagerly and under graph replay."""
-    from test_gpu_model import make_pair, prompt
+    from test_gpu_model import make_pair, prompt, replayed
     ocfg, w, model = make_pair(seed=2, init="healthy", dtype=torch.bfloat16, mlp_scale=2, n_embd=256, n_layers=4,
                                n_heads=2, window_size=24, num_eigh=24, seq_len=256, vocab_size=2003,
                                stu_decode_mode="lds")
@@ -256,8 +256,9 @@ def test_c5_shape_bf16_sampling_spread_over_the_chip(hip, rows):
     ids = prompt(rows, P, ocfg.vocab_size, 4)
     got, gl = model.generate(ids.cuda(), max_length=P + N, temperature=0.8, top_k=40, do_sample=True, seed=2,
                              return_logits=True)
-    again = model.generate(ids.cuda(), max_length=P + N, temperature=0.8, top_k=40, do_sample=True, seed=2)
-    assert torch.equal(again, got)
+    how = dict(temperature=0.8, top_k=40, do_sample=True, seed=2)
+    assert torch.equal(model.generate(ids.cuda(), max_length=P + N, **how), got)
+    assert torch.equal(replayed(model, ids.cuda(), P + N, **how), got)
     miss = 0
     for t in range(N):
         lt = gl[:, t].contiguous()
@@ -274,15 +275,15 @@ def test_c5_shape_bf16_lds_teacher_forced(rows):
     """Same structure in bf16 with the recurrence state, logits within the bf16 tolerance.  17..32 rows step as one
     chunk: projections, MLP and head once over all rows on the packed-weight kernels (two row tiles per weight
     fragment), the state operators over all rows in one launch each."""
-    from test_gpu_model import make_pair, prompt, _teacher_forced
+    from test_gpu_model import make_pair, prompt, _teacher_forced, replayed
     ocfg, w, model = make_pair(seed=2, init="healthy", dtype=torch.bfloat16, mlp_scale=2, n_embd=256, n_layers=4,
                                n_heads=2, window_size=24, num_eigh=24, seq_len=256, vocab_size=2003,
                                stu_decode_mode="lds")
     P, N = 20, 60
     ids = prompt(rows, P, ocfg.vocab_size, 4)
     got, gl = model.generate(ids.cuda(), max_length=P + N, do_sample=False, return_logits=True)
-    again = model.generate(ids.cuda(), max_length=P + N, do_sample=False)        # graph replay
-    assert torch.equal(again, got)
+    assert torch.equal(model.generate(ids.cuda(), max_length=P + N, do_sample=False), got)
+    assert torch.equal(replayed(model, ids.cuda(), P + N), got)
     ref = _teacher_forced(w, ocfg, got.cpu(), P).float()
     err = (gl.float().cpu() - ref).abs().amax(-1) / ref.abs().amax(-1)
     assert float(err.max()) <= 2e-2
@@ -318,15 +319,15 @@ def test_c5_width_bf16_step_kernels(d, heads, rows):
     balanced gate/up kernel and its norm prologue; 17..32 rows take the packed-weight kernels with two row tiles per
     weight fragment for the MLP, the small projections and the head): two layers, bf16, logits against the
     teacher-forced oracle."""
-    from test_gpu_model import make_pair, prompt, _teacher_forced
+    from test_gpu_model import make_pair, prompt, _teacher_forced, replayed
     ocfg, w, model = make_pair(seed=4, init="healthy", dtype=torch.bfloat16, mlp_scale=4, n_embd=d, n_layers=2,
                                n_heads=heads, window_size=32, num_eigh=24, seq_len=128, vocab_size=1511,
                                stu_decode_mode="lds")
     P, N = 12, 28
     ids = prompt(rows, P, ocfg.vocab_size, 6)
     got, gl = model.generate(ids.cuda(), max_length=P + N, do_sample=False, return_logits=True)
-    again = model.generate(ids.cuda(), max_length=P + N, do_sample=False)        # graph replay
-    assert torch.equal(again, got)
+    assert torch.equal(model.generate(ids.cuda(), max_length=P + N, do_sample=False), got)
+    assert torch.equal(replayed(model, ids.cuda(), P + N), got)
     ref = _teacher_forced(w, ocfg, got.cpu(), P).float()
     err = (gl.float().cpu() - ref).abs().amax(-1) / ref.abs().amax(-1)
     assert float(err.max()) <= 2e-2
@@ -341,7 +342,7 @@ def test_c5_full_architecture_decode_against_full_sequence_recompute():
     cut to 1100 tokens to keep the test short: longer than the 1025-slot ring, so the prompt pass fills a wrapped
     ring and every decode step reads the full window through the streamed head-dim-128 attention kernel."""
     from flash_stu import FlashSTU, FlashSTUConfig
-    from test_gpu_model import prompt
+    from test_gpu_model import prompt, replayed
     torch.manual_seed(2)
     cfg = FlashSTUConfig(n_embd=2048, n_layers=24, n_heads=16, window_size=1024, seq_len=8192, vocab_size=50257,
                          num_eigh=24, mlp_scale=12, torch_dtype=torch.bfloat16)
@@ -353,9 +354,8 @@ def test_c5_full_architecture_decode_against_full_sequence_recompute():
     ids = prompt(B, P, cfg.vocab_size, 2).cuda()
     kw = dict(max_length=P + N, do_sample=True, top_k=40, temperature=0.8, seed=2)
     eager, logits = model.generate(ids, return_logits=True, **kw)
-    graph = model.generate(ids, **kw)
-    assert torch.equal(graph, eager)
-    assert torch.equal(model.generate(ids, **kw), graph)
+    assert torch.equal(replayed(model, ids, **kw), eager)
+    assert torch.equal(model.generate(ids, **kw), eager)
     worst = 0.0
     for s in (0, 5, N - 1):
         full = model(eager[:, :P + s].contiguous()).logits[:, -1, :].float()

@@ -37,6 +37,31 @@ def prompt(B, P, V, seed):
     return torch.randint(0, V, (B, P), generator=torch.Generator().manual_seed(seed))
 
 
+def replayed(model, ids, max_length, steps=8, do_sample=False, temperature=1.0, top_k=None, top_p=None, seed=0, between=None):
+    """generate() with every step from a captured graph, whatever the number of chunks: graphs of `steps` steps, the rest as
+    single-step graphs; `between` runs between the launches."""
+    from flash_stu import _hip
+    eng, (B, P) = model.decode_engine(), ids.shape
+    how = (temperature, top_k, top_p, do_sample, seed)
+    tokens = torch.zeros(B, max_length, dtype=torch.int64, device="cuda")
+    tokens[:, :P] = ids
+    with torch.no_grad():
+        _hip.sample(eng.prefill(tokens[:, :P], max_length), tokens[:, P], *how, 0)
+    done, todo = 0, max_length - P - 1
+    try:
+        for n in (steps, 1):
+            if todo - done >= n:
+                eng.graph_begin(tokens, P + done, 1 + done, *how, steps_per_graph=n)
+            while todo - done >= n:
+                eng.graph_step()
+                done += n
+                if between is not None:
+                    between()
+    finally:
+        eng.graph_end()
+    return tokens
+
+
 @pytest.mark.parametrize("init,mlp_scale", [("reference", 12), ("healthy", 12), ("healthy", 4)])
 def test_c1_fp32_greedy_ids_bit_exact(init, mlp_scale):
     """64-token prompt, 64 greedy tokens, fp32, seed 0."""
@@ -84,12 +109,14 @@ def test_graph_replay_equals_eager_steps(do_sample):
     ids = prompt(3, 6, ocfg.vocab_size, 9).cuda()
     kw = dict(max_length=70, do_sample=do_sample, temperature=0.9, top_k=20, seed=5)
     eager = model.generate(ids, use_graph=False, **kw)
-    for _ in range(3):
-        junk = torch.randn(256, 256, device="cuda") @ torch.randn(256, 256, device="cuda")   # unrelated eager work
+
+    def unrelated():
+        torch.randn(256, 256, device="cuda") @ torch.randn(256, 256, device="cuda")
         torch.cuda.synchronize()
-        got = model.generate(ids, use_graph=True, **kw)
-        assert torch.equal(got, eager)
-    del junk
+    for steps in (1, 8, 3):
+        unrelated()
+        assert torch.equal(model.generate(ids, use_graph=True, **kw), eager)
+        assert torch.equal(replayed(model, ids, steps=steps, between=unrelated, **kw), eager)
 
 
 @pytest.mark.parametrize("do_sample", [False, True])
@@ -222,12 +249,11 @@ def test_input_projection_gradients(B, T, d):
     g = torch.Generator().manual_seed(B * T)
     x, m, w = (torch.randn(*s, generator=g).bfloat16().cuda() for s in ((B, T, d), (d, 2 * d), (B, T, 2 * d)))
     assert ProjectInputs.takes(x, m) == (B * T % 64 == 0)
-    if not ProjectInputs.takes(x, m):
-        return
+    project = ProjectInputs.apply if ProjectInputs.takes(x, m) else torch.matmul
     shifted = torch.empty(B * T * d + 1, dtype=torch.bfloat16, device="cuda")[1:].view(B, T, d).copy_(x)
     for xi in (x, shifted, x[:1].expand(B, T, d)):
         xi, mi = xi.detach().requires_grad_(True), m.clone().requires_grad_(True)
-        y = ProjectInputs.apply(xi, mi)
+        y = project(xi, mi)
         y.backward(w)
         xd, md, wd = xi.detach().double().reshape(-1, d), m.double(), w.double().reshape(-1, 2 * d)
         for got, a, b in ((y.detach(), xd, md), (xi.grad, wd, md.t()), (mi.grad, xd.t(), wd)):
@@ -235,7 +261,7 @@ def test_input_projection_gradients(B, T, d):
             err = (got.double().reshape(ref.shape) - ref).abs()
             assert bool((err <= 2.0 ** -8 * ref.abs() + a.shape[1] * 2.0 ** -23 * mag).all())
     xi = x.clone().requires_grad_(True)
-    ProjectInputs.apply(xi, m).backward(w)             # m needs no gradient
+    project(xi, m).backward(w)                         # m needs no gradient
     assert xi.grad.shape == x.shape and m.grad is None
 
 
@@ -344,8 +370,8 @@ def test_c2_full_size_decode_against_full_sequence_recompute():
     B, P, N = 8, 512, 40
     ids = prompt(B, P, cfg.vocab_size, 1).cuda()
     eager, logits = model.generate(ids, max_length=P + N, do_sample=False, return_logits=True)      # step by step
-    graph = model.generate(ids, max_length=P + N, do_sample=False)                                  # 8-step graphs
-    assert torch.equal(graph, eager)
+    assert torch.equal(model.generate(ids, max_length=P + N, do_sample=False), eager)
+    assert torch.equal(replayed(model, ids, P + N), eager)                                          # 8-step graphs
     worst = 0.0
     for s in (0, 1, 7, 20, N - 1):          # logits that picked token P+s come from positions < P+s
         full = model(eager[:, :P + s].contiguous()).logits[:, -1, :].float()
@@ -370,7 +396,8 @@ def test_single_token_prompt_and_ragged_batches(dtype):
             got, gl = model.generate(ids.cuda(), max_length=20, do_sample=False, return_logits=True)
             ref = _teacher_forced(w, ocfg, got.cpu(), 1).float()
             assert float(((gl.float().cpu() - ref).abs().amax(-1) / ref.abs().amax(-1)).max()) <= 2e-2
-            assert torch.equal(model.generate(ids.cuda(), max_length=20, do_sample=False), got)      # graph path
+            assert torch.equal(model.generate(ids.cuda(), max_length=20, do_sample=False), got)
+            assert torch.equal(replayed(model, ids.cuda(), 20), got)
         one = model.generate(ids.cuda(), max_length=2, do_sample=False)
         assert one.shape == (B, 2) and torch.equal(one[:, :2], got[:, :2])
         assert torch.equal(model.generate(ids.cuda(), max_length=1), ids.cuda())
@@ -456,6 +483,29 @@ def test_one_call_step_equals_the_layers_own_calls(dtype, extra, rows):
             assert a.shape == b.shape and a.dtype == b.dtype
             if a.numel():
                 assert float((a.float() - b.float()).abs().max()) <= tol * max(float(b.float().abs().max()), 1e-6)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_weights_changed_between_two_steps_on_caches_are_seen(dtype):
+    """Every parameter scaled in place between two positions: the second step is that of the layers' own calls (sums in another
+    order, bounds as above) and not that of the weights before."""
+    _, _, model = make_pair(seed=5, init="healthy", dtype=dtype, mlp_scale=2, n_embd=128, n_layers=4, n_heads=2, window_size=8,
+                            num_eigh=8, seq_len=64, vocab_size=777)
+    ids = prompt(3, 8, 777, 2).cuda()
+    out = model(ids[:, :6], use_cache=True)
+    past = model(ids[:, 6:7], past_key_values=out.past_key_values, use_cache=True).past_key_values
+    copies = [tuple(tuple(t.clone() for t in c) for c in past) for _ in range(2)]
+    before = model(ids[:, 7:8], past_key_values=past, use_cache=True).logits.float()
+    with torch.no_grad():
+        for i, p in enumerate(model.parameters()):
+            p.mul_(1.0 + 0.1 * (i % 3))
+    one = model(ids[:, 7:8], past_key_values=copies[0], use_cache=True).logits.float()
+    hook = model.norm.register_forward_hook(lambda *a: None)
+    layers = model(ids[:, 7:8], past_key_values=copies[1], use_cache=True).logits.float()
+    hook.remove()
+    scale = float(layers.abs().max())
+    assert float((one - layers).abs().max()) <= (1e-4 if dtype == torch.float32 else 2e-2) * scale
+    assert float((one - before).abs().max()) > 5e-2 * scale
 
 
 class _Scaled(torch.nn.Module):
