@@ -89,6 +89,9 @@ class STU(nn.Module):
             hit[3] = _stay_behind(hit[3])
         return hit[1]
 
+    def __getstate__(self):
+        return {**self.__dict__, "_derived": {}}       # a copy derives its own: streams and addresses are this object's
+
     def decode_mode(self) -> str:
         mode = self.config.resolved_stu_decode_mode()
         if mode == "lds" and self.use_approx and self.use_hankel_L and self.phi.shape[0] % 2 != 0:

@@ -595,7 +595,9 @@ def test_replaced_methods_run_in_a_step_on_caches(what, monkeypatch):
 
 def test_derived_tensors_are_complete_on_every_stream():
     """Transposed weights and filter spectra that one stream has only just been given, read by the next call on another: the
-    values of a model that nothing else runs beside."""
+    values of a model that nothing else runs beside.  A module that has been called can still be copied and pickled."""
+    import copy
+    import pickle
     from flash_stu import STU, FlashSTUConfig
     cfg = FlashSTUConfig(n_embd=256, n_heads=4, n_layers=2, seq_len=512, num_eigh=8, vocab_size=64, torch_dtype=torch.bfloat16)
     g = torch.Generator().manual_seed(2)
@@ -620,6 +622,8 @@ def test_derived_tensors_are_complete_on_every_stream():
         assert torch.equal(there, want)
         torch.cuda.synchronize()
         assert torch.equal(stu(x), want) and stu._derived["mit"][3] is None
+    for copied in (copy.deepcopy(stu), pickle.loads(pickle.dumps(stu))):
+        assert torch.equal(copied(x), want)
 
 
 def test_forward_accepts_reference_style_kv_cache():
