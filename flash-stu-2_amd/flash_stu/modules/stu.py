@@ -28,26 +28,13 @@ from ..utils.lds_fit import check_lds_fit, fit_even_lag_lds
 FFT_MIN_T = 32     # shorter inputs take the time-domain kernel (a 64-point transform would be mostly padding)
 
 
-def _end_of_stream(device):
-    """What the current stream has been given so far, for a tensor that outlives the call: (event, stream), or None."""
-    if device.type != "cuda" or torch.cuda.is_current_stream_capturing():
-        return None
-    stream, event = torch.cuda.current_stream(device), torch.cuda.Event()
-    event.record(stream)
-    return event, stream
-
-
-def _stay_behind(made):
-    """Orders the current stream behind `made`; returns None once that has been reached."""
+def _wait_for(stream) -> bool:
+    """Orders the current stream behind what `stream` has been given; a stream that is being captured cannot wait for
+    work outside the capture."""
     if torch.cuda.is_current_stream_capturing():
-        return made
-    event, stream = made
-    if event.query():
-        return None
-    now = torch.cuda.current_stream(stream.device)
-    if now != stream:
-        now.wait_event(event)
-    return made
+        return False
+    torch.cuda.current_stream(stream.device).wait_event(stream.record_event())
+    return True
 
 
 class STU(nn.Module):
@@ -83,10 +70,15 @@ class STU(nn.Module):
         ver = tuple((p._version, p.data_ptr()) for p in params)
         hit = self._derived.get(key)
         if hit is None or hit[0] != ver:
-            hit = [ver, build(), [p.detach() for p in params], _end_of_stream(params[0].device)]
+            # behind the sources: the device, the streams that are behind the launch, and the one that made it (an event
+            # recorded here would delay the first call by some 16 us)
+            dev, value = params[0].device, build()
+            stream = torch.cuda.current_stream(dev) if dev.type == "cuda" else None
+            hit = (ver, value, [p.detach() for p in params], -1 if stream is None else dev.index,
+                   {None if stream is None else stream.cuda_stream}, stream)
             self._derived[key] = hit
-        elif hit[3] is not None:
-            hit[3] = _stay_behind(hit[3])
+        elif hit[3] >= 0 and _hip.raw_stream(hit[3]) not in hit[4] and _wait_for(hit[5]):
+            hit[4].add(_hip.raw_stream(hit[3]))
         return hit[1]
 
     def __getstate__(self):

@@ -621,7 +621,7 @@ def test_derived_tensors_are_complete_on_every_stream():
         torch.cuda.current_stream().wait_stream(other)
         assert torch.equal(there, want)
         torch.cuda.synchronize()
-        assert torch.equal(stu(x), want) and stu._derived["mit"][3] is None
+        assert torch.equal(stu(x), want) and stu._derived["mit"][4] == {other.cuda_stream, torch.cuda.current_stream().cuda_stream}
     for copied in (copy.deepcopy(stu), pickle.loads(pickle.dumps(stu))):
         assert torch.equal(copied(x), want)
 
