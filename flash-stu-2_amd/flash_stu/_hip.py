@@ -639,13 +639,16 @@ _twiddle_cache = {}
 
 
 def fft_twiddles(n: int, device) -> torch.Tensor:
-    """exp(-2 pi i j / n) as (n, 2) fp32 on `device`, built once per (n, device)."""
+    """The twiddle tables of the n-point kernels, (n, 2) fp32 on `device` in the transforms' own order, built once per
+    (n, device).  Whichever stream asks for them next finds them written; a graph that is being captured builds its own."""
     key = (int(n), torch.device(device).index if torch.device(device).index is not None else torch.cuda.current_device())
     tw = _twiddle_cache.get(key)
     if tw is None:
         tw = torch.empty(n, 2, dtype=torch.float32, device=device)
         _check(load().fstu_fft_twiddles(_p(tw), n, _stream()), "fstu_fft_twiddles")
-        _twiddle_cache[key] = tw
+        if not torch.cuda.is_current_stream_capturing():
+            torch.cuda.current_stream().synchronize()
+            _twiddle_cache[key] = tw
     return tw
 
 

@@ -73,6 +73,8 @@ class STU(nn.Module):
             # behind the sources: the device, the streams that are behind the launch, and the one that made it (an event
             # recorded here would delay the first call by some 16 us)
             dev, value = params[0].device, build()
+            if dev.type == "cuda" and torch.cuda.is_current_stream_capturing():
+                return value             # part of the graph: written when it is replayed
             stream = torch.cuda.current_stream(dev) if dev.type == "cuda" else None
             hit = (ver, value, [p.detach() for p in params], -1 if stream is None else dev.index,
                    {None if stream is None else stream.cuda_stream}, stream)

@@ -626,6 +626,35 @@ def test_derived_tensors_are_complete_on_every_stream():
         assert torch.equal(copied(x), want)
 
 
+@pytest.mark.parametrize("dtype,T", [(torch.bfloat16, 300), (torch.float32, 20), (torch.float32, 100)])
+def test_tensors_derived_under_capture_stay_in_the_graph(dtype, T, monkeypatch):
+    """The first call on new weights inside a capture: calls beside the graph do not read what only its replay writes, and
+    replays, with other work between them, give the values of an uncaptured module on each input."""
+    from flash_stu import STU, FlashSTUConfig, _hip
+    cfg = FlashSTUConfig(n_embd=256, n_heads=4, n_layers=2, seq_len=512, num_eigh=8, vocab_size=64, torch_dtype=dtype)
+    g = torch.Generator().manual_seed(3)
+    phi = torch.randn(512, 8, generator=g).to(dtype)
+    new, reference = STU(cfg, phi, 1024).cuda(), STU(cfg, phi, 1024).cuda()
+    with torch.no_grad():
+        for p in new.parameters():
+            p.copy_(torch.randn(p.shape, generator=g))
+    reference.load_state_dict(new.state_dict())
+    x, others = torch.randn(2, T, 256, generator=g).to(dtype).cuda(), torch.randn(3, 2, T, 256, generator=g).to(dtype).cuda()
+    want = [reference(t) for t in (x, *others)]         # (also the kernels' one-time set-up)
+    torch.cuda.synchronize()
+    monkeypatch.setattr(_hip, "_twiddle_cache", {})
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = new(x)
+    assert not new._derived and not _hip._twiddle_cache
+    assert torch.equal(new(x), want[0])
+    for t, w in zip(others, want[1:]):
+        x.copy_(t)
+        graph.replay()
+        assert torch.equal(y, w)
+        assert torch.equal(new(t), w)
+
+
 def test_forward_accepts_reference_style_kv_cache():
     from flash_stu import Attention, FlashSTUConfig
     cfg = FlashSTUConfig(n_embd=128, n_heads=2, n_layers=2, seq_len=64, window_size=6, vocab_size=11, mlp_scale=2,
