@@ -1072,9 +1072,12 @@ static int conv_fft_launch(const char* name, const void* x, int64_t x_sb, int64_
   FSTU_REQUIRE(fstu_aligned(spec, 16) && fstu_aligned(tw, 16), FSTU_EALIGN, "%s: spec and tw must be 16-byte aligned", name);
   const int cols = fft_cols(logn - 1), esz = dtype == FSTU_BF16 ? 2 : 4, ch = 16 / esz, chw = cols > ch ? cols : ch;
   // Channel-contiguous operands whose rows split into whole 16-byte pieces per workgroup: the row-piece kernel.  The long
-  // transforms take a workgroup's channels one after the other: with fewer than two workgroups per compute unit the
-  // one-column kernel, eight times the workgroups, is the faster one.
-  const bool enough = logn < 13 || (long long)(d / chw) * B >= 512;
+  // transforms take a workgroup's channels one after the other, so that few groups of them leave compute units idle, and the
+  // one-column kernel, eight (fp32 four) times the workgroups but two bytes (four) of a line at a time, is the faster one.
+  // us, one column / row pieces: 4096 positions, bf16, 128 groups 43 / 62, 256 75 / 67, 384 106 / 93, fp32 192 37 / 36, 384
+  // 60 / 51; 2500 positions, bf16, 256 groups 62 / 64; 8192 positions, bf16, 96 groups 96 / 107, 128 112 / 108, 256 230 /
+  // 138, fp32 64 groups 37 / 59, 192 91 / 67.
+  const bool enough = logn < 13 || (long long)(d / chw) * B >= (logn == 13 ? 320 : 128);
   if (K == 1 && mode != 2 && enough && x_sc == 1 && y_sc == 1 && d % chw == 0 && x_st % ch == 0 && y_st % ch == 0 &&
       x_sb % ch == 0 && y_sb % ch == 0 && fstu_aligned(x, 16) && fstu_aligned(y, 16)) {
     const int gx = d / chw;

@@ -272,10 +272,12 @@ class STU(nn.Module):
 
     @staticmethod
     def _few_long_sequences(B: int, T: int, d: int, esz: int) -> bool:
-        """A few long sequences: the channel-contiguous FFT kernel, which takes a workgroup's 16 bytes of channels one
-        after the other, would leave compute units idle, and the one-column kernel reads a (B, L, d) tensor two bytes
-        at a time.  Time-major slabs let that kernel's loads and stores coalesce (measured at L=4096, d=2048, one
-        row: 100 us + 8 us per transpose against 137 us), with identical results."""
+        """A few long sequences: the FFT kernels for (B, L, d) operands take a workgroup's 16 bytes of channels one after the
+        other or read a tensor two bytes at a time.  Time-major slabs let every load and store coalesce, with identical
+        results (bf16, us, slab / (B, L, d): 1 x 4096 x 2048 49 / 75, 1 x 8192 x 2048 119 / 138, 2 x 4096 x 2048, where the
+        line lies, 86 / 100).  A transpose of the result is 8 to 15 of them; the projection that comes out as slabs costs
+        none, and where a decode state needs (B, L, d) rows as well a second transpose leaves 64 / 75, 139 / 138 and 111 /
+        100."""
         return T >= FFT_MIN_T and _hip.fft_length(T) >= 8192 and (d // (16 // esz)) * B < 512
 
     def _convolve_time_major(self, xt: torch.Tensor, n: int) -> torch.Tensor:
