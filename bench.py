@@ -6,7 +6,8 @@ window 512 / 24 filters / seq_len 2048 / vocab 50257, random-init bf16 (seed 1),
 random ids, greedy decode.  One "step" is one decode step of the whole batch (8 tokens).  The prompt is prefilled
 (untimed, reported separately), W warm-up steps run, then exactly K steps are timed with the inputs, weights and decode
 state resident in HBM.  The steps replay as HIP graphs of `--graph-steps` steps; what does not divide runs as
-single-step graphs, so any --steps / --warmup keeps the long graphs.
+single-step graphs, so any --steps / --warmup keeps the long graphs.  (generate() launches the same kernels step by step
+where the rows fit one chunk, up to 32: at these sizes the two take the same time per step.)
 
 Prints one JSON line.  `roofline` is the dominant kernel (the gate/up GLU projection, the largest weight stream of a
 step), timed live with HIP events on the launch stream; `step_roofline` is the whole step against the HBM roofline;
@@ -315,7 +316,9 @@ def run_lm(args, torch, _hip, which):
         "dtype": "bf16" if dt == torch.bfloat16 else "f32", "data": "synthetic",
         "config": {"workload": label, "mlp_scale": cfg.mlp_scale, "params": res["params"], "batch": B, "prompt": P,
                    "stu_decode_mode": stu_mode, "stu_prefill_mode": args.stu_prefill, "hip_graph": res["hip_graph"],
-                   "graph_steps": args.graph_steps, "stu_state_dim": cfg.stu_lds_state_dim if stu_mode == "lds" else None,
+                   "graph_steps": args.graph_steps,
+                   "token_loop": "the step's kernels replayed as graphs" if res["hip_graph"] else "the step's kernels launched one by one, as generate() does for one chunk of rows",
+                   "stu_state_dim": cfg.stu_lds_state_dim if stu_mode == "lds" else None,
                    "stu_fir_taps": cfg.stu_lds_fir_taps if stu_mode == "lds" else None},
         "step_roofline": res["step_roofline"],
         "prefill_tokens_per_s": res.get("prefill_tokens_per_s"), "prefill_ms": res.get("prefill_ms"),
@@ -536,10 +539,10 @@ def run_ref(args, torch, _hip):
                        "published": {"ms_per_call": published_ms, "hardware": "NVIDIA H100 PCIe (another GPU: context, not a like-for-like bar)",
                                      "source": "tests/tilling/standard_memory_profile.txt:48-59"}},
             "kernels_ms": {"x @ M_inputs (gemm_bf16_kernel, time-major output)": ms_proj,
-                           "spectral convolution (fft_conv_kernel on time-major slabs)": ms_conv,
-                           "result back to (L, d) (transpose_tiles_kernel)": ms_tr,
+                           "spectral convolution (fft_slab_kernel on time-major slabs)": ms_conv,
+                           "result back to (L, d) (transpose16_kernel)": ms_tr,
                            "projection_tflops": flops / (ms_proj * 1e-3) / 1e12},
-            "roofline": {"bound": "hbm", "kernel": "fft_conv_kernel (spectral convolution of the projected inputs, both sign branches, one column per workgroup)",
+            "roofline": {"bound": "hbm", "kernel": "fft_slab_kernel (spectral convolution of the projected inputs, both sign branches, on time-major slabs)",
                          "achieved": conv_gbps, "peak": HBM_PEAK_GBPS, "unit": "GB/s", "frac": conv_gbps / HBM_PEAK_GBPS,
                          "traffic": None, "bytes_per_launch": conv_bytes, "avg_launch_us": ms_conv * 1e3}}
 

@@ -19,7 +19,7 @@
 // and the last produces half.  The two innermost groups exchange among 16 threads of one wave, without a barrier.
 //
 // What bounds it: vector-ALU issue.  The exact-mode bank of 4 x 8192 x 1024 positions and channels and 24 filters issues 1.6 k
-// instructions per thread and filter, 4.9 M cycles of every compute unit's four SIMDs, and takes 2.73 ms = 5.6 M cycles
+// instructions per thread and filter, takes 2.86 to 2.98 ms and keeps the vector ALUs busy for 90 % of its 5.5 M cycles
 // (4.66 ms on transforms of 16384 points in 139 KB of LDS, one workgroup per compute unit; 3.77 ms while spectra and
 // twiddles lay in position order, so that every load of a wave touched up to 64 lines).  bf16, before -> now, us: 8 x 512 x
 // 768 24.5 -> 17.4, 32 x 300 x 2048 188 -> 105, 4 x 4096 x 2048 296 -> 218, one time-major sequence of 4096 x 2048 95 -> 50.
@@ -749,8 +749,9 @@ fft_conv_rows_kernel(const T* __restrict__ x, size_t x_sb, size_t x_st, const cp
 // the forward kernel on time-reversed fp32 copies the same took 18 n/2-point transforms per column, one launch and one
 // filter transform per batch row, and flips, sums and casts in between.  Rows' parts of the filter gradient go to memory in
 // fp32 and are added by fft_corr_finish_kernel in the order of the rows (no atomics: the same bits every time).
-// Vector-ALU issue bounds it as it does the convolution.  bf16, 8 x 2048 x 768: 120 us and 10 us for the sum over the rows,
-// where the composed form took 0.95 ms; a training step at that size 1.34 -> 0.37 ms.
+// The vector ALUs are busy for 44 % of it at 8 x 2048 x 768 bf16: the rest are the barriers and the staging between its
+// transforms.  111 us there and 10 us for the sum over the rows, where the composed form took 0.95 ms; a training step at that
+// size 1.69 -> 0.32 ms.
 // A workgroup owns the COLS neighbouring channels that its threads transform and reads them as pieces of a row.
 template <typename T, int LOGN> struct CorrCut {
   static constexpr int COLS = 1 << fft_lcols<LOGN>(), NE = COLS < RowVec<T>::CH ? COLS : RowVec<T>::CH, VR = COLS / NE;

@@ -362,7 +362,7 @@ int gemm_launch_tile(const void* A, long long lda, const void* W, const void* W2
 // although it reads the same operands twice as often (1.30 -> 1.33-1.42 PFLOP/s).  Measured against the kernel above
 // (256 x 256 tile) and hipBLASLt, us: 16384 x 2048 x 24576 with the residual 1127 / 1395 / 1366 (1.46 PFLOP/s), 16384 x 6144
 // x 2048 291 / 384 / 294, 16384 x 50257 x 2048 2550 / 3339 / 2500; gate+up 16384 x 2 x 24576 x 2048 2487 / 3148, 4096 x
-// 2 x 9216 x 768 109 / 121.  What keeps K = 2048 below K = 24576: the epilogue (in mode 1 the GELU's 70 cycles per element).
+// 2 x 9216 x 768 118 / 133.  What keeps K = 2048 below K = 24576: the epilogue (in mode 1 the GELU's 70 cycles per element).
 #define PP_STAGE 65536u
 #define PP_PART 16384u
 #define PP_LDS (2 * PP_STAGE + 32768u)   // + what the epilogue passes the rows through
