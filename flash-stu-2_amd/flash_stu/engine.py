@@ -234,9 +234,9 @@ class DecodeEngine:
         """MFMA-fragment-ordered copy of the (N,K) bf16 weight at `place` in the model, rebuilt only when the weight changes.
         The entry holds the storage that it was made from: while it is there no other tensor can come to lie at the address
         it is recognised by."""
-        hit = self._packed.get(place)
-        if hit is None or hit[0] != (w._version, w.data_ptr()):
-            hit = ((w._version, w.data_ptr()), _hip.pack_rows(w), w.detach())
+        hit, made_from = self._packed.get(place), (_hip.version(w), w.data_ptr())
+        if hit is None or hit[0] != made_from:
+            hit = (made_from, _hip.pack_rows(w), w.detach())
             self._packed[place] = hit
             self._unfinished = True
         return hit[1]

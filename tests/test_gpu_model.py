@@ -655,6 +655,28 @@ def test_tensors_derived_under_capture_stay_in_the_graph(dtype, T, monkeypatch):
         assert torch.equal(new(t), w)
 
 
+@pytest.mark.parametrize("d,rows", [(256, 3), (256, 20), (128, 20)])
+def test_generate_under_inference_mode(d, rows):
+    """torch.inference_mode() around the first call, and calls outside after it: the tokens of a call under no_grad, and those of
+    changed weights after a change."""
+    kw = dict(seed=5, init="healthy", dtype=torch.bfloat16, mlp_scale=2, n_embd=d, n_layers=4, n_heads=2, window_size=8,
+              num_eigh=8, seq_len=64, vocab_size=777)
+    ids = prompt(rows, 6, 777, rows).cuda()
+    _, _, model = make_pair(**kw)
+    _, _, other = make_pair(**kw)
+    run = lambda m: m.generate(ids, max_length=16, do_sample=False)
+    with torch.inference_mode():
+        first = run(model)
+    assert torch.equal(first, run(other)) and torch.equal(first, run(model))
+    with torch.no_grad():
+        for m in (model, other):
+            for p in m.parameters():
+                p.mul_(0.75)
+    with torch.inference_mode():
+        second = run(model)
+    assert torch.equal(second, run(other)) and torch.equal(second, run(model))
+
+
 def test_forward_accepts_reference_style_kv_cache():
     from flash_stu import Attention, FlashSTUConfig
     cfg = FlashSTUConfig(n_embd=128, n_heads=2, n_layers=2, seq_len=64, window_size=6, vocab_size=11, mlp_scale=2,
