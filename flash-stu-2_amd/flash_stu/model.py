@@ -80,6 +80,9 @@ class FlashSTU(nn.Module):
         self.apply(self._init_weights)
         self._engine = None
 
+    def __getstate__(self):
+        return {**self.__dict__, "_engine": None}      # a copy builds its own: descriptors hold this object's addresses
+
     # ------------------------------------------------------------ init
     def _init_weights(self, module):
         """model.py:428-452, including the model-level std that every SCALE_INIT

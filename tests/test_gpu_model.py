@@ -677,6 +677,23 @@ def test_generate_under_inference_mode(d, rows):
     assert torch.equal(second, run(other)) and torch.equal(second, run(model))
 
 
+def test_models_that_have_generated_can_be_copied():
+    """deepcopy and pickle of a model with an engine: the copy generates the same tokens and follows its own weights."""
+    import copy
+    import pickle
+    _, _, model = make_pair(seed=5, init="healthy", dtype=torch.bfloat16, mlp_scale=2, n_embd=256, n_layers=4, n_heads=2,
+                            window_size=8, num_eigh=8, seq_len=64, vocab_size=777)
+    ids = prompt(2, 6, 777, 1).cuda()
+    want = model.generate(ids, max_length=16, do_sample=False)
+    for other in (copy.deepcopy(model), pickle.loads(pickle.dumps(model))):
+        assert torch.equal(other.generate(ids, max_length=16, do_sample=False), want)
+        assert other.tok_emb.weight is other.lm_head.weight
+        with torch.no_grad():
+            for p in other.parameters():
+                p.zero_()
+        assert torch.equal(model.generate(ids, max_length=16, do_sample=False), want)
+
+
 def test_forward_accepts_reference_style_kv_cache():
     from flash_stu import Attention, FlashSTUConfig
     cfg = FlashSTUConfig(n_embd=128, n_heads=2, n_layers=2, seq_len=64, window_size=6, vocab_size=11, mlp_scale=2,
