@@ -422,12 +422,19 @@ class STU(nn.Module):
         hist[:, :T] = src
         return (hist, torch.empty(B, 0, dtype=torch.float32, device=src.device), pos)
 
+    def _project_step(self, x: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
+        """x (B,d) @ M_inputs into the rows of out, as many rows per launch as the skinny kernel takes."""
+        w, R = self.m_inputs_t(), _hip.MAX_DECODE_ROWS
+        for b in range(0, x.shape[0], R):
+            _hip.linear_decode(x[b:b + R], w, out[b:b + R])
+        return out
+
     def _step(self, x: torch.Tensor, past_state):
         hist, state, pos_t = past_state
         pos = int(pos_t[0])
         B, d = x.shape
         if self.use_approx and state.numel() > 0:
-            xp = _hip.linear_decode(x, self.m_inputs_t())
+            xp = self._project_step(x, x.new_empty(B, self.d_out))
             if self.use_hankel_L:
                 a, ce, co = self.lds_single_params()
                 y = _hip.stu_step_lds(state, xp, a, ce, pos, co=co)
@@ -454,7 +461,7 @@ class STU(nn.Module):
         if pos >= self.phi.shape[0]:
             raise ValueError(f"position {pos} is past the filter length {self.phi.shape[0]}")
         if self.use_approx:
-            _hip.linear_decode(x, self.m_inputs_t(), hist[:, pos, :])
+            self._project_step(x, hist[:, pos, :])
             nsplit = _hist_nsplit(pos + 1)
             eo = _hip.stu_step_hist(hist, self.effective_filter(), pos, nsplit)
             y = torch.zeros(B, d, dtype=x.dtype, device=x.device)

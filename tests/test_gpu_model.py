@@ -694,6 +694,26 @@ def test_models_that_have_generated_can_be_copied():
         assert torch.equal(model.generate(ids, max_length=16, do_sample=False), want)
 
 
+@pytest.mark.parametrize("dtype,extra", [(torch.float32, {}), (torch.bfloat16, {}), (torch.bfloat16, dict(use_hankel_L=True)),
+                                         (torch.float32, dict(use_hankel_L=True))])
+def test_steps_on_caches_of_more_rows_than_one_launch_takes(dtype, extra):
+    """forward() with caches for 37 rows (three launches of the skinny projection, one of each state operator) against the same
+    rows in groups of 16, whose sums are formed in another order: bounds as in the test of the one-call step."""
+    _, _, model = make_pair(seed=5, init="healthy", dtype=dtype, mlp_scale=2, n_embd=128, n_layers=4, n_heads=2, window_size=8,
+                            num_eigh=8, seq_len=64, vocab_size=777, **extra)
+    ids = prompt(37, 10, 777, 3).cuda()
+
+    def run(rows):
+        past, logits = model(rows[:, :6], use_cache=True).past_key_values, []
+        for t in range(6, 10):
+            out = model(rows[:, t:t + 1], past_key_values=past, use_cache=True)
+            past = out.past_key_values
+            logits.append(out.logits.float())
+        return torch.cat(logits, 1)
+    got, want = run(ids), torch.cat([run(ids[b:b + 16]) for b in range(0, 37, 16)])
+    assert float((got - want).abs().max()) <= (1e-4 if dtype == torch.float32 else 2e-2) * float(want.abs().max())
+
+
 def test_forward_accepts_reference_style_kv_cache():
     from flash_stu import Attention, FlashSTUConfig
     cfg = FlashSTUConfig(n_embd=128, n_heads=2, n_layers=2, seq_len=64, window_size=6, vocab_size=11, mlp_scale=2,
