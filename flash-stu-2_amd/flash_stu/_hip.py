@@ -170,11 +170,6 @@ def _p(t: Optional[torch.Tensor]):
     return None if t is None else t.data_ptr()
 
 
-def version(t: torch.Tensor):
-    """The counter of a tensor's in-place changes; None for one made under torch.inference_mode(), which has none."""
-    return None if t.is_inference() else t._version
-
-
 raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)    # handle of a device's current stream (0.1 us; the object 2.9)
 
 

@@ -230,11 +230,13 @@ class DecodeEngine:
         self._gstreams = []
 
     # ------------------------------------------------------------------
-    def _pack(self, w: torch.Tensor, place) -> torch.Tensor:
+    def _pack(self, w: torch.Tensor, place, derived: bool = False) -> torch.Tensor:
         """MFMA-fragment-ordered copy of the (N,K) bf16 weight at `place` in the model, rebuilt only when the weight changes.
         The entry holds the storage that it was made from: while it is there no other tensor can come to lie at the address
-        it is recognised by."""
-        hit, made_from = self._packed.get(place), (_hip.version(w), w.data_ptr())
+        it is recognised by.  derived: w is itself a copy that its module forms anew when the parameter changes and that
+        nothing writes to afterwards, so its address alone tells it (one formed under torch.inference_mode() has no counter of
+        its changes)."""
+        hit, made_from = self._packed.get(place), (0 if derived else w._version, w.data_ptr())
         if hit is None or hit[0] != made_from:
             hit = (made_from, _hip.pack_rows(w), w.detach())
             self._packed[place] = hit
@@ -413,7 +415,7 @@ class DecodeEngine:
                 if "qkv" in w:
                     ld.wp_qkv, ld.wp_proj = ptr(self._pack(w["qkv"], (i, "qkv"))), ptr(self._pack(w["proj"], (i, "proj")))
                 elif mode == "lds":
-                    ld.wp_m_inputs = ptr(self._pack(w["m_inputs"], (i, "m_inputs")))
+                    ld.wp_m_inputs = ptr(self._pack(w["m_inputs"], (i, "m_inputs"), derived=True))
         if dt == torch.bfloat16 and self.lib.fstu_glu_packed_supported(min(B, _hip.MAX_DECODE_ROWS), d, V):
             m.wp_emb = ptr(self._pack(emb, "emb"))      # the head streams a packed copy of the embedding
         ch.arr, ch.desc = arr, m

@@ -67,7 +67,7 @@ class STU(nn.Module):
     # made from, so that no other tensor can come to lie at the address it is recognised by (a parametrized weight is a
     # new tensor on every access).  A call on another stream than the one that launched the copy waits for it.
     def _cached(self, key, params, build):
-        ver = tuple((_hip.version(p), p.data_ptr()) for p in params)
+        ver = tuple((p._version, p.data_ptr()) for p in params)
         hit = self._derived.get(key)
         if hit is None or hit[0] != ver:
             # behind the sources: the device, the streams that are behind the launch, and the one that made it (an event

@@ -273,3 +273,15 @@ def test_derived_copies_follow_weights_that_are_new_tensors_every_time(monkeypat
         assert torch.equal(engine._pack(w, (0, "m_inputs")), w)
         del w
     assert len(places) > 1 and len(engine._packed) == 1
+
+
+def test_weights_whose_changes_cannot_be_seen_are_refused():
+    """Parameters made under torch.inference_mode() have no counter of their in-place changes: what is derived from them could
+    be out of date without a sign of it."""
+    from flash_stu import STU, FlashSTUConfig
+    cfg = FlashSTUConfig(n_embd=64, n_heads=2, n_layers=2, seq_len=32, num_eigh=4, vocab_size=64, torch_dtype=torch.float32)
+    with torch.inference_mode():
+        stu = STU(cfg, torch.randn(32, 4), 64)
+        for derive in (stu.m_inputs_t, stu.effective_filter):
+            with pytest.raises(RuntimeError, match="version counter"):
+                derive()
