@@ -28,12 +28,13 @@ from ..utils.lds_fit import check_lds_fit, fit_even_lag_lds
 FFT_MIN_T = 32     # shorter inputs take the time-domain kernel (a 64-point transform would be mostly padding)
 
 
-def _wait_for(stream) -> bool:
-    """Orders the current stream behind what `stream` has been given; a stream that is being captured cannot wait for
-    work outside the capture."""
+def _wait_for(handle: int, device: int) -> bool:
+    """Orders the device's current stream behind what the stream of that handle has been given; a stream that is being
+    captured cannot wait for work outside the capture."""
     if torch.cuda.is_current_stream_capturing():
         return False
-    torch.cuda.current_stream(stream.device).wait_event(stream.record_event())
+    stream = torch.cuda.ExternalStream(handle, device=device) if handle else torch.cuda.default_stream(device)
+    torch.cuda.current_stream(device).wait_event(stream.record_event())
     return True
 
 
@@ -70,16 +71,16 @@ class STU(nn.Module):
         ver = tuple((p._version, p.data_ptr()) for p in params)
         hit = self._derived.get(key)
         if hit is None or hit[0] != ver:
-            # behind the sources: the device, the streams that are behind the launch, and the one that made it (an event
-            # recorded here would delay the first call by some 16 us)
-            dev, value = params[0].device, build()
-            if dev.type == "cuda" and torch.cuda.is_current_stream_capturing():
-                return value             # part of the graph: written when it is replayed
-            stream = torch.cuda.current_stream(dev) if dev.type == "cuda" else None
-            hit = (ver, value, [p.detach() for p in params], -1 if stream is None else dev.index,
-                   {None if stream is None else stream.cuda_stream}, stream)
+            # behind the sources: the device, the handles of the streams that are behind the launch and of the one that made
+            # it (an event recorded here would delay the first call by some 16 us, the stream objects by 9)
+            dev, value, here = params[0].device, build(), None
+            if dev.type == "cuda":
+                if torch.cuda.is_current_stream_capturing():
+                    return value             # part of the graph: written when it is replayed
+                here = _hip.raw_stream(dev.index)
+            hit = (ver, value, [p.detach() for p in params], -1 if here is None else dev.index, {here}, here)
             self._derived[key] = hit
-        elif hit[3] >= 0 and _hip.raw_stream(hit[3]) not in hit[4] and _wait_for(hit[5]):
+        elif hit[3] >= 0 and _hip.raw_stream(hit[3]) not in hit[4] and _wait_for(hit[5], hit[3]):
             hit[4].add(_hip.raw_stream(hit[3]))
         return hit[1]
 

@@ -604,7 +604,8 @@ def test_derived_tensors_are_complete_on_every_stream():
     phi, x = torch.randn(512, 8, generator=g).bfloat16(), torch.randn(2, 300, 256, generator=g).bfloat16().cuda()
     stu = STU(cfg, phi, 1024).cuda()
     other, big = torch.cuda.Stream(), torch.randn(4096, 4096, device="cuda")
-    for turn in range(3):
+    default = torch.cuda.current_stream()
+    for first, second in ((other, default), (default, other)) * 2:
         with torch.no_grad():
             for p in stu.parameters():
                 p.copy_(torch.randn(p.shape, generator=g))
@@ -612,16 +613,16 @@ def test_derived_tensors_are_complete_on_every_stream():
         fresh.load_state_dict(stu.state_dict())
         want = fresh(x)
         torch.cuda.synchronize()
-        with torch.cuda.stream(other):
+        with torch.cuda.stream(first):
             for _ in range(8):                  # some milliseconds in front of the copies
                 big @ big
             there = stu(x)
-        here = stu(x)
-        assert torch.equal(here, want)
-        torch.cuda.current_stream().wait_stream(other)
-        assert torch.equal(there, want)
+        with torch.cuda.stream(second):
+            here = stu(x)
+            assert torch.equal(here, want)
         torch.cuda.synchronize()
-        assert torch.equal(stu(x), want) and stu._derived["mit"][4] == {other.cuda_stream, torch.cuda.current_stream().cuda_stream}
+        assert torch.equal(there, want)
+        assert torch.equal(stu(x), want) and stu._derived["mit"][4] == {other.cuda_stream, default.cuda_stream}
     for copied in (copy.deepcopy(stu), pickle.loads(pickle.dumps(stu))):
         assert torch.equal(copied(x), want)
 
