@@ -66,7 +66,8 @@ class STU(nn.Module):
 
     # ---- tensors derived from the parameters, rebuilt when a parameter changes; an entry holds the storage that it was
     # made from, so that no other tensor can come to lie at the address it is recognised by (a parametrized weight is a
-    # new tensor on every access).  A call on another stream than the one that launched the copy waits for it.
+    # new tensor on every access).  A call on another stream than the one that launched the copy waits for it, and its memory
+    # is not given out again before that stream has read it.
     def _cached(self, key, params, build):
         ver = tuple((p._version, p.data_ptr()) for p in params)
         hit = self._derived.get(key)
@@ -82,6 +83,9 @@ class STU(nn.Module):
             self._derived[key] = hit
         elif hit[3] >= 0 and _hip.raw_stream(hit[3]) not in hit[4] and _wait_for(hit[5], hit[3]):
             hit[4].add(_hip.raw_stream(hit[3]))
+            for t in hit[1] if isinstance(hit[1], tuple) else hit[1:2]:
+                if t is not None:
+                    t.record_stream(torch.cuda.current_stream(hit[3]))
         return hit[1]
 
     def __getstate__(self):

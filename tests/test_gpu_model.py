@@ -627,6 +627,37 @@ def test_derived_tensors_are_complete_on_every_stream():
         assert torch.equal(copied(x), want)
 
 
+def test_derived_tensors_outlive_what_other_streams_read():
+    """Spectra that another stream has still to read while a call of another length replaces them, and memory of their size that
+    the stream that made them asks for then and fills."""
+    from flash_stu import STU, FlashSTUConfig
+    cfg = FlashSTUConfig(n_embd=256, n_heads=4, n_layers=2, seq_len=1024, num_eigh=8, vocab_size=64, torch_dtype=torch.bfloat16)
+    g = torch.Generator().manual_seed(2)
+    phi = torch.randn(1024, 8, generator=g).bfloat16()
+    x, longer = (torch.randn(2, T, 256, generator=g).bfloat16().cuda() for T in (300, 700))
+    stu = STU(cfg, phi, 2048).cuda()
+    with torch.no_grad():
+        for p in stu.parameters():
+            p.copy_(torch.randn(p.shape, generator=g))
+    stu(longer)
+    other, big = torch.cuda.Stream(), torch.randn(4096, 4096, device="cuda")
+    want = stu(x)
+    spec = stu._derived["spec"][1]
+    shape, at = spec.shape, spec.data_ptr()
+    del spec
+    torch.cuda.synchronize()
+    with torch.cuda.stream(other):
+        for _ in range(8):
+            big @ big
+        there = stu(x)
+    stu(longer)
+    assert stu._derived["spec"][1].shape != shape
+    fills = [torch.full(shape, 7.0, device="cuda") for _ in range(3)]
+    assert at not in [t.data_ptr() for t in fills]
+    torch.cuda.synchronize()
+    assert torch.equal(there, want)
+
+
 @pytest.mark.parametrize("dtype,T", [(torch.bfloat16, 300), (torch.float32, 20), (torch.float32, 100)])
 def test_tensors_derived_under_capture_stay_in_the_graph(dtype, T, monkeypatch):
     """The first call on new weights inside a capture: calls beside the graph do not read what only its replay writes, and
