@@ -23,6 +23,14 @@
 // (4.66 ms on transforms of 16384 points in 139 KB of LDS, one workgroup per compute unit; 3.77 ms while spectra and
 // twiddles lay in position order, so that every load of a wave touched up to 64 lines).  bf16, before -> now, us: 8 x 512 x
 // 768 24.5 -> 17.4, 32 x 300 x 2048 188 -> 105, 4 x 4096 x 2048 296 -> 218, one time-major sequence of 4096 x 2048 95 -> 50.
+//
+// Error.  A group that forms half of its twiddles from the others (turn32) rounds them twice more, and v = 2a - u carries u's
+// roundings on.  Beside the rounding of bf16 results neither shows.  fp32 operands take their twiddles from the table, each
+// rounded once, and where sums over all positions follow (filter spectra, gradients) butterflies of two rounded outputs each.
+// Relative error of fp32 results against float64, transforms of the whole sequence in radix 16 / these with formed twiddles /
+// now: 1000 positions 1.80e-7 / 2.03e-7 / 1.66e-7, filter's gradient 2.18e-7 / 2.60e-7 / 2.04e-7; 8000 positions 2.16e-7 /
+// 2.50e-7 / 1.90e-7 and 2.54e-7 / 3.24e-7 / 2.35e-7.  us, formed / now: 8 x 2048 x 768 64 / 64, gradients 105 / 110 (of both
+// branches 164 / 181); 4 x 4096 x 2048 210 / 210; 32 x 300 x 2048 106 / 104.
 #include "fstu_common.h"
 
 #include <type_traits>
@@ -36,6 +44,12 @@ typedef float2 cpx;
 __device__ __forceinline__ int phys(int i) { return i + (i >> 4); }
 
 // ---------------------------------------------------------------- butterflies
+// How exact a transform is (see the note above).  FORMED: half the twiddles formed by turn32; TABLE: all from the table; TABLE_STEPS:
+// the same stage by stage, for the row pieces, whose other registers leave the scheduler no room to run stages into each
+// other (4 x 4096 x 2048 rows 314 us without, 264 with; the bank of filters 122 us without, 139 with); DIRECT: all from the table and both
+// outputs of a butterfly formed from its inputs.
+enum { FORMED, TABLE, TABLE_STEPS, DIRECT };
+template <typename T, int HOW> __host__ __device__ constexpr int fine() { return sizeof(T) == 4 ? HOW : FORMED; }
 // (a, b) <- (a + w r b, a - w r b), r = 1 or (ROT) the quarter turn of the direction (-i forward, +i inverse)
 template <bool INV, bool ROT>
 __device__ __forceinline__ cpx turn(cpx b) {
@@ -48,11 +62,12 @@ __device__ __forceinline__ void bfly1(cpx& a, cpx& b) {
   b = make_float2(a.x - t.x, a.y - t.y);
   a = make_float2(a.x + t.x, a.y + t.y);
 }
-template <bool INV, bool ROT>
+template <bool INV, bool ROT, int HOW>
 __device__ __forceinline__ void bfly(cpx& a, cpx& b, cpx w) {
   const cpx t = turn<INV, ROT>(b);
   const cpx u = make_float2(fmaf(-w.y, t.y, fmaf(w.x, t.x, a.x)), fmaf(w.y, t.x, fmaf(w.x, t.y, a.y)));
-  b = make_float2(fmaf(2.f, a.x, -u.x), fmaf(2.f, a.y, -u.y));
+  b = HOW == DIRECT ? make_float2(fmaf(w.y, t.y, fmaf(-w.x, t.x, a.x)), fmaf(-w.y, t.x, fmaf(-w.x, t.y, a.y)))
+           : make_float2(fmaf(2.f, a.x, -u.x), fmaf(2.f, a.y, -u.y));
   a = u;
 }
 // a + w r b alone
@@ -83,20 +98,25 @@ __host__ __device__ constexpr int brev_bits(int v, int bits) {
   for (int i = 0; i < bits; ++i) r |= ((v >> i) & 1) << (bits - 1 - i);
   return r;
 }
-template <int G> struct Powers { cpx w[G]; };     // w^(2^i)
+// The twiddles of G stages: w^(2^i), which the first butterfly (block) of stage G-1-i uses; but for FORMED those of the others
+// up to quarter turns too.
+template <int G, int HOW> struct Powers { cpx w[HOW != FORMED ? 1 << (G - 1) : G]; };
+// where the twiddle of stage s and q steps of 2^(4-s)/32 turns lies
+__host__ __device__ constexpr int twiddle_at(int G, int s, int q) { return q == 0 ? G - 1 - s : s == 2 ? G : q == 2 ? 5 : q == 1 ? 6 : 7; }
 
 // G forward stages on 2^G points a fixed distance apart, natural order in, bit-reversed out.  TW: times the block's
 // twiddles t; HALF0: the upper half of the inputs is zero.
-template <int G, bool TW, bool HALF0>
-__device__ __forceinline__ void fwd_stages(cpx* v, const Powers<G>& t) {
+template <int G, bool TW, bool HALF0, int HOW>
+__device__ __forceinline__ void fwd_stages(cpx* v, const Powers<G, HOW>& t) {
 #pragma unroll
   for (int s = 0; s < G; ++s) {
     const int dist = 1 << (G - 1 - s);
+    if constexpr (HOW == TABLE_STEPS) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int b = 0; b < (1 << s); ++b) {
       const int k = brev_bits(b, s), quarter = s > 0 ? 1 << (s - 1) : 1;
       const bool rot = s > 0 && k >= quarter;
-      const int kr = (rot ? k - quarter : k) << (4 - s);            // in 1/32 turns
+      const int q = rot ? k - quarter : k, kr = q << (4 - s);       // in 1/32 turns
 #pragma unroll
       for (int j = 0; j < dist; ++j) {
         cpx &x = v[b * 2 * dist + j], &y = v[b * 2 * dist + j + dist];
@@ -104,8 +124,8 @@ __device__ __forceinline__ void fwd_stages(cpx* v, const Powers<G>& t) {
         if (!TW && kr == 0) {
           if (rot) bfly1<false, true>(x, y); else bfly1<false, false>(x, y);
         } else {
-          const cpx w = TW ? turn32<false>(t.w[G - 1 - s], kr) : root32<false>(kr);
-          if (rot) bfly<false, true>(x, y, w); else bfly<false, false>(x, y, w);
+          const cpx w = !TW ? root32<false>(kr) : HOW != FORMED ? t.w[twiddle_at(G, s, q)] : turn32<false>(t.w[G - 1 - s], kr);
+          if (rot) bfly<false, true, HOW>(x, y, w); else bfly<false, false, HOW>(x, y, w);
         }
       }
     }
@@ -113,26 +133,27 @@ __device__ __forceinline__ void fwd_stages(cpx* v, const Powers<G>& t) {
 }
 // G inverse stages, bit-reversed in, natural out; t holds the conjugate twiddles of the position.  LOWER: only the lower
 // half of the results is produced.
-template <int G, bool TW, bool LOWER>
-__device__ __forceinline__ void inv_stages(cpx* v, const Powers<G>& t) {
+template <int G, bool TW, bool LOWER, int HOW>
+__device__ __forceinline__ void inv_stages(cpx* v, const Powers<G, HOW>& t) {
 #pragma unroll
   for (int s = 0; s < G; ++s) {
     const int dist = 1 << s;
+    if constexpr (HOW == TABLE_STEPS) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int b = 0; b < (1 << s); ++b) {
       const int quarter = s > 0 ? 1 << (s - 1) : 1;
       const bool rot = s > 0 && b >= quarter;
-      const int kr = (rot ? b - quarter : b) << (4 - s);
+      const int q = rot ? b - quarter : b, kr = q << (4 - s);
 #pragma unroll
       for (int g = 0; g < (1 << G); g += 2 * dist) {
         cpx &x = v[g + b], &y = v[g + b + dist];
-        const cpx w = TW ? turn32<true>(t.w[G - 1 - s], kr) : root32<true>(kr);
+        const cpx w = !TW ? root32<true>(kr) : HOW != FORMED ? t.w[twiddle_at(G, s, q)] : turn32<true>(t.w[G - 1 - s], kr);
         if (LOWER && s == G - 1) {
           if (rot) x = bsum<true, true>(x, y, w); else x = bsum<true, false>(x, y, w);
         } else if (!TW && kr == 0) {
           if (rot) bfly1<true, true>(x, y); else bfly1<true, false>(x, y);
         } else {
-          if (rot) bfly<true, true>(x, y, w); else bfly<true, false>(x, y, w);
+          if (rot) bfly<true, true, HOW>(x, y, w); else bfly<true, false, HOW>(x, y, w);
         }
       }
     }
@@ -163,33 +184,32 @@ template <int LOGN> __device__ __forceinline__ void col_sync() {
 }
 
 // The twiddle table: for every group the powers 1, 2, 4, 8 of the twiddles of its positions (inverse, conjugated) or
-// blocks (forward, in block order), as planes of two powers each, so that the lanes of a wave read whole lines and a
-// group's twiddles are at most two loads.  All of it fits the n entries of exp(-2 pi i j / n).
+// blocks (forward, in block order) and behind them what twiddle_at names, as planes of two each, so that the lanes of a wave
+// read whole lines and a group's twiddles are at most four loads (FORMED: two).  All of it fits n entries.
 template <int LOGN> struct Table {
   using W = Half<LOGN>;
-  static constexpr int planes(int stages) { return stages == 1 ? 1 : stages == 2 ? 2 : 4; }    // entries per position
+  static constexpr int planes(int stages) { return 1 << (stages - 1); }                        // entries per position
   static constexpr int INV1 = 0;                                                   // stride 16: 16 positions
-  static constexpr int INV2 = INV1 + (W::MID >= 1 ? 16 * 4 : 0);                   // stride 256
-  static constexpr int OUTER = INV2 + (W::MID >= 2 ? 256 * 4 : 0);                 // outermost group: Q positions
+  static constexpr int INV2 = INV1 + (W::MID >= 1 ? 16 * 8 : 0);                   // stride 256
+  static constexpr int OUTER = INV2 + (W::MID >= 2 ? 256 * 8 : 0);                 // outermost group: Q positions
   static constexpr int FWD2 = OUTER + W::Q * planes(W::GL);
-  static constexpr int FWD1 = FWD2 + (W::MID >= 2 ? (W::N >> 12) * 4 : 0);         // stride 16: N / 256 blocks
-  static constexpr int FWD0 = FWD1 + (W::MID >= 1 ? (W::N >> 8) * 4 : 0);          // stride 1: N / 16 blocks
-  static constexpr int END = FWD0 + (W::N >> 4) * 4;
+  static constexpr int FWD1 = FWD2 + (W::MID >= 2 ? (W::N >> 12) * 8 : 0);         // stride 16: N / 256 blocks
+  static constexpr int FWD0 = FWD1 + (W::MID >= 1 ? (W::N >> 8) * 8 : 0);          // stride 1: N / 16 blocks
+  static constexpr int END = FWD0 + (W::N >> 4) * 8;
   static_assert(END <= 2 * W::N, "the table fits n entries");
 };
-// GS powers of entry i of a part of the table that has `count` entries
-template <int GS> __device__ __forceinline__ Powers<GS> powers(const cpx* __restrict__ part, int count, int i) {
-  Powers<GS> t;
+// the twiddles of GS stages of entry i of a part of the table that has `count` entries
+template <int GS, int HOW> __device__ __forceinline__ Powers<GS, HOW> powers(const cpx* __restrict__ part, int count, int i) {
+  constexpr int NW = HOW != FORMED ? 1 << (GS - 1) : GS;
+  Powers<GS, HOW> t;
   if constexpr (GS == 1) {
     t.w[0] = part[i];
   } else {
-    const float4 a = ((const float4*)part)[i];
-    t.w[0] = make_float2(a.x, a.y);
-    t.w[1] = make_float2(a.z, a.w);
-    if constexpr (GS > 2) {
-      const float4 c = ((const float4*)part)[count + i];
-      t.w[2] = make_float2(c.x, c.y);
-      if constexpr (GS > 3) t.w[3] = make_float2(c.z, c.w);
+#pragma unroll
+    for (int p = 0; p < (NW + 1) / 2; ++p) {
+      const float4 a = ((const float4*)part)[p * count + i];
+      t.w[2 * p] = make_float2(a.x, a.y);
+      if (2 * p + 1 < NW) t.w[2 * p + 1] = make_float2(a.z, a.w);
     }
   }
   return t;
@@ -208,36 +228,36 @@ template <int LOGN> __device__ __forceinline__ int butterfly_at(int u, int i) {
 }
 
 // four stages at stride 16^LEVEL, in place
-template <int LOGN, int LEVEL>
+template <int LOGN, int LEVEL, int HOW>
 __device__ __forceinline__ void fwd_mid(cpx* __restrict__ col, const cpx* __restrict__ tw, int u) {
   constexpr int LQ = 4 * LEVEL, S = LOGN - 4 - LQ, ST = (1 << LQ) + (1 << LQ) / 16;
   const int blk = u >> LQ;
-  const Powers<4> t = powers<4>(tw + (LEVEL == 1 ? Table<LOGN>::FWD1 : Table<LOGN>::FWD2), 1 << S, blk);
+  const Powers<4, HOW> t = powers<4, HOW>(tw + (LEVEL == 1 ? Table<LOGN>::FWD1 : Table<LOGN>::FWD2), 1 << S, blk);
   cpx* p = col + phys((blk << (LQ + 4)) + (u & ((1 << LQ) - 1)));
   cpx v[16];
 #pragma unroll
   for (int m = 0; m < 16; ++m) v[m] = p[m * ST];
-  fwd_stages<4, true, false>(v, t);
+  fwd_stages<4, true, false, HOW>(v, t);
 #pragma unroll
   for (int m = 0; m < 16; ++m) p[m * ST] = v[m];
 }
-template <int LOGN, int LEVEL>
+template <int LOGN, int LEVEL, int HOW>
 __device__ __forceinline__ void inv_mid(cpx* __restrict__ col, const cpx* __restrict__ tw, int u) {
   constexpr int LQ = 4 * LEVEL, ST = (1 << LQ) + (1 << LQ) / 16;
   const int r = u & ((1 << LQ) - 1);
-  const Powers<4> t = powers<4>(tw + (LEVEL == 1 ? Table<LOGN>::INV1 : Table<LOGN>::INV2), 1 << LQ, r);
+  const Powers<4, HOW> t = powers<4, HOW>(tw + (LEVEL == 1 ? Table<LOGN>::INV1 : Table<LOGN>::INV2), 1 << LQ, r);
   cpx* p = col + phys(((u >> LQ) << (LQ + 4)) + r);
   cpx v[16];
 #pragma unroll
   for (int m = 0; m < 16; ++m) v[m] = p[m * ST];
-  inv_stages<4, true, false>(v, t);
+  inv_stages<4, true, false, HOW>(v, t);
 #pragma unroll
   for (int m = 0; m < 16; ++m) p[m * ST] = v[m];
 }
 
 // z: the thread's 8 points of the lower half -> xs: spectrum of positions 16u .. 16u+15 (bit-reversed order).  When it
 // returns, a thread may overwrite its own 16 positions of the column.
-template <int LOGN>
+template <int LOGN, int HOW>
 __device__ __forceinline__ void fft_forward(cpx* __restrict__ col, const cpx* __restrict__ tw, int u, const cpx (&z)[8], cpx (&xs)[16]) {
   using W = Half<LOGN>;
 #pragma unroll
@@ -245,42 +265,42 @@ __device__ __forceinline__ void fft_forward(cpx* __restrict__ col, const cpx* __
     cpx v[W::R];
 #pragma unroll
     for (int m = 0; m < W::H; ++m) v[m] = z[i * W::H + m];
-    fwd_stages<W::GL, false, true>(v, Powers<W::GL>{});
+    fwd_stages<W::GL, false, true, HOW>(v, Powers<W::GL, HOW>{});
     cpx* p = col + butterfly_at<LOGN>(u, i);
 #pragma unroll
     for (int m = 0; m < W::R; ++m) p[m * (W::Q + W::Q / 16)] = v[m];
   }
-  if constexpr (W::MID >= 2) { col_sync<LOGN>(); fwd_mid<LOGN, 2>(col, tw, u); }
-  if constexpr (W::MID >= 1) { col_sync<LOGN>(); fwd_mid<LOGN, 1>(col, tw, u); }
+  if constexpr (W::MID >= 2) { col_sync<LOGN>(); fwd_mid<LOGN, 2, HOW>(col, tw, u); }
+  if constexpr (W::MID >= 1) { col_sync<LOGN>(); fwd_mid<LOGN, 1, HOW>(col, tw, u); }
   if constexpr (W::MID == 0) col_sync<LOGN>();
   else wave_sync();
-  const Powers<4> t = powers<4>(tw + Table<LOGN>::FWD0, W::G, u);
+  const Powers<4, HOW> t = powers<4, HOW>(tw + Table<LOGN>::FWD0, W::G, u);
 #pragma unroll
   for (int m = 0; m < 16; ++m) xs[m] = col[17 * u + m];
-  fwd_stages<4, true, false>(xs, t);
+  fwd_stages<4, true, false, HOW>(xs, t);
 }
 
 // v: spectrum of positions 16u .. 16u+15 -> r: the thread's 8 points of the lower half of the result.  The thread's own 16
 // positions of the column must be free; when it returns, other threads may still read the column.
-template <int LOGN>
+template <int LOGN, int HOW>
 __device__ __forceinline__ void fft_inverse(cpx* __restrict__ col, const cpx* __restrict__ tw, int u, cpx (&v)[16], cpx (&r)[8]) {
   using W = Half<LOGN>;
-  inv_stages<4, false, false>(v, Powers<4>{});
+  inv_stages<4, false, false, HOW>(v, Powers<4, HOW>{});
 #pragma unroll
   for (int m = 0; m < 16; ++m) col[17 * u + m] = v[m];
   if constexpr (W::MID == 0) col_sync<LOGN>();
   else wave_sync();
-  if constexpr (W::MID >= 1) { inv_mid<LOGN, 1>(col, tw, u); col_sync<LOGN>(); }
-  if constexpr (W::MID >= 2) { inv_mid<LOGN, 2>(col, tw, u); col_sync<LOGN>(); }
+  if constexpr (W::MID >= 1) { inv_mid<LOGN, 1, HOW>(col, tw, u); col_sync<LOGN>(); }
+  if constexpr (W::MID >= 2) { inv_mid<LOGN, 2, HOW>(col, tw, u); col_sync<LOGN>(); }
 #pragma unroll
   for (int i = 0; i < W::NI; ++i) {
     const int rr = u + i * W::G;
-    const Powers<W::GL> t = powers<W::GL>(tw + Table<LOGN>::OUTER, W::Q, rr);
+    const Powers<W::GL, HOW> t = powers<W::GL, HOW>(tw + Table<LOGN>::OUTER, W::Q, rr);
     const cpx* p = col + butterfly_at<LOGN>(u, i);
     cpx x[W::R];
 #pragma unroll
     for (int m = 0; m < W::R; ++m) x[m] = p[m * (W::Q + W::Q / 16)];
-    inv_stages<W::GL, true, true>(x, t);
+    inv_stages<W::GL, true, true, HOW>(x, t);
 #pragma unroll
     for (int m = 0; m < W::H; ++m) r[i * W::H + m] = x[m];
   }
@@ -358,29 +378,35 @@ __global__ void __launch_bounds__(256) fft_twiddle_kernel(cpx* __restrict__ tw) 
   if (j >= 2 * W::N) return;
   // entry j: its part, its index there, its power and its angle in turns
   struct Part { int begin, count, entries, shift; bool fwd; };
-  const Part parts[6] = {{B::INV1, 16, W::MID >= 1 ? 4 : 0, 8, false},
-                         {B::INV2, 256, W::MID >= 2 ? 4 : 0, 12, false},
+  const Part parts[6] = {{B::INV1, 16, W::MID >= 1 ? 8 : 0, 8, false},
+                         {B::INV2, 256, W::MID >= 2 ? 8 : 0, 12, false},
                          {B::OUTER, W::Q, B::planes(W::GL), LOGN, false},
-                         {B::FWD2, W::N >> 12, W::MID >= 2 ? 4 : 0, 0, true},
-                         {B::FWD1, W::N >> 8, W::MID >= 1 ? 4 : 0, 0, true},
-                         {B::FWD0, W::N >> 4, 4, 0, true}};
+                         {B::FWD2, W::N >> 12, W::MID >= 2 ? 8 : 0, 0, true},
+                         {B::FWD1, W::N >> 8, W::MID >= 1 ? 8 : 0, 0, true},
+                         {B::FWD0, W::N >> 4, 8, 0, true}};
   double turns = 0.0;
   for (int q = 0; q < 6; ++q) {
     const Part& p = parts[q];
     const int o = j - p.begin;
     if (p.entries == 0 || o < 0 || o >= p.count * p.entries) continue;
-    int i = o, power = 0;
+    int i = o, power = 0, steps = 0;                   // w^(2^power), `steps` of 1/32 turns further
     if (p.entries > 1) {
       i = (o >> 1) % p.count;
-      power = 2 * ((o >> 1) / p.count) + (o & 1);
+      const int at = 2 * ((o >> 1) / p.count) + (o & 1), G = p.entries == 8 ? 4 : p.entries == 4 ? 3 : 2;
+      for (int st = 0; st < G; ++st)
+        for (int k = 0; k < (st < 2 ? 1 : 1 << (st - 1)); ++k)
+          if (twiddle_at(G, st, k) == at) {
+            power = G - 1 - st;
+            steps = k << (4 - st);
+          }
     }
     if (p.fwd) {
       int lg = 0;
       while ((1 << lg) < p.count) ++lg;
       const double f = lg ? (double)(__brev((unsigned)i) >> (32 - lg)) : 0.0;
-      turns = -f * (double)(1 << power) / (double)(p.count * 16);
+      turns = -f * (double)(1 << power) / (double)(p.count * 16) - steps / 32.0;
     } else {
-      turns = (double)i * (double)(1 << power) / (double)(1 << p.shift);
+      turns = (double)i * (double)(1 << power) / (double)(1 << p.shift) + steps / 32.0;
     }
   }
   double s, c;
@@ -442,7 +468,7 @@ fft_filter_kernel(const T* __restrict__ filt, size_t f_ls, size_t f_cs, cpx* __r
 #pragma unroll
   for (int k = 0; k < 8; ++k) z[k] = col[phys(point<LOGN>(u, k))];
   __syncthreads();
-  fft_forward<LOGN>(col, tw, u, z, v);
+  fft_forward<LOGN, fine<T, DIRECT>()>(col, tw, u, z, v);
 #pragma unroll
   for (int m = 0; m < 16; ++m) col[17 * u + m] = v[m];
   __syncthreads();
@@ -492,7 +518,7 @@ fft_slab_kernel(const T* __restrict__ x, size_t x_sb, size_t x_sc, const cpx* __
     if (t + 1 < Tn) z[k] = Pair<T>::get(*(const typename Pair<T>::mem*)(xp + t));
     else if (t < Tn) z[k].x = DT<T>::ld(xp + t);
   }
-  fft_forward<LOGN>(col, tw, u, z, xs);
+  fft_forward<LOGN, fine<T, TABLE>()>(col, tw, u, z, xs);
   const cpx* sp = spec + (K == 1 ? (size_t)min(c, d - 1) * (2 * N) : 0) + 2 * u;
   T* yp = y + (size_t)b * y_sb + (size_t)c * y_sc;
   T* yp2 = y2 + (size_t)b * y_sb + (size_t)c * y_sc;
@@ -500,10 +526,10 @@ fft_slab_kernel(const T* __restrict__ x, size_t x_sb, size_t x_sc, const cpx* __
     cpx v[16], e[8], o[8];
     float prev[8];
     product16<LOGN>(sp, xs, v);
-    fft_inverse<LOGN>(col, here(tw), here(u), v, e);
+    fft_inverse<LOGN, fine<T, TABLE>()>(col, here(tw), here(u), v, e);
     col_sync<LOGN>();
     product16<LOGN>(sp + N, xs, v);
-    fft_inverse<LOGN>(col, here(tw), here(u), v, o);
+    fft_inverse<LOGN, fine<T, TABLE>()>(col, here(tw), here(u), v, o);
     earlier_im<LOGN>(o, prev, rec, u);
     const int uo = here(u), tmax = live ? Tn - 1 : 0;  // pairs t, t + 1 <= tmax are stored
 #pragma unroll
@@ -567,16 +593,16 @@ fft_conv_kernel(const T* __restrict__ x, size_t x_sb, size_t x_st, size_t x_sc, 
 #pragma unroll
   for (int k = 0; k < 8; ++k) z[k] = col[phys(point<LOGN>(u, k))];
   __syncthreads();
-  fft_forward<LOGN>(col, tw, u, z, xs);
+  fft_forward<LOGN, fine<T, TABLE>()>(col, tw, u, z, xs);
   const cpx* sp = spec + (size_t)(K == 1 ? min(c0 + mycol, d - 1) : k0) * (2 * N) + 2 * u;
   for (int k = k0; k < k1; ++k, sp += 2 * N) {
     cpx v[16], e[8], o[8];
     float prev[8];
     product16<LOGN>(sp, xs, v);
-    fft_inverse<LOGN>(col, here(tw), here(u), v, e);
+    fft_inverse<LOGN, fine<T, TABLE>()>(col, here(tw), here(u), v, e);
     col_sync<LOGN>();
     product16<LOGN>(sp + N, xs, v);
-    fft_inverse<LOGN>(col, here(tw), here(u), v, o);
+    fft_inverse<LOGN, fine<T, TABLE>()>(col, here(tw), here(u), v, o);
     earlier_im<LOGN>(o, prev, rec, u);
     for (int br = 0; br < (mode == 2 ? 2 : 1); ++br) {
       __syncthreads();
@@ -685,6 +711,9 @@ fft_conv_rows_kernel(const T* __restrict__ x, size_t x_sb, size_t x_st, const cp
   float* rec = (float*)(fft_lds + (size_t)COLS * W::STRIDE);
   pair_t* stage = (pair_t*)fft_lds;                    // [column][pair], in the columns' place
   const cpx* sp = spec + (size_t)(c0 + mycol) * (2 * N) + 2 * u;
+  // with the table's twiddles the inverse of 4096 points spills 23 registers, and the error is small enough without (3000 / 4096
+  // positions 1.80e-7 / 1.99e-7, radix 16 2.04e-7 / 2.12e-7)
+  constexpr int BACK = LOGN == 12 ? FORMED : TABLE_STEPS;
   for (int g = 0; g < R::NG; ++g, sp += (size_t)COLS * (2 * N)) {
     if (g > 0) __syncthreads();                        // the previous group's results have been collected
     const int tid = here((int)threadIdx.x), ug = here(u);
@@ -704,13 +733,13 @@ fft_conv_rows_kernel(const T* __restrict__ x, size_t x_sb, size_t x_st, const cp
 #pragma unroll
       for (int k = 0; k < 8; ++k) z[k] = Pair<T>::get(stage[mycol * PST + point<LOGN>(ug, k)]);
       __syncthreads();
-      fft_forward<LOGN>(col, twg, ug, z, xs);
+      fft_forward<LOGN, fine<T, TABLE_STEPS>()>(col, twg, ug, z, xs);
     }
     product16<LOGN>(sp, xs, v);
-    fft_inverse<LOGN>(col, here(tw), ug, v, e);
+    fft_inverse<LOGN, fine<T, BACK>()>(col, here(tw), ug, v, e);
     col_sync<LOGN>();
     product16<LOGN>(sp + N, xs, v);
-    fft_inverse<LOGN>(col, here(tw), ug, v, o);
+    fft_inverse<LOGN, fine<T, BACK>()>(col, here(tw), ug, v, o);
     earlier_im<LOGN>(o, prev, rec, ug);
     __syncthreads();
 #pragma unroll
@@ -795,8 +824,9 @@ __device__ __forceinline__ void conj_product16(const cpx* __restrict__ sp, const
   }
 }
 
+// (both branches in fp32 at 2048 points: 155 registers are one workgroup per compute unit, 8 x 2048 x 768 212 us; held to 128, two, 181)
 template <typename T, int LOGN, bool ODD>
-__global__ void __launch_bounds__(fft_threads<LOGN>(), ODD ? 2 : 4)
+__global__ void __launch_bounds__(fft_threads<LOGN>(), ODD && !(LOGN == 11 && sizeof(T) == 4) ? 2 : 4)
 fft_corr_kernel(const T* __restrict__ g1, const T* __restrict__ g2, const T* __restrict__ x, const cpx* __restrict__ spec,
                 T* __restrict__ gx, float* __restrict__ part, const cpx* __restrict__ tw, int Tn, int d, int lags, int vec,
                 int xcd_remap) {
@@ -881,16 +911,16 @@ fft_corr_kernel(const T* __restrict__ g1, const T* __restrict__ g2, const T* __r
   }
   put_stage(std::integral_constant<int, 1>{});
   take(z);
-  fft_forward<LOGN>(col, tw, u, z, xe);
+  fft_forward<LOGN, fine<T, DIRECT>()>(col, tw, u, z, xe);
   if (gx) conj_product16<LOGN>(sp, xe, w, false);
   if constexpr (ODD) {
     cpx xx[16];
     if (part) {
       __syncthreads();
-      fft_forward<LOGN>(col, here(tw), here(u), zx, xx);
+      fft_forward<LOGN, fine<T, DIRECT>()>(col, here(tw), here(u), zx, xx);
 #pragma unroll
       for (int k = 0; k < 16; ++k) xe[k] = cmul(xe[k], make_float2(xx[k].x, -xx[k].y));
-      fft_inverse<LOGN>(col, here(tw), here(u), xe, r8);
+      fft_inverse<LOGN, fine<T, DIRECT>()>(col, here(tw), here(u), xe, r8);
       put_part(r8, 0);
     } else {
       __syncthreads();
@@ -906,18 +936,18 @@ fft_corr_kernel(const T* __restrict__ g1, const T* __restrict__ g2, const T* __r
       }
     }
     __syncthreads();
-    fft_forward<LOGN>(col, here(tw), here(u), z, xe);
+    fft_forward<LOGN, fine<T, DIRECT>()>(col, here(tw), here(u), z, xe);
     if (gx) conj_product16<LOGN>(sp + N, xe, w, true);
     if (part) {
 #pragma unroll
       for (int k = 0; k < 16; ++k) xe[k] = cmul(xe[k], make_float2(xx[k].x, -xx[k].y));
-      fft_inverse<LOGN>(col, here(tw), here(u), xe, r8);
+      fft_inverse<LOGN, fine<T, DIRECT>()>(col, here(tw), here(u), xe, r8);
       put_part(r8, 1);
     }
   }
   if (gx) {
     if (ODD) __syncthreads();
-    fft_inverse<LOGN>(col, here(tw), here(u), w, r8);
+    fft_inverse<LOGN, fine<T, DIRECT>()>(col, here(tw), here(u), w, r8);
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < 8; ++k) stage[mycol * PST + point<LOGN>(here(u), k)] = r8[k];
@@ -941,10 +971,10 @@ fft_corr_kernel(const T* __restrict__ g1, const T* __restrict__ g2, const T* __r
     if (part) {
       cpx xx[16];
       __syncthreads();
-      fft_forward<LOGN>(col, here(tw), here(u), zx, xx);
+      fft_forward<LOGN, fine<T, DIRECT>()>(col, here(tw), here(u), zx, xx);
 #pragma unroll
       for (int k = 0; k < 16; ++k) xe[k] = cmul(xe[k], make_float2(xx[k].x, -xx[k].y));
-      fft_inverse<LOGN>(col, here(tw), here(u), xe, r8);
+      fft_inverse<LOGN, fine<T, DIRECT>()>(col, here(tw), here(u), xe, r8);
       put_part(r8, 0);
     }
   }

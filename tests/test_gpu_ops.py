@@ -1874,3 +1874,31 @@ def test_kernels_against_committed_known_answers(hip):
                 assert keep[b, t], (kw, b, t)
                 seen[b, t] = True
         assert np.array_equal(seen, keep)
+
+
+@pytest.mark.parametrize("T,d,bound,grad_bound", [(40, 64, 1.20e-7, 1.39e-7), (300, 64, 1.54e-7, 1.78e-7), (1000, 64, 1.81e-7, 2.18e-7),
+                                                  (1500, 1024, 1.95e-7, 2.31e-7), (4000, 64, 2.11e-7, 2.51e-7),
+                                                  (4000, 1024, 2.11e-7, 2.51e-7), (8000, 64, 2.16e-7, 2.54e-7), (8000, 1024, 2.16e-7, 2.54e-7)])
+def test_fp32_convolution_error_against_float64(T, d, bound, grad_bound):
+    """Relative error of the fp32 convolution and its gradients, which are sums of positions and lags through three transforms.
+    The bounds are what a radix-16 transform of the whole sequence with twiddles rounded once shows on these inputs."""
+    from flash_stu.utils.stu_utils import convolve
+    errors = []
+    for seed in range(3):
+        g = torch.Generator(device="cuda").manual_seed(seed)
+        u, w = (torch.randn(2, T, d, generator=g, device="cuda") for _ in range(2))
+        v = torch.randn(T, d, generator=g, device="cuda") * torch.arange(1, T + 1, device="cuda")[:, None] ** -0.5
+        n = 1 << (2 * T).bit_length()
+        got, want = [], []
+        for uu, vv, out in ((u, v, got), (u.double(), v.double(), want)):
+            uu, vv = uu.detach().requires_grad_(True), vv.detach().requires_grad_(True)
+            if out is got:
+                y = sum(convolve(uu, vv, n))
+            else:                       # twice the even lags
+                even = 2.0 * (torch.arange(T, device="cuda") % 2 == 0).double()[:, None]
+                y = torch.fft.irfft(torch.fft.rfft(uu, n, dim=1) * torch.fft.rfft(vv * even, n, dim=0), n, dim=1)[:, :T]
+            y.backward(w.to(y.dtype))
+            out += [y.detach(), uu.grad, vv.grad]
+        errors.append([float((a.double() - b).norm() / b.norm()) for a, b in zip(got, want)])
+    forward, inputs, filters = (sum(e) / len(e) for e in zip(*errors))
+    assert forward <= bound and inputs <= bound and filters <= grad_bound, (forward, inputs, filters)
