@@ -8,6 +8,7 @@ is missing or a tensor is not on the GPU the call raises.
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 from typing import Optional
 
@@ -298,6 +299,11 @@ def gemm_supported(x2: torch.Tensor, weight: torch.Tensor, plain: bool = False) 
             K <= x2.stride(0) < GEMM_MAX_STRIDE and x2.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0)
 
 
+@functools.lru_cache(maxsize=256)
+def _gemm_slices(M: int, N: int, K: int, nbatch: int) -> int:
+    return load().fstu_gemm_bf16_slices(M, N, K, nbatch)
+
+
 def gemm(x2: torch.Tensor, weight: torch.Tensor, up_weight: Optional[torch.Tensor] = None,
          residual: Optional[torch.Tensor] = None, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """x2 (M,K) @ weight (N,K)^T on the matrix cores (bf16).  up_weight: the gated pair
@@ -328,7 +334,7 @@ def gemm(x2: torch.Tensor, weight: torch.Tensor, up_weight: Optional[torch.Tenso
         mode, ldr = 2, residual.stride(0)
     slices, partial = 1, None
     if K >= GEMM_MIN_SLICED_K and mode != 1 and out.stride(0) % 4 == 0 and out.data_ptr() % 8 == 0:
-        slices = load().fstu_gemm_bf16_slices(M, N, K, 1)
+        slices = _gemm_slices(M, N, K, 1)
         if slices > 1:
             partial = torch.empty(slices, M, N, dtype=torch.float32, device=x2.device)
     _check(load().fstu_gemm_bf16_ws(_p(x2), x2.stride(0), _p(weight), _p(up_weight), _p(residual), ldr, _p(out), out.stride(0),
@@ -380,7 +386,7 @@ def gemm_ta(slabs: torch.Tensor, weight: torch.Tensor, residual: Optional[torch.
         if t is not None and (t.shape != (nb, M, N) or t.stride(2) != 1 or t.dtype != slabs.dtype):
             raise FlashSTUHipError(f"gemm_ta: {name} must be (nb, M, N) with contiguous rows")
     mode = 2 if residual is not None else 0
-    slices = load().fstu_gemm_bf16_slices(M, N, K, nb) if K >= GEMM_MIN_SLICED_K else 1
+    slices = _gemm_slices(M, N, K, nb) if K >= GEMM_MIN_SLICED_K else 1
     partial = torch.empty(slices, nb, M, N, dtype=torch.float32, device=slabs.device) if slices > 1 else None
     _check(load().fstu_gemm_bf16_ta_ws(_p(slabs), slabs.stride(1), slabs.stride(0) if nb > 1 else 0, _p(weight), _p(residual),
                                        residual.stride(1) if residual is not None else 0,

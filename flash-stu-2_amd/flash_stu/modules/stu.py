@@ -255,12 +255,12 @@ class STU(nn.Module):
     # ---- full-sequence evaluation
     def _project(self, x: torch.Tensor) -> torch.Tensor:
         B, T, d = x.shape
+        w, x2 = self.m_inputs_t(), x.reshape(B * T, d)
         if B * T <= _hip.MAX_DECODE_ROWS:
-            return _hip.linear_decode(x.reshape(B * T, d), self.m_inputs_t()).reshape(B, T, self.d_out)
-        x2 = x.reshape(B * T, d)
-        if _hip.gemm_supported(x2, self.m_inputs_t()):
-            return _hip.gemm(x2, self.m_inputs_t()).reshape(B, T, self.d_out)
-        return _hip.gemm_any(x2, self.m_inputs_t()).reshape(B, T, self.d_out)
+            y = _hip.linear_decode(x2, w)
+        else:
+            y = _hip.gemm(x2, w) if _hip.gemm_supported(x2, w) else _hip.gemm_any(x2, w)
+        return y.reshape(B, T, self.d_out)
 
     def _convolve(self, xp: torch.Tensor) -> torch.Tensor:
         """Approx-mode convolution of the projected inputs with phi_proj (stu.py:89-98,120): the FFT form of
