@@ -402,8 +402,9 @@ static void launch_f32_u(const LinArgs& a, int ksplit, hipStream_t s) {
   dim3 grid((a.N + NWV * NF - 1) / (NWV * NF), ksplit);
   // The head's large workgroups leave a thread 128 registers: two chunks ahead fit them up to two rows (four rows and more
   // spilled; 50257 features, K = 1024, us with two chunks / one: 4 rows 207 / 44, 8 rows 553 / 65, 16 rows 296 / 150;
-  // K = 512, 8 rows 263 / 42).
-  if constexpr (MODE != LIN_ARGMAX || RB <= 2) {
+  // K = 512, 8 rows 263 / 42).  Elsewhere 16 rows of two chunks are 128 registers of activations alone (9 to 16 rows, two
+  // chunks / one: 9216 x 768 50 / 18, as the gated pair 83 / 31, 24576 x 2048 224 / 102, pair 384 / 159, 768 x 9216 35 / 35).
+  if constexpr (MODE != LIN_ARGMAX ? RB <= 8 : RB <= 2) {
     if (a.kw > 256) {
       hipLaunchKernelGGL((linear_f32_kernel<MODE, RB, NF, 2>), grid, dim3(NWV * 64), 0, s, (const float*)a.x, (const float*)a.W, (const float*)a.W2, (float*)a.y, a.best, a.ldx, a.ldy, a.rows, a.N, a.K, a.kw, a.temperature);
       return;
@@ -481,7 +482,9 @@ extern "C" int fstu_linear_decode_splitk(const void* x, int ldx, const void* W, 
     if (mfma_ok(x, ldx, W, nullptr, K, ksplit)) launch_mfma<LIN_PARTIAL>(a, ksplit, (hipStream_t)stream);
     else launch_valu<bf16_t, LIN_PARTIAL>(a, ksplit, (hipStream_t)stream);
   } else if (dtype == FSTU_F32) {
-    if (f32_ok(a)) launch_f32<LIN_PARTIAL>(a, ksplit, (hipStream_t)stream);
+    // slices of less than 64 k leave most of a wave's lanes idle; with 9 rows and more the row walk is then the faster one (us,
+    // 8 slices, this kernel / the walk: 9 x 50257 x 256 327 / 216, 9 x 3072 x 300 22 / 15, but 9 x 9216 x 768 63 / 66)
+    if (f32_ok(a) && (rows <= 8 || K >= 64 * ksplit)) launch_f32<LIN_PARTIAL>(a, ksplit, (hipStream_t)stream);
     else launch_valu<float, LIN_PARTIAL>(a, ksplit, (hipStream_t)stream);
   } else {
     fstu_set_error("fstu_linear_decode_splitk: unknown dtype %d", dtype);
