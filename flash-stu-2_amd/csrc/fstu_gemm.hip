@@ -955,9 +955,11 @@ static int fstu_join_slices(const float* part, int ns, const void* R, long long 
 // 11.7 (18), 300 x 768 x 9216 60 / 19.3 (12), 1400 x 768 x 9216 64 / 41 (3), 2331 x 768 x 9216 65 / 47 (4), 3000 x 768 x 9216
 // 67 / 57 (3), 700 x 2048 x 24576 187 / 87 (4), 1500 x 2048 x 24576 198 / 165 (2), 300 x 2048 x 2048 22.5 / 14.8 (4); slabs 1 x
 // 1024 x 1024 x 24576 219 / 63 (8), 1 x 128 x 256 x 6144 50 / 12 (12).  Where it picks none, without / with two: 4096 x 768 x
-// 9216 70.7 / 73.3, 1000 x 2048 x 2048 23.9 / 23.4, 300 x 6144 x 2048 20.5 / 23.8, 1000 x 768 x 768 10.5 / 12.7.
+// 9216 70.7 / 73.3, 1000 x 2048 x 2048 23.9 / 23.4, 300 x 6144 x 2048 20.5 / 23.8, 1000 x 768 x 768 10.5 / 12.7.  Below K = 2048 the
+// GPU gains less than the second launch and the slices' allocation cost the host (calls of 300 x 384 x 1536 one behind the other
+// 16.0 us with three slices, 13.2 without).
 extern "C" int fstu_gemm_bf16_slices(int M, int N, int K, int nbatch) {
-  if (M <= 32 || N % 4 != 0 || K % 64 != 0) return 1;
+  if (M <= 32 || N % 4 != 0 || K % 64 != 0 || K < 2048) return 1;
   const long long cus = gemm_cus(), tiles = (long long)((M + 127) / 128) * ((N + 127) / 128) * nbatch;
   const int nkt = K / 64;
   double least = 0.41 * nkt;

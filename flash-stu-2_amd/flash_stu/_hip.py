@@ -19,7 +19,7 @@ LIB_PATH = os.path.join(os.path.dirname(_HERE), "csrc", "libflashstu_hip.so")
 
 FSTU_F32, FSTU_BF16 = 0, 1
 MAX_DECODE_ROWS = 16
-GEMM_MIN_SLICED_K = 1024      # fstu_gemm_bf16_slices takes slices of at least 512
+GEMM_MIN_SLICED_K = 2048      # where fstu_gemm_bf16_slices begins to take slices
 GEMM_MAX_STRIDE = 1 << 22     # elements between rows that the matrix-core GEMM's 32-bit offsets cover
 
 _lib = None
