@@ -254,14 +254,19 @@ def convolve(u: torch.Tensor, v: torch.Tensor, n: int, use_approx: bool = True, 
     else:
         spec = _hip.stu_fft_filter(v.contiguous(), nn_, single_branch=not return_both)
         ut = _hip.transpose(u.contiguous()).transpose(1, 2)        # time-major copy: coalesced column loads
-        if nn_ < 16384:
-            _hip.stu_conv_bank_fft(ut, spec, up, um)
-        else:
+        slabs = None
+        if nn_ == 16384:
             # A workgroup has one channel: into (T,K,d) it would store one element of a line at a time, and with two of them to
             # a compute unit more lines are open than the L2s hold.  Time-major slabs of one row, transposed instead: 24
             # filters, both branches, us, into (T,K,d) / slabs, 1 x 8000 x 1024 bf16 4118 / 1074, fp32 5453 / 1604 (one
             # workgroup to a compute unit 2651 and 4123), 1 x 8000 x 256 bf16 666 / 331, 4 x 5000 x 768 5028 / 2690.
-            slabs = torch.empty(1 + bool(return_both), K, d, T, dtype=u.dtype, device=u.device)
+            try:
+                slabs = torch.empty(1 + bool(return_both), K, d, T, dtype=u.dtype, device=u.device)
+            except torch.OutOfMemoryError:
+                pass                                               # results that leave no room for them
+        if slabs is None:
+            _hip.stu_conv_bank_fft(ut, spec, up, um)
+        else:
             views = [t[None].permute(0, 3, 1, 2) for t in slabs] + [None]
             for b in range(B):
                 _hip.stu_conv_bank_fft(ut[b:b + 1], spec, views[0], views[1])

@@ -1907,8 +1907,9 @@ def test_fp32_convolution_error_against_float64(T, d, bound, grad_bound):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("both", [False, True])
 @pytest.mark.parametrize("B,T,K,d", [(2, 4097, 3, 24), (1, 5000, 2, 17), (3, 8192, 4, 8), (1, 4096, 2, 16)])
-def test_convolve_exact_long_equals_the_bank_into_its_layout(hip, B, T, K, d, both, dtype):
-    """Lengths beyond 4096 go through time-major slabs: the bits of the kernel that writes (B,T,K,d) itself."""
+def test_convolve_exact_long_equals_the_bank_into_its_layout(hip, B, T, K, d, both, dtype, monkeypatch):
+    """Lengths beyond 4096 go through time-major slabs: the bits of the kernel that writes (B,T,K,d) itself, which runs where
+    there is no memory for them."""
     from flash_stu.utils.stu_utils import convolve
     u, v = torch.randn(B, T, d, device="cuda", dtype=dtype), torch.randn(T, K, device="cuda", dtype=dtype)
     got = convolve(u, v, 1 << (2 * T).bit_length(), use_approx=False, return_both=both)
@@ -1916,3 +1917,12 @@ def test_convolve_exact_long_equals_the_bank_into_its_layout(hip, B, T, K, d, bo
     want = [torch.empty(B, T, K, d, device="cuda", dtype=dtype) for _ in range(1 + int(both))] + [None]
     hip.stu_conv_bank_fft(u, hip.stu_fft_filter(v, n, single_branch=not both), want[0], want[1])
     assert torch.equal(got[0], want[0]) and (torch.equal(got[1], want[1]) if both else got[1] is None)
+    empty = torch.empty
+
+    def short(*shape, **kw):
+        if shape == (1 + int(both), K, d, T):
+            raise torch.OutOfMemoryError()
+        return empty(*shape, **kw)
+    monkeypatch.setattr(torch, "empty", short)
+    again = convolve(u, v, 1 << (2 * T).bit_length(), use_approx=False, return_both=both)
+    assert torch.equal(again[0], want[0]) and (torch.equal(again[1], want[1]) if both else again[1] is None)
