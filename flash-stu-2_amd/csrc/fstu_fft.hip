@@ -44,10 +44,10 @@ typedef float2 cpx;
 __device__ __forceinline__ int phys(int i) { return i + (i >> 4); }
 
 // ---------------------------------------------------------------- butterflies
-// How exact a transform is (see the note above).  FORMED: half the twiddles formed by turn32; TABLE: all from the table; TABLE_STEPS:
-// the same stage by stage, for the row pieces, whose other registers leave the scheduler no room to run stages into each
-// other (4 x 4096 x 2048 rows 314 us without, 264 with; the bank of filters 122 us without, 139 with); DIRECT: all from the table and both
-// outputs of a butterfly formed from its inputs.
+// How exact a transform is (see the note above).  FORMED: half the twiddles formed by turn32; TABLE: all from the table;
+// TABLE_STEPS: the same stage by stage, for the row pieces, whose other registers leave the scheduler no room to run stages
+// into each other (8 x 2048 x 768 72 us without, 64 with; the bank of filters of 2 x 2048 x 256 122 without, 139 with); DIRECT:
+// all from the table and both outputs of a butterfly formed from its inputs.
 enum { FORMED, TABLE, TABLE_STEPS, DIRECT };
 template <typename T, int HOW> __host__ __device__ constexpr int fine() { return sizeof(T) == 4 ? HOW : FORMED; }
 // (a, b) <- (a + w r b, a - w r b), r = 1 or (ROT) the quarter turn of the direction (-i forward, +i inverse)
