@@ -520,12 +520,10 @@ def run_ref(args, torch, _hip):
     ms = (time.perf_counter() - t0) / K * 1e3
     assert bool(torch.isfinite(y.float()).all())
     # the two launches of the operator on their own (HIP events on the launch stream)
-    # (x @ M_inputs as time-major slabs, the convolution on them, the transpose of its result)
-    ms_proj, xt = timed(lambda: stu._project_time_major(x), K)
-    yt = torch.empty_like(xt)
-    spec = stu.filter_spectrum(_hip.fft_length(L))
-    ms_conv, _ = timed(lambda: _hip.stu_conv_fft_strided(xt.transpose(1, 2), spec, yt.transpose(1, 2)), K)
-    ms_tr, _ = timed(lambda: _hip.transpose(yt), K)
+    # (x @ M_inputs, the convolution)
+    ms_proj, xp = timed(lambda: stu._project(x), K)
+    taps = stu.filter_taps(L)
+    ms_conv, _ = timed(lambda: _hip.stu_conv_mfma(xp, taps), K)
     conv_bytes = 2 * B * L * d * 2 + L * d * 2          # x_proj in, y out, the filter once
     conv_gbps = conv_bytes / (ms_conv * 1e-3) / 1e9
     flops = 2.0 * B * L * d * d
@@ -538,11 +536,10 @@ def run_ref(args, torch, _hip):
                        "batch": B, "L": L, "d": d, "K": Kf,
                        "published": {"ms_per_call": published_ms, "hardware": "NVIDIA H100 PCIe (another GPU: context, not a like-for-like bar)",
                                      "source": "tests/tilling/standard_memory_profile.txt:48-59"}},
-            "kernels_ms": {"x @ M_inputs (gemm_bf16_kernel, time-major output)": ms_proj,
-                           "spectral convolution (fft_slab_kernel on time-major slabs)": ms_conv,
-                           "result back to (L, d) (transpose16_kernel)": ms_tr,
+            "kernels_ms": {"x @ M_inputs (gemm_bf16_kernel)": ms_proj,
+                           "spectral convolution (conv_mfma_kernel)": ms_conv,
                            "projection_tflops": flops / (ms_proj * 1e-3) / 1e12},
-            "roofline": {"bound": "hbm", "kernel": "fft_slab_kernel (spectral convolution of the projected inputs, both sign branches, on time-major slabs)",
+            "roofline": {"bound": "hbm", "kernel": "conv_mfma_kernel (spectral convolution of the projected inputs, both sign branches, as a Toeplitz product)",
                          "achieved": conv_gbps, "peak": HBM_PEAK_GBPS, "unit": "GB/s", "frac": conv_gbps / HBM_PEAK_GBPS,
                          "traffic": None, "bytes_per_launch": conv_bytes, "avg_launch_us": ms_conv * 1e3}}
 

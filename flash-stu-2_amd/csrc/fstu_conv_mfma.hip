@@ -1,0 +1,325 @@
+// Spectral convolution of the STU as a Toeplitz product on the matrix cores (bf16, up to 4096 positions).
+//
+// Both operands of the convolution are bf16 (the projected inputs and phi_proj, flash_stu/modules/stu.py:88-98 of the
+// reference), so every product x[u] f[t-u] is exact in fp32 and the sums are fp32: no transform, no twiddle rounding.  The two
+// sign branches are plus = E + O and minus = E - O with E, O the sums over the even and odd lags (stu_utils.py:214-228); lags of
+// one parity connect positions of fixed parities, so with x_p[m] = x[2m+p], fe[j] = f[2j], fo[j] = f[2j+1]
+//   E_p[m] = sum_j fe[j] x_p[m-j],   O_1[m] = sum_j fo[j] x_0[m-j],   O_0[m+1] = W[m] = sum_j fo[j] x_1[m-j].
+//
+// One v_mfma_f32_16x16x32_bf16 forms 16 positions (rows i) of 16 columns, a column being a block of 64 positions of one
+// parity of one sequence: D[i][col] += sum_k A[i][k] B[k][col] with B = 32 consecutive inputs of the column's own sequence, 32 s
+// positions before the end of its block, and A[i][k] = f[16 a + i - k], a = 2s - 2 + row tile, the same for every column.  Four
+// row tiles and the two filters share a B fragment, all tiles of columns share the filter fragments, and a fragment serves the
+// row tiles of two successive steps from registers.
+// A lane's 8 filter values start at any alignment, so the filter lies in LDS eight times, shifted by one element each; a wave
+// expands 64 lags at a time into a ring of its own, from a time-major reversed copy (fstu_stu_conv_taps) read ahead.
+//
+// A workgroup has 8 channels (16 bytes of a row) of R sequences with R * NB = 8 blocks to a tile; the rows travel through LDS
+// once, transposed 8 x 8 in registers, and a wave works on a channel by itself, so there are two barriers in all.  The result
+// replaces the channel's inputs in LDS and leaves the way it came.
+//
+// us, transforms -> this: 8 x 512 x 768 16 -> 10.5, 32 x 300 x 2048 100 -> 51, 8 x 2048 x 768 61 -> 45, 1 x 4096 x 2048 56 (with a
+// transpose) -> 45.  What bounds the longest two is the matrix cores: 2.36 and 2.62 M products of 16 x 16 x 32, which this card
+// issues every 20 cycles on random operands, are 19 and 21 us; the rows' way in and out, 5 and 2 us, is not hidden behind them,
+// because all workgroups that fit start together.  Blocks of 32 positions would save a sixth of the products, but the filter
+// fragments then serve half as many each and the LDS becomes the bound (47 us).
+#include "fstu_common.h"
+#include <type_traits>
+
+namespace {
+
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef float floatx4_t __attribute__((ext_vector_type(4)));
+
+constexpr int CM_RING = 4096;        // bytes of a wave's ring: 2 filters x 16 groups of 8 lags x 8 shifts x 16 bytes
+// A 16-byte LDS read serves 16 lanes at a time, the lanes 0-3, 12-15, 20-27 of each half wave and then the others, from 64 banks.
+// The 16-byte pieces of a block of 64 positions are permuted by the block's number, the parities lie whole multiples of 256
+// bytes apart and the sequences NB blocks more, and in the ring the shifts of every other pair of groups are rotated by four:
+// 16 different slots for every read of the products.
+constexpr int cm_region(int HB) { return (128 * (1 + HB) + 255) & ~255; }      // a channel's parity, a block of zeros in front
+constexpr int cm_row(int HB, int NB) { return 16 * cm_region(HB) + (NB < 8 ? 128 * NB : 0); }
+__device__ __forceinline__ int ring_at(int n, int shift) { return (n & 15) * 128 + ((shift * 16) ^ (n & 2 ? 64 : 0)); }
+__device__ __forceinline__ int piece_at(int block, int piece) { return 128 * block + ((piece ^ (block & 6)) * 16); }   // block -1: zeros
+
+__device__ __forceinline__ bf16x8_t as_frag(uint4 v) { return __builtin_bit_cast(bf16x8_t, v); }
+
+// LDS accesses of one wave are served in order: what one lane writes another lane reads once the compiler keeps the order too.
+__device__ __forceinline__ void wave_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// The workgroup's 8 channels and first sequence.  The 8 workgroups that share the 128-byte lines of 64 channels run on one XCD
+// (consecutive workgroups are dealt to the 8 XCDs in turn), so that a line is fetched into one L2.
+__device__ __forceinline__ bool cm_place(int d, int rows, int R, int& c0, int& row0) {
+  const int nu = (d + 63) >> 6, unit = (blockIdx.x >> 6) * 8 + (blockIdx.x & 7);
+  c0 = unit % nu * 64 + ((blockIdx.x >> 3) & 7) * 8;
+  row0 = unit / nu * R;
+  return row0 < rows && c0 < d;
+}
+
+// 8 positions of one parity x 8 channels, dwords [position][channel pair] -> [channel][position pair] or back
+__device__ __forceinline__ void transpose8(const unsigned (&v)[8][4], unsigned (&o)[8][4]) {
+#pragma unroll
+  for (int c = 0; c < 8; ++c)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      o[c][j] = __builtin_amdgcn_perm(v[2 * j + 1][c >> 1], v[2 * j][c >> 1], (c & 1) ? 0x07060302 : 0x05040100);
+}
+
+// NT tiles of NB = 1 << NBS blocks to a parity, NW waves, OCC of them to a SIMD
+template <int NT, int NBS, int NW, int OCC>
+__global__ void __launch_bounds__(NW * 64, OCC)
+conv_mfma_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ taps, bf16_t* __restrict__ y, int B, int T, int d,
+                 int single) {
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  constexpr int NB = 1 << NBS, R = 8 >> NBS, HB = NB * NT;   // blocks of a tile, sequences, blocks of a parity
+  constexpr int rg = cm_region(HB), rws = cm_row(HB, NB);
+  int c0, row0;
+  if (!cm_place(d, B, R, c0, row0)) return;
+  const int tid = threadIdx.x;
+  const int pieces = R * HB * 16;                           // (sequence, 8 positions of one parity)
+  for (int v = tid; v < R * 128; v += NW * 64)               // the zeros in front of every region
+    *(uint4*)(lds + (v >> 7) * rws + ((v >> 3) & 15) * rg + (v & 7) * 16) = make_uint4(0, 0, 0, 0);
+  for (int v = tid; v < pieces; v += NW * 64) {
+    const int mu = v & (HB * 8 - 1), p = (v / (HB * 8)) & 1, row = v / (HB * 16), t0 = 16 * mu + p;
+    const bf16_t* src = x + ((size_t)(row0 + row) * T + t0) * d + c0;
+    unsigned a[8][4], o[8][4];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      uint4 q = make_uint4(0, 0, 0, 0);
+      if (t0 + 2 * e < T && row0 + row < B) q = *(const uint4*)(src + (size_t)(2 * e) * d);
+      a[e][0] = q.x; a[e][1] = q.y; a[e][2] = q.z; a[e][3] = q.w;
+    }
+    transpose8(a, o);
+    char* dst = lds + row * rws + p * rg + 128 + piece_at(mu >> 3, mu & 7);
+#pragma unroll
+    for (int c = 0; c < 8; ++c) *(uint4*)(dst + c * 2 * rg) = make_uint4(o[c][0], o[c][1], o[c][2], o[c][3]);
+  }
+  __syncthreads();
+
+  const int lane = tid & 63, wave = tid >> 6, col = lane & 15, g = lane >> 4;
+  const int par = col >> 3, cc = col & 7, row = cc >> NBS, q = cc & (NB - 1);
+  char* const ring = lds + R * rws + wave * CM_RING;
+  // expansion: 5 dwords of the reversed taps give the shifts 2a and 2a+1 of a group of 8 lags
+  const int xf = lane >> 5, xn = (lane >> 2) & 7, xa = lane & 3;
+  constexpr int cap = 64 * HB, S = cap + 16;                 // HB pairs of steps
+  char* const xdst = ring + xf * 2048 + ring_at(xn, 2 * xa);
+  const int fh = (col >> 3) - g;                             // group of the lane's first filter value
+  int fat[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) fat[k] = ring_at(fh + 2 * k, col & 7);
+
+  for (int ch = wave; ch < 8; ch += NW) {
+    const unsigned* tp = (const unsigned*)(taps + ((size_t)(c0 + ch) * 2 + xf) * S + cap - 8 * xn - 2 * xa - 2);
+    constexpr int DEPTH = HB < 2 ? 1 : NT == 4 ? 4 : 2;      // groups of 64 taps on their way
+    unsigned w[DEPTH][5], wf[5];
+    auto fetch = [&](unsigned (&r)[5], int P) {
+      const unsigned* src = tp - 32 * min(P, HB - 1);
+#pragma unroll
+      for (int k = 0; k < 5; ++k) r[k] = src[k];
+    };
+    auto expand = [&](const unsigned (&r)[5], bool odd) {
+      char* dst = xdst + odd * 1024;
+      *(uint4*)dst = make_uint4(r[1], r[2], r[3], r[4]);
+      *(uint4*)(dst + 16) = make_uint4(__builtin_amdgcn_alignbit(r[1], r[0], 16), __builtin_amdgcn_alignbit(r[2], r[1], 16),
+                                       __builtin_amdgcn_alignbit(r[3], r[2], 16), __builtin_amdgcn_alignbit(r[4], r[3], 16));
+    };
+    fetch(wf, 0);
+#pragma unroll
+    for (int k = 0; k < DEPTH; ++k) fetch(w[k], k + 1);
+    wave_order();
+    if (lane < 48) *(uint4*)(ring + (lane / 24) * 2048 + 13 * 128 + (lane % 24) * 16) = make_uint4(0, 0, 0, 0);   // lags below 0
+    expand(wf, false);
+    wave_order();
+    floatx4_t E[NT][4], O[NT][4];
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) E[j][r] = O[j][r] = (floatx4_t){0.f, 0.f, 0.f, 0.f};
+    char* const region = lds + row * rws + (ch * 2 + par) * rg + 128;
+    uint4 fa[2][2], fb[2][2];                                 // [filter][a]: fragments of the row tiles 0, 1 and 2, 3
+#pragma unroll
+    for (int k = 0; k < 2; ++k) fa[k][0] = fa[k][1] = make_uint4(0, 0, 0, 0);
+    // A pair of steps, 64 lags, for the tiles from J0 on; the next 64 lags are expanded behind the last reads of these.
+    auto pair = [&](auto first, int P, bool odd, unsigned (&r)[5]) {
+      constexpr int J0 = decltype(first)::value;
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        uint4 (&old)[2][2] = s ? fb : fa;
+        uint4 (&now)[2][2] = s ? fa : fb;
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+          const char* p = ring + (odd ? fat[2 * s + k] ^ 1024 : fat[2 * s + k]);
+          now[0][k] = *(const uint4*)p;
+          now[1][k] = *(const uint4*)(p + 2048);
+        }
+        uint4 b[NT];
+#pragma unroll
+        for (int j = J0; j < NT; ++j) b[j] = *(const uint4*)(region + piece_at(max(q + NB * j - P, -1), s ? g : g + 4));
+        if (s == 1) {
+          wave_order();
+          expand(r, !odd);
+          fetch(r, P + 1 + DEPTH);
+          wave_order();
+        }
+#pragma unroll
+        for (int j = J0; j < NT; ++j)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            E[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_frag(i < 2 ? old[0][i] : now[0][i - 2]), as_frag(b[j]), E[j][i], 0, 0, 0);
+            O[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_frag(i < 2 ? old[1][i] : now[1][i - 2]), as_frag(b[j]), O[j][i], 0, 0, 0);
+          }
+      }
+    };
+    // tile j sees the lags of its own and all earlier blocks: j + 1 phases of NB pairs
+    auto phase = [&](auto first) {
+      constexpr int J = decltype(first)::value;
+      if constexpr (J < NT) {
+#pragma unroll 1
+        for (int P = J * NB; P < (J + 1) * NB; P += DEPTH)
+#pragma unroll
+          for (int k = 0; k < DEPTH; ++k) pair(first, P + k, k & 1, w[k]);
+      }
+    };
+    phase(std::integral_constant<int, 0>{});
+    phase(std::integral_constant<int, 1>{});
+    phase(std::integral_constant<int, 2>{});
+    phase(std::integral_constant<int, 3>{});
+    wave_order();
+
+    // Branches and rounding.  A lane of an x_0 column has E_0 and O_1, of an x_1 column E_1 and W = O_0 one position early.  The other
+    // column's values cross over by a rotation within 16 lanes; W of the position before the lane's four comes from the lane 16
+    // below, of the row tile or block before it where the lane has the first four.
+    const int from = (g ? lane - 16 : lane + 48) * 4, from_block = (g ? lane - 16 : 48 + (col & 8) + (cc + 7) % 8) * 4;
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+      floatx4_t cross[4];
+      const float tile_before = j ? fstu_dpp<0x128>(O[j ? j - 1 : 0][3][3]) : 0.f;
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) cross[r][k] = fstu_dpp<0x128>(O[j][r][k]);          // row_ror:8
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        float last;                                            // what this lane hands on
+        if (r) {
+          last = g == 3 ? cross[r - 1][3] : cross[r][3];
+        } else {
+          last = g != 3 ? cross[0][3] : q == NB - 1 ? tile_before : cross[3][3];
+        }
+        int src = r ? from : from_block;
+        if (r == 0 && NB < 8 && g == 0 && q == 0) src = (48 + (col & 8) + cc + NB - 1) * 4;    // its own sequence's last block
+        const float prev = __int_as_float(__builtin_amdgcn_ds_bpermute(src, __float_as_int(last)));
+        float v[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const float o = par ? cross[r][k] : k ? cross[r][k ? k - 1 : 0] : prev;
+          const float e = E[j][r][k];
+          v[k] = single ? e + o : DT<bf16_t>::rnd(e + o) + DT<bf16_t>::rnd(e - o);
+        }
+        *(uint2*)(region + piece_at(q + NB * j, 2 * r + (g >> 1)) + (g & 1) * 8) = make_uint2(pack2_bf16(v[0], v[1]), pack2_bf16(v[2], v[3]));
+      }
+    }
+    wave_order();
+  }
+  __syncthreads();
+
+  for (int v = tid; v < pieces; v += NW * 64) {
+    const int mu = v & (HB * 8 - 1), p = (v / (HB * 8)) & 1, rw = v / (HB * 16), t0 = 16 * mu + p;
+    if (t0 >= T || row0 + rw >= B) continue;
+    const char* src = lds + rw * rws + p * rg + 128 + piece_at(mu >> 3, mu & 7);
+    unsigned a[8][4], o[8][4];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      const uint4 t = *(const uint4*)(src + c * 2 * rg);
+      a[c][0] = t.x; a[c][1] = t.y; a[c][2] = t.z; a[c][3] = t.w;
+    }
+    transpose8(a, o);
+    bf16_t* dst = y + ((size_t)(row0 + rw) * T + t0) * d + c0;
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      if (t0 + 2 * e < T) *(uint4*)(dst + (size_t)(2 * e) * d) = make_uint4(o[e][0], o[e][1], o[e][2], o[e][3]);
+  }
+}
+
+// taps[c][p][cap - j] = f[2j+p][c] for 0 <= j, zero where the filter has no such lag; 8 channels x 8 places per thread
+__global__ void __launch_bounds__(256)
+conv_taps_kernel(const bf16_t* __restrict__ f, bf16_t* __restrict__ taps, int L, int d, int cap) {
+  const int S = cap + 16, places = S >> 3, groups = d >> 3;
+  const int v = blockIdx.x * 256 + threadIdx.x;
+  if (v >= 2 * places * groups) return;
+  const int c0 = v % groups * 8, p = v / groups & 1, i0 = v / groups / 2 * 8;
+  unsigned a[8][4], o[8][4];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const int j = cap - i0 - e, s = 2 * j + p;
+    uint4 t = make_uint4(0, 0, 0, 0);
+    if (j >= 0 && s < L) t = *(const uint4*)(f + (size_t)s * d + c0);
+    a[e][0] = t.x; a[e][1] = t.y; a[e][2] = t.z; a[e][3] = t.w;
+  }
+  transpose8(a, o);
+#pragma unroll
+  for (int c = 0; c < 8; ++c)
+    *(uint4*)(taps + ((size_t)(c0 + c) * 2 + p) * S + i0) = make_uint4(o[c][0], o[c][1], o[c][2], o[c][3]);
+}
+
+// log2 of the blocks of a tile and the tiles for T positions
+void cm_shape(int T, int& nbs, int& nt) {
+  nbs = T <= 128 ? 0 : T <= 256 ? 1 : T <= 512 ? 2 : 3;
+  nt = T <= 1024 ? 1 : T <= 2048 ? 2 : 4;
+}
+
+}  // namespace
+
+extern "C" int fstu_stu_conv_taps_len(int T) {
+  if (T < 1 || T > 4096) return 0;
+  int nbs, nt;
+  cm_shape(T, nbs, nt);
+  return 64 * (nt << nbs) + 16;
+}
+
+extern "C" int fstu_stu_conv_taps(const void* filt, void* taps, int L, int d, int S, void* stream) {
+  FSTU_REQUIRE(filt && taps, FSTU_ENULL, "fstu_stu_conv_taps: null pointer");
+  FSTU_REQUIRE(L >= 1 && d >= 8 && d % 8 == 0 && d <= 1 << 20 && S >= 80 && S <= 2064 && S % 64 == 16, FSTU_ESHAPE,
+               "fstu_stu_conv_taps: L=%d d=%d S=%d (d a multiple of 8, S of fstu_stu_conv_taps_len)", L, d, S);
+  FSTU_REQUIRE(fstu_aligned(filt, 16) && fstu_aligned(taps, 16), FSTU_EALIGN, "fstu_stu_conv_taps: pointers must be 16-byte aligned");
+  const int n = 2 * (S / 8) * (d / 8);
+  hipLaunchKernelGGL(conv_taps_kernel, dim3((n + 255) / 256), dim3(256), 0, (hipStream_t)stream, (const bf16_t*)filt, (bf16_t*)taps, L, d,
+                     S - 16);
+  FSTU_CHECK_LAUNCH("fstu_stu_conv_taps");
+  return FSTU_OK;
+}
+
+extern "C" int fstu_stu_conv_mfma(const void* x, const void* taps, void* y, int B, int T, int d, int single_branch, void* stream) {
+  FSTU_REQUIRE(x && taps && y, FSTU_ENULL, "fstu_stu_conv_mfma: null pointer");
+  FSTU_REQUIRE(B >= 1 && B <= 65535 && T >= 1 && T <= 4096 && d >= 8 && d % 8 == 0 && d <= 1 << 20, FSTU_ESHAPE,
+               "fstu_stu_conv_mfma: B=%d T=%d d=%d (T up to 4096, d a multiple of 8)", B, T, d);
+  FSTU_REQUIRE(fstu_aligned(x, 16) && fstu_aligned(taps, 16) && fstu_aligned(y, 16), FSTU_EALIGN,
+               "fstu_stu_conv_mfma: pointers must be 16-byte aligned");
+  int nbs, nt;
+  cm_shape(T, nbs, nt);
+  const int R = 8 >> nbs;
+  const long long units = (long long)((d + 63) / 64) * ((B + R - 1) / R);
+  FSTU_REQUIRE(units < 1 << 24, FSTU_ESHAPE, "fstu_stu_conv_mfma: B=%d d=%d", B, d);
+  const dim3 grid((unsigned)((units + 7) / 8 * 64));
+#define CM_GO(NT, NBS, NW, OCC)                                                                                                     \
+  do {                                                                                                                              \
+    constexpr int lds__ = (8 >> NBS) * cm_row(NT << NBS, 1 << NBS) + NW * CM_RING;                                                  \
+    static const hipError_t ok =                                                                                                    \
+        hipFuncSetAttribute((const void*)conv_mfma_kernel<NT, NBS, NW, OCC>, hipFuncAttributeMaxDynamicSharedMemorySize, lds__);    \
+    FSTU_REQUIRE(ok == hipSuccess, (int)ok, "fstu_stu_conv_mfma: %d bytes of LDS refused: %s", lds__, hipGetErrorString(ok));       \
+    hipLaunchKernelGGL((conv_mfma_kernel<NT, NBS, NW, OCC>), grid, dim3(NW * 64), lds__, (hipStream_t)stream, (const bf16_t*)x,     \
+                       (const bf16_t*)taps, (bf16_t*)y, B, T, d, single_branch);                                                    \
+  } while (0)
+  if (nt == 4) CM_GO(4, 3, 8, 2);
+  else if (nt == 2) CM_GO(2, 3, 4, 3);
+  else if (nbs == 3) CM_GO(1, 3, 4, 4);
+  else if (nbs == 2) CM_GO(1, 2, 4, 4);
+  else if (nbs == 1) CM_GO(1, 1, 4, 4);
+  else CM_GO(1, 0, 4, 4);
+#undef CM_GO
+  FSTU_CHECK_LAUNCH("fstu_stu_conv_mfma");
+  return FSTU_OK;
+}

@@ -54,6 +54,9 @@ SIGNATURES = {
     "fstu_fft_length": [_i],
     "fstu_fft_twiddles": [_vp, _i, _vp],
     "fstu_stu_fft_filter": [_vp, _i64, _i64, _vp, _vp, _i, _i, _i, _i, _i, _vp],
+    "fstu_stu_conv_taps_len": [_i],
+    "fstu_stu_conv_taps": [_vp, _vp, _i, _i, _i, _vp],
+    "fstu_stu_conv_mfma": [_vp, _vp, _vp, _i, _i, _i, _i, _vp],
     "fstu_stu_conv_fft": [_vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _vp],
     "fstu_stu_conv_fft_strided": [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _vp],
     "fstu_transpose": [_vp, _vp, _i, _i, _i, _i, _vp],
@@ -713,6 +716,46 @@ def stu_conv_fft_strided(xp: torch.Tensor, spec: torch.Tensor, out: torch.Tensor
     ys = (ctypes.c_int64 * 3)(*out.stride())
     _check(load().fstu_stu_conv_fft_strided(_p(xp), xs, _p(spec), _p(out), ys, _p(fft_twiddles(n, xp.device)), B, T, d, n,
                                             int(single_branch), _dt(xp), _stream()), "fstu_stu_conv_fft_strided")
+    return out
+
+
+def stu_conv_taps_len(T: int) -> int:
+    """Places of a channel's parity in the operand of stu_conv_mfma for T positions; 0 if T is too long for it."""
+    return int(load().fstu_stu_conv_taps_len(int(T)))
+
+
+def stu_conv_mfma_takes(B: int, T: int, d: int, dtype: torch.dtype) -> bool:
+    """Whether the convolution of (B,T,d) runs as a Toeplitz product (stu_conv_mfma) or through transforms: bf16, T up to 4096.
+    us, product / best of the transforms' kernels: 8 x 100 x 768 7.1 / 7.7, 8 x 512 x 768 10.5 / 16, 32 x 300 x 2048 51 / 100,
+    1 x 2048 x 768 18 / 23, 8 x 2048 x 768 45 / 61.  Beyond 2048 positions a workgroup fills a compute unit, and its 38 us pay
+    for themselves where a round of 256 of them is filled by 70 %: 1 x 4096 x 2048 45 / 56, 2 x 4096 x 768 41 / 45, 4 x 4096 x
+    2048 167 / 204, but 1 x 4096 x 1024 36 / 32 and 3 x 4096 x 768 75 / 63.  Beyond 4096 the product's operations, which grow
+    with the square of the length, cost more than the transforms."""
+    if dtype != torch.bfloat16 or not 32 <= T <= 4096 or d % 8 != 0:
+        return False
+    groups = B * (d // 8)
+    return T <= 2048 or 10 * groups >= 7 * 256 * -(-groups // 256)
+
+
+def stu_conv_taps(filt: torch.Tensor, S: int) -> torch.Tensor:
+    """filt (L,d) bf16 -> (d,2,S): its columns time-major, even and odd lags apart, reversed, as stu_conv_mfma reads them."""
+    _dev(filt)
+    L, d = filt.shape
+    if filt.dtype != torch.bfloat16:
+        raise FlashSTUHipError("stu_conv_taps takes bfloat16 filters")
+    taps = torch.empty(d, 2, S, dtype=filt.dtype, device=filt.device)
+    _check(load().fstu_stu_conv_taps(_p(filt), _p(taps), L, d, int(S), _stream()), "fstu_stu_conv_taps")
+    return taps
+
+
+def stu_conv_mfma(xp: torch.Tensor, taps: torch.Tensor, single_branch: bool = False) -> torch.Tensor:
+    """xp (B,T,d) bf16 convolved with the filters of taps (stu_conv_taps for stu_conv_taps_len(T) places)."""
+    _dev(xp, taps)
+    B, T, d = xp.shape
+    if xp.dtype != torch.bfloat16 or taps.dtype != torch.bfloat16 or taps.shape != (d, 2, stu_conv_taps_len(T)):
+        raise FlashSTUHipError(f"stu_conv_mfma takes bfloat16 operands and taps ({d}, 2, {stu_conv_taps_len(T)}), got {tuple(taps.shape)} {taps.dtype}")
+    out = torch.empty_like(xp)
+    _check(load().fstu_stu_conv_mfma(_p(xp), _p(taps), _p(out), B, T, d, int(single_branch), _stream()), "fstu_stu_conv_mfma")
     return out
 
 

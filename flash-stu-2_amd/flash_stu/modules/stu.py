@@ -122,6 +122,14 @@ class STU(nn.Module):
             self._derived.pop("spec")
         return self._cached("spec", params, lambda: _hip.stu_fft_filter(src, n, single_branch=self.use_hankel_L))
 
+    def filter_taps(self, T: int) -> torch.Tensor:
+        """The convolution filters as the Toeplitz product reads them for T positions (approx mode, bf16).  One length is kept."""
+        S = _hip.stu_conv_taps_len(T)
+        hit = self._derived.get("taps")
+        if hit is not None and hit[1].shape[2] != S:
+            self._derived.pop("taps")
+        return self._cached("taps", (self.phi, self.M_filters), lambda: _hip.stu_conv_taps(self.effective_filter(), S))
+
     def m_inputs_eff(self) -> torch.Tensor:
         """M_inputs as the forward uses it: the parameter itself, or its block-diagonal part when tiling is on."""
         if self.tile_size >= self.d_in:
@@ -263,10 +271,12 @@ class STU(nn.Module):
         return y.reshape(B, T, self.d_out)
 
     def _convolve(self, xp: torch.Tensor) -> torch.Tensor:
-        """Approx-mode convolution of the projected inputs with phi_proj (stu.py:89-98,120): the FFT form of
-        the reference from FFT_MIN_T positions on, the time-domain kernel for shorter inputs and for lengths
-        beyond the longest in-LDS transform."""
+        """Approx-mode convolution of the projected inputs with phi_proj (stu.py:89-98,120): from FFT_MIN_T positions on the
+        Toeplitz product on the matrix cores (bf16, up to 4096 positions) or the FFT form of the reference, the time-domain
+        kernel for shorter inputs and for lengths beyond the longest in-LDS transform."""
         T = xp.shape[1]
+        if _hip.stu_conv_mfma_takes(*xp.shape, xp.dtype):
+            return _hip.stu_conv_mfma(xp, self.filter_taps(T), single_branch=self.use_hankel_L)
         n = _hip.fft_length(T) if T >= FFT_MIN_T else 0
         if n == 0:
             return _hip.stu_conv_direct(xp, self.effective_filter(), single_branch=self.use_hankel_L)
@@ -386,7 +396,8 @@ class STU(nn.Module):
                 return y, self._state_from_sequence(xp)
             if self.use_approx:
                 xt = None
-                if not use_cache and self._few_long_sequences(B, T, self.d_out, x.element_size()):
+                if (not use_cache and self._few_long_sequences(B, T, self.d_out, x.element_size())
+                        and not _hip.stu_conv_mfma_takes(B, T, self.d_out, x.dtype)):
                     xt = self._project_time_major(x)       # no transpose in front of the time-major convolution
                 if xt is not None:
                     return self._convolve_time_major(xt, _hip.fft_length(T))

@@ -276,6 +276,13 @@ int fstu_stu_conv_fft(const void* xp, const float* spec, void* y, const float* t
  * channels x batch rows), where the channel-contiguous kernel leaves compute units idle. */
 int fstu_stu_conv_fft_strided(const void* xp, const int64_t* x_strides, const float* spec, void* y, const int64_t* y_strides,
                               const float* tw, int B, int T, int d, int n, int single_branch, int dtype, void* stream);
+/* The same convolution as a Toeplitz product on the matrix cores: bf16, T up to 4096, d a multiple of 8, 16-byte aligned
+ * contiguous operands.  taps (d, 2, S) bf16, S = fstu_stu_conv_taps_len(T) (0: T is not taken), holds the columns of filt (L, d)
+ * time-major, the even and the odd lags apart, reversed and padded with zeros; fstu_stu_conv_taps writes it.
+ * y[b,t,c] = T( T(plus) + T(minus) ) (or T(plus) if single_branch), each position's bits the same whatever T and B. */
+int fstu_stu_conv_taps_len(int T);
+int fstu_stu_conv_taps(const void* filt, void* taps, int L, int d, int S, void* stream);
+int fstu_stu_conv_mfma(const void* x, const void* taps, void* y, int B, int T, int d, int single_branch, void* stream);
 /* Gradients of the convolution: g1, g2 (B,T,d) those of the plus and minus branch (branches = 2), g1 alone that of the plus
  * branch (branches = 1) or that of y = plus + minus (branches = 0), x (B,T,d) the forward input, spec (d, n) the filters'
  * spectra.  Writes gx (B,T,d) and gf (L,d), each in dtype and skipped where null; gf needs x and part, fp32 scratch of

@@ -489,6 +489,41 @@ def test_stu_conv_fft(hip, dtype, B, T, d, L):
     check(hip.stu_conv_fft(dev(xp), spec1, single_branch=True), plus, dtype, frac=0.05)
 
 
+@pytest.mark.parametrize("B,T,d,L", [(2, 1, 8, 5), (3, 33, 8, 64), (9, 127, 64, 50), (1, 128, 72, 256), (5, 129, 8, 129), (2, 257, 72, 300),
+                                     (3, 512, 136, 512), (1, 513, 64, 1024), (2, 1024, 8, 777), (2, 1025, 72, 1025), (1, 2048, 64, 2048),
+                                     (1, 2049, 520, 4096), (2, 4096, 16, 4096)])
+def test_stu_conv_toeplitz_product(hip, B, T, d, L):
+    """The convolution on the matrix cores at the edges of its tiles, against float64: the products are exact, T of them are added
+    in fp32 (T * 2^-24 of the absolute sum at most), each branch and the sum of both rounded once (2^-8 of its value).  A position's
+    bits do not depend on the length or the other rows, and what a row holds does not reach another."""
+    g = gen(T)
+    x = torch.randn(B, T, d, generator=g).bfloat16()
+    f = (torch.randn(L, d, generator=g) / math.sqrt(L)).bfloat16()
+    sgn = (-1.0) ** torch.arange(L, dtype=torch.float64)[:, None]
+
+    def conv(a, b):
+        n = 2 * max(T, L)
+        return torch.fft.irfft(torch.fft.rfft(a, n, 1) * torch.fft.rfft(b, n, 0), n, 1)[:, :T]
+    plus, minus = conv(x.double(), f.double()), conv(x.double(), f.double() * sgn)
+    slack = T * 2.0 ** -24 * conv(x.double().abs(), f.double().abs())
+    S = hip.stu_conv_taps_len(T)
+    taps = hip.stu_conv_taps(dev(f), S)
+    one, both = (hip.stu_conv_mfma(dev(x), taps, single).cpu().double() for single in (True, False))
+    assert bool(((one - plus).abs() <= 2.0 ** -8 * plus.abs() + slack).all())
+    want = plus + minus
+    assert bool(((both - want).abs() <= 2.0 ** -8 * (plus.abs() + minus.abs() + want.abs()) + 3 * slack).all())
+    t = (T + 1) // 2
+    short = hip.stu_conv_mfma(dev(x[:, :t].contiguous()), hip.stu_conv_taps(dev(f), hip.stu_conv_taps_len(t)))
+    assert torch.equal(short.cpu().double(), both[:, :t])
+    if B > 1:
+        x[0] = float("nan")
+        assert torch.equal(hip.stu_conv_mfma(dev(x), taps).cpu().double()[1:], both[1:])
+    assert hip.stu_conv_taps_len(4097) == 0
+    for bad in (lambda: hip.stu_conv_mfma(dev(x), taps[:, :, 8:].contiguous()), lambda: hip.stu_conv_mfma(dev(x.float()), taps)):
+        with pytest.raises(hip.FlashSTUHipError):
+            bad()
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("B,T,d,K", [(1, 40, 3, 2), (1, 64, 256, 24), (2, 100, 72, 7), (3, 300, 200, 24), (1, 1000, 256, 24), (40, 33, 256, 5)])
 def test_stu_conv_bank_in_slices(hip, dtype, B, T, d, K):
