@@ -173,12 +173,13 @@ conv_mfma_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ taps, 
           }
       }
     };
-    // tile j sees the lags of its own and all earlier blocks: j + 1 phases of NB pairs
+    // tile j sees the lags of its own and all earlier blocks, j + 1 phases of NB pairs, as far as there are positions
+    const int blocks = (T + 127) >> 7;
     auto phase = [&](auto first) {
       constexpr int J = decltype(first)::value;
       if constexpr (J < NT) {
 #pragma unroll 1
-        for (int P = J * NB; P < (J + 1) * NB; P += DEPTH)
+        for (int P = J * NB; P < min((J + 1) * NB, blocks); P += DEPTH)
 #pragma unroll
           for (int k = 0; k < DEPTH; ++k) pair(first, P + k, k & 1, w[k]);
       }
@@ -244,6 +245,218 @@ conv_mfma_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ taps, 
   }
 }
 
+// ---------------------------------------------------------------- gradients
+// y = plus + minus = 2 E, so only the even lags have gradients: with g the gradient of y,
+//   gx_p[m] = 2 sum_j fe[j] g_p[m+j],   gfe[j] = 2 sum_{rows, p, v} g_p[v] x_p[v-j].
+// Both are products with the same Hankel matrix of g, A[i][k] = g_p[32 s + 16 r + i + k]: for block c of 64 positions (or lags)
+// and row tile r, B[k][c] = fe[32 s + k - 64 c] gives gx_p[64 c + 16 r + i] and x_p[32 s + k - 64 c] gives gfe[64 c + 16 r + i].
+// Eight of an MFMA's 16 columns are blocks of lags and eight of positions, so both come out of one pass over g, whose shifted
+// copies a wave expands into its ring from g in LDS.  A workgroup has 8 channels, a wave each, and goes through R rows: the sums
+// of the filter's gradient stay in registers, and the next row is on its way while this one is worked on.  What it leaves are
+// its rows' fp32 sums, (chunks of rows, lags, channels), added in the order of the rows by conv_grad_finish_kernel.
+//
+// us, transforms -> this, both launches: 8 x 512 x 768 29 -> 26, 8 x 1024 x 768 51 -> 38, 2 x 2048 x 768 42 -> 26, 8 x 2048 x 768
+// 117 -> 73.  At 2048 positions LDS holds one workgroup, 8 waves: a row takes 16 us, of which the products are 6.4 (384 of them
+// to a wave), 11 with the LDS reads in front of them, and the way in and out 4 that nothing else runs beside.  Both parities
+// interleaved in a wave 10.5, a step's fragments requested a step ahead 11.
+constexpr int cg_rows(int HB) { return 128 * HB + 256; }        // bytes of a parity of g: zeros behind it
+
+template <int NT>
+__global__ void __launch_bounds__(512, NT == 1 ? 4 : 2)
+conv_grad_mfma_kernel(const bf16_t* __restrict__ gy, const bf16_t* __restrict__ x, const bf16_t* __restrict__ f, bf16_t* __restrict__ gx,
+                      float* __restrict__ part, int B, int T, int L, int d, int R) {
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  constexpr int HB = 8 * NT, cap = 64 * HB, rg = cm_region(HB), gg = cg_rows(HB), PC = HB * 16;
+  char* const xl = lds;                                       // 16 regions as in the forward
+  char* const fl = xl + 16 * rg;                              // 8 regions: the even taps
+  char* const gl = fl + 8 * rg;                               // 16 of g, in order
+  char* const rings = gl + 16 * gg;
+  int c0, row0;
+  if (!cm_place(d, B, R, c0, row0)) return;
+  const int tid = threadIdx.x, rows = min(R, B - row0);
+  for (int v = tid; v < 24 * 8; v += 512) *(uint4*)(lds + (v >> 3) * rg + (v & 7) * 16) = make_uint4(0, 0, 0, 0);
+  for (int v = tid; v < 16 * 16; v += 512) *(uint4*)(gl + (v >> 4) * gg + 128 * HB + (v & 15) * 16) = make_uint4(0, 0, 0, 0);
+  if (tid < HB * 8) {
+    unsigned a[8][4], o[8][4];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int t = 2 * (8 * tid + e);
+      uint4 v = make_uint4(0, 0, 0, 0);
+      if (t < L) v = *(const uint4*)(f + (size_t)t * d + c0);
+      a[e][0] = v.x; a[e][1] = v.y; a[e][2] = v.z; a[e][3] = v.w;
+    }
+    transpose8(a, o);
+#pragma unroll
+    for (int c = 0; c < 8; ++c)
+      *(uint4*)(fl + c * rg + 128 + piece_at(tid >> 3, tid & 7)) = make_uint4(o[c][0], o[c][1], o[c][2], o[c][3]);
+  }
+  // A thread's piece: 8 positions of one parity of x (the first PC threads) or of g
+  const int piece = tid % PC, mu = piece & (HB * 8 - 1), pp = piece / (HB * 8), t0 = 16 * mu + pp;
+  const bool has = tid < 2 * PC, is_g = tid >= PC;
+  unsigned in[8][4];
+  auto request = [&](int row) {
+    const bf16_t* src = (is_g ? gy : x) + ((size_t)row * T + t0) * d + c0;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      uint4 v = make_uint4(0, 0, 0, 0);
+      if (has && t0 + 2 * e < T) v = *(const uint4*)(src + (size_t)(2 * e) * d);
+      in[e][0] = v.x; in[e][1] = v.y; in[e][2] = v.z; in[e][3] = v.w;
+    }
+  };
+  request(row0);
+
+  const int lane = tid & 63, ch = tid >> 6, col = lane & 15, g = lane >> 4, c = col & 7;
+  char* const ring = rings + ch * 2048;
+  const int xn = lane >> 3, xs = lane & 7, odd = (xs & 1) * 16;   // expansion: one shift of a group of 8
+  const int xdst = ring_at(xn, xs);
+  const int fh = (col >> 3) + g;
+  int fat[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) fat[k] = ring_at(fh + 4 + 2 * k, col & 7);
+  const int fat0 = ring_at(fh, col & 7), fat1 = ring_at(fh + 2, col & 7);
+  const int blocks = (T + 127) >> 7;
+  floatx4_t S[NT][4];
+#pragma unroll
+  for (int j = 0; j < NT; ++j)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) S[j][r] = (floatx4_t){0.f, 0.f, 0.f, 0.f};
+
+  for (int row = 0; row < rows; ++row) {
+    if (has) {
+      unsigned o[8][4];
+      transpose8(in, o);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        char* dst = is_g ? gl + (k * 2 + pp) * gg + mu * 16 : xl + (k * 2 + pp) * rg + 128 + piece_at(mu >> 3, mu & 7);
+        *(uint4*)dst = make_uint4(o[k][0], o[k][1], o[k][2], o[k][3]);
+      }
+    }
+    __syncthreads();
+    if (row + 1 < rows) request(row0 + row + 1);
+    for (int p = 0; p < 2; ++p) {
+      char* const own = gl + (ch * 2 + p) * gg;
+      const char* const bl = (col < 8 ? xl + (ch * 2 + p) * rg : fl + ch * rg) + 128;
+      const char* const win = own + xn * 16 + (xs >> 1) * 4;
+      unsigned w[5];
+      auto window = [&](int P) {
+#pragma unroll
+        for (int k = 0; k < 5; ++k) w[k] = *(const unsigned*)(win + 128 * min(P, HB) + 4 * k);
+      };
+      auto expand = [&](bool oddp) {
+        *(uint4*)(ring + xdst + oddp * 1024) =
+            make_uint4(__builtin_amdgcn_alignbit(w[1], w[0], odd), __builtin_amdgcn_alignbit(w[2], w[1], odd),
+                       __builtin_amdgcn_alignbit(w[3], w[2], odd), __builtin_amdgcn_alignbit(w[4], w[3], odd));
+      };
+      wave_order();
+      window(0);
+      expand(false);
+      window(1);
+      expand(true);
+      window(2);
+      wave_order();
+      uint4 fa[2], fb[2];
+      fa[0] = *(const uint4*)(ring + fat0);
+      fa[1] = *(const uint4*)(ring + fat1);
+      // A pair of steps, 64 positions of g, for the tiles up to J1: fragments of row tiles 0, 1 from the step before, 2, 3 now
+      auto pair = [&](auto last, int P, bool oddp) {
+        constexpr int J1 = decltype(last)::value;
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+          uint4 (&old)[2] = s ? fb : fa;
+          uint4 (&now)[2] = s ? fa : fb;
+#pragma unroll
+          for (int k = 0; k < 2; ++k) now[k] = *(const uint4*)(ring + (oddp ? fat[2 * s + k] ^ 1024 : fat[2 * s + k]));
+          uint4 b[NT];
+#pragma unroll
+          for (int j = 0; j <= J1; ++j) b[j] = *(const uint4*)(bl + piece_at(max(P - c - 8 * j, -1), s ? g + 4 : g));
+          if (s == 1) {
+            wave_order();
+            expand(oddp);
+            window(P + 3);
+            wave_order();
+          }
+#pragma unroll
+          for (int j = 0; j <= J1; ++j)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+              S[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_frag(i < 2 ? old[i] : now[i - 2]), as_frag(b[j]), S[j][i], 0, 0, 0);
+        }
+      };
+#pragma unroll 1
+      for (int P = 0; P < min(8, blocks); P += 2) {
+        pair(std::integral_constant<int, 0>{}, P, false);
+        pair(std::integral_constant<int, 0>{}, P + 1, true);
+      }
+      if constexpr (NT == 2) {
+#pragma unroll 1
+        for (int P = 8; P < blocks; P += 2) {
+          pair(std::integral_constant<int, 1>{}, P, false);
+          pair(std::integral_constant<int, 1>{}, P + 1, true);
+        }
+      }
+      // this parity's gradient of x takes g's place; its columns start from zero again
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (col >= 8) {
+            *(uint2*)(own + ((c + 8 * j) * 64 + 16 * r + 4 * g) * 2) = make_uint2(pack2_bf16(2.f * S[j][r][0], 2.f * S[j][r][1]),
+                                                                                pack2_bf16(2.f * S[j][r][2], 2.f * S[j][r][3]));
+            S[j][r] = (floatx4_t){0.f, 0.f, 0.f, 0.f};
+          }
+    }
+    __syncthreads();
+    if (gx && tid < PC && t0 < T) {
+      unsigned a[8][4], o[8][4];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        const uint4 v = *(const uint4*)(gl + (k * 2 + pp) * gg + mu * 16);
+        a[k][0] = v.x; a[k][1] = v.y; a[k][2] = v.z; a[k][3] = v.w;
+      }
+      transpose8(a, o);
+      bf16_t* dst = gx + ((size_t)(row0 + row) * T + t0) * d + c0;
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        if (t0 + 2 * e < T) *(uint4*)(dst + (size_t)(2 * e) * d) = make_uint4(o[e][0], o[e][1], o[e][2], o[e][3]);
+    }
+    if (row + 1 < rows) __syncthreads();
+  }
+  if (!part) return;
+  // lags of a channel -> channels of a lag, through the space of x
+  float* const fl32 = (float*)xl;
+  if (col < 8) {
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) *(floatx4_t*)(fl32 + ch * (cap + 4) + (c + 8 * j) * 64 + 16 * r + 4 * g) = S[j][r];
+  }
+  __syncthreads();
+  const int lags = min(cap, (min(L, T) + 1) >> 1);
+  float* const out = part + (size_t)(row0 / R) * lags * d + c0;
+  for (int v = tid; v < lags * 2; v += 512) {
+    const float* s = fl32 + (v & 1) * 4 * (cap + 4) + (v >> 1);
+    *(float4*)(out + (size_t)(v >> 1) * d + (v & 1) * 4) = make_float4(s[0], s[cap + 4], s[2 * (cap + 4)], s[3 * (cap + 4)]);
+  }
+}
+
+// gf[2j][c] = 2 * (the chunks' sums in their order), zero at odd lags and beyond the input; 8 channels per thread
+__global__ void __launch_bounds__(256) conv_grad_finish_kernel(const float* __restrict__ part, bf16_t* __restrict__ gf, int chunks, int lags,
+                                                               int L, int d) {
+  const int groups = d >> 3, v = blockIdx.x * 256 + threadIdx.x;
+  if (v >= L * groups) return;
+  const int s = v / groups, c0 = v % groups * 8;
+  float a[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  if (!(s & 1) && (s >> 1) < lags)
+    for (int k = 0; k < chunks; ++k) {
+      const float* p = part + ((size_t)k * lags + (s >> 1)) * d + c0;
+      const float4 u = *(const float4*)p, w = *(const float4*)(p + 4);
+      a[0] += u.x; a[1] += u.y; a[2] += u.z; a[3] += u.w;
+      a[4] += w.x; a[5] += w.y; a[6] += w.z; a[7] += w.w;
+    }
+  *(uint4*)(gf + (size_t)s * d + c0) = make_uint4(pack2_bf16(2.f * a[0], 2.f * a[1]), pack2_bf16(2.f * a[2], 2.f * a[3]),
+                                                  pack2_bf16(2.f * a[4], 2.f * a[5]), pack2_bf16(2.f * a[6], 2.f * a[7]));
+}
+
 // taps[c][p][cap - j] = f[2j+p][c] for 0 <= j, zero where the filter has no such lag; 8 channels x 8 places per thread
 __global__ void __launch_bounds__(256)
 conv_taps_kernel(const bf16_t* __restrict__ f, bf16_t* __restrict__ taps, int L, int d, int cap) {
@@ -269,6 +482,19 @@ conv_taps_kernel(const bf16_t* __restrict__ f, bf16_t* __restrict__ taps, int L,
 void cm_shape(int T, int& nbs, int& nt) {
   nbs = T <= 128 ? 0 : T <= 256 ? 1 : T <= 512 ? 2 : 3;
   nt = T <= 1024 ? 1 : T <= 2048 ? 2 : 4;
+}
+
+// Rows a workgroup of the gradients goes through: as many as make its time, one part for the way in and out and one per row, times
+// the rounds of workgroups that the chip runs, the shortest.
+int cg_rows_per_group(int B, int T, int d) {
+  const long long groups = (d + 7) / 8, slots = T <= 1024 ? 512 : 256;
+  int best = 1;
+  long long least = -1;
+  for (int r = 1; r <= B && r <= 64; ++r) {
+    const long long cost = (groups * ((B + r - 1) / r) + slots - 1) / slots * (1 + r);
+    if (least < 0 || cost < least) { least = cost; best = r; }
+  }
+  return best;
 }
 
 }  // namespace
@@ -321,5 +547,42 @@ extern "C" int fstu_stu_conv_mfma(const void* x, const void* taps, void* y, int 
   else CM_GO(1, 0, 4, 4);
 #undef CM_GO
   FSTU_CHECK_LAUNCH("fstu_stu_conv_mfma");
+  return FSTU_OK;
+}
+
+extern "C" int64_t fstu_stu_conv_mfma_grad_ws(int B, int T, int d, int L) {
+  if (B < 1 || T < 1 || T > 2048 || d < 8 || L < 1) return 0;
+  const int R = cg_rows_per_group(B, T, d), lags = ((L < T ? L : T) + 1) / 2;
+  return (int64_t)((B + R - 1) / R) * lags * d;
+}
+
+extern "C" int fstu_stu_conv_mfma_grad(const void* gy, const void* x, const void* filt, void* gx, void* gf, float* part, int B, int T, int d,
+                                       int L, void* stream) {
+  FSTU_REQUIRE(gy && x && filt && (gx || gf) && (!gf || part), FSTU_ENULL, "fstu_stu_conv_mfma_grad: null pointer");
+  FSTU_REQUIRE(B >= 1 && B <= 65535 && T >= 1 && T <= 2048 && d >= 8 && d % 8 == 0 && d <= 1 << 20 && L >= 1 && (int64_t)L * d < 1ll << 31,
+               FSTU_ESHAPE, "fstu_stu_conv_mfma_grad: B=%d T=%d d=%d L=%d (T up to 2048, d a multiple of 8)", B, T, d, L);
+  FSTU_REQUIRE(fstu_aligned(gy, 16) && fstu_aligned(x, 16) && fstu_aligned(filt, 16) && fstu_aligned(gx, 16) && fstu_aligned(gf, 16) &&
+                   fstu_aligned(part, 16), FSTU_EALIGN, "fstu_stu_conv_mfma_grad: pointers must be 16-byte aligned");
+  const int R = cg_rows_per_group(B, T, d), chunks = (B + R - 1) / R, lags = ((L < T ? L : T) + 1) / 2;
+  const long long units = (long long)((d + 63) / 64) * chunks;
+  FSTU_REQUIRE(units < 1 << 24, FSTU_ESHAPE, "fstu_stu_conv_mfma_grad: B=%d d=%d", B, d);
+  const dim3 grid((unsigned)((units + 7) / 8 * 64));
+#define CG_GO(NT)                                                                                                                   \
+  do {                                                                                                                              \
+    constexpr int lds__ = 24 * cm_region(8 * NT) + 16 * cg_rows(8 * NT) + 8 * 2048;                                                 \
+    static const hipError_t ok =                                                                                                    \
+        hipFuncSetAttribute((const void*)conv_grad_mfma_kernel<NT>, hipFuncAttributeMaxDynamicSharedMemorySize, lds__);             \
+    FSTU_REQUIRE(ok == hipSuccess, (int)ok, "fstu_stu_conv_mfma_grad: %d bytes of LDS refused: %s", lds__, hipGetErrorString(ok));  \
+    hipLaunchKernelGGL((conv_grad_mfma_kernel<NT>), grid, dim3(512), lds__, (hipStream_t)stream, (const bf16_t*)gy, (const bf16_t*)x, \
+                       (const bf16_t*)filt, (bf16_t*)gx, gf ? part : nullptr, B, T, L, d, R);                                       \
+  } while (0)
+  if (T <= 1024) CG_GO(1);
+  else CG_GO(2);
+#undef CG_GO
+  FSTU_CHECK_LAUNCH("fstu_stu_conv_mfma_grad");
+  if (!gf) return FSTU_OK;
+  hipLaunchKernelGGL(conv_grad_finish_kernel, dim3((unsigned)(((long long)L * (d / 8) + 255) / 256)), dim3(256), 0, (hipStream_t)stream, part,
+                     (bf16_t*)gf, chunks, lags, L, d);
+  FSTU_CHECK_LAUNCH("fstu_stu_conv_mfma_grad");
   return FSTU_OK;
 }

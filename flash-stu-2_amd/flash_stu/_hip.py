@@ -56,6 +56,8 @@ SIGNATURES = {
     "fstu_stu_fft_filter": [_vp, _i64, _i64, _vp, _vp, _i, _i, _i, _i, _i, _vp],
     "fstu_stu_conv_taps_len": [_i],
     "fstu_stu_conv_taps": [_vp, _vp, _i, _i, _i, _vp],
+    "fstu_stu_conv_mfma_grad_ws": [_i, _i, _i, _i],
+    "fstu_stu_conv_mfma_grad": [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _vp],
     "fstu_stu_conv_mfma": [_vp, _vp, _vp, _i, _i, _i, _i, _vp],
     "fstu_stu_conv_fft": [_vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _vp],
     "fstu_stu_conv_fft_strided": [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _vp],
@@ -137,6 +139,7 @@ def load(path: Optional[str] = None):
     lib.fstu_swa_prefill_ws_elems.restype = ctypes.c_int64
     lib.fstu_lds_sequence_ws_floats.restype = ctypes.c_size_t
     lib.fstu_stu_conv_fft_grad_ws.restype = ctypes.c_int64
+    lib.fstu_stu_conv_mfma_grad_ws.restype = ctypes.c_int64
     if path is None:
         _lib = lib
     return lib
@@ -757,6 +760,31 @@ def stu_conv_mfma(xp: torch.Tensor, taps: torch.Tensor, single_branch: bool = Fa
     out = torch.empty_like(xp)
     _check(load().fstu_stu_conv_mfma(_p(xp), _p(taps), _p(out), B, T, d, int(single_branch), _stream()), "fstu_stu_conv_mfma")
     return out
+
+
+def stu_conv_mfma_grad_takes(B: int, T: int, d: int, dtype: torch.dtype) -> bool:
+    """Whether the gradients of plus + minus are formed on the matrix cores: bf16, T up to 2048.  us, there / through transforms:
+    1 x 300 x 768 12.6 / 14.8, 4 x 600 x 768 20 / 26, 8 x 1025 x 768 44 / 82, 8 x 2048 x 768 73 / 117.  Up to 256 positions a
+    workgroup's latency decides, and more than 256 of them lose: 4 x 200 x 512 12.3 / 13.9, but 8 x 200 x 768 20 / 15."""
+    return dtype == torch.bfloat16 and 32 <= T <= 2048 and d % 8 == 0 and (T > 256 or B * (d // 8) <= 256)
+
+
+def stu_conv_mfma_grad(gy: torch.Tensor, x: torch.Tensor, filt: torch.Tensor, want_x: bool = True, want_filter: bool = True):
+    """Gradients of y = plus + minus of the convolution of x (B,T,d) with filt (L,d), bf16, T up to 2048, in x and filt."""
+    _dev(gy, x, filt)
+    B, T, d = x.shape
+    if gy.shape != x.shape or filt.shape[1] != d or not gy.dtype == x.dtype == filt.dtype == torch.bfloat16:
+        raise FlashSTUHipError("stu_conv_mfma_grad takes bfloat16 operands, gy of x's shape and one filter per channel")
+    L = filt.shape[0]
+    gx = torch.empty_like(x) if want_x else None
+    gf = part = None
+    if want_filter:
+        gf = torch.empty_like(filt)
+        part = torch.empty(int(load().fstu_stu_conv_mfma_grad_ws(B, T, d, L)), dtype=torch.float32, device=x.device)
+    if want_x or want_filter:
+        _check(load().fstu_stu_conv_mfma_grad(_p(gy), _p(x), _p(filt), _p(gx), _p(gf), _p(part), B, T, d, L, _stream()),
+               "fstu_stu_conv_mfma_grad")
+    return gx, gf
 
 
 def stu_conv_fft_grad(g1: torch.Tensor, g2: Optional[torch.Tensor], x: torch.Tensor, spec: torch.Tensor, taps: int,

@@ -91,8 +91,8 @@ def _causal_conv(u: torch.Tensor, v: torch.Tensor) -> torch.Tensor:
 def _convolve_grads(ctx, u, v, spec, gp, gm, branches):
     """Gradients of the convolution in u and v, formed in fp32 whatever the input dtype (the reference differentiates
     through an fp32 FFT, stu_utils.py:226-228) and rounded once at the end.  branches 0: gp is the gradient of
-    plus + minus; 1: of plus alone; 2: gp and gm are those of plus and minus.  With the forward's spectra one launch of
-    the gradient kernel; without (the lengths of the time-domain kernel), and where the gradients are to be differentiated
+    plus + minus; 1: of plus alone; 2: gp and gm are those of plus and minus.  One launch on the matrix cores (branches 0,
+    bf16), or from the filters' spectra one launch of the transforms' gradient kernel; at the lengths of the time-domain kernel, and where the gradients are to be differentiated
     themselves (create_graph=True: the composition carries its graph), as convolutions: the minus branch
     sgn * conv(sgn * u, v) equals conv(u, v * (-1)^s), and
       d/du: correlation with the filter     = time-reversed convolution of the time-reversed gradient
@@ -101,6 +101,11 @@ def _convolve_grads(ctx, u, v, spec, gp, gm, branches):
     from .. import _hip
     want_u, want_v = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
     graph = torch.is_grad_enabled()
+    if branches == 0 and not graph and v.dtype == u.dtype == gp.dtype and _hip.stu_conv_mfma_grad_takes(*u.shape, u.dtype):
+        return _hip.stu_conv_mfma_grad(_aligned(gp), _aligned(u), _aligned(v), want_u, want_v)
+    n = _conv_length(u.shape[1])
+    if spec is None and n and not graph:
+        spec = _hip.stu_fft_filter(v.contiguous(), n)            # the forward was a Toeplitz product
     if spec is not None and not graph:
         return _hip.stu_conv_fft_grad(gp.contiguous(), gm.contiguous() if branches == 2 else None, u.contiguous(), spec,
                                       v.shape[0], branches, want_u, want_v)
@@ -165,6 +170,9 @@ class ApproxConvolveSum(torch.autograd.Function):
     @staticmethod
     def forward(ctx, u, v):
         from .. import _hip
+        if v.dtype == u.dtype and _hip.stu_conv_mfma_takes(*u.shape, u.dtype):
+            ctx.save_for_backward(u, v, None)
+            return _hip.stu_conv_mfma(_aligned(u), _hip.stu_conv_taps(_aligned(v), _hip.stu_conv_taps_len(u.shape[1])))
         n = _conv_length(u.shape[1])
         spec = _hip.stu_fft_filter(v.contiguous(), n) if n else None
         ctx.save_for_backward(u, v, spec)

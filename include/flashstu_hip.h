@@ -283,6 +283,12 @@ int fstu_stu_conv_fft_strided(const void* xp, const int64_t* x_strides, const fl
 int fstu_stu_conv_taps_len(int T);
 int fstu_stu_conv_taps(const void* filt, void* taps, int L, int d, int S, void* stream);
 int fstu_stu_conv_mfma(const void* x, const void* taps, void* y, int B, int T, int d, int single_branch, void* stream);
+/* Gradients of y = plus + minus on the matrix cores, under the conditions of fstu_stu_conv_mfma and for T up to 2048: gy, x
+ * (B,T,d) and filt (L,d) -> gx (B,T,d) and gf (L,d), each skipped where null; gf needs part, fp32 scratch of
+ * fstu_stu_conv_mfma_grad_ws elements.  Sums in fp32, one rounding at the end, the same bits every time. */
+int64_t fstu_stu_conv_mfma_grad_ws(int B, int T, int d, int L);
+int fstu_stu_conv_mfma_grad(const void* gy, const void* x, const void* filt, void* gx, void* gf, float* part, int B, int T, int d,
+                            int L, void* stream);
 /* Gradients of the convolution: g1, g2 (B,T,d) those of the plus and minus branch (branches = 2), g1 alone that of the plus
  * branch (branches = 1) or that of y = plus + minus (branches = 0), x (B,T,d) the forward input, spec (d, n) the filters'
  * spectra.  Writes gx (B,T,d) and gf (L,d), each in dtype and skipped where null; gf needs x and part, fp32 scratch of

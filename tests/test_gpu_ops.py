@@ -714,6 +714,60 @@ def test_convolution_gradient_kernel(hip, dtype, B, T, d, L, branches):
     assert none_f is None and none_x is None and torch.equal(only_x, gxd) and torch.equal(only_f, gfd)
 
 
+@pytest.mark.parametrize("B,T,d,L", [(1, 1, 8, 4), (2, 33, 8, 64), (9, 127, 64, 50), (5, 129, 8, 129), (130, 65, 24, 70), (3, 511, 136, 512),
+                                     (1, 513, 64, 1024), (2, 1000, 72, 777), (1, 1024, 8, 2048), (5, 1025, 520, 1025), (2, 2048, 64, 2048)])
+def test_convolution_gradients_on_the_matrix_cores(hip, B, T, d, L):
+    """Gradients of plus + minus at the edges of the tiles, one and several rows per workgroup, against float64 sums: exact products,
+    fp32 sums (T, for the filter B * T terms, 2^-24 of the absolute sum each at most), one rounding to bf16."""
+    g = gen(T)
+    x, gy = (torch.randn(B, T, d, generator=g).bfloat16() for _ in range(2))
+    f = (torch.randn(L, d, generator=g) / L ** 0.5).bfloat16()
+    even = (torch.arange(L) % 2 == 0).double()[:, None]
+    n = 2 * max(T, L)
+
+    def corr(p, q):                       # sum_t p[t + s] q[t] for s >= 0
+        return torch.fft.irfft(torch.fft.rfft(p, n, 1) * torch.fft.rfft(q, n, 1).conj(), n, 1)
+    xd, gd, fd = x.double(), gy.double(), f.double() * even
+    gx, ax = (2 * corr(a, b[None])[:, :T] for a, b in ((gd, fd), (gd.abs(), fd.abs())))
+    gf, af = (2 * corr(a, b)[:, :L].sum(0) * even for a, b in ((gd, xd), (gd.abs(), xd.abs())))
+    gf[T:] = 0
+    run = lambda *w: hip.stu_conv_mfma_grad(dev(gy), dev(x), dev(f), *w)
+    gxd, gfd = run()
+    for got, want, total, terms in ((gxd, gx, ax, T), (gfd, gf, af, B * T)):
+        bound = 2.0 ** -8 * want.abs() + terms * 2.0 ** -24 * total.abs() + 1e-12 * float(total.abs().max())
+        assert bool(((got.cpu().double() - want).abs() <= bound).all())
+    assert float(gfd[1::2].abs().sum()) == 0 and float(gfd[T:].abs().sum()) == 0
+    only_x, none_f = run(True, False)
+    none_x, only_f = run(False, True)
+    assert none_f is None and none_x is None and torch.equal(only_x, gxd) and torch.equal(only_f, gfd)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("B,T,d", [(2, 100, 64), (8, 200, 768), (1, 2100, 2048), (2, 300, 12), (1, 20, 64)])
+def test_sum_convolution_and_gradients_through_autograd(hip, dtype, B, T, d):
+    """y = T(T(plus) + T(minus)) and its gradients as the STU's training forward calls them, whichever kernels take the shape, with
+    operands at addresses and strides of their own."""
+    from flash_stu.utils.stu_utils import ApproxConvolveSum
+    g = gen(T + d)
+    base = dev(torch.randn(B * T * d + 4, generator=g).to(dtype))
+    u = base[4:].view(B, T, d).requires_grad_(True)
+    v = dev((torch.randn(d, T, generator=g) / T ** 0.5).to(dtype)).t().requires_grad_(True)
+    gy = dev(torch.randn(B, d, T, generator=g).to(dtype)).transpose(1, 2)
+    y = ApproxConvolveSum.apply(u, v)
+    y.backward(gy)
+    ud, vd = u.detach().double().requires_grad_(True), v.detach().double().requires_grad_(True)
+    ev = (torch.arange(T, device="cuda") % 2 == 0).double()[:, None]
+    n = 2 * T
+    conv = lambda f: torch.fft.irfft(torch.fft.rfft(ud, n, 1) * torch.fft.rfft(f, n, 0), n, 1)[:, :T]
+    want = 2 * conv(vd * ev)
+    want.backward(gy.double())
+    eps = 2.0 ** -8 if dtype == torch.bfloat16 else 1e-5
+    both = conv(vd).abs() + conv(vd * (2 * ev - 1)).abs()
+    assert bool(((y.double() - want).abs() <= eps * (both + want.abs()) + 1e-5 * float(want.detach().abs().max())).all())
+    for got, ref in ((u.grad, ud.grad), (v.grad, vd.grad)):
+        assert bool(((got.double() - ref).abs() <= eps * ref.abs() + 2e-5 * float(ref.abs().max())).all())
+
+
 @pytest.mark.parametrize("rows", [1, 2, 3, 5, 8, 9, 16])
 @pytest.mark.parametrize("N,K", [(1, 4), (7, 252), (258, 256), (130, 260), (33, 1028), (16389, 264)])
 def test_linear_fp32_rows(hip, rows, N, K):
