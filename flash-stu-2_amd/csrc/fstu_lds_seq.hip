@@ -14,32 +14,18 @@
 // Weights are given transposed (B^T (S,d_in), C^T (d_out,S)) so that every MFMA fragment is one 16-byte piece; both
 // travel through LDS so that the four waves of a workgroup share one fetch.
 #include "fstu_common.h"
+#include <type_traits>
 
 namespace {
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float floatx4_t __attribute__((ext_vector_type(4)));
-typedef __amdgpu_buffer_rsrc_t rsrc_t;
-typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
 
 #define LSQ_TB 128        // positions per block
 #define LSQ_NTMAX 16      // state tiles of 16 (S <= 256)
-#define LSQ_OOB 0xfffffff0u
 
-__device__ __forceinline__ bf16x8_t as_bf16x8(uint4 v) { return __builtin_bit_cast(bf16x8_t, v); }
-__device__ __forceinline__ rsrc_t make_rsrc(const void* p, size_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (unsigned)bytes, 0x00020000);
-}
-__device__ __forceinline__ uint4 buf_load16(rsrc_t rs, unsigned off) {
-  u32x4_t v = __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, 0);
-  return make_uint4(v.x, v.y, v.z, v.w);
-}
+template <typename V> __device__ __forceinline__ bf16x8_t as_bf16x8(V v) { return __builtin_bit_cast(bf16x8_t, v); }
 
-// NT: state tiles of 16 the instantiation holds registers for (S <= 16 NT).  Two workgroups share a compute unit (a
-// workgroup's life is a chain of short barrier-separated phases, so one alone leaves the unit idle most of the time):
-// at most 256 registers, and U without padding, 128 x S floats = 80 KB at S = 160.  Instead of a pad, the 16-byte slot
-// of element (row, mode) is XOR-ed with bits 1..3 of the row, which keeps the 16 rows of a tile access on 16 different
-// slots; the scan, one thread per mode, follows the same map.
 #define LSQ_SPIN_LIMIT (1 << 18)   // polls of one batch of published states before the wait gives up
 #define LSQ_LOOK 8                 // published states requested at a time
 
@@ -54,141 +40,154 @@ __device__ __forceinline__ uint4 swap8(uint4 v) {
 typedef unsigned uintx4_t __attribute__((ext_vector_type(4)));
 typedef uintx4_t uintx4_a8_t __attribute__((aligned(8)));
 // outputs are 8-byte aligned
-__device__ __forceinline__ void store16_past(bf16_t* p, uint4 v) { __builtin_nontemporal_store(__builtin_bit_cast(uintx4_t, v), (uintx4_a8_t*)p); }
+template <bool PAST>
+__device__ __forceinline__ void store16(bf16_t* p, uint4 v) {
+  if constexpr (PAST) __builtin_nontemporal_store(__builtin_bit_cast(uintx4_t, v), (uintx4_a8_t*)p);
+  else *(uintx4_a8_t*)p = __builtin_bit_cast(uintx4_t, v);
+}
 
-// PAST: the outputs leave in whole lines and past the L2s, where they are more than those hold (32 MB): what they would push
-// out are the weights that every workgroup fetches again, and the next kernel would not find them there.  us, through the L2s
-// from the accumulators / past them: 64 x 4096 x 1024, state 160, 407 / 389 (whole lines through the L2s 404), 51 x 3262 x 256
-// 121 / 111; 2 x 776 x 512 54.2 / 54.9, 2 x 437 x 256 39.0 / 39.5.
-
+// Two workgroups share a compute unit up to S = 160 (a workgroup's life is a chain of short barrier-separated phases, so one
+// alone leaves the unit idle most of the time): at most 256 registers, and U without padding, 128 x S floats = 80 KB at S = 160.
+// Instead of a pad, the 16-byte slot of element (row, mode) is XOR-ed with bits 1..3 of the row, which keeps the 16 rows of a
+// tile access on 16 different slots; the scan, one thread per mode, follows the same map.
+//
+// NT = S / 16 is exact and every load of the two products unconditional (rows and chunks behind the end are clamped to the last
+// ones, whose results nobody reads): with the number of tiles in a register and loads under conditions the loops were made of
+// branches, each fragment read was waited for by itself and every chunk for all loads in flight.  us, so / now: 64 rows x 4096 x
+// 1024, state 160, 389 / 331 (state 128 355 / 301), 51 x 3262 x 256, 96, 91 / 71, 8 x 2048 x 512, 128, 53 / 38, 1 x 4096 x 1024,
+// 160, 87 / 55, 64 x 300 x 1024, 160, 88 / 55.  (x, BmT and CmT carry no __restrict__: loads of memory that nothing may change are
+// moved behind the barriers to where their values are used.)
+// What bounds the first: its 1.07 GB.  Without the stores of y it takes 246, without the trips of x to HBM 295, without either
+// 208, with the weights from the compute unit's own cache besides 162.  No gain: x past the caches (360: a line comes in two
+// halves), the blocks of a row side by side (351), the two lines of 128 features of a row stored together (337), another first
+// group of features for every row (340), the scans left out (322).
+//
+// PAST: the outputs leave past the L2s, where they are more than those hold (32 MB): what they would push out are the weights
+// that every workgroup fetches again, and the next kernel would not find them there.
 template <int NT, bool PAST>
 __global__ void __launch_bounds__(256, NT <= 10 ? 2 : 1)   // beyond S = 160 one workgroup fills the LDS anyway
-lds_seq_kernel(const bf16_t* __restrict__ x, const float* __restrict__ A, const bf16_t* __restrict__ BmT,
-               const bf16_t* __restrict__ CmT, bf16_t* __restrict__ y, const float* __restrict__ h0,
+lds_seq_kernel(const bf16_t* x, const float* __restrict__ A, const bf16_t* BmT, const bf16_t* CmT, bf16_t* y, const float* __restrict__ h0,
                float* __restrict__ hnew, unsigned long long* __restrict__ etag, unsigned* __restrict__ status, unsigned tag,
-               int T, int Bt, int d_in, int S, int d_out) {
+               int T, int Bt, int d_in, int d_out, int nblk) {
+  constexpr int S = 16 * NT;
   extern __shared__ __align__(16) float Us[];       // LSQ_TB x S
-  const int ldu = S;
   auto uslot = [](int row, int slot) { return slot ^ ((row >> 1) & 7); };   // 16-byte slot of a row (S/4 slots, a multiple of 8)
-  const int blk = blockIdx.x, b = blockIdx.y;
+  // rows of the batch first: the blocks in front of a workgroup's are then long through when it asks for their states
+  const int blk = (int)(blockIdx.z * gridDim.y + blockIdx.y), b = blockIdx.x;
+  if (blk >= nblk) return;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, r = lane & 15, g = lane >> 4;
   const int t0 = blk * LSQ_TB;
   const int nvalid = min(LSQ_TB, T - t0);
-  const int nt = S >> 4;
+  constexpr int WPT = NT / 2;                       // 16-byte pieces of a chunk of weights per thread
   // ---- U = X_blk B: wave w owns positions 32w .. 32w+31 (two tiles of 16).  The four waves need the same weight
   // fragments: B^T travels through LDS in chunks of 64 k (S rows of 128 bytes, 16-byte pieces XOR-ed with bits of the
   // row so that the 16 rows of a fragment read fall into 16 different slots), double-buffered in the space that U
-  // takes afterwards, so a workgroup fetches every weight once instead of once per wave (a compute unit's
-  // vector-memory path, not HBM or the matrix cores, is what this kernel runs against).
+  // takes afterwards, so a workgroup fetches every weight once instead of once per wave.
+  // Both are requested three chunks ahead, x into three sets of registers and the weights into two: one chunk's products
+  // are shorter than a trip to memory.
   {
     unsigned char* wst = (unsigned char*)Us;                 // two stages of S * 128 bytes
-    const unsigned wstage = (unsigned)S * 128u;
-    const int npiece = S * 8;                                // 16-byte pieces per chunk
-    constexpr int WPT = (NT * 16 * 8 + 255) / 256;    // pieces per thread at the largest S
+    constexpr unsigned wstage = S * 128u;
     floatx4_t acc[2][NT];
 #pragma unroll
     for (int m = 0; m < 2; ++m)
 #pragma unroll
       for (int n = 0; n < NT; ++n) acc[m][n] = floatx4_t{0.f, 0.f, 0.f, 0.f};
     const bf16_t* xr[2];
-    bool xok[2];
 #pragma unroll
-    for (int m = 0; m < 2; ++m) {
-      const int t = t0 + 32 * w + 16 * m + r;
-      xok[m] = t < T;
-      xr[m] = x + ((size_t)(xok[m] ? t : 0) * Bt + b) * d_in + g * 8;
-    }
-    auto wload = [&](int k0, uint4 (&v)[WPT]) {
+    for (int m = 0; m < 2; ++m) xr[m] = x + ((size_t)min(t0 + 32 * w + 16 * m + r, T - 1) * Bt + b) * d_in + g * 8;
+    const int swz = (r >> 1) & 7;                            // rows 16n + r and 32i + row share these bits
+    const unsigned char* const wrd[2] = {wst + r * 128 + ((g ^ swz) << 4), wst + r * 128 + (((g + 4) ^ swz) << 4)};
+    auto multiply = [&](int kk, unsigned stage, const uintx4_t (&xs)[2]) __attribute__((always_inline)) {
 #pragma unroll
-      for (int i = 0; i < WPT; ++i) {
-        const int q = tid + i * 256, row = q >> 3, c = q & 7;
-        v[i] = (q < npiece && k0 + c * 8 < d_in) ? *(const uint4*)(BmT + (size_t)row * d_in + k0 + c * 8) : make_uint4(0, 0, 0, 0);
+      for (int n = 0; n < NT; ++n) {
+        const bf16x8_t wa = as_bf16x8(*(const uint4*)(wrd[kk] + stage + n * 2048));
+        acc[0][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa, as_bf16x8(xs[0]), acc[0][n], 0, 0, 0);
+        acc[1][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa, as_bf16x8(xs[1]), acc[1][n], 0, 0, 0);
       }
     };
-    auto wstore = [&](int stage, const uint4 (&v)[WPT]) {
+    const int nk = d_in >> 6;                                // whole chunks; 32 k may be left
+    if (nk) {
+      const bf16_t* const wsrc = BmT + (size_t)(tid >> 3) * d_in + (tid & 7) * 8;       // piece i: 32 i rows further
+      unsigned char* const wdst = wst + (tid >> 3) * 128 + (((tid & 7) ^ ((tid >> 4) & 7)) << 4);
+      auto wload = [&](int c, uintx4_t (&v)[WPT]) {
+        const bf16_t* src = wsrc + 64 * min(c, nk - 1);
 #pragma unroll
-      for (int i = 0; i < WPT; ++i) {
-        const int q = tid + i * 256, row = q >> 3, c = q & 7;
-        if (q < npiece) *(uint4*)(wst + stage * wstage + row * 128 + ((c ^ ((row >> 1) & 7)) << 4)) = v[i];
+        for (int i = 0; i < WPT; ++i) v[i] = *(const uintx4_t*)(src + (size_t)(32 * i) * d_in);
+      };
+      auto wstore = [&](unsigned stage, const uintx4_t (&v)[WPT]) {
+#pragma unroll
+        for (int i = 0; i < WPT; ++i) *(uintx4_t*)(wdst + stage + i * 4096) = v[i];
+      };
+      auto xload = [&](int c, uintx4_t (&v)[2][2]) {            // the two k steps of a chunk, both position tiles
+        const int k0 = 64 * min(c, nk - 1);
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+          for (int m = 0; m < 2; ++m) v[kk][m] = *(const uintx4_t*)(xr[m] + k0 + 32 * kk);
+      };
+      uintx4_t wa[WPT], wb[WPT], xa[2][2], xb[2][2], xc[2][2];
+      wload(0, wa);
+      xload(0, xa);
+      wload(1, wb);
+      xload(1, xb);
+      wstore(0, wa);
+      wload(2, wa);
+      xload(2, xc);
+      __syncthreads();
+      int c = 0;
+      unsigned stage = 0;
+      auto pass = [&](uintx4_t (&xs)[2][2], uintx4_t (&wn)[WPT]) __attribute__((always_inline)) { // chunk c; wn: the weights of chunk c + 1
+        multiply(0, stage, xs[0]);
+        multiply(1, stage, xs[1]);
+        stage = wstage - stage;
+        wstore(stage, wn);
+        wload(c + 3, wn);
+        xload(c + 3, xs);
+        __syncthreads();
+        return ++c < nk;
+      };
+      while (pass(xa, wb) && pass(xb, wa) && pass(xc, wb) && pass(xa, wa) && pass(xb, wb) && pass(xc, wa)) {
       }
-    };
-    auto xload = [&](int k0, uint4 (&v)[2][2]) {             // the two k steps of a chunk, both position tiles
-#pragma unroll
-      for (int kk = 0; kk < 2; ++kk)
-#pragma unroll
-        for (int m = 0; m < 2; ++m)
-          v[kk][m] = (xok[m] && k0 + 32 * kk < d_in) ? *(const uint4*)(xr[m] + k0 + 32 * kk) : make_uint4(0, 0, 0, 0);
-    };
-    // chunks are requested two iterations before the iteration that moves them to LDS (one iteration of MFMAs is
-    // shorter than a trip to memory): wv0 / wv1 and xb / xc hold the next two chunks
-    uint4 wv0[WPT], wv1[WPT], xa[2][2], xb[2][2], xc[2][2];
-    wload(0, wv0);
-    xload(0, xa);
-    wload(64, wv1);
-    xload(64, xb);
-    wstore(0, wv0);
-    wload(128, wv0);
-    xload(128, xc);
-    __syncthreads();
-    // one pass: multiply chunk k0 from stage `cur`, move chunk k0+64 (registers NXT) to the other stage, request
-    // chunk k0+192 into those registers
-#define LSQ_PASS(NXT)                                                                                         \
-    {                                                                                                         \
-      const unsigned char* ws = wst + cur * wstage;                                                           \
-      _Pragma("unroll") for (int kk = 0; kk < 2; ++kk) {                                                      \
-        _Pragma("unroll") for (int n = 0; n < NT; ++n) {                                                      \
-          if (n < nt) {                                                                                       \
-            const int row = 16 * n + r, c = kk * 4 + g;                                                       \
-            const uint4 wa = *(const uint4*)(ws + row * 128 + ((c ^ ((row >> 1) & 7)) << 4));                 \
-            acc[0][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(wa), as_bf16x8(xa[kk][0]), acc[0][n], 0, 0, 0); \
-            acc[1][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(wa), as_bf16x8(xa[kk][1]), acc[1][n], 0, 0, 0); \
-          }                                                                                                   \
-        }                                                                                                     \
-      }                                                                                                       \
-      if (k0 + 64 < d_in) wstore(cur ^ 1, NXT);                                                               \
-      wload(k0 + 192, NXT);                                                                                   \
-      _Pragma("unroll") for (int kk = 0; kk < 2; ++kk)                                                        \
-        _Pragma("unroll") for (int m = 0; m < 2; ++m) { xa[kk][m] = xb[kk][m]; xb[kk][m] = xc[kk][m]; }       \
-      xload(k0 + 192, xc);                                                                                    \
-      __syncthreads();                                                                                        \
-      cur ^= 1;                                                                                               \
-      k0 += 64;                                                                                               \
     }
-    int cur = 0, k0 = 0;
-    while (k0 < d_in) {
-      LSQ_PASS(wv1)
-      if (k0 < d_in) LSQ_PASS(wv0)
+    if (d_in & 32) {
+      uintx4_t xs[2];
+#pragma unroll
+      for (int m = 0; m < 2; ++m) xs[m] = *(const uintx4_t*)(xr[m] + 64 * nk);
+      for (int q = tid; q < S * 4; q += 256)
+        *(uint4*)(wst + (q >> 2) * 128 + (((q & 3) ^ ((q >> 3) & 7)) << 4)) = *(const uint4*)(BmT + (size_t)(q >> 2) * d_in + 64 * nk + (q & 3) * 8);
+      __syncthreads();
+      multiply(0, 0, xs);
+      __syncthreads();
     }
-#undef LSQ_PASS
-    // (the last barrier of the loop: every wave is through with the weight stages, U may overwrite them)
+    // (behind the last barrier every wave is through with the weight stages, U may overwrite them)
     // D layout: lane (r, g) holds modes 16n + 4g + i of position r of the tile
 #pragma unroll
     for (int m = 0; m < 2; ++m)
 #pragma unroll
       for (int n = 0; n < NT; ++n)
-        if (n < nt)
-          *(float4*)(Us + (size_t)(32 * w + 16 * m + r) * ldu + 4 * uslot(32 * w + 16 * m + r, 4 * n + g)) = make_float4(acc[m][n][0], acc[m][n][1], acc[m][n][2], acc[m][n][3]);
+        *(float4*)(Us + (32 * w + 16 * m + r) * S + 4 * uslot(32 * w + 16 * m + r, 4 * n + g)) = make_float4(acc[m][n][0], acc[m][n][1], acc[m][n][2], acc[m][n][3]);
   }
   __syncthreads();
   // ---- scan over the block's positions: thread = mode
   if (tid < S) {
     const float a = A[tid];
-    // element (p, tid) sits at p * ldu + 4 * uslot(p, tid / 4) + tid % 4
-    auto at = [&](int p_) { return Us + (size_t)p_ * ldu + 4 * uslot(p_, tid >> 2) + (tid & 3); };
+    // element (p, tid) sits at p * S + 4 * uslot(p, tid / 4) + tid % 4
+    auto at = [&](int p_) { return Us + p_ * S + 4 * uslot(p_, tid >> 2) + (tid & 3); };
     // 1: the block's end state from zero, published as (tag, value)
     float e = 0.f;
     {
       int p = 0;
-      for (; p + 8 <= nvalid; p += 8) {
-        float u[8];
+      for (; p + 16 <= nvalid; p += 16) {
+        float u[16];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) u[i] = *at(p + i);
+        for (int i = 0; i < 16; ++i) u[i] = *at(p + i);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) e = fmaf(a, e, u[i]);
+        for (int i = 0; i < 16; ++i) e = fmaf(a, e, u[i]);
       }
       for (; p < nvalid; ++p) e = fmaf(a, e, *at(p));
     }
-    const size_t rowbase = (size_t)b * gridDim.x * S;
+    const size_t rowbase = (size_t)b * nblk * S;
     __hip_atomic_store(etag + rowbase + (size_t)blk * S + tid, ((unsigned long long)tag << 32) | __float_as_uint(e),
                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     // 2: the state that enters this block (every block in front of it is a full one)
@@ -217,18 +216,18 @@ lds_seq_kernel(const bf16_t* __restrict__ x, const float* __restrict__ A, const 
         if (j0 + i < blk) h = fmaf(ap_full, h, __uint_as_float((unsigned)wv[i]));
     }
     if (timed_out) atomicOr(status, 1u);
-    if (blk == (int)gridDim.x - 1) {
+    if (blk == nblk - 1) {
       const float ap = nvalid == LSQ_TB ? ap_full : (float)pow(ad, (double)nvalid);
       hnew[(size_t)b * S + tid] = fmaf(ap, h, e);
     }
     // 3: the true states of the block's positions
     int p = 0;
-    for (; p + 8 <= nvalid; p += 8) {
-      float u[8];
+    for (; p + 16 <= nvalid; p += 16) {
+      float u[16];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) u[i] = *at(p + i);
+      for (int i = 0; i < 16; ++i) u[i] = *at(p + i);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
+      for (int i = 0; i < 16; ++i) {
         h = fmaf(a, h, u[i]);
         *at(p + i) = h;
       }
@@ -241,138 +240,109 @@ lds_seq_kernel(const bf16_t* __restrict__ x, const float* __restrict__ A, const 
   __syncthreads();
   // ---- Y = H C: wave w, positions 32w .. 32w+31; H as bf16 head + remainder
   {
-    constexpr int KS = (NT + 1) / 2;   // k steps of 32 modes this instantiation holds registers for
-    const int ks2 = S >> 5;            // k steps of 32 modes (<= KS)
+    constexpr int KS = NT / 2;         // k steps of 32 modes
     uint4 hb[2][KS], lb[2][KS];
 #pragma unroll
     for (int m = 0; m < 2; ++m) {
       const int hrow = 32 * w + 16 * m + r;
-      const float* hr = Us + (size_t)hrow * ldu;
+      const float* hr = Us + hrow * S;
 #pragma unroll
       for (int k = 0; k < KS; ++k) {
-        if (k < ks2) {
-          const float4 v0 = *(const float4*)(hr + 4 * uslot(hrow, 8 * k + 2 * g)), v1 = *(const float4*)(hr + 4 * uslot(hrow, 8 * k + 2 * g + 1));
-          const float v[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
-          unsigned hi[4], lo[4];
+        const float4 v0 = *(const float4*)(hr + 4 * uslot(hrow, 8 * k + 2 * g)), v1 = *(const float4*)(hr + 4 * uslot(hrow, 8 * k + 2 * g + 1));
+        const float v[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
+        unsigned hi[4], lo[4];
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            hi[i] = pack2_bf16(v[2 * i], v[2 * i + 1]);
-            lo[i] = pack2_bf16(v[2 * i] - __uint_as_float(hi[i] << 16), v[2 * i + 1] - __uint_as_float(hi[i] & 0xffff0000u));
-          }
-          hb[m][k] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
-          lb[m][k] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+        for (int i = 0; i < 4; ++i) {
+          hi[i] = pack2_bf16(v[2 * i], v[2 * i + 1]);
+          lo[i] = pack2_bf16(v[2 * i] - __uint_as_float(hi[i] << 16), v[2 * i + 1] - __uint_as_float(hi[i] & 0xffff0000u));
         }
+        hb[m][k] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
+        lb[m][k] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
       }
     }
-    // PAST: a lane stores 16 bytes, the eight lanes of a line next to each other in one instruction (straight from the
-    // accumulators an instruction covers 32 bytes of 16 rows): the rows of the
-    // two tiles of 32 features are dealt so that lane (r, g) ends up with features 8g .. 8g+7 of position r, and lanes r and
-    // r ^ 8 swap pieces, so that lanes r and r ^ 8 hold the two halves of a line of 64 features.
+    // A lane stores 16 bytes, the eight lanes of a line next to each other in one instruction (straight from the
+    // accumulators an instruction covers 32 bytes of 16 rows): the rows of the two tiles of 32 features are dealt so
+    // that lane (r, g) ends up with features 8g .. 8g+7 of position r, and lanes r and r ^ 8 swap pieces, so that
+    // they hold the two halves of a line of 64 features.
     const int trow = t0 + 32 * w + (r & 7), fcol = 32 * (r >> 3) + 8 * g;
     bf16_t* yr[4];                                           // position trow + 8 q
 #pragma unroll
     for (int q = 0; q < 4; ++q) yr[q] = y + ((size_t)min(trow + 8 * q, T - 1) * Bt + b) * d_out + fcol;
-    const int tA = t0 + 32 * w + r, tB = tA + 16;
-    bf16_t* yA = y + ((size_t)min(tA, T - 1) * Bt + b) * d_out + 4 * g;
-    bf16_t* yB = y + ((size_t)min(tB, T - 1) * Bt + b) * d_out + 4 * g;
-    const int nto = d_out >> 4;
     // C^T travels through LDS like B^T above, 64 output features (4 tiles) at a time, double-buffered in the space of
     // U now that every wave holds its H fragments in registers.  Rows are S * 2 + 16 bytes: an odd number of 16-byte
-    // slots, so the 16 rows of a fragment read fall into 16 different slots.  With PAST feature 32p + 8g + 4h + i lies
-    // in row 32p + 16h + 4g + i.
+    // slots, so the 16 rows of a fragment read fall into 16 different slots.  Feature 32p + 8g + 4h + i lies in row
+    // 32p + 16h + 4g + i.
     __syncthreads();
     unsigned char* cst = (unsigned char*)Us;
-    const unsigned RS = (unsigned)S * 2u + 16u, cstage = 64u * RS;
-    const int ppr = S >> 3, npc = 64 * ppr;                  // 16-byte pieces per row and per stage
-    constexpr int CPT = (64 * (NT * 16 / 8) + 255) / 256;
-    auto cload = [&](int o0, uint4 (&v)[CPT]) {
+    constexpr unsigned RS = S * 2u + 16u, cstage = 64u * RS;
+    constexpr int PPR = S / 8;                               // 16-byte pieces per row; a stage's lie in memory one after the other
+    const int npiece = d_out * PPR;
+    unsigned cdst[WPT];
 #pragma unroll
-      for (int i = 0; i < CPT; ++i) {
-        const int q = tid + i * 256, row = q / ppr, c = q - row * ppr;
-        v[i] = (q < npc && o0 + row < d_out) ? *(const uint4*)(CmT + (size_t)(o0 + row) * S + c * 8) : make_uint4(0, 0, 0, 0);
-      }
-    };
-    auto cstore = [&](int stage, const uint4 (&v)[CPT]) {
+    for (int i = 0; i < WPT; ++i) {
+      const int q = tid + i * 256, row = q / PPR, c = q - row * PPR;
+      cdst[i] = (unsigned)((row & 0x23) | ((row & 0x18) >> 1) | ((row & 4) << 2)) * RS + c * 16;
+    }
+    auto cload = [&](int o0, uintx4_t (&v)[WPT]) {
 #pragma unroll
-      for (int i = 0; i < CPT; ++i) {
-        const int q = tid + i * 256, row = q / ppr, c = q - row * ppr;
-        const int at = !PAST ? row : (row & 0x23) | ((row & 0x18) >> 1) | ((row & 4) << 2);
-        if (q < npc) *(uint4*)(cst + stage * cstage + at * RS + c * 16) = v[i];
-      }
+      for (int i = 0; i < WPT; ++i) v[i] = *(const uintx4_t*)(CmT + 8 * (size_t)min(o0 * PPR + tid + i * 256, npiece - 1));
     };
-    uint4 cv0[CPT], cv1[CPT];     // the next two groups of output features
-    cload(0, cv0);
-    cload(64, cv1);
-    cstore(0, cv0);
-    cload(128, cv0);
+    auto cstore = [&](unsigned stage, const uintx4_t (&v)[WPT]) {
+#pragma unroll
+      for (int i = 0; i < WPT; ++i) *(uintx4_t*)(cst + stage + cdst[i]) = v[i];
+    };
+    const unsigned char* const crd = cst + r * RS + g * 16;
+    uintx4_t ca[WPT], cb[WPT];                                  // the next groups of output features
+    cload(0, ca);
+    cload(64, cb);
+    cstore(0, ca);
+    cload(128, ca);
     __syncthreads();
-#define LSQ_OUT(NXT)                                                                                          \
-    {                                                                                                         \
-      const unsigned char* cs = cst + cur * cstage;                                                           \
-      if constexpr (!PAST) {                                                                                  \
-      _Pragma("unroll") for (int j = 0; j < 4; ++j) {                                                         \
-        const int ot = (o0 >> 4) + j;                                                                         \
-        if (ot < nto) {                                                                                       \
-          floatx4_t a0 = {0.f, 0.f, 0.f, 0.f}, a1 = {0.f, 0.f, 0.f, 0.f};                                     \
-          _Pragma("unroll") for (int k = 0; k < KS; ++k) {                                                    \
-            if (k < ks2) {                                                                                    \
-              const uint4 wc = *(const uint4*)(cs + (16 * j + r) * RS + (32 * k + 8 * g) * 2);                \
-              a0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(wc), as_bf16x8(hb[0][k]), a0, 0, 0, 0);  \
-              a0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(wc), as_bf16x8(lb[0][k]), a0, 0, 0, 0);  \
-              a1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(wc), as_bf16x8(hb[1][k]), a1, 0, 0, 0);  \
-              a1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(wc), as_bf16x8(lb[1][k]), a1, 0, 0, 0);  \
-            }                                                                                                 \
-          }                                                                                                   \
-          if (tA < T) *(uint2*)(yA + ot * 16) = make_uint2(pack2_bf16(a0[0], a0[1]), pack2_bf16(a0[2], a0[3])); \
-          if (tB < T) *(uint2*)(yB + ot * 16) = make_uint2(pack2_bf16(a1[0], a1[1]), pack2_bf16(a1[2], a1[3])); \
-        }                                                                                                     \
-      }                                                                                                       \
-      } else {                                                                                                \
-      uint4 pc[2][2];                                                                                         \
-      _Pragma("unroll") for (int p = 0; p < 2; ++p) {                                                         \
-        if (o0 + 32 * p < d_out) {                                                                            \
-          floatx4_t acc[2][2];                                                                                \
-          _Pragma("unroll") for (int h = 0; h < 2; ++h) {                                                     \
-            floatx4_t a0 = {0.f, 0.f, 0.f, 0.f}, a1 = {0.f, 0.f, 0.f, 0.f};                                   \
-            _Pragma("unroll") for (int k = 0; k < KS; ++k) {                                                  \
-              if (k < ks2) {                                                                                  \
-                const uint4 wc = *(const uint4*)(cs + (32 * p + 16 * h + r) * RS + (32 * k + 8 * g) * 2);     \
-                a0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(wc), as_bf16x8(hb[0][k]), a0, 0, 0, 0);\
-                a0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(wc), as_bf16x8(lb[0][k]), a0, 0, 0, 0);\
-                a1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(wc), as_bf16x8(hb[1][k]), a1, 0, 0, 0);\
-                a1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(wc), as_bf16x8(lb[1][k]), a1, 0, 0, 0);\
-              }                                                                                               \
-            }                                                                                                 \
-            acc[0][h] = a0;                                                                                   \
-            acc[1][h] = a1;                                                                                   \
-          }                                                                                                   \
-          _Pragma("unroll") for (int m = 0; m < 2; ++m)                                                       \
-            pc[m][p] = make_uint4(pack2_bf16(acc[m][0][0], acc[m][0][1]), pack2_bf16(acc[m][0][2], acc[m][0][3]),\
-                                  pack2_bf16(acc[m][1][0], acc[m][1][1]), pack2_bf16(acc[m][1][2], acc[m][1][3]));\
-        } else {                                                                                              \
-          pc[0][p] = pc[1][p] = make_uint4(0, 0, 0, 0);                                                       \
-        }                                                                                                     \
-      }                                                                                                       \
-      _Pragma("unroll") for (int m = 0; m < 2; ++m) {                                                         \
-        const uint4 other = swap8(r < 8 ? pc[m][1] : pc[m][0]);                                               \
-        if (o0 + fcol < d_out) {                                                                              \
-          if (trow + 16 * m < T) store16_past(yr[2 * m] + o0, r < 8 ? pc[m][0] : other);                     \
-          if (trow + 16 * m + 8 < T) store16_past(yr[2 * m + 1] + o0, r < 8 ? other : pc[m][1]);             \
-        }                                                                                                     \
-      }                                                                                                       \
-      }                                                                                                       \
-      if (o0 + 64 < d_out) cstore(cur ^ 1, NXT);                                                              \
-      cload(o0 + 192, NXT);                                                                                   \
-      __syncthreads();                                                                                        \
-      cur ^= 1;                                                                                               \
-      o0 += 64;                                                                                               \
-    }
-    int cur = 0, o0 = 0;
-    while (o0 < d_out) {
-      LSQ_OUT(cv1)
-      if (o0 < d_out) LSQ_OUT(cv0)
-    }
-#undef LSQ_OUT
+    auto outputs = [&](auto whole) __attribute__((always_inline)) {                         // whole: no position and no feature is behind the end
+      int o0 = 0;
+      unsigned stage = 0;
+      auto pass = [&](uintx4_t (&cn)[WPT]) __attribute__((always_inline)) {
+        uint4 pc[2][2];
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+          floatx4_t acc[2][2];
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            floatx4_t a0 = {0.f, 0.f, 0.f, 0.f}, a1 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int k = 0; k < KS; ++k) {
+              const bf16x8_t wc = as_bf16x8(*(const uint4*)(crd + stage + (32 * p + 16 * h) * RS + 64 * k));
+              a0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wc, as_bf16x8(hb[0][k]), a0, 0, 0, 0);
+              a1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wc, as_bf16x8(hb[1][k]), a1, 0, 0, 0);
+              a0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wc, as_bf16x8(lb[0][k]), a0, 0, 0, 0);
+              a1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wc, as_bf16x8(lb[1][k]), a1, 0, 0, 0);
+            }
+            acc[0][h] = a0;
+            acc[1][h] = a1;
+          }
+#pragma unroll
+          for (int m = 0; m < 2; ++m)
+            pc[m][p] = make_uint4(pack2_bf16(acc[m][0][0], acc[m][0][1]), pack2_bf16(acc[m][0][2], acc[m][0][3]),
+                                  pack2_bf16(acc[m][1][0], acc[m][1][1]), pack2_bf16(acc[m][1][2], acc[m][1][3]));
+        }
+        stage = cstage - stage;
+        cstore(stage, cn);
+        cload(o0 + 192, cn);
+#pragma unroll
+        for (int m = 0; m < 2; ++m) {
+          const uint4 other = swap8(r < 8 ? pc[m][1] : pc[m][0]);
+          const uint4 lo = r < 8 ? pc[m][0] : other, hi = r < 8 ? other : pc[m][1];
+          if (decltype(whole)::value || (o0 + fcol < d_out && trow + 16 * m < T)) store16<PAST>(yr[2 * m] + o0, lo);
+          if (decltype(whole)::value || (o0 + fcol < d_out && trow + 16 * m + 8 < T)) store16<PAST>(yr[2 * m + 1] + o0, hi);
+        }
+        __syncthreads();
+        return (o0 += 64) < d_out;
+      };
+      while (pass(cb) && pass(ca)) {
+      }
+    };
+    if (nvalid == LSQ_TB && d_out % 64 == 0) outputs(std::true_type{});
+    else outputs(std::false_type{});
   }
 }
 
@@ -413,37 +383,30 @@ extern "C" int fstu_lds_sequence(float* h, const void* x, const float* A, const 
   float* hnew = ws + 64 + 2 * (size_t)nblk * BtS;
   const size_t shm = (size_t)LSQ_TB * S * sizeof(float);
   hipStream_t s = (hipStream_t)stream;
-  const dim3 grid(nblk, Bt);
+  const unsigned ny = nblk < 32768 ? (unsigned)nblk : 32768u;
+  const dim3 grid((unsigned)Bt, ny, ((unsigned)nblk + ny - 1) / ny);
   const size_t nwords = (size_t)nblk * BtS;
   unsigned cgrid = (unsigned)((nwords + 255) / 256);
   if (cgrid > 1024u) cgrid = 1024u;
-#define LSQ_RUN2(NTV, PASTV)                                                                                          \
-  do {                                                                                                        \
-    static const hipError_t e1 = hipFuncSetAttribute((const void*)lds_seq_kernel<NTV, PASTV>,                        \
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024); \
-    if (e1 != hipSuccess) {                                                                                   \
-      fstu_set_error("fstu_lds_sequence: hipFuncSetAttribute: %s", hipGetErrorString(e1));                    \
-      return (int)e1;                                                                                         \
-    }                                                                                                         \
-    hipLaunchKernelGGL(lds_seq_clear_kernel, dim3(cgrid), dim3(256), 0, s, etag, nwords, status);             \
-    hipLaunchKernelGGL((lds_seq_kernel<NTV, PASTV>), grid, dim3(256), shm, s, (const bf16_t*)x, A, (const bf16_t*)BmT,\
-                       (const bf16_t*)CmT, (bf16_t*)y, (const float*)h, hnew, etag, status, 1u, T, Bt, d_in, S, d_out);\
-    hipLaunchKernelGGL(lds_seq_finish_kernel, dim3((unsigned)((BtS + 255) / 256)), dim3(256), 0, s, h, (const float*)hnew,\
-                       (int)BtS);                                                                             \
-  } while (0)
-#define LSQ_RUN(NTV)            \
-  do {                          \
-    if (past)                   \
-      LSQ_RUN2(NTV, true);      \
-    else                        \
-      LSQ_RUN2(NTV, false);     \
-  } while (0)
   const bool past = (size_t)T * Bt * d_out * sizeof(bf16_t) > (size_t)32 << 20;
-  if (S <= 64) LSQ_RUN(4);
-  else if (S <= 160) LSQ_RUN(10);
-  else LSQ_RUN(16);
-#undef LSQ_RUN
-#undef LSQ_RUN2
+  hipError_t e = hipSuccess;
+  auto run = [&](auto kernel) {
+    e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024);
+    if (e != hipSuccess) return;
+    hipLaunchKernelGGL(lds_seq_clear_kernel, dim3(cgrid), dim3(256), 0, s, etag, nwords, status);
+    hipLaunchKernelGGL(kernel, grid, dim3(256), shm, s, (const bf16_t*)x, A, (const bf16_t*)BmT, (const bf16_t*)CmT, (bf16_t*)y,
+                       (const float*)h, hnew, etag, status, 1u, T, Bt, d_in, d_out, nblk);
+    hipLaunchKernelGGL(lds_seq_finish_kernel, dim3((unsigned)((BtS + 255) / 256)), dim3(256), 0, s, h, (const float*)hnew, (int)BtS);
+  };
+#define LSQ_CASE(n) case 32 * n: past ? run(lds_seq_kernel<2 * n, true>) : run(lds_seq_kernel<2 * n, false>); break
+  switch (S) {
+    LSQ_CASE(1); LSQ_CASE(2); LSQ_CASE(3); LSQ_CASE(4); LSQ_CASE(5); LSQ_CASE(6); LSQ_CASE(7); LSQ_CASE(8);
+  }
+#undef LSQ_CASE
+  if (e != hipSuccess) {
+    fstu_set_error("fstu_lds_sequence: hipFuncSetAttribute: %s", hipGetErrorString(e));
+    return (int)e;
+  }
   FSTU_CHECK_LAUNCH("fstu_lds_sequence");
   return FSTU_OK;
 }

@@ -1548,6 +1548,14 @@ def test_lds_sequence_edges_of_its_stores(hip, T, Bt, d_in, S, d_out):
     assert bool(((h.double().cpu() - state).abs() <= (d_in + 2 * T) * 2.0 ** -23 * size).all())
 
 
+@pytest.mark.parametrize("T,Bt,d_in,S,d_out", [(128, 2, 64, 32, 64), (131, 1, 128, 64, 128), (260, 3, 192, 96, 192), (128, 1, 448, 128, 320),
+                                               (300, 2, 480, 160, 384), (129, 1, 864, 192, 272), (256, 2, 1024, 224, 64), (140, 1, 416, 256, 448)])
+def test_lds_sequence_chunks_in_flight(hip, T, Bt, d_in, S, d_out):
+    """Every number of state tiles, with fewer and more chunks of d_in and groups of features than are requested ahead, whole and
+    cut ones, to the same bounds."""
+    test_lds_sequence_edges_of_its_stores(hip, T, Bt, d_in, S, d_out)
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_lds_steps_dense(hip, dtype):
     g = gen(13)
