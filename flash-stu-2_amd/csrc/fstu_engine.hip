@@ -301,6 +301,11 @@ static int decode_step_impl(const fstu_model_desc* m, const int64_t* tok_in, int
   void* xc = m->x;
   void* xo = m->x2;
   const bool glu_bal = dt == FSTU_BF16 && m->glu_packed && fstu_glu_packed_supported(B, d, I);
+  const bool rm = m->row_major;   // no packed copies: the same launches on the parameters themselves
+  auto gate = [&](const fstu_layer_desc& L) { return rm ? L.w_gate : L.wp_gate; };
+  auto up = [&](const fstu_layer_desc& L) { return rm ? L.w_up : L.wp_up; };
+  auto down = [&](const fstu_layer_desc& L) { return rm ? L.w_down : L.wp_down; };
+  auto qkv = [&](const fstu_layer_desc& L) { return rm ? L.w_qkv : L.wp_qkv; };
   // Merged norms: the down projection leaves 4 split-K slices and the first projection of the NEXT layer adds them
   // to the residual stream and normalises it in its own prologue, so the add+norm launch between two layers is gone
   // (the one in front of the head stays).
@@ -308,7 +313,7 @@ static int decode_step_impl(const fstu_model_desc* m, const int64_t* tok_in, int
                     (size_t)B * (d / 8) <= 1024 && I % 128 == 0 && I / 128 <= 96;
   for (int l = 0; l < m->n_layers && merge_norm; ++l) {
     const fstu_layer_desc& L = m->layers[l];
-    merge_norm = L.wp_gate && L.wp_up && L.wp_down && (L.kind == 0 || L.wp_qkv);
+    merge_norm = gate(L) && up(L) && down(L) && (L.kind == 0 || qkv(L));
   }
   bool pending_slices = false;   // m->partial holds 4 slices of the previous layer's MLP output, not yet added
   for (int l = 0; l < m->n_layers; ++l) {
@@ -340,8 +345,7 @@ static int decode_step_impl(const fstu_model_desc* m, const int64_t* tok_in, int
       }
     } else {
       if (pending_slices) {
-        TIMED(PC_PROJ, fstu_linear_packed_res(xc, m->partial, 4, xo, L.norm1_w, m->eps, L.wp_qkv, m->qkv, 3 * d, B, 3 * d, d,
-                                              stream));
+        TIMED(PC_PROJ, fstu_linear_res_impl(xc, m->partial, 4, xo, L.norm1_w, m->eps, qkv(L), m->qkv, 3 * d, B, 3 * d, d, rm, stream));
         void* t = xc; xc = xo; xo = t;
         pending_slices = false;
       } else if (glu_bal && L.wp_qkv)
@@ -354,9 +358,9 @@ static int decode_step_impl(const fstu_model_desc* m, const int64_t* tok_in, int
       pending_y = true;
     }
     const void* next_w = (l + 1 < m->n_layers) ? m->layers[l + 1].norm1_w : m->final_norm_w;
-    if (pending_y && glu_bal && m->x2 && L.wp_gate && L.wp_up) {
+    if (pending_y && glu_bal && m->x2 && gate(L) && up(L)) {
       // residual add + mlp_norm as the prologue of the balanced gate/up launch; the stream moves to the other buffer
-      TIMED(PC_GLU, fstu_glu_packed_norm(xc, m->y, xo, L.mlp_norm_w, m->eps, L.wp_gate, L.wp_up, m->act, I, B, I, d, stream));
+      TIMED(PC_GLU, fstu_glu_norm_impl(xc, m->y, xo, L.mlp_norm_w, m->eps, gate(L), up(L), m->act, I, B, I, d, rm, stream));
       void* t = xc; xc = xo; xo = t;
     } else {
       if (pending_y) TIMED(PC_NORM, fstu_add_rmsnorm(xc, m->y, 0, 1, 0, L.mlp_norm_w, m->h, B, d, m->eps, dt, stream));
@@ -367,7 +371,7 @@ static int decode_step_impl(const fstu_model_desc* m, const int64_t* tok_in, int
     }
     if (merge_norm) {
       int nsl = 4;
-      TIMED(PC_DOWN, fstu_down_packed_splitk(m->act, I, L.wp_down, m->partial, B, d, I, &nsl, stream));
+      TIMED(PC_DOWN, fstu_down_splitk_impl(m->act, I, down(L), m->partial, B, d, I, &nsl, rm, stream));
       if (l + 1 == m->n_layers)   // the head reads normalised rows
         TIMED(PC_NORM, fstu_add_rmsnorm(xc, m->partial, 1, nsl, 0, next_w, m->h, B, d, m->eps, dt, stream));
       else
@@ -375,8 +379,8 @@ static int decode_step_impl(const fstu_model_desc* m, const int64_t* tok_in, int
       continue;
     }
     int nsl = 16;
-    if (glu_bal && m->down_packed && L.wp_down && d % 16 == 0 && I % 512 == 0 && I / 512 <= 64)
-      TIMED(PC_DOWN, fstu_down_packed_splitk(m->act, I, L.wp_down, m->partial, B, d, I, &nsl, stream));
+    if (glu_bal && m->down_packed && down(L) && d % 16 == 0 && I % 512 == 0 && I / 512 <= 64)
+      TIMED(PC_DOWN, fstu_down_splitk_impl(m->act, I, down(L), m->partial, B, d, I, &nsl, rm, stream));
     else {
       nsl = m->ksplit_down;
       TIMED(PC_DOWN, fstu_linear_decode_splitk(m->act, I, L.w_down, m->partial, B, d, I, m->ksplit_down, dt, stream));

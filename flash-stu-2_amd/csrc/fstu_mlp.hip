@@ -141,7 +141,11 @@ struct GluArgs {
 // (arguments passed one by one so that the command processor can preload the leading ones into SGPRs)
 // NB = 2 (no prologue): rows 16..31 are a second B tile of the same weight fragments, so 17..32 rows read every weight
 // once; the partial sums of the two row tiles then lie behind each other in dynamic LDS.
-template <int KSA, int PRO, int EPI, int NB = 1>
+// RM: the weights are row-major as nn.Linear holds them (a caller that steps on the parameters themselves): a load
+// instruction then covers 64 bytes of 16 rows, the other half of each 128-byte line is the next one's, so these loads stay in
+// the caches.  us at 768 x 9216, 4 rows, in the step: 8.8 with its norm (packed 8.1), 10.4 and 2.3 as a launch of 16 features to a
+// workgroup and one of the norm; down projection 5.6 with four slices, 5.0 with twelve; QKV 5.5 with its norm, 3.6 and 2.3.
+template <int KSA, int PRO, int EPI, int NB = 1, bool RM = false>
 __global__ void __launch_bounds__(512)
 glu_balanced_kernel(const bf16_t* h, const uint4* wp_gate, const uint4* wp_up, bf16_t* act, const bf16_t* x_in,
                     const void* delta, bf16_t* x_out, const bf16_t* norm_w, int rows, int d, int I, int ldh, int ldact,
@@ -179,18 +183,18 @@ glu_balanced_kernel(const bf16_t* h, const uint4* wp_gate, const uint4* wp_up, b
   }
   const int ta0 = f0 >> 4, ta1 = (f1 > f0) ? ((f1 + 15) >> 4) : ta0;
   const size_t tsa = (size_t)(a.d >> 5) * 64;
-  const size_t wa_bytes = (size_t)((a.I + 15) >> 4) * tsa * 16;
+  const size_t wa_bytes = RM ? (size_t)a.I * a.d * 2 : (size_t)((a.I + 15) >> 4) * tsa * 16;
   const rsrc_t rg = make_rsrc(a.wp_gate, wa_bytes), ru = make_rsrc(a.wp_up, wa_bytes);
-  const unsigned abase = ((unsigned)(w * KSA) * 64 + lane) * 16u;
+  const unsigned abase = RM ? (unsigned)r * (unsigned)a.d * 2u + (unsigned)(w * KSA) * 64u + (unsigned)g * 16u : ((unsigned)(w * KSA) * 64 + lane) * 16u;
   uint4 wa[DA][KSA], wb[DA][KSA];
   auto load_a = [&](int j, int tile) {
     const int f = tile * 16 + r;
     const bool ok = tile < ta1 && f >= f0 && f < f1;
 #pragma unroll
     for (int u = 0; u < KSA; ++u) {
-      const unsigned off = ok ? abase + ((unsigned)tile * (unsigned)tsa + (unsigned)u * 64u) * 16u : MLP_OOB;
-      wa[j][u] = buf_load16_stream(rg, off);
-      if (GLU) wb[j][u] = buf_load16_stream(ru, off);
+      const unsigned off = ok ? abase + (unsigned)tile * (unsigned)tsa * 16u + (unsigned)u * (RM ? 64u : 1024u) : MLP_OOB;
+      wa[j][u] = RM ? buf_load16(rg, off) : buf_load16_stream(rg, off);
+      if (GLU) wb[j][u] = RM ? buf_load16(ru, off) : buf_load16_stream(ru, off);
     }
   };
   // a tile beyond the workgroup's range is skipped by a uniform branch: a load of nothing still costs its address cycles
@@ -538,7 +542,7 @@ struct DownSkArgs {
 };
 
 // NB = 2: rows 16..31 as a second B tile of the same weight fragments (17..32 rows read every weight once).
-template <int KSB, int NB = 1>
+template <int KSB, int NB = 1, bool RM = false>
 __global__ void __launch_bounds__(512)
 down_splitk_balanced_kernel(const bf16_t* act, const uint4* wp_down, float* partial, int rows, int d, int I, int ldact, int KS,
                             int tpw, int tiles_out, int kch) {
@@ -568,12 +572,15 @@ down_splitk_balanced_kernel(const bf16_t* act, const uint4* wp_down, float* part
       xb2[u] = buf_load16(rx, (xrow2 && u < nks) ? xbase + (unsigned)(16 * a.ldact) * 2u + (unsigned)u * 64u : MLP_OOB);
   }
   const rsrc_t rdn = make_rsrc(a.wp_down, (size_t)a.tiles_out * tsb * 16);
-  const unsigned bbase = ((unsigned)(chunk * a.kch + ksb0) * 64 + lane) * 16u;
+  const unsigned bbase = RM ? (unsigned)r * (unsigned)a.I * 2u + (unsigned)(chunk * a.kch + ksb0) * 64u + (unsigned)g * 16u
+                            : ((unsigned)(chunk * a.kch + ksb0) * 64 + lane) * 16u;
   uint4 wd[DB][KSB];
   auto load_b = [&](int j, int tile) {
 #pragma unroll
-    for (int u = 0; u < KSB; ++u)
-      wd[j][u] = buf_load16_stream(rdn, (u < nks && tile < tb1) ? bbase + ((unsigned)tile * (unsigned)tsb + (unsigned)u * 64u) * 16u : MLP_OOB);
+    for (int u = 0; u < KSB; ++u) {
+      const unsigned off = (u < nks && tile < tb1) ? bbase + (unsigned)tile * (unsigned)tsb * 16u + (unsigned)u * (RM ? 64u : 1024u) : MLP_OOB;
+      wd[j][u] = RM ? buf_load16(rdn, off) : buf_load16_stream(rdn, off);
+    }
   };
   // waves beyond the chunk's k steps and tiles beyond the group's range are skipped by uniform branches: a load of
   // nothing still costs its address cycles
@@ -656,7 +663,17 @@ extern "C" int fstu_mlp_packed_rows32_supported(int rows, int d, int I) {
 }
 
 template <int KSA>
-static int glu_launch_ksa(GluArgs& a, int pro, int epi, int G, size_t shm, const char* name, hipStream_t s) {
+static int glu_launch_ksa(GluArgs& a, int pro, int epi, int G, size_t shm, const char* name, hipStream_t s, bool row_major) {
+  if constexpr (KSA <= 4) if (row_major) {       // 1..16 rows behind a norm prologue, widths up to 1024
+    auto go = [&](auto kernel) -> int {
+      hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
+      FSTU_REQUIRE(e == hipSuccess, (int)e, "%s: %zu bytes of dynamic LDS refused", name, shm);
+      hipLaunchKernelGGL(kernel, dim3(G), dim3(512), shm, s, a.h, a.wp_gate, a.wp_up, a.act, a.x_in, a.delta, a.x_out, a.norm_w, a.rows,
+                         a.d, a.I, a.ldh, a.ldact, a.fpw, a.eps, a.nslices, a.best, a.temperature);
+      return FSTU_OK;
+    };
+    return pro == 2 ? go(glu_balanced_kernel<KSA, 2, 1, 1, true>) : go(glu_balanced_kernel<KSA, 1, 0, 1, true>);
+  }
 #define GLU_GO(PRO, GLUF)                                                                                        \
   do {                                                                                                           \
     if (shm > 0) {                                                                                               \
@@ -700,9 +717,10 @@ static int glu_launch_ksa(GluArgs& a, int pro, int epi, int G, size_t shm, const
   return FSTU_OK;
 }
 
-static int glu_launch(GluArgs& a, int pro, int epi, const char* name, hipStream_t s) {
+static int glu_launch(GluArgs& a, int pro, int epi, const char* name, hipStream_t s, bool row_major = false) {
   int G = query_cus();
   FSTU_REQUIRE(G > 0, FSTU_EARG, "%s: no device", name);
+  FSTU_REQUIRE(!row_major || a.d <= 1024, FSTU_ESHAPE, "%s: row-major weights of width %d", name, a.d);
   // Features are dealt out in groups of 8: no 128-byte line is shared between two workgroups (HBM traffic of the
   // gate/up launch 1.00x the algorithmic bytes instead of 1.125x with groups of 4), at the price of workgroups of 32
   // and 40 features instead of 36 each.
@@ -718,11 +736,11 @@ static int glu_launch(GluArgs& a, int pro, int epi, const char* name, hipStream_
   const size_t shm = (pro == 1 || pro == 2) ? (size_t)a.rows * (a.d + 8) * 2 : 0;
   int rc;
   switch (a.d / 256) {
-    case 1: rc = glu_launch_ksa<1>(a, pro, epi, G, shm, name, s); break;
-    case 2: rc = glu_launch_ksa<2>(a, pro, epi, G, shm, name, s); break;
-    case 3: rc = glu_launch_ksa<3>(a, pro, epi, G, shm, name, s); break;
-    case 4: rc = glu_launch_ksa<4>(a, pro, epi, G, shm, name, s); break;
-    default: rc = glu_launch_ksa<8>(a, pro, epi, G, shm, name, s); break;
+    case 1: rc = glu_launch_ksa<1>(a, pro, epi, G, shm, name, s, row_major); break;
+    case 2: rc = glu_launch_ksa<2>(a, pro, epi, G, shm, name, s, row_major); break;
+    case 3: rc = glu_launch_ksa<3>(a, pro, epi, G, shm, name, s, row_major); break;
+    case 4: rc = glu_launch_ksa<4>(a, pro, epi, G, shm, name, s, row_major); break;
+    default: rc = glu_launch_ksa<8>(a, pro, epi, G, shm, name, s, row_major); break;
   }
   if (rc) return rc;
   hipError_t e = hipGetLastError();
@@ -747,14 +765,13 @@ extern "C" int fstu_glu_packed(const void* h, int ldh, const void* wp_gate, cons
   return glu_launch(a, 0, 0, "fstu_glu_packed", (hipStream_t)stream);
 }
 
-extern "C" int fstu_glu_packed_norm(const void* x_in, const void* delta, void* x_out, const void* norm_w, float eps,
-                                    const void* wp_gate, const void* wp_up, void* act, int ldact, int rows, int I, int d,
-                                    void* stream) {
+int fstu_glu_norm_impl(const void* x_in, const void* delta, void* x_out, const void* norm_w, float eps, const void* wp_gate,
+                       const void* wp_up, void* act, int ldact, int rows, int I, int d, bool row_major, void* stream) {
   FSTU_REQUIRE(x_in && norm_w && wp_gate && wp_up && act, FSTU_ENULL, "fstu_glu_packed_norm: null pointer");
   // 17..32 rows: the norm is formed in the matrix-core fragments (two row tiles) of a stream that already holds the
   // sub-layer's output (fstu_linear_packed_add, the recurrence step with a residual): no delta, nothing stored
   const bool wide = rows > FSTU_MAX_DECODE_ROWS;
-  FSTU_REQUIRE(wide ? fstu_mlp_packed_rows32_supported(rows, d, I) : fstu_glu_packed_supported(rows, d, I), FSTU_ESHAPE,
+  FSTU_REQUIRE(wide ? !row_major && fstu_mlp_packed_rows32_supported(rows, d, I) : fstu_glu_packed_supported(rows, d, I), FSTU_ESHAPE,
                "fstu_glu_packed_norm: unsupported shape rows=%d d=%d I=%d", rows, d, I);
   FSTU_REQUIRE(!wide || (delta == nullptr && x_out == nullptr), FSTU_EARG,
                "fstu_glu_packed_norm: more than %d rows take the summed stream (delta and x_out must be NULL)", FSTU_MAX_DECODE_ROWS);
@@ -769,7 +786,13 @@ extern "C" int fstu_glu_packed_norm(const void* x_in, const void* delta, void* x
   a.rows = rows; a.d = d; a.I = I; a.ldh = d; a.ldact = ldact;
   a.x_in = (const bf16_t*)x_in; a.delta = delta; a.x_out = (bf16_t*)x_out; a.norm_w = (const bf16_t*)norm_w;
   a.eps = eps;
-  return glu_launch(a, wide ? 3 : 1, 0, "fstu_glu_packed_norm", (hipStream_t)stream);
+  return glu_launch(a, wide ? 3 : 1, 0, "fstu_glu_packed_norm", (hipStream_t)stream, row_major);
+}
+
+extern "C" int fstu_glu_packed_norm(const void* x_in, const void* delta, void* x_out, const void* norm_w, float eps,
+                                    const void* wp_gate, const void* wp_up, void* act, int ldact, int rows, int I, int d,
+                                    void* stream) {
+  return fstu_glu_norm_impl(x_in, delta, x_out, norm_w, eps, wp_gate, wp_up, act, ldact, rows, I, d, false, stream);
 }
 
 // y = T(x W^T) over packed W (N,K): x given normalised (norm_w == NULL, x = h with row stride ldx) or as the residual
@@ -834,8 +857,8 @@ extern "C" int fstu_head_maxima_packed(const void* x, int ldx, const void* wp, v
 // y = T(h W^T) with h = rmsnorm(x') * norm_w and x' = T(x_in + T(sum of nslices fp32 slices)): the add+norm launch
 // between a split-K projection and the next projection, folded into the latter.  x' is stored to x_out by one
 // workgroup (x_out must not alias x_in: the other workgroups still read it).
-extern "C" int fstu_linear_packed_res(const void* x_in, const float* partial, int nslices, void* x_out, const void* norm_w,
-                                      float eps, const void* wp, void* y, int ldy, int rows, int N, int K, void* stream) {
+int fstu_linear_res_impl(const void* x_in, const float* partial, int nslices, void* x_out, const void* norm_w, float eps,
+                         const void* wp, void* y, int ldy, int rows, int N, int K, bool row_major, void* stream) {
   FSTU_REQUIRE(x_in && partial && x_out && norm_w && wp && y, FSTU_ENULL, "fstu_linear_packed_res: null pointer");
   FSTU_REQUIRE((fstu_glu_packed_supported(rows, K, N) && NormPrologue<512, 2, 4>::supported(rows, K)), FSTU_ESHAPE,
                "fstu_linear_packed_res: unsupported shape rows=%d K=%d N=%d", rows, K, N);
@@ -850,13 +873,19 @@ extern "C" int fstu_linear_packed_res(const void* x_in, const float* partial, in
   a.wp_gate = (const uint4*)wp; a.wp_up = (const uint4*)wp; a.act = (bf16_t*)y;
   a.rows = rows; a.d = K; a.I = N; a.ldh = K; a.ldact = ldy; a.eps = eps;
   a.x_in = (const bf16_t*)x_in; a.delta = partial; a.nslices = nslices; a.x_out = (bf16_t*)x_out; a.norm_w = (const bf16_t*)norm_w;
-  return glu_launch(a, 2, 1, "fstu_linear_packed_res", (hipStream_t)stream);
+  return glu_launch(a, 2, 1, "fstu_linear_packed_res", (hipStream_t)stream, row_major);
+}
+
+extern "C" int fstu_linear_packed_res(const void* x_in, const float* partial, int nslices, void* x_out, const void* norm_w,
+                                      float eps, const void* wp, void* y, int ldy, int rows, int N, int K, void* stream) {
+  return fstu_linear_res_impl(x_in, partial, nslices, x_out, norm_w, eps, wp, y, ldy, rows, N, K, false, stream);
 }
 
 // Balanced split-K down projection: partial (ksplit, rows, d) fp32 slices, summed by fstu_add_rmsnorm(delta_mode 1).
 // Returns the number of slices through *ksplit_out (16, the K chunks of the launch).
-extern "C" int fstu_down_packed_splitk(const void* act, int ldact, const void* wp_down, float* partial, int rows, int d, int I,
-                                       int* ksplit_io, void* stream) {
+int fstu_down_splitk_impl(const void* act, int ldact, const void* wp_down, float* partial, int rows, int d, int I, int* ksplit_io,
+                          bool row_major, void* stream) {
+  FSTU_REQUIRE(!row_major || rows <= FSTU_MAX_DECODE_ROWS, FSTU_ESHAPE, "fstu_down_splitk: rows=%d over row-major weights", rows);
   FSTU_REQUIRE(act && wp_down && partial, FSTU_ENULL, "fstu_down_packed_splitk: null pointer");
   // *ksplit_io on entry: the number of K slices wanted (4, 8 or 16; anything else: 16); on return: the number written
   const int want = ksplit_io ? *ksplit_io : 16;
@@ -883,7 +912,10 @@ extern "C" int fstu_down_packed_splitk(const void* act, int ldact, const void* w
   hipStream_t s = (hipStream_t)stream;
 #define DOWN_GO(KSB)                                                                                                          \
   do {                                                                                                                         \
-    if (rows > FSTU_MAX_DECODE_ROWS)                                                                                           \
+    if (row_major)                                                                                                             \
+      hipLaunchKernelGGL((down_splitk_balanced_kernel<KSB, 1, true>), grid, dim3(512), 0, s, a.act, a.wp_down, a.partial, a.rows, \
+                         a.d, a.I, a.ldact, a.KS, a.tpw, a.tiles_out, a.kch);                                                  \
+    else if (rows > FSTU_MAX_DECODE_ROWS)                                                                                      \
       hipLaunchKernelGGL((down_splitk_balanced_kernel<KSB, 2>), grid, dim3(512), 0, s, a.act, a.wp_down, a.partial, a.rows, a.d, \
                          a.I, a.ldact, a.KS, a.tpw, a.tiles_out, a.kch);                                                       \
     else                                                                                                                       \
@@ -902,4 +934,9 @@ extern "C" int fstu_down_packed_splitk(const void* act, int ldact, const void* w
   FSTU_CHECK_LAUNCH("fstu_down_packed_splitk");
   if (ksplit_io) *ksplit_io = KS;
   return FSTU_OK;
+}
+
+extern "C" int fstu_down_packed_splitk(const void* act, int ldact, const void* wp_down, float* partial, int rows, int d, int I,
+                                       int* ksplit_io, void* stream) {
+  return fstu_down_splitk_impl(act, ldact, wp_down, partial, rows, d, I, ksplit_io, false, stream);
 }

@@ -44,7 +44,8 @@ class ModelDesc(ctypes.Structure):
                 ("eps", _f), ("softcap", _f), ("emb", _vp), ("final_norm_w", _vp), ("layers", ctypes.POINTER(LayerDesc)),
                 ("x", _vp), ("h", _vp), ("qkv", _vp), ("attn", _vp), ("act", _vp), ("xp", _vp), ("y", _vp),
                 ("partial", _vp), ("eo", _vp), ("logits", _vp), ("best", _vp), ("samp_ws", _vp),
-                ("wp_emb", _vp), ("x2", _vp), ("glu_packed", _i), ("down_packed", _i), ("merge_norm", _i)]
+                ("wp_emb", _vp), ("x2", _vp), ("glu_packed", _i), ("down_packed", _i), ("merge_norm", _i),
+                ("row_major", _i)]
 
 
 def pick_ksplit_down(I: int) -> int:
@@ -96,12 +97,13 @@ def step_on_caches(model, ids: torch.Tensor, past):
             or model.lm_head.bias is not None or d != cfg.n_embd or d % H != 0 or model.norm.eps != eps):
         return None
     I, hd = d * cfg.mlp_scale, d // H
-    good = True
+    good = aligned = True
     keep = []
 
     def ptr(t, *shape, dtype=dt):
-        nonlocal good
+        nonlocal good, aligned
         keep.append(t)
+        aligned = aligned and t is not None and t.data_ptr() % 16 == 0
         good = good and t is not None and t.dtype == dtype and t.device == dev and t.shape == shape and t.is_contiguous()
         return t.data_ptr() if good else None
     arr = (LayerDesc * n)()
@@ -176,7 +178,14 @@ def step_on_caches(model, ids: torch.Tensor, past):
     logits = torch.empty(B, 1, V, dtype=dt, device=dev)
     m.logits = logits.data_ptr()
     esz = emb.element_size()
-    sizes = dict(x=B * d * esz, h=B * d * esz, y=B * d * esz, xp=B * d * esz, attn=B * d * esz, qkv=3 * B * d * esz,
+    if aligned and dt == torch.bfloat16 and d <= 1024:
+        # The launches of the packed step (norms as prologues, down projection in a few slices) on the parameters themselves.
+        # 24 positions behind a prompt of 600, ms so / through the row-major kernels and launches of their own: 12 layers of 768,
+        # 4 rows 11.8 / 13.1, 16 rows 16.7 / 17.9; 8 layers of 1024, 4 rows 8.9 / 9.4; but of 2048, where the bytes decide and one
+        # workgroup to a compute unit fetches rows in halves of a line, 25.2 / 24.1.
+        m.glu_packed = m.row_major = 1
+        m.down_packed = m.merge_norm = int(I % 512 == 0)
+    sizes = dict(x=B * d * esz, x2=B * d * esz, h=B * d * esz, y=B * d * esz, xp=B * d * esz, attn=B * d * esz, qkv=3 * B * d * esz,
                  act=B * I * esz, partial=max(m.ksplit_down, 16) * B * d * 4,
                  eo=0 if lds else DecodeEngine.HIST_NSPLIT_MAX * 2 * B * d * 4)
     ws = torch.empty(sum((v + 255) // 256 * 256 for v in sizes.values()), dtype=torch.uint8, device=dev)

@@ -612,6 +612,8 @@ typedef struct {
                                attention layers, B*d <= 8192): the down projection leaves 4 split-K slices and the next
                                layer's first projection adds and normalises them in its prologue
                                (fstu_stu_res_inproj_step / fstu_linear_packed_res); one add+norm launch less per layer */
+  int row_major;            /* != 0 (1..16 rows, d <= 1024): glu_packed, down_packed and merge_norm hold without packed copies, the same
+                               launches read w_gate, w_up, w_down and w_qkv themselves (16-byte aligned) */
 } fstu_model_desc;
 
 /* tok_in[b*tok_stride] is the token at absolute position pos; the sampled next

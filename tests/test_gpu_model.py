@@ -746,6 +746,29 @@ def test_steps_on_caches_of_more_rows_than_one_launch_takes(dtype, extra):
     assert float((got - want).abs().max()) <= (1e-4 if dtype == torch.float32 else 2e-2) * float(want.abs().max())
 
 
+@pytest.mark.parametrize("d,scale,rows,mode", [(256, 2, 1, "lds"), (256, 4, 16, "lds"), (512, 4, 3, "lds"), (768, 2, 10, "lds"), (768, 12, 11, "lds"),
+                                               (1024, 4, 8, "lds"), (1024, 3, 9, "lds"), (2048, 2, 4, "lds"), (2048, 4, 5, "lds"), (512, 2, 4, "history")])
+def test_one_call_step_on_the_parameters_themselves(d, scale, rows, mode):
+    """The step on caches reads row-major weights in the launches that generate() runs over packed copies: every width those take,
+    with the norms merged (rows * d up to 8192, feature counts of 512) and beside them, against the layers' own calls.  Sums of the
+    same products in other orders: the bounds of the one-call step's other tests."""
+    _, _, model = make_pair(seed=5, init="healthy", dtype=torch.bfloat16, mlp_scale=scale, n_embd=d, n_layers=4, n_heads=d // 64, window_size=8,
+                            num_eigh=8, seq_len=64, vocab_size=777, stu_decode_mode=mode)
+    ids = prompt(rows, 10, 777, 3).cuda()
+
+    def run():
+        past, logits = model(ids[:, :6], use_cache=True).past_key_values, []
+        for t in range(6, 10):
+            out = model(ids[:, t:t + 1], past_key_values=past, use_cache=True)
+            past = out.past_key_values
+            logits.append(out.logits.float())
+        return torch.cat(logits, 1)
+    got = run()
+    model.layers[0].mlp.register_forward_hook(lambda *a: None)     # the layers' own calls run
+    want = run()
+    assert float((got - want).abs().max()) <= 2e-2 * float(want.abs().max())
+
+
 def test_forward_accepts_reference_style_kv_cache():
     from flash_stu import Attention, FlashSTUConfig
     cfg = FlashSTUConfig(n_embd=128, n_heads=2, n_layers=2, seq_len=64, window_size=6, vocab_size=11, mlp_scale=2,
