@@ -37,12 +37,6 @@ typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
 #define GM_MAX_LD (1 << 22)
 
 __device__ __forceinline__ float rnd_bf16(float v) { return bf16_to_f32(f32_to_bf16(v)); }
-__device__ __forceinline__ float gelu_tanh_fast(float x) {
-  const float inner = 0.7978845608028654f * (x + 0.044715f * x * x * x);
-  const float e = __builtin_amdgcn_exp2f(2.8853900817779268f * inner);   // exp(2 inner)
-  const float th = 1.0f - 2.0f * __builtin_amdgcn_rcpf(e + 1.0f);
-  return 0.5f * x * (1.0f + th);
-}
 
 // 16 bytes per lane from global memory into LDS without a stop in registers: the 64 lanes fill 64 consecutive 16-byte
 // slots from `l` (wave-uniform) on.  The source is a buffer descriptor (base and range in SGPRs), a 32-bit byte offset
