@@ -903,6 +903,8 @@ extern "C" int fstu_gemm_bf16_splitk(const void* A, int64_t lda, const void* W, 
                (long long)lda, K);
   int rc;
   if (M <= 32) rc = gemm_launch_tile<TileRows32, 3>(A, lda, W, nullptr, nullptr, 0, partial, N, M, N, K, (hipStream_t)stream, ksplit);
+  else if ((long long)((M + 127) / 128) * ((N + 127) / 128) * ksplit <= gemm_cus())
+    rc = gemm_launch_tile<TileDeep, 3>(A, lda, W, nullptr, nullptr, 0, partial, N, M, N, K, (hipStream_t)stream, ksplit);
   else rc = gemm_launch_tile<TileSmall, 3>(A, lda, W, nullptr, nullptr, 0, partial, N, M, N, K, (hipStream_t)stream, ksplit);
   if (rc) return rc;
   FSTU_CHECK_LAUNCH("fstu_gemm_bf16_splitk");
@@ -943,15 +945,16 @@ static int fstu_join_slices(const float* part, int ns, const void* R, long long 
   return FSTU_OK;
 }
 
-// Slices of K for a product of few output tiles (1: none).  Without slices a workgroup walks all of K alone, 0.41 us per k tile
-// of 64 whatever the grid; two to a compute unit 0.62 us each; joining costs a launch and the slices' bytes out and back at
-// 4 TB/s.  The estimate only has to rank: us without / with the slices it picks, rows x features x K: 37 x 768 x 9216 58.8 /
-// 11.7 (18), 300 x 768 x 9216 60 / 19.3 (12), 1400 x 768 x 9216 64 / 41 (3), 2331 x 768 x 9216 65 / 47 (4), 3000 x 768 x 9216
-// 67 / 57 (3), 700 x 2048 x 24576 187 / 87 (4), 1500 x 2048 x 24576 198 / 165 (2), 300 x 2048 x 2048 22.5 / 14.8 (4); slabs 1 x
-// 1024 x 1024 x 24576 219 / 63 (8), 1 x 128 x 256 x 6144 50 / 12 (12).  Where it picks none, without / with two: 4096 x 768 x
-// 9216 70.7 / 73.3, 1000 x 2048 x 2048 23.9 / 23.4, 300 x 6144 x 2048 20.5 / 23.8, 1000 x 768 x 768 10.5 / 12.7.  Below K = 2048 the
-// GPU gains less than the second launch and the slices' allocation cost the host (calls of 300 x 384 x 1536 one behind the other
-// 16.0 us with three slices, 13.2 without).
+// Slices of K for a product of few output tiles (1: none).  A workgroup that has a compute unit to itself takes 0.41 us per k tile
+// of 64 on the deep pipeline (0.9 with two stages, which is what slices that leave one to a unit ran on before), two to a unit 0.61
+// each; joining costs a launch and the slices' bytes out and back at 4 TB/s.  The estimate only has to rank: us without / with the
+// slices it picks, rows x features x K: 300 x 768 x 9216 60 / 17.7 (12), 1000 x 768 x 9216 60 / 27.5 (4; 31.4 with two stages), 1400
+// 60 / 34.0 (3; 39.7), 2400 61 / 44.7 (4; 47.2 with two, which were picked before and took 53.8), 3000 63 / 53 (3), 700 x 2048 x
+// 24576 180 / 85 (4), 1500 x 2048 x 24576 184 / 160 (2), 300 x 2048 x 2048 21.8 / 15.0 (4); slabs 1 x 1024 x 1024 x 24576 219 / 63
+// (8), 1 x 128 x 256 x 6144 50 / 12 (12).  Where it picks none, without / with two: 4096 x 768 x 9216 66.6 / 68.8, 600 x 2048 x
+// 2048 22.0 / 18.8, 300 x 6144 x 2048 20.5 / 23.8, 1000 x 768 x 768 10.5 / 12.7.  Below K = 2048 the GPU gains less than the second
+// launch and the slices' allocation cost the host (calls of 300 x 384 x 1536 one behind the other 16.0 us with three slices, 13.2
+// without).
 extern "C" int fstu_gemm_bf16_slices(int M, int N, int K, int nbatch) {
   if (M <= 32 || N % 4 != 0 || K % 64 != 0 || K < 2048) return 1;
   const long long cus = gemm_cus(), tiles = (long long)((M + 127) / 128) * ((N + 127) / 128) * nbatch;
@@ -960,7 +963,7 @@ extern "C" int fstu_gemm_bf16_slices(int M, int N, int K, int nbatch) {
   int best = 1;
   for (int s = 2; s <= 32 && K / s >= 512 && tiles * s <= 2 * cus; ++s) {
     if (nkt % s != 0) continue;
-    const double us = nkt / s * (tiles * s <= cus ? 0.41 : 0.62) + 4.0 + 8e-6 / 4.0 * s * nbatch * (double)M * N;
+    const double us = nkt / s * (tiles * s <= cus ? 0.41 : 0.61) + 3.0 + 8e-6 / 4.0 * s * nbatch * (double)M * N;
     if (us < least) { least = us; best = s; }
   }
   return best;
