@@ -13,6 +13,7 @@ consecutive row chunks of 16 against the same weights and batch-first state.
 """
 from __future__ import annotations
 
+import array
 import ctypes
 from typing import List, Optional
 
@@ -73,6 +74,19 @@ def _as_written(m, cls) -> bool:
     return type(m) is cls and not m._forward_hooks and not m._forward_pre_hooks and _OWN_NAMES.isdisjoint(m.__dict__)
 
 
+# LayerDesc as words of 8 bytes: every field is a pointer but the first, an int in a word of its own
+_LAYER_WORDS = [name for name, _ in LayerDesc._fields_]
+_AT = {name: i for i, name in enumerate(_LAYER_WORDS)}
+assert ctypes.sizeof(LayerDesc) == 8 * len(_LAYER_WORDS) and all(getattr(LayerDesc, name).offset == 8 * i for name, i in _AT.items())
+
+
+def _weight(m):
+    """The weight of a norm or a linear layer; past the module's attribute lookup where its class is the plain one (a
+    parametrized module has a class of its own, and forms a temporary on each access)."""
+    w = m._parameters.get("weight") if type(m) in (torch.nn.Linear, RMSNorm) else None
+    return m.weight if w is None else w
+
+
 @torch.no_grad()
 def step_on_caches(model, ids: torch.Tensor, past):
     """One position of each row, ids (B,1), against the caches that model(..., use_cache=True) returned: (logits (B,1,V),
@@ -97,49 +111,54 @@ def step_on_caches(model, ids: torch.Tensor, past):
             or model.lm_head.bias is not None or d != cfg.n_embd or d % H != 0 or model.norm.eps != eps):
         return None
     I, hd = d * cfg.mlp_scale, d // H
-    good = aligned = True
-    keep = []
-
-    def ptr(t, *shape, dtype=dt):
-        nonlocal good, aligned
-        keep.append(t)
-        aligned = aligned and t is not None and t.data_ptr() % 16 == 0
-        good = good and t is not None and t.dtype == dtype and t.device == dev and t.shape == shape and t.is_contiguous()
-        return t.data_ptr() if good else None
-    arr = (LayerDesc * n)()
+    # What every launch reads or writes, its shape and the descriptor field it goes to, layer behind layer: checked below all
+    # together, since a check of its own for each of some 130 tensors took the host longer than the GPU takes for the step (a step's host
+    # side at 12 layers 430 us, 390 so; of both the launches are 140).
+    tensors, shapes, places = [], [], []     # of the model's dtype
+    tensors32, shapes32, places32 = [], [], []
+    vec, mat_id, mat_di, mat_dd, mat_3d = (d,), (I, d), (d, I), (d, d), (3 * d, d)
+    ring = (B, H, W + 1, hd)
     out = []
     pos = hist_cap = fir_taps = None
     S = 0
-    for layer, ld, entry in zip(model.layers, arr, past):
+    for i, (layer, entry) in enumerate(zip(model.layers, past)):
         stu_layer = type(layer) is STULayer
         if not _as_written(layer, STULayer if stu_layer else AttentionLayer) or not isinstance(entry, tuple) or len(entry) != 3:
             return None
-        op, norm1 = (layer.stu, layer.stu_norm) if stu_layer else (layer.attn, layer.attn_norm)
-        mlp, norm2 = layer.mlp, layer.mlp_norm
+        sub = layer._modules                 # (of exactly these classes: what the attributes of the layer are)
+        op, norm1 = (sub["stu"], sub["stu_norm"]) if stu_layer else (sub["attn"], sub["attn_norm"])
+        mlp, norm2 = sub["mlp"], sub["mlp_norm"]
         if not (_as_written(op, STU if stu_layer else Attention) and _as_written(norm1, RMSNorm) and type(norm2) is RMSNorm
-                and _OWN_NAMES.isdisjoint(norm2.__dict__)
-                and _as_written(mlp, MLP) and norm1.eps == eps and norm2.eps == eps and mlp.gate_proj.bias is None):
+                and _OWN_NAMES.isdisjoint(norm2.__dict__) and _as_written(mlp, MLP) and norm1.eps == eps and norm2.eps == eps):
             return None
+        proj = mlp._modules
+        gate, up, down = proj["gate_proj"], proj["up_proj"], proj["down_proj"]
         a0, a1, pos_t = entry
-        if pos_t.is_cuda or pos_t.dim() != 1 or pos_t.numel() < 1:
+        if gate.bias is not None or pos_t.is_cuda or pos_t.dim() != 1 or pos_t.numel() < 1:
             return None
-        p = int(pos_t[0])
+        p = pos_t.tolist()[0]
         if pos is not None and p != pos:
             return None
         pos = p
-        ld.norm1_w, ld.mlp_norm_w = ptr(norm1.weight, d), ptr(norm2.weight, d)
-        ld.w_gate, ld.w_up, ld.w_down = ptr(mlp.gate_proj.weight, I, d), ptr(mlp.up_proj.weight, I, d), ptr(mlp.down_proj.weight, d, I)
+        at = i * len(_LAYER_WORDS)
+        tensors += (_weight(norm1), _weight(norm2), _weight(gate), _weight(up), _weight(down))
+        shapes += (vec, vec, mat_id, mat_id, mat_di)
+        places += (at + _AT["norm1_w"], at + _AT["mlp_norm_w"], at + _AT["w_gate"], at + _AT["w_up"], at + _AT["w_down"])
         if not stu_layer:
-            ld.kind = 1
             if op.n_heads != H or op.window_size != W or op.softcap != cap0 or op.c_attn.bias is not None or op.c_proj.bias is not None:
                 return None
-            ld.w_qkv, ld.w_proj = ptr(op.c_attn.weight, 3 * d, d), ptr(op.c_proj.weight, d, d)
-            ld.kring, ld.vring = ptr(a0, B, H, W + 1, hd), ptr(a1, B, H, W + 1, hd)
-            ld.slopes = ptr(op.alibi_slopes, H, dtype=torch.float32)
+            tensors += (_weight(op.c_attn), _weight(op.c_proj), a0, a1)
+            shapes += (mat_3d, mat_dd, ring, ring)
+            places += (at + _AT["w_qkv"], at + _AT["w_proj"], at + _AT["kring"], at + _AT["vring"])
+            tensors32.append(op.alibi_slopes)
+            shapes32.append((H,))
+            places32.append(at + _AT["slopes"])
         else:
             if op.M_inputs.device != dev or op.d_in != d or op.config is not cfg:
                 return None
-            ld.m_inputs_t = ptr(op.m_inputs_t(), d, d)
+            tensors.append(op.m_inputs_t())
+            shapes.append(mat_dd)
+            places.append(at + _AT["m_inputs_t"])
             if lds:
                 a, ce, co = op.lds_params()
                 fir = op.lds_fir()
@@ -147,21 +166,41 @@ def step_on_caches(model, ids: torch.Tensor, past):
                 if fir_taps not in (None, taps) or S not in (0, a.numel()) or (taps == 0 and a0.numel() != 0):
                     return None
                 fir_taps, S = taps, a.numel()
-                ld.lds_a, ld.lds_ce, ld.lds_co = (ptr(a, S, dtype=torch.float32), ptr(ce, S, d, dtype=torch.float32),
-                                                  ptr(co, S, d, dtype=torch.float32))
-                ld.lds_state = ptr(a1, B, 2, S, d, dtype=torch.float32)
+                tensors32 += (a, ce, co, a1)
+                shapes32 += ((S,), (S, d), (S, d), (B, 2, S, d))
+                places32 += (at + _AT["lds_a"], at + _AT["lds_ce"], at + _AT["lds_co"], at + _AT["lds_state"])
                 if taps:
-                    ld.lds_ring, ld.lds_fir = ptr(a0, B, taps, d), ptr(fir, taps, d, dtype=torch.float32)
+                    tensors.append(a0)
+                    shapes.append((B, taps, d))
+                    places.append(at + _AT["lds_ring"])
+                    tensors32.append(fir)
+                    shapes32.append((taps, d))
+                    places32.append(at + _AT["lds_fir"])
             else:
                 filt = op.effective_filter()
                 if a0.dim() != 3 or hist_cap not in (None, a0.shape[1]) or a1.numel() != 0 or pos >= a0.shape[1] or pos >= filt.shape[0]:
                     return None
                 hist_cap = a0.shape[1]
-                ld.filt, ld.hist = ptr(filt, filt.shape[0], d), ptr(a0, B, hist_cap, d)
                 S = filt.shape[0]
-        if not good:
-            return None
-        out.append((a0, a1, pos_t))
+                tensors += (filt, a0)
+                shapes += ((S, d), (B, hist_cap, d))
+                places += (at + _AT["filt"], at + _AT["hist"])
+        out.append(entry)
+    tensors += (emb, _weight(model.norm))
+    shapes += ((V, d), vec)
+    every = tensors + tensors32
+    if (pos < 0 or any(t is None for t in every) or [t.shape for t in tensors] != shapes
+            or [t.shape for t in tensors32] != shapes32 or {t.dtype for t in tensors} != {dt} or {t.dtype for t in tensors32} - {torch.float32}
+            or {t.device for t in every} != {dev} or not all(map(torch.Tensor.is_contiguous, every))):
+        return None
+    ptrs = list(map(torch.Tensor.data_ptr, every))
+    aligned = not any(q % 16 for q in ptrs)
+    words = array.array("Q", bytes(8 * n * len(_LAYER_WORDS)))
+    for place, q in zip(places + places32, ptrs[:len(places)] + ptrs[len(tensors):]):
+        words[place] = q
+    for i, layer in enumerate(model.layers):
+        if type(layer) is not STULayer:
+            words[i * len(_LAYER_WORDS)] = 1          # kind, the low half of its word
     m = ModelDesc()
     m.dtype = _hip.FSTU_BF16 if dt == torch.bfloat16 else _hip.FSTU_F32
     m.B, m.d, m.I, m.V, m.n_layers = B, d, I, V, n
@@ -171,10 +210,8 @@ def step_on_caches(model, ids: torch.Tensor, past):
     m.ksplit_down = pick_ksplit_down(I) if dt == torch.bfloat16 else min(8, max(1, I // 512))
     m.hist_nsplit_max = DecodeEngine.HIST_NSPLIT_MAX
     m.eps, m.softcap = float(eps), cap0
-    m.emb, m.final_norm_w = ptr(emb, V, d), ptr(model.norm.weight, d)
-    if not good or pos < 0:
-        return None
-    m.layers = ctypes.cast(arr, ctypes.POINTER(LayerDesc))
+    m.emb, m.final_norm_w = ptrs[len(places)], ptrs[len(places) + 1]
+    m.layers = ctypes.cast(words.buffer_info()[0], ctypes.POINTER(LayerDesc))
     logits = torch.empty(B, 1, V, dtype=dt, device=dev)
     m.logits = logits.data_ptr()
     esz = emb.element_size()
