@@ -977,6 +977,155 @@ template <> __device__ __forceinline__ float lsh_load<bf16_t>(__amdgpu_buffer_rs
   return bf16_to_f32((bf16_t)__builtin_amdgcn_raw_buffer_load_b16(rs, off, 0, 0));
 }
 
+// Up to 64 modes: the state is a sum of powers times inputs, sum_t a_j^(t_last - t) x_t, and the sum over 16 positions of a parity is
+// a product of (modes x positions) powers and (positions x channels) inputs on the fp32 matrix cores; between the groups of 16 the
+// accumulators decay by a^16.  A wave has 32 channels of one row and parity and one of P pieces of the sequence, counted from the
+// end (what lies in front of the first position is zeros, which a state from zero does not see); the pieces meet in LDS in their
+// order.  Powers are formed in double and rounded once, so there are P + T / (8 P) roundings in a row where a step per position
+// makes T / 2.  The decay by a^16 itself is the same for every group, so its rounding adds up: below 8 pieces it carries its
+// remainder.  Off from float64 at 8192 positions, poles up to 0.9998: 4.7e-7 of the state with 8 pieces, 8.0e-7 with one, 8.0e-7 before;
+// at 777 1.6e-7, 3.2e-7 before.
+// What bounded the scan of a position per step (8 waves of 8 modes over 64 channels) was the vector ALUs of the few compute units
+// it has workgroups for.  us, before / now: 3 x 777 x 768 21.4 / 11.6, 8 x 512 x 768 15.3 / 13.2, 1 x 8192 x 1024 164 / 48, 32 x 300 x
+// 2048 54 / 39, 32 x 4096 x 2048 503 / 349 (the matrix cores' fp32 rate would be 220).
+constexpr int LSM_W = 8;
+template <typename T, int P>
+__global__ void __launch_bounds__(LSM_W * 64, 4)
+lds_state_mfma_kernel(const T* __restrict__ hist, const float* __restrict__ a, float* __restrict__ state, int S, int d, int t_last,
+                      int cap, T* __restrict__ ring, int R) {
+  typedef float floatx4_t __attribute__((ext_vector_type(4)));
+  __shared__ float part[P > 1 ? LSM_W : 1][P > 1 ? 64 * 32 : 1];
+  const int b = blockIdx.y, p = blockIdx.z;
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, r = lane & 15, g = lane >> 4, piece = w % P;
+  const int c0 = (blockIdx.x * (LSM_W / P) + w / P) * 32;
+  const int n = t_last < p ? 0 : (t_last - p) / 2 + 1;             // positions of this parity: t = p + 2 m
+  const int chunks = (n + 16 * P - 1) / (16 * P);                  // groups of 16 to a piece
+  const int m0 = n - (P - piece) * 16 * chunks;                    // this wave's first position, < 0: zeros up to 0
+  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<T*>(hist + (size_t)b * cap * d), 0, (unsigned)((size_t)(t_last + 1) * d * sizeof(T)), 0x00020000);
+  const int c[2] = {c0 + r, c0 + 16 + r};
+  // operand B: lane (r, g) has position 4 s + g of the group and channel r of either half (behind the last position: beyond the
+  // descriptor's range, zeros)
+  auto load = [&](int k, float (&x)[4][2]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const int m = m0 + 16 * k + 4 * s + g;
+      const unsigned row = (unsigned)(p + 2 * m) * (unsigned)d;
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        x[s][h] = lsh_load<T>(rs, m >= 0 && c[h] < d ? (row + (unsigned)c[h]) * (unsigned)sizeof(T) : 0xfffffff0u);
+    }
+  };
+  const int k0 = m0 < 0 ? min(chunks, (-m0) / 16) : 0;             // groups that are all zeros
+  float xa[4][2], xb[4][2];
+  load(k0, xa);
+  load(k0 + 1, xb);
+  float v[4][4], a16[4][4], a16r[4][4];     // powers: operand A by tile of modes and step; of 16, head and remainder, by accumulator
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    const int j = 16 * t + r;
+    const double q = j < S ? (double)a[j] : 0.0, q2 = q * q, q4 = q2 * q2, q8 = q4 * q4;
+    const double e = g == 3 ? 1.0 : g == 2 ? q : g == 1 ? q2 : q2 * q;
+    v[t][3] = (float)e;
+    v[t][2] = (float)(e * q4);
+    v[t][1] = (float)(e * q8);
+    v[t][0] = (float)(e * q8 * q4);
+    const float q16 = (float)(q8 * q8), q16r = (float)(q8 * q8 - (double)q16);   // of mode 16 t + r; the accumulators are 16 t + 4 g + i
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      a16[t][i] = __shfl(q16, 4 * g + i, 64);
+      a16r[t][i] = __shfl(q16r, 4 * g + i, 64);
+    }
+  }
+  // the decay over a piece, of the modes that this thread joins
+  auto decay = [&](float (&al)[4]) __attribute__((always_inline)) {
+    double z[4], len[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int j = ((tid >> 5) + 16 * q) & 63;
+      z[q] = j < S ? (double)a[j] : 0.0;
+      len[q] = 1.0;
+    }
+    for (int e = 16 * chunks; e; e >>= 1) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        if (e & 1) len[q] *= z[q];
+        z[q] *= z[q];
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) al[q] = (float)len[q];
+  };
+  float al[4];
+  if constexpr (P == 8) decay(al);
+  floatx4_t acc[4][2];
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) acc[t][h] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+  auto group = [&](int k, float (&x)[4][2]) __attribute__((always_inline)) {
+    // the exact head's ring: position t in slot t % R for the last R positions (every slot is covered when the sequence has R
+    // positions; a shorter one leaves the others as the caller zeroed them)
+    if (ring && p + 2 * (m0 + 16 * k + 15) > t_last - R) {
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const int m = m0 + 16 * k + 4 * s + g, t = p + 2 * m;
+          if (m >= 0 && t > t_last - R && c[h] < d) DT<T>::st(ring + ((size_t)b * R + (t & (R - 1))) * d + c[h], x[s][h]);
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[t][h][i] = P == 8 ? acc[t][h][i] * a16[t][i] : fmaf(acc[t][h][i], a16[t][i], acc[t][h][i] * a16r[t][i]);
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) acc[t][h] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[t][s], x[s][h], acc[t][h], 0, 0, 0);
+    load(k + 2, x);
+  };
+  for (int k = k0; k < chunks; k += 2) {
+    group(k, xa);
+    if (k + 1 < chunks) group(k + 1, xb);
+  }
+  float* const st = state + ((size_t)b * 2 + p) * S * d;
+  if constexpr (P == 1) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int j = 16 * t + 4 * g + i;
+          if (j < S && c[h] < d) st[(size_t)j * d + c[h]] = acc[t][h][i];
+        }
+  } else {
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) part[w][(16 * t + 4 * g + i) * 32 + 16 * h + r] = acc[t][h][i];
+    if constexpr (P < 8) decay(al);
+    __syncthreads();
+#pragma unroll
+    for (int f = 0; f < LSM_W / P; ++f)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int o = tid + 512 * q, j = o >> 5, ch = (blockIdx.x * (LSM_W / P) + f) * 32 + (o & 31);
+        float h = part[f * P][o];
+#pragma unroll
+        for (int e = 1; e < P; ++e) h = fmaf(al[q], h, part[f * P + e][o]);
+        if (j < S && ch < d) st[(size_t)j * d + ch] = h;
+      }
+  }
+}
+
 template <typename T, int MAXJ, int NG /* waves of a workgroup, each with up to MAXJ modes of the same 64 channels */>
 __global__ void __launch_bounds__(NG * 64)
 lds_state_from_hist_kernel(const T* __restrict__ hist, const float* __restrict__ a, float* __restrict__ state, int S,
@@ -1051,15 +1200,26 @@ extern "C" int fstu_stu_lds_state_ring_from_hist(const void* hist, const float* 
                "fstu_stu_lds_state_from_hist: S=%d outside 1..%d", S, LSH_JG * LSH_MAXJ);
   FSTU_REQUIRE(t_last >= -1 && t_last < cap, FSTU_EARG, "fstu_stu_lds_state_from_hist: t_last=%d cap=%d", t_last, cap);
   FSTU_REQUIRE((size_t)cap * d * 4 < 0xfff00000ull, FSTU_ESHAPE, "fstu_stu_lds_state_from_hist: cap*d too large for 32-bit offsets");
-  dim3 grid((d + 63) / 64, B, 2);
   if (S <= 64) {
-    // 8 waves of 8 modes: two waves per SIMD cover each other's dependent fused multiply-adds
-    FSTU_DISPATCH_DTYPE(dtype, "fstu_stu_lds_state_from_hist",
-                        hipLaunchKernelGGL((lds_state_from_hist_kernel<T, 8, 8>), grid, dim3(512), 0, (hipStream_t)stream,
-                                           (const T*)hist, a, state, S, d, t_last, cap, (T*)ring, R));
+    const long long waves = (long long)B * 2 * ((d + 31) / 32);
+    // Pieces by how far the (row, parity, 32 channels) fill the chip's 4096 places, and not of few groups each.  us with 1 / 2 / 4 /
+    // 8 pieces, waves without pieces: 3 x 777 x 768 (144) 39 / 24.5 / 16.5 / 11.6, 8 x 512 x 1024 (512) 28 / 18.9 / 13.4 / 13.5, 8 x
+    // 300 x 2048 (1024) 21.3 / 15.9 / 17.2 / 22.1, 16 x 600 x 1024 (1024) 34.6 / 22.8 / 22.7 / 33, 32 x 128 x 768 (1536) 14.4 / 16.4 /
+    // 17.1 / 22, 24 x 1000 x 1024 (1536) 54 / 52 / 45 / 58, 16 x 300 x 2048 (2048) 23.9 / 25.4 / 31.6 / 48.
+    const int P = waves >= 1792 ? 1 : waves < 640 ? 8 : t_last >= 400 ? 4 : t_last >= 200 ? 2 : 1;
+    FSTU_DISPATCH_DTYPE(dtype, "fstu_stu_lds_state_from_hist", {
+      auto run = [&](auto kernel, int pieces) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)((d + 32 * (LSM_W / pieces) - 1) / (32 * (LSM_W / pieces))), B, 2), dim3(LSM_W * 64), 0,
+                           (hipStream_t)stream, (const T*)hist, a, state, S, d, t_last, cap, (T*)ring, R);
+      };
+      if (P == 8) run(lds_state_mfma_kernel<T, 8>, 8);
+      else if (P == 4) run(lds_state_mfma_kernel<T, 4>, 4);
+      else if (P == 2) run(lds_state_mfma_kernel<T, 2>, 2);
+      else run(lds_state_mfma_kernel<T, 1>, 1);
+    });
   } else {
     FSTU_DISPATCH_DTYPE(dtype, "fstu_stu_lds_state_from_hist",
-                        hipLaunchKernelGGL((lds_state_from_hist_kernel<T, LSH_MAXJ, LSH_JG>), grid, dim3(256), 0,
+                        hipLaunchKernelGGL((lds_state_from_hist_kernel<T, LSH_MAXJ, LSH_JG>), dim3((d + 63) / 64, B, 2), dim3(256), 0,
                                            (hipStream_t)stream, (const T*)hist, a, state, S, d, t_last, cap, (T*)ring, R));
   }
   FSTU_CHECK_LAUNCH("fstu_stu_lds_state_from_hist");

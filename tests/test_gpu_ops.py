@@ -830,6 +830,23 @@ def test_stu_step_lds_recurrence(hip, dtype):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("B,S,d,T", [(1, 64, 24, 1), (1, 64, 768, 2), (2, 40, 200, 33), (1, 64, 65, 257), (3, 24, 768, 520), (21, 64, 520, 402),
+                                     (11, 64, 1000, 250), (22, 7, 500, 130), (28, 64, 1050, 65), (30, 33, 1024, 31), (2, 64, 40, 2049)])
+def test_state_from_hist_against_float64(hip, dtype, B, S, d, T):
+    """Every number of pieces that the sequence is cut into, ragged channels, modes and positions, a cap beyond the last position:
+    powers rounded once, at most T / 2 + 16 sums and decays in a row, 2^-24 each of the absolute sum."""
+    g = gen(T + d)
+    hist = torch.randn(B, T + 3, d, generator=g).to(dtype)
+    a = (1 - torch.exp(torch.linspace(math.log(2e-4), math.log(0.9), S))).float()
+    st = hip.stu_lds_state_from_hist(dev(hist), dev(a), T - 1)
+    for p in range(2):
+        xs = dev(hist)[:, p:T:2].double()
+        V = dev(a).double()[:, None] ** torch.arange(xs.shape[1] - 1, -1, -1, device="cuda", dtype=torch.float64)
+        ref, mag = V @ xs, V @ xs.abs()
+        assert bool(((st[:, p].double() - ref).abs() <= (T / 2 + 16) * 2.0 ** -24 * mag).all())
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("B,S,d,T,t_start", [(3, 64, 256, 41, 0), (2, 64, 768, 512, 0), (2, 40, 200, 37, 5), (1, 128, 64, 130, 1),
                                              (2, 64, 128, 1, 3), (2, 8, 72, 16, 0)])
 def test_stu_scan_lds_equals_steps_and_float64(hip, dtype, B, S, d, T, t_start):
