@@ -63,6 +63,10 @@ int fstu_linear_res_impl(const void* x_in, const float* partial, int nslices, vo
                          const void* wp, void* y, int ldy, int rows, int N, int K, bool row_major, void* stream);
 int fstu_down_splitk_impl(const void* act, int ldact, const void* wp_down, float* partial, int rows, int d, int I, int* ksplit_io,
                           bool row_major, void* stream);
+// fstu_linear.hip: an fp32 projection (or gated pair) behind the residual add and RMSNorm of its rows
+bool fstu_linear_f32_norm_ok(int rows, int K);
+int fstu_linear_f32_norm(const void* x, const float* delta, int nslices, void* x_out, const void* norm_w, float eps, const void* W,
+                         const void* W2, void* y, int ldy, int rows, int N, int K, void* stream);
 bool fstu_linear_rows32_ok(const void* x, int ldx, const void* W, int K, int dtype);
 int fstu_linear_rows32(const void* x, int ldx, const void* W, void* y, int ldy, int rows, int N, int K, float temperature,
                        void* best_ws /*NULL: plain projection; else the head's packed maxima, rows*64 words*/, void* stream);

@@ -1,6 +1,7 @@
 // Host-side driver of one decode step: the launch sequence over the layer
 // stack, with every residual add fused into the RMSNorm that follows it.
 #include "fstu_common.h"
+#include <utility>
 
 #define STEP(call)          \
   do {                      \
@@ -315,6 +316,31 @@ static int decode_step_impl(const fstu_model_desc* m, const int64_t* tok_in, int
     const fstu_layer_desc& L = m->layers[l];
     merge_norm = gate(L) && up(L) && down(L) && (L.kind == 0 || qkv(L));
   }
+  // fp32, one or two rows: a sub-layer's output joins the stream in the projection behind it, which normalises the sum.  (Not the
+  // history step's, up to 32 slices a row that every wave would read again: 1 row, 300 positions behind, 64 tokens 5.1 ms without, 6.4
+  // with it, 6.5 with all norms as launches of their own; four rows 7.2 / 7.2 / 6.8.)
+  bool merge_f32 = dt == FSTU_F32 && m->x2 && fstu_linear_f32_norm_ok(B, d) && fstu_aligned(m->x, 16) && fstu_aligned(m->x2, 16) &&
+                   fstu_aligned(m->partial, 16) && fstu_aligned(m->y, 16);
+  for (int l = 0; l < m->n_layers && merge_f32; ++l) {
+    const fstu_layer_desc& L = m->layers[l];
+    merge_f32 = fstu_aligned(L.norm1_w, 16) && fstu_aligned(L.mlp_norm_w, 16) && fstu_aligned(L.w_gate, 16) && fstu_aligned(L.w_up, 16) &&
+                fstu_aligned(L.kind == 0 ? L.m_inputs_t : L.w_qkv, 16);
+  }
+  int pending_f32 = 0;           // slices in m->partial of the previous layer's MLP output, not yet added
+  // the layer's first projection
+  auto first = [&](const fstu_layer_desc& L, const void* W, void* y, int ldy, int N) -> int {
+    if (!pending_f32) return fstu_linear_decode(m->h, d, W, y, ldy, B, N, d, dt, stream);
+    const int rc = fstu_linear_f32_norm(xc, (const float*)m->partial, pending_f32, xo, L.norm1_w, m->eps, W, nullptr, y, ldy, B, N, d, stream);
+    std::swap(xc, xo);
+    pending_f32 = 0;
+    return rc;
+  };
+  // the gated pair behind the sub-layer's output
+  auto glu_f32 = [&](const fstu_layer_desc& L) -> int {
+    const int rc = fstu_linear_f32_norm(xc, (const float*)m->y, 1, xo, L.mlp_norm_w, m->eps, L.w_gate, L.w_up, m->act, I, B, I, d, stream);
+    std::swap(xc, xo);
+    return rc;
+  };
   bool pending_slices = false;   // m->partial holds 4 slices of the previous layer's MLP output, not yet added
   for (int l = 0; l < m->n_layers; ++l) {
     const fstu_layer_desc& L = m->layers[l];
@@ -322,7 +348,7 @@ static int decode_step_impl(const fstu_model_desc* m, const int64_t* tok_in, int
     if (L.kind == 0) {
       if (m->stu_mode == 0) {
         char* row = (char*)L.hist + (size_t)pos * d * esz;  // hist[:, pos, :] with row stride hist_cap*d
-        TIMED(PC_PROJ, fstu_linear_decode(m->h, d, L.m_inputs_t, row, m->hist_cap * d, B, d, d, dt, stream));
+        TIMED(PC_PROJ, first(L, L.m_inputs_t, row, m->hist_cap * d, d));
         int ns = hist_nsplit(pos + 1, m->hist_nsplit_max);
         TIMED(PC_STU, fstu_stu_step_hist(L.hist, L.filt, m->eo, B, d, pos, m->hist_cap, m->L, ns, dt, stream));
         TIMED(PC_NORM, fstu_add_rmsnorm(xc, m->eo, 2, ns, m->single_branch, L.mlp_norm_w, m->h, B, d, m->eps, dt, stream));
@@ -338,7 +364,7 @@ static int decode_step_impl(const fstu_model_desc* m, const int64_t* tok_in, int
                                                  L.lds_fir ? m->lds_fir_taps : 0, m->y, d, nullptr, B, m->lds_S, d, d, stu_pos(pos),
                                                  stu_dyn(dyn), dyn, stream));
         } else {
-          TIMED(PC_PROJ, fstu_linear_decode(m->h, d, L.m_inputs_t, m->xp, d, B, d, d, dt, stream));
+          TIMED(PC_PROJ, first(L, L.m_inputs_t, m->xp, d, d));
           TIMED(PC_STU, stu_step(L, m, stu_pos(pos), stu_dyn(dyn), dyn, stream));
         }
         pending_y = true;
@@ -351,14 +377,16 @@ static int decode_step_impl(const fstu_model_desc* m, const int64_t* tok_in, int
       } else if (glu_bal && L.wp_qkv)
         TIMED(PC_PROJ, fstu_linear_packed(m->h, d, nullptr, 0.f, L.wp_qkv, m->qkv, 3 * d, B, 3 * d, d, stream));
       else
-        TIMED(PC_PROJ, fstu_linear_decode(m->h, d, L.w_qkv, m->qkv, 3 * d, B, 3 * d, d, dt, stream));
+        TIMED(PC_PROJ, first(L, L.w_qkv, m->qkv, 3 * d, 3 * d));
       TIMED(PC_SWA, fstu_swa_decode_impl(m->qkv, L.kring, L.vring, m->attn, L.slopes, B, m->n_heads, m->head_dim,
                                          m->kv_cap, pos, m->window, m->softcap, 1, dyn, dt, stream));
       TIMED(PC_PROJ, fstu_linear_decode(m->attn, d, L.w_proj, m->y, d, B, d, d, dt, stream));
       pending_y = true;
     }
     const void* next_w = (l + 1 < m->n_layers) ? m->layers[l + 1].norm1_w : m->final_norm_w;
-    if (pending_y && glu_bal && m->x2 && gate(L) && up(L)) {
+    if (merge_f32 && pending_y) {
+      TIMED(PC_GLU, glu_f32(L));
+    } else if (pending_y && glu_bal && m->x2 && gate(L) && up(L)) {
       // residual add + mlp_norm as the prologue of the balanced gate/up launch; the stream moves to the other buffer
       TIMED(PC_GLU, fstu_glu_norm_impl(xc, m->y, xo, L.mlp_norm_w, m->eps, gate(L), up(L), m->act, I, B, I, d, rm, stream));
       void* t = xc; xc = xo; xo = t;
@@ -385,7 +413,8 @@ static int decode_step_impl(const fstu_model_desc* m, const int64_t* tok_in, int
       nsl = m->ksplit_down;
       TIMED(PC_DOWN, fstu_linear_decode_splitk(m->act, I, L.w_down, m->partial, B, d, I, m->ksplit_down, dt, stream));
     }
-    TIMED(PC_NORM, fstu_add_rmsnorm(xc, m->partial, 1, nsl, 0, next_w, m->h, B, d, m->eps, dt, stream));
+    if (merge_f32 && l + 1 < m->n_layers) pending_f32 = nsl;
+    else TIMED(PC_NORM, fstu_add_rmsnorm(xc, m->partial, 1, nsl, 0, next_w, m->h, B, d, m->eps, dt, stream));
   }
   if (logits_only) {
     TIMED(PC_HEAD, fstu_linear_decode(m->h, d, m->emb, m->logits, m->V, B, m->V, d, dt, stream));

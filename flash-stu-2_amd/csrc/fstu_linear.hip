@@ -237,10 +237,23 @@ linear_valu_kernel(LinArgs a) {
 // waves to an atomic).
 // Waves per workgroup: the head's are large, as every workgroup costs an atomic per row
 template <int MODE, int RB> __host__ __device__ constexpr int f32_waves() { return MODE != LIN_ARGMAX ? 4 : RB <= 8 ? 16 : 8; }
-template <int MODE, int RB, int NF, int U>
-__global__ void __launch_bounds__((f32_waves<MODE, RB>() * 64))
-linear_f32_kernel(const float* x, const float* W, const float* W2, float* y, unsigned long long* best, int ldx, int ldy, int rows,
-                  int N, int K, int kw, float temperature) {
+//
+// linear_f32_norm_kernel (NORM; rows of K <= 256 U, dense): the activations are RMSNorm(x + delta) * norm_w, delta the sum of fp32 slices (rows, K) in their
+// order, formed by every wave in the registers that its product reads them from; the first wave of the launch stores x + delta.
+// That takes the add+norm launch out from between two projections, whose waves read 1 KB per row and slice more from the L2: the
+// small fp32 model's step of 29 launches, which the host enqueues more slowly than the GPU runs them, has 24 (64 + 64 tokens of one
+// row 6.5 -> 5.5 ms).
+constexpr int F32_NORM_ROWS = 2;
+struct F32Norm {
+  const float* delta;      // nslices x rows x K
+  float* x_out;            // x + delta (not x: other waves still read it)
+  const float* w;
+  float eps;
+  int nslices;
+};
+template <int MODE, int RB, int NF, int U, bool NORM>
+__device__ __forceinline__ void linear_f32_body(const float* x, const float* W, const float* W2, float* y, unsigned long long* best, int ldx,
+                                                int ldy, int rows, int N, int K, int kw, float temperature, const F32Norm& norm) {
   constexpr int NW = (MODE == LIN_GLU) ? 2 : 1, NWV = f32_waves<MODE, RB>();
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int n0 = (blockIdx.x * NWV + w) * NF;
@@ -266,6 +279,47 @@ linear_f32_kernel(const float* x, const float* W, const float* W2, float* y, uns
       }
 #pragma unroll
       for (int b = 0; b < RB; ++b) xv[u][b] = *(const float4*)(x + (size_t)min(b, rows - 1) * ldx + kk);
+    }
+    if constexpr (NORM) {
+      auto add4 = [](float4& a, const float4& c) { a.x += c.x; a.y += c.y; a.z += c.z; a.w += c.w; };
+      const size_t slice = (size_t)rows * K;
+      float4 nw[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int k = u * 256 + lane * 4;
+        nw[u] = *(const float4*)(norm.w + (k < K ? k : 0));
+      }
+#pragma unroll
+      for (int b = 0; b < RB; ++b) {
+        float ss = 0.f;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int k = u * 256 + lane * 4;
+          const float* src = norm.delta + (size_t)min(b, rows - 1) * K + (k < K ? k : 0);
+          float4 dv = *(const float4*)src;
+          for (int s0 = 1; s0 < norm.nslices; s0 += 8) {       // eight requested at a time (beyond the last: the last, dropped)
+            float4 c[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) c[i] = *(const float4*)(src + (size_t)min(s0 + i, norm.nslices - 1) * slice);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+              if (s0 + i >= norm.nslices) c[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+              add4(dv, c[i]);
+            }
+          }
+          float4& v = xv[u][b];
+          add4(v, dv);
+          if (k >= K) v = make_float4(0.f, 0.f, 0.f, 0.f);
+          ss += v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w;
+          if (blockIdx.x == 0 && w == 0 && b < rows && k < K) *(float4*)(norm.x_out + (size_t)b * K + k) = v;
+        }
+        const float rstd = rsqrtf(wave_sum(ss) / (float)K + norm.eps);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          float4& v = xv[u][b];
+          v = make_float4((v.x * rstd) * nw[u].x, (v.y * rstd) * nw[u].y, (v.z * rstd) * nw[u].z, (v.w * rstd) * nw[u].w);
+        }
+      }
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -329,6 +383,18 @@ linear_f32_kernel(const float* x, const float* W, const float* W2, float* y, uns
       if (m != 0ull) atomicMax(best + (size_t)threadIdx.x * 64 + (blockIdx.x & 63), m);
     }
   }
+}
+
+template <int MODE, int RB, int NF, int U>
+__global__ void __launch_bounds__((f32_waves<MODE, RB>() * 64))
+linear_f32_kernel(const float* x, const float* W, const float* W2, float* y, unsigned long long* best, int ldx, int ldy, int rows,
+                  int N, int K, int kw, float temperature) {
+  linear_f32_body<MODE, RB, NF, U, false>(x, W, W2, y, best, ldx, ldy, rows, N, K, kw, temperature, F32Norm{});
+}
+template <int MODE, int RB, int U>
+__global__ void __launch_bounds__(256)
+linear_f32_norm_kernel(const float* x, const float* W, const float* W2, float* y, int ldy, int rows, int N, int K, F32Norm norm) {
+  linear_f32_body<MODE, RB, 1, U, true>(x, W, W2, y, nullptr, K, ldy, rows, N, K, K, 1.0f, norm);
 }
 
 static int check_common(const char* name, const void* x, const void* W, const void* y, int ldx, int rows, int N, int K) {
@@ -429,6 +495,29 @@ static void launch_f32(LinArgs a, int ksplit, hipStream_t s) {
   else if (a.rows <= 4) launch_f32_rows<MODE, 4>(a, ksplit, s);
   else if (a.rows <= 8) launch_f32_rows<MODE, 8>(a, ksplit, s);
   else launch_f32_rows<MODE, 16>(a, ksplit, s);
+}
+
+// y = RMSNorm(x + delta) * norm_w against W (W2: the gated pair), as linear_f32_kernel forms it with NORM.
+bool fstu_linear_f32_norm_ok(int rows, int K) { return rows >= 1 && rows <= F32_NORM_ROWS && K >= 4 && K % 4 == 0 && K <= 512; }
+int fstu_linear_f32_norm(const void* x, const float* delta, int nslices, void* x_out, const void* norm_w, float eps, const void* W,
+                         const void* W2, void* y, int ldy, int rows, int N, int K, void* stream) {
+  FSTU_REQUIRE(x && delta && x_out && norm_w && W && y && x_out != x, FSTU_ENULL, "fstu_linear_f32_norm: null pointer, or x_out is x");
+  FSTU_REQUIRE(fstu_linear_f32_norm_ok(rows, K) && N >= 1 && ldy >= N && nslices >= 1, FSTU_ESHAPE, "fstu_linear_f32_norm: rows=%d N=%d K=%d nslices=%d", rows, N, K, nslices);
+  FSTU_REQUIRE(fstu_aligned(x, 16) && fstu_aligned(delta, 16) && fstu_aligned(x_out, 16) && fstu_aligned(norm_w, 16) && fstu_aligned(W, 16) && fstu_aligned(W2, 16),
+               FSTU_EALIGN, "fstu_linear_f32_norm: pointers must be 16-byte aligned");
+  const F32Norm norm{delta, (float*)x_out, (const float*)norm_w, eps, nslices};
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((N + 3) / 4), dim3(256), 0, (hipStream_t)stream, (const float*)x, (const float*)W, (const float*)W2, (float*)y,
+                       ldy, rows, N, K, norm);
+  };
+#define F32N(RB)                                                                                                                \
+  (W2 ? (K > 256 ? go(linear_f32_norm_kernel<LIN_GLU, RB, 2>) : go(linear_f32_norm_kernel<LIN_GLU, RB, 1>))                      \
+      : (K > 256 ? go(linear_f32_norm_kernel<LIN_PLAIN, RB, 2>) : go(linear_f32_norm_kernel<LIN_PLAIN, RB, 1>)))
+  if (rows == 1) F32N(1);
+  else F32N(2);
+#undef F32N
+  FSTU_CHECK_LAUNCH("fstu_linear_f32_norm");
+  return FSTU_OK;
 }
 
 extern "C" int fstu_linear_decode(const void* x, int ldx, const void* W, void* y, int ldy, int rows, int N, int K,

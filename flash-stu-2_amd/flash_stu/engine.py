@@ -435,6 +435,8 @@ class DecodeEngine:
         m.eo = buf(self.HIST_NSPLIT_MAX, 2, B, d, dtype=torch.float32).data_ptr()
         m.logits = ch.logits.data_ptr()
         m.best = buf(32 * 64, dtype=torch.int64).data_ptr()
+        if dt == torch.float32:
+            m.x2 = buf(B, d).data_ptr()         # the stream behind the norms that a projection forms itself
         m.samp_ws = buf((int(self.lib.fstu_sample_ws_bytes()) + 7) // 8, dtype=torch.int64).data_ptr()
         if dt == torch.bfloat16 and self.lib.fstu_glu_packed_supported(B, d, I):
             # gate/up projection over packed weights, one workgroup per CU with equal bytes each

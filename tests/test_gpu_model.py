@@ -769,6 +769,28 @@ def test_one_call_step_on_the_parameters_themselves(d, scale, rows, mode):
     assert float((got - want).abs().max()) <= 2e-2 * float(want.abs().max())
 
 
+@pytest.mark.parametrize("d,rows,extra", [(64, 1, {}), (64, 5, {}), (192, 2, dict(stu_decode_mode="lds")), (256, 2, {}), (288, 1, dict(use_hankel_L=True)),
+                                          (320, 3, {}), (512, 2, dict(stu_decode_mode="lds")), (512, 1, {}), (544, 2, {})])
+def test_fp32_step_with_its_norms_in_the_projections(d, rows, extra):
+    """One and two fp32 rows of up to 512 features: the projections normalise the stream themselves (544 features and more rows keep
+    the launches of their own), histories of 1 to 16 slices, against the layers' own calls: the bounds of the fp32 step."""
+    _, _, model = make_pair(seed=5, init="healthy", dtype=torch.float32, mlp_scale=3, n_embd=d, n_layers=4, n_heads=d // 32, window_size=8,
+                            num_eigh=8, seq_len=320, vocab_size=777, **extra)
+    ids = prompt(rows, 300, 777, 3).cuda()
+
+    def run(first, count):
+        past, logits = model(ids[:, :first], use_cache=True).past_key_values, []
+        for t in range(first, first + count):
+            out = model(ids[:, t:t + 1], past_key_values=past, use_cache=True)
+            past = out.past_key_values
+            logits.append(out.logits)
+        return torch.cat(logits, 1)
+    got = [run(3, 3), run(70, 2), run(290, 2)]
+    model.layers[0].mlp.register_forward_hook(lambda *a: None)     # the layers' own calls run
+    for a, b in zip(got, [run(3, 3), run(70, 2), run(290, 2)]):
+        assert float((a - b).abs().max()) <= 1e-4 * float(b.abs().max())
+
+
 def test_forward_accepts_reference_style_kv_cache():
     from flash_stu import Attention, FlashSTUConfig
     cfg = FlashSTUConfig(n_embd=128, n_heads=2, n_layers=2, seq_len=64, window_size=6, vocab_size=11, mlp_scale=2,
