@@ -951,14 +951,14 @@ __device__ __forceinline__ float key16_f32(unsigned k16) {
 __global__ void __launch_bounds__(256)
 sample_topk_kernel(const bf16_t* __restrict__ logits, int64_t ldl, unsigned long long* __restrict__ best,
                    SampWs* __restrict__ ws, int64_t* __restrict__ out, int64_t out_stride, int V, float temperature, int top_k,
-                   float top_p, uint64_t seed, int step, int row0, int* __restrict__ dyn, int advance) {
+                   float top_p, uint64_t seed, int step, int row0, int* __restrict__ dyn, int advance, int nrows) {
   __shared__ SampleShared sh;
   __shared__ int s_wtot[4], s_last, s_n, s_over;
   __shared__ int s_off[SAMP_MAX_CHUNKS + 1];
   __shared__ unsigned short c_idx[SAMP_MAX_CHUNKS * SAMP_CHUNK_CAP], c_key[SAMP_MAX_CHUNKS * SAMP_CHUNK_CAP];
   __shared__ float c_e[SAMP_MAX_CHUNKS * SAMP_CHUNK_CAP];
   __shared__ unsigned long long c_mass[SAMP_MAX_CHUNKS * SAMP_CHUNK_CAP];
-  const int b = blockIdx.y, g = blockIdx.x, G = gridDim.x, nrows = gridDim.y;
+  const int b = blockIdx.y, g = blockIdx.x, G = (V + SAMP_CHUNK - 1) / SAMP_CHUNK;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   int pos_off = 0;
   if (dyn) { pos_off = dyn[0]; step = dyn[1]; }
@@ -1229,7 +1229,7 @@ int fstu_sample_topk_dyn(const void* logits, int64_t ldl, void* best_ws, void* s
   const dim3 grid((V + SAMP_CHUNK - 1) / SAMP_CHUNK, B);
   hipLaunchKernelGGL(sample_topk_kernel, grid, dim3(256), 0, (hipStream_t)stream, (const bf16_t*)logits, ldl,
                      (unsigned long long*)best_ws, (SampWs*)samp_ws, out, out_stride, V, temperature, top_k, top_p, seed, step, row0,
-                     dyn, advance);
+                     dyn, advance, B);
   FSTU_CHECK_LAUNCH("fstu_sample_topk");
   return FSTU_OK;
 }

@@ -2,6 +2,7 @@
 // CU with equal bytes each: the gate/up projection with the GLU epilogue (and the QKV / plain projections on the same
 // launch), optionally with the sub-layer's residual add + RMSNorm as its prologue, and the split-K down projection
 // (flash_stu/modules/swiglu.py:22-29, flash_stu/layers/stu_layer.py:93-96, flash_stu/layers/attention_layer.py:59-62).
+#include <atomic>
 #include <type_traits>
 #include "fstu_common.h"
 #include "fstu_prologue.h"
@@ -112,7 +113,8 @@ struct GluArgs {
   const uint4* wp_gate;
   const uint4* wp_up;
   bf16_t* act;
-  int rows, d, I, ldh, ldact, fpw;
+  int rows, d, I, ldh, ldact;
+  int wgs;                // workgroups of the launch (gridDim would add 256 bytes of launch arguments, and a load of them)
   // prologue (PRO): h = rmsnorm(T(x_in + delta)) * norm_w computed by every workgroup; workgroup 0 stores the sum
   // (PRO 2: delta = up to 4 fp32 split-K slices of (rows x d), summed in order and rounded before the add)
   const bf16_t* x_in;
@@ -140,10 +142,10 @@ template <int KSA, int PRO, int EPI, int NB = 1, bool RM = false>
 __global__ void __launch_bounds__(512)
 glu_balanced_kernel(const bf16_t* h, const uint4* wp_gate, const uint4* wp_up, bf16_t* act, const bf16_t* x_in,
                     const void* delta, bf16_t* x_out, const bf16_t* norm_w, int rows, int d, int I, int ldh, int ldact,
-                    int fpw, float eps, int nslices, unsigned long long* best, float temperature) {
+                    int wgs, float eps, int nslices, unsigned long long* best, float temperature) {
   GluArgs a;
   a.h = h; a.wp_gate = wp_gate; a.wp_up = wp_up; a.act = act; a.rows = rows; a.d = d; a.I = I; a.ldh = ldh; a.ldact = ldact;
-  a.fpw = fpw; a.x_in = x_in; a.delta = delta; a.x_out = x_out; a.norm_w = norm_w; a.eps = eps; a.nslices = nslices;
+  a.wgs = wgs; a.x_in = x_in; a.delta = delta; a.x_out = x_out; a.norm_w = norm_w; a.eps = eps; a.nslices = nslices;
   a.best = best; a.temperature = temperature;
   constexpr bool GLU = EPI == 0;
   constexpr int DA = KSA <= 3 ? 4 : (KSA == 4 ? 3 : 2);
@@ -161,17 +163,11 @@ glu_balanced_kernel(const bf16_t* h, const uint4* wp_gate, const uint4* wp_up, b
   uint4 xa2[NB == 2 ? KSA : 1];                               // B fragments of rows 16..31
   const int nchunk = a.d >> 3, total = a.rows * nchunk;
   // weight addressing
-  // Features are dealt out in groups of 8 (a.fpw == 0): with the packed layout a group of 8 rows is one whole 128-byte
+  // Features are dealt out in groups of 8: with the packed layout a group of 8 rows is one whole 128-byte
   // line per k group, so no line is shared with (and fetched again by) the neighbouring workgroup on another XCD.
-  int f0, f1;
-  if (a.fpw > 0) {
-    f0 = wgi * a.fpw;
-    f1 = min(a.I, f0 + a.fpw);
-  } else {
-    const long long ngr = (a.I + 7) >> 3;
-    f0 = (int)(ngr * wgi / gridDim.x) * 8;
-    f1 = min(a.I, (int)(ngr * (wgi + 1) / gridDim.x) * 8);
-  }
+  const unsigned ngr = (unsigned)(a.I + 7) >> 3;              // (times the workgroups: below 2^32 for every I the launch takes)
+  const int f0 = (int)(ngr * (unsigned)wgi / (unsigned)a.wgs) * 8;
+  const int f1 = min(a.I, (int)(ngr * (unsigned)(wgi + 1) / (unsigned)a.wgs) * 8);
   const int ta0 = f0 >> 4, ta1 = (f1 > f0) ? ((f1 + 15) >> 4) : ta0;
   const size_t tsa = (size_t)(a.d >> 5) * 64;
   const size_t wa_bytes = RM ? (size_t)a.I * a.d * 2 : (size_t)((a.I + 15) >> 4) * tsa * 16;
@@ -653,27 +649,37 @@ extern "C" int fstu_mlp_packed_rows32_supported(int rows, int d, int I) {
          I % 512 == 0 && (size_t)rows * I * 2 < 0x7ff00000ull;
 }
 
+// Raises a kernel's limit of dynamic LDS where a launch needs more than any before it did
+static int allow_lds(const void* kernel, std::atomic<size_t>& most, size_t shm, const char* name) {
+  if (shm <= most.load(std::memory_order_relaxed)) return FSTU_OK;
+  hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
+  FSTU_REQUIRE(e == hipSuccess, (int)e, "%s: %zu bytes of dynamic LDS refused", name, shm);
+  most.store(shm, std::memory_order_relaxed);
+  return FSTU_OK;
+}
+
 template <int KSA>
 static int glu_launch_ksa(GluArgs& a, int pro, int epi, int G, size_t shm, const char* name, hipStream_t s, bool row_major) {
   if constexpr (KSA <= 4) if (row_major) {       // 1..16 rows behind a norm prologue, widths up to 1024
-    auto go = [&](auto kernel) -> int {
-      hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
-      FSTU_REQUIRE(e == hipSuccess, (int)e, "%s: %zu bytes of dynamic LDS refused", name, shm);
+    auto go = [&](auto which) -> int {              // (a type for each kernel: a record of its own)
+      constexpr auto kernel = decltype(which)::value;
+      static std::atomic<size_t> most{0};
+      const int rc = allow_lds(reinterpret_cast<const void*>(kernel), most, shm, name);
+      if (rc) return rc;
       hipLaunchKernelGGL(kernel, dim3(G), dim3(512), shm, s, a.h, a.wp_gate, a.wp_up, a.act, a.x_in, a.delta, a.x_out, a.norm_w, a.rows,
-                         a.d, a.I, a.ldh, a.ldact, a.fpw, a.eps, a.nslices, a.best, a.temperature);
+                         a.d, a.I, a.ldh, a.ldact, a.wgs, a.eps, a.nslices, a.best, a.temperature);
       return FSTU_OK;
     };
-    return pro == 2 ? go(glu_balanced_kernel<KSA, 2, 1, 1, true>) : go(glu_balanced_kernel<KSA, 1, 0, 1, true>);
+    return pro == 2 ? go(std::integral_constant<decltype(&glu_balanced_kernel<KSA, 2, 1, 1, true>), glu_balanced_kernel<KSA, 2, 1, 1, true>>{})
+                    : go(std::integral_constant<decltype(&glu_balanced_kernel<KSA, 1, 0, 1, true>), glu_balanced_kernel<KSA, 1, 0, 1, true>>{});
   }
 #define GLU_GO(PRO, GLUF)                                                                                        \
   do {                                                                                                           \
-    if (shm > 0) {                                                                                               \
-      hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(glu_balanced_kernel<KSA, PRO, GLUF>),     \
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);                  \
-      FSTU_REQUIRE(e == hipSuccess, (int)e, "%s: %zu bytes of dynamic LDS refused", name, shm);                  \
-    }                                                                                                            \
+    static std::atomic<size_t> most{0};                                                                          \
+    const int rc = allow_lds(reinterpret_cast<const void*>(glu_balanced_kernel<KSA, PRO, GLUF>), most, shm, name); \
+    if (rc) return rc;                                                                                           \
     hipLaunchKernelGGL((glu_balanced_kernel<KSA, PRO, GLUF>), dim3(G), dim3(512), shm, s, a.h, a.wp_gate, a.wp_up, a.act, a.x_in,    \
-                       a.delta, a.x_out, a.norm_w, a.rows, a.d, a.I, a.ldh, a.ldact, a.fpw, a.eps, a.nslices, a.best, a.temperature); \
+                       a.delta, a.x_out, a.norm_w, a.rows, a.d, a.I, a.ldh, a.ldact, a.wgs, a.eps, a.nslices, a.best, a.temperature); \
   } while (0)
   if (a.rows > FSTU_MAX_DECODE_ROWS) {
     // two row tiles: the partial sums of both lie in dynamic LDS
@@ -687,7 +693,7 @@ static int glu_launch_ksa(GluArgs& a, int pro, int epi, int G, size_t shm, const
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)red2);               \
     FSTU_REQUIRE(attr_err == hipSuccess, (int)attr_err, "%s: %zu bytes of dynamic LDS refused", name, red2);               \
     hipLaunchKernelGGL((glu_balanced_kernel<KSA, PRO, EPI, 2>), dim3(G), dim3(512), red2, s, a.h, a.wp_gate, a.wp_up, a.act, \
-                       a.x_in, a.delta, a.x_out, a.norm_w, a.rows, a.d, a.I, a.ldh, a.ldact, a.fpw, a.eps, a.nslices, a.best,  \
+                       a.x_in, a.delta, a.x_out, a.norm_w, a.rows, a.d, a.I, a.ldh, a.ldact, a.wgs, a.eps, a.nslices, a.best,  \
                        a.temperature);                                                                                      \
   } while (0)
     if (pro == 3 && epi == 0) GLU_GO2(3, 0);
@@ -723,7 +729,7 @@ static int glu_launch(GluArgs& a, int pro, int epi, const char* name, hipStream_
   // workgroup rather than half tiles on every CU: every workgroup repeats the norm prologue, and its operands come
   // out of one L2 per XCD
   if (epi != 0 && G > (a.I + 15) / 16) G = (a.I + 15) / 16;
-  a.fpw = 0;
+  a.wgs = G;
   const size_t shm = (pro == 1 || pro == 2) ? (size_t)a.rows * (a.d + 8) * 2 : 0;
   int rc;
   switch (a.d / 256) {

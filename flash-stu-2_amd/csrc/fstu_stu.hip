@@ -600,7 +600,8 @@ stu_inproj_step_kernel(const bf16_t* __restrict__ h, const bf16_t* __restrict__ 
   // XCDs, so consecutive tiles are dealt to one XCD (workgroups i, i+8, ...): both halves of a line then meet in the
   // same L2 and the line comes from HBM once instead of twice.
   int tile = blockIdx.x;
-  if ((gridDim.x & 15) == 0) tile = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+  const int ntiles = (d + 15) >> 4;      // the grid's width (gridDim would add 256 bytes of launch arguments, and a load of them)
+  if ((ntiles & 15) == 0) tile = (blockIdx.x & 7) * (ntiles >> 3) + (blockIdx.x >> 3);
   const int c0 = tile * 16;
   const int b0 = blockIdx.y * INPROJ_RB, rows = min(INPROJ_RB, B - b0);
   // residual update + norm of this workgroup's rows in the prologue
