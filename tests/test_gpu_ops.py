@@ -1628,6 +1628,28 @@ def test_argument_errors_do_not_launch(hip):
                        torch.zeros(2, device="cuda"), 3, 8, 50.0)
 
 
+@pytest.mark.parametrize("softcap", [0.0, 30.0])
+@pytest.mark.parametrize("B,H,hd,W,T,slope", [(1, 2, 64, 0, 70, 0.5), (2, 3, 64, 31, 129, 0.0), (1, 2, 64, 200, 333, 2.0), (1, 2, 128, 33, 290, 0.01),
+                                              (2, 1, 128, 500, 400, 1.0), (1, 1, 128, 64, 1, 0.3), (1, 2, 64, 95, 64, -0.2)])
+def test_swa_prefill_maxima_and_masks(hip, B, H, hd, W, T, slope, softcap):
+    """Blocks with and without hidden keys, maxima that rise in every block (steep slopes) and never again (one early key above all),
+    against float64: exponents of at most 100 on fp32 (2^-17 of a probability), P in two bf16 parts (2^-17), T fp32 sums, one rounding."""
+    g = gen(W + T)
+    qkv = torch.randn(B, T, 3 * H * hd, generator=g)
+    qkv[:, :1, H * hd: 2 * H * hd] *= 3
+    qkv = qkv.bfloat16()
+    slopes = torch.full((H,), slope)
+    q, k, v = (t.double().view(B, T, H, hd).transpose(1, 2) for t in qkv.chunk(3, 2))
+    s = q @ k.transpose(-1, -2).contiguous() * hd ** -0.5
+    s = softcap * torch.tanh(s / softcap) if softcap else s
+    dist = torch.arange(T)[None, :] - torch.arange(T)[:, None]
+    s = (s + slope * dist).masked_fill((dist > 0) | (dist < -W), float("-inf"))
+    p = s.softmax(-1)
+    want, mag = ((p @ t).transpose(1, 2).reshape(B, T, H * hd) for t in (v, v.abs()))
+    got = hip.swa_prefill(dev(qkv), dev(slopes), H, W, softcap).cpu().double()
+    assert bool(((got - want).abs() <= 2.0 ** -8 * want.abs() + (3 * 2.0 ** -17 + T * 2.0 ** -24) * mag + 1e-30).all())
+
+
 @pytest.mark.parametrize("B,H,hd,W,T", [(2, 4, 64, 16, 50), (2, 12, 64, 512, 700), (1, 4, 128, 32, 100),
                                          (1, 2, 64, 1000, 333), (1, 2, 128, 64, 17)])
 def test_swa_prefill_mfma(hip, B, H, hd, W, T):
