@@ -969,6 +969,21 @@ extern "C" int fstu_gemm_bf16_slices(int M, int N, int K, int nbatch) {
   return best;
 }
 
+// Rows of a plain or residual product that whole rounds of 256 x 256 tiles take (0: no split).  A last round of few large tiles
+// costs nearly what a full one does; its rows by themselves run in slices of K or on small tiles, of which the chip holds as many at
+// once as there are compute units.  us in one launch / split, rows x features x K: 9600 x 2048 x 24576 970 / 743, 8500 x 2048 x 24576
+// 1029 / 590, 17000 x 2048 x 24576 1490 / 1152, 22500 x 768 x 9216 409 / 237, 3000 x 6144 x 2048 83 / 65, 10240 x 2048 x 2048 81 /
+// 73, 22500 x 768 x 768 42 / 37, 33000 x 512 x 512 31 / 28.  The line: 12288 x 2048 x 24576 (512 small tiles left) 962 / 953, below K
+// = 2048 26000 x 768 x 768 (204) 38.5 / 39.3, 18500 x 1024 x 1024 (136) 44.9 / 43.1.
+extern "C" int fstu_gemm_bf16_head_rows(int M, int N, int K) {
+  if (M <= 256 || N < 256 || N % 4 != 0 || K % 64 != 0 || K < 512) return 0;
+  const long long cus = gemm_cus(), nt = (N + 255) / 256, tiles = (long long)((M + 255) / 256) * nt;
+  const long long head = tiles / cus * cus / nt * 256;
+  if (head <= 0 || head >= M) return 0;
+  const long long left = (M - head + 127) / 128 * ((N + 127) / 128);
+  return left <= (K < 2048 ? cus / 2 : cus) ? (int)head : 0;
+}
+
 extern "C" int fstu_gemm_bf16(const void* A, int64_t lda, const void* W, const void* W2, const void* R, int64_t ldr, void* C,
                               int64_t ldc, int M, int N, int K, int mode, void* stream) {
   return fstu_gemm_bf16_ws(A, lda, W, W2, R, ldr, C, ldc, M, N, K, mode, nullptr, 1, stream);

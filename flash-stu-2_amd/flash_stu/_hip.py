@@ -103,6 +103,7 @@ SIGNATURES = {
     "fstu_gemm_bf16_splitk": [_vp, _i64, _vp, _vp, _i, _i, _i, _i, _vp],
     "fstu_gemm_any": [_vp, _i64, _i64, _vp, _i64, _i64, _vp, _i64, _i, _i, _i, _i, _vp],
     "fstu_gemm_bf16_slices": [_i, _i, _i, _i],
+    "fstu_gemm_bf16_head_rows": [_i, _i, _i],
     "fstu_gemm_bf16_ws": [_vp, _i64, _vp, _vp, _vp, _i64, _vp, _i64, _i, _i, _i, _i, _vp, _i, _vp],
     "fstu_gemm_bf16_ta_ws": [_vp, _i64, _i64, _vp, _vp, _i64, _i64, _vp, _i64, _i64, _i, _i, _i, _i, _i, _vp, _i, _vp],
     "fstu_gemm_bf16_ta": [_vp, _i64, _i64, _vp, _vp, _i64, _i64, _vp, _i64, _i64, _i, _i, _i, _i, _i, _vp],
@@ -310,6 +311,11 @@ def _gemm_slices(M: int, N: int, K: int, nbatch: int) -> int:
     return load().fstu_gemm_bf16_slices(M, N, K, nbatch)
 
 
+@functools.lru_cache(maxsize=256)
+def _gemm_head_rows(M: int, N: int, K: int) -> int:
+    return load().fstu_gemm_bf16_head_rows(M, N, K)
+
+
 def gemm(x2: torch.Tensor, weight: torch.Tensor, up_weight: Optional[torch.Tensor] = None,
          residual: Optional[torch.Tensor] = None, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """x2 (M,K) @ weight (N,K)^T on the matrix cores (bf16).  up_weight: the gated pair
@@ -338,6 +344,18 @@ def gemm(x2: torch.Tensor, weight: torch.Tensor, up_weight: Optional[torch.Tenso
         if residual.shape != (M, N) or residual.stride(1) != 1 or residual.dtype != x2.dtype:
             raise FlashSTUHipError("gemm: residual must be (M,N) with contiguous rows")
         mode, ldr = 2, residual.stride(0)
+    head = _gemm_head_rows(M, N, K) if mode != 1 and M > 256 else 0
+    if head:
+        for rows in (slice(0, head), slice(head, M)):
+            _gemm_rows(x2[rows], weight, None, None if residual is None else residual[rows], out[rows], mode, ldr)
+    else:
+        _gemm_rows(x2, weight, up_weight, residual, out, mode, ldr)
+    return out
+
+
+def _gemm_rows(x2, weight, up_weight, residual, out, mode: int, ldr: int) -> None:
+    """One product of checked operands, its K in slices where those pay."""
+    (M, K), N = x2.shape, weight.shape[0]
     slices, partial = 1, None
     if K >= GEMM_MIN_SLICED_K and mode != 1 and out.stride(0) % 4 == 0 and out.data_ptr() % 8 == 0:
         slices = _gemm_slices(M, N, K, 1)
@@ -345,7 +363,6 @@ def gemm(x2: torch.Tensor, weight: torch.Tensor, up_weight: Optional[torch.Tenso
             partial = torch.empty(slices, M, N, dtype=torch.float32, device=x2.device)
     _check(load().fstu_gemm_bf16_ws(_p(x2), x2.stride(0), _p(weight), _p(up_weight), _p(residual), ldr, _p(out), out.stride(0),
                                     M, N, K, mode, _p(partial), slices, _stream()), "fstu_gemm_bf16")
-    return out
 
 
 def gemm_any(a: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:

@@ -446,6 +446,8 @@ int fstu_gemm_bf16_ta(const void* A, int64_t lda, int64_t batch_stride_a, const 
  * second launch adds in order.  fstu_gemm_bf16_slices says how many pay (1: none; nbatch = 1 for fstu_gemm_bf16_ws); partial
  * holds ksplit * nbatch * M * N floats, 16-byte aligned. */
 int fstu_gemm_bf16_slices(int M, int N, int K, int nbatch);
+/* Rows in front that fill whole rounds of the large tiles, where the others are faster in a call of their own (0: one call). */
+int fstu_gemm_bf16_head_rows(int M, int N, int K);
 int fstu_gemm_bf16_ws(const void* A, int64_t lda, const void* W, const void* W2, const void* R, int64_t ldr, void* C,
                       int64_t ldc, int M, int N, int K, int mode, float* partial, int ksplit, void* stream);
 int fstu_gemm_bf16_ta_ws(const void* A, int64_t lda, int64_t batch_stride_a, const void* W, const void* R, int64_t ldr,

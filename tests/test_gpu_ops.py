@@ -274,6 +274,23 @@ def test_linear_rows_of_any_stride(hip, N):
         assert bool(((hip.linear(x, W).double() - ref).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("M,N,K,head", [(2049, 8192, 512, 2048), (1820, 8200, 576, 1792), (2176, 8192, 2048, 2048), (2600, 6144, 512, 2560),
+                                        (2304, 8192, 1024, 2048), (2305, 8192, 1024, 0), (2048, 8192, 512, 0)])
+def test_gemm_bf16_whole_rounds_and_the_rest(hip, M, N, K, head):
+    """Rows that fill rounds of large tiles and the others in a call of their own, plain and added to the residual in place, rows of a
+    stride of their own: fp32 sums of exact products stay within K * 2^-24 of the absolute sum, one or two roundings to bf16."""
+    g = gen(M + K)
+    assert hip.load().fstu_gemm_bf16_head_rows(M, N, K) == head
+    A, W = dev(torch.randn(M, K + 8, generator=g).bfloat16())[:, :K], dev(torch.randn(N, K, generator=g).bfloat16())
+    out = dev(torch.randn(M, N + 4, generator=g).bfloat16())[:, :N]
+    R = out.clone()
+    ref = torch.matmul(A.float(), W.float().t().contiguous())     # fp32 on the library: K * 2^-24 of the absolute sum like the kernel's
+    bound = 2 * K * 2.0 ** -24 * torch.matmul(A.float().abs(), W.float().abs().t().contiguous()) + 2.0 ** -8 * ref.abs()
+    assert bool(((hip.gemm(A, W).float() - ref).abs() <= bound).all())
+    hip.gemm(A, W, residual=out, out=out)
+    assert bool(((out.float() - (R.float() + ref)).abs() <= bound + 2.0 ** -8 * (R.float() + ref).abs()).all())
+
+
 @pytest.mark.parametrize("nb,M,N,K,slices", [(1, 128, 132, 4096, 8), (3, 256, 260, 6144, 12), (1, 384, 1024, 3072, 6)])
 def test_gemm_bf16_in_slices(hip, nb, M, N, K, slices):
     """Few output tiles and a long K: both prompt GEMMs in slices of K, plain and with the residual, ragged tiles and strided
