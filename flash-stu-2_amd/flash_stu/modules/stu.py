@@ -123,12 +123,13 @@ class STU(nn.Module):
         return self._cached("spec", params, lambda: _hip.stu_fft_filter(src, n, single_branch=self.use_hankel_L))
 
     def filter_taps(self, T: int) -> torch.Tensor:
-        """The convolution filters as the Toeplitz product reads them for T positions (approx mode, bf16).  One length is kept."""
+        """The convolution filters as the Toeplitz product reads them for T positions, (d,2,S) (approx mode, bf16).  In the place
+        of the spectra: one operand of the convolution is kept, for one length."""
         S = _hip.stu_conv_taps_len(T)
-        hit = self._derived.get("taps")
+        hit = self._derived.get("spec")
         if hit is not None and hit[1].shape[2] != S:
-            self._derived.pop("taps")
-        return self._cached("taps", (self.phi, self.M_filters), lambda: _hip.stu_conv_taps(self.effective_filter(), S))
+            self._derived.pop("spec")
+        return self._cached("spec", (self.phi, self.M_filters), lambda: _hip.stu_conv_taps(self.effective_filter(), S))
 
     def m_inputs_eff(self) -> torch.Tensor:
         """M_inputs as the forward uses it: the parameter itself, or its block-diagonal part when tiling is on."""
