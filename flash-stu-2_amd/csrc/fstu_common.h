@@ -157,13 +157,6 @@ __device__ __forceinline__ float gelu_tanh_f32(float x) {
   return 0.5f * x * (1.0f + tanhf(inner));
 }
 
-// The same for epilogues that round to bf16, on the hardware exp and reciprocal: x (1 + tanh t) / 2 = x / (1 + exp(-2 t)), five
-// full-rate and two quarter-rate instructions (eleven and two as 1 - 2 / (exp(2 t) + 1), which also cancelled for negative x: off
-// by 1.5e-3 of the value at x = -4, 4e-6 so)
-__device__ __forceinline__ float gelu_tanh_fast(float x) {
-  return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x * fmaf(x * x, -0.10294324f, -2.3022082f)));
-}
-
 #define FSTU_DISPATCH_DTYPE(dtype, NAME, ...)                      \
   do {                                                             \
     if ((dtype) == FSTU_F32) {                                     \

@@ -37,6 +37,12 @@ typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
 #define GM_MAX_LD (1 << 22)
 
 __device__ __forceinline__ float rnd_bf16(float v) { return bf16_to_f32(f32_to_bf16(v)); }
+// The tanh-approximated GELU on the hardware exp and reciprocal, x (1 + tanh t) / 2 = x / (1 + exp(-2 t)): five full-rate and two
+// quarter-rate instructions (eleven and two as 1 - 2 / (exp(2 t) + 1), which also cancelled for negative x: off by 1.5e-3 of the
+// value at x = -4, 4e-6 so)
+__device__ __forceinline__ float gelu_tanh_fast(float x) {
+  return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x * fmaf(x * x, -0.10294324f, -2.3022082f)));
+}
 
 // 16 bytes per lane from global memory into LDS without a stop in registers: the 64 lanes fill 64 consecutive 16-byte
 // slots from `l` (wave-uniform) on.  The source is a buffer descriptor (base and range in SGPRs), a 32-bit byte offset

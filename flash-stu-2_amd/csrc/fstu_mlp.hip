@@ -58,6 +58,16 @@ __device__ __forceinline__ float half_wave_sum(float v) {
   return v;
 }
 
+// tanh-approximated GELU with tanh(t) = 1 - 2 / (exp(2t) + 1) on the hardware exp and reciprocal: absolute error of 1 + tanh about
+// 1e-7, far below the bf16 rounding that follows.  (The prompt GEMM's shorter form gains nothing here: a decode launch has two
+// features to a lane and waits for memory.)
+__device__ __forceinline__ float gelu_tanh_fast(float x) {
+  const float inner = 0.7978845608028654f * (x + 0.044715f * x * x * x);
+  const float e = __builtin_amdgcn_exp2f(2.8853900817779268f * inner);   // exp(2 inner)
+  const float th = 1.0f - 2.0f * __builtin_amdgcn_rcpf(e + 1.0f);
+  return 0.5f * x * (1.0f + th);
+}
+
 // rows of `src` (LDS, bf16, stride ld) -> T((v * rstd) * w) into dst (stride ld_dst); wave per row.
 // nwv holds the norm weights of this lane's first four column chunks (c = lane*8 + k*512), loaded early.
 __device__ __forceinline__ void norm_rows(const bf16_t* src, int ld, bf16_t* dst, int ld_dst, const bf16_t* __restrict__ nw,
