@@ -25,6 +25,7 @@
 // fragments then serve half as many each and the LDS becomes the bound (47 us).
 #include "fstu_common.h"
 #include <type_traits>
+#include <algorithm>
 
 namespace {
 
@@ -59,12 +60,13 @@ __device__ __forceinline__ bool cm_place(int d, int rows, int R, int& c0, int& r
   return row0 < rows && c0 < d;
 }
 
-// 8 positions of one parity x 8 channels, dwords [position][channel pair] -> [channel][position pair] or back
-__device__ __forceinline__ void transpose8(const unsigned (&v)[8][4], unsigned (&o)[8][4]) {
+// M positions of one parity x 8 channels, dwords [position][channel pair] -> [channel][position pair], or N channels back
+template <int M, int N>
+__device__ __forceinline__ void transpose8(const unsigned (&v)[M][N / 2], unsigned (&o)[N][M / 2]) {
 #pragma unroll
-  for (int c = 0; c < 8; ++c)
+  for (int c = 0; c < N; ++c)
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < M / 2; ++j)
       o[c][j] = __builtin_amdgcn_perm(v[2 * j + 1][c >> 1], v[2 * j][c >> 1], (c & 1) ? 0x07060302 : 0x05040100);
 }
 
@@ -92,7 +94,7 @@ conv_mfma_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ taps, 
       if (t0 + 2 * e < T && row0 + row < B) q = *(const uint4*)(src + (size_t)(2 * e) * d);
       a[e][0] = q.x; a[e][1] = q.y; a[e][2] = q.z; a[e][3] = q.w;
     }
-    transpose8(a, o);
+    transpose8<8, 8>(a, o);
     char* dst = lds + row * rws + p * rg + 128 + piece_at(mu >> 3, mu & 7);
 #pragma unroll
     for (int c = 0; c < 8; ++c) *(uint4*)(dst + c * 2 * rg) = make_uint4(o[c][0], o[c][1], o[c][2], o[c][3]);
@@ -237,7 +239,7 @@ conv_mfma_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ taps, 
       const uint4 t = *(const uint4*)(src + c * 2 * rg);
       a[c][0] = t.x; a[c][1] = t.y; a[c][2] = t.z; a[c][3] = t.w;
     }
-    transpose8(a, o);
+    transpose8<8, 8>(a, o);
     bf16_t* dst = y + ((size_t)(row0 + rw) * T + t0) * d + c0;
 #pragma unroll
     for (int e = 0; e < 8; ++e)
@@ -251,31 +253,32 @@ conv_mfma_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ taps, 
 // Both are products with the same Hankel matrix of g, A[i][k] = g_p[32 s + 16 r + i + k]: for block c of 64 positions (or lags)
 // and row tile r, B[k][c] = fe[32 s + k - 64 c] gives gx_p[64 c + 16 r + i] and x_p[32 s + k - 64 c] gives gfe[64 c + 16 r + i].
 // Eight of an MFMA's 16 columns are blocks of lags and eight of positions, so both come out of one pass over g, whose shifted
-// copies a wave expands into its ring from g in LDS.  A workgroup has 8 channels, a wave each, and goes through R rows: the sums
-// of the filter's gradient stay in registers, and the next row is on its way while this one is worked on.  What it leaves are
-// its rows' fp32 sums, (chunks of rows, lags, channels), added in the order of the rows by conv_grad_finish_kernel.
+// copies a wave expands into its ring from g in LDS.  The parities of a row meet only in the filter's sums, so an item of work is one
+// parity of one row: 70 KB of LDS at 2048 positions, and a second workgroup on the compute unit works while this one's operands come
+// and its results go.  A workgroup has 8 channels, a wave each, and goes through R items: the sums of the filter's gradient stay in
+// registers, and the next item is on its way while this one is worked on.  What it leaves are its items' fp32 sums, (chunks of
+// items, lags, channels), added in the order of the items by conv_grad_finish_kernel.
 //
-// us, transforms -> this, both launches: 8 x 512 x 768 29 -> 26, 8 x 1024 x 768 51 -> 38, 2 x 2048 x 768 42 -> 26, 8 x 2048 x 768
-// 117 -> 73.  At 2048 positions LDS holds one workgroup, 8 waves: a row takes 16 us, of which the products are 6.4 (384 of them
-// to a wave), 11 with the LDS reads in front of them, and the way in and out 4 that nothing else runs beside.  Both parities
-// interleaved in a wave 10.5, a step's fragments requested a step ahead 11.
-constexpr int cg_rows(int HB) { return 128 * HB + 256; }        // bytes of a parity of g: zeros behind it
+// us, transforms -> whole rows (106 KB, one workgroup to a compute unit) -> this, both launches: 8 x 512 x 768 29 -> 26 -> 22, 8 x 1024 x
+// 768 51 -> 39 -> 32, 2 x 2048 x 768 42 -> 27 -> 25, 8 x 2048 x 768 117 -> 80 -> 62, 8 x 2048 x 2048 - -> 163 -> 128.  A row's products alone
+// are 6.4 us of a compute unit, 11 with the LDS reads in front of them; the latter bound it now.
+constexpr int cg_rows(int HB) { return 128 * HB + 256; }        // bytes of a channel of g: zeros behind it
 
 template <int NT>
-__global__ void __launch_bounds__(512, NT == 1 ? 4 : 2)
+__global__ void __launch_bounds__(512, 4)
 conv_grad_mfma_kernel(const bf16_t* __restrict__ gy, const bf16_t* __restrict__ x, const bf16_t* __restrict__ f, bf16_t* __restrict__ gx,
                       float* __restrict__ part, int B, int T, int L, int d, int R) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
   constexpr int HB = 8 * NT, cap = 64 * HB, rg = cm_region(HB), gg = cg_rows(HB), PC = HB * 16;
-  char* const xl = lds;                                       // 16 regions as in the forward
-  char* const fl = xl + 16 * rg;                              // 8 regions: the even taps
-  char* const gl = fl + 8 * rg;                               // 16 of g, in order
-  char* const rings = gl + 16 * gg;
-  int c0, row0;
-  if (!cm_place(d, B, R, c0, row0)) return;
-  const int tid = threadIdx.x, rows = min(R, B - row0);
-  for (int v = tid; v < 24 * 8; v += 512) *(uint4*)(lds + (v >> 3) * rg + (v & 7) * 16) = make_uint4(0, 0, 0, 0);
-  for (int v = tid; v < 16 * 16; v += 512) *(uint4*)(gl + (v >> 4) * gg + 128 * HB + (v & 15) * 16) = make_uint4(0, 0, 0, 0);
+  char* const xl = lds;                                       // 8 regions as in the forward
+  char* const fl = xl + 8 * rg;                               // 8 more: the even taps
+  char* const gl = fl + 8 * rg;                               // 8 of g, in order
+  char* const rings = gl + 8 * gg;
+  int c0, item0;                                              // item 2 b + p: parity p of row b
+  if (!cm_place(d, 2 * B, R, c0, item0)) return;
+  const int tid = threadIdx.x, end = min(item0 + R, 2 * B);
+  if (tid < 16 * 8) *(uint4*)(lds + (tid >> 3) * rg + (tid & 7) * 16) = make_uint4(0, 0, 0, 0);
+  if (tid < 8 * 16) *(uint4*)(gl + (tid >> 4) * gg + 128 * HB + (tid & 15) * 16) = make_uint4(0, 0, 0, 0);
   if (tid < HB * 8) {
     unsigned a[8][4], o[8][4];
 #pragma unroll
@@ -285,25 +288,26 @@ conv_grad_mfma_kernel(const bf16_t* __restrict__ gy, const bf16_t* __restrict__ 
       if (t < L) v = *(const uint4*)(f + (size_t)t * d + c0);
       a[e][0] = v.x; a[e][1] = v.y; a[e][2] = v.z; a[e][3] = v.w;
     }
-    transpose8(a, o);
+    transpose8<8, 8>(a, o);
 #pragma unroll
     for (int c = 0; c < 8; ++c)
       *(uint4*)(fl + c * rg + 128 + piece_at(tid >> 3, tid & 7)) = make_uint4(o[c][0], o[c][1], o[c][2], o[c][3]);
   }
-  // A thread's piece: 8 positions of one parity of x (the first PC threads) or of g
-  const int piece = tid % PC, mu = piece & (HB * 8 - 1), pp = piece / (HB * 8), t0 = 16 * mu + pp;
+  // A thread's piece: 4 positions of the item's parity of x (the first PC threads) or of g
+  const int mu = tid % PC;
   const bool has = tid < 2 * PC, is_g = tid >= PC;
-  unsigned in[8][4];
-  auto request = [&](int row) {
-    const bf16_t* src = (is_g ? gy : x) + ((size_t)row * T + t0) * d + c0;
+  unsigned in[4][4];
+  auto request = [&](int item) {
+    const int t0 = 8 * mu + (item & 1);
+    const bf16_t* src = (is_g ? gy : x) + ((size_t)(item >> 1) * T + t0) * d + c0;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
+    for (int e = 0; e < 4; ++e) {
       uint4 v = make_uint4(0, 0, 0, 0);
       if (has && t0 + 2 * e < T) v = *(const uint4*)(src + (size_t)(2 * e) * d);
       in[e][0] = v.x; in[e][1] = v.y; in[e][2] = v.z; in[e][3] = v.w;
     }
   };
-  request(row0);
+  request(item0);
 
   const int lane = tid & 63, ch = tid >> 6, col = lane & 15, g = lane >> 4, c = col & 7;
   char* const ring = rings + ch * 2048;
@@ -321,108 +325,105 @@ conv_grad_mfma_kernel(const bf16_t* __restrict__ gy, const bf16_t* __restrict__ 
 #pragma unroll
     for (int r = 0; r < 4; ++r) S[j][r] = (floatx4_t){0.f, 0.f, 0.f, 0.f};
 
-  for (int row = 0; row < rows; ++row) {
+  for (int item = item0; item < end; ++item) {
     if (has) {
-      unsigned o[8][4];
-      transpose8(in, o);
+      unsigned o[8][2];
+      transpose8<4, 8>(in, o);
+      char* const dst = is_g ? gl + mu * 8 : xl + 128 + piece_at(mu >> 4, (mu >> 1) & 7) + (mu & 1) * 8;
 #pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        char* dst = is_g ? gl + (k * 2 + pp) * gg + mu * 16 : xl + (k * 2 + pp) * rg + 128 + piece_at(mu >> 3, mu & 7);
-        *(uint4*)dst = make_uint4(o[k][0], o[k][1], o[k][2], o[k][3]);
-      }
+      for (int k = 0; k < 8; ++k) *(uint2*)(dst + k * (is_g ? gg : rg)) = make_uint2(o[k][0], o[k][1]);
     }
     __syncthreads();
-    if (row + 1 < rows) request(row0 + row + 1);
-    for (int p = 0; p < 2; ++p) {
-      char* const own = gl + (ch * 2 + p) * gg;
-      const char* const bl = (col < 8 ? xl + (ch * 2 + p) * rg : fl + ch * rg) + 128;
-      const char* const win = own + xn * 16 + (xs >> 1) * 4;
-      unsigned w[5];
-      auto window = [&](int P) {
+    if (item + 1 < end) request(item + 1);
+    char* const own = gl + ch * gg;
+    const char* const bl = (col < 8 ? xl : fl) + ch * rg + 128;
+    const char* const win = own + xn * 16 + (xs >> 1) * 4;
+    unsigned w[5];
+    auto window = [&](int P) {
 #pragma unroll
-        for (int k = 0; k < 5; ++k) w[k] = *(const unsigned*)(win + 128 * min(P, HB) + 4 * k);
-      };
-      auto expand = [&](bool oddp) {
-        *(uint4*)(ring + xdst + oddp * 1024) =
-            make_uint4(__builtin_amdgcn_alignbit(w[1], w[0], odd), __builtin_amdgcn_alignbit(w[2], w[1], odd),
-                       __builtin_amdgcn_alignbit(w[3], w[2], odd), __builtin_amdgcn_alignbit(w[4], w[3], odd));
-      };
-      wave_order();
-      window(0);
-      expand(false);
-      window(1);
-      expand(true);
-      window(2);
-      wave_order();
-      uint4 fa[2], fb[2];
-      fa[0] = *(const uint4*)(ring + fat0);
-      fa[1] = *(const uint4*)(ring + fat1);
-      // A pair of steps, 64 positions of g, for the tiles up to J1: fragments of row tiles 0, 1 from the step before, 2, 3 now
-      auto pair = [&](auto last, int P, bool oddp) {
-        constexpr int J1 = decltype(last)::value;
+      for (int k = 0; k < 5; ++k) w[k] = *(const unsigned*)(win + 128 * min(P, HB) + 4 * k);
+    };
+    auto expand = [&](bool oddp) {
+      *(uint4*)(ring + xdst + oddp * 1024) =
+          make_uint4(__builtin_amdgcn_alignbit(w[1], w[0], odd), __builtin_amdgcn_alignbit(w[2], w[1], odd),
+                     __builtin_amdgcn_alignbit(w[3], w[2], odd), __builtin_amdgcn_alignbit(w[4], w[3], odd));
+    };
+    wave_order();
+    window(0);
+    expand(false);
+    window(1);
+    expand(true);
+    window(2);
+    wave_order();
+    uint4 fa[2], fb[2];
+    fa[0] = *(const uint4*)(ring + fat0);
+    fa[1] = *(const uint4*)(ring + fat1);
+    // A pair of steps, 64 positions of g, for the tiles up to J1: fragments of row tiles 0, 1 from the step before, 2, 3 now
+    auto pair = [&](auto last, int P, bool oddp) {
+      constexpr int J1 = decltype(last)::value;
 #pragma unroll
-        for (int s = 0; s < 2; ++s) {
-          uint4 (&old)[2] = s ? fb : fa;
-          uint4 (&now)[2] = s ? fa : fb;
+      for (int s = 0; s < 2; ++s) {
+        uint4 (&old)[2] = s ? fb : fa;
+        uint4 (&now)[2] = s ? fa : fb;
 #pragma unroll
-          for (int k = 0; k < 2; ++k) now[k] = *(const uint4*)(ring + (oddp ? fat[2 * s + k] ^ 1024 : fat[2 * s + k]));
-          uint4 b[NT];
+        for (int k = 0; k < 2; ++k) now[k] = *(const uint4*)(ring + (oddp ? fat[2 * s + k] ^ 1024 : fat[2 * s + k]));
+        uint4 b[NT];
 #pragma unroll
-          for (int j = 0; j <= J1; ++j) b[j] = *(const uint4*)(bl + piece_at(max(P - c - 8 * j, -1), s ? g + 4 : g));
-          if (s == 1) {
-            wave_order();
-            expand(oddp);
-            window(P + 3);
-            wave_order();
-          }
-#pragma unroll
-          for (int j = 0; j <= J1; ++j)
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-              S[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_frag(i < 2 ? old[i] : now[i - 2]), as_frag(b[j]), S[j][i], 0, 0, 0);
+        for (int j = 0; j <= J1; ++j) b[j] = *(const uint4*)(bl + piece_at(max(P - c - 8 * j, -1), s ? g + 4 : g));
+        if (s == 1) {
+          wave_order();
+          expand(oddp);
+          window(P + 3);
+          wave_order();
         }
-      };
-#pragma unroll 1
-      for (int P = 0; P < min(8, blocks); P += 2) {
-        pair(std::integral_constant<int, 0>{}, P, false);
-        pair(std::integral_constant<int, 0>{}, P + 1, true);
-      }
-      if constexpr (NT == 2) {
-#pragma unroll 1
-        for (int P = 8; P < blocks; P += 2) {
-          pair(std::integral_constant<int, 1>{}, P, false);
-          pair(std::integral_constant<int, 1>{}, P + 1, true);
-        }
-      }
-      // this parity's gradient of x takes g's place; its columns start from zero again
 #pragma unroll
-      for (int j = 0; j < NT; ++j)
+        for (int j = 0; j <= J1; ++j)
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (col >= 8) {
-            *(uint2*)(own + ((c + 8 * j) * 64 + 16 * r + 4 * g) * 2) = make_uint2(pack2_bf16(2.f * S[j][r][0], 2.f * S[j][r][1]),
-                                                                                pack2_bf16(2.f * S[j][r][2], 2.f * S[j][r][3]));
-            S[j][r] = (floatx4_t){0.f, 0.f, 0.f, 0.f};
-          }
+          for (int i = 0; i < 4; ++i)
+            S[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_frag(i < 2 ? old[i] : now[i - 2]), as_frag(b[j]), S[j][i], 0, 0, 0);
+      }
+    };
+#pragma unroll 1
+    for (int P = 0; P < min(8, blocks); P += 2) {
+      pair(std::integral_constant<int, 0>{}, P, false);
+      pair(std::integral_constant<int, 0>{}, P + 1, true);
     }
+    if constexpr (NT == 2) {
+#pragma unroll 1
+      for (int P = 8; P < blocks; P += 2) {
+        pair(std::integral_constant<int, 1>{}, P, false);
+        pair(std::integral_constant<int, 1>{}, P + 1, true);
+      }
+    }
+    // this parity's gradient of x takes g's place; its columns start from zero again
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (col >= 8) {
+          *(uint2*)(own + ((c + 8 * j) * 64 + 16 * r + 4 * g) * 2) = make_uint2(pack2_bf16(2.f * S[j][r][0], 2.f * S[j][r][1]),
+                                                                              pack2_bf16(2.f * S[j][r][2], 2.f * S[j][r][3]));
+          S[j][r] = (floatx4_t){0.f, 0.f, 0.f, 0.f};
+        }
     __syncthreads();
+    const int t0 = 8 * mu + (item & 1);
     if (gx && tid < PC && t0 < T) {
-      unsigned a[8][4], o[8][4];
+      unsigned a[8][2], o[4][4];
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
-        const uint4 v = *(const uint4*)(gl + (k * 2 + pp) * gg + mu * 16);
-        a[k][0] = v.x; a[k][1] = v.y; a[k][2] = v.z; a[k][3] = v.w;
+        const uint2 v = *(const uint2*)(gl + k * gg + mu * 8);
+        a[k][0] = v.x; a[k][1] = v.y;
       }
-      transpose8(a, o);
-      bf16_t* dst = gx + ((size_t)(row0 + row) * T + t0) * d + c0;
+      transpose8<8, 4>(a, o);
+      bf16_t* dst = gx + ((size_t)(item >> 1) * T + t0) * d + c0;
 #pragma unroll
-      for (int e = 0; e < 8; ++e)
+      for (int e = 0; e < 4; ++e)
         if (t0 + 2 * e < T) *(uint4*)(dst + (size_t)(2 * e) * d) = make_uint4(o[e][0], o[e][1], o[e][2], o[e][3]);
     }
-    if (row + 1 < rows) __syncthreads();
+    if (item + 1 < end) __syncthreads();
   }
   if (!part) return;
-  // lags of a channel -> channels of a lag, through the space of x
+  // lags of a channel -> channels of a lag, through the space of x and the taps
   float* const fl32 = (float*)xl;
   if (col < 8) {
 #pragma unroll
@@ -432,7 +433,7 @@ conv_grad_mfma_kernel(const bf16_t* __restrict__ gy, const bf16_t* __restrict__ 
   }
   __syncthreads();
   const int lags = min(cap, (min(L, T) + 1) >> 1);
-  float* const out = part + (size_t)(row0 / R) * lags * d + c0;
+  float* const out = part + (size_t)(item0 / R) * lags * d + c0;
   for (int v = tid; v < lags * 2; v += 512) {
     const float* s = fl32 + (v & 1) * 4 * (cap + 4) + (v >> 1);
     *(float4*)(out + (size_t)(v >> 1) * d + (v & 1) * 4) = make_float4(s[0], s[cap + 4], s[2 * (cap + 4)], s[3 * (cap + 4)]);
@@ -472,7 +473,7 @@ conv_taps_kernel(const bf16_t* __restrict__ f, bf16_t* __restrict__ taps, int L,
     if (j >= 0 && s < L) t = *(const uint4*)(f + (size_t)s * d + c0);
     a[e][0] = t.x; a[e][1] = t.y; a[e][2] = t.z; a[e][3] = t.w;
   }
-  transpose8(a, o);
+  transpose8<8, 8>(a, o);
 #pragma unroll
   for (int c = 0; c < 8; ++c)
     *(uint4*)(taps + ((size_t)(c0 + c) * 2 + p) * S + i0) = make_uint4(o[c][0], o[c][1], o[c][2], o[c][3]);
@@ -484,17 +485,16 @@ void cm_shape(int T, int& nbs, int& nt) {
   nt = T <= 1024 ? 1 : T <= 2048 ? 2 : 4;
 }
 
-// Rows a workgroup of the gradients goes through: as many as make its time, one part for the way in and out and one per row, times
-// the rounds of workgroups that the chip runs, the shortest.
-int cg_rows_per_group(int B, int T, int d) {
-  const long long groups = (d + 7) / 8, slots = T <= 1024 ? 512 : 256;
-  int best = 1;
-  long long least = -1;
-  for (int r = 1; r <= B && r <= 64; ++r) {
-    const long long cost = (groups * ((B + r - 1) / r) + slots - 1) / slots * (1 + r);
-    if (least < 0 || cost < least) { least = cost; best = r; }
-  }
-  return best;
+// Items (a row's two parities) that a workgroup of the gradients goes through: the whole row, or more rows where there are more than
+// two workgroups to a compute unit and the parts of the filter's gradient grow; one item where even those leave compute units idle.
+// us with 1 / 2 / 4 / 8 items, rows x positions x channels: 1 x 2000 x 768 18 / 22 / - / -, 4 x 2048 x 256 21.5 / 23.4 / 33 / 60,
+// 2 x 2048 x 768 28 / 25 / 37 / -, 8 x 2048 x 768 70 / 62 / 65 / 68, 8 x 2048 x 2048 206 / 159 / 133 / 124, 5 x 700 x 1024 27 / 25 / 22 /
+// 28, 8 x 512 x 768 29 / 22.9 / 22.0 / 23.5, 64 x 300 x 256 80 / 56 / 44 / 38.
+int cg_items(int B, int T, int d) {
+  const int groups = (d + 7) / 8;
+  if ((long long)groups * 2 * B <= 256) return 1;
+  const int chunks = std::max(1, std::min(B, (T <= 1024 ? 512 : 768) / groups));
+  return 2 * ((B + chunks - 1) / chunks);
 }
 
 }  // namespace
@@ -552,8 +552,8 @@ extern "C" int fstu_stu_conv_mfma(const void* x, const void* taps, void* y, int 
 
 extern "C" int64_t fstu_stu_conv_mfma_grad_ws(int B, int T, int d, int L) {
   if (B < 1 || T < 1 || T > 2048 || d < 8 || L < 1) return 0;
-  const int R = cg_rows_per_group(B, T, d), lags = ((L < T ? L : T) + 1) / 2;
-  return (int64_t)((B + R - 1) / R) * lags * d;
+  const int R = cg_items(B, T, d), lags = ((L < T ? L : T) + 1) / 2;
+  return (int64_t)((2 * B + R - 1) / R) * lags * d;
 }
 
 extern "C" int fstu_stu_conv_mfma_grad(const void* gy, const void* x, const void* filt, void* gx, void* gf, float* part, int B, int T, int d,
@@ -563,13 +563,13 @@ extern "C" int fstu_stu_conv_mfma_grad(const void* gy, const void* x, const void
                FSTU_ESHAPE, "fstu_stu_conv_mfma_grad: B=%d T=%d d=%d L=%d (T up to 2048, d a multiple of 8)", B, T, d, L);
   FSTU_REQUIRE(fstu_aligned(gy, 16) && fstu_aligned(x, 16) && fstu_aligned(filt, 16) && fstu_aligned(gx, 16) && fstu_aligned(gf, 16) &&
                    fstu_aligned(part, 16), FSTU_EALIGN, "fstu_stu_conv_mfma_grad: pointers must be 16-byte aligned");
-  const int R = cg_rows_per_group(B, T, d), chunks = (B + R - 1) / R, lags = ((L < T ? L : T) + 1) / 2;
+  const int R = cg_items(B, T, d), chunks = (2 * B + R - 1) / R, lags = ((L < T ? L : T) + 1) / 2;
   const long long units = (long long)((d + 63) / 64) * chunks;
   FSTU_REQUIRE(units < 1 << 24, FSTU_ESHAPE, "fstu_stu_conv_mfma_grad: B=%d d=%d", B, d);
   const dim3 grid((unsigned)((units + 7) / 8 * 64));
 #define CG_GO(NT)                                                                                                                   \
   do {                                                                                                                              \
-    constexpr int lds__ = 24 * cm_region(8 * NT) + 16 * cg_rows(8 * NT) + 8 * 2048;                                                 \
+    constexpr int lds__ = 16 * cm_region(8 * NT) + 8 * cg_rows(8 * NT) + 8 * 2048;                                                 \
     static const hipError_t ok =                                                                                                    \
         hipFuncSetAttribute((const void*)conv_grad_mfma_kernel<NT>, hipFuncAttributeMaxDynamicSharedMemorySize, lds__);             \
     FSTU_REQUIRE(ok == hipSuccess, (int)ok, "fstu_stu_conv_mfma_grad: %d bytes of LDS refused: %s", lds__, hipGetErrorString(ok));  \

@@ -781,8 +781,8 @@ def stu_conv_mfma(xp: torch.Tensor, taps: torch.Tensor, single_branch: bool = Fa
 
 def stu_conv_mfma_grad_takes(B: int, T: int, d: int, dtype: torch.dtype) -> bool:
     """Whether the gradients of plus + minus are formed on the matrix cores: bf16, T up to 2048.  us, there / through transforms:
-    1 x 300 x 768 12.6 / 14.8, 4 x 600 x 768 20 / 26, 8 x 1025 x 768 44 / 82, 8 x 2048 x 768 73 / 117.  Up to 256 positions a
-    workgroup's latency decides, and more than 256 of them lose: 4 x 200 x 512 12.3 / 13.9, but 8 x 200 x 768 20 / 15."""
+    1 x 300 x 768 12.6 / 14.8, 4 x 600 x 768 17 / 26, 8 x 1025 x 768 38 / 82, 8 x 2048 x 768 62 / 117.  Up to 256 positions a
+    workgroup's latency decides, and more than 256 of them lose: 4 x 200 x 512 12.7 / 13.9, but 8 x 200 x 768 17.5 / 15."""
     return dtype == torch.bfloat16 and 32 <= T <= 2048 and d % 8 == 0 and (T > 256 or B * (d // 8) <= 256)
 
 

@@ -732,9 +732,10 @@ def test_convolution_gradient_kernel(hip, dtype, B, T, d, L, branches):
 
 
 @pytest.mark.parametrize("B,T,d,L", [(1, 1, 8, 4), (2, 33, 8, 64), (9, 127, 64, 50), (5, 129, 8, 129), (130, 65, 24, 70), (3, 511, 136, 512),
-                                     (1, 513, 64, 1024), (2, 1000, 72, 777), (1, 1024, 8, 2048), (5, 1025, 520, 1025), (2, 2048, 64, 2048)])
+                                     (1, 513, 64, 1024), (2, 1000, 72, 777), (1, 1024, 8, 2048), (5, 1025, 520, 1025), (2, 2048, 64, 2048),
+                                     (9, 130, 1032, 130), (5, 1100, 2048, 1100)])
 def test_convolution_gradients_on_the_matrix_cores(hip, B, T, d, L):
-    """Gradients of plus + minus at the edges of the tiles, one and several rows per workgroup, against float64 sums: exact products,
+    """Gradients of plus + minus at the edges of the tiles, one parity, one and several rows per workgroup, against float64 sums: exact products,
     fp32 sums (T, for the filter B * T terms, 2^-24 of the absolute sum each at most), one rounding to bf16."""
     g = gen(T)
     x, gy = (torch.randn(B, T, d, generator=g).bfloat16() for _ in range(2))
