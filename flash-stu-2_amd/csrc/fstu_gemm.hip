@@ -405,6 +405,7 @@ struct Frag8 { u32x2_t lo, hi; };
 // X part are then 64 k of 128 columns, filled 16 bytes = 8 columns per lane and read with transposing reads, k and k + 4 of a
 // fragment's half; the 32-byte pieces of a row are XOR-ed with bits 0, 1 and 3 of k so that the eight rows that two blocks of
 // lanes read together lie in different banks.  `mts` row tiles per slab, slabs sa / sc / sr elements apart.
+// MODE 3: slices of K, outermost, each into fp32 sums of its own (C: slices x M x N floats), straight from the accumulators.
 template <int MODE, bool TA = false>
 __global__ void __launch_bounds__(512)
 gemm_pp_bf16_kernel(const bf16_t* __restrict__ A, long long lda, const bf16_t* __restrict__ W, const bf16_t* __restrict__ W2,
@@ -420,6 +421,8 @@ gemm_pp_bf16_kernel(const bf16_t* __restrict__ A, long long lda, const bf16_t* _
   size_t wbytes, abytes;
   const bf16_t *wb, *wb2, *ab, *rb = R;
   bf16_t* cb = C;
+  float* part = nullptr;
+  const int KS = MODE == 3 ? K / (mt / mts) : K;       // MODE 3: this workgroup's share of K
 #define PP_OPEN_TILE                                                                     \
   {                                                                                      \
     const int o_ = xcd + idx;                                                            \
@@ -427,6 +430,14 @@ gemm_pp_bf16_kernel(const bf16_t* __restrict__ A, long long lda, const bf16_t* _
     const int pw_ = min(GM_PANEL, nt - panel_ * GM_PANEL);                               \
     int bm_ = in_panel_ / pw_;                                                           \
     ab = A;                                                                              \
+    wb = W;                                                                              \
+    if constexpr (MODE == 3) {                                                           \
+      const int slice_ = bm_ / mts;                                                      \
+      bm_ -= slice_ * mts;                                                               \
+      ab += (size_t)slice_ * KS;                                                         \
+      wb += (size_t)slice_ * KS;                                                         \
+      part = (float*)C + (size_t)slice_ * M * N;                                         \
+    }                                                                                    \
     if constexpr (TA) {                                                                  \
       const int slab_ = bm_ / mts;                                                       \
       bm_ -= slab_ * mts;                                                                \
@@ -436,9 +447,9 @@ gemm_pp_bf16_kernel(const bf16_t* __restrict__ A, long long lda, const bf16_t* _
     }                                                                                    \
     m0 = bm_ * 256;                                                                      \
     n0 = (panel_ * GM_PANEL + in_panel_ % pw_) * NF;                                     \
-    wbytes = (size_t)min(NF, N - n0) * K * 2;                                            \
-    abytes = TA ? ((size_t)(K - 1) * lda + 256) * 2 : ((size_t)(min(256, M - m0) - 1) * lda + K) * 2; \
-    wb = W + (size_t)n0 * K;                                                             \
+    wbytes = ((size_t)(min(NF, N - n0) - 1) * K + KS) * 2;                               \
+    abytes = TA ? ((size_t)(K - 1) * lda + 256) * 2 : ((size_t)(min(256, M - m0) - 1) * lda + KS) * 2; \
+    wb += (size_t)n0 * K;                                                                \
     wb2 = MODE == 1 ? W2 + (size_t)n0 * K : wb;                                          \
     ab += TA ? (size_t)m0 : (size_t)m0 * lda;                                            \
   }
@@ -457,7 +468,7 @@ gemm_pp_bf16_kernel(const bf16_t* __restrict__ A, long long lda, const bf16_t* _
     }
   }
   const unsigned w1off = MODE == 1 ? 0u : 128u * (unsigned)K * 2u, x1off = TA ? 256u : 128u * (unsigned)lda * 2u;
-  const int nkt = K >> 6;
+  const int nkt = KS >> 6;
   unsigned char* fill0 = gm_smem + (unsigned)wv * 2048u;
   // requests part P (0 W0, 1 X0, 2 W1, 3 X1) of k tile kt_; beyond the last tile the descriptor is empty: nothing is fetched
 #define PP_FETCH(P, kt_, stage_)                                                                                           \
@@ -569,6 +580,7 @@ gemm_pp_bf16_kernel(const bf16_t* __restrict__ A, long long lda, const bf16_t* _
     const int em0 = m0, en0 = n0;
     bf16_t* const ec = TA ? cb : C;
     const bf16_t* const er = TA ? rb : R;
+    float* const ep = part;
     idx += (int)(gridDim.x >> 3);
     const bool more = idx < share && xcd + idx < tiles;
     if (more) {
@@ -576,6 +588,19 @@ gemm_pp_bf16_kernel(const bf16_t* __restrict__ A, long long lda, const bf16_t* _
       PP_FIRST
     }
     // D of a 16x16 tile: lane l holds row l % 16 and features 4*(l/16) + e
+    if constexpr (MODE == 3) {                         // fp32 sums, straight from the accumulators
+#pragma unroll
+      for (int hw = 0; hw < 2; ++hw)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int hx = 0; hx < 2; ++hx)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              const int m = em0 + hx * 128 + wm * 64 + j * 16 + l16, f = en0 + hw * 128 + wn * 32 + i * 16 + 4 * lq;
+              if (m < M && f < N) *(floatx4_t*)(ep + (size_t)m * N + f) = acc[hw][i][hx][j];
+            }
+    } else
 #pragma unroll
     for (int hx = 0; hx < 2; ++hx)
 #pragma unroll
@@ -856,27 +881,34 @@ using TileRows32 = GemmTile<2, 1, 2, 1, 64, 4>;  // 128 features x 32 rows, 2 wa
 using Tile96 = GemmTile<1, 4, 3, 1, 64, 4>;      // 96 features x 128 rows, 4 waves, 112 KB: N = 768 or 2304 in whole tiles
 using TileK32 = GemmTile<2, 2, 4, 2, 32, 3>;     // 256 x 128, 4 waves, 72 KB, k tiles of 32 for K % 64 != 0
 
+// Whether a product (K % 64 == 0) runs on 256 x 256 tiles.
+// A round of 256 x 256 tiles (one per compute unit) in the alternating-group kernel takes as long as 2.25 rounds of 128 x
+// 128 tiles (K = 2048: 40 us against 18 us), so the large tile wins where its last round is not too empty.  Both sides
+// of the line, us (large / small): 2048 x 4096 x 2048 (128 large tiles) 39.8 / 37.6, 2331 x 4096 x 2048 (160) 40.0 / 54.1;
+// 3072 x 2304 x 768 (108) 20.9 / 19.0, 4096 x 2304 x 768 (144) 21.5 / 27.9; 777 x 2 x 9216 x 768 (288) 41 / 28,
+// 1536 x 2 x 9216 x 768 (432) 43 / 51; 384 x 50257 x 768 (394) 38.5 / 45.6.
+// In mode 1 a round ends in the GELU of its whole tile, beside which a short K hides little, while two small tiles on a
+// compute unit cover each other's: us, large / small tiles, 20000 x 2 x 512 (two rounds, 2.44 small tiles per place in them)
+// K = 64 20.5 / 15.4, 256 25.8 / 21.4, 512 33.6 / 30.4, 768 42.2 / 39.8; 8192 x 2 x 2304 (three rounds, 3) 28.6 / 24.8, 39.8 /
+// 36.1, 53.6 / 51.5, 68.7 / 69.3; 4096 x 2 x 1536 (one round, 3) K = 256 14.8 / 14.0, 512 18.7 / 20.5; 6000 x 2 x 2304 (two,
+// 3.3) K = 64 20.6 / 20.0, 256 27.1 / 29.2.
+bool pp_takes(int mode, int M, int N, int K) {
+  const int nf = mode == 1 ? 2 : 1;
+  const long long big = (long long)((M + 255) / 256) * (((long long)N * nf + 255) / 256);
+  const long long small = (long long)((M + 127) / 128) * (((long long)N * nf + 127) / 128);
+  const long long rounds = (big + gemm_cus() - 1) / gemm_cus();
+  const int quarters = mode != 1 || K >= 1024 ? 9 : K < 256 ? 14 : K < 512 ? 13 : rounds == 1 ? 9 : 11;
+  return quarters * rounds * gemm_cus() < 4 * small;
+}
+
 template <int MODE>
 int gemm_launch(const void* A, long long lda, const void* W, const void* W2, const void* R, long long ldr, void* C, long long ldc,
                 int M, int N, int K, hipStream_t s) {
   if (K % 64 != 0) return gemm_launch_tile<TileK32, MODE>(A, lda, W, W2, R, ldr, C, ldc, M, N, K, s);
   if (M <= 32) return gemm_launch_tile<TileRows32, MODE>(A, lda, W, W2, R, ldr, C, ldc, M, N, K, s);
   const int nf = MODE == 1 ? 2 : 1;
-  const long long big = (long long)((M + 255) / 256) * (((long long)N * nf + 255) / 256);
   const long long small = (long long)((M + 127) / 128) * (((long long)N * nf + 127) / 128);
-  // A round of 256 x 256 tiles (one per compute unit) in the alternating-group kernel takes as long as 2.25 rounds of 128 x
-  // 128 tiles (K = 2048: 40 us against 18 us), so the large tile wins where its last round is not too empty.  Both sides
-  // of the line, us (large / small): 2048 x 4096 x 2048 (128 large tiles) 39.8 / 37.6, 2331 x 4096 x 2048 (160) 40.0 / 54.1;
-  // 3072 x 2304 x 768 (108) 20.9 / 19.0, 4096 x 2304 x 768 (144) 21.5 / 27.9; 777 x 2 x 9216 x 768 (288) 41 / 28,
-  // 1536 x 2 x 9216 x 768 (432) 43 / 51; 384 x 50257 x 768 (394) 38.5 / 45.6.
-  // In mode 1 a round ends in the GELU of its whole tile, beside which a short K hides little, while two small tiles on a
-  // compute unit cover each other's: us, large / small tiles, 20000 x 2 x 512 (two rounds, 2.44 small tiles per place in them)
-  // K = 64 20.5 / 15.4, 256 25.8 / 21.4, 512 33.6 / 30.4, 768 42.2 / 39.8; 8192 x 2 x 2304 (three rounds, 3) 28.6 / 24.8, 39.8 /
-  // 36.1, 53.6 / 51.5, 68.7 / 69.3; 4096 x 2 x 1536 (one round, 3) K = 256 14.8 / 14.0, 512 18.7 / 20.5; 6000 x 2 x 2304 (two,
-  // 3.3) K = 64 20.6 / 20.0, 256 27.1 / 29.2.
-  const long long rounds = (big + gemm_cus() - 1) / gemm_cus();
-  const int quarters = MODE != 1 || K >= 1024 ? 9 : K < 256 ? 14 : K < 512 ? 13 : rounds == 1 ? 9 : 11;
-  if (quarters * rounds * gemm_cus() < 4 * small)
+  if (pp_takes(MODE, M, N, K))
     return gemm_pp_launch<MODE>(A, lda, W, W2, R, ldr, C, ldc, M, N, K, s);
   // A grid that leaves one workgroup per compute unit anyway gains from the deeper pipeline when K is long (M=4096, N=768,
   // K=9216: 83 us against 93 us).
@@ -896,6 +928,72 @@ int gemm_launch(const void* A, long long lda, const void* W, const void* W2, con
 
 }  // namespace
 
+// Slices of K for a product of few output tiles (1: none).  A workgroup that has a compute unit to itself takes 0.41 us per k tile
+// of 64 on the deep pipeline (0.9 with two stages, which is what slices that leave one to a unit ran on before), two to a unit 0.61
+// each; joining costs a launch and the slices' bytes out and back at 4 TB/s.  The estimate only has to rank: us without / with the
+// slices it picks, rows x features x K: 300 x 768 x 9216 60 / 17.7 (12), 1000 x 768 x 9216 60 / 27.5 (4; 31.4 with two stages), 1400
+// 60 / 34.0 (3; 39.7), 2400 61 / 44.7 (4; 47.2 with two, which were picked before and took 53.8), 3000 63 / 53 (3), 700 x 2048 x
+// 24576 180 / 85 (4), 1500 x 2048 x 24576 184 / 160 (2), 300 x 2048 x 2048 21.8 / 15.0 (4); slabs 1 x 1024 x 1024 x 24576 219 / 63
+// (8), 1 x 128 x 256 x 6144 50 / 12 (12).  Where it picks none, without / with two: 4096 x 768 x 9216 66.6 / 68.8, 600 x 2048 x
+// 2048 22.0 / 18.8, 300 x 6144 x 2048 20.5 / 23.8, 1000 x 768 x 768 10.5 / 12.7.  Below K = 2048 the GPU gains less than the second
+// launch and the slices' allocation cost the host (calls of 300 x 384 x 1536 one behind the other 16.0 us with three slices, 13.2
+// without).
+extern "C" int fstu_gemm_bf16_slices(int M, int N, int K, int nbatch) {
+  if (M <= 32 || N % 4 != 0 || K % 64 != 0 || K < 2048) return 1;
+  const long long cus = gemm_cus(), tiles = (long long)((M + 127) / 128) * ((N + 127) / 128) * nbatch;
+  const int nkt = K / 64;
+  double least = 0.41 * nkt;
+  int best = 1;
+  for (int s = 2; s <= 32 && K / s >= 512 && tiles * s <= 2 * cus; ++s) {
+    if (nkt % s != 0) continue;
+    const double us = nkt / s * (tiles * s <= cus ? 0.41 : 0.61) + 3.0 + 8e-6 / 4.0 * s * nbatch * (double)M * N;
+    if (us < least) { least = us; best = s; }
+  }
+  return best;
+}
+
+namespace {
+
+// The same for rows (k contiguous in both operands), whose slices can also run on 256 x 256 tiles in the alternating-group kernel:
+// half the operands' bytes through the LDS for a product, and every compute unit at work where M and N leave it idle.  A k tile of
+// 64 takes those 1 us in a nearly empty round and 1.35 in a full one, which draws the matrix cores' power; 128 x 128 tiles 0.43 us alone on
+// a compute unit and 0.55 to 0.9 of two in pairs.  us before / with the slices it picks (L: large tiles), rows x features x K:
+// 1408 x 2048 x 24576 177 / 137 (L4), 1900 213 / 159 (L4), 2500 363 / 203 (L3), 3200 379 / 264 (L2), 4096 400 / 295 (L2), 5000 452 / 398
+// (L3); 5500 x 768 x 9216 99 / 81 (L3), 7000 125 / 95 (L3), 9000 136 / 116 (L2), 12000 266 / 170 (L3).  Where it stays as it was, with
+// the best slices of large tiles: 1000 x 2048 x 24576 105 / 91 (6), 6100 485 / 498 (4), 4096 x 768 x 9216 66 / 61 (4), 16000 x 768 x
+// 9216 180 / 230 (2), 2500 x 2048 x 2048 31 / 39 (2).
+struct RowSlices { int count; bool large; };
+RowSlices row_slices(int M, int N, int K) {
+  const int before = fstu_gemm_bf16_slices(M, N, K, 1);
+  if (M <= 256 || N % 4 != 0 || K % 64 != 0 || K < 2048) return {before, false};
+  const long long cus = gemm_cus();
+  const long long small = (long long)((M + 127) / 128) * ((N + 127) / 128), big = (long long)((M + 255) / 256) * ((N + 255) / 256);
+  const int nkt = K / 64;
+  const auto join = [&](int s) { return s == 1 ? 0.0 : 3.0 + 8e-6 / 4.0 * s * (double)M * N; };
+  const auto large = [&](int s) {
+    const long long rounds = (big * s + cus - 1) / cus;
+    const double full = (double)(big * s) / (double)(rounds * cus);
+    return rounds * (nkt / s) * (1.0 + 0.35 * full * full) + join(s);
+  };
+  const auto little = [&](int s) {
+    if (small * s <= cus) return nkt / s * 0.43 + join(s);
+    const long long rounds = (small * s + 2 * cus - 1) / (2 * cus);
+    return rounds * (nkt / s) * (0.55 + 0.35 * (double)(small * s) / (double)(rounds * 2 * cus)) + join(s);
+  };
+  double least = 0.95 * (before == 1 && pp_takes(0, M, N, K) ? large(1) : little(before));
+  RowSlices best = {before, false};
+  for (int s = 2; s <= 32 && K / s >= 512 && big * s <= 2 * cus; ++s) {
+    if (nkt % s != 0) continue;
+    const double us = large(s);
+    if (us < least) { least = us; best = {s, true}; }
+  }
+  return best;
+}
+
+}  // namespace
+
+extern "C" int fstu_gemm_bf16_row_slices(int M, int N, int K) { return row_slices(M, N, K).count; }
+
 extern "C" int fstu_gemm_bf16_splitk(const void* A, int64_t lda, const void* W, float* partial, int M, int N, int K, int ksplit,
                                      void* stream) {
   FSTU_REQUIRE(A && W && partial, FSTU_ENULL, "fstu_gemm_bf16_splitk: null pointer");
@@ -908,7 +1006,10 @@ extern "C" int fstu_gemm_bf16_splitk(const void* A, int64_t lda, const void* W, 
   FSTU_REQUIRE(lda < GM_MAX_LD && K < GM_MAX_LD, FSTU_ESHAPE, "fstu_gemm_bf16_splitk: lda=%lld / K=%d beyond the 32-bit tile offsets",
                (long long)lda, K);
   int rc;
+  const RowSlices plan = row_slices(M, N, K);
   if (M <= 32) rc = gemm_launch_tile<TileRows32, 3>(A, lda, W, nullptr, nullptr, 0, partial, N, M, N, K, (hipStream_t)stream, ksplit);
+  else if (plan.large && plan.count == ksplit)
+    rc = gemm_pp_launch<3>(A, lda, W, nullptr, nullptr, 0, partial, N, M, N, K, (hipStream_t)stream, ksplit);
   else if ((long long)((M + 127) / 128) * ((N + 127) / 128) * ksplit <= gemm_cus())
     rc = gemm_launch_tile<TileDeep, 3>(A, lda, W, nullptr, nullptr, 0, partial, N, M, N, K, (hipStream_t)stream, ksplit);
   else rc = gemm_launch_tile<TileSmall, 3>(A, lda, W, nullptr, nullptr, 0, partial, N, M, N, K, (hipStream_t)stream, ksplit);
@@ -951,35 +1052,11 @@ static int fstu_join_slices(const float* part, int ns, const void* R, long long 
   return FSTU_OK;
 }
 
-// Slices of K for a product of few output tiles (1: none).  A workgroup that has a compute unit to itself takes 0.41 us per k tile
-// of 64 on the deep pipeline (0.9 with two stages, which is what slices that leave one to a unit ran on before), two to a unit 0.61
-// each; joining costs a launch and the slices' bytes out and back at 4 TB/s.  The estimate only has to rank: us without / with the
-// slices it picks, rows x features x K: 300 x 768 x 9216 60 / 17.7 (12), 1000 x 768 x 9216 60 / 27.5 (4; 31.4 with two stages), 1400
-// 60 / 34.0 (3; 39.7), 2400 61 / 44.7 (4; 47.2 with two, which were picked before and took 53.8), 3000 63 / 53 (3), 700 x 2048 x
-// 24576 180 / 85 (4), 1500 x 2048 x 24576 184 / 160 (2), 300 x 2048 x 2048 21.8 / 15.0 (4); slabs 1 x 1024 x 1024 x 24576 219 / 63
-// (8), 1 x 128 x 256 x 6144 50 / 12 (12).  Where it picks none, without / with two: 4096 x 768 x 9216 66.6 / 68.8, 600 x 2048 x
-// 2048 22.0 / 18.8, 300 x 6144 x 2048 20.5 / 23.8, 1000 x 768 x 768 10.5 / 12.7.  Below K = 2048 the GPU gains less than the second
-// launch and the slices' allocation cost the host (calls of 300 x 384 x 1536 one behind the other 16.0 us with three slices, 13.2
-// without).
-extern "C" int fstu_gemm_bf16_slices(int M, int N, int K, int nbatch) {
-  if (M <= 32 || N % 4 != 0 || K % 64 != 0 || K < 2048) return 1;
-  const long long cus = gemm_cus(), tiles = (long long)((M + 127) / 128) * ((N + 127) / 128) * nbatch;
-  const int nkt = K / 64;
-  double least = 0.41 * nkt;
-  int best = 1;
-  for (int s = 2; s <= 32 && K / s >= 512 && tiles * s <= 2 * cus; ++s) {
-    if (nkt % s != 0) continue;
-    const double us = nkt / s * (tiles * s <= cus ? 0.41 : 0.61) + 3.0 + 8e-6 / 4.0 * s * nbatch * (double)M * N;
-    if (us < least) { least = us; best = s; }
-  }
-  return best;
-}
-
 // Rows of a plain or residual product that whole rounds of 256 x 256 tiles take (0: no split).  A last round of few large tiles
 // costs nearly what a full one does; its rows by themselves run in slices of K or on small tiles, of which the chip holds as many at
-// once as there are compute units.  us in one launch / split, rows x features x K: 9600 x 2048 x 24576 970 / 743, 8500 x 2048 x 24576
-// 1029 / 590, 17000 x 2048 x 24576 1490 / 1152, 22500 x 768 x 9216 409 / 237, 3000 x 6144 x 2048 83 / 65, 10240 x 2048 x 2048 81 /
-// 73, 22500 x 768 x 768 42 / 37, 33000 x 512 x 512 31 / 28.  The line: 12288 x 2048 x 24576 (512 small tiles left) 962 / 953, below K
+// once as there are compute units.  us in one launch / split, rows x features x K: 9600 x 2048 x 24576 970 / 687, 8500 x 2048 x 24576
+// 1029 / 590, 10500 x 2048 x 24576 971 / 739, 13500 1024 / 959, 17000 1490 / 1152, 20480 1502 / 1369, 22500 x 768 x 9216 409 / 237, 3000 x 6144 x 2048 83 / 65, 10240 x 2048 x 2048 81 /
+// 73, 22500 x 768 x 768 42 / 37, 33000 x 512 x 512 31 / 28.  The line: 14500 x 2048 x 24576 (no slices of the rest) 1041 / 1015, below K
 // = 2048 26000 x 768 x 768 (204) 38.5 / 39.3, 18500 x 1024 x 1024 (136) 44.9 / 43.1.
 extern "C" int fstu_gemm_bf16_head_rows(int M, int N, int K) {
   if (M <= 256 || N < 256 || N % 4 != 0 || K % 64 != 0 || K < 512) return 0;
@@ -987,7 +1064,8 @@ extern "C" int fstu_gemm_bf16_head_rows(int M, int N, int K) {
   const long long head = tiles / cus * cus / nt * 256;
   if (head <= 0 || head >= M) return 0;
   const long long left = (M - head + 127) / 128 * ((N + 127) / 128);
-  return left <= (K < 2048 ? cus / 2 : cus) ? (int)head : 0;
+  if (left <= (K < 2048 ? cus / 2 : cus) || row_slices((int)(M - head), N, K).large) return (int)head;
+  return 0;
 }
 
 extern "C" int fstu_gemm_bf16(const void* A, int64_t lda, const void* W, const void* W2, const void* R, int64_t ldr, void* C,

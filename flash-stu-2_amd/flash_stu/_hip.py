@@ -103,6 +103,7 @@ SIGNATURES = {
     "fstu_gemm_bf16_splitk": [_vp, _i64, _vp, _vp, _i, _i, _i, _i, _vp],
     "fstu_gemm_any": [_vp, _i64, _i64, _vp, _i64, _i64, _vp, _i64, _i, _i, _i, _i, _vp],
     "fstu_gemm_bf16_slices": [_i, _i, _i, _i],
+    "fstu_gemm_bf16_row_slices": [_i, _i, _i],
     "fstu_gemm_bf16_head_rows": [_i, _i, _i],
     "fstu_gemm_bf16_ws": [_vp, _i64, _vp, _vp, _vp, _i64, _vp, _i64, _i, _i, _i, _i, _vp, _i, _vp],
     "fstu_gemm_bf16_ta_ws": [_vp, _i64, _i64, _vp, _vp, _i64, _i64, _vp, _i64, _i64, _i, _i, _i, _i, _i, _vp, _i, _vp],
@@ -312,6 +313,11 @@ def _gemm_slices(M: int, N: int, K: int, nbatch: int) -> int:
 
 
 @functools.lru_cache(maxsize=256)
+def _gemm_row_slices(M: int, N: int, K: int) -> int:
+    return load().fstu_gemm_bf16_row_slices(M, N, K)
+
+
+@functools.lru_cache(maxsize=256)
 def _gemm_head_rows(M: int, N: int, K: int) -> int:
     return load().fstu_gemm_bf16_head_rows(M, N, K)
 
@@ -358,7 +364,7 @@ def _gemm_rows(x2, weight, up_weight, residual, out, mode: int, ldr: int) -> Non
     (M, K), N = x2.shape, weight.shape[0]
     slices, partial = 1, None
     if K >= GEMM_MIN_SLICED_K and mode != 1 and out.stride(0) % 4 == 0 and out.data_ptr() % 8 == 0:
-        slices = _gemm_slices(M, N, K, 1)
+        slices = _gemm_row_slices(M, N, K)
         if slices > 1:
             partial = torch.empty(slices, M, N, dtype=torch.float32, device=x2.device)
     _check(load().fstu_gemm_bf16_ws(_p(x2), x2.stride(0), _p(weight), _p(up_weight), _p(residual), ldr, _p(out), out.stride(0),

@@ -291,6 +291,24 @@ def test_gemm_bf16_whole_rounds_and_the_rest(hip, M, N, K, head):
     assert bool(((out.float() - (R.float() + ref)).abs() <= bound + 2.0 ** -8 * (R.float() + ref).abs()).all())
 
 
+@pytest.mark.parametrize("M,N,K,slices", [(400, 4100, 8192, 4), (1000, 2052, 8192, 4), (400, 8200, 6144, 3)])
+def test_gemm_bf16_in_slices_of_large_tiles(hip, M, N, K, slices):
+    """Slices of K on the 256 x 256 tiles, ragged tiles of rows and features, rows of a stride of their own, nothing read or written
+    behind them: fp32 sums of exact products stay within (K + slices) * 2^-24 of the absolute sum, one or two roundings to bf16."""
+    g = gen(M + N)
+    assert hip.load().fstu_gemm_bf16_row_slices(M, N, K) == slices != hip.load().fstu_gemm_bf16_slices(M, N, K, 1)
+    wide = torch.full((M + 1, K + 8), float("nan"), dtype=torch.bfloat16, device="cuda")
+    wide[:M, :K] = dev(torch.randn(M, K, generator=g).bfloat16())
+    W, R = dev(torch.randn(N, K, generator=g).bfloat16()), dev(torch.randn(M, N, generator=g).bfloat16())
+    out = torch.full((M + 1, N + 4), float("nan"), dtype=torch.bfloat16, device="cuda")
+    ref = torch.matmul(wide[:M, :K].float(), W.float().t().contiguous())     # fp32 on the library: K * 2^-24 of the absolute sum too
+    bound = (2 * K + slices) * 2.0 ** -24 * torch.matmul(wide[:M, :K].float().abs(), W.float().abs().t().contiguous()) + 2.0 ** -8 * ref.abs()
+    y = hip.gemm(wide[:M, :K], W, out=out[:M, :N])
+    assert bool(((y.float() - ref).abs() <= bound).all())
+    assert bool(out[M:].isnan().all()) and bool(out[:, N:].isnan().all())
+    assert torch.equal(hip.gemm(wide[:M, :K], W, residual=R, out=R.clone()), (R.float() + y.float()).bfloat16())
+
+
 @pytest.mark.parametrize("nb,M,N,K,slices", [(1, 128, 132, 4096, 8), (3, 256, 260, 6144, 12), (1, 384, 1024, 3072, 6)])
 def test_gemm_bf16_in_slices(hip, nb, M, N, K, slices):
     """Few output tiles and a long K: both prompt GEMMs in slices of K, plain and with the residual, ragged tiles and strided
