@@ -405,12 +405,13 @@ struct Frag8 { u32x2_t lo, hi; };
 // X part are then 64 k of 128 columns, filled 16 bytes = 8 columns per lane and read with transposing reads, k and k + 4 of a
 // fragment's half; the 32-byte pieces of a row are XOR-ed with bits 0, 1 and 3 of k so that the eight rows that two blocks of
 // lanes read together lie in different banks.  `mts` row tiles per slab, slabs sa / sc / sr elements apart.
-// MODE 3: slices of K, outermost, each into fp32 sums of its own (C: slices x M x N floats), straight from the accumulators.
+// MODE 3: slices of K, outermost, each into fp32 sums of its own (C: slices x nb slabs x M x N floats), straight from the
+// accumulators.
 template <int MODE, bool TA = false>
 __global__ void __launch_bounds__(512)
 gemm_pp_bf16_kernel(const bf16_t* __restrict__ A, long long lda, const bf16_t* __restrict__ W, const bf16_t* __restrict__ W2,
                     const bf16_t* __restrict__ R, long long ldr, bf16_t* __restrict__ C, long long ldc, int M, int N, int K,
-                    int mt, int nt, int share, int mts, long long sa, long long sc, long long sr) {
+                    int mt, int nt, int share, int mts, long long sa, long long sc, long long sr, int nb) {
   constexpr int NF = MODE == 1 ? 128 : 256;
   extern __shared__ __align__(16) unsigned char gm_smem[];   // stage: W0 | W1 | X0 | X1
   const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -422,7 +423,7 @@ gemm_pp_bf16_kernel(const bf16_t* __restrict__ A, long long lda, const bf16_t* _
   const bf16_t *wb, *wb2, *ab, *rb = R;
   bf16_t* cb = C;
   float* part = nullptr;
-  const int KS = MODE == 3 ? K / (mt / mts) : K;       // MODE 3: this workgroup's share of K
+  const int KS = MODE == 3 ? K / (mt / mts / nb) : K;       // MODE 3: this workgroup's share of K
 #define PP_OPEN_TILE                                                                     \
   {                                                                                      \
     const int o_ = xcd + idx;                                                            \
@@ -432,13 +433,12 @@ gemm_pp_bf16_kernel(const bf16_t* __restrict__ A, long long lda, const bf16_t* _
     ab = A;                                                                              \
     wb = W;                                                                              \
     if constexpr (MODE == 3) {                                                           \
-      const int slice_ = bm_ / mts;                                                      \
-      bm_ -= slice_ * mts;                                                               \
-      ab += (size_t)slice_ * KS;                                                         \
+      const int part_ = bm_ / mts, slice_ = part_ / nb;                                  \
+      bm_ -= part_ * mts;                                                                \
+      ab += TA ? (size_t)(part_ - slice_ * nb) * sa + (size_t)slice_ * KS * lda : (size_t)slice_ * KS; \
       wb += (size_t)slice_ * KS;                                                         \
-      part = (float*)C + (size_t)slice_ * M * N;                                         \
-    }                                                                                    \
-    if constexpr (TA) {                                                                  \
+      part = (float*)C + (size_t)part_ * M * N;                                          \
+    } else if constexpr (TA) {                                                           \
       const int slab_ = bm_ / mts;                                                       \
       bm_ -= slab_ * mts;                                                                \
       ab += (size_t)slab_ * sa;                                                          \
@@ -448,7 +448,7 @@ gemm_pp_bf16_kernel(const bf16_t* __restrict__ A, long long lda, const bf16_t* _
     m0 = bm_ * 256;                                                                      \
     n0 = (panel_ * GM_PANEL + in_panel_ % pw_) * NF;                                     \
     wbytes = ((size_t)(min(NF, N - n0) - 1) * K + KS) * 2;                               \
-    abytes = TA ? ((size_t)(K - 1) * lda + 256) * 2 : ((size_t)(min(256, M - m0) - 1) * lda + KS) * 2; \
+    abytes = TA ? ((size_t)(KS - 1) * lda + 256) * 2 : ((size_t)(min(256, M - m0) - 1) * lda + KS) * 2; \
     wb += (size_t)n0 * K;                                                                \
     wb2 = MODE == 1 ? W2 + (size_t)n0 * K : wb;                                          \
     ab += TA ? (size_t)m0 : (size_t)m0 * lda;                                            \
@@ -651,14 +651,14 @@ gemm_pp_bf16_kernel(const bf16_t* __restrict__ A, long long lda, const bf16_t* _
 
 template <int MODE, bool TA = false>
 int gemm_pp_launch(const void* A, long long lda, const void* W, const void* W2, const void* R, long long ldr, void* C,
-                   long long ldc, int M, int N, int K, hipStream_t s, int nbatch = 1, long long sa = 0, long long sc = 0, long long sr = 0) {
+                   long long ldc, int M, int N, int K, hipStream_t s, int nbatch = 1, long long sa = 0, long long sc = 0, long long sr = 0, int nb = 1) {
   constexpr int NF = MODE == 1 ? 128 : 256;
   static hipError_t attr_err = hipFuncSetAttribute((const void*)gemm_pp_bf16_kernel<MODE, TA>, hipFuncAttributeMaxDynamicSharedMemorySize, PP_LDS);
   if (attr_err != hipSuccess) { fstu_set_error("fstu_gemm_bf16: hipFuncSetAttribute: %s", hipGetErrorString(attr_err)); return (int)attr_err; }
   const int mts = (M + 255) / 256, mt = mts * nbatch, nt = (N + NF - 1) / NF;
   const int share = (int)(((long long)mt * nt + 7) / 8);
   hipLaunchKernelGGL((gemm_pp_bf16_kernel<MODE, TA>), dim3(8u * (unsigned)std::min(share, gemm_cus() / 8)), dim3(512), PP_LDS, s, (const bf16_t*)A, lda,
-                     (const bf16_t*)W, (const bf16_t*)W2, (const bf16_t*)R, ldr, (bf16_t*)C, ldc, M, N, K, mt, nt, share, mts, sa, sc, sr);
+                     (const bf16_t*)W, (const bf16_t*)W2, (const bf16_t*)R, ldr, (bf16_t*)C, ldc, M, N, K, mt, nt, share, mts, sa, sc, sr, nb);
   return 0;
 }
 
@@ -954,22 +954,23 @@ extern "C" int fstu_gemm_bf16_slices(int M, int N, int K, int nbatch) {
 
 namespace {
 
-// The same for rows (k contiguous in both operands), whose slices can also run on 256 x 256 tiles in the alternating-group kernel:
+// The same where the slices can also run on 256 x 256 tiles in the alternating-group kernel (rows, or slabs of whole tiles of them):
 // half the operands' bytes through the LDS for a product, and every compute unit at work where M and N leave it idle.  A k tile of
 // 64 takes those 1 us in a nearly empty round and 1.35 in a full one, which draws the matrix cores' power; 128 x 128 tiles 0.43 us alone on
 // a compute unit and 0.55 to 0.9 of two in pairs.  us before / with the slices it picks (L: large tiles), rows x features x K:
 // 1408 x 2048 x 24576 177 / 137 (L4), 1900 213 / 159 (L4), 2500 363 / 203 (L3), 3200 379 / 264 (L2), 4096 400 / 295 (L2), 5000 452 / 398
-// (L3); 5500 x 768 x 9216 99 / 81 (L3), 7000 125 / 95 (L3), 9000 136 / 116 (L2), 12000 266 / 170 (L3).  Where it stays as it was, with
-// the best slices of large tiles: 1000 x 2048 x 24576 105 / 91 (6), 6100 485 / 498 (4), 4096 x 768 x 9216 66 / 61 (4), 16000 x 768 x
-// 9216 180 / 230 (2), 2500 x 2048 x 2048 31 / 39 (2).
-struct RowSlices { int count; bool large; };
-RowSlices row_slices(int M, int N, int K) {
-  const int before = fstu_gemm_bf16_slices(M, N, K, 1);
-  if (M <= 256 || N % 4 != 0 || K % 64 != 0 || K < 2048) return {before, false};
+// (L3); 5500 x 768 x 9216 99 / 81 (L3), 7000 125 / 95 (L3), 12000 266 / 170 (L3).  Where it stays as it was, with
+// the best slices of large tiles: 1000 x 2048 x 24576 105 / 91 (6), 6100 485 / 498 (4), 4096 x 768 x 9216 66 / 61 (4), 9000 136 / 116
+// (2), 16000 180 / 230 (2), 2500 x 2048 x 2048 31 / 39 (2).  Slabs: 1 x 8192 x 1024 x 24576 451 / 309 (L2), 4 x 2048 454 / 303 (L2), 2 x
+// 2048 242 / 159 (L4), 1 x 4096 x 768 x 18432 142 / 111 (L4).
+struct SlicePlan { int count; bool large; };
+SlicePlan slice_plan(int M, int N, int K, int nb) {
+  const int before = fstu_gemm_bf16_slices(M, N, K, nb);
+  if (M < 256 || N % 4 != 0 || K % 64 != 0 || K < 2048) return {before, false};
   const long long cus = gemm_cus();
-  const long long small = (long long)((M + 127) / 128) * ((N + 127) / 128), big = (long long)((M + 255) / 256) * ((N + 255) / 256);
+  const long long small = (long long)((M + 127) / 128) * ((N + 127) / 128) * nb, big = (long long)((M + 255) / 256) * ((N + 255) / 256) * nb;
   const int nkt = K / 64;
-  const auto join = [&](int s) { return s == 1 ? 0.0 : 3.0 + 8e-6 / 4.0 * s * (double)M * N; };
+  const auto join = [&](int s) { return s == 1 ? 0.0 : 3.0 + 8e-6 / 4.0 * s * nb * (double)M * N; };
   const auto large = [&](int s) {
     const long long rounds = (big * s + cus - 1) / cus;
     const double full = (double)(big * s) / (double)(rounds * cus);
@@ -980,8 +981,8 @@ RowSlices row_slices(int M, int N, int K) {
     const long long rounds = (small * s + 2 * cus - 1) / (2 * cus);
     return rounds * (nkt / s) * (0.55 + 0.35 * (double)(small * s) / (double)(rounds * 2 * cus)) + join(s);
   };
-  double least = 0.95 * (before == 1 && pp_takes(0, M, N, K) ? large(1) : little(before));
-  RowSlices best = {before, false};
+  double least = 0.95 * (before == 1 && 9 * ((big + cus - 1) / cus) * cus < 4 * small ? large(1) : little(before));
+  SlicePlan best = {before, false};
   for (int s = 2; s <= 32 && K / s >= 512 && big * s <= 2 * cus; ++s) {
     if (nkt % s != 0) continue;
     const double us = large(s);
@@ -992,7 +993,10 @@ RowSlices row_slices(int M, int N, int K) {
 
 }  // namespace
 
-extern "C" int fstu_gemm_bf16_row_slices(int M, int N, int K) { return row_slices(M, N, K).count; }
+extern "C" int fstu_gemm_bf16_row_slices(int M, int N, int K) { return slice_plan(M, N, K, 1).count; }
+extern "C" int fstu_gemm_bf16_slab_slices(int M, int N, int K, int nbatch) {
+  return M % 256 == 0 ? slice_plan(M, N, K, nbatch).count : fstu_gemm_bf16_slices(M, N, K, nbatch);
+}
 
 extern "C" int fstu_gemm_bf16_splitk(const void* A, int64_t lda, const void* W, float* partial, int M, int N, int K, int ksplit,
                                      void* stream) {
@@ -1006,7 +1010,7 @@ extern "C" int fstu_gemm_bf16_splitk(const void* A, int64_t lda, const void* W, 
   FSTU_REQUIRE(lda < GM_MAX_LD && K < GM_MAX_LD, FSTU_ESHAPE, "fstu_gemm_bf16_splitk: lda=%lld / K=%d beyond the 32-bit tile offsets",
                (long long)lda, K);
   int rc;
-  const RowSlices plan = row_slices(M, N, K);
+  const SlicePlan plan = slice_plan(M, N, K, 1);
   if (M <= 32) rc = gemm_launch_tile<TileRows32, 3>(A, lda, W, nullptr, nullptr, 0, partial, N, M, N, K, (hipStream_t)stream, ksplit);
   else if (plan.large && plan.count == ksplit)
     rc = gemm_pp_launch<3>(A, lda, W, nullptr, nullptr, 0, partial, N, M, N, K, (hipStream_t)stream, ksplit);
@@ -1064,7 +1068,7 @@ extern "C" int fstu_gemm_bf16_head_rows(int M, int N, int K) {
   const long long head = tiles / cus * cus / nt * 256;
   if (head <= 0 || head >= M) return 0;
   const long long left = (M - head + 127) / 128 * ((N + 127) / 128);
-  if (left <= (K < 2048 ? cus / 2 : cus) || row_slices((int)(M - head), N, K).large) return (int)head;
+  if (left <= (K < 2048 ? cus / 2 : cus) || slice_plan((int)(M - head), N, K, 1).large) return (int)head;
   return 0;
 }
 
@@ -1141,7 +1145,10 @@ extern "C" int fstu_gemm_bf16_ta_ws(const void* A, int64_t lda, int64_t batch_st
   int rc;
   if (ksplit > 1) {
     if ((rc = split_check("fstu_gemm_bf16_ta_ws", N, K, ksplit, partial))) return rc;
-    rc = gemm_ta_launch_tile<TileSmall, 3>(A, lda, batch_stride_a, W, partial, 0, 0, C, 0, 0, M, N, K, nbatch, s, ksplit);
+    const SlicePlan plan = slice_plan(M, N, K, nbatch);
+    if (M % 256 == 0 && plan.large && plan.count == ksplit)
+      rc = gemm_pp_launch<3, true>(A, lda, W, nullptr, nullptr, 0, partial, N, M, N, K, s, ksplit * nbatch, batch_stride_a, 0, 0, nbatch);
+    else rc = gemm_ta_launch_tile<TileSmall, 3>(A, lda, batch_stride_a, W, partial, 0, 0, C, 0, 0, M, N, K, nbatch, s, ksplit);
     if (rc) return rc;
     FSTU_CHECK_LAUNCH("fstu_gemm_bf16_ta_ws");
     return fstu_join_slices(partial, ksplit, mode == 2 ? R : nullptr, ldr, batch_stride_r, C, ldc, batch_stride_c, nbatch, M, N, stream);

@@ -104,6 +104,7 @@ SIGNATURES = {
     "fstu_gemm_any": [_vp, _i64, _i64, _vp, _i64, _i64, _vp, _i64, _i, _i, _i, _i, _vp],
     "fstu_gemm_bf16_slices": [_i, _i, _i, _i],
     "fstu_gemm_bf16_row_slices": [_i, _i, _i],
+    "fstu_gemm_bf16_slab_slices": [_i, _i, _i, _i],
     "fstu_gemm_bf16_head_rows": [_i, _i, _i],
     "fstu_gemm_bf16_ws": [_vp, _i64, _vp, _vp, _vp, _i64, _vp, _i64, _i, _i, _i, _i, _vp, _i, _vp],
     "fstu_gemm_bf16_ta_ws": [_vp, _i64, _i64, _vp, _vp, _i64, _i64, _vp, _i64, _i64, _i, _i, _i, _i, _i, _vp, _i, _vp],
@@ -308,8 +309,8 @@ def gemm_supported(x2: torch.Tensor, weight: torch.Tensor, plain: bool = False) 
 
 
 @functools.lru_cache(maxsize=256)
-def _gemm_slices(M: int, N: int, K: int, nbatch: int) -> int:
-    return load().fstu_gemm_bf16_slices(M, N, K, nbatch)
+def _gemm_slab_slices(M: int, N: int, K: int, nbatch: int) -> int:
+    return load().fstu_gemm_bf16_slab_slices(M, N, K, nbatch)
 
 
 @functools.lru_cache(maxsize=256)
@@ -415,7 +416,7 @@ def gemm_ta(slabs: torch.Tensor, weight: torch.Tensor, residual: Optional[torch.
         if t is not None and (t.shape != (nb, M, N) or t.stride(2) != 1 or t.dtype != slabs.dtype):
             raise FlashSTUHipError(f"gemm_ta: {name} must be (nb, M, N) with contiguous rows")
     mode = 2 if residual is not None else 0
-    slices = _gemm_slices(M, N, K, nb) if K >= GEMM_MIN_SLICED_K else 1
+    slices = _gemm_slab_slices(M, N, K, nb) if K >= GEMM_MIN_SLICED_K else 1
     partial = torch.empty(slices, nb, M, N, dtype=torch.float32, device=slabs.device) if slices > 1 else None
     _check(load().fstu_gemm_bf16_ta_ws(_p(slabs), slabs.stride(1), slabs.stride(0) if nb > 1 else 0, _p(weight), _p(residual),
                                        residual.stride(1) if residual is not None else 0,

@@ -446,8 +446,9 @@ int fstu_gemm_bf16_ta(const void* A, int64_t lda, int64_t batch_stride_a, const 
  * second launch adds in order.  fstu_gemm_bf16_slices says how many pay (1: none; nbatch = 1 for fstu_gemm_bf16_ws); partial
  * holds ksplit * nbatch * M * N floats, 16-byte aligned. */
 int fstu_gemm_bf16_slices(int M, int N, int K, int nbatch);
-/* The same for fstu_gemm_bf16_ws and fstu_gemm_bf16_splitk, whose slices also run on the large tiles. */
+/* The same for fstu_gemm_bf16_ws and fstu_gemm_bf16_splitk, and for fstu_gemm_bf16_ta_ws, whose slices also run on the large tiles. */
 int fstu_gemm_bf16_row_slices(int M, int N, int K);
+int fstu_gemm_bf16_slab_slices(int M, int N, int K, int nbatch);
 /* Rows in front that fill whole rounds of the large tiles, where the others are faster in a call of their own (0: one call). */
 int fstu_gemm_bf16_head_rows(int M, int N, int K);
 int fstu_gemm_bf16_ws(const void* A, int64_t lda, const void* W, const void* W2, const void* R, int64_t ldr, void* C,

@@ -309,6 +309,22 @@ def test_gemm_bf16_in_slices_of_large_tiles(hip, M, N, K, slices):
     assert torch.equal(hip.gemm(wide[:M, :K], W, residual=R, out=R.clone()), (R.float() + y.float()).bfloat16())
 
 
+@pytest.mark.parametrize("nb,M,N,K,slices", [(1, 512, 4100, 8192, 4), (2, 256, 4100, 8192, 4), (2, 1024, 4100, 6144, 3)])
+def test_gemm_bf16_slabs_in_slices_of_large_tiles(hip, nb, M, N, K, slices):
+    """The same with the reduction index slowest: several slabs, rows of a wider buffer, a ragged last tile of features."""
+    g = gen(M + N)
+    assert hip.load().fstu_gemm_bf16_slab_slices(M, N, K, nb) == slices != hip.load().fstu_gemm_bf16_slices(M, N, K, nb)
+    wide = torch.full((nb, K, M + 64), float("nan"), dtype=torch.bfloat16, device="cuda")
+    wide[:, :, :M] = dev(torch.randn(nb, K, M, generator=g).bfloat16())
+    W, R = dev(torch.randn(N, K, generator=g).bfloat16()), dev(torch.randn(nb, M, N, generator=g).bfloat16())
+    rows, Wt = wide[:, :, :M].transpose(1, 2).float().contiguous(), W.float().t().contiguous()
+    ref = torch.matmul(rows, Wt)                                  # fp32 on the library: K * 2^-24 of the absolute sum too
+    bound = (2 * K + slices) * 2.0 ** -24 * torch.matmul(rows.abs(), Wt.abs()) + 2.0 ** -8 * ref.abs()
+    y = hip.gemm_ta(wide[:, :, :M], W)
+    assert bool(((y.float() - ref).abs() <= bound).all())
+    assert torch.equal(hip.gemm_ta(wide[:, :, :M], W, residual=R), (R.float() + y.float()).bfloat16())
+
+
 @pytest.mark.parametrize("nb,M,N,K,slices", [(1, 128, 132, 4096, 8), (3, 256, 260, 6144, 12), (1, 384, 1024, 3072, 6)])
 def test_gemm_bf16_in_slices(hip, nb, M, N, K, slices):
     """Few output tiles and a long K: both prompt GEMMs in slices of K, plain and with the residual, ragged tiles and strided
