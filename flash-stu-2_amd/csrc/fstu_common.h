@@ -1,5 +1,7 @@
 // Shared device/host helpers for the gfx950 kernels of libflashstu_hip.so.
 #pragma once
+#include <atomic>
+#include <mutex>
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include <stdio.h>
@@ -155,6 +157,22 @@ __device__ __forceinline__ float gelu_tanh_f32(float x) {
   const float kKappa = 0.044715f;
   float inner = kBeta * (x + kKappa * x * x * x);
   return 0.5f * x * (1.0f + tanhf(inner));
+}
+
+// Raises a kernel's limit of dynamic LDS on the current device where a launch needs more than any there before it did.
+struct fstu_lds_limit { std::atomic<int> most[16] = {}; };     // by device
+inline hipError_t fstu_allow_lds(const void* kernel, fstu_lds_limit& limit, int bytes) {
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return e;
+  const bool known = dev >= 0 && dev < 16;
+  if (known && bytes <= limit.most[dev].load(std::memory_order_acquire)) return hipSuccess;
+  static std::mutex one;                                       // a smaller limit does not replace a larger one
+  std::lock_guard<std::mutex> hold(one);
+  if (known && bytes <= limit.most[dev].load(std::memory_order_relaxed)) return hipSuccess;
+  e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+  if (e == hipSuccess && known) limit.most[dev].store(bytes, std::memory_order_release);
+  return e;
 }
 
 #define FSTU_DISPATCH_DTYPE(dtype, NAME, ...)                      \

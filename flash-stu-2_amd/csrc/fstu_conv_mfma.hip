@@ -533,8 +533,8 @@ extern "C" int fstu_stu_conv_mfma(const void* x, const void* taps, void* y, int 
 #define CM_GO(NT, NBS, NW, OCC)                                                                                                     \
   do {                                                                                                                              \
     constexpr int lds__ = (8 >> NBS) * cm_row(NT << NBS, 1 << NBS) + NW * CM_RING;                                                  \
-    static const hipError_t ok =                                                                                                    \
-        hipFuncSetAttribute((const void*)conv_mfma_kernel<NT, NBS, NW, OCC>, hipFuncAttributeMaxDynamicSharedMemorySize, lds__);    \
+    static fstu_lds_limit most;                                                                                                     \
+    const hipError_t ok = fstu_allow_lds((const void*)conv_mfma_kernel<NT, NBS, NW, OCC>, most, lds__);                             \
     FSTU_REQUIRE(ok == hipSuccess, (int)ok, "fstu_stu_conv_mfma: %d bytes of LDS refused: %s", lds__, hipGetErrorString(ok));       \
     hipLaunchKernelGGL((conv_mfma_kernel<NT, NBS, NW, OCC>), grid, dim3(NW * 64), lds__, (hipStream_t)stream, (const bf16_t*)x,     \
                        (const bf16_t*)taps, (bf16_t*)y, B, T, d, single_branch);                                                    \
@@ -570,8 +570,8 @@ extern "C" int fstu_stu_conv_mfma_grad(const void* gy, const void* x, const void
 #define CG_GO(NT)                                                                                                                   \
   do {                                                                                                                              \
     constexpr int lds__ = 16 * cm_region(8 * NT) + 8 * cg_rows(8 * NT) + 8 * 2048;                                                 \
-    static const hipError_t ok =                                                                                                    \
-        hipFuncSetAttribute((const void*)conv_grad_mfma_kernel<NT>, hipFuncAttributeMaxDynamicSharedMemorySize, lds__);             \
+    static fstu_lds_limit most;                                                                                                     \
+    const hipError_t ok = fstu_allow_lds((const void*)conv_grad_mfma_kernel<NT>, most, lds__);                                      \
     FSTU_REQUIRE(ok == hipSuccess, (int)ok, "fstu_stu_conv_mfma_grad: %d bytes of LDS refused: %s", lds__, hipGetErrorString(ok));  \
     hipLaunchKernelGGL((conv_grad_mfma_kernel<NT>), grid, dim3(512), lds__, (hipStream_t)stream, (const bf16_t*)gy, (const bf16_t*)x, \
                        (const bf16_t*)filt, (bf16_t*)gx, gf ? part : nullptr, B, T, L, d, R);                                       \

@@ -2,7 +2,6 @@
 // CU with equal bytes each: the gate/up projection with the GLU epilogue (and the QKV / plain projections on the same
 // launch), optionally with the sub-layer's residual add + RMSNorm as its prologue, and the split-K down projection
 // (flash_stu/modules/swiglu.py:22-29, flash_stu/layers/stu_layer.py:93-96, flash_stu/layers/attention_layer.py:59-62).
-#include <atomic>
 #include <type_traits>
 #include "fstu_common.h"
 #include "fstu_prologue.h"
@@ -659,12 +658,9 @@ extern "C" int fstu_mlp_packed_rows32_supported(int rows, int d, int I) {
          I % 512 == 0 && (size_t)rows * I * 2 < 0x7ff00000ull;
 }
 
-// Raises a kernel's limit of dynamic LDS where a launch needs more than any before it did
-static int allow_lds(const void* kernel, std::atomic<size_t>& most, size_t shm, const char* name) {
-  if (shm <= most.load(std::memory_order_relaxed)) return FSTU_OK;
-  hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
+static int allow_lds(const void* kernel, fstu_lds_limit& limit, size_t shm, const char* name) {
+  const hipError_t e = fstu_allow_lds(kernel, limit, (int)shm);
   FSTU_REQUIRE(e == hipSuccess, (int)e, "%s: %zu bytes of dynamic LDS refused", name, shm);
-  most.store(shm, std::memory_order_relaxed);
   return FSTU_OK;
 }
 
@@ -673,7 +669,7 @@ static int glu_launch_ksa(GluArgs& a, int pro, int epi, int G, size_t shm, const
   if constexpr (KSA <= 4) if (row_major) {       // 1..16 rows behind a norm prologue, widths up to 1024
     auto go = [&](auto which) -> int {              // (a type for each kernel: a record of its own)
       constexpr auto kernel = decltype(which)::value;
-      static std::atomic<size_t> most{0};
+      static fstu_lds_limit most;
       const int rc = allow_lds(reinterpret_cast<const void*>(kernel), most, shm, name);
       if (rc) return rc;
       hipLaunchKernelGGL(kernel, dim3(G), dim3(512), shm, s, a.h, a.wp_gate, a.wp_up, a.act, a.x_in, a.delta, a.x_out, a.norm_w, a.rows,
@@ -685,7 +681,7 @@ static int glu_launch_ksa(GluArgs& a, int pro, int epi, int G, size_t shm, const
   }
 #define GLU_GO(PRO, GLUF)                                                                                        \
   do {                                                                                                           \
-    static std::atomic<size_t> most{0};                                                                          \
+    static fstu_lds_limit most;                                                                          \
     const int rc = allow_lds(reinterpret_cast<const void*>(glu_balanced_kernel<KSA, PRO, GLUF>), most, shm, name); \
     if (rc) return rc;                                                                                           \
     hipLaunchKernelGGL((glu_balanced_kernel<KSA, PRO, GLUF>), dim3(G), dim3(512), shm, s, a.h, a.wp_gate, a.wp_up, a.act, a.x_in,    \
