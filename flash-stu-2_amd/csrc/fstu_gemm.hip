@@ -957,11 +957,11 @@ namespace {
 // The same where the slices can also run on 256 x 256 tiles in the alternating-group kernel (rows, or slabs of whole tiles of them):
 // half the operands' bytes through the LDS for a product, and every compute unit at work where M and N leave it idle.  A k tile of
 // 64 takes those 1 us in a nearly empty round and 1.35 in a full one, which draws the matrix cores' power; 128 x 128 tiles 0.43 us alone on
-// a compute unit and 0.55 to 0.9 of two in pairs.  us before / with the slices it picks (L: large tiles), rows x features x K:
+// a compute unit and, two to a unit, 0.55 to 0.9 in slices and up to 1.05 over a whole long K.  us before / with the slices it picks (L: large tiles), rows x features x K:
 // 1408 x 2048 x 24576 177 / 137 (L4), 1900 213 / 159 (L4), 2500 363 / 203 (L3), 3200 379 / 264 (L2), 4096 400 / 295 (L2), 5000 452 / 398
-// (L3); 5500 x 768 x 9216 99 / 81 (L3), 7000 125 / 95 (L3), 12000 266 / 170 (L3).  Where it stays as it was, with
-// the best slices of large tiles: 1000 x 2048 x 24576 105 / 91 (6), 6100 485 / 498 (4), 4096 x 768 x 9216 66 / 61 (4), 9000 136 / 116
-// (2), 16000 180 / 230 (2), 2500 x 2048 x 2048 31 / 39 (2).  Slabs: 1 x 8192 x 1024 x 24576 451 / 309 (L2), 4 x 2048 454 / 303 (L2), 2 x
+// (L3); 5500 x 768 x 9216 99 / 81 (L3), 7000 125 / 95 (L3), 7700 145 / 121 (L2), 9000 139 / 119 (L2), 12000
+// 266 / 170 (L3); 8300 x 512 x 6144 75 / 60 (L3), 7800 x 1024 x 12288 225 / 161 (L2).  Where it stays as it was, with
+// the best slices of large tiles: 1000 x 2048 x 24576 105 / 91 (6), 6100 485 / 498 (4), 4096 x 768 x 9216 66 / 61 (4), 16000 180 / 230 (2), 2500 x 2048 x 2048 31 / 39 (2).  Slabs: 1 x 8192 x 1024 x 24576 451 / 309 (L2), 4 x 2048 454 / 303 (L2), 2 x
 // 2048 242 / 159 (L4), 1 x 4096 x 768 x 18432 142 / 111 (L4).
 struct SlicePlan { int count; bool large; };
 SlicePlan slice_plan(int M, int N, int K, int nb) {
@@ -979,7 +979,7 @@ SlicePlan slice_plan(int M, int N, int K, int nb) {
   const auto little = [&](int s) {
     if (small * s <= cus) return nkt / s * 0.43 + join(s);
     const long long rounds = (small * s + 2 * cus - 1) / (2 * cus);
-    return rounds * (nkt / s) * (0.55 + 0.35 * (double)(small * s) / (double)(rounds * 2 * cus)) + join(s);
+    return rounds * (nkt / s) * (0.55 + (s == 1 ? 0.5 : 0.35) * (double)(small * s) / (double)(rounds * 2 * cus)) + join(s);
   };
   double least = 0.95 * (before == 1 && 9 * ((big + cus - 1) / cus) * cus < 4 * small ? large(1) : little(before));
   SlicePlan best = {before, false};
