@@ -159,6 +159,17 @@ __device__ __forceinline__ float gelu_tanh_f32(float x) {
   return 0.5f * x * (1.0f + tanhf(inner));
 }
 
+// Compute units of the GPU, 256 where none can be asked.
+inline int fstu_cus() {
+  static const int cus = [] {
+    int dev = 0;
+    hipDeviceProp_t p;
+    if (hipGetDevice(&dev) != hipSuccess || hipGetDeviceProperties(&p, dev) != hipSuccess) return 256;
+    return p.multiProcessorCount;
+  }();
+  return cus;
+}
+
 // Raises a kernel's limit of dynamic LDS on the current device where a launch needs more than any there before it did.
 struct fstu_lds_limit { std::atomic<int> most[16] = {}; };     // by device
 inline hipError_t fstu_allow_lds(const void* kernel, fstu_lds_limit& limit, int bytes) {

@@ -506,6 +506,18 @@ extern "C" int fstu_stu_conv_taps_len(int T) {
   return 64 * (nt << nbs) + 16;
 }
 
+// From the length and the width alone, so that a row has the same bits whatever stands beside it, and one layer's operand of a
+// length is either taps or spectra.  us, product / best of the transforms' kernels: 8 x 100 x 768 7.1 / 7.7, 8 x 512 x 768 10.5 /
+// 16, 32 x 300 x 2048 51 / 100, 1 x 2048 x 768 18 / 23, 8 x 2048 x 768 45 / 61.  Beyond 2048 positions a workgroup fills a compute
+// unit, and its 38 us pay for themselves where a round of workgroups is filled by 70 % with any number of rows: 1 x 4096 x 2048
+// 45 / 56, 4 x 4096 x 2048 167 / 204.  A width of 1024 would gain with two rows and lose with one (36 / 32), of 768 lose with three
+// (75 / 63).  Beyond 4096 the product's operations, which grow with the square of the length, cost more than the transforms.
+extern "C" int fstu_stu_conv_mfma_takes(int T, int d) {
+  if (T < 32 || T > 4096 || d < 8 || d % 8 != 0 || d > 1 << 20) return 0;
+  const int groups = d / 8, cus = fstu_cus();
+  return T <= 2048 || 10 * groups >= 7 * cus * ((groups + cus - 1) / cus);
+}
+
 extern "C" int fstu_stu_conv_taps(const void* filt, void* taps, int L, int d, int S, void* stream) {
   FSTU_REQUIRE(filt && taps, FSTU_ENULL, "fstu_stu_conv_taps: null pointer");
   FSTU_REQUIRE(L >= 1 && d >= 8 && d % 8 == 0 && d <= 1 << 20 && S >= 80 && S <= 2064 && S % 64 == 16, FSTU_ESHAPE,

@@ -110,15 +110,7 @@ __device__ __forceinline__ void store_feat4(bf16_t* p, int left, unsigned lo, un
   }
 }
 
-int gemm_cus() {
-  static int cus = [] {
-    int dev = 0;
-    hipDeviceProp_t p;
-    if (hipGetDevice(&dev) != hipSuccess || hipGetDeviceProperties(&p, dev) != hipSuccess) return 256;
-    return p.multiProcessorCount;
-  }();
-  return cus;
-}
+int gemm_cus() { return fstu_cus(); }
 
 template <int WFN_, int WTN_, int FI_, int TJ_, int BK_, int NS_>
 struct GemmTile {

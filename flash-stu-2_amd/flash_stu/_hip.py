@@ -54,6 +54,7 @@ SIGNATURES = {
     "fstu_fft_length": [_i],
     "fstu_fft_twiddles": [_vp, _i, _vp],
     "fstu_stu_fft_filter": [_vp, _i64, _i64, _vp, _vp, _i, _i, _i, _i, _i, _vp],
+    "fstu_stu_conv_mfma_takes": [_i, _i],
     "fstu_stu_conv_taps_len": [_i],
     "fstu_stu_conv_taps": [_vp, _vp, _i, _i, _i, _vp],
     "fstu_stu_conv_mfma_grad_ws": [_i, _i, _i, _i],
@@ -751,17 +752,16 @@ def stu_conv_taps_len(T: int) -> int:
     return int(load().fstu_stu_conv_taps_len(int(T)))
 
 
-def stu_conv_mfma_takes(B: int, T: int, d: int, dtype: torch.dtype) -> bool:
-    """Whether the convolution of (B,T,d) runs as a Toeplitz product (stu_conv_mfma) or through transforms: bf16, T up to 4096.
-    us, product / best of the transforms' kernels: 8 x 100 x 768 7.1 / 7.7, 8 x 512 x 768 10.5 / 16, 32 x 300 x 2048 51 / 100,
-    1 x 2048 x 768 18 / 23, 8 x 2048 x 768 45 / 61.  Beyond 2048 positions a workgroup fills a compute unit, and its 38 us pay
-    for themselves where a round of 256 of them is filled by 70 %: 1 x 4096 x 2048 45 / 56, 2 x 4096 x 768 41 / 45, 4 x 4096 x
-    2048 167 / 204, but 1 x 4096 x 1024 36 / 32 and 3 x 4096 x 768 75 / 63.  Beyond 4096 the product's operations, which grow
-    with the square of the length, cost more than the transforms."""
-    if dtype != torch.bfloat16 or not 32 <= T <= 4096 or d % 8 != 0:
-        return False
-    groups = B * (d // 8)
-    return T <= 2048 or 10 * groups >= 7 * 256 * -(-groups // 256)
+@functools.lru_cache(maxsize=256)
+def _conv_mfma_takes(T: int, d: int) -> bool:
+    return bool(load().fstu_stu_conv_mfma_takes(T, d))
+
+
+def stu_conv_mfma_takes(T: int, d: int, dtype: torch.dtype) -> bool:
+    """Whether the convolution of (B,T,d) runs as a Toeplitz product (stu_conv_mfma) or through transforms: bf16, up to 2048
+    positions, and up to 4096 in widths that fill the chip.  The number of rows has no part in it: both forms' results differ in
+    their last bits."""
+    return dtype == torch.bfloat16 and _conv_mfma_takes(T, d)
 
 
 def stu_conv_taps(filt: torch.Tensor, S: int) -> torch.Tensor:

@@ -273,10 +273,10 @@ class STU(nn.Module):
 
     def _convolve(self, xp: torch.Tensor) -> torch.Tensor:
         """Approx-mode convolution of the projected inputs with phi_proj (stu.py:89-98,120): from FFT_MIN_T positions on the
-        Toeplitz product on the matrix cores (bf16, up to 4096 positions) or the FFT form of the reference, the time-domain
-        kernel for shorter inputs and for lengths beyond the longest in-LDS transform."""
+        Toeplitz product on the matrix cores (bf16, up to 2048 positions, 4096 in wide layers) or the FFT form of the reference,
+        whatever the number of rows, the time-domain kernel for shorter inputs and for lengths beyond the longest in-LDS transform."""
         T = xp.shape[1]
-        if _hip.stu_conv_mfma_takes(*xp.shape, xp.dtype):
+        if _hip.stu_conv_mfma_takes(T, xp.shape[2], xp.dtype):
             return _hip.stu_conv_mfma(xp, self.filter_taps(T), single_branch=self.use_hankel_L)
         n = _hip.fft_length(T) if T >= FFT_MIN_T else 0
         if n == 0:
@@ -398,7 +398,7 @@ class STU(nn.Module):
             if self.use_approx:
                 xt = None
                 if (not use_cache and self._few_long_sequences(B, T, self.d_out, x.element_size())
-                        and not _hip.stu_conv_mfma_takes(B, T, self.d_out, x.dtype)):
+                        and not _hip.stu_conv_mfma_takes(T, self.d_out, x.dtype)):
                     xt = self._project_time_major(x)       # no transpose in front of the time-major convolution
                 if xt is not None:
                     return self._convolve_time_major(xt, _hip.fft_length(T))

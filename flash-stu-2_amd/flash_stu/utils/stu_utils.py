@@ -170,7 +170,7 @@ class ApproxConvolveSum(torch.autograd.Function):
     @staticmethod
     def forward(ctx, u, v):
         from .. import _hip
-        if v.dtype == u.dtype and _hip.stu_conv_mfma_takes(*u.shape, u.dtype):
+        if v.dtype == u.dtype and _hip.stu_conv_mfma_takes(u.shape[1], u.shape[2], u.dtype):
             ctx.save_for_backward(u, v, None)
             return _hip.stu_conv_mfma(_aligned(u), _hip.stu_conv_taps(_aligned(v), _hip.stu_conv_taps_len(u.shape[1])))
         n = _conv_length(u.shape[1])

@@ -279,7 +279,9 @@ int fstu_stu_conv_fft_strided(const void* xp, const int64_t* x_strides, const fl
 /* The same convolution as a Toeplitz product on the matrix cores: bf16, T up to 4096, d a multiple of 8, 16-byte aligned
  * contiguous operands.  taps (d, 2, S) bf16, S = fstu_stu_conv_taps_len(T) (0: T is not taken), holds the columns of filt (L, d)
  * time-major, the even and the odd lags apart, reversed and padded with zeros; fstu_stu_conv_taps writes it.
- * y[b,t,c] = T( T(plus) + T(minus) ) (or T(plus) if single_branch), each position's bits the same whatever T and B. */
+ * y[b,t,c] = T( T(plus) + T(minus) ) (or T(plus) if single_branch), each position's bits the same whatever T and B.
+ * fstu_stu_conv_mfma_takes says where it is the faster form, for any number of rows (its last bits are not the transforms'). */
+int fstu_stu_conv_mfma_takes(int T, int d);
 int fstu_stu_conv_taps_len(int T);
 int fstu_stu_conv_taps(const void* filt, void* taps, int L, int d, int S, void* stream);
 int fstu_stu_conv_mfma(const void* x, const void* taps, void* y, int B, int T, int d, int single_branch, void* stream);

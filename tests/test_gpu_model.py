@@ -658,6 +658,33 @@ def test_derived_tensors_outlive_what_other_streams_read():
     assert torch.equal(there, want)
 
 
+@pytest.mark.parametrize("T,d", [(2049, 512), (3000, 768), (4096, 1024), (2100, 1536), (4096, 2048), (300, 256)])
+def test_operator_rows_and_graphs_do_not_depend_on_the_rows_of_other_calls(T, d):
+    """A row of the operator has the bits that it has alone, and a graph captured for one row still gives them after calls of
+    other numbers of rows and other memory filled."""
+    from flash_stu import STU, FlashSTUConfig
+    cfg = FlashSTUConfig(n_embd=d, n_heads=d // 64, n_layers=2, seq_len=4096, num_eigh=8, vocab_size=64, torch_dtype=torch.bfloat16)
+    g = torch.Generator().manual_seed(T)
+    stu = STU(cfg, (torch.randn(4096, 8, generator=g) / 64).bfloat16(), 8192).cuda()
+    with torch.no_grad():
+        for p in stu.parameters():
+            p.copy_(torch.randn(p.shape, generator=g) * d ** -0.5)
+    xp = torch.randn(5, T, d, generator=g).bfloat16().cuda()
+    one = xp[:1].clone()
+    with torch.no_grad():
+        want = [stu._convolve(xp[b:b + 1].contiguous()) for b in range(5)]
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            y = stu._convolve(one)
+        for rows in (2, 3, 5):
+            assert torch.equal(stu._convolve(xp[:rows].contiguous()), torch.cat(want[:rows]))
+            fills = [torch.full((d, n), 7.0, device="cuda") for n in (2064 * 2, 4096, 8192 * 2)]
+            one.copy_(xp[rows - 1:rows])
+            graph.replay()
+            assert torch.equal(y, want[rows - 1])
+            del fills
+
+
 @pytest.mark.parametrize("dtype,T", [(torch.bfloat16, 300), (torch.float32, 20), (torch.float32, 100)])
 def test_tensors_derived_under_capture_stay_in_the_graph(dtype, T, monkeypatch):
     """The first call on new weights inside a capture: calls beside the graph do not read what only its replay writes, and

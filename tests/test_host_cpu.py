@@ -285,3 +285,38 @@ def test_weights_whose_changes_cannot_be_seen_are_refused():
         for derive in (stu.m_inputs_t, stu.effective_filter):
             with pytest.raises(RuntimeError, match="version counter"):
                 derive()
+
+
+def _operand_stand_ins(monkeypatch):
+    """STU._convolve without a GPU: its kernels return their first operand, its operands are empty tensors of the real shapes."""
+    from flash_stu import _hip
+    monkeypatch.setattr(_hip, "gemm_any", lambda a, w: torch.empty(a.shape[0], w.shape[0], dtype=a.dtype))
+    monkeypatch.setattr(_hip, "stu_fft_filter", lambda f, n, single_branch=False: torch.empty(f.shape[1], n, 2))
+    monkeypatch.setattr(_hip, "stu_conv_taps", lambda f, S: torch.empty(f.shape[1], 2, S, dtype=f.dtype))
+    monkeypatch.setattr(_hip, "transpose", lambda t: t.transpose(1, 2).contiguous())
+    for name in ("stu_conv_mfma", "stu_conv_fft", "stu_conv_fft_strided", "stu_conv_direct"):
+        monkeypatch.setattr(_hip, name, lambda x, *a, **kw: x)
+
+
+def _bf16_stu(d, L):
+    from flash_stu import STU, FlashSTUConfig
+    cfg = FlashSTUConfig(n_embd=d, n_heads=1, n_layers=2, seq_len=L, num_eigh=4, vocab_size=64, torch_dtype=torch.bfloat16)
+    stu = STU(cfg, torch.randn(L, 4).bfloat16(), 2 * L)
+    for p in stu.parameters():
+        torch.nn.init.normal_(p)
+    return stu
+
+
+@pytest.mark.parametrize("d", [8, 256, 512, 768, 1024, 1280, 1536, 2048, 2560])
+def test_operand_of_the_convolution_is_one_for_every_number_of_rows(d, monkeypatch):
+    """A captured graph holds the address of the operand that its call read: calls of the same length with other numbers of rows,
+    each the form that it takes, read the same one."""
+    _operand_stand_ins(monkeypatch)
+    stu = _bf16_stu(d, 4096)
+    for T in (32, 700, 2048, 2049, 3000, 4096):
+        with torch.no_grad():
+            stu._convolve(torch.empty(1, T, d, dtype=torch.bfloat16))
+            first = stu._derived["spec"][1]
+            for rows in (2, 3, 4, 5, 9):
+                stu._convolve(torch.empty(rows, T, d, dtype=torch.bfloat16))
+                assert stu._derived["spec"][1] is first, (T, rows)
