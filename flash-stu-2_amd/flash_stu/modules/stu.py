@@ -68,10 +68,15 @@ class STU(nn.Module):
     # made from, so that no other tensor can come to lie at the address it is recognised by (a parametrized weight is a
     # new tensor on every access).  A call on another stream than the one that launched the copy waits for it, and its memory
     # is not given out again before that stream has read it.
-    def _cached(self, key, params, build):
-        ver = tuple((p._version, p.data_ptr()) for p in params)
+    # `form` tells what else an entry was made for (the length of a convolution): one form is kept, and an entry is looked up once,
+    # so that calls of other forms in other threads cannot come in between.
+    def _cached(self, key, params, build, form=None):
+        ver = (form, *((p._version, p.data_ptr()) for p in params))
         hit = self._derived.get(key)
         if hit is None or hit[0] != ver:
+            if hit is not None and hit[0][0] != form and not (params[0].is_cuda and torch.cuda.is_current_stream_capturing()):
+                self._derived.pop(key, None)     # its memory first
+                hit = None
             # behind the sources: the device, the handles of the streams that are behind the launch and of the one that made
             # it (an event recorded here would delay the first call by some 16 us, the stream objects by 9)
             dev, value, here = params[0].device, build(), None
@@ -117,19 +122,13 @@ class STU(nn.Module):
         exact mode (the reference keeps its own phi_fft the same way, stu.py:43-53).  One length is kept."""
         src = self.effective_filter() if self.use_approx else self.phi
         params = (self.phi, self.M_filters) if self.use_approx else (self.phi,)
-        hit = self._derived.get("spec")
-        if hit is not None and hit[1].shape[1] != n:
-            self._derived.pop("spec")
-        return self._cached("spec", params, lambda: _hip.stu_fft_filter(src, n, single_branch=self.use_hankel_L))
+        return self._cached("spec", params, lambda: _hip.stu_fft_filter(src, n, single_branch=self.use_hankel_L), form=n)
 
     def filter_taps(self, T: int) -> torch.Tensor:
         """The convolution filters as the Toeplitz product reads them for T positions, (d,2,S) (approx mode, bf16).  In the place
         of the spectra: one operand of the convolution is kept, for one length."""
         S = _hip.stu_conv_taps_len(T)
-        hit = self._derived.get("spec")
-        if hit is not None and hit[1].shape[2] != S:
-            self._derived.pop("spec")
-        return self._cached("spec", (self.phi, self.M_filters), lambda: _hip.stu_conv_taps(self.effective_filter(), S))
+        return self._cached("spec", (self.phi, self.M_filters), lambda: _hip.stu_conv_taps(self.effective_filter(), S), form=-S)
 
     def m_inputs_eff(self) -> torch.Tensor:
         """M_inputs as the forward uses it: the parameter itself, or its block-diagonal part when tiling is on."""

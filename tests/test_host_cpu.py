@@ -320,3 +320,35 @@ def test_operand_of_the_convolution_is_one_for_every_number_of_rows(d, monkeypat
             for rows in (2, 3, 4, 5, 9):
                 stu._convolve(torch.empty(rows, T, d, dtype=torch.bfloat16))
                 assert stu._derived["spec"][1] is first, (T, rows)
+
+
+def test_operands_of_several_lengths_in_several_threads(monkeypatch):
+    """Calls of other lengths that replace or drop the kept operand at any point of a call: each call gets its own length's, and one of
+    the same length stays."""
+    _operand_stand_ins(monkeypatch)
+    stu = _bf16_stu(64, 4096)
+    with torch.no_grad():
+        other = {T: (lambda T=T: stu.filter_taps(T) if T <= 2048 else stu.filter_spectrum(2 * T)) for T in (300, 2048, 4096)}
+        kept = {}
+        for T, form in other.items():
+            form()
+            kept[T] = stu._derived["spec"]
+
+        class Replaced(dict):
+            after = None                       # what another thread leaves behind each look
+            def get(self, key, default=None):
+                hit = super().get(key, default)
+                if key == "spec":
+                    if self.after is None:
+                        super().pop(key, None)
+                    else:
+                        self[key] = self.after
+                return hit
+        for T, form in other.items():
+            for before in (None, *kept.values()):
+                for after in (None, *kept.values()):
+                    stu._derived = Replaced({} if before is None else {"spec": before})
+                    stu._derived.after = after
+                    assert form().shape == kept[T][1].shape
+        stu._derived = {"spec": kept[300]}
+        assert stu.filter_taps(300) is stu.filter_taps(257) is kept[300][1]
