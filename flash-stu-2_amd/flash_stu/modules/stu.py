@@ -270,12 +270,17 @@ class STU(nn.Module):
             y = _hip.gemm(x2, w) if _hip.gemm_supported(x2, w) else _hip.gemm_any(x2, w)
         return y.reshape(B, T, self.d_out)
 
+    def _as_product(self, T: int, dtype: torch.dtype) -> bool:
+        """Whether T positions are convolved as a Toeplitz product, whose both operands are bf16: filters kept in fp32 beside bf16
+        inputs go through transforms."""
+        return _hip.stu_conv_mfma_takes(T, self.d_out, dtype) and self.phi.dtype == self.M_filters.dtype == dtype
+
     def _convolve(self, xp: torch.Tensor) -> torch.Tensor:
         """Approx-mode convolution of the projected inputs with phi_proj (stu.py:89-98,120): from FFT_MIN_T positions on the
         Toeplitz product on the matrix cores (bf16, up to 2048 positions, 4096 in wide layers) or the FFT form of the reference,
         whatever the number of rows, the time-domain kernel for shorter inputs and for lengths beyond the longest in-LDS transform."""
         T = xp.shape[1]
-        if _hip.stu_conv_mfma_takes(T, xp.shape[2], xp.dtype):
+        if self._as_product(T, xp.dtype):
             return _hip.stu_conv_mfma(xp, self.filter_taps(T), single_branch=self.use_hankel_L)
         n = _hip.fft_length(T) if T >= FFT_MIN_T else 0
         if n == 0:
@@ -397,7 +402,7 @@ class STU(nn.Module):
             if self.use_approx:
                 xt = None
                 if (not use_cache and self._few_long_sequences(B, T, self.d_out, x.element_size())
-                        and not _hip.stu_conv_mfma_takes(T, self.d_out, x.dtype)):
+                        and not self._as_product(T, x.dtype)):
                     xt = self._project_time_major(x)       # no transpose in front of the time-major convolution
                 if xt is not None:
                     return self._convolve_time_major(xt, _hip.fft_length(T))

@@ -685,6 +685,27 @@ def test_operator_rows_and_graphs_do_not_depend_on_the_rows_of_other_calls(T, d)
             del fills
 
 
+@pytest.mark.parametrize("T", [64, 700, 4096])
+def test_fp32_filters_beside_bf16_inputs(T):
+    """Filters and their projection kept in fp32, inputs and M_inputs in bf16: the convolution against float64 sums of the same
+    operands, fp32 transforms (1e-6 of the largest sum is five times their error) and each branch and the sum of both rounded once."""
+    from flash_stu import STU, FlashSTUConfig
+    cfg = FlashSTUConfig(n_embd=2048, n_heads=32, n_layers=2, seq_len=4096, num_eigh=8, vocab_size=64, torch_dtype=torch.bfloat16)
+    g = torch.Generator().manual_seed(T)
+    stu = STU(cfg, (torch.randn(4096, 8, generator=g) / 64).bfloat16(), 8192).cuda()
+    with torch.no_grad():
+        for p in stu.parameters():
+            p.copy_(torch.randn(p.shape, generator=g) * 2048 ** -0.5)
+    stu.phi, stu.M_filters.data = stu.phi.float(), stu.M_filters.data.float()
+    x = torch.randn(1, T, 2048, generator=g).bfloat16().cuda()
+    y = stu(x).double()
+    xp, f = stu._project(x).double(), stu.effective_filter().double()
+    n, sgn = 2 * T, (-1.0) ** torch.arange(T, device="cuda", dtype=torch.float64)[:, None]
+    plus, minus = (torch.fft.irfft(torch.fft.rfft(xp, n, 1) * torch.fft.rfft(v, n, 0), n, 1)[:, :T] for v in (f[:T], f[:T] * sgn))
+    bound = 2.0 ** -8 * (plus.abs() + minus.abs() + (plus + minus).abs()) + 1e-6 * float(plus.abs().max())
+    assert bool(((y - plus - minus).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("dtype,T", [(torch.bfloat16, 300), (torch.float32, 20), (torch.float32, 100)])
 def test_tensors_derived_under_capture_stay_in_the_graph(dtype, T, monkeypatch):
     """The first call on new weights inside a capture: calls beside the graph do not read what only its replay writes, and
