@@ -562,6 +562,15 @@ extern "C" int fstu_stu_conv_mfma(const void* x, const void* taps, void* y, int 
   return FSTU_OK;
 }
 
+// Up to 192 positions an item is latency (a workgroup's tiles are made for 1024), and from some rows on the transforms' launches are
+// shorter.  GPU us of a whole training step with both directions as products / as transforms, rows x positions x channels: 8 x 64 x 768
+// 79.5 / 78.3, 32 x 64 x 768 117 / 99, 8 x 100 x 768 73 / 76, 24 x 100 x 768 108 / 104, 16 x 128 x 1024 117 / 116, 64 x 128 x 2048 416 / 328,
+// 4 x 200 x 512 63 / 76, 8 x 200 x 768 94 / 101, 16 x 200 x 1024 124 / 127, 64 x 256 x 1024 265 / 267, 8 x 300 x 768 100 / 113.
+extern "C" int fstu_stu_conv_mfma_grad_takes(int B, int T, int d, int L) {
+  if (B < 1 || T < 32 || T > 2048 || d < 8 || d % 8 != 0 || d > 1 << 20 || L < 1 || (int64_t)L * d >= 1ll << 31) return 0;
+  return T > 192 || (long long)B * (d / 8) <= 4 * fstu_cus();
+}
+
 extern "C" int64_t fstu_stu_conv_mfma_grad_ws(int B, int T, int d, int L) {
   if (B < 1 || T < 1 || T > 2048 || d < 8 || L < 1) return 0;
   const int R = cg_items(B, T, d), lags = ((L < T ? L : T) + 1) / 2;

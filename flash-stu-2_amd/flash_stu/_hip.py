@@ -57,6 +57,7 @@ SIGNATURES = {
     "fstu_stu_conv_mfma_takes": [_i, _i],
     "fstu_stu_conv_taps_len": [_i],
     "fstu_stu_conv_taps": [_vp, _vp, _i, _i, _i, _vp],
+    "fstu_stu_conv_mfma_grad_takes": [_i, _i, _i, _i],
     "fstu_stu_conv_mfma_grad_ws": [_i, _i, _i, _i],
     "fstu_stu_conv_mfma_grad": [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _vp],
     "fstu_stu_conv_mfma": [_vp, _vp, _vp, _i, _i, _i, _i, _vp],
@@ -786,11 +787,15 @@ def stu_conv_mfma(xp: torch.Tensor, taps: torch.Tensor, single_branch: bool = Fa
     return out
 
 
-def stu_conv_mfma_grad_takes(B: int, T: int, d: int, dtype: torch.dtype) -> bool:
-    """Whether the gradients of plus + minus are formed on the matrix cores: bf16, T up to 2048.  us, there / through transforms:
-    1 x 300 x 768 12.6 / 14.8, 4 x 600 x 768 17 / 26, 8 x 1025 x 768 38 / 82, 8 x 2048 x 768 62 / 117.  Up to 256 positions a
-    workgroup's latency decides, and more than 256 of them lose: 4 x 200 x 512 12.7 / 13.9, but 8 x 200 x 768 17.5 / 15."""
-    return dtype == torch.bfloat16 and 32 <= T <= 2048 and d % 8 == 0 and (T > 256 or B * (d // 8) <= 256)
+@functools.lru_cache(maxsize=256)
+def _conv_mfma_grad_takes(B: int, T: int, d: int, L: int) -> bool:
+    return bool(load().fstu_stu_conv_mfma_grad_takes(B, T, d, L))
+
+
+def stu_conv_mfma_grad_takes(B: int, T: int, d: int, L: int, dtype: torch.dtype) -> bool:
+    """Whether the gradients of plus + minus of (B,T,d) and (L,d) are formed on the matrix cores: bf16, up to 2048 positions, but
+    not for many short rows.  A training step's forward goes the same way, so that the filter is laid out once."""
+    return dtype == torch.bfloat16 and _conv_mfma_grad_takes(B, T, d, L)
 
 
 def stu_conv_mfma_grad(gy: torch.Tensor, x: torch.Tensor, filt: torch.Tensor, want_x: bool = True, want_filter: bool = True):

@@ -101,11 +101,11 @@ def _convolve_grads(ctx, u, v, spec, gp, gm, branches):
     from .. import _hip
     want_u, want_v = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
     graph = torch.is_grad_enabled()
-    if branches == 0 and not graph and v.dtype == u.dtype == gp.dtype and _hip.stu_conv_mfma_grad_takes(*u.shape, u.dtype):
+    if branches == 0 and not graph and v.dtype == u.dtype == gp.dtype and _hip.stu_conv_mfma_grad_takes(*u.shape, v.shape[0], u.dtype):
         return _hip.stu_conv_mfma_grad(_aligned(gp), _aligned(u), _aligned(v), want_u, want_v)
     n = _conv_length(u.shape[1])
     if spec is None and n and not graph:
-        spec = _hip.stu_fft_filter(v.contiguous(), n)            # the forward was a Toeplitz product
+        spec = _hip.stu_fft_filter(v.contiguous(), n)            # the forward was a Toeplitz product of more than 2048 positions
     if spec is not None and not graph:
         return _hip.stu_conv_fft_grad(gp.contiguous(), gm.contiguous() if branches == 2 else None, u.contiguous(), spec,
                                       v.shape[0], branches, want_u, want_v)
@@ -170,7 +170,12 @@ class ApproxConvolveSum(torch.autograd.Function):
     @staticmethod
     def forward(ctx, u, v):
         from .. import _hip
-        if v.dtype == u.dtype and _hip.stu_conv_mfma_takes(u.shape[1], u.shape[2], u.dtype):
+        # The form that the gradients will take, so that the filter is laid out once.  Beyond 2048 positions their only form are the
+        # transforms, and a product in front of them pays for their spectra: GPU us of a step, 2 x 3000 x 2048 540 / 549 with
+        # transforms in both directions, 1 x 4096 x 1536 337 / 347.
+        B, T, d = u.shape
+        if v.dtype == u.dtype and (_hip.stu_conv_mfma_grad_takes(B, T, d, v.shape[0], u.dtype) if T <= 2048 else
+                                   _hip.stu_conv_mfma_takes(T, d, u.dtype)):
             ctx.save_for_backward(u, v, None)
             return _hip.stu_conv_mfma(_aligned(u), _hip.stu_conv_taps(_aligned(v), _hip.stu_conv_taps_len(u.shape[1])))
         n = _conv_length(u.shape[1])

@@ -288,6 +288,7 @@ int fstu_stu_conv_mfma(const void* x, const void* taps, void* y, int B, int T, i
 /* Gradients of y = plus + minus on the matrix cores, under the conditions of fstu_stu_conv_mfma and for T up to 2048: gy, x
  * (B,T,d) and filt (L,d) -> gx (B,T,d) and gf (L,d), each skipped where null; gf needs part, fp32 scratch of
  * fstu_stu_conv_mfma_grad_ws elements.  Sums in fp32, one rounding at the end, the same bits every time. */
+int fstu_stu_conv_mfma_grad_takes(int B, int T, int d, int L);   /* where it is the faster form of a whole step */
 int64_t fstu_stu_conv_mfma_grad_ws(int B, int T, int d, int L);
 int fstu_stu_conv_mfma_grad(const void* gy, const void* x, const void* filt, void* gx, void* gf, float* part, int B, int T, int d,
                             int L, void* stream);

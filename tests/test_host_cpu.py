@@ -352,3 +352,25 @@ def test_operands_of_several_lengths_in_several_threads(monkeypatch):
                     assert form().shape == kept[T][1].shape
         stu._derived = {"spec": kept[300]}
         assert stu.filter_taps(300) is stu.filter_taps(257) is kept[300][1]
+
+
+@pytest.mark.parametrize("B,T,d", [(1, 64, 768), (8, 64, 768), (32, 100, 768), (8, 192, 1032), (8, 200, 768), (8, 256, 768), (64, 256, 1024),
+                                   (8, 257, 768), (3, 2048, 64), (2, 300, 12), (2, 20, 64)])
+def test_training_step_lays_its_filter_out_once(B, T, d, monkeypatch):
+    """The convolution of a training step and its gradients are both products or both transforms: taps or spectra, not both."""
+    from flash_stu import _hip
+    from flash_stu.utils.stu_utils import ApproxConvolveSum
+    made = []
+
+    def stand_in(name, result):
+        monkeypatch.setattr(_hip, name, lambda *a, **kw: (made.append(name), result(*a))[1])
+    stand_in("stu_conv_taps", lambda v, S: v.new_empty(v.shape[1], 2, S))
+    stand_in("stu_fft_filter", lambda v, n: torch.empty(v.shape[1], n, 2))
+    for name in ("stu_conv_mfma", "stu_conv_fft", "stu_conv_direct", "_causal_conv"):
+        monkeypatch.setattr(_hip, name, lambda x, *a, **kw: x.clone(), raising=False)
+    stand_in("stu_conv_mfma_grad", lambda g, x, v, *a: (g, torch.zeros_like(v)))
+    stand_in("stu_conv_fft_grad", lambda g, m, x, s, L, *a: (g, g.new_zeros(L, g.shape[2])))
+    u, v = torch.zeros(B, T, d).bfloat16().requires_grad_(True), torch.zeros(T, d).bfloat16().requires_grad_(True)
+    ApproxConvolveSum.apply(u, v).sum().backward()
+    assert made in (["stu_conv_taps", "stu_conv_mfma_grad"], ["stu_fft_filter", "stu_conv_fft_grad"], []), made
+    assert (made == []) == (T < 32)
