@@ -325,6 +325,16 @@ def _gemm_head_rows(M: int, N: int, K: int) -> int:
     return load().fstu_gemm_bf16_head_rows(M, N, K)
 
 
+def _slice_sums(slices: int, *shape: int, device):
+    """(slices, memory for their fp32 sums), up to 134 MB; one slice, which needs none, where that is not to be had."""
+    if slices > 1:
+        try:
+            return slices, torch.empty(slices, *shape, dtype=torch.float32, device=device)
+        except torch.OutOfMemoryError:
+            pass
+    return 1, None
+
+
 def gemm(x2: torch.Tensor, weight: torch.Tensor, up_weight: Optional[torch.Tensor] = None,
          residual: Optional[torch.Tensor] = None, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """x2 (M,K) @ weight (N,K)^T on the matrix cores (bf16).  up_weight: the gated pair
@@ -367,9 +377,7 @@ def _gemm_rows(x2, weight, up_weight, residual, out, mode: int, ldr: int) -> Non
     (M, K), N = x2.shape, weight.shape[0]
     slices, partial = 1, None
     if K >= GEMM_MIN_SLICED_K and mode != 1 and out.stride(0) % 4 == 0 and out.data_ptr() % 8 == 0:
-        slices = _gemm_row_slices(M, N, K)
-        if slices > 1:
-            partial = torch.empty(slices, M, N, dtype=torch.float32, device=x2.device)
+        slices, partial = _slice_sums(_gemm_row_slices(M, N, K), M, N, device=x2.device)
     _check(load().fstu_gemm_bf16_ws(_p(x2), x2.stride(0), _p(weight), _p(up_weight), _p(residual), ldr, _p(out), out.stride(0),
                                     M, N, K, mode, _p(partial), slices, _stream()), "fstu_gemm_bf16")
 
@@ -418,8 +426,7 @@ def gemm_ta(slabs: torch.Tensor, weight: torch.Tensor, residual: Optional[torch.
         if t is not None and (t.shape != (nb, M, N) or t.stride(2) != 1 or t.dtype != slabs.dtype):
             raise FlashSTUHipError(f"gemm_ta: {name} must be (nb, M, N) with contiguous rows")
     mode = 2 if residual is not None else 0
-    slices = _gemm_slab_slices(M, N, K, nb) if K >= GEMM_MIN_SLICED_K else 1
-    partial = torch.empty(slices, nb, M, N, dtype=torch.float32, device=slabs.device) if slices > 1 else None
+    slices, partial = _slice_sums(_gemm_slab_slices(M, N, K, nb) if K >= GEMM_MIN_SLICED_K else 1, nb, M, N, device=slabs.device)
     _check(load().fstu_gemm_bf16_ta_ws(_p(slabs), slabs.stride(1), slabs.stride(0) if nb > 1 else 0, _p(weight), _p(residual),
                                        residual.stride(1) if residual is not None else 0,
                                        residual.stride(0) if residual is not None and nb > 1 else 0, _p(out), out.stride(1),

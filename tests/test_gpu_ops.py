@@ -325,6 +325,27 @@ def test_gemm_bf16_slabs_in_slices_of_large_tiles(hip, nb, M, N, K, slices):
     assert torch.equal(hip.gemm_ta(wide[:, :, :M], W, residual=R), (R.float() + y.float()).bfloat16())
 
 
+@pytest.mark.parametrize("M,N,K", [(400, 4100, 8192), (300, 768, 9216)])
+def test_gemm_bf16_without_memory_for_the_slices(hip, M, N, K, monkeypatch):
+    """Products whose K pays in slices, on large tiles and on small ones, where the slices' fp32 sums cannot be allocated: K in one
+    piece.  fp32 sums of exact products stay within K * 2^-24 of the absolute sum, one rounding to bf16."""
+    assert hip._gemm_row_slices(M, N, K) > 1 and hip._gemm_slab_slices(512, N, K, 1) > 1
+    g = gen(M)
+    A, W = dev(torch.randn(512, K, generator=g).bfloat16()), dev(torch.randn(N, K, generator=g).bfloat16())
+    Wt, slab = W.float().t().contiguous(), A.t().contiguous()[None]
+    ref, mag = torch.matmul(A.float(), Wt), torch.matmul(A.float().abs(), Wt.abs())
+    bound = 2 * K * 2.0 ** -24 * mag + 2.0 ** -8 * ref.abs()
+    empty = torch.empty
+
+    def short(*shape, dtype=None, **kw):
+        if dtype == torch.float32:
+            raise torch.OutOfMemoryError()
+        return empty(*shape, dtype=dtype, **kw)
+    monkeypatch.setattr(torch, "empty", short)
+    assert bool(((hip.gemm(A[:M], W).float() - ref[:M]).abs() <= bound[:M]).all())
+    assert bool(((hip.gemm_ta(slab, W)[0].float() - ref).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("nb,M,N,K,slices", [(1, 128, 132, 4096, 8), (3, 256, 260, 6144, 12), (1, 384, 1024, 3072, 6)])
 def test_gemm_bf16_in_slices(hip, nb, M, N, K, slices):
     """Few output tiles and a long K: both prompt GEMMs in slices of K, plain and with the residual, ragged tiles and strided
