@@ -185,6 +185,12 @@ inline hipError_t fstu_allow_lds(const void* kernel, fstu_lds_limit& limit, int 
   if (e == hipSuccess && known) limit.most[dev].store(bytes, std::memory_order_release);
   return e;
 }
+// The same as an entry point's return code, with its message.
+inline int fstu_need_lds(const void* kernel, fstu_lds_limit& limit, size_t bytes, const char* name) {
+  const hipError_t e = fstu_allow_lds(kernel, limit, (int)bytes);
+  FSTU_REQUIRE(e == hipSuccess, (int)e, "%s: %zu bytes of dynamic LDS refused: %s", name, bytes, hipGetErrorString(e));
+  return FSTU_OK;
+}
 
 #define FSTU_DISPATCH_DTYPE(dtype, NAME, ...)                      \
   do {                                                             \

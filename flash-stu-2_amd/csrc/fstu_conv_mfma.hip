@@ -546,8 +546,8 @@ extern "C" int fstu_stu_conv_mfma(const void* x, const void* taps, void* y, int 
   do {                                                                                                                              \
     constexpr int lds__ = (8 >> NBS) * cm_row(NT << NBS, 1 << NBS) + NW * CM_RING;                                                  \
     static fstu_lds_limit most;                                                                                                     \
-    const hipError_t ok = fstu_allow_lds((const void*)conv_mfma_kernel<NT, NBS, NW, OCC>, most, lds__);                             \
-    FSTU_REQUIRE(ok == hipSuccess, (int)ok, "fstu_stu_conv_mfma: %d bytes of LDS refused: %s", lds__, hipGetErrorString(ok));       \
+    const int rc__ = fstu_need_lds((const void*)conv_mfma_kernel<NT, NBS, NW, OCC>, most, lds__, "fstu_stu_conv_mfma");             \
+    if (rc__) return rc__;                                                                                                          \
     hipLaunchKernelGGL((conv_mfma_kernel<NT, NBS, NW, OCC>), grid, dim3(NW * 64), lds__, (hipStream_t)stream, (const bf16_t*)x,     \
                        (const bf16_t*)taps, (bf16_t*)y, B, T, d, single_branch);                                                    \
   } while (0)
@@ -592,8 +592,8 @@ extern "C" int fstu_stu_conv_mfma_grad(const void* gy, const void* x, const void
   do {                                                                                                                              \
     constexpr int lds__ = 16 * cm_region(8 * NT) + 8 * cg_rows(8 * NT) + 8 * 2048;                                                 \
     static fstu_lds_limit most;                                                                                                     \
-    const hipError_t ok = fstu_allow_lds((const void*)conv_grad_mfma_kernel<NT>, most, lds__);                                      \
-    FSTU_REQUIRE(ok == hipSuccess, (int)ok, "fstu_stu_conv_mfma_grad: %d bytes of LDS refused: %s", lds__, hipGetErrorString(ok));  \
+    const int rc__ = fstu_need_lds((const void*)conv_grad_mfma_kernel<NT>, most, lds__, "fstu_stu_conv_mfma_grad");                 \
+    if (rc__) return rc__;                                                                                                          \
     hipLaunchKernelGGL((conv_grad_mfma_kernel<NT>), grid, dim3(512), lds__, (hipStream_t)stream, (const bf16_t*)gy, (const bf16_t*)x, \
                        (const bf16_t*)filt, (bf16_t*)gx, gf ? part : nullptr, B, T, L, d, R);                                       \
   } while (0)

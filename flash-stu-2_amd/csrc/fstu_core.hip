@@ -1266,9 +1266,9 @@ int fstu_sample_dyn(const void* logits, int64_t* out, int64_t out_stride, int B,
   if (B == 0) return FSTU_OK;
   if (dtype == FSTU_BF16 && do_sample && V <= 65536) {
     const size_t shm = ((size_t)V * 2 + 15) & ~(size_t)15;
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(sample_kernel<bf16_t, true>),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024);
-    FSTU_REQUIRE(e == hipSuccess, (int)e, "fstu_sample: %d bytes of dynamic LDS refused", 128 * 1024);
+    static fstu_lds_limit most;
+    const int rc = fstu_need_lds(reinterpret_cast<const void*>(sample_kernel<bf16_t, true>), most, shm, "fstu_sample");
+    if (rc) return rc;
     hipLaunchKernelGGL((sample_kernel<bf16_t, true>), dim3(B), dim3(FSTU_SAMPLE_THREADS), shm, (hipStream_t)stream,
                        (const bf16_t*)logits, out, out_stride, V, temperature, top_k, top_p, do_sample, seed, step, row0, dyn);
     FSTU_CHECK_LAUNCH("fstu_sample");

@@ -998,17 +998,6 @@ int ilog2_exact(int n) {
   return ((1 << l) == n) ? l : -1;
 }
 
-template <typename K> int allow_lds(K kernel, size_t bytes, const char* name) {
-  if (bytes <= 48 * 1024) return 0;
-  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                     (int)bytes);
-  if (e != hipSuccess) {
-    fstu_set_error("%s: %zu bytes of LDS refused: %s", name, bytes, hipGetErrorString(e));
-    return (int)e;
-  }
-  return 0;
-}
-
 int fft_cols(int half_logn) { return half_logn >= 13 ? 1 : half_logn == 12 ? 2 : half_logn == 11 ? 4 : half_logn >= 9 ? 8 : half_logn >= 6 ? 16 : 32; }
 
 }  // namespace
@@ -1022,7 +1011,8 @@ extern "C" int fstu_fft_length(int T_) {
 // KERNEL: one of the launchers below, given LOGN of the half-length transform
 #define FFT_GO(KERNEL, THREADS, SHM, GRID, NAME, ...)                                                  \
   do {                                                                                                 \
-    static int rc__ = allow_lds(KERNEL, SHM, NAME);                                                    \
+    static fstu_lds_limit most__;                                                                      \
+    const int rc__ = fstu_need_lds(reinterpret_cast<const void*>(KERNEL), most__, SHM, NAME);          \
     if (rc__) return rc__;                                                                             \
     hipLaunchKernelGGL(KERNEL, GRID, dim3(THREADS), SHM, (hipStream_t)stream, __VA_ARGS__);            \
   } while (0)

@@ -321,8 +321,8 @@ template <class G, int MODE>
 int gemm_launch_tile(const void* A, long long lda, const void* W, const void* W2, const void* R, long long ldr, void* C,
                      long long ldc, int M, int N, int K, hipStream_t s, int ksplit = 1) {
   constexpr int NF = MODE == 1 ? G::BF / 2 : G::BF;
-  static hipError_t attr_err = hipFuncSetAttribute((const void*)gemm_bf16_kernel<G, MODE>, hipFuncAttributeMaxDynamicSharedMemorySize, G::LDS);
-  if (attr_err != hipSuccess) { fstu_set_error("fstu_gemm_bf16: hipFuncSetAttribute: %s", hipGetErrorString(attr_err)); return (int)attr_err; }
+  static fstu_lds_limit most;
+  if (const int rc = fstu_need_lds((const void*)gemm_bf16_kernel<G, MODE>, most, G::LDS, "fstu_gemm_bf16")) return rc;
   const int mt = (M + G::BT - 1) / G::BT, nt = (N + NF - 1) / NF;
   const long long tiles = (long long)mt * nt * ksplit;
   const int share = (int)((tiles + 7) / 8);
@@ -645,8 +645,8 @@ template <int MODE, bool TA = false>
 int gemm_pp_launch(const void* A, long long lda, const void* W, const void* W2, const void* R, long long ldr, void* C,
                    long long ldc, int M, int N, int K, hipStream_t s, int nbatch = 1, long long sa = 0, long long sc = 0, long long sr = 0, int nb = 1) {
   constexpr int NF = MODE == 1 ? 128 : 256;
-  static hipError_t attr_err = hipFuncSetAttribute((const void*)gemm_pp_bf16_kernel<MODE, TA>, hipFuncAttributeMaxDynamicSharedMemorySize, PP_LDS);
-  if (attr_err != hipSuccess) { fstu_set_error("fstu_gemm_bf16: hipFuncSetAttribute: %s", hipGetErrorString(attr_err)); return (int)attr_err; }
+  static fstu_lds_limit most;
+  if (const int rc = fstu_need_lds((const void*)gemm_pp_bf16_kernel<MODE, TA>, most, PP_LDS, "fstu_gemm_bf16")) return rc;
   const int mts = (M + 255) / 256, mt = mts * nbatch, nt = (N + NF - 1) / NF;
   const int share = (int)(((long long)mt * nt + 7) / 8);
   hipLaunchKernelGGL((gemm_pp_bf16_kernel<MODE, TA>), dim3(8u * (unsigned)std::min(share, gemm_cus() / 8)), dim3(512), PP_LDS, s, (const bf16_t*)A, lda,
@@ -855,8 +855,8 @@ gemm_ta_bf16_kernel(const bf16_t* __restrict__ A, long long lda, long long sa, c
 template <class G, int MODE>
 int gemm_ta_launch_tile(const void* A, long long lda, long long sa, const void* W, const void* R, long long ldr, long long sr,
                         void* C, long long ldc, long long sc, int M, int N, int K, int nbatch, hipStream_t s, int ksplit = 1) {
-  static hipError_t attr_err = hipFuncSetAttribute((const void*)gemm_ta_bf16_kernel<G, MODE>, hipFuncAttributeMaxDynamicSharedMemorySize, G::LDS);
-  if (attr_err != hipSuccess) { fstu_set_error("fstu_gemm_bf16_ta: hipFuncSetAttribute: %s", hipGetErrorString(attr_err)); return (int)attr_err; }
+  static fstu_lds_limit most;
+  if (const int rc = fstu_need_lds((const void*)gemm_ta_bf16_kernel<G, MODE>, most, G::LDS, "fstu_gemm_bf16_ta")) return rc;
   const int mt = M / G::BT, nt = (N + G::BF - 1) / G::BF;
   const long long tiles = (long long)mt * nt * nbatch * ksplit;
   const int share = (int)((tiles + 7) / 8);

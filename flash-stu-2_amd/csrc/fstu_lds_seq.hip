@@ -389,24 +389,24 @@ extern "C" int fstu_lds_sequence(float* h, const void* x, const float* A, const 
   unsigned cgrid = (unsigned)((nwords + 255) / 256);
   if (cgrid > 1024u) cgrid = 1024u;
   const bool past = (size_t)T * Bt * d_out * sizeof(bf16_t) > (size_t)32 << 20;
-  hipError_t e = hipSuccess;
-  auto run = [&](auto kernel) {
-    e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024);
-    if (e != hipSuccess) return;
+  int rc = FSTU_OK;
+  auto run = [&](auto which) {                          // (a type for each kernel: a record of its own)
+    constexpr auto kernel = decltype(which)::value;
+    static fstu_lds_limit most;
+    if ((rc = fstu_need_lds((const void*)kernel, most, shm, "fstu_lds_sequence"))) return;
     hipLaunchKernelGGL(lds_seq_clear_kernel, dim3(cgrid), dim3(256), 0, s, etag, nwords, status);
     hipLaunchKernelGGL(kernel, grid, dim3(256), shm, s, (const bf16_t*)x, A, (const bf16_t*)BmT, (const bf16_t*)CmT, (bf16_t*)y,
                        (const float*)h, hnew, etag, status, 1u, T, Bt, d_in, d_out, nblk);
     hipLaunchKernelGGL(lds_seq_finish_kernel, dim3((unsigned)((BtS + 255) / 256)), dim3(256), 0, s, h, (const float*)hnew, (int)BtS);
   };
-#define LSQ_CASE(n) case 32 * n: past ? run(lds_seq_kernel<2 * n, true>) : run(lds_seq_kernel<2 * n, false>); break
+#define LSQ_RUN(...) run(std::integral_constant<decltype(&lds_seq_kernel<__VA_ARGS__>), lds_seq_kernel<__VA_ARGS__>>{})
+#define LSQ_CASE(n) case 32 * n: past ? LSQ_RUN(2 * n, true) : LSQ_RUN(2 * n, false); break
   switch (S) {
     LSQ_CASE(1); LSQ_CASE(2); LSQ_CASE(3); LSQ_CASE(4); LSQ_CASE(5); LSQ_CASE(6); LSQ_CASE(7); LSQ_CASE(8);
   }
 #undef LSQ_CASE
-  if (e != hipSuccess) {
-    fstu_set_error("fstu_lds_sequence: hipFuncSetAttribute: %s", hipGetErrorString(e));
-    return (int)e;
-  }
+#undef LSQ_RUN
+  if (rc) return rc;
   FSTU_CHECK_LAUNCH("fstu_lds_sequence");
   return FSTU_OK;
 }

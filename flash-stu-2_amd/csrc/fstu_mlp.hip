@@ -658,19 +658,13 @@ extern "C" int fstu_mlp_packed_rows32_supported(int rows, int d, int I) {
          I % 512 == 0 && (size_t)rows * I * 2 < 0x7ff00000ull;
 }
 
-static int allow_lds(const void* kernel, fstu_lds_limit& limit, size_t shm, const char* name) {
-  const hipError_t e = fstu_allow_lds(kernel, limit, (int)shm);
-  FSTU_REQUIRE(e == hipSuccess, (int)e, "%s: %zu bytes of dynamic LDS refused", name, shm);
-  return FSTU_OK;
-}
-
 template <int KSA>
 static int glu_launch_ksa(GluArgs& a, int pro, int epi, int G, size_t shm, const char* name, hipStream_t s, bool row_major) {
   if constexpr (KSA <= 4) if (row_major) {       // 1..16 rows behind a norm prologue, widths up to 1024
     auto go = [&](auto which) -> int {              // (a type for each kernel: a record of its own)
       constexpr auto kernel = decltype(which)::value;
       static fstu_lds_limit most;
-      const int rc = allow_lds(reinterpret_cast<const void*>(kernel), most, shm, name);
+      const int rc = fstu_need_lds(reinterpret_cast<const void*>(kernel), most, shm, name);
       if (rc) return rc;
       hipLaunchKernelGGL(kernel, dim3(G), dim3(512), shm, s, a.h, a.wp_gate, a.wp_up, a.act, a.x_in, a.delta, a.x_out, a.norm_w, a.rows,
                          a.d, a.I, a.ldh, a.ldact, a.wgs, a.eps, a.nslices, a.best, a.temperature);
@@ -682,7 +676,7 @@ static int glu_launch_ksa(GluArgs& a, int pro, int epi, int G, size_t shm, const
 #define GLU_GO(PRO, GLUF)                                                                                        \
   do {                                                                                                           \
     static fstu_lds_limit most;                                                                          \
-    const int rc = allow_lds(reinterpret_cast<const void*>(glu_balanced_kernel<KSA, PRO, GLUF>), most, shm, name); \
+    const int rc = fstu_need_lds(reinterpret_cast<const void*>(glu_balanced_kernel<KSA, PRO, GLUF>), most, shm, name); \
     if (rc) return rc;                                                                                           \
     hipLaunchKernelGGL((glu_balanced_kernel<KSA, PRO, GLUF>), dim3(G), dim3(512), shm, s, a.h, a.wp_gate, a.wp_up, a.act, a.x_in,    \
                        a.delta, a.x_out, a.norm_w, a.rows, a.d, a.I, a.ldh, a.ldact, a.wgs, a.eps, a.nslices, a.best, a.temperature); \
@@ -695,9 +689,9 @@ static int glu_launch_ksa(GluArgs& a, int pro, int epi, int G, size_t shm, const
                  name, FSTU_MAX_DECODE_ROWS);
 #define GLU_GO2(PRO, EPI)                                                                                                  \
   do {                                                                                                                     \
-    static hipError_t attr_err = hipFuncSetAttribute(reinterpret_cast<const void*>(glu_balanced_kernel<KSA, PRO, EPI, 2>),  \
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)red2);               \
-    FSTU_REQUIRE(attr_err == hipSuccess, (int)attr_err, "%s: %zu bytes of dynamic LDS refused", name, red2);               \
+    static fstu_lds_limit most;                                                                                            \
+    const int rc = fstu_need_lds(reinterpret_cast<const void*>(glu_balanced_kernel<KSA, PRO, EPI, 2>), most, red2, name);  \
+    if (rc) return rc;                                                                                                     \
     hipLaunchKernelGGL((glu_balanced_kernel<KSA, PRO, EPI, 2>), dim3(G), dim3(512), red2, s, a.h, a.wp_gate, a.wp_up, a.act, \
                        a.x_in, a.delta, a.x_out, a.norm_w, a.rows, a.d, a.I, a.ldh, a.ldact, a.wgs, a.eps, a.nslices, a.best,  \
                        a.temperature);                                                                                      \

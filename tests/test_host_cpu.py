@@ -374,3 +374,11 @@ def test_training_step_lays_its_filter_out_once(B, T, d, monkeypatch):
     ApproxConvolveSum.apply(u, v).sum().backward()
     assert made in (["stu_conv_taps", "stu_conv_mfma_grad"], ["stu_fft_filter", "stu_conv_fft_grad"], []), made
     assert (made == []) == (T < 32)
+
+
+def test_limits_of_dynamic_lds_are_raised_by_device():
+    """A kernel's limit of dynamic LDS holds on the device where it was raised: every launcher goes through the record by device, none
+    raises it by itself or once for the process."""
+    csrc = os.path.join(ROOT, "flash-stu-2_amd", "csrc")
+    where = {f for f in os.listdir(csrc) if f.endswith((".hip", ".h")) and "hipFuncSetAttribute" in open(os.path.join(csrc, f)).read()}
+    assert where == {"fstu_common.h"}, where
