@@ -136,7 +136,7 @@ def step_on_caches(model, ids: torch.Tensor, past):
         a0, a1, pos_t = entry
         if gate.bias is not None or pos_t.is_cuda or pos_t.dim() != 1 or pos_t.numel() < 1:
             return None
-        p = pos_t.tolist()[0]
+        p = int(pos_t.tolist()[0])           # (any dtype that holds it)
         if pos is not None and p != pos:
             return None
         pos = p

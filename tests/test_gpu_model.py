@@ -794,6 +794,22 @@ def test_steps_on_caches_of_more_rows_than_one_launch_takes(dtype, extra):
     assert float((got - want).abs().max()) <= (1e-4 if dtype == torch.float32 else 2e-2) * float(want.abs().max())
 
 
+@pytest.mark.parametrize("dtype", [torch.int32, torch.float32, torch.float64])
+def test_steps_on_caches_whose_positions_were_cast(dtype):
+    """Caches that a program has cast as a whole still step, through the one call."""
+    from flash_stu.engine import step_on_caches
+    _, _, model = make_pair(seed=5, init="healthy", dtype=torch.float32, mlp_scale=2, n_embd=64, n_layers=2, n_heads=1, window_size=8,
+                            num_eigh=8, seq_len=64, vocab_size=77)
+    ids = prompt(2, 8, 77, 3).cuda()
+    past = model(ids[:, :6], use_cache=True).past_key_values
+    cast = [(a.clone(), b.clone(), p.to(dtype)) for a, b, p in past]
+    for t in (6, 7):
+        want = model(ids[:, t:t + 1], past_key_values=past, use_cache=True)
+        past = want.past_key_values
+        logits, cast = step_on_caches(model, ids[:, t:t + 1], cast)
+        assert torch.equal(logits, want.logits)
+
+
 @pytest.mark.parametrize("d,scale,rows,mode", [(256, 2, 1, "lds"), (256, 4, 16, "lds"), (512, 4, 3, "lds"), (768, 2, 10, "lds"), (768, 12, 11, "lds"),
                                                (1024, 4, 8, "lds"), (1024, 3, 9, "lds"), (2048, 2, 4, "lds"), (2048, 4, 5, "lds"), (512, 2, 4, "history")])
 def test_one_call_step_on_the_parameters_themselves(d, scale, rows, mode):
