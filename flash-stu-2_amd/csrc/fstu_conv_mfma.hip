@@ -491,9 +491,9 @@ void cm_shape(int T, int& nbs, int& nt) {
 // 2 x 2048 x 768 28 / 25 / 37 / -, 8 x 2048 x 768 70 / 62 / 65 / 68, 8 x 2048 x 2048 206 / 159 / 133 / 124, 5 x 700 x 1024 27 / 25 / 22 /
 // 28, 8 x 512 x 768 29 / 22.9 / 22.0 / 23.5, 64 x 300 x 256 80 / 56 / 44 / 38.
 int cg_items(int B, int T, int d) {
-  const int groups = (d + 7) / 8;
-  if ((long long)groups * 2 * B <= 256) return 1;
-  const int chunks = std::max(1, std::min(B, (T <= 1024 ? 512 : 768) / groups));
+  const int groups = (d + 7) / 8, cus = fstu_cus();
+  if ((long long)groups * 2 * B <= cus) return 1;
+  const int chunks = std::max(1, std::min(B, (T <= 1024 ? 2 : 3) * cus / groups));
   return 2 * ((B + chunks - 1) / chunks);
 }
 
