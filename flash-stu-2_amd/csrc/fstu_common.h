@@ -58,7 +58,8 @@ int fstu_sample_dyn(const void* logits, int64_t* out, int64_t out_stride, int B,
                     float top_p, int do_sample, uint64_t seed, int step, int row0, const int* dyn, int dtype, void* stream);
 int fstu_advance_dyn(int* dyn, void* stream);
 // fstu_mlp.hip: fstu_glu_packed_norm, fstu_linear_packed_res and fstu_down_packed_splitk; row_major (1..16 rows): over the
-// (N,K) row-major weights themselves
+// (N,K) row-major weights themselves (names without C++ types for these and the fp32 one: their tests call them)
+extern "C" {
 int fstu_glu_norm_impl(const void* x_in, const void* delta, void* x_out, const void* norm_w, float eps, const void* wp_gate,
                        const void* wp_up, void* act, int ldact, int rows, int I, int d, bool row_major, void* stream);
 int fstu_linear_res_impl(const void* x_in, const float* partial, int nslices, void* x_out, const void* norm_w, float eps,
@@ -66,9 +67,10 @@ int fstu_linear_res_impl(const void* x_in, const float* partial, int nslices, vo
 int fstu_down_splitk_impl(const void* act, int ldact, const void* wp_down, float* partial, int rows, int d, int I, int* ksplit_io,
                           bool row_major, void* stream);
 // fstu_linear.hip: an fp32 projection (or gated pair) behind the residual add and RMSNorm of its rows
-bool fstu_linear_f32_norm_ok(int rows, int K);
 int fstu_linear_f32_norm(const void* x, const float* delta, int nslices, void* x_out, const void* norm_w, float eps, const void* W,
                          const void* W2, void* y, int ldy, int rows, int N, int K, void* stream);
+}
+bool fstu_linear_f32_norm_ok(int rows, int K);
 bool fstu_linear_rows32_ok(const void* x, int ldx, const void* W, int K, int dtype);
 int fstu_linear_rows32(const void* x, int ldx, const void* W, void* y, int ldy, int rows, int N, int K, float temperature,
                        void* best_ws /*NULL: plain projection; else the head's packed maxima, rows*64 words*/, void* stream);

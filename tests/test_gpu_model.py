@@ -810,6 +810,12 @@ def test_steps_on_caches_whose_positions_were_cast(dtype):
         assert torch.equal(logits, want.logits)
 
 
+def _takes_one_call(model, ids, past) -> bool:
+    """Whether a step on these caches is the one call (made on copies of them)."""
+    from flash_stu.engine import step_on_caches
+    return step_on_caches(model, ids, tuple(tuple(t.clone() for t in c) for c in past)) is not None
+
+
 @pytest.mark.parametrize("d,scale,rows,mode", [(256, 2, 1, "lds"), (256, 4, 16, "lds"), (512, 4, 3, "lds"), (768, 2, 10, "lds"), (768, 12, 11, "lds"),
                                                (1024, 4, 8, "lds"), (1024, 3, 9, "lds"), (2048, 2, 4, "lds"), (2048, 4, 5, "lds"), (512, 2, 4, "history")])
 def test_one_call_step_on_the_parameters_themselves(d, scale, rows, mode):
@@ -820,16 +826,17 @@ def test_one_call_step_on_the_parameters_themselves(d, scale, rows, mode):
                             num_eigh=8, seq_len=64, vocab_size=777, stu_decode_mode=mode)
     ids = prompt(rows, 10, 777, 3).cuda()
 
-    def run():
+    def run(one_call):
         past, logits = model(ids[:, :6], use_cache=True).past_key_values, []
+        assert _takes_one_call(model, ids[:, 6:7], past) == one_call
         for t in range(6, 10):
             out = model(ids[:, t:t + 1], past_key_values=past, use_cache=True)
             past = out.past_key_values
             logits.append(out.logits.float())
         return torch.cat(logits, 1)
-    got = run()
+    got = run(True)
     model.layers[0].mlp.register_forward_hook(lambda *a: None)     # the layers' own calls run
-    want = run()
+    want = run(False)
     assert float((got - want).abs().max()) <= 2e-2 * float(want.abs().max())
 
 
@@ -842,16 +849,17 @@ def test_fp32_step_with_its_norms_in_the_projections(d, rows, extra):
                             num_eigh=8, seq_len=320, vocab_size=777, **extra)
     ids = prompt(rows, 300, 777, 3).cuda()
 
-    def run(first, count):
+    def run(first, count, one_call):
         past, logits = model(ids[:, :first], use_cache=True).past_key_values, []
+        assert _takes_one_call(model, ids[:, first:first + 1], past) == one_call
         for t in range(first, first + count):
             out = model(ids[:, t:t + 1], past_key_values=past, use_cache=True)
             past = out.past_key_values
             logits.append(out.logits)
         return torch.cat(logits, 1)
-    got = [run(3, 3), run(70, 2), run(290, 2)]
+    got = [run(3, 3, True), run(70, 2, True), run(290, 2, True)]
     model.layers[0].mlp.register_forward_hook(lambda *a: None)     # the layers' own calls run
-    for a, b in zip(got, [run(3, 3), run(70, 2), run(290, 2)]):
+    for a, b in zip(got, [run(3, 3, False), run(70, 2, False), run(290, 2, False)]):
         assert float((a - b).abs().max()) <= 1e-4 * float(b.abs().max())
 
 

@@ -5,6 +5,7 @@ Tolerances: fp32 results differ from the oracle only by summation order
 (1e-5 relative to the result scale); bf16 results must equal the oracle's
 rounded values except where a different fp32 summation order flips a rounding:
 at most one bf16 ulp (2^-7 relative) on a small fraction of elements."""
+import ctypes
 import math
 
 import numpy as np
@@ -1838,6 +1839,65 @@ def test_glu_packed_norm_prologue(hip, rows, d, I):
     assert float((diff > 0).float().mean()) <= 0.10
     x_out2, act2 = hip.glu_packed_norm(dev(x), None, dev(nw), O.RMS_EPS_DEFAULT, pg, pu, I)
     assert torch.equal(x_out2.cpu(), x)
+
+
+def _internal(hip, name, *types):
+    fn = getattr(hip.load(), name)
+    fn.argtypes, fn.restype = types, ctypes.c_int
+
+    def call(*args):
+        hip._check(fn(*(hip._p(a) if isinstance(a, torch.Tensor) else a for a in args), hip._stream()), name)
+    return call
+
+
+@pytest.mark.parametrize("rows,d,I", [(1, 256, 512), (16, 256, 520), (3, 512, 1536), (10, 768, 4096), (11, 768, 2312), (8, 1024, 1024), (16, 1024, 40)])
+def test_launches_over_row_major_weights_have_the_bits_of_the_packed_ones(hip, rows, d, I):
+    """Gate/up behind a residual and its norm, a projection behind the sum of four slices and its norm, the down projection in four
+    slices: over the parameters as nn.Linear holds them and over packed copies, which the tests beside this one hold to references."""
+    p, i, f, b = ctypes.c_void_p, ctypes.c_int, ctypes.c_float, ctypes.c_bool
+    g = gen(rows + d + I)
+    x, delta, nw = (dev(torch.randn(*s, generator=g).bfloat16()) for s in ((rows, d), (rows, d), (d,)))
+    W, U = (dev((torch.randn(I, d, generator=g) * d ** -0.5).bfloat16()) for _ in range(2))
+    x_out, act = torch.empty_like(x), torch.full((rows, I), float("nan"), dtype=x.dtype, device="cuda")
+    _internal(hip, "fstu_glu_norm_impl", p, p, p, p, f, p, p, p, i, i, i, i, b, p)(x, delta, x_out, nw, 1e-6, W, U, act, I, rows, I, d, True)
+    want = hip.glu_packed_norm(x, delta, nw, 1e-6, hip.pack_rows(W), hip.pack_rows(U), I)
+    assert torch.equal(x_out, want[0]) and torch.equal(act, want[1])
+    if rows * d <= 8192:
+        part = dev(torch.randn(4, rows, d, generator=g))
+        y = torch.full((rows, I), float("nan"), dtype=x.dtype, device="cuda")
+        _internal(hip, "fstu_linear_res_impl", p, p, i, p, p, f, p, p, i, i, i, i, b, p)(x, part, 4, x_out, nw, 1e-6, W, y, I, rows, I, d, True)
+        want = hip.linear_packed_res(x, part, nw, 1e-6, hip.pack_rows(W), I)
+        assert torch.equal(x_out, want[0]) and torch.equal(y, want[1])
+    if I % 512 == 0:
+        D = dev((torch.randn(d, I, generator=g) * I ** -0.5).bfloat16())
+        for ks in (4, 16):
+            out, n = torch.full((ks, rows, d), float("nan"), device="cuda"), ctypes.c_int(ks)
+            _internal(hip, "fstu_down_splitk_impl", p, i, p, p, i, i, i, p, b, p)(act, I, D, out, rows, d, I, ctypes.byref(n), True)
+            assert n.value == ks and torch.equal(out, hip.down_packed_splitk(act, hip.pack_rows(D), d, ks))
+
+
+@pytest.mark.parametrize("rows,K,N,slices", [(1, 4, 3, 1), (2, 64, 77, 2), (1, 256, 768, 8), (2, 256, 1, 3), (1, 260, 130, 9), (2, 512, 515, 16)])
+def test_linear_fp32_behind_its_norm(hip, rows, K, N, slices):
+    """One and two fp32 rows: the slices' sum in their order and the residual exactly, the projection and the gated pair of the
+    normalised rows against float64: K sums and the norm's K + 8 roundings of 2^-24 of the absolute sum, the GELU's slope at most 1.13."""
+    p, i, f = ctypes.c_void_p, ctypes.c_int, ctypes.c_float
+    g = gen(rows + K + N)
+    x, nw, part = dev(torch.randn(rows, K, generator=g)), dev(torch.randn(K, generator=g)), dev(torch.randn(slices, rows, K, generator=g))
+    W, U = (dev(torch.randn(N, K, generator=g) * K ** -0.5) for _ in range(2))
+    total = part[0].clone()
+    for s in range(1, slices):
+        total += part[s]
+    stream = x + total
+    h = stream.double() * torch.rsqrt((stream.double() ** 2).mean(1, keepdim=True) + 1e-6) * nw.double()
+    gate, up, slack = h @ W.double().t(), h @ U.double().t(), (2 * K + 8) * 2.0 ** -24
+    dg, du = slack * (h.abs() @ W.double().abs().t()), slack * (h.abs() @ U.double().abs().t())
+    gated = F.gelu(gate, approximate="tanh")
+    call = _internal(hip, "fstu_linear_f32_norm", p, p, i, p, p, f, p, p, p, i, i, i, i, p)
+    for W2, want, bound in ((None, gate, dg), (U, gated * up, 1.13 * dg * (up.abs() + du) + gated.abs() * du + 1e-6 * gate.abs() * up.abs())):
+        x_out, y = torch.full_like(x, float("nan")), torch.full((rows, N + 1), float("nan"), device="cuda")
+        call(x, part, slices, x_out, nw, 1e-6, W, W2, y, N + 1, rows, N, K)
+        assert torch.equal(x_out, stream) and bool(y[:, N].isnan().all())
+        assert bool(((y[:, :N].double() - want).abs() <= bound).all())
 
 
 @pytest.mark.parametrize("rows,d,I", [(32, 2048, 4096), (17, 2048, 1024), (24, 1024, 2048), (32, 768, 1536), (29, 256, 512)])
