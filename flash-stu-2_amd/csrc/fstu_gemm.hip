@@ -39,8 +39,9 @@ typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ float rnd_bf16(float v) { return bf16_to_f32(f32_to_bf16(v)); }
 // The tanh-approximated GELU on the hardware exp and reciprocal, x (1 + tanh t) / 2 = x / (1 + exp(-2 t)): five full-rate and two
 // quarter-rate instructions (eleven and two as 1 - 2 / (exp(2 t) + 1), which also cancelled for negative x: off by 1.5e-3 of the
-// value at x = -4, 4e-6 so)
-__device__ __forceinline__ float gelu_tanh_fast(float x) {
+// value at x = -4, 4e-6 so).  Of the 26820 bf16 inputs between 1e-30 and 40 in size 72 leave it not correctly rounded, 106 the longer form, which
+// the packed decode launches keep.
+__device__ __forceinline__ float gelu_tanh_short(float x) {
   return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x * fmaf(x * x, -0.10294324f, -2.3022082f)));
 }
 
@@ -287,7 +288,7 @@ gemm_bf16_kernel(const bf16_t* __restrict__ A, long long lda, const bf16_t* __re
           float v[4];
 #pragma unroll
           for (int e = 0; e < 4; ++e)
-            v[e] = rnd_bf16(gelu_tanh_fast(rnd_bf16(acc[i][j][q * 4 + e]))) * rnd_bf16(acc[i + FI / 2][j][q * 4 + e]);
+            v[e] = rnd_bf16(gelu_tanh_short(rnd_bf16(acc[i][j][q * 4 + e]))) * rnd_bf16(acc[i + FI / 2][j][q * 4 + e]);
           *(uint2*)(C + (size_t)m * ldc + f) = make_uint2(pack2_bf16(v[0], v[1]), pack2_bf16(v[2], v[3]));
         }
     } else {
@@ -607,7 +608,7 @@ gemm_pp_bf16_kernel(const bf16_t* __restrict__ A, long long lda, const bf16_t* _
               float v[4];
 #pragma unroll
               for (int e = 0; e < 4; ++e)
-                v[e] = MODE == 1 ? rnd_bf16(gelu_tanh_fast(rnd_bf16(acc[0][i][hx][2 * j + t][e]))) * rnd_bf16(acc[1][i][hx][2 * j + t][e])
+                v[e] = MODE == 1 ? rnd_bf16(gelu_tanh_short(rnd_bf16(acc[0][i][hx][2 * j + t][e]))) * rnd_bf16(acc[1][i][hx][2 * j + t][e])
                                  : acc[hw][i][hx][2 * j + t][e];
               const u32x2_t p = {pack2_bf16(v[0], v[1]), pack2_bf16(v[2], v[3])};
               asm volatile("ds_write_b64 %0, %1" ::"v"(scratch + (unsigned)(r * RBY + ((c ^ (r & (CH - 1))) << 4) + (lq & 1) * 8)), "v"(p) : "memory");
@@ -925,8 +926,10 @@ int gemm_launch(const void* A, long long lda, const void* W, const void* W2, con
 // each; joining costs a launch and the slices' bytes out and back at 4 TB/s.  The estimate only has to rank: us without / with the
 // slices it picks, rows x features x K: 300 x 768 x 9216 60 / 17.7 (12), 1000 x 768 x 9216 60 / 27.5 (4; 31.4 with two stages), 1400
 // 60 / 34.0 (3; 39.7), 2400 61 / 44.7 (4; 47.2 with two, which were picked before and took 53.8), 3000 63 / 53 (3), 700 x 2048 x
-// 24576 180 / 85 (4), 1500 x 2048 x 24576 184 / 160 (2), 300 x 2048 x 2048 21.8 / 15.0 (4); slabs 1 x 1024 x 1024 x 24576 219 / 63
-// (8), 1 x 128 x 256 x 6144 50 / 12 (12).  Where it picks none, without / with two: 4096 x 768 x 9216 66.6 / 68.8, 600 x 2048 x
+// 24576 180 / 85 (4), 1500 x 2048 x 24576 184 / 160 (2), 300 x 2048 x 2048 21.8 / 15.0 (4).  Slabs take 0.6 us a k tile alone on a
+// compute unit and 0.86 each two to a unit, with four stages no less than with the two that they run on; the counts are the best or
+// within 12 % of it all the same: without / picked / best, 1 x 1024 x 1024 x 24576 219 / 58.5 (8), 1 x 512 x 1024 x 24576 226 / 40.6 (8) / 37.1
+// (16), 4 x 512 x 512 x 12288 112 / 40.7 (4) / 37.0 (8), 2 x 256 x 512 x 12288 119 / 19.7 (12), 1 x 128 x 256 x 6144 54 / 12.5 (12).  Where it picks none, without / with two: 4096 x 768 x 9216 66.6 / 68.8, 600 x 2048 x
 // 2048 22.0 / 18.8, 300 x 6144 x 2048 20.5 / 23.8, 1000 x 768 x 768 10.5 / 12.7.  Below K = 2048 the GPU gains less than the second
 // launch and the slices' allocation cost the host (calls of 300 x 384 x 1536 one behind the other 16.0 us with three slices, 13.2
 // without).
@@ -1053,7 +1056,8 @@ static int fstu_join_slices(const float* part, int ns, const void* R, long long 
 // once as there are compute units.  us in one launch / split, rows x features x K: 9600 x 2048 x 24576 970 / 687, 8500 x 2048 x 24576
 // 1029 / 590, 10500 x 2048 x 24576 971 / 739, 13500 1024 / 959, 17000 1490 / 1152, 20480 1502 / 1369, 22500 x 768 x 9216 409 / 237, 3000 x 6144 x 2048 83 / 65, 10240 x 2048 x 2048 81 /
 // 73, 22500 x 768 x 768 42 / 37, 33000 x 512 x 512 31 / 28.  The line: 14500 x 2048 x 24576 (no slices of the rest) 1041 / 1015, below K
-// = 2048 26000 x 768 x 768 (204) 38.5 / 39.3, 18500 x 1024 x 1024 (136) 44.9 / 43.1.
+// = 2048 26000 x 768 x 768 (204) 38.5 / 39.3, 18500 x 1024 x 1024 (136) 44.9 / 43.1.  The dearest rest are 1 to 32 rows of a long K, which
+// take no slices: 8200 x 2048 x 24576 1021 / 641, of which the 8 rows alone 108, but 8232 573 and 22; 21768 x 768 x 9216 396 / 248.
 extern "C" int fstu_gemm_bf16_head_rows(int M, int N, int K) {
   if (M <= 256 || N < 256 || N % 4 != 0 || K % 64 != 0 || K < 512) return 0;
   const long long cus = gemm_cus(), nt = (N + 255) / 256, tiles = (long long)((M + 255) / 256) * nt;

@@ -985,7 +985,7 @@ template <> __device__ __forceinline__ float lsh_load<bf16_t>(__amdgpu_buffer_rs
 // order.  Powers are formed in double and rounded once, so there are P + T / (8 P) roundings in a row where a step per position
 // makes T / 2.  The decay by a^16 itself is the same for every group, so its rounding adds up: below 8 pieces it carries its
 // remainder.  Off from float64 at 8192 positions, poles up to 0.9998: 4.7e-7 of the state with 8 pieces, 8.0e-7 with one, 8.0e-7 before;
-// at 777 1.6e-7, 3.2e-7 before.
+// at 777 1.6e-7, 3.2e-7 before.  (The number of pieces depends on the rows, so the last bits of a row's state do too.)
 // What bounded the scan of a position per step (8 waves of 8 modes over 64 channels) was the vector ALUs of the few compute units
 // it has workgroups for.  us, before / now: 3 x 777 x 768 21.4 / 11.6, 8 x 512 x 768 15.3 / 13.2, 1 x 8192 x 1024 164 / 48, 32 x 300 x
 // 2048 54 / 39, 32 x 4096 x 2048 503 / 349 (the matrix cores' fp32 rate would be 220).

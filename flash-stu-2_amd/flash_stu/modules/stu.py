@@ -292,12 +292,13 @@ class STU(nn.Module):
 
     @staticmethod
     def _few_long_sequences(B: int, T: int, d: int, esz: int) -> bool:
-        """A few long sequences: the FFT kernels for (B, L, d) operands take a workgroup's 16 bytes of channels one after the
-        other or read a tensor two bytes at a time.  Time-major slabs let every load and store coalesce, with identical
-        results (bf16, us, slab / (B, L, d): 1 x 4096 x 2048 49 / 75, 1 x 8192 x 2048 119 / 138, 2 x 4096 x 2048, where the
-        line lies, 86 / 100).  A transpose of the result is 8 to 15 of them; the projection that comes out as slabs costs
-        none, and where a decode state needs (B, L, d) rows as well a second transpose leaves 64 / 75, 139 / 138 and 111 /
-        100."""
+        """A few long sequences through transforms: fp32, bf16 beyond 4096 positions and narrow bf16 layers from 2049 on.  The FFT
+        kernels for (B, L, d) operands take a workgroup's 16 bytes of channels one after the other or read a tensor two bytes at
+        a time.  Time-major slabs let every load and store coalesce, with identical results (us, slab / (B, L, d): bf16 1 x 4096 x
+        1024 31 / 42, 3 x 4096 x 768 63 / 88, 1 x 8192 x 1024 61 / 107, and where the line lies 4 x 4096 x 1024 99 / 93, 2 x 8192 x
+        2048 253 / 271; fp32 1 x 4096 x 1024 41 / 44, 1 x 8192 x 1024 76 / 73, at the line 2 x 4096 x 1024 66 / 54).  A transpose of
+        the result is 4 to 15 of them; the projection that comes out as slabs costs none, and where a decode state needs (B, L, d)
+        rows as well a second transpose leaves 36, 73 and 68 in bf16."""
         return T >= FFT_MIN_T and _hip.fft_length(T) >= 8192 and (d // (16 // esz)) * B < 512
 
     def _convolve_time_major(self, xt: torch.Tensor, n: int) -> torch.Tensor:
