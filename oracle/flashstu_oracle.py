@@ -1,6 +1,6 @@
 """CPU oracle for Flash STU's autoregressive token loop.
 
-TEST INFRASTRUCTURE ONLY.  This module is the checker the HIP path is compared
+TEST INFRASTRUCTURE ONLY.  This module is what the HIP path is compared
 against; nothing in the product package imports it.  Only tests, the smoke
 entry and the benchmark's CPU-baseline leg may call it.
 
