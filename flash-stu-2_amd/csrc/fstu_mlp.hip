@@ -60,8 +60,8 @@ __device__ __forceinline__ float half_wave_sum(float v) {
 // tanh-approximated GELU with tanh(t) = 1 - 2 / (exp(2t) + 1) on the hardware exp and reciprocal: absolute error of 1 + tanh about
 // 1e-7, far below the bf16 rounding that follows.  (The prompt GEMM's shorter form, off by less for negative x, gains no time here: a decode
 // launch has two features to a lane and waits for memory.  It changes one result in some hundreds by a rounding, and what generate() picks
-// afterwards with it: of 2000 greedy picks of 768-d, 12 layers, the oracle's own agreement with itself moves by as much, and over six
-// prompts 97.89 % of them agree with the oracle so and 98.03 % with the shorter form.)
+// afterwards with it: of 2000 greedy picks of 768-d, 12 layers, an evaluation in plain PyTorch under two orders of summation agrees with
+// itself in 98 to 99 %, with this form, over six prompts, in 97.89 % and with the shorter one in 98.03 %.)
 __device__ __forceinline__ float gelu_tanh_packed(float x) {
   const float inner = 0.7978845608028654f * (x + 0.044715f * x * x * x);
   const float e = __builtin_amdgcn_exp2f(2.8853900817779268f * inner);   // exp(2 inner)
