@@ -21,6 +21,7 @@
 // 8 XCDs; each XCD works through its own contiguous share of the tiles in panels of 8 feature tiles, so the workgroups
 // resident on an XCD share a few weight and activation tiles in its L2.
 #include <algorithm>
+#include <type_traits>
 #include "fstu_common.h"
 
 namespace {
@@ -347,18 +348,22 @@ int gemm_launch_tile(const void* A, long long lda, const void* W, const void* W2
 // that ends a memory phase) and waited for three phases later: vmcnt(8) at the end of a memory phase leaves the two
 // youngest requests in flight, at 512 cycles a phase and group that is longer than a trip to the memory-side cache.
 // The grid is one workgroup per compute unit, each walks its share of the tiles: the first k tiles of the next output tile
-// are requested before this one is stored.  The epilogue passes 32 rows at a time through LDS beside the stages, so that
-// rows leave in 16-byte pieces, whole lines per instruction; straight from the accumulators a store instruction covers 16
-// rows of 32 bytes.
+// are requested before this one is stored.  The W rows are dealt so that a lane ends up with 8 consecutive features of a row,
+// 16 bytes: the gated pair (the four lanes of a row hold 64 bytes) and the fp32 sums (128) leave straight from the accumulators
+// without a barrier, us, through LDS / so: 16384 x 2 x 24576 x 2048 2324 / 2268, 2331 x 2 x 9216 x 768 69.3 / 64.7, 4096 x 2 x 9216 x
+// 768 113 / 107, 2500 x 2048 x 24576 in three slices 203 / 196.  Plain and residual rows pass 32 at a time through LDS beside the
+// stages and leave 512 bytes in a row: straight from the accumulators 2331 x 50257 x 768, whose rows begin anywhere, takes 213 us,
+// 167 so.  The stores of a whole tile are not waited for before the next tile's first products (16384 x 2048 x 2048 with the
+// residual 112 / 104, 16384 x 768 x 768 21.7 / 20.8).
 // What bounds it: the power the matrix cores draw.  A loop of nothing but v_mfma on random bf16 operands runs at 1.77
 // PFLOP/s in the 32x32x16 form and 2.03 in the 16x16x32 form on this card (2.42 on zeros): hence the smaller instruction,
 // although it reads the same operands twice as often (1.30 -> 1.33-1.42 PFLOP/s).  Measured against the kernel above
-// (256 x 256 tile) and hipBLASLt, us: 16384 x 2048 x 24576 with the residual 1127 / 1395 / 1366 (1.46 PFLOP/s), 16384 x 6144
-// x 2048 291 / 384 / 294, 16384 x 50257 x 2048 2550 / 3339 / 2500; gate+up 16384 x 2 x 24576 x 2048 2487 / 3148, 4096 x
-// 2 x 9216 x 768 118 / 133.  What keeps K = 2048 below K = 24576: the epilogue (in mode 1 the GELU's 70 cycles per element).
+// (256 x 256 tile) and hipBLASLt, us: 16384 x 2048 x 24576 with the residual 1099 / 1395 / 1190 (1.50 PFLOP/s; on zeros 888), 16384 x
+// 6144 x 2048 288 / 384 / 292, 16384 x 50257 x 2048 2570 / 3339 / 2510; gate+up 16384 x 2 x 24576 x 2048 2268 / 3148, 4096 x
+// 2 x 9216 x 768 107 / 133 (84 on zeros).  What keeps K = 2048 below K = 24576: the epilogue (in mode 1 the GELU's 70 cycles per element).
 #define PP_STAGE 65536u
 #define PP_PART 16384u
-#define PP_LDS (2 * PP_STAGE + 32768u)   // + what the epilogue passes the rows through
+#define PP_LDS(MODE) (2 * PP_STAGE + ((MODE) == 1 || (MODE) == 3 ? 0u : 32768u))   // + what the epilogue passes the rows through
 typedef unsigned u32x4_any_t __attribute__((ext_vector_type(4), aligned(2)));
 typedef unsigned u32x2_t __attribute__((ext_vector_type(2)));
 
@@ -452,7 +457,8 @@ gemm_pp_bf16_kernel(const bf16_t* __restrict__ A, long long lda, const bf16_t* _
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
     const int row = wv * 16 + j * 8 + (lane >> 3), ch = (lane & 7) ^ ((row >> 1) & 7);
-    wvoff[j] = (unsigned)row * (unsigned)K * 2u + (unsigned)ch * 16u;
+    const int feat = MODE == 1 ? row : (row & 31) + 2 * (row & 96);
+    wvoff[j] = (unsigned)feat * (unsigned)K * 2u + (unsigned)((lane & 7) ^ (((row >> 1) & 1) | ((row >> 2) & 6))) * 16u;
     if constexpr (TA) {
       const int kr = wv * 8 + j * 4 + (lane >> 4);
       avoff[j] = (unsigned)kr * (unsigned)lda * 2u + (unsigned)((lane & 15) ^ (4 * (kr & 3)) ^ (2 * ((kr >> 3) & 1))) * 16u;
@@ -460,7 +466,7 @@ gemm_pp_bf16_kernel(const bf16_t* __restrict__ A, long long lda, const bf16_t* _
       avoff[j] = (unsigned)row * (unsigned)lda * 2u + (unsigned)ch * 16u;
     }
   }
-  const unsigned w1off = MODE == 1 ? 0u : 128u * (unsigned)K * 2u, x1off = TA ? 256u : 128u * (unsigned)lda * 2u;
+  const unsigned w1off = MODE == 1 ? 0u : 32u * (unsigned)K * 2u, x1off = TA ? 256u : 128u * (unsigned)lda * 2u;
   const int nkt = KS >> 6;
   unsigned char* fill0 = gm_smem + (unsigned)wv * 2048u;
   // requests part P (0 W0, 1 X0, 2 W1, 3 X1) of k tile kt_; beyond the last tile the descriptor is empty: nothing is fetched
@@ -477,8 +483,8 @@ gemm_pp_bf16_kernel(const bf16_t* __restrict__ A, long long lda, const bf16_t* _
   unsigned fw_off[2], fx_off[2];                       // fragment addresses of the two k steps inside a part
 #pragma unroll
   for (int kk = 0; kk < 2; ++kk) {
-    const int rw = wn * 32 + l16, rx = wm * 64 + l16, c = kk * 4 + lq;
-    fw_off[kk] = (unsigned)rw * 128u + (unsigned)((c ^ ((rw >> 1) & 7)) << 4);
+    const int rw = wn * 32 + 8 * (l16 >> 2) + (l16 & 3), rx = wm * 64 + l16, c = kk * 4 + lq;
+    fw_off[kk] = (unsigned)rw * 128u + (unsigned)((c ^ (((rw >> 1) & 1) | ((rw >> 2) & 6))) << 4);
     fx_off[kk] = 2 * PP_PART + (unsigned)rx * 128u + (unsigned)((c ^ ((rx >> 1) & 7)) << 4);
   }
   const unsigned smem0 = lds_addr(gm_smem);
@@ -496,9 +502,9 @@ gemm_pp_bf16_kernel(const bf16_t* __restrict__ A, long long lda, const bf16_t* _
 #define PP_READ_W(stage_)                                                                              \
   _Pragma("unroll") for (int kk = 0; kk < 2; ++kk) {                                                   \
     wa[4 * kk] = lds_read16<0>(smem0 + (stage_) * PP_STAGE + fw_off[kk]);                              \
-    wa[4 * kk + 1] = lds_read16<2048>(smem0 + (stage_) * PP_STAGE + fw_off[kk]);                       \
+    wa[4 * kk + 1] = lds_read16<512>(smem0 + (stage_) * PP_STAGE + fw_off[kk]);                       \
     wa[4 * kk + 2] = lds_read16<16384>(smem0 + (stage_) * PP_STAGE + fw_off[kk]);                      \
-    wa[4 * kk + 3] = lds_read16<16384 + 2048>(smem0 + (stage_) * PP_STAGE + fw_off[kk]);               \
+    wa[4 * kk + 3] = lds_read16<16384 + 512>(smem0 + (stage_) * PP_STAGE + fw_off[kk]);               \
   }
 #define PP_READ_X(stage_, H)                                                                           \
   if constexpr (TA) {                                                                                  \
@@ -513,15 +519,22 @@ gemm_pp_bf16_kernel(const bf16_t* __restrict__ A, long long lda, const bf16_t* _
     _Pragma("unroll") for (int kk = 0; kk < 2; ++kk)                                                   \
       lds_read_rows<4, 2048>(xf + 4 * kk, smem0 + (stage_) * PP_STAGE + (H) * 16384u + fx_off[kk]);    \
   }
+  // all but the 8 youngest fills have landed; the stores of the tile before count with them while they are younger than what is waited for
+  constexpr int STORES = MODE == 1 ? 8 : MODE == 3 ? 32 : 16;
+  bool young = false;
+#define PP_LANDED                                                               \
+  if (young) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(8 + STORES) : "memory");  \
+  else asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
   // end of a memory phase: this wave's reads are complete, its share of the parts that the next phase reads has landed
 #define PP_MEM_END                                                                                     \
+  PP_LANDED                                                                                            \
   if constexpr (TA)                                                                                    \
-    asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)"                                                       \
+    asm volatile("s_waitcnt lgkmcnt(0)"                                                                \
                : "+v"(xt[0]), "+v"(xt[1]), "+v"(xt[2]), "+v"(xt[3]), "+v"(xt[4]), "+v"(xt[5]), "+v"(xt[6]), "+v"(xt[7]), \
                  "+v"(xt[8]), "+v"(xt[9]), "+v"(xt[10]), "+v"(xt[11]), "+v"(xt[12]), "+v"(xt[13]), "+v"(xt[14]), "+v"(xt[15]), \
                  "+v"(wa[0]), "+v"(wa[1]), "+v"(wa[2]), "+v"(wa[3]), "+v"(wa[4]), "+v"(wa[5]), "+v"(wa[6]), "+v"(wa[7])::"memory"); \
   else                                                                                                 \
-    asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)"                                                       \
+    asm volatile("s_waitcnt lgkmcnt(0)"                                                                \
                : "+v"(xf[0]), "+v"(xf[1]), "+v"(xf[2]), "+v"(xf[3]), "+v"(xf[4]), "+v"(xf[5]), "+v"(xf[6]), "+v"(xf[7]), \
                  "+v"(wa[0]), "+v"(wa[1]), "+v"(wa[2]), "+v"(wa[3]), "+v"(wa[4]), "+v"(wa[5]), "+v"(wa[6]), "+v"(wa[7])::"memory"); \
   __builtin_amdgcn_s_barrier();                                                                        \
@@ -545,9 +558,7 @@ gemm_pp_bf16_kernel(const bf16_t* __restrict__ A, long long lda, const bf16_t* _
 #define PP_FIRST                                                         \
   PP_FETCH(0, 0, 0) PP_FETCH(2, 0, 0) PP_FETCH(1, 0, 0) PP_FETCH(3, 0, 0) \
   PP_FETCH(0, 1, 1) PP_FETCH(2, 1, 1) PP_FETCH(1, 1, 1)
-  // epilogue addresses: a group passes 32 rows at a time through 16 KB of its own, chunks XOR-ed with the row
-  constexpr int CH = NF / 8, RBY = NF * 2, NST = 32 * CH / 256;      // 16-byte chunks per row, row bytes, chunks per lane
-  const unsigned scratch = smem0 + 2 * PP_STAGE + (unsigned)wm * 16384u;
+  const unsigned scratch = smem0 + 2 * PP_STAGE + (unsigned)wm * 16384u;   // modes 0 and 2: 16 KB a group
   const int gl = tid & 255;
   PP_OPEN_TILE
   PP_FIRST
@@ -556,12 +567,13 @@ gemm_pp_bf16_kernel(const bf16_t* __restrict__ A, long long lda, const bf16_t* _
     for (int i = 0; i < 8; ++i)
 #pragma unroll
       for (int j = 0; j < 4; ++j) acc[i >> 2][(i >> 1) & 1][i & 1][j] = floatx4_t{0.f, 0.f, 0.f, 0.f};
-    asm volatile("s_waitcnt vmcnt(8)" ::: "memory");   // W0, W1 and X0 of k tile 0
+    PP_LANDED                                          // W0, W1 and X0 of k tile 0
     __builtin_amdgcn_s_barrier();
     if (wm) __builtin_amdgcn_s_barrier();              // the second group runs half a phase later
     __builtin_amdgcn_sched_barrier(0);
     for (int kt = 0;; ++kt) {
       PP_TILE(0)
+      young = false;
       if (++kt >= nkt) break;
       PP_TILE(1)
       if (kt + 1 >= nkt) break;
@@ -580,56 +592,66 @@ gemm_pp_bf16_kernel(const bf16_t* __restrict__ A, long long lda, const bf16_t* _
       PP_OPEN_TILE
       PP_FIRST
     }
-    // D of a 16x16 tile: lane l holds row l % 16 and features 4*(l/16) + e
-    if constexpr (MODE == 3) {                         // fp32 sums, straight from the accumulators
+    asm volatile("" ::: "memory");
+    // D of a 16x16 tile: lane l holds row l % 16, and of the two feature tiles of a W half features 8*(l/16) .. + 7 of its 32.
+    // whole: no row and no feature is behind the end
+    auto leave = [&](auto whole) __attribute__((always_inline)) {
+      auto put = [&](u32x4_t v, int m, int f) __attribute__((always_inline)) {
+        if (decltype(whole)::value || (m < M && f < N))
+          store_feat8<MODE>(v, MODE == 2 ? er + (size_t)m * ldr + f : nullptr, ec + (size_t)m * ldc + f, decltype(whole)::value ? 8 : N - f);
+      };
 #pragma unroll
-      for (int hw = 0; hw < 2; ++hw)
+      for (int hx = 0; hx < 2; ++hx) {
+        const int mrow = em0 + hx * 128 + wm * 64;
+        if constexpr (MODE == 1 || MODE == 3) {        // straight from the accumulators
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+          for (int j = 0; j < 4; ++j) {
+            const int m = mrow + j * 16 + l16, f = en0 + wn * (MODE == 1 ? 32 : 64) + 8 * lq;
+            if constexpr (MODE == 3) {
 #pragma unroll
-          for (int hx = 0; hx < 2; ++hx)
+              for (int q = 0; q < 4; ++q) {
+                const int fq = f + (q >> 1) * 32 + (q & 1) * 4;
+                if (decltype(whole)::value || (m < M && fq < N)) *(floatx4_t*)(ep + (size_t)m * N + fq) = acc[q >> 1][q & 1][hx][j];
+              }
+            } else {
+              float v[8];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-              const int m = em0 + hx * 128 + wm * 64 + j * 16 + l16, f = en0 + hw * 128 + wn * 32 + i * 16 + 4 * lq;
-              if (m < M && f < N) *(floatx4_t*)(ep + (size_t)m * N + f) = acc[hw][i][hx][j];
+              for (int e = 0; e < 8; ++e)
+                v[e] = rnd_bf16(gelu_tanh_short(rnd_bf16(acc[0][e >> 2][hx][j][e & 3]))) * rnd_bf16(acc[1][e >> 2][hx][j][e & 3]);
+              put(u32x4_t{pack2_bf16(v[0], v[1]), pack2_bf16(v[2], v[3]), pack2_bf16(v[4], v[5]), pack2_bf16(v[6], v[7])}, m, f);
             }
-    } else
+          }
+        } else {                                       // 32 rows at a time through LDS, chunks XOR-ed with the row
 #pragma unroll
-    for (int hx = 0; hx < 2; ++hx)
+          for (int j = 0; j < 4; j += 2) {
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
+            for (int t = 0; t < 2; ++t)
 #pragma unroll
-        for (int hw = 0; hw < (MODE == 1 ? 1 : 2); ++hw)
+              for (int hw = 0; hw < 2; ++hw) {
+                const int r = t * 16 + l16, c = wn * 8 + hw * 4 + lq;
+                const floatx4_t a = acc[hw][0][hx][j + t], b = acc[hw][1][hx][j + t];
+                const u32x4_t v = {pack2_bf16(a[0], a[1]), pack2_bf16(a[2], a[3]), pack2_bf16(b[0], b[1]), pack2_bf16(b[2], b[3])};
+                asm volatile("ds_write_b128 %0, %1" ::"v"(scratch + (unsigned)(r * 512 + ((c ^ r) << 4))), "v"(v) : "memory");
+              }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            u32x4_t o[4];
 #pragma unroll
-          for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int t = 0; t < 2; ++t) {
-              const int c = hw * 16 + wn * 4 + i * 2 + (lq >> 1), r = t * 16 + l16;
-              float v[4];
-#pragma unroll
-              for (int e = 0; e < 4; ++e)
-                v[e] = MODE == 1 ? rnd_bf16(gelu_tanh_short(rnd_bf16(acc[0][i][hx][2 * j + t][e]))) * rnd_bf16(acc[1][i][hx][2 * j + t][e])
-                                 : acc[hw][i][hx][2 * j + t][e];
-              const u32x2_t p = {pack2_bf16(v[0], v[1]), pack2_bf16(v[2], v[3])};
-              asm volatile("ds_write_b64 %0, %1" ::"v"(scratch + (unsigned)(r * RBY + ((c ^ (r & (CH - 1))) << 4) + (lq & 1) * 8)), "v"(p) : "memory");
+            for (int i = 0; i < 4; ++i) {
+              const int r = i * 8 + (gl >> 5), c = gl & 31;
+              o[i] = lds_read16<0>(scratch + (unsigned)(r * 512 + ((c ^ r) << 4)));
             }
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        __builtin_amdgcn_s_barrier();
-        u32x4_t o[NST];
+            lds_wait<0>(o);
+            __builtin_amdgcn_s_barrier();
 #pragma unroll
-        for (int i = 0; i < NST; ++i) {
-          const int r = (i * 256 + gl) / CH, c = gl % CH;
-          o[i] = lds_read16<0>(scratch + (unsigned)(r * RBY + ((c ^ (r & (CH - 1))) << 4)));
-        }
-        lds_wait<0>(o);
-        __builtin_amdgcn_s_barrier();
-#pragma unroll
-        for (int i = 0; i < NST; ++i) {
-          const int r = (i * 256 + gl) / CH, c = gl % CH;
-          const int m = em0 + hx * 128 + wm * 64 + j * 32 + r, f = en0 + c * 8;
-          if (m < M && f < N) store_feat8<MODE>(o[i], MODE == 2 ? er + (size_t)m * ldr + f : nullptr, ec + (size_t)m * ldc + f, N - f);
+            for (int i = 0; i < 4; ++i) put(o[i], mrow + j * 16 + i * 8 + (gl >> 5), en0 + (gl & 31) * 8);
+          }
         }
       }
+    };
+    young = !TA && em0 + 256 <= M && en0 + NF <= N;    // with transposing reads the loop is 2 to 5 % slower for the other waits
+    if (young) leave(std::true_type{});
+    else leave(std::false_type{});
     if (!more) break;
   }
 #undef PP_OPEN_TILE
@@ -647,10 +669,10 @@ int gemm_pp_launch(const void* A, long long lda, const void* W, const void* W2, 
                    long long ldc, int M, int N, int K, hipStream_t s, int nbatch = 1, long long sa = 0, long long sc = 0, long long sr = 0, int nb = 1) {
   constexpr int NF = MODE == 1 ? 128 : 256;
   static fstu_lds_limit most;
-  if (const int rc = fstu_need_lds((const void*)gemm_pp_bf16_kernel<MODE, TA>, most, PP_LDS, "fstu_gemm_bf16")) return rc;
+  if (const int rc = fstu_need_lds((const void*)gemm_pp_bf16_kernel<MODE, TA>, most, PP_LDS(MODE), "fstu_gemm_bf16")) return rc;
   const int mts = (M + 255) / 256, mt = mts * nbatch, nt = (N + NF - 1) / NF;
   const int share = (int)(((long long)mt * nt + 7) / 8);
-  hipLaunchKernelGGL((gemm_pp_bf16_kernel<MODE, TA>), dim3(8u * (unsigned)std::min(share, gemm_cus() / 8)), dim3(512), PP_LDS, s, (const bf16_t*)A, lda,
+  hipLaunchKernelGGL((gemm_pp_bf16_kernel<MODE, TA>), dim3(8u * (unsigned)std::min(share, gemm_cus() / 8)), dim3(512), PP_LDS(MODE), s, (const bf16_t*)A, lda,
                      (const bf16_t*)W, (const bf16_t*)W2, (const bf16_t*)R, ldr, (bf16_t*)C, ldc, M, N, K, mt, nt, share, mts, sa, sc, sr, nb);
   return 0;
 }
@@ -874,34 +896,30 @@ using TileRows32 = GemmTile<2, 1, 2, 1, 64, 4>;  // 128 features x 32 rows, 2 wa
 using Tile96 = GemmTile<1, 4, 3, 1, 64, 4>;      // 96 features x 128 rows, 4 waves, 112 KB: N = 768 or 2304 in whole tiles
 using TileK32 = GemmTile<2, 2, 4, 2, 32, 3>;     // 256 x 128, 4 waves, 72 KB, k tiles of 32 for K % 64 != 0
 
-// Whether a product (K % 64 == 0) runs on 256 x 256 tiles.
-// A round of 256 x 256 tiles (one per compute unit) in the alternating-group kernel takes as long as 2.25 rounds of 128 x
-// 128 tiles (K = 2048: 40 us against 18 us), so the large tile wins where its last round is not too empty.  Both sides
-// of the line, us (large / small): 2048 x 4096 x 2048 (128 large tiles) 39.8 / 37.6, 2331 x 4096 x 2048 (160) 40.0 / 54.1;
-// 3072 x 2304 x 768 (108) 20.9 / 19.0, 4096 x 2304 x 768 (144) 21.5 / 27.9; 777 x 2 x 9216 x 768 (288) 41 / 28,
-// 1536 x 2 x 9216 x 768 (432) 43 / 51; 384 x 50257 x 768 (394) 38.5 / 45.6.
-// In mode 1 a round ends in the GELU of its whole tile, beside which a short K hides little, while two small tiles on a
-// compute unit cover each other's: us, large / small tiles, 20000 x 2 x 512 (two rounds, 2.44 small tiles per place in them)
-// K = 64 20.5 / 15.4, 256 25.8 / 21.4, 512 33.6 / 30.4, 768 42.2 / 39.8; 8192 x 2 x 2304 (three rounds, 3) 28.6 / 24.8, 39.8 /
-// 36.1, 53.6 / 51.5, 68.7 / 69.3; 4096 x 2 x 1536 (one round, 3) K = 256 14.8 / 14.0, 512 18.7 / 20.5; 6000 x 2 x 2304 (two,
-// 3.3) K = 64 20.6 / 20.0, 256 27.1 / 29.2.
-bool pp_takes(int mode, int M, int N, int K) {
-  const int nf = mode == 1 ? 2 : 1;
-  const long long big = (long long)((M + 255) / 256) * (((long long)N * nf + 255) / 256);
-  const long long small = (long long)((M + 127) / 128) * (((long long)N * nf + 127) / 128);
-  const long long rounds = (big + gemm_cus() - 1) / gemm_cus();
-  const int quarters = mode != 1 || K >= 1024 ? 9 : K < 256 ? 14 : K < 512 ? 13 : rounds == 1 ? 9 : 11;
-  return quarters * rounds * gemm_cus() < 4 * small;
+// Whether a product (K % 64 == 0) of that many tiles of either size runs on 256 x 256 tiles: both sides' estimate in twentieths of
+// a round of small tiles, two to a compute unit.  A last round of small tiles costs 0.4 of a full one however few they are, and
+// their stores, a quarter of a line at a time, 0.2 more than the large tiles' do.  A round of large tiles, one to a compute
+// unit, takes 1.15 of them, and in mode 1, whose GELU covers only half of its round's products, 1.4 where K is long and 1.55
+// where it is short.  us, large / small tiles.  Mode 0: 4096 x 2304 (144 large tiles, 576 small) K = 64 8.8 / 13.1, 768 17.8 / 25.9,
+// 2048 37.9 / 53.0; 2048 x 4096 (128, 512) 8.8 / 12.2, 17.8 / 19.6, 35.7 / 37.1; 8192 x 2304 (288, 1152) K = 768 38.5 / 42.9, 2048
+// 78.6 / 82.6; the line: 3840 x 2048 (120, 480) K = 256 10.7 / 11.4, 2048 39.0 / 35.4.  Mode 1: 4096 x 2 x 1152 (144, 576) K = 64
+// 9.4 / 9.8, 768 18.9 / 23.2, 2048 36.7 / 50.9; 8192 x 2 x 2304 (576, 2304) 21.6 / 22.3, 57.4 / 62.6, 128 / 144; the line: 8192
+// x 2 x 1152 (288, 1152) 15.7 / 14.2, 37.1 / 36.5, 81.6 / 80.6, 20000 x 2 x 512 (316, 1256) 15.7 / 14.2, 36.8 / 35.7, 80.5 / 81.1.
+bool pp_takes(int mode, int K, long long big, long long small) {
+  const long long cus = gemm_cus(), full = small / (2 * cus), rest = small % (2 * cus);
+  const long long little = (mode == 1 ? 6 : 4) + 20 * full + (rest ? 8 + 6 * rest / cus : 0);
+  return (mode != 1 ? 23 : K >= 1024 ? 28 : 31) * ((big + cus - 1) / cus) < little;
 }
+long long tiles_of(int side, int M, int N) { return (long long)((M + side - 1) / side) * (((long long)N + side - 1) / side); }
 
 template <int MODE>
 int gemm_launch(const void* A, long long lda, const void* W, const void* W2, const void* R, long long ldr, void* C, long long ldc,
                 int M, int N, int K, hipStream_t s) {
   if (K % 64 != 0) return gemm_launch_tile<TileK32, MODE>(A, lda, W, W2, R, ldr, C, ldc, M, N, K, s);
   if (M <= 32) return gemm_launch_tile<TileRows32, MODE>(A, lda, W, W2, R, ldr, C, ldc, M, N, K, s);
-  const int nf = MODE == 1 ? 2 : 1;
-  const long long small = (long long)((M + 127) / 128) * (((long long)N * nf + 127) / 128);
-  if (pp_takes(MODE, M, N, K))
+  const int columns = MODE == 1 ? 2 * N : N;
+  const long long small = tiles_of(128, M, columns);
+  if (pp_takes(MODE, K, tiles_of(256, M, columns), small))
     return gemm_pp_launch<MODE>(A, lda, W, W2, R, ldr, C, ldc, M, N, K, s);
   // A grid that leaves one workgroup per compute unit anyway gains from the deeper pipeline when K is long (M=4096, N=768,
   // K=9216: 83 us against 93 us).
@@ -963,7 +981,7 @@ SlicePlan slice_plan(int M, int N, int K, int nb) {
   const int before = fstu_gemm_bf16_slices(M, N, K, nb);
   if (M < 256 || N % 4 != 0 || K % 64 != 0 || K < 2048) return {before, false};
   const long long cus = gemm_cus();
-  const long long small = (long long)((M + 127) / 128) * ((N + 127) / 128) * nb, big = (long long)((M + 255) / 256) * ((N + 255) / 256) * nb;
+  const long long small = tiles_of(128, M, N) * nb, big = tiles_of(256, M, N) * nb;
   const int nkt = K / 64;
   const auto join = [&](int s) { return s == 1 ? 0.0 : 3.0 + 8e-6 / 4.0 * s * nb * (double)M * N; };
   const auto large = [&](int s) {
@@ -1137,7 +1155,6 @@ extern "C" int fstu_gemm_bf16_ta_ws(const void* A, int64_t lda, int64_t batch_st
   FSTU_REQUIRE(fstu_aligned(A, 16) && fstu_aligned(W, 16) && fstu_aligned(C, 8) && fstu_aligned(R, 8), FSTU_EALIGN,
                "fstu_gemm_bf16_ta: pointers must be 16-byte aligned (C, R: 8)");
   hipStream_t s = (hipStream_t)stream;
-  const long long big = (long long)(M / 256) * ((N + 255) / 256) * nbatch;
   int rc;
   if (ksplit > 1) {
     if ((rc = split_check("fstu_gemm_bf16_ta_ws", N, K, ksplit, partial))) return rc;
@@ -1154,12 +1171,10 @@ extern "C" int fstu_gemm_bf16_ta_ws(const void* A, int64_t lda, int64_t batch_st
                                             nbatch, s)                                                                           \
              : gemm_ta_launch_tile<TILE, 2>(A, lda, batch_stride_a, W, R, ldr, batch_stride_r, C, ldc, batch_stride_c, M, N, K,  \
                                             nbatch, s))
-  // The line between the tiles is gemm_launch's (a round of large tiles against 2.25 of small ones).  Large / 128 x 128 tiles
-  // (or 256 x 256 tiles all in step, the form before), us, K = 24 N: 4 x 8192 x 1024 (512 large tiles) 1155 / 1475, 2 x 8192 x
-  // 1024 (256) 547 / 833, 4 x 8192 x 768 (384) 758 / 880, 4 x 8192 x 512 (256) 295 / 458, 4 x 2048 x 1024 (128) 432 / 453,
-  // 1 x 8192 x 1024 (128) 443 / 440, 1 x 4096 x 768 (48) 176 / 179.
-  const long long small = (long long)(M / 128) * ((N + 127) / 128) * nbatch;
-  if (M % 256 == 0 && 9 * ((big + gemm_cus() - 1) / gemm_cus()) * gemm_cus() < 4 * small)
+  // The line between the tiles is gemm_launch's.  Large / 128 x 128 tiles (or 256 x 256 tiles all in step, the form before), us,
+  // K = 24 N: 4 x 8192 x 1024 (512 large tiles) 1155 / 1475, 2 x 8192 x 1024 (256) 547 / 833, 4 x 8192 x 768 (384) 758 / 880,
+  // 4 x 8192 x 512 (256) 295 / 458, 4 x 2048 x 1024 (128) 432 / 453, 1 x 8192 x 1024 (128) 443 / 440, 1 x 4096 x 768 (48) 176 / 179.
+  if (M % 256 == 0 && pp_takes(0, K, tiles_of(256, M, N) * nbatch, tiles_of(128, M, N) * nbatch))
     rc = mode == 0 ? gemm_pp_launch<0, true>(A, lda, W, nullptr, R, ldr, C, ldc, M, N, K, s, nbatch, batch_stride_a, batch_stride_c, batch_stride_r)
                    : gemm_pp_launch<2, true>(A, lda, W, nullptr, R, ldr, C, ldc, M, N, K, s, nbatch, batch_stride_a, batch_stride_c, batch_stride_r);
   else rc = TA_GO(TileSmall);

@@ -393,6 +393,31 @@ def test_gemm_bf16_transposed_activations_large_tiles(hip, nb, M, N, K):
     assert torch.equal(hip.gemm_ta(wide[:, :, :M], W), got)
 
 
+@pytest.mark.parametrize("M,N,K", [(4196, 4356, 64), (4352, 4355, 128), (4097, 4360, 192), (2049, 4104, 128)])
+def test_gemm_bf16_large_tiles_one_behind_the_other(hip, M, N, K):
+    """More 256 x 256 tiles than compute units (the last shape: fewer, more than a round of small tiles), whole ones in front of ragged
+    ones and the other way round, one to three k tiles: plain, residual and gated pair, nothing written behind the rows."""
+    g = gen(M + K)
+    A, W, U = (dev(torch.randn(n, K, generator=g).bfloat16()) for n in (M, N, N))
+    out = torch.full((M + 1, N + 5), float("nan"), dtype=torch.bfloat16, device="cuda")
+    ref = torch.matmul(A.float(), W.float().t().contiguous())     # fp32 on the library: K * 2^-24 of the absolute sum like the kernel's
+    bound = 2 * K * 2.0 ** -24 * torch.matmul(A.float().abs(), W.float().abs().t().contiguous()) + 2.0 ** -8 * ref.abs()
+    y = hip.gemm(A, W, out=out[:M, :N])
+    assert bool(((y.float() - ref).abs() <= bound).all())
+    assert bool(out[M:].isnan().all()) and bool(out[:, N:].isnan().all())
+    if N % 4 == 0:
+        R = dev(torch.randn(M, N, generator=g).bfloat16())
+        assert torch.equal(hip.gemm(A, W, residual=R, out=R.clone()), (R.float() + y.float()).bfloat16())
+        out = torch.full((M + 1, N + 4), float("nan"), dtype=torch.bfloat16, device="cuda")
+        act = hip.gemm(A, W, up_weight=U, out=out[:M, :N])
+        gate, up = ref.bfloat16(), torch.matmul(A.float(), U.float().t().contiguous()).bfloat16()
+        r = (F.gelu(gate, approximate="tanh") * up).float()
+        # the bound of test_gemm_bf16_gated_pair
+        tol = r.abs() * 2.0 ** -6 + 1.2 * 2.0 ** -7 * (gate.float() * up.float()).abs() + 1e-3 * 2.0 ** -7 * float(r.abs().max())
+        assert bool(((act.float() - r).abs() <= tol).all())
+        assert bool(out[M:].isnan().all()) and bool(out[:, N:].isnan().all())
+
+
 @pytest.mark.parametrize("M,d,I", [(4096, 768, 3072), (300, 256, 1000), (2048, 1024, 8192), (100, 96, 132)])
 def test_gemm_bf16_gated_pair(hip, M, d, I):
     """Mode 1: T(T(gelu_tanh(T(x Wg^T))) * T(x Wu^T)) in one kernel equals the three-step bf16 chain of the reference
