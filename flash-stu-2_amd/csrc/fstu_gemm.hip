@@ -706,15 +706,32 @@ template <int N> __device__ __forceinline__ void pin2(u32x2_t* f) {
   for (int i = 0; i < N; ++i) asm volatile("" : "+v"(f[i]));
 }
 
-template <class G, int MODE>
+template <bool TW, int FI> struct WeightFrags {
+  u32x4_t f[FI];
+  __device__ __forceinline__ bf16x8_t frag(int i) const { return __builtin_bit_cast(bf16x8_t, f[i]); }
+  __device__ __forceinline__ void pin() { pin4<FI>(f); }
+};
+template <int FI> struct WeightFrags<true, FI> {
+  u32x2_t f[2 * FI];
+  __device__ __forceinline__ bf16x8_t frag(int i) const { return __builtin_bit_cast(bf16x8_t, (Frag8{f[2 * i], f[2 * i + 1]})); }
+  __device__ __forceinline__ void pin() { pin2<2 * FI>(f); }
+};
+
+// TW: the weights come the same way, (K, N) with rows of ldw elements and N a multiple of the tile, and take the same way through
+// LDS: the gradient of a weight, whose sum over all positions has both operands' reduction index slowest.  What bounds it is a
+// workgroup's chain of k tiles, 0.6 us each alone on a compute unit (the fills, which four stages do not shorten: M = N = 768,
+// K = 16384 in 7 slices 31.7 us with four, 32.3 with two; two workgroups to a unit 48 and 36 in 8).
+template <class G, int MODE, bool TW = false>
 __global__ void __launch_bounds__(G::THREADS)
-gemm_ta_bf16_kernel(const bf16_t* __restrict__ A, long long lda, long long sa, const bf16_t* __restrict__ W,
+gemm_ta_bf16_kernel(const bf16_t* __restrict__ A, long long lda, long long sa, const bf16_t* __restrict__ W, long long ldw,
                     const bf16_t* __restrict__ R, long long ldr, long long sr, bf16_t* __restrict__ C, long long ldc,
                     long long sc, int M, int N, int K, int mt, int nt, int share, int nbatch, int ksplit) {
   constexpr int FI = G::FI, TJ = G::TJ, BF = G::BF, BT = G::BT, WL = G::WL, AL = G::AL, NS = G::NS, KK = G::KK;
   constexpr unsigned STAGE = G::STAGE;
   constexpr int RBT = BT * 2, CPRT = BT / 8;              // bytes and 16-byte chunks of an activation row (one k)
-  constexpr int NRD = FI + 2 * TJ;                        // LDS reads per k step
+  constexpr int RBW = BF * 2, CPRW = BF / 8;              // TW: the same of a weight row
+  constexpr int NRD = (TW ? 2 : 1) * FI + 2 * TJ;         // LDS reads per k step
+  static_assert(!TW || MODE == 0 || MODE == 3, "TW: plain or split-K epilogue");
   static_assert(G::BK == 64 && BT >= 128, "k tile of 64, at least 128 columns");
   static_assert((MODE == 0 || MODE == 2 || MODE == 3), "plain, residual or split-K epilogue");
   extern __shared__ __align__(16) unsigned char gm_smem[];
@@ -724,19 +741,21 @@ gemm_ta_bf16_kernel(const bf16_t* __restrict__ A, long long lda, long long sa, c
   if ((int)(blockIdx.x >> 3) >= share || o >= mt * nt * nbatch * ksplit) return;
   const int bs = o / (mt * nt), slice = bs / nbatch, batch = bs - slice * nbatch;    // MODE 3: slices of K outermost
   o -= bs * (mt * nt);
-  const int KS = MODE == 3 ? K / ksplit : K;           // this workgroup's share of K
+  const int kbeg = MODE == 3 ? (int)((long long)(K / G::BK) * slice / ksplit) * G::BK : 0;      // this workgroup's share of K
+  const int KS = MODE == 3 ? (int)((long long)(K / G::BK) * (slice + 1) / ksplit) * G::BK - kbeg : K;
   const int per_panel = mt * GM_PANEL;
   const int panel = o / per_panel, in_panel = o - panel * per_panel;
   const int pw = min(GM_PANEL, nt - panel * GM_PANEL);
   const int bt = in_panel / pw, bf = panel * GM_PANEL + in_panel % pw;
   const int m0 = bt * BT, n0 = bf * BF;
-  A += (size_t)batch * sa + (MODE == 3 ? (size_t)slice * KS * lda : 0);
-  if (MODE == 3) W += (size_t)slice * KS;
+  A += (size_t)batch * sa + (MODE == 3 ? (size_t)kbeg * lda : 0);
+  if (MODE == 3) W += TW ? (size_t)kbeg * ldw : (size_t)kbeg;
   C += (size_t)batch * sc;
   if (MODE == 2) R += (size_t)batch * sr;
   const int wv = __builtin_amdgcn_readfirstlane(w);
   const int rows_w = min(BF, N - n0);
-  const rsrc_t rs_w = make_rsrc(W + (size_t)n0 * K, ((size_t)(rows_w - 1) * K + KS) * 2);
+  const rsrc_t rs_w = TW ? make_rsrc(W + n0, ((size_t)(KS - 1) * ldw + BF) * 2)
+                         : make_rsrc(W + (size_t)n0 * K, ((size_t)(rows_w - 1) * K + KS) * 2);
   const rsrc_t rs_a = make_rsrc(A + m0, ((size_t)(KS - 1) * lda + BT) * 2);    // M % BT == 0: whole rows of BT columns
   unsigned wvoff[WL], avoff[AL];
 #pragma unroll
@@ -744,6 +763,10 @@ gemm_ta_bf16_kernel(const bf16_t* __restrict__ A, long long lda, long long sa, c
     const int slot = (wv * WL + j) * 64 + lane, row = slot / G::CPR;
     const int ch = (int)((G::swz(row, slot % G::CPR) - (unsigned)row * G::RB) >> 4);
     wvoff[j] = (unsigned)row * (unsigned)K * 2u + (unsigned)ch * 16u;
+    if constexpr (TW) {
+      const int kr = slot / CPRW;
+      wvoff[j] = (unsigned)kr * (unsigned)ldw * 2u + (unsigned)((slot % CPRW) ^ (4 * (kr & 3))) * 16u;
+    }
   }
 #pragma unroll
   for (int j = 0; j < AL; ++j) {
@@ -755,7 +778,7 @@ gemm_ta_bf16_kernel(const bf16_t* __restrict__ A, long long lda, long long sa, c
 #define GT_FETCH(stage_, k0)                                                                                 \
   {                                                                                                          \
     unsigned char* st_ = gm_smem + (unsigned)(stage_) * STAGE;                                               \
-    const unsigned sw_ = (unsigned)(k0) * 2u;                                                                \
+    const unsigned sw_ = TW ? (unsigned)((size_t)(k0) * (size_t)ldw * 2u) : (unsigned)(k0) * 2u;              \
     const unsigned sa_ = (unsigned)((size_t)(k0) * (size_t)lda * 2u);                                        \
     _Pragma("unroll") for (int j = 0; j < WL; ++j) buf_load16_to_lds(rs_w, wvoff[j], sw_, st_ + wslot + j * 1024); \
     _Pragma("unroll") for (int j = 0; j < AL; ++j) buf_load16_to_lds(rs_a, avoff[j], sa_, st_ + aslot + j * 1024); \
@@ -764,8 +787,7 @@ gemm_ta_bf16_kernel(const bf16_t* __restrict__ A, long long lda, long long sa, c
   _Pragma("unroll") for (int i = 0; i < FI; ++i)                                                             \
     _Pragma("unroll") for (int j = 0; j < TJ; ++j) {                                                         \
       const Frag8 b_ = {fx_[2 * j], fx_[2 * j + 1]};                                                         \
-      acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, fw_[i]),              \
-                                                          __builtin_bit_cast(bf16x8_t, b_), acc[i][j], 0, 0, 0); \
+      acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fw_.frag(i), __builtin_bit_cast(bf16x8_t, b_), acc[i][j], 0, 0, 0); \
     }
   const int l32 = lane & 31, lh = lane >> 5;
   unsigned fw_off[KK];
@@ -777,6 +799,11 @@ gemm_ta_bf16_kernel(const bf16_t* __restrict__ A, long long lda, long long sa, c
 #pragma unroll
   for (int j = 0; j < TJ; ++j)
     ta_off[j] = (unsigned)BF * G::RB + (unsigned)(8 * (blk >> 1) + key) * RBT + (unsigned)(((wt * TJ + j) ^ key) << 6) +
+                (unsigned)(2 * (blk & 1) + ((i16 & 3) >> 1)) * 16u + (unsigned)(i16 & 1) * 8u;
+  unsigned tw_off[FI];                                    // TW: the same for the feature tiles
+#pragma unroll
+  for (int i = 0; i < FI; ++i)
+    tw_off[i] = (unsigned)(8 * (blk >> 1) + key) * RBW + (unsigned)(((wf * FI + i) ^ key) << 6) +
                 (unsigned)(2 * (blk & 1) + ((i16 & 3) >> 1)) * 16u + (unsigned)(i16 & 1) * 8u;
   floatx16_t acc[FI][TJ];
 #pragma unroll
@@ -795,19 +822,24 @@ gemm_ta_bf16_kernel(const bf16_t* __restrict__ A, long long lda, long long sa, c
   else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __builtin_amdgcn_s_barrier();
   if (NS - 1 < nkt) GT_FETCH(NS - 1, (NS - 1) * G::BK)
-  u32x4_t wa_[FI], wb_[FI];                           // weight fragments of alternate k steps
+  WeightFrags<TW, FI> wa_, wb_;                       // weight fragments of alternate k steps
   u32x2_t xa_[2 * TJ], xb_[2 * TJ];                   // activation fragments (two halves per column tile)
-  unsigned ta[TJ];
+  unsigned ta[TJ], tw[FI];
 #define GT_READ(fw_, fx_, base_, kk_)                                                                        \
   {                                                                                                          \
-    lds_read_rows<FI, 32 * G::RB>(fw_, (base_) + fw_off[kk_]);                                               \
+    if constexpr (TW) {                                                                                      \
+      _Pragma("unroll") for (int i = 0; i < FI; ++i) tw[i] = (base_) + tw_off[i] + (unsigned)(kk_) * 16u * RBW; \
+      lds_read_tr_cols<FI, RBW>(fw_.f, tw);                                                                  \
+    } else {                                                                                                 \
+      lds_read_rows<FI, 32 * G::RB>(fw_.f, (base_) + fw_off[kk_]);                                           \
+    }                                                                                                        \
     _Pragma("unroll") for (int j = 0; j < TJ; ++j) ta[j] = (base_) + ta_off[j] + (unsigned)(kk_) * 16u * RBT; \
     lds_read_tr_cols<TJ, RBT>(fx_, ta);                                                                      \
   }
 #define GT_WAIT(left_, fw_, fx_)                                                                             \
   {                                                                                                          \
     lds_wait_n<left_>();                                                                                     \
-    pin4<FI>(fw_);                                                                                           \
+    fw_.pin();                                                                                               \
     pin2<2 * TJ>(fx_);                                                                                       \
   }
   GT_READ(wa_, xa_, smem0, 0)
@@ -875,16 +907,16 @@ gemm_ta_bf16_kernel(const bf16_t* __restrict__ A, long long lda, long long sa, c
   }
 }
 
-template <class G, int MODE>
+template <class G, int MODE, bool TW = false>
 int gemm_ta_launch_tile(const void* A, long long lda, long long sa, const void* W, const void* R, long long ldr, long long sr,
-                        void* C, long long ldc, long long sc, int M, int N, int K, int nbatch, hipStream_t s, int ksplit = 1) {
+                        void* C, long long ldc, long long sc, int M, int N, int K, int nbatch, hipStream_t s, int ksplit = 1, long long ldw = 0) {
   static fstu_lds_limit most;
-  if (const int rc = fstu_need_lds((const void*)gemm_ta_bf16_kernel<G, MODE>, most, G::LDS, "fstu_gemm_bf16_ta")) return rc;
+  if (const int rc = fstu_need_lds((const void*)gemm_ta_bf16_kernel<G, MODE, TW>, most, G::LDS, "fstu_gemm_bf16_ta")) return rc;
   const int mt = M / G::BT, nt = (N + G::BF - 1) / G::BF;
   const long long tiles = (long long)mt * nt * nbatch * ksplit;
   const int share = (int)((tiles + 7) / 8);
-  hipLaunchKernelGGL((gemm_ta_bf16_kernel<G, MODE>), dim3((unsigned)share * 8u), dim3(G::THREADS), G::LDS, s, (const bf16_t*)A, lda, sa,
-                     (const bf16_t*)W, (const bf16_t*)R, ldr, sr, (bf16_t*)C, ldc, sc, M, N, K, mt, nt, share, nbatch, ksplit);
+  hipLaunchKernelGGL((gemm_ta_bf16_kernel<G, MODE, TW>), dim3((unsigned)share * 8u), dim3(G::THREADS), G::LDS, s, (const bf16_t*)A, lda, sa,
+                     (const bf16_t*)W, ldw, (const bf16_t*)R, ldr, sr, (bf16_t*)C, ldc, sc, M, N, K, mt, nt, share, nbatch, ksplit);
   return 0;
 }
 
@@ -1181,5 +1213,53 @@ extern "C" int fstu_gemm_bf16_ta_ws(const void* A, int64_t lda, int64_t batch_st
 #undef TA_GO
   if (rc) return rc;
   FSTU_CHECK_LAUNCH("fstu_gemm_bf16_ta");
+  return FSTU_OK;
+}
+
+// Slices of K for fstu_gemm_bf16_tt, any number of k tiles to each: the least of an estimate, a chain of k tiles at 0.6 us alone on a
+// compute unit and 0.86 two to a unit, and the join as in fstu_gemm_bf16_slices.  us, joined, with the slices it picks / one fewer / one
+// more (or the next tried) / the transpose and fstu_gemm_bf16_ta in slices of one length, rows x features x K: 768 x 768 x 16384 32.3 (7) /
+// 34.2 / 36.4 / 50.5, x 8192 22.3 (7) / 23.1 / 26.3 / 34.1, 512 x 512 x 4096 15.7 (8) / 15.3 / 15.3 / 22.9, 256 x 256 x 16384 17.2 (32) / 16.7
+// (28) / - / 24.3, 768 x 768 x 1024 12.3 (1) / - / 13.4 / 18.2, 1024 x 1024 x 16384 43.9 (8) / 45.1 / 53.1 (10) / 63.8, 2048 x 2048 x 16384
+// 135.6 (2) / 166.6 / 143.8 / 138.1.
+extern "C" int fstu_gemm_bf16_tt_slices(int M, int N, int K) {
+  if (M % 128 != 0 || N % 128 != 0 || K % 64 != 0 || M < 1 || N < 1 || K < 64) return 1;
+  const long long cus = gemm_cus(), tiles = (long long)(M / 128) * (N / 128);
+  const int nkt = K / 64;
+  double least = 1e30;
+  int best = 1;
+  for (int s = 1; s <= 32 && s <= nkt && (s == 1 || tiles * s <= 2 * cus); ++s) {
+    const double us = (nkt + s - 1) / s * (tiles * s <= cus ? 0.6 : 0.86 * (double)((tiles * s + 2 * cus - 1) / (2 * cus))) + (s == 1 ? 0.0 : 3.0 + 8e-6 / 4.0 * s * (double)M * N);
+    if (us < least) { least = us; best = s; }
+  }
+  return best;
+}
+
+// C[m, n] = T(sum_k A[k, m] W[k, n]) for A (K, M) and W (K, N), rows of lda and ldw elements, M and N multiples of 128, K of 64, in
+// ksplit slices of K (partial: ksplit * M * N fp32), which a second launch adds
+extern "C" int fstu_gemm_bf16_tt(const void* A, int64_t lda, const void* W, int64_t ldw, void* C, int64_t ldc, int M, int N, int K,
+                                 float* partial, int ksplit, void* stream) {
+  FSTU_REQUIRE(A && W && C, FSTU_ENULL, "fstu_gemm_bf16_tt: null pointer");
+  FSTU_REQUIRE(M >= 128 && M % 128 == 0 && N >= 128 && N % 128 == 0 && K >= 64 && K % 64 == 0, FSTU_ESHAPE,
+               "fstu_gemm_bf16_tt: need M %% 128 == 0, N %% 128 == 0, K %% 64 == 0 (M=%d N=%d K=%d)", M, N, K);
+  FSTU_REQUIRE(lda >= M && lda % 8 == 0 && ldw >= N && ldw % 8 == 0 && ldc >= N && ldc % 4 == 0, FSTU_ESHAPE,
+               "fstu_gemm_bf16_tt: row strides (lda=%lld ldw=%lld ldc=%lld)", (long long)lda, (long long)ldw, (long long)ldc);
+  // 32-bit byte offsets inside both operands (buffer addressing)
+  FSTU_REQUIRE(lda < GM_MAX_LD && ldw < GM_MAX_LD && (unsigned long long)K * (unsigned long long)std::max(lda, ldw) * 2ull < 0xfff00000ull,
+               FSTU_ESHAPE, "fstu_gemm_bf16_tt: an operand exceeds 4 GB of 32-bit offsets");
+  FSTU_REQUIRE(fstu_aligned(A, 16) && fstu_aligned(W, 16) && fstu_aligned(C, 8), FSTU_EALIGN,
+               "fstu_gemm_bf16_tt: pointers must be 16-byte aligned (C: 8)");
+  hipStream_t s = (hipStream_t)stream;
+  int rc;
+  if (ksplit > 1) {
+    FSTU_REQUIRE(partial && fstu_aligned(partial, 16) && ksplit <= 64 && ksplit <= K / 64, FSTU_ESHAPE, "fstu_gemm_bf16_tt: %d slices of K=%d", ksplit, K);
+    rc = gemm_ta_launch_tile<TileSmall, 3, true>(A, lda, 0, W, partial, 0, 0, C, 0, 0, M, N, K, 1, s, ksplit, ldw);
+    if (rc) return rc;
+    FSTU_CHECK_LAUNCH("fstu_gemm_bf16_tt");
+    return fstu_join_slices(partial, ksplit, nullptr, 0, 0, C, ldc, 0, 1, M, N, stream);
+  }
+  rc = gemm_ta_launch_tile<TileSmall, 0, true>(A, lda, 0, W, nullptr, 0, 0, C, ldc, 0, M, N, K, 1, s, 1, ldw);
+  if (rc) return rc;
+  FSTU_CHECK_LAUNCH("fstu_gemm_bf16_tt");
   return FSTU_OK;
 }

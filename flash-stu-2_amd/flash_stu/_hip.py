@@ -111,6 +111,8 @@ SIGNATURES = {
     "fstu_gemm_bf16_ws": [_vp, _i64, _vp, _vp, _vp, _i64, _vp, _i64, _i, _i, _i, _i, _vp, _i, _vp],
     "fstu_gemm_bf16_ta_ws": [_vp, _i64, _i64, _vp, _vp, _i64, _i64, _vp, _i64, _i64, _i, _i, _i, _i, _i, _vp, _i, _vp],
     "fstu_gemm_bf16_ta": [_vp, _i64, _i64, _vp, _vp, _i64, _i64, _vp, _i64, _i64, _i, _i, _i, _i, _i, _vp],
+    "fstu_gemm_bf16_tt_slices": [_i, _i, _i],
+    "fstu_gemm_bf16_tt": [_vp, _i64, _vp, _i64, _vp, _i64, _i, _i, _i, _vp, _i, _vp],
     "fstu_lds_sequence_ws_floats": [_i, _i, _i],
     "fstu_lds_sequence_status": [_vp, _vp],
     "fstu_lds_sequence": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp],
@@ -432,6 +434,24 @@ def gemm_ta(slabs: torch.Tensor, weight: torch.Tensor, residual: Optional[torch.
                                        residual.stride(0) if residual is not None and nb > 1 else 0, _p(out), out.stride(1),
                                        out.stride(0) if nb > 1 else 0, M, N, K, nb, mode, _p(partial), slices, _stream()),
            "fstu_gemm_bf16_ta")
+    return out
+
+
+@functools.lru_cache(maxsize=256)
+def _gemm_tt_slices(M: int, N: int, K: int) -> int:
+    return load().fstu_gemm_bf16_tt_slices(M, N, K)
+
+
+def gemm_tt(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
+    """a^T @ b for a (K, M) and b (K, N) bf16 with contiguous rows, rounded once: a weight's gradient, summed over all positions.
+    M and N multiples of 128, K of 64."""
+    _dev(a, b)
+    (K, M), N = a.shape, b.shape[1]
+    if b.shape[0] != K or a.dtype != torch.bfloat16 or b.dtype != torch.bfloat16:
+        raise FlashSTUHipError(f"gemm_tt: operands {tuple(a.shape)} {a.dtype}, {tuple(b.shape)} {b.dtype}")
+    out = torch.empty(M, N, dtype=a.dtype, device=a.device)
+    slices, partial = _slice_sums(_gemm_tt_slices(M, N, K), M, N, device=a.device)
+    _check(load().fstu_gemm_bf16_tt(_p(a), M, _p(b), N, _p(out), N, M, N, K, _p(partial), slices, _stream()), "fstu_gemm_bf16_tt")
     return out
 
 

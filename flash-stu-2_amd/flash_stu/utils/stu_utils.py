@@ -193,8 +193,8 @@ class ApproxConvolveSum(torch.autograd.Function):
 
 class ProjectInputs(torch.autograd.Function):
     """x (B,T,d_in) @ m (d_in,d_out) in bf16 with its gradients on the matrix-core kernels.  The gradient of m sums over all
-    B*T positions: x is the contraction's slab as it lies (reduction index slowest), the output gradient is transposed once,
-    and the long sum is taken in slices (8 x 2048 positions of 768: 60 us with the transpose, the library product 97).
+    B*T positions: both operands are read as they lie (reduction index slowest), the long sum is taken in slices (8 x 2048
+    positions of 768: 32 us; with the output's gradient transposed in front 50, the library product 94).
     Where the gradients are to be differentiated themselves (create_graph=True) they are plain products."""
 
     @staticmethod
@@ -224,7 +224,7 @@ class ProjectInputs(torch.autograd.Function):
         gm = None
         if ctx.needs_input_grad[1]:
             x2 = _aligned(x.reshape(-1, x.shape[2]))
-            gm = _hip.gemm_ta(x2[None], _hip.transpose(g2[None])[0])[0]
+            gm = _hip.gemm_tt(x2, g2)
         return gx, gm
 
 

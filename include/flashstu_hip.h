@@ -459,6 +459,13 @@ int fstu_gemm_bf16_ws(const void* A, int64_t lda, const void* W, const void* W2,
 int fstu_gemm_bf16_ta_ws(const void* A, int64_t lda, int64_t batch_stride_a, const void* W, const void* R, int64_t ldr,
                          int64_t batch_stride_r, void* C, int64_t ldc, int64_t batch_stride_c, int M, int N, int K,
                          int nbatch, int mode, float* partial, int ksplit, void* stream);
+/* A weight's gradient: C (M,N) = T(A^T W) for A (K,M) and W (K,N), both with the reduction index slowest, rows of lda and ldw
+ * elements.  M, N % 128 == 0, K % 64 == 0, lda, ldw % 8 == 0, K*lda*2 and K*ldw*2 below 4 GB; A, W 16-byte aligned, C 8.  ksplit
+ * slices of K (1: none; fstu_gemm_bf16_tt_slices says how many pay), not all of one length, joined in order by a second launch;
+ * partial holds ksplit * M * N floats, 16-byte aligned. */
+int fstu_gemm_bf16_tt_slices(int M, int N, int K);
+int fstu_gemm_bf16_tt(const void* A, int64_t lda, const void* W, int64_t ldw, void* C, int64_t ldc, int M, int N, int K, float* partial,
+                      int ksplit, void* stream);
 
 /* ---- dense LDS (mini_stu/lds.py:95-101) ------------------------------------
  * T_steps consecutive steps with the fp32 state h (Bt,S) carried in place:

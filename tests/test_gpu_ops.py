@@ -418,6 +418,20 @@ def test_gemm_bf16_large_tiles_one_behind_the_other(hip, M, N, K):
         assert bool(out[M:].isnan().all()) and bool(out[:, N:].isnan().all())
 
 
+@pytest.mark.parametrize("K,M,N,slices", [(64, 128, 128, 1), (128, 256, 128, 1), (4160, 128, 384, None), (9280, 768, 768, 7), (2048, 2048, 2048, 1)])
+def test_gemm_bf16_tt(hip, K, M, N, slices):
+    """Both operands with the reduction index slowest, whole and in slices of unequal lengths: fp32 sums of exact products stay within
+    (K + slices) * 2^-24 of the absolute sum, one rounding to bf16."""
+    g = gen(K + N)
+    ns = hip.load().fstu_gemm_bf16_tt_slices(M, N, K)
+    assert ns == slices if slices else (ns > 1 and (K // 64) % ns)
+    A, B = (dev(torch.randn(K, n, generator=g).bfloat16()) for n in (M, N))
+    At = A.t().contiguous().float()
+    ref = torch.matmul(At, B.float())                                        # fp32 on the library: K * 2^-24 of the absolute sum too
+    bound = (2 * K + ns) * 2.0 ** -24 * torch.matmul(At.abs(), B.float().abs()) + 2.0 ** -8 * ref.abs()
+    assert bool(((hip.gemm_tt(A, B).float() - ref).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("M,d,I", [(4096, 768, 3072), (300, 256, 1000), (2048, 1024, 8192), (100, 96, 132)])
 def test_gemm_bf16_gated_pair(hip, M, d, I):
     """Mode 1: T(T(gelu_tanh(T(x Wg^T))) * T(x Wu^T)) in one kernel equals the three-step bf16 chain of the reference
