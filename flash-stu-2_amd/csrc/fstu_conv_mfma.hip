@@ -257,7 +257,12 @@ conv_mfma_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ taps, 
 // parity of one row: 70 KB of LDS at 2048 positions, and a second workgroup on the compute unit works while this one's operands come
 // and its results go.  A workgroup has 8 channels, a wave each, and goes through R items: the sums of the filter's gradient stay in
 // registers, and the next item is on its way while this one is worked on.  What it leaves are its items' fp32 sums, (chunks of
-// items, lags, channels), added in the order of the items by conv_grad_finish_kernel.
+// items, lags, channels), added in the order of the items by conv_grad_finish_kernel.  Where the filter is phi @ M_filters, it leaves
+// their product with the even rows of phi instead, phi_e (filters to whole tiles of 16, P lags), (chunks, filters, channels): a 42nd
+// of the bytes at 1024 lags and 24 filters, and no product behind the launch.  Eight of an MFMA's columns are the channels' sums rounded to
+// bf16, the other eight what that leaves of them, so a sum enters with 16 bits (8 as the gradient of the filter itself: 2.83e-3 off
+// float64 after its rounding, 2.44e-3 so).  8 x 2048 x 768 with the launch behind it 56 + 5 + 17 us (sums, their join, the library's
+// product) -> 60 + 5.
 //
 // us, transforms -> whole rows (106 KB, one workgroup to a compute unit) -> this, both launches: 8 x 512 x 768 29 -> 26 -> 22, 8 x 1024 x
 // 768 51 -> 39 -> 32, 2 x 2048 x 768 42 -> 27 -> 25, 8 x 2048 x 768 117 -> 80 -> 62, 8 x 2048 x 2048 - -> 163 -> 128.  A row's products alone
@@ -267,7 +272,7 @@ constexpr int cg_rows(int HB) { return 128 * HB + 256; }        // bytes of a ch
 template <int NT>
 __global__ void __launch_bounds__(512, 4)
 conv_grad_mfma_kernel(const bf16_t* __restrict__ gy, const bf16_t* __restrict__ x, const bf16_t* __restrict__ f, bf16_t* __restrict__ gx,
-                      float* __restrict__ part, int B, int T, int L, int d, int R) {
+                      float* __restrict__ part, const bf16_t* __restrict__ phi_e, int K, int P, int B, int T, int L, int d, int R) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
   constexpr int HB = 8 * NT, cap = 64 * HB, rg = cm_region(HB), gg = cg_rows(HB), PC = HB * 16;
   char* const xl = lds;                                       // 8 regions as in the forward
@@ -423,6 +428,19 @@ conv_grad_mfma_kernel(const bf16_t* __restrict__ gy, const bf16_t* __restrict__ 
     if (item + 1 < end) __syncthreads();
   }
   if (!part) return;
+  constexpr int STEPS = cap / 256;
+  const int lag0 = ch * (cap / 8) + 8 * g;
+  uint4 ph[2][STEPS];
+  auto rows_of_phi = [&](int k0) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int step = 0; step < STEPS; ++step) {
+        ph[t][step] = make_uint4(0, 0, 0, 0);
+        if (k0 + 16 * t < K && lag0 + 32 * step < P) ph[t][step] = *(const uint4*)(phi_e + (size_t)(k0 + 16 * t + col) * P + lag0 + 32 * step);
+      }
+  };
+  if (phi_e) rows_of_phi(0);
   // lags of a channel -> channels of a lag, through the space of x and the taps
   float* const fl32 = (float*)xl;
   if (col < 8) {
@@ -432,6 +450,45 @@ conv_grad_mfma_kernel(const bf16_t* __restrict__ gy, const bf16_t* __restrict__ 
       for (int r = 0; r < 4; ++r) *(floatx4_t*)(fl32 + ch * (cap + 4) + (c + 8 * j) * 64 + 16 * r + 4 * g) = S[j][r];
   }
   __syncthreads();
+  if (phi_e) {
+    // wave ch: an eighth of the lags; the waves' tiles of 2 x 16 filters x (8 channels, 8 remainders) meet in the space of g and the rings
+    float* const red = (float*)gl;
+    for (int k0 = 0; k0 < K; k0 += 32) {
+      floatx4_t acc[2];
+      acc[0] = acc[1] = (floatx4_t){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int step = 0; step < STEPS; ++step) {
+        const float* s = fl32 + c * (cap + 4) + lag0 + 32 * step;
+        const float4 v0 = *(const float4*)s, v1 = *(const float4*)(s + 4);
+        float v[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
+        if (col >= 8)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const float head = DT<bf16_t>::rnd(v[e]);
+            v[e] = head == v[e] ? 0.f : v[e] - head;           // an infinite sum leaves nothing
+          }
+        const bf16x8_t b = as_frag(make_uint4(pack2_bf16(v[0], v[1]), pack2_bf16(v[2], v[3]), pack2_bf16(v[4], v[5]), pack2_bf16(v[6], v[7])));
+#pragma unroll
+        for (int t = 0; t < 2; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_frag(ph[t][step]), b, acc[t], 0, 0, 0);
+      }
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) red[ch * 512 + (16 * t + 4 * g + e) * 16 + col] = acc[t][e];
+      __syncthreads();
+      if (tid < 256 && k0 + (tid >> 3) < K) {
+        float sum = 0.f;
+#pragma unroll
+        for (int w8 = 0; w8 < 8; ++w8) sum += red[w8 * 512 + (tid >> 3) * 16 + (tid & 7)] + red[w8 * 512 + (tid >> 3) * 16 + 8 + (tid & 7)];
+        part[((size_t)(item0 / R) * K + k0 + (tid >> 3)) * d + c0 + (tid & 7)] = sum;
+      }
+      if (k0 + 32 < K) {
+        rows_of_phi(k0 + 32);
+        __syncthreads();
+      }
+    }
+    return;
+  }
   const int lags = min(cap, (min(L, T) + 1) >> 1);
   float* const out = part + (size_t)(item0 / R) * lags * d + c0;
   for (int v = tid; v < lags * 2; v += 512) {
@@ -458,6 +515,16 @@ __global__ void __launch_bounds__(256) conv_grad_finish_kernel(const float* __re
                                                   pack2_bf16(2.f * a[4], 2.f * a[5]), pack2_bf16(2.f * a[6], 2.f * a[7]));
 }
 
+// gm[i] = 2 * (the chunks' products in their order)
+__global__ void __launch_bounds__(256) conv_grad_join_kernel(const float* __restrict__ part, bf16_t* __restrict__ gm, int chunks, int n) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) return;
+  float a = 0.f;
+#pragma unroll 8
+  for (int k = 0; k < chunks; ++k) a += part[(size_t)k * n + i];
+  gm[i] = f32_to_bf16(2.f * a);
+}
+
 // taps[c][p][cap - j] = f[2j+p][c] for 0 <= j, zero where the filter has no such lag; 8 channels x 8 places per thread
 __global__ void __launch_bounds__(256)
 conv_taps_kernel(const bf16_t* __restrict__ f, bf16_t* __restrict__ taps, int L, int d, int cap) {
@@ -477,6 +544,70 @@ conv_taps_kernel(const bf16_t* __restrict__ f, bf16_t* __restrict__ taps, int L,
 #pragma unroll
   for (int c = 0; c < 8; ++c)
     *(uint4*)(taps + ((size_t)(c0 + c) * 2 + p) * S + i0) = make_uint4(o[c][0], o[c][1], o[c][2], o[c][3]);
+}
+
+// The same taps of f = T(phi @ m), and f's first Lf rows.  A workgroup forms 64 places of 128 channels, a whole line of a channel's
+// taps, 8 places of 4 channels to a thread, from LDS: both operands come in one trip (2048 x 24 @ 24 x 768 8.8 us; with a trip
+// for phi and three for m 11; the product and the taps in launches of their own 7.8 + 5.3).
+__global__ void __launch_bounds__(256)
+conv_taps_project_kernel(const bf16_t* __restrict__ phi, const bf16_t* __restrict__ m, bf16_t* __restrict__ f, bf16_t* __restrict__ taps, int L,
+                         int Lf, int K, int d, int cap) {
+  extern __shared__ __attribute__((aligned(16))) float rows[];      // [filter][place], then m's 128 channels, [filter][channel]
+  const int tid = threadIdx.x, S = cap + 16, p = blockIdx.y & 1, i0 = (int)(blockIdx.y >> 1) * 64, j0 = cap - i0;
+  bf16_t* const cols = (bf16_t*)(rows + 64 * K);
+  const int place = tid & 63, s0 = 2 * (j0 - place) + p, piece = (tid & 15) * 8, cp = blockIdx.x * 128 + piece;
+  const bool lag = j0 >= place && s0 < L;
+  const bf16_t* const src = phi + (size_t)(lag ? s0 : 0) * K;
+  for (int k0 = 0; k0 < K; k0 += 32) {
+    bf16_t v[8];
+    uint4 w[2];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = lag ? src[min(k0 + 4 * i + (tid >> 6), K - 1)] : 0;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int k = k0 + 16 * i + (tid >> 4);
+      w[i] = make_uint4(0, 0, 0, 0);
+      if (k < K && cp < d) w[i] = *(const uint4*)(m + (size_t)k * d + cp);
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int k = k0 + 4 * i + (tid >> 6);
+      if (k < K) rows[k * 64 + place] = bf16_to_f32(v[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int k = k0 + 16 * i + (tid >> 4);
+      if (k < K) *(uint4*)(cols + k * 128 + piece) = w[i];
+    }
+  }
+  __syncthreads();
+  const int e0 = (tid & 7) * 8, c0 = blockIdx.x * 128 + (tid >> 3) * 4;
+  if (c0 >= d || i0 + e0 >= S) return;
+  float acc[4][8];
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc[c][e] = 0.f;
+#pragma unroll 8
+  for (int k = 0; k < K; ++k) {
+    const uint2 w = *(const uint2*)(cols + k * 128 + (tid >> 3) * 4);
+    const float wv[4] = {__uint_as_float(w.x << 16), __uint_as_float(w.x & 0xffff0000u), __uint_as_float(w.y << 16), __uint_as_float(w.y & 0xffff0000u)};
+    const float4 r0 = *(const float4*)(rows + k * 64 + e0), r1 = *(const float4*)(rows + k * 64 + e0 + 4);
+    const float r[8] = {r0.x, r0.y, r0.z, r0.w, r1.x, r1.y, r1.z, r1.w};
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) acc[c][e] = fmaf(r[e], wv[c], acc[c][e]);
+  }
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+    *(uint4*)(taps + ((size_t)(c0 + c) * 2 + p) * S + i0 + e0) = make_uint4(pack2_bf16(acc[c][0], acc[c][1]), pack2_bf16(acc[c][2], acc[c][3]),
+                                                                            pack2_bf16(acc[c][4], acc[c][5]), pack2_bf16(acc[c][6], acc[c][7]));
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const int j = j0 - e0 - e, s = 2 * j + p;
+    if (j >= 0 && s < Lf) *(uint2*)(f + (size_t)s * d + c0) = make_uint2(pack2_bf16(acc[0][e], acc[1][e]), pack2_bf16(acc[2][e], acc[3][e]));
+  }
 }
 
 // log2 of the blocks of a tile and the tiles for T positions
@@ -530,6 +661,18 @@ extern "C" int fstu_stu_conv_taps(const void* filt, void* taps, int L, int d, in
   return FSTU_OK;
 }
 
+extern "C" int fstu_stu_conv_taps_project(const void* phi, const void* m, void* f, void* taps, int L, int K, int d, int S, void* stream) {
+  FSTU_REQUIRE(phi && m && f && taps, FSTU_ENULL, "fstu_stu_conv_taps_project: null pointer");
+  FSTU_REQUIRE(L >= 1 && K >= 1 && K <= 128 && d >= 8 && d % 8 == 0 && d <= 1 << 20 && S >= 80 && S <= 2064 && S % 64 == 16, FSTU_ESHAPE,
+               "fstu_stu_conv_taps_project: L=%d K=%d d=%d S=%d (K up to 128, d a multiple of 8, S of fstu_stu_conv_taps_len)", L, K, d, S);
+  FSTU_REQUIRE(fstu_aligned(phi, 2) && fstu_aligned(m, 16) && fstu_aligned(f, 16) && fstu_aligned(taps, 16), FSTU_EALIGN,
+               "fstu_stu_conv_taps_project: m, f and taps must be 16-byte aligned");
+  hipLaunchKernelGGL(conv_taps_project_kernel, dim3((d + 127) / 128, 2 * ((S + 63) / 64)), dim3(256), 512 * (size_t)K, (hipStream_t)stream, (const bf16_t*)phi,
+                     (const bf16_t*)m, (bf16_t*)f, (bf16_t*)taps, L, std::min(L, 2 * (S - 16)), K, d, S - 16);
+  FSTU_CHECK_LAUNCH("fstu_stu_conv_taps_project");
+  return FSTU_OK;
+}
+
 extern "C" int fstu_stu_conv_mfma(const void* x, const void* taps, void* y, int B, int T, int d, int single_branch, void* stream) {
   FSTU_REQUIRE(x && taps && y, FSTU_ENULL, "fstu_stu_conv_mfma: null pointer");
   FSTU_REQUIRE(B >= 1 && B <= 65535 && T >= 1 && T <= 4096 && d >= 8 && d % 8 == 0 && d <= 1 << 20, FSTU_ESHAPE,
@@ -577,33 +720,63 @@ extern "C" int64_t fstu_stu_conv_mfma_grad_ws(int B, int T, int d, int L) {
   return (int64_t)((2 * B + R - 1) / R) * lags * d;
 }
 
-extern "C" int fstu_stu_conv_mfma_grad(const void* gy, const void* x, const void* filt, void* gx, void* gf, float* part, int B, int T, int d,
-                                       int L, void* stream) {
-  FSTU_REQUIRE(gy && x && filt && (gx || gf) && (!gf || part), FSTU_ENULL, "fstu_stu_conv_mfma_grad: null pointer");
+namespace {
+
+int cg_launch(const char* name, const void* gy, const void* x, const void* filt, void* gx, float* part, const void* phi_e, int K, int P, int B, int T,
+              int d, int L, int R, hipStream_t s) {
   FSTU_REQUIRE(B >= 1 && B <= 65535 && T >= 1 && T <= 2048 && d >= 8 && d % 8 == 0 && d <= 1 << 20 && L >= 1 && (int64_t)L * d < 1ll << 31,
-               FSTU_ESHAPE, "fstu_stu_conv_mfma_grad: B=%d T=%d d=%d L=%d (T up to 2048, d a multiple of 8)", B, T, d, L);
-  FSTU_REQUIRE(fstu_aligned(gy, 16) && fstu_aligned(x, 16) && fstu_aligned(filt, 16) && fstu_aligned(gx, 16) && fstu_aligned(gf, 16) &&
-                   fstu_aligned(part, 16), FSTU_EALIGN, "fstu_stu_conv_mfma_grad: pointers must be 16-byte aligned");
-  const int R = cg_items(B, T, d), chunks = (2 * B + R - 1) / R, lags = ((L < T ? L : T) + 1) / 2;
-  const long long units = (long long)((d + 63) / 64) * chunks;
-  FSTU_REQUIRE(units < 1 << 24, FSTU_ESHAPE, "fstu_stu_conv_mfma_grad: B=%d d=%d", B, d);
+               FSTU_ESHAPE, "%s: B=%d T=%d d=%d L=%d (T up to 2048, d a multiple of 8)", name, B, T, d, L);
+  FSTU_REQUIRE(fstu_aligned(gy, 16) && fstu_aligned(x, 16) && fstu_aligned(filt, 16) && fstu_aligned(gx, 16) && fstu_aligned(part, 16) &&
+                   fstu_aligned(phi_e, 16), FSTU_EALIGN, "%s: pointers must be 16-byte aligned", name);
+  const long long units = (long long)((d + 63) / 64) * ((2 * B + R - 1) / R);
+  FSTU_REQUIRE(units < 1 << 24, FSTU_ESHAPE, "%s: B=%d d=%d", name, B, d);
   const dim3 grid((unsigned)((units + 7) / 8 * 64));
 #define CG_GO(NT)                                                                                                                   \
   do {                                                                                                                              \
     constexpr int lds__ = 16 * cm_region(8 * NT) + 8 * cg_rows(8 * NT) + 8 * 2048;                                                 \
     static fstu_lds_limit most;                                                                                                     \
-    const int rc__ = fstu_need_lds((const void*)conv_grad_mfma_kernel<NT>, most, lds__, "fstu_stu_conv_mfma_grad");                 \
+    const int rc__ = fstu_need_lds((const void*)conv_grad_mfma_kernel<NT>, most, lds__, name);                                      \
     if (rc__) return rc__;                                                                                                          \
-    hipLaunchKernelGGL((conv_grad_mfma_kernel<NT>), grid, dim3(512), lds__, (hipStream_t)stream, (const bf16_t*)gy, (const bf16_t*)x, \
-                       (const bf16_t*)filt, (bf16_t*)gx, gf ? part : nullptr, B, T, L, d, R);                                       \
+    hipLaunchKernelGGL((conv_grad_mfma_kernel<NT>), grid, dim3(512), lds__, s, (const bf16_t*)gy, (const bf16_t*)x, (const bf16_t*)filt, \
+                       (bf16_t*)gx, part, (const bf16_t*)phi_e, K, P, B, T, L, d, R);                                               \
   } while (0)
   if (T <= 1024) CG_GO(1);
   else CG_GO(2);
 #undef CG_GO
-  FSTU_CHECK_LAUNCH("fstu_stu_conv_mfma_grad");
-  if (!gf) return FSTU_OK;
+  FSTU_CHECK_LAUNCH(name);
+  return FSTU_OK;
+}
+
+}  // namespace
+
+extern "C" int fstu_stu_conv_mfma_grad(const void* gy, const void* x, const void* filt, void* gx, void* gf, float* part, int B, int T, int d,
+                                       int L, void* stream) {
+  FSTU_REQUIRE(gy && x && filt && (gx || gf) && (!gf || part), FSTU_ENULL, "fstu_stu_conv_mfma_grad: null pointer");
+  FSTU_REQUIRE(fstu_aligned(gf, 16), FSTU_EALIGN, "fstu_stu_conv_mfma_grad: pointers must be 16-byte aligned");
+  const int R = cg_items(B, T, d), chunks = (2 * B + R - 1) / R, lags = ((L < T ? L : T) + 1) / 2;
+  const int rc = cg_launch("fstu_stu_conv_mfma_grad", gy, x, filt, gx, gf ? part : nullptr, nullptr, 0, 0, B, T, d, L, R, (hipStream_t)stream);
+  if (rc || !gf) return rc;
   hipLaunchKernelGGL(conv_grad_finish_kernel, dim3((unsigned)(((long long)L * (d / 8) + 255) / 256)), dim3(256), 0, (hipStream_t)stream, part,
                      (bf16_t*)gf, chunks, lags, L, d);
   FSTU_CHECK_LAUNCH("fstu_stu_conv_mfma_grad");
+  return FSTU_OK;
+}
+
+extern "C" int64_t fstu_stu_conv_mfma_grad_project_ws(int B, int T, int d, int K) {
+  if (B < 1 || T < 1 || T > 2048 || d < 8 || K < 1) return 0;
+  const int R = cg_items(B, T, d);
+  return (int64_t)((2 * B + R - 1) / R) * K * d;
+}
+
+extern "C" int fstu_stu_conv_mfma_grad_project(const void* gy, const void* x, const void* filt, const void* phi_e, int P, void* gx, void* gm,
+                                               float* part, int B, int T, int d, int L, int K, void* stream) {
+  FSTU_REQUIRE(gy && x && filt && phi_e && gm && part, FSTU_ENULL, "fstu_stu_conv_mfma_grad_project: null pointer");
+  FSTU_REQUIRE(K >= 1 && K <= 128 && P >= 8 && P % 8 == 0 && T <= L && 2 * (int64_t)P >= L, FSTU_ESHAPE,
+               "fstu_stu_conv_mfma_grad_project: K=%d P=%d T=%d L=%d (K up to 128, P a multiple of 8 of at least L / 2, T up to L)", K, P, T, L);
+  const int R = cg_items(B, T, d), n = K * d;
+  const int rc = cg_launch("fstu_stu_conv_mfma_grad_project", gy, x, filt, gx, part, phi_e, K, P, B, T, d, L, R, (hipStream_t)stream);
+  if (rc) return rc;
+  hipLaunchKernelGGL(conv_grad_join_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream, part, (bf16_t*)gm, (2 * B + R - 1) / R, n);
+  FSTU_CHECK_LAUNCH("fstu_stu_conv_mfma_grad_project");
   return FSTU_OK;
 }

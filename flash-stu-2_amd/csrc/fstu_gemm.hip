@@ -741,8 +741,9 @@ gemm_ta_bf16_kernel(const bf16_t* __restrict__ A, long long lda, long long sa, c
   if ((int)(blockIdx.x >> 3) >= share || o >= mt * nt * nbatch * ksplit) return;
   const int bs = o / (mt * nt), slice = bs / nbatch, batch = bs - slice * nbatch;    // MODE 3: slices of K outermost
   o -= bs * (mt * nt);
-  const int kbeg = MODE == 3 ? (int)((long long)(K / G::BK) * slice / ksplit) * G::BK : 0;      // this workgroup's share of K
-  const int KS = MODE == 3 ? (int)((long long)(K / G::BK) * (slice + 1) / ksplit) * G::BK - kbeg : K;
+  const int nk = (K + G::BK - 1) / G::BK;              // TW: the last k tile may be ragged, rows behind the end are zeros
+  const int kbeg = MODE == 3 ? (int)((long long)nk * slice / ksplit) * G::BK : 0;              // this workgroup's share of K
+  const int KS = MODE == 3 ? min((int)((long long)nk * (slice + 1) / ksplit) * G::BK, K) - kbeg : K;
   const int per_panel = mt * GM_PANEL;
   const int panel = o / per_panel, in_panel = o - panel * per_panel;
   const int pw = min(GM_PANEL, nt - panel * GM_PANEL);
@@ -812,7 +813,7 @@ gemm_ta_bf16_kernel(const bf16_t* __restrict__ A, long long lda, long long sa, c
     for (int j = 0; j < TJ; ++j)
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
-  const int nkt = KS / G::BK;
+  const int nkt = TW ? (KS + G::BK - 1) / G::BK : KS / G::BK;
   constexpr int LPT = WL + AL;
 #pragma unroll
   for (int t = 0; t < NS - 1; ++t)
@@ -1223,9 +1224,9 @@ extern "C" int fstu_gemm_bf16_ta_ws(const void* A, int64_t lda, int64_t batch_st
 // (28) / - / 24.3, 768 x 768 x 1024 12.3 (1) / - / 13.4 / 18.2, 1024 x 1024 x 16384 43.9 (8) / 45.1 / 53.1 (10) / 63.8, 2048 x 2048 x 16384
 // 135.6 (2) / 166.6 / 143.8 / 138.1.
 extern "C" int fstu_gemm_bf16_tt_slices(int M, int N, int K) {
-  if (M % 128 != 0 || N % 128 != 0 || K % 64 != 0 || M < 1 || N < 1 || K < 64) return 1;
+  if (M % 128 != 0 || N % 128 != 0 || M < 1 || N < 1 || K < 1) return 1;
   const long long cus = gemm_cus(), tiles = (long long)(M / 128) * (N / 128);
-  const int nkt = K / 64;
+  const int nkt = (K + 63) / 64;
   double least = 1e30;
   int best = 1;
   for (int s = 1; s <= 32 && s <= nkt && (s == 1 || tiles * s <= 2 * cus); ++s) {
@@ -1235,13 +1236,13 @@ extern "C" int fstu_gemm_bf16_tt_slices(int M, int N, int K) {
   return best;
 }
 
-// C[m, n] = T(sum_k A[k, m] W[k, n]) for A (K, M) and W (K, N), rows of lda and ldw elements, M and N multiples of 128, K of 64, in
+// C[m, n] = T(sum_k A[k, m] W[k, n]) for A (K, M) and W (K, N), rows of lda and ldw elements, M and N multiples of 128, in
 // ksplit slices of K (partial: ksplit * M * N fp32), which a second launch adds
 extern "C" int fstu_gemm_bf16_tt(const void* A, int64_t lda, const void* W, int64_t ldw, void* C, int64_t ldc, int M, int N, int K,
                                  float* partial, int ksplit, void* stream) {
   FSTU_REQUIRE(A && W && C, FSTU_ENULL, "fstu_gemm_bf16_tt: null pointer");
-  FSTU_REQUIRE(M >= 128 && M % 128 == 0 && N >= 128 && N % 128 == 0 && K >= 64 && K % 64 == 0, FSTU_ESHAPE,
-               "fstu_gemm_bf16_tt: need M %% 128 == 0, N %% 128 == 0, K %% 64 == 0 (M=%d N=%d K=%d)", M, N, K);
+  FSTU_REQUIRE(M >= 128 && M % 128 == 0 && N >= 128 && N % 128 == 0 && K >= 1, FSTU_ESHAPE,
+               "fstu_gemm_bf16_tt: need M %% 128 == 0, N %% 128 == 0 (M=%d N=%d K=%d)", M, N, K);
   FSTU_REQUIRE(lda >= M && lda % 8 == 0 && ldw >= N && ldw % 8 == 0 && ldc >= N && ldc % 4 == 0, FSTU_ESHAPE,
                "fstu_gemm_bf16_tt: row strides (lda=%lld ldw=%lld ldc=%lld)", (long long)lda, (long long)ldw, (long long)ldc);
   // 32-bit byte offsets inside both operands (buffer addressing)
@@ -1252,7 +1253,7 @@ extern "C" int fstu_gemm_bf16_tt(const void* A, int64_t lda, const void* W, int6
   hipStream_t s = (hipStream_t)stream;
   int rc;
   if (ksplit > 1) {
-    FSTU_REQUIRE(partial && fstu_aligned(partial, 16) && ksplit <= 64 && ksplit <= K / 64, FSTU_ESHAPE, "fstu_gemm_bf16_tt: %d slices of K=%d", ksplit, K);
+    FSTU_REQUIRE(partial && fstu_aligned(partial, 16) && ksplit <= 64 && ksplit <= (K + 63) / 64, FSTU_ESHAPE, "fstu_gemm_bf16_tt: %d slices of K=%d", ksplit, K);
     rc = gemm_ta_launch_tile<TileSmall, 3, true>(A, lda, 0, W, partial, 0, 0, C, 0, 0, M, N, K, 1, s, ksplit, ldw);
     if (rc) return rc;
     FSTU_CHECK_LAUNCH("fstu_gemm_bf16_tt");

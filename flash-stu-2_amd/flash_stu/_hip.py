@@ -59,6 +59,9 @@ SIGNATURES = {
     "fstu_stu_conv_taps": [_vp, _vp, _i, _i, _i, _vp],
     "fstu_stu_conv_mfma_grad_takes": [_i, _i, _i, _i],
     "fstu_stu_conv_mfma_grad_ws": [_i, _i, _i, _i],
+    "fstu_stu_conv_taps_project": [_vp, _vp, _vp, _vp, _i, _i, _i, _i, _vp],
+    "fstu_stu_conv_mfma_grad_project_ws": [_i, _i, _i, _i],
+    "fstu_stu_conv_mfma_grad_project": [_vp, _vp, _vp, _vp, _i, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp],
     "fstu_stu_conv_mfma_grad": [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _vp],
     "fstu_stu_conv_mfma": [_vp, _vp, _vp, _i, _i, _i, _i, _vp],
     "fstu_stu_conv_fft": [_vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _vp],
@@ -147,6 +150,7 @@ def load(path: Optional[str] = None):
     lib.fstu_lds_sequence_ws_floats.restype = ctypes.c_size_t
     lib.fstu_stu_conv_fft_grad_ws.restype = ctypes.c_int64
     lib.fstu_stu_conv_mfma_grad_ws.restype = ctypes.c_int64
+    lib.fstu_stu_conv_mfma_grad_project_ws.restype = ctypes.c_int64
     if path is None:
         _lib = lib
     return lib
@@ -444,7 +448,7 @@ def _gemm_tt_slices(M: int, N: int, K: int) -> int:
 
 def gemm_tt(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
     """a^T @ b for a (K, M) and b (K, N) bf16 with contiguous rows, rounded once: a weight's gradient, summed over all positions.
-    M and N multiples of 128, K of 64."""
+    M and N multiples of 128."""
     _dev(a, b)
     (K, M), N = a.shape, b.shape[1]
     if b.shape[0] != K or a.dtype != torch.bfloat16 or b.dtype != torch.bfloat16:
@@ -841,6 +845,35 @@ def stu_conv_mfma_grad(gy: torch.Tensor, x: torch.Tensor, filt: torch.Tensor, wa
         _check(load().fstu_stu_conv_mfma_grad(_p(gy), _p(x), _p(filt), _p(gx), _p(gf), _p(part), B, T, d, L, _stream()),
                "fstu_stu_conv_mfma_grad")
     return gx, gf
+
+
+def stu_conv_taps_project(phi: torch.Tensor, m: torch.Tensor, T: int):
+    """The taps of T(phi @ m) for T positions (stu_conv_taps), phi (L,K) and m (K,d) bf16, and those of its rows that stand for the
+    filter in the gradients."""
+    _dev(phi, m)
+    (L, K), d, S = phi.shape, m.shape[1], stu_conv_taps_len(T)
+    if m.shape[0] != K or not phi.dtype == m.dtype == torch.bfloat16:
+        raise FlashSTUHipError("stu_conv_taps_project takes bfloat16 operands (L,K) and (K,d)")
+    filt = torch.empty(min(L, 2 * (S - 16)), d, dtype=m.dtype, device=m.device)
+    taps = torch.empty(d, 2, S, dtype=m.dtype, device=m.device)
+    _check(load().fstu_stu_conv_taps_project(_p(phi), _p(m), _p(filt), _p(taps), L, K, d, S, _stream()), "fstu_stu_conv_taps_project")
+    return filt, taps
+
+
+def stu_conv_mfma_grad_project(gy: torch.Tensor, x: torch.Tensor, filt: torch.Tensor, phi_e: torch.Tensor, K: int, want_x: bool = True):
+    """The gradients of stu_conv_mfma_grad where the filter is phi @ m (stu_conv_taps_project): those of x and of m (K,d).  phi_e: the
+    even rows of phi transposed, filled up with zeros to whole tiles of 16 filters and of 8 lags."""
+    _dev(gy, x, filt, phi_e)
+    B, T, d = x.shape
+    L, (rows, P) = filt.shape[0], phi_e.shape
+    if gy.shape != x.shape or filt.shape[1] != d or rows < K or rows % 16 or not gy.dtype == x.dtype == filt.dtype == phi_e.dtype == torch.bfloat16:
+        raise FlashSTUHipError("stu_conv_mfma_grad_project takes bfloat16 operands, gy of x's shape, one filter per channel and phi_e of whole tiles")
+    gx = torch.empty_like(x) if want_x else None
+    gm = torch.empty(K, d, dtype=x.dtype, device=x.device)
+    part = torch.empty(int(load().fstu_stu_conv_mfma_grad_project_ws(B, T, d, K)), dtype=torch.float32, device=x.device)
+    _check(load().fstu_stu_conv_mfma_grad_project(_p(gy), _p(x), _p(filt), _p(phi_e), P, _p(gx), _p(gm), _p(part), B, T, d, L, K, _stream()),
+           "fstu_stu_conv_mfma_grad_project")
+    return gx, gm
 
 
 def stu_conv_fft_grad(g1: torch.Tensor, g2: Optional[torch.Tensor], x: torch.Tensor, spec: torch.Tensor, taps: int,

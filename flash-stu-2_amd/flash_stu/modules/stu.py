@@ -117,6 +117,14 @@ class STU(nn.Module):
             return torch.matmul(self.phi, self.M_filters).contiguous()
         return self._cached("filt", (self.phi, self.M_filters), build)
 
+    def phi_even_t(self) -> torch.Tensor:
+        """The even rows of phi transposed, filled up with zeros to whole tiles of 16 filters and of 8 lags, as the gradient of
+        M_filters reads them."""
+        def build():
+            even = self.phi[0::2].detach()
+            return torch.nn.functional.pad(even.t(), (0, -even.shape[0] % 8, 0, -self.K % 16)).contiguous()
+        return self._cached("phie", (self.phi,), build)
+
     def filter_spectrum(self, n: int) -> torch.Tensor:
         """Spectra of the convolution filters for transform length n, (d,n,2) fp32 in approx mode, (K,n,2) in
         exact mode (the reference keeps its own phi_fft the same way, stu.py:43-53).  One length is kept."""
@@ -365,13 +373,16 @@ class STU(nn.Module):
 
     def forward_differentiable(self, x: torch.Tensor) -> torch.Tensor:
         """Training-side forward of the approx-mode STU (stu.py:81-98,120) under autograd: gradients reach x, M_inputs and
-        M_filters.  The convolution and its gradients are the HIP kernels, the input projection too where they take its
-        shape (flash_stu.utils.stu_utils), the small filter projection is a library GEMM.  No decode state."""
-        from ..utils.stu_utils import ApproxConvolveSum, ProjectInputs, convolve, nearest_power_of_two
+        M_filters.  The convolution and its gradients are the HIP kernels, both projections too where they take their
+        shapes (flash_stu.utils.stu_utils); elsewhere the filter's is a library GEMM.  No decode state."""
+        from ..utils.stu_utils import ApproxConvolveSum, ApproxUnit, ProjectInputs, convolve, nearest_power_of_two
         if not self.use_approx:
             raise NotImplementedError("forward_differentiable covers use_approx=True")
         if self.tile_size < self.d_in:
             raise NotImplementedError("forward_differentiable does not cover d_in_tile / d_out_tile")
+        m_inputs, m_filters = self.M_inputs, self.M_filters
+        if not self.use_hankel_L and ApproxUnit.takes(x, self.phi, m_inputs, m_filters):
+            return ApproxUnit.apply(x, self.phi, self.phi_even_t(), m_inputs, m_filters)
         x_proj = ProjectInputs.apply(x, self.M_inputs) if ProjectInputs.takes(x, self.M_inputs) else x @ self.M_inputs
         phi_proj = self.phi @ self.M_filters
         n = nearest_power_of_two(2 * self.phi.shape[0] - 1, round_up=True)

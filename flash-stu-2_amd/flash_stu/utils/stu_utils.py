@@ -228,6 +228,56 @@ class ProjectInputs(torch.autograd.Function):
         return gx, gm
 
 
+class ApproxUnit(torch.autograd.Function):
+    """The whole approx-mode STU, conv(x @ m_inputs, phi @ m_filters) with its branches added, in bf16 where its convolution and the
+    gradients are products: five launches forward and seven backward, none of them a library's, and one node for the host to
+    go through (8 x 2048 x 768: as four nodes, two of them library products, the host took longer than the GPU).  phi_e holds the even
+    rows of phi as the gradient of m_filters reads them.  Where the gradients are to be differentiated themselves
+    (create_graph=True) they are those of the composed operators."""
+
+    @staticmethod
+    def takes(x, phi, m_inputs, m_filters) -> bool:
+        from .. import _hip
+        if x.dim() != 3 or not x.is_cuda or torch.is_autocast_enabled() or phi.requires_grad:
+            return False
+        if any(t.dtype != torch.bfloat16 or t.device != x.device or not t.is_contiguous() or t.data_ptr() % 16 for t in (phi, m_inputs, m_filters)):
+            return False
+        (B, T, d_in), (L, K), d = x.shape, phi.shape, m_inputs.shape[1]
+        return (x.dtype == torch.bfloat16 and m_inputs.shape[0] == d_in and m_filters.shape == (K, d) and T <= L and K <= 128
+                and B * T >= 128 and d_in % 128 == 0 and d % 128 == 0 and B * T * d_in < 1 << 30 and B * T * d < 1 << 30
+                and _hip.stu_conv_mfma_grad_takes(B, T, d, L, x.dtype))
+
+    @staticmethod
+    def forward(ctx, x, phi, phi_e, m_inputs, m_filters):
+        from .. import _hip
+        x2 = _aligned(x.reshape(-1, x.shape[2]))
+        u = _hip.gemm(x2, _hip.transpose(m_inputs[None])[0]).view(*x.shape[:2], m_inputs.shape[1])
+        v, taps = _hip.stu_conv_taps_project(phi, m_filters, x.shape[1])
+        ctx.save_for_backward(x, phi, phi_e, m_inputs, m_filters, u, v)
+        return _hip.stu_conv_mfma(u, taps)
+
+    @staticmethod
+    def backward(ctx, gy):
+        from .. import _hip
+        x, phi, phi_e, m_inputs, m_filters, u, v = ctx.saved_tensors
+        want_x, _, _, want_i, want_f = ctx.needs_input_grad
+        if torch.is_grad_enabled():
+            wanted = [t for t, w in ((x, want_x), (m_inputs, want_i), (m_filters, want_f)) if w]
+            grads = iter(torch.autograd.grad(ApproxConvolveSum.apply(x @ m_inputs, phi @ m_filters), wanted, gy, create_graph=True))
+            return next(grads) if want_x else None, None, None, next(grads) if want_i else None, next(grads) if want_f else None
+        gy, gf = _aligned(gy), None
+        if want_f:
+            gu, gf = _hip.stu_conv_mfma_grad_project(gy, u, v, phi_e, phi.shape[1], want_x or want_i)
+        else:
+            gu, _ = _hip.stu_conv_mfma_grad(gy, u, v, True, False)
+        if not (want_x or want_i):
+            return None, None, None, None, gf
+        gu = gu.view(-1, gu.shape[2])
+        gx = _hip.gemm(gu, m_inputs).view_as(x) if want_x else None
+        gi = _hip.gemm_tt(_aligned(x.reshape(-1, x.shape[2])), gu) if want_i else None
+        return gx, None, None, gi, gf
+
+
 def _aligned(t: torch.Tensor) -> torch.Tensor:
     """t with dense rows at a 16-byte address, as the matrix-core kernels read it."""
     t = t.contiguous()

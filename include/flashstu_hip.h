@@ -292,6 +292,14 @@ int fstu_stu_conv_mfma_grad_takes(int B, int T, int d, int L);   /* where it is 
 int64_t fstu_stu_conv_mfma_grad_ws(int B, int T, int d, int L);
 int fstu_stu_conv_mfma_grad(const void* gy, const void* x, const void* filt, void* gx, void* gf, float* part, int B, int T, int d,
                             int L, void* stream);
+/* A training step whose filter is phi (L,K) @ m (K,d): the taps of T(phi @ m) in one launch, with its first min(L, 2 (S - 16)) rows
+ * in f, which stand for filt (with that L) in the gradients of up to 2 (S - 16) positions; and gx and gm (K,d), the gradient of m, from
+ * phi_e, the even rows of phi transposed and padded with zeros to (whole 16 filters, P), 2 P >= L, T <= L.  K up to 128; all but phi
+ * 16-byte aligned; part: fp32 scratch of fstu_stu_conv_mfma_grad_project_ws elements. */
+int fstu_stu_conv_taps_project(const void* phi, const void* m, void* f, void* taps, int L, int K, int d, int S, void* stream);
+int64_t fstu_stu_conv_mfma_grad_project_ws(int B, int T, int d, int K);
+int fstu_stu_conv_mfma_grad_project(const void* gy, const void* x, const void* filt, const void* phi_e, int P, void* gx, void* gm, float* part,
+                                    int B, int T, int d, int L, int K, void* stream);
 /* Gradients of the convolution: g1, g2 (B,T,d) those of the plus and minus branch (branches = 2), g1 alone that of the plus
  * branch (branches = 1) or that of y = plus + minus (branches = 0), x (B,T,d) the forward input, spec (d, n) the filters'
  * spectra.  Writes gx (B,T,d) and gf (L,d), each in dtype and skipped where null; gf needs x and part, fp32 scratch of
@@ -460,7 +468,7 @@ int fstu_gemm_bf16_ta_ws(const void* A, int64_t lda, int64_t batch_stride_a, con
                          int64_t batch_stride_r, void* C, int64_t ldc, int64_t batch_stride_c, int M, int N, int K,
                          int nbatch, int mode, float* partial, int ksplit, void* stream);
 /* A weight's gradient: C (M,N) = T(A^T W) for A (K,M) and W (K,N), both with the reduction index slowest, rows of lda and ldw
- * elements.  M, N % 128 == 0, K % 64 == 0, lda, ldw % 8 == 0, K*lda*2 and K*ldw*2 below 4 GB; A, W 16-byte aligned, C 8.  ksplit
+ * elements.  M, N % 128 == 0, any K, lda, ldw % 8 == 0, K*lda*2 and K*ldw*2 below 4 GB; A, W 16-byte aligned, C 8.  ksplit
  * slices of K (1: none; fstu_gemm_bf16_tt_slices says how many pay), not all of one length, joined in order by a second launch;
  * partial holds ksplit * M * N floats, 16-byte aligned. */
 int fstu_gemm_bf16_tt_slices(int M, int N, int K);

@@ -240,6 +240,47 @@ def test_stu_forward_differentiable_second_order(hankel, T):
         assert float((got.cpu() - want).abs().max()) <= 1e-3 * float(want.abs().max())
 
 
+@pytest.mark.parametrize("B,T,d", [(4, 32, 128), (3, 201, 256), (1, 1025, 128)])
+def test_training_step_as_one_node(B, T, d, monkeypatch):
+    """forward_differentiable in bf16 as one autograd node against its composed operators: outputs and gradients, x expanded, off its
+    alignment and strided, parameters frozen, and the gradients of the gradients.  Three roundings to bf16 (2^-8 each) lie
+    between the two in any of them."""
+    from flash_stu import STU, FlashSTUConfig
+    from flash_stu.utils.stu_utils import ApproxUnit
+    L, K = 1040, 24
+    g = torch.Generator().manual_seed(T)
+    cfg = FlashSTUConfig(n_embd=d, n_heads=2, n_layers=2, seq_len=L, num_eigh=K, vocab_size=11, torch_dtype=torch.bfloat16)
+    stu = STU(cfg, torch.randn(L, K, generator=g).div(L ** 0.5).bfloat16().cuda(), 4096).cuda()
+    with torch.no_grad():
+        for p in (stu.M_inputs, stu.M_filters):
+            p.copy_(torch.randn(p.shape, generator=g) / p.shape[0] ** 0.5)
+    x, gy = (torch.randn(B, T, d, generator=g).bfloat16().cuda() for _ in range(2))
+    shifted = torch.empty(B * T * d + 1, dtype=torch.bfloat16, device="cuda")[1:].view(B, T, d).copy_(x)
+    strided = torch.empty(T, B, d, dtype=torch.bfloat16, device="cuda").transpose(0, 1).copy_(x)
+    close = lambda a, b: float((a.float() - b.float()).norm()) <= 3 * 2.0 ** -8 * float(b.float().norm())
+    made = []
+    takes = ApproxUnit.takes
+
+    def pass_of(xi, wanted, second=False):
+        xi = xi.detach().requires_grad_(0 in wanted)
+        for i, p in enumerate((stu.M_inputs, stu.M_filters), 1):
+            p.requires_grad_(i in wanted)
+        leaves = [t for i, t in enumerate((xi, stu.M_inputs, stu.M_filters)) if i in wanted]
+        y = stu.forward_differentiable(xi)
+        grads = torch.autograd.grad(y, leaves, gy, create_graph=second)
+        if second:
+            grads = torch.autograd.grad(sum(t.float().square().sum() / t.detach().float().square().sum() for t in grads), leaves)
+        return y.detach(), *grads
+    for xi, wanted, second in ((x, (0, 1, 2), False), (shifted, (0, 1, 2), False), (strided, (1, 2), False), (x[:1].expand(B, T, d), (0, 2), False),
+                               (x, (2,), False), (x, (1,), False), (x, (0,), False), (x, (0, 1, 2), True)):
+        both = []
+        for node in (True, False):
+            monkeypatch.setattr(ApproxUnit, "takes", staticmethod(lambda *a: made.append(takes(*a)) or (node and made[-1])))
+            both.append(pass_of(xi, wanted, second))
+        assert len(both[0]) == 1 + len(wanted) and all(close(a, b) and a.shape == b.shape for a, b in zip(*both))
+    assert all(made)
+
+
 @pytest.mark.parametrize("B,T,d", [(1, 128, 128), (3, 320, 256), (2, 97, 128)])
 def test_input_projection_gradients(B, T, d):
     """x @ M_inputs and its gradients on the matrix-core kernels (and, for rows they do not take, the library's product)

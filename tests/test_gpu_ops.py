@@ -418,14 +418,14 @@ def test_gemm_bf16_large_tiles_one_behind_the_other(hip, M, N, K):
         assert bool(out[M:].isnan().all()) and bool(out[:, N:].isnan().all())
 
 
-@pytest.mark.parametrize("K,M,N,slices", [(64, 128, 128, 1), (128, 256, 128, 1), (4160, 128, 384, None), (9280, 768, 768, 7), (2048, 2048, 2048, 1)])
+@pytest.mark.parametrize("K,M,N,slices", [(64, 128, 128, 1), (128, 256, 128, 1), (4160, 128, 384, None), (100, 128, 128, 1), (4131, 256, 128, None), (9280, 768, 768, 7), (2048, 2048, 2048, 1)])
 def test_gemm_bf16_tt(hip, K, M, N, slices):
     """Both operands with the reduction index slowest, whole and in slices of unequal lengths: fp32 sums of exact products stay within
     (K + slices) * 2^-24 of the absolute sum, one rounding to bf16."""
     g = gen(K + N)
     ns = hip.load().fstu_gemm_bf16_tt_slices(M, N, K)
-    assert ns == slices if slices else (ns > 1 and (K // 64) % ns)
-    A, B = (dev(torch.randn(K, n, generator=g).bfloat16()) for n in (M, N))
+    assert ns == slices if slices else (ns > 1 and -(-K // 64) % ns)
+    A, B = (torch.full((K + 64, n), float("nan"), dtype=torch.bfloat16, device="cuda")[:K].copy_(torch.randn(K, n, generator=g)) for n in (M, N))
     At = A.t().contiguous().float()
     ref = torch.matmul(At, B.float())                                        # fp32 on the library: K * 2^-24 of the absolute sum too
     bound = (2 * K + ns) * 2.0 ** -24 * torch.matmul(At.abs(), B.float().abs()) + 2.0 ** -8 * ref.abs()
@@ -853,6 +853,36 @@ def test_convolution_gradients_on_the_matrix_cores(hip, B, T, d, L):
     only_x, none_f = run(True, False)
     none_x, only_f = run(False, True)
     assert none_f is None and none_x is None and torch.equal(only_x, gxd) and torch.equal(only_f, gfd)
+
+
+@pytest.mark.parametrize("B,T,L,K,d", [(1, 32, 33, 1, 8), (3, 129, 600, 17, 24), (2, 1025, 1030, 33, 136), (9, 700, 2048, 24, 256), (2, 2048, 2048, 70, 64)])
+def test_convolution_by_a_product_of_filters(hip, B, T, L, K, d):
+    """The taps of T(phi @ m), and the gradient of m behind that of the convolution, against float64: fp32 sums of exact products
+    rounded once (2^-8), the filter's gradient as two bf16 parts (2^-16 of it) times exact rows of phi."""
+    g = gen(T + K)
+    phi, m, x, gy = (dev(torch.randn(*s, generator=g).bfloat16()) for s in ((L, K), (K, d), (B, T, d), (B, T, d)))
+    filt, taps = hip.stu_conv_taps_project(phi, m, T)
+    cap, Lf = taps.shape[2] - 16, filt.shape[0]
+    assert Lf == min(L, 2 * cap) >= T
+    pd, md = phi.double()[:Lf], m.double()
+    assert bool(((filt.double() - pd @ md).abs() <= 2.0 ** -8 * (pd @ md).abs() + K * 2.0 ** -24 * (pd.abs() @ md.abs())).all())
+    want = torch.zeros(d, 2, cap + 1, dtype=torch.bfloat16, device="cuda")          # by lag of a parity
+    for p in (0, 1):
+        f = filt[p::2].t()
+        want[:, p, :f.shape[1]] = f
+    got = taps[:, :, :cap + 1].flip(2)
+    assert torch.equal(got[:, :, :cap], want[:, :, :cap]) and float(taps[:, :, cap + 1:].abs().sum()) == 0
+    even = phi[0::2]
+    phi_e = F.pad(even.t(), (0, -even.shape[0] % 8, 0, -K % 16)).contiguous()
+    gx, gm = hip.stu_conv_mfma_grad_project(gy, x, filt, phi_e, K)
+    assert torch.equal(gx, hip.stu_conv_mfma_grad(gy, x, filt)[0])
+    n = 2 * T
+    corr = lambda p, q: torch.fft.irfft(torch.fft.rfft(p, n, 1) * torch.fft.rfft(q, n, 1).conj(), n, 1)[:, :T:2].sum(0)
+    gf, af = (2 * corr(a, b) for a, b in ((gy.double(), x.double()), (gy.double().abs(), x.double().abs())))
+    pe = even.double()[:gf.shape[0]].t()
+    ref, total = pe @ gf, pe.abs() @ af
+    bound = 2.0 ** -8 * ref.abs() + 2.0 ** -16 * (pe.abs() @ gf.abs()) + (B * T + T) * 2.0 ** -24 * total + 1e-12 * float(total.max())
+    assert bool(((gm.double() - ref).abs() <= bound).all())
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
