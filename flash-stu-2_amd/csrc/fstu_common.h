@@ -48,9 +48,10 @@ int fstu_head_argmax_dyn(const void* x, int ldx, const void* W, void* logits, in
 int fstu_transpose16_launch(const void* in, size_t in_sb, size_t in_row, void* out, size_t out_sb, size_t out_row, int B, int R,
                             int Rp, int C, void* stream);
 int fstu_argmax_finish_launch(void* best_ws, int64_t* tok_out, int64_t tok_stride, int rows, int* dyn, int advance, void* stream);
-bool fstu_finish_embed_supported(int rows, int d, const void* table, const void* x, const void* w, const void* h);
+bool fstu_finish_embed_supported(int rows, int d, const void* table, const void* x, const void* w, const void* h, int dtype);
 int fstu_finish_embed_rmsnorm(void* best_ws, int64_t* tok_out, int64_t tok_stride, const void* table, void* x, const void* w,
-                              void* h, int* dyn, int rows, int d, int vocab, float eps, void* stream);
+                              void* h, int* dyn, int rows, int d, int vocab, float eps, int dtype, void* stream);
+bool fstu_head_argmax_f32_pick(const void* x, int ldx, const void* W, int rows, int N, int K);
 bool fstu_head_argmax_fused_pick(const void* x, int ldx, const void* W, int K, int dtype);
 int fstu_embed_rmsnorm(const int64_t* ids, int64_t id_stride, const void* table, void* x, const void* w, void* h, int rows,
                        int d, int vocab, float eps, int dtype, void* stream, const int* dyn);

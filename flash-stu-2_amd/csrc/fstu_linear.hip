@@ -622,6 +622,11 @@ bool fstu_head_argmax_fused_pick(const void* x, int ldx, const void* W, int K, i
   return dtype == FSTU_BF16 && mfma_ok(x, ldx, W, nullptr, K, 1);
 }
 
+// the same of fp32 rows with dense logits
+bool fstu_head_argmax_f32_pick(const void* x, int ldx, const void* W, int rows, int N, int K) {
+  return f32_ok(LinArgs{x, ldx, W, nullptr, nullptr, N, rows, N, K, K, nullptr, 1.f});
+}
+
 int fstu_head_argmax_dyn(const void* x, int ldx, const void* W, void* logits, int ldy, int rows, int N, int K,
                          float temperature, void* best_ws, int64_t* tok_out, int64_t tok_stride, int* dyn, int advance,
                          int dtype, void* stream) {
@@ -646,8 +651,9 @@ int fstu_head_argmax_dyn(const void* x, int ldx, const void* W, void* logits, in
     // the maxima as a by-product of the head instead of one workgroup per row walking the logits again (1 row of 50257
     // logits: 15.8 us, against 3.4 us for the reduction of 64 maxima)
     launch_f32<LIN_ARGMAX>(a, 1, (hipStream_t)stream);
-    hipLaunchKernelGGL(argmax_finish_kernel, dim3(1), dim3(rows * 64), 0, (hipStream_t)stream, (unsigned long long*)best_ws,
-                       tok_out, tok_stride, rows, dyn, advance > 0 ? 1 : 0);
+    if (advance >= 0)
+      hipLaunchKernelGGL(argmax_finish_kernel, dim3(1), dim3(rows * 64), 0, (hipStream_t)stream, (unsigned long long*)best_ws,
+                         tok_out, tok_stride, rows, dyn, advance);
     FSTU_CHECK_LAUNCH("fstu_head_argmax");
     return FSTU_OK;
   }

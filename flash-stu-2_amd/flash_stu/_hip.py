@@ -96,6 +96,7 @@ SIGNATURES = {
     "fstu_down_packed_splitk": [_vp, _i, _vp, _vp, _i, _i, _i, _vp, _vp],
     "fstu_decode_logits": [_vp, _vp, _i64, _i, _vp],
     "fstu_decode_step": [_vp, _vp, _vp, _i64, _i, _f, _i, _f, _i, _u64, _i, _vp],
+    "fstu_decode_steps": [_vp, _vp, _i64, _i, _i, _f, _i, _f, _i, _u64, _i, _vp],
     "fstu_decode_graph_create": [_vp, _vp, _i64, _vp, _i, _i, _f, _i, _f, _i, _u64, _vp, _vp],
     "fstu_decode_graph_launch": [_vp, _vp],
     "fstu_decode_graph_seek": [_vp, ctypes.c_longlong],

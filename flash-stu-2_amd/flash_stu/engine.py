@@ -1,6 +1,6 @@
 """Decode engine behind FlashSTU.generate(): prefill through the module path,
-then one C-ABI call per token (fstu_decode_step) that launches the fused kernel
-sequence for the whole layer stack against preallocated state and workspaces,
+then one C-ABI call (fstu_decode_steps) that launches the fused kernel sequence
+of every token for the whole layer stack against preallocated state and workspaces,
 or, for several row chunks, the same steps captured as a HIP graph per chunk.
 
 The token buffer (B, max_length) lives on the GPU for the whole loop; each step
@@ -474,7 +474,17 @@ class DecodeEngine:
             _hip.gemm(wx, ww, up_weight=ww)
             _hip.gemm_splitk(wx, ww, 1)
 
-    # ------------------------------------------------------------------ eager step
+    # ------------------------------------------------------------------ eager steps
+    def steps(self, tokens: torch.Tensor, pos: int, n: int, temperature, top_k, top_p, do_sample, seed, step_idx):
+        """n steps of every chunk: the first feeds tokens[:, pos], each writes the token that the next one feeds."""
+        stride = tokens.stride(0)
+        for ch in self.chunks:
+            rc = self.lib.fstu_decode_steps(ctypes.byref(ch.desc), tokens.data_ptr() + 8 * (ch.b0 * stride + pos), stride, pos, int(n),
+                                            float(temperature), int(top_k) if top_k else 0, float(top_p) if top_p else 0.0,
+                                            int(bool(do_sample)), int(seed) & ((1 << 64) - 1), int(step_idx),
+                                            torch.cuda.current_stream().cuda_stream)
+            _hip._check(rc, "fstu_decode_steps")
+
     def step(self, tokens: torch.Tensor, pos: int, temperature, top_k, top_p, do_sample, seed, step_idx):
         """Feeds tokens[:, pos], writes the sampled id to tokens[:, pos+1]."""
         stride = tokens.stride(0)
@@ -611,8 +621,10 @@ class DecodeEngine:
             finally:
                 self.graph_end()
             return tokens
+        if not return_logits:
+            self.steps(tokens, P, n_new - 1, temperature, top_k, top_p, do_sample, seed, 1)
+            return tokens
         for s in range(1, n_new):
             self.step(tokens, P + s - 1, temperature, top_k, top_p, do_sample, seed, s)
-            if return_logits:
-                all_logits.append(self.logits.clone())
-        return (tokens, torch.stack(all_logits, 1)) if return_logits else tokens
+            all_logits.append(self.logits.clone())
+        return tokens, torch.stack(all_logits, 1)

@@ -322,6 +322,24 @@ def test_input_projection_gradients_of_gradients():
         assert float((got.float() - ref.float()).norm()) <= 2.0 ** -7 * float(ref.float().norm())
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("B,d", [(1, 64), (3, 256), (16, 512)])
+def test_greedy_steps_in_one_call(dtype, B, d):
+    """fstu_decode_steps, whose picks are finished in the launch that begins the next step, against a call per step: the same tokens, and
+    nothing left of one call's maxima for the next."""
+    from flash_stu import FlashSTU, FlashSTUConfig
+    torch.manual_seed(B)
+    cfg = FlashSTUConfig(n_embd=d, n_heads=2, n_layers=2, seq_len=64, window_size=16, vocab_size=501, num_eigh=8, torch_dtype=dtype)
+    model = FlashSTU(cfg).cuda().eval()
+    with torch.no_grad():
+        model.lm_head.weight.normal_(0.0, 1.0)         # the picks are clear ones: another order of the norm's sum does not change them
+    ids = torch.randint(0, 501, (B, 9), generator=torch.Generator().manual_seed(d)).cuda()
+    for n in (1, 2, 3, 30):
+        one = model.generate(ids, max_length=9 + n, do_sample=False)
+        each, _ = model.generate(ids, max_length=9 + n, do_sample=False, return_logits=True)
+        assert torch.equal(one, each), n
+
+
 def _teacher_forced(w, ocfg, tokens, P):
     logits, _ = O.model_forward(w, ocfg, tokens[:, :-1])
     return logits[:, P - 1:, :]          # predictions for positions P..end
