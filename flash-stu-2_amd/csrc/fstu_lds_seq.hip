@@ -57,10 +57,12 @@ __device__ __forceinline__ void store16(bf16_t* p, uint4 v) {
 // 1024, state 160, 389 / 331 (state 128 355 / 301), 51 x 3262 x 256, 96, 91 / 71, 8 x 2048 x 512, 128, 53 / 38, 1 x 4096 x 1024,
 // 160, 87 / 55, 64 x 300 x 1024, 160, 88 / 55.  (x, BmT and CmT carry no __restrict__: loads of memory that nothing may change are
 // moved behind the barriers to where their values are used.)
-// What bounds the first: its 1.07 GB.  Without the stores of y it takes 246, without the trips of x to HBM 295, without either
+// What bounds the first: its 1.07 GB, which a copy moves in 208 us, and too few waves to keep memory, matrix cores (busy 38 % of the time)
+// and LDS (32 %) at work at once: two a SIMD, of up to 256 registers.  Without the stores of y it takes 246, without the trips of x to HBM 295, without either
 // 208, with the weights from the compute unit's own cache besides 162.  No gain: x past the caches (360: a line comes in two
 // halves), the blocks of a row side by side (351), the two lines of 128 features of a row stored together (337), another first
-// group of features for every row (340), the scans left out (322).
+// group of features for every row (340), the scans left out (322).  With whole lines of x to a load (half a line of twice as many
+// rows before) 327 / 322, state 128 304 / 298.
 //
 // PAST: the outputs leave past the L2s, where they are more than those hold (32 MB): what they would push out are the weights
 // that every workgroup fetches again, and the next kernel would not find them there.
@@ -96,6 +98,13 @@ lds_seq_kernel(const bf16_t* x, const float* __restrict__ A, const bf16_t* BmT, 
     const bf16_t* xr[2];
 #pragma unroll
     for (int m = 0; m < 2; ++m) xr[m] = x + ((size_t)min(t0 + 32 * w + 16 * m + r, T - 1) * Bt + b) * d_in + g * 8;
+    // A chunk of a row is a line.  The first eight lanes of a row's sixteen have its first half, the others the second, of rows 0..7 of a
+    // tile in one load and of rows 8..15 in another: whole lines; lanes r and r ^ 8 swap pieces in front of the products.
+    const bf16_t* xl[2][2];
+#pragma unroll
+    for (int m = 0; m < 2; ++m)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) xl[m][h] = x + ((size_t)min(t0 + 32 * w + 16 * m + 8 * h + (r & 7), T - 1) * Bt + b) * d_in + 32 * (r >> 3) + g * 8;
     const int swz = (r >> 1) & 7;                            // rows 16n + r and 32i + row share these bits
     const unsigned char* const wrd[2] = {wst + r * 128 + ((g ^ swz) << 4), wst + r * 128 + (((g + 4) ^ swz) << 4)};
     auto multiply = [&](int kk, unsigned stage, const uintx4_t (&xs)[2]) __attribute__((always_inline)) {
@@ -119,12 +128,12 @@ lds_seq_kernel(const bf16_t* x, const float* __restrict__ A, const bf16_t* BmT, 
 #pragma unroll
         for (int i = 0; i < WPT; ++i) *(uintx4_t*)(wdst + stage + i * 4096) = v[i];
       };
-      auto xload = [&](int c, uintx4_t (&v)[2][2]) {            // the two k steps of a chunk, both position tiles
+      auto xload = [&](int c, uintx4_t (&v)[2][2]) {            // both halves of both position tiles
         const int k0 = 64 * min(c, nk - 1);
 #pragma unroll
-        for (int kk = 0; kk < 2; ++kk)
+        for (int h = 0; h < 2; ++h)
 #pragma unroll
-          for (int m = 0; m < 2; ++m) v[kk][m] = *(const uintx4_t*)(xr[m] + k0 + 32 * kk);
+          for (int m = 0; m < 2; ++m) v[h][m] = *(const uintx4_t*)(xl[m][h] + k0);
       };
       uintx4_t wa[WPT], wb[WPT], xa[2][2], xb[2][2], xc[2][2];
       wload(0, wa);
@@ -138,8 +147,15 @@ lds_seq_kernel(const bf16_t* x, const float* __restrict__ A, const bf16_t* BmT, 
       int c = 0;
       unsigned stage = 0;
       auto pass = [&](uintx4_t (&xs)[2][2], uintx4_t (&wn)[WPT]) __attribute__((always_inline)) { // chunk c; wn: the weights of chunk c + 1
-        multiply(0, stage, xs[0]);
-        multiply(1, stage, xs[1]);
+        uintx4_t x0[2], x1[2];
+#pragma unroll
+        for (int m = 0; m < 2; ++m) {
+          const uintx4_t o = __builtin_bit_cast(uintx4_t, swap8(__builtin_bit_cast(uint4, r < 8 ? xs[1][m] : xs[0][m])));
+          x0[m] = r < 8 ? xs[0][m] : o;
+          x1[m] = r < 8 ? o : xs[1][m];
+        }
+        multiply(0, stage, x0);
+        multiply(1, stage, x1);
         stage = wstage - stage;
         wstore(stage, wn);
         wload(c + 3, wn);
@@ -346,29 +362,51 @@ lds_seq_kernel(const bf16_t* x, const float* __restrict__ A, const bf16_t* BmT, 
   }
 }
 
-// clears the published states of the call about to start
-__global__ void __launch_bounds__(256) lds_seq_clear_kernel(unsigned long long* __restrict__ etag, size_t n, unsigned* __restrict__ status) {
-  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) etag[i] = 0ull;
-  if (blockIdx.x == 0 && threadIdx.x == 0) *status = 0u;
-}
-// the state behind the sequence replaces the caller's h (every block has read h by the time this launch starts)
-__global__ void __launch_bounds__(256) lds_seq_finish_kernel(float* __restrict__ h, const float* __restrict__ hnew, int n) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i < n) h[i] = hnew[i];
+// What a call needs before its blocks start: the published states cleared, the state that enters copied (the last block of a row leaves
+// the new one in its place while others still read it) and, where the weights come as they lie, Bm (d_in, S) and Cm (S, d_out) transposed, a tile
+// of 32 x 32 to each of the first nt workgroups.  One launch of 4.3 to 5.9 us: two transposes, the clearing and a copy of the state at the end
+// took launches of their own (5.4 + 5.4 + 5.4 + 5.2 by the profiler; behind each other they hide in part: 64 rows x 4096 x 1024, state 160,
+// with the whole lines of x above 327 -> 322 us a call).
+__global__ void __launch_bounds__(256)
+lds_seq_prepare_kernel(unsigned long long* __restrict__ etag, size_t n, unsigned* __restrict__ status, const float* __restrict__ h, float* __restrict__ h0,
+                       int nh, const bf16_t* __restrict__ Bm, const bf16_t* __restrict__ Cm, bf16_t* __restrict__ wt, int d_in, int S, int d_out, int nb, int nt) {
+  __shared__ bf16_t tile[32][34];
+  const int tid = threadIdx.x;
+  if ((int)blockIdx.x < nt) {
+    const bool first = (int)blockIdx.x < nb;
+    const int t = blockIdx.x - (first ? 0 : nb), rows = first ? d_in : S, cols = first ? S : d_out, across = (cols + 31) >> 5;
+    const bf16_t* const src = first ? Bm : Cm;
+    bf16_t* const dst = wt + (first ? 0 : (size_t)S * d_in);
+    const int r0 = t / across * 32, c0 = t % across * 32, i = tid >> 5, j = tid & 31;
+#pragma unroll
+    for (int k = 0; k < 32; k += 8)
+      if (c0 + j < cols) tile[i + k][j] = src[(size_t)(r0 + i + k) * cols + c0 + j];       // rows: a multiple of 32
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 32; k += 8)
+      if (c0 + i + k < cols) dst[(size_t)(c0 + i + k) * rows + r0 + j] = tile[j][i + k];
+    return;
+  }
+  const size_t first = (size_t)(blockIdx.x - nt) * 256 + tid, step = (size_t)(gridDim.x - nt) * 256;
+  for (size_t i = first; i < n; i += step) etag[i] = 0ull;
+  for (size_t i = first; i < (size_t)nh; i += step) h0[i] = h[i];
+  if (first == 0) *status = 0u;
 }
 
 }  // namespace
 
-// workspace: 64 floats of header (status word), the published block states (nblk * Bt * S 64-bit words), the new h
+// workspace: 64 floats of header (status word), the published block states (nblk * Bt * S 64-bit words), the state that enters
 extern "C" size_t fstu_lds_sequence_ws_floats(int T, int Bt, int S) {
   if (T < 0 || Bt < 1 || S < 1) return 0;
   const size_t nblk = (size_t)(T + LSQ_TB - 1) / LSQ_TB;
   return 64 + (2 * nblk + 1) * (size_t)Bt * S;
 }
 
-extern "C" int fstu_lds_sequence(float* h, const void* x, const float* A, const void* BmT, const void* CmT, void* y, float* ws,
-                                 int T, int Bt, int d_in, int S, int d_out, void* stream) {
-  FSTU_REQUIRE(h && x && A && BmT && CmT && y && ws, FSTU_ENULL, "fstu_lds_sequence: null pointer");
+// wt null: Bm and Cm are given transposed
+static int lds_sequence(float* h, const void* x, const float* A, const void* Bm, const void* Cm, void* wt, void* y, float* ws, int T, int Bt,
+                        int d_in, int S, int d_out, void* stream) {
+  const void *const BmT = wt ? wt : Bm, *const CmT = wt ? (const void*)((const bf16_t*)wt + (size_t)S * d_in) : Cm;
+  FSTU_REQUIRE(h && x && A && Bm && Cm && y && ws, FSTU_ENULL, "fstu_lds_sequence: null pointer");
   FSTU_REQUIRE(T >= 0 && Bt >= 1 && Bt <= 65535, FSTU_ESHAPE, "fstu_lds_sequence: T=%d Bt=%d", T, Bt);
   FSTU_REQUIRE(d_in >= 32 && d_in % 32 == 0 && S >= 32 && S % 32 == 0 && S <= 16 * LSQ_NTMAX && d_out >= 16 && d_out % 16 == 0,
                FSTU_ESHAPE, "fstu_lds_sequence: need d_in %% 32 == 0, S %% 32 == 0 (<= %d), d_out %% 16 == 0 (d_in=%d S=%d d_out=%d)",
@@ -380,7 +418,8 @@ extern "C" int fstu_lds_sequence(float* h, const void* x, const float* A, const 
   const size_t BtS = (size_t)Bt * S;
   unsigned* status = (unsigned*)ws;
   unsigned long long* etag = (unsigned long long*)(ws + 64);
-  float* hnew = ws + 64 + 2 * (size_t)nblk * BtS;
+  float* h0 = ws + 64 + 2 * (size_t)nblk * BtS;
+  const int nb = wt ? d_in / 32 * (S / 32) : 0, nt = wt ? nb + S / 32 * ((d_out + 31) / 32) : 0;
   const size_t shm = (size_t)LSQ_TB * S * sizeof(float);
   hipStream_t s = (hipStream_t)stream;
   const unsigned ny = nblk < 32768 ? (unsigned)nblk : 32768u;
@@ -394,10 +433,10 @@ extern "C" int fstu_lds_sequence(float* h, const void* x, const float* A, const 
     constexpr auto kernel = decltype(which)::value;
     static fstu_lds_limit most;
     if ((rc = fstu_need_lds((const void*)kernel, most, shm, "fstu_lds_sequence"))) return;
-    hipLaunchKernelGGL(lds_seq_clear_kernel, dim3(cgrid), dim3(256), 0, s, etag, nwords, status);
+    hipLaunchKernelGGL(lds_seq_prepare_kernel, dim3(nt + cgrid), dim3(256), 0, s, etag, nwords, status, (const float*)h, h0, (int)BtS, (const bf16_t*)Bm,
+                       (const bf16_t*)Cm, (bf16_t*)wt, d_in, S, d_out, nb, nt);
     hipLaunchKernelGGL(kernel, grid, dim3(256), shm, s, (const bf16_t*)x, A, (const bf16_t*)BmT, (const bf16_t*)CmT, (bf16_t*)y,
-                       (const float*)h, hnew, etag, status, 1u, T, Bt, d_in, d_out, nblk);
-    hipLaunchKernelGGL(lds_seq_finish_kernel, dim3((unsigned)((BtS + 255) / 256)), dim3(256), 0, s, h, (const float*)hnew, (int)BtS);
+                       (const float*)h0, h, etag, status, 1u, T, Bt, d_in, d_out, nblk);
   };
 #define LSQ_RUN(...) run(std::integral_constant<decltype(&lds_seq_kernel<__VA_ARGS__>), lds_seq_kernel<__VA_ARGS__>>{})
 #define LSQ_CASE(n) case 32 * n: past ? LSQ_RUN(2 * n, true) : LSQ_RUN(2 * n, false); break
@@ -409,6 +448,17 @@ extern "C" int fstu_lds_sequence(float* h, const void* x, const float* A, const 
   if (rc) return rc;
   FSTU_CHECK_LAUNCH("fstu_lds_sequence");
   return FSTU_OK;
+}
+
+extern "C" int fstu_lds_sequence(float* h, const void* x, const float* A, const void* BmT, const void* CmT, void* y, float* ws,
+                                 int T, int Bt, int d_in, int S, int d_out, void* stream) {
+  return lds_sequence(h, x, A, BmT, CmT, nullptr, y, ws, T, Bt, d_in, S, d_out, stream);
+}
+
+extern "C" int fstu_lds_sequence_bc(float* h, const void* x, const float* A, const void* Bm, const void* Cm, void* wt, void* y, float* ws,
+                                    int T, int Bt, int d_in, int S, int d_out, void* stream) {
+  FSTU_REQUIRE(wt, FSTU_ENULL, "fstu_lds_sequence_bc: null pointer");
+  return lds_sequence(h, x, A, Bm, Cm, wt, y, ws, T, Bt, d_in, S, d_out, stream);
 }
 
 // 0, or 1 when a wait of the last fstu_lds_sequence call on this workspace ran out (synchronous read of the status word)

@@ -119,6 +119,7 @@ SIGNATURES = {
     "fstu_gemm_bf16_tt": [_vp, _i64, _vp, _i64, _vp, _i64, _i, _i, _i, _vp, _i, _vp],
     "fstu_lds_sequence_ws_floats": [_i, _i, _i],
     "fstu_lds_sequence_status": [_vp, _vp],
+    "fstu_lds_sequence_bc": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp],
     "fstu_lds_sequence": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp],
     "fstu_lds_steps": [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _vp],
 }
@@ -1186,16 +1187,21 @@ def lds_steps(h: torch.Tensor, x: torch.Tensor, A: torch.Tensor, Bm: torch.Tenso
         out = torch.empty(T, Bt, d_out, dtype=x.dtype, device=x.device)
     if (x.dtype == torch.bfloat16 and T >= 1 and d_in % 32 == 0 and S % 32 == 0 and S <= 256 and d_out % 16 == 0
             and x.is_contiguous() and out.is_contiguous()):
-        # blocks of 128 positions in parallel on the matrix cores (weights passed transposed)
+        # blocks of 128 positions in parallel on the matrix cores, which read the weights transposed
         lib = load()
         need = int(lib.fstu_lds_sequence_ws_floats(T, Bt, S))
         if ws is None:
             ws = torch.empty(need, dtype=torch.float32, device=x.device)
         assert ws.dtype == torch.float32 and ws.numel() >= need and ws.is_contiguous()
-        bmt, cmt = transposed if transposed is not None else (Bm.t().contiguous(), Cm.t().contiguous())
-        assert bmt.shape == (S, d_in) and cmt.shape == (d_out, S) and bmt.is_contiguous() and cmt.is_contiguous()
-        _check(lib.fstu_lds_sequence(_p(h), _p(x), _p(A), _p(bmt), _p(cmt), _p(out), _p(ws), T, Bt, d_in, S, d_out, _stream()),
-               "fstu_lds_sequence")
+        if transposed is None:
+            wt = torch.empty(S * (d_in + d_out), dtype=x.dtype, device=x.device)
+            _check(lib.fstu_lds_sequence_bc(_p(h), _p(x), _p(A), _p(Bm), _p(Cm), _p(wt), _p(out), _p(ws), T, Bt, d_in, S, d_out, _stream()),
+                   "fstu_lds_sequence_bc")
+        else:
+            bmt, cmt = transposed
+            assert bmt.shape == (S, d_in) and cmt.shape == (d_out, S) and bmt.is_contiguous() and cmt.is_contiguous()
+            _check(lib.fstu_lds_sequence(_p(h), _p(x), _p(A), _p(bmt), _p(cmt), _p(out), _p(ws), T, Bt, d_in, S, d_out, _stream()),
+                   "fstu_lds_sequence")
         if check_status:
             err = ctypes.c_int(0)
             _check(lib.fstu_lds_sequence_status(_p(ws), ctypes.byref(err)), "fstu_lds_sequence_status")

@@ -496,6 +496,10 @@ size_t fstu_lds_sequence_ws_floats(int T, int Bt, int S);
 int fstu_lds_sequence_status(const float* ws, int* err_out);
 int fstu_lds_sequence(float* h, const void* x, const float* A, const void* BmT, const void* CmT, void* y, float* ws,
                       int T, int Bt, int d_in, int S, int d_out, void* stream);
+/* The same from Bm (d_in,S) and Cm (S,d_out) as they lie, which the first of the call's two launches transposes into wt, bf16 scratch of
+ * S * (d_in + d_out) elements. */
+int fstu_lds_sequence_bc(float* h, const void* x, const float* A, const void* Bm, const void* Cm, void* wt, void* y, float* ws,
+                         int T, int Bt, int d_in, int S, int d_out, void* stream);
 
 /* ---- packed weights -------------------------------------------------------------
  * Packed layout of an (N,K) bf16 row-major weight, K % 32 == 0 (fstu_pack_rows):

@@ -1758,6 +1758,18 @@ def test_lds_sequence_on_the_matrix_cores(hip, T, Bt, din, S, dout):
     assert torch.equal(torch.cat([ya, yb]), y) and torch.equal(h2, h)
 
 
+@pytest.mark.parametrize("T,Bt,din,S,dout", [(300, 3, 96, 32, 48), (129, 2, 1024, 160, 16), (1, 1, 32, 256, 208)])
+def test_lds_sequence_from_weights_as_they_lie(hip, T, Bt, din, S, dout):
+    """The call that transposes the weights itself against the one that is given them transposed, with a state to begin from: the same bits."""
+    g = gen(16)
+    A, h0 = dev(0.9 + 0.099 * torch.rand(S, generator=g)), dev(torch.randn(Bt, S, generator=g))
+    Bm, Cm, x = (dev((torch.randn(*s, generator=g) / s[0] ** 0.5).bfloat16()) for s in ((din, S), (S, dout), (T, Bt, din)))
+    h1, h2 = h0.clone(), h0.clone()
+    y1 = hip.lds_steps(h1, x, A, Bm, Cm, check_status=True)
+    y2 = hip.lds_steps(h2, x, A, Bm, Cm, transposed=(Bm.t().contiguous(), Cm.t().contiguous()), check_status=True)
+    assert torch.equal(y1, y2) and torch.equal(h1, h2) and not torch.equal(h1, h0)
+
+
 def test_argument_errors_do_not_launch(hip):
     x = torch.zeros(17, 64, dtype=torch.bfloat16, device="cuda")
     W = torch.zeros(32, 64, dtype=torch.bfloat16, device="cuda")
