@@ -18,8 +18,8 @@
 // once, transposed 8 x 8 in registers, and a wave works on a channel by itself, so there are two barriers in all.  The result
 // replaces the channel's inputs in LDS and leaves the way it came.
 //
-// us, transforms -> this: 8 x 512 x 768 16 -> 10.5, 32 x 300 x 2048 100 -> 51, 8 x 2048 x 768 61 -> 45, 1 x 4096 x 2048 56 (with a
-// transpose) -> 45.  What bounds the longest two is the matrix cores: 2.36 and 2.62 M products of 16 x 16 x 32, which this card
+// us, transforms -> this: 8 x 512 x 768 16 -> 10.1, 32 x 300 x 2048 100 -> 47.5, 8 x 2048 x 768 61 -> 41, 1 x 4096 x 2048 56 (with a
+// transpose) -> 43.6.  What bounds the longest two is the matrix cores: 2.36 and 2.62 M products of 16 x 16 x 32, which this card
 // issues every 20 cycles on random operands, are 19 and 21 us; the rows' way in and out, 5 and 2 us, is not hidden behind them,
 // because all workgroups that fit start together.  Blocks of 32 positions would save a sixth of the products, but the filter
 // fragments then serve half as many each and the LDS becomes the bound (47 us).
@@ -70,6 +70,15 @@ __device__ __forceinline__ void transpose8(const unsigned (&v)[M][N / 2], unsign
       o[c][j] = __builtin_amdgcn_perm(v[2 * j + 1][c >> 1], v[2 * j][c >> 1], (c & 1) ? 0x07060302 : 0x05040100);
 }
 
+// 5 dwords of taps, loaded as they are stored: the last four are a write of their own.  Where the compiler loads the first four together it
+// copies them to where the write wants them as soon as they are there, that is, waits for them one product after they were requested:
+// us so / apart / apart and a channel's first taps with the inputs or in front of the results before, 4 x 4096 x 2048 164 / 155.6 / 153.4,
+// 1 x 4096 x 2048 46.1 / 44.3 / 43.6, 32 x 300 x 2048 50.8 / 49.8 / 47.5, 8 x 2048 x 768 42.5 / 42.2 / 41.3, 8 x 1024 x 768 20.4 / 19.1,
+// 3 x 777 x 768 12.0 / 11.1.
+typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
+typedef u32x4_t u32x4_a4_t __attribute__((aligned(4)));
+struct Taps5 { unsigned first; u32x4_t rest; };
+
 // NT tiles of NB = 1 << NBS blocks to a parity, NW waves, OCC of them to a SIMD
 template <int NT, int NBS, int NW, int OCC>
 __global__ void __launch_bounds__(NW * 64, OCC)
@@ -80,7 +89,28 @@ conv_mfma_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ taps, 
   constexpr int rg = cm_region(HB), rws = cm_row(HB, NB);
   int c0, row0;
   if (!cm_place(d, B, R, c0, row0)) return;
-  const int tid = threadIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  // expansion: 5 dwords of the reversed taps give the shifts 2a and 2a+1 of a group of 8 lags
+  const int xf = lane >> 5, xn = (lane >> 2) & 7, xa = lane & 3;
+  constexpr int cap = 64 * HB, S = cap + 16;                 // HB pairs of steps
+  constexpr int DEPTH = HB < 2 ? 1 : NT == 4 ? 4 : 2;        // groups of 64 taps on their way
+  constexpr bool EARLY = NT > 1 || NBS < 3;                  // the next channel's are requested in front of this one's results, where registers are left
+  unsigned one = 1;
+  asm("" : "+v"(one));                                       // two loads: see Taps5
+  const unsigned *tp, *tp1;
+  Taps5 w[DEPTH], wf;
+  auto fetch = [&](Taps5& r, int P) {
+    r.first = *(tp - 32 * min(P, HB - 1));
+    r.rest = *(const u32x4_a4_t*)(tp1 - 32 * min(P, HB - 1));
+  };
+  auto first_taps = [&](int ch) {
+    tp = (const unsigned*)(taps + ((size_t)(c0 + ch) * 2 + xf) * S + cap - 8 * xn - 2 * xa - 2);
+    tp1 = tp + one;
+    fetch(wf, 0);
+#pragma unroll
+    for (int k = 0; k < DEPTH; ++k) fetch(w[k], k + 1);
+  };
+  if (EARLY) first_taps(wave);                               // with the inputs: one trip
   const int pieces = R * HB * 16;                           // (sequence, 8 positions of one parity)
   for (int v = tid; v < R * 128; v += NW * 64)               // the zeros in front of every region
     *(uint4*)(lds + (v >> 7) * rws + ((v >> 3) & 15) * rg + (v & 7) * 16) = make_uint4(0, 0, 0, 0);
@@ -101,12 +131,9 @@ conv_mfma_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ taps, 
   }
   __syncthreads();
 
-  const int lane = tid & 63, wave = tid >> 6, col = lane & 15, g = lane >> 4;
+  const int col = lane & 15, g = lane >> 4;
   const int par = col >> 3, cc = col & 7, row = cc >> NBS, q = cc & (NB - 1);
   char* const ring = lds + R * rws + wave * CM_RING;
-  // expansion: 5 dwords of the reversed taps give the shifts 2a and 2a+1 of a group of 8 lags
-  const int xf = lane >> 5, xn = (lane >> 2) & 7, xa = lane & 3;
-  constexpr int cap = 64 * HB, S = cap + 16;                 // HB pairs of steps
   char* const xdst = ring + xf * 2048 + ring_at(xn, 2 * xa);
   const int fh = (col >> 3) - g;                             // group of the lane's first filter value
   int fat[4];
@@ -114,23 +141,13 @@ conv_mfma_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ taps, 
   for (int k = 0; k < 4; ++k) fat[k] = ring_at(fh + 2 * k, col & 7);
 
   for (int ch = wave; ch < 8; ch += NW) {
-    const unsigned* tp = (const unsigned*)(taps + ((size_t)(c0 + ch) * 2 + xf) * S + cap - 8 * xn - 2 * xa - 2);
-    constexpr int DEPTH = HB < 2 ? 1 : NT == 4 ? 4 : 2;      // groups of 64 taps on their way
-    unsigned w[DEPTH][5], wf[5];
-    auto fetch = [&](unsigned (&r)[5], int P) {
-      const unsigned* src = tp - 32 * min(P, HB - 1);
-#pragma unroll
-      for (int k = 0; k < 5; ++k) r[k] = src[k];
-    };
-    auto expand = [&](const unsigned (&r)[5], bool odd) {
+    auto expand = [&](const Taps5& r, bool odd) {
       char* dst = xdst + odd * 1024;
-      *(uint4*)dst = make_uint4(r[1], r[2], r[3], r[4]);
-      *(uint4*)(dst + 16) = make_uint4(__builtin_amdgcn_alignbit(r[1], r[0], 16), __builtin_amdgcn_alignbit(r[2], r[1], 16),
-                                       __builtin_amdgcn_alignbit(r[3], r[2], 16), __builtin_amdgcn_alignbit(r[4], r[3], 16));
+      *(u32x4_t*)dst = r.rest;
+      *(uint4*)(dst + 16) = make_uint4(__builtin_amdgcn_alignbit(r.rest[0], r.first, 16), __builtin_amdgcn_alignbit(r.rest[1], r.rest[0], 16),
+                                       __builtin_amdgcn_alignbit(r.rest[2], r.rest[1], 16), __builtin_amdgcn_alignbit(r.rest[3], r.rest[2], 16));
     };
-    fetch(wf, 0);
-#pragma unroll
-    for (int k = 0; k < DEPTH; ++k) fetch(w[k], k + 1);
+    if (!EARLY) first_taps(ch);
     wave_order();
     if (lane < 48) *(uint4*)(ring + (lane / 24) * 2048 + 13 * 128 + (lane % 24) * 16) = make_uint4(0, 0, 0, 0);   // lags below 0
     expand(wf, false);
@@ -145,7 +162,7 @@ conv_mfma_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ taps, 
 #pragma unroll
     for (int k = 0; k < 2; ++k) fa[k][0] = fa[k][1] = make_uint4(0, 0, 0, 0);
     // A pair of steps, 64 lags, for the tiles from J0 on; the next 64 lags are expanded behind the last reads of these.
-    auto pair = [&](auto first, int P, bool odd, unsigned (&r)[5]) {
+    auto pair = [&](auto first, int P, bool odd, Taps5& r) {
       constexpr int J0 = decltype(first)::value;
 #pragma unroll
       for (int s = 0; s < 2; ++s) {
@@ -191,6 +208,8 @@ conv_mfma_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ taps, 
     phase(std::integral_constant<int, 2>{});
     phase(std::integral_constant<int, 3>{});
     wave_order();
+
+    if (EARLY && ch + NW < 8) first_taps(ch + NW);
 
     // Branches and rounding.  A lane of an x_0 column has E_0 and O_1, of an x_1 column E_1 and W = O_0 one position early.  The other
     // column's values cross over by a rotation within 16 lanes; W of the position before the lane's four comes from the lane 16
