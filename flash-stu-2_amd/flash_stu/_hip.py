@@ -162,6 +162,18 @@ def is_available() -> bool:
     return os.path.exists(LIB_PATH) and torch.cuda.is_available()
 
 
+def inference(fn):
+    """The function under torch.no_grad(), which is entered only where gradients are on: the parts of a model call each other some sixty
+    times a prompt, each entry and exit 0.9 us."""
+    @functools.wraps(fn)
+    def wrapped(*args, **kwargs):
+        if torch.is_grad_enabled():
+            with torch.no_grad():
+                return fn(*args, **kwargs)
+        return fn(*args, **kwargs)
+    return wrapped
+
+
 def _check(rc: int, name: str):
     if rc != 0:
         msg = load().fstu_last_error().decode("utf-8", "replace")
@@ -393,9 +405,8 @@ def _gemm_rows(x2, weight, up_weight, residual, out, mode: int, ldr: int) -> Non
 def gemm_any(a: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """out (M,N) = T(a @ w^T) for ANY strided 2-D views a (M,K) and w (N,K) of one dtype (fp32 or bf16): the general
     kernel behind everything the bf16 matrix-core GEMM does not take.  fp32 accumulation, one rounding."""
-    for t in (a, w, out):
-        if t is not None and not t.is_cuda:
-            raise FlashSTUHipError("tensor is not on the GPU: the HIP path has no CPU fallback")
+    if not (a.is_cuda and w.is_cuda and (out is None or out.is_cuda)):
+        raise FlashSTUHipError("tensor is not on the GPU: the HIP path has no CPU fallback")
     if a.dim() != 2 or w.dim() != 2 or a.shape[1] != w.shape[1] or a.dtype != w.dtype:
         raise FlashSTUHipError(f"gemm_any: operands {tuple(a.shape)} {a.dtype} x {tuple(w.shape)} {w.dtype}")
     M, K = a.shape
@@ -404,11 +415,12 @@ def gemm_any(a: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = Non
         out = torch.empty(M, N, dtype=a.dtype, device=a.device)
     if out.shape != (M, N) or out.stride(1) != 1 or out.dtype != a.dtype:
         raise FlashSTUHipError("gemm_any: out must be (M,N) with contiguous rows")
-    # a size-1 dimension may carry any stride: give it a positive one; an expanded one is laid out
-    a, w = (t.contiguous() if any(n > 1 and st == 0 for n, st in zip(t.shape, t.stride())) else t for t in (a, w))
-    sam, sak = max(a.stride(0), 1), max(a.stride(1), 1)
-    swn, swk = max(w.stride(0), 1), max(w.stride(1), 1)
-    _check(load().fstu_gemm_any(_p(a), sam, sak, _p(w), swn, swk, _p(out), out.stride(0), M, N, K, _dt(a), _stream()),
+    (sam, sak), (swn, swk) = a.stride(), w.stride()
+    if not (sam and sak and swn and swk):
+        # a size-1 dimension may carry any stride: give it a positive one; an expanded one is laid out
+        a, w = (t.contiguous() if any(n > 1 and st == 0 for n, st in zip(t.shape, t.stride())) else t for t in (a, w))
+        sam, sak, swn, swk = (max(st, 1) for st in (*a.stride(), *w.stride()))
+    _check(load().fstu_gemm_any(a.data_ptr(), sam, sak, w.data_ptr(), swn, swk, out.data_ptr(), out.stride(0), M, N, K, _dt(a), _stream()),
            "fstu_gemm_any")
     return out
 
@@ -701,6 +713,7 @@ def stu_conv_direct(xp: torch.Tensor, filt: torch.Tensor, single_branch: bool = 
     return out
 
 
+@functools.lru_cache(maxsize=256)
 def fft_length(T: int) -> int:
     """Smallest supported transform length (power of two, 64..16384) with n >= 2T; 0 if T is too long."""
     return int(load().fstu_fft_length(int(T)))
@@ -712,7 +725,11 @@ _twiddle_cache = {}
 def fft_twiddles(n: int, device) -> torch.Tensor:
     """The twiddle tables of the n-point kernels, (n, 2) fp32 on `device` in the transforms' own order, built once per
     (n, device).  Whichever stream asks for them next finds them written; a graph that is being captured builds its own."""
-    key = (int(n), torch.device(device).index if torch.device(device).index is not None else torch.cuda.current_device())
+    tw = _twiddle_cache.get((n, device))         # a tensor's device: it has an index
+    if tw is not None:
+        return tw
+    dev = torch.device(device)
+    key = (int(n), dev if dev.index is not None else torch.device(dev.type, torch.cuda.current_device()))
     tw = _twiddle_cache.get(key)
     if tw is None:
         tw = torch.empty(n, 2, dtype=torch.float32, device=device)

@@ -87,7 +87,7 @@ def _weight(m):
     return m.weight if w is None else w
 
 
-@torch.no_grad()
+@_hip.inference
 def step_on_caches(model, ids: torch.Tensor, past):
     """One position of each row, ids (B,1), against the caches that model(..., use_cache=True) returned: (logits (B,1,V),
     caches one position on) through the one-call step, the state in the caches advanced in place, or None where a row
@@ -423,21 +423,22 @@ class DecodeEngine:
         m.emb, m.final_norm_w = emb.data_ptr(), ptr(model.norm.weight)
         m.layers = ctypes.cast(arr, ctypes.POINTER(LayerDesc))
 
-        def buf(*shape, dtype=dt):
-            t = torch.zeros(*shape, dtype=dtype, device=dev)
-            keep(t)
-            return t
-        ch.logits = buf(B, V)
-        m.x, m.h = buf(B, d).data_ptr(), buf(B, d).data_ptr()
-        m.qkv, m.attn = buf(B, 3 * d).data_ptr(), buf(B, d).data_ptr()
-        m.act, m.xp, m.y = buf(B, I).data_ptr(), buf(B, d).data_ptr(), buf(B, d).data_ptr()
-        m.partial = buf(max(m.ksplit_down, 16), B, d, dtype=torch.float32).data_ptr()
-        m.eo = buf(self.HIST_NSPLIT_MAX, 2, B, d, dtype=torch.float32).data_ptr()
+        ch.logits = keep(torch.zeros(B, V, dtype=dt, device=dev))
         m.logits = ch.logits.data_ptr()
-        m.best = buf(32 * 64, dtype=torch.int64).data_ptr()
-        if dt == torch.float32:
-            m.x2 = buf(B, d).data_ptr()         # the stream behind the norms that a projection forms itself
-        m.samp_ws = buf((int(self.lib.fstu_sample_ws_bytes()) + 7) // 8, dtype=torch.int64).data_ptr()
+        # the other workspaces in one piece, cleared by one launch: rows of d in the model's dtype, the others by their bytes
+        esz = ch.logits.element_size()
+        sizes = dict(x=B * d * esz, h=B * d * esz, qkv=3 * B * d * esz, attn=B * d * esz, act=B * I * esz, xp=B * d * esz, y=B * d * esz,
+                     x2=B * d * esz,             # the stream behind the norms that a projection forms itself
+                     partial=max(m.ksplit_down, 16) * B * d * 4, eo=self.HIST_NSPLIT_MAX * 2 * B * d * 4, best=32 * 64 * 8,
+                     samp_ws=int(self.lib.fstu_sample_ws_bytes()))
+        at = keep(torch.zeros(sum(-(-n // 256) * 256 for n in sizes.values()), dtype=torch.uint8, device=dev)).data_ptr()
+        place = {}
+        for name, size in sizes.items():
+            place[name] = at
+            at += -(-size // 256) * 256
+        for name in sizes:
+            if name != "x2" or dt == torch.float32:
+                setattr(m, name, place[name])
         if dt == torch.bfloat16 and self.lib.fstu_glu_packed_supported(B, d, I):
             # gate/up projection over packed weights, one workgroup per CU with equal bytes each
             for i, (ld, w) in enumerate(zip(arr, weights)):
@@ -448,7 +449,7 @@ class DecodeEngine:
                     ld.wp_down = ptr(self._pack(w["down"], (i, "down")))
                 m.down_packed = 1
             if B * (d + 8) * 2 <= 96 * 1024:
-                m.x2 = buf(B, d).data_ptr()     # second residual buffer: the MLP norm runs as the gate/up prologue
+                m.x2 = place["x2"]              # second residual buffer: the MLP norm runs as the gate/up prologue
                 if mode == "lds" and d % 256 == 0 and m.down_packed and B * (d // 8) <= 1024 and I % 128 == 0:
                     # the add+norm between two layers runs as the prologue of the next layer's first projection
                     # (the down projection leaves 4 split-K slices for it): one launch less per layer
@@ -570,7 +571,7 @@ class DecodeEngine:
         self._gstreams = []
 
     # ------------------------------------------------------------------
-    @torch.no_grad()
+    @_hip.inference
     def prefill(self, input_ids: torch.Tensor, total_len: int):
         """Runs the prompt through the module path with caches, returns the
         logits of the last position (B,V) and prepares the step descriptors."""
@@ -583,7 +584,7 @@ class DecodeEngine:
         self.caches = self._build(caches, B, total_len)
         return logits
 
-    @torch.no_grad()
+    @_hip.inference
     def generate(self, input_ids: torch.Tensor, n_new: int, temperature=1.0, top_k=None, top_p=None, do_sample=True,
                  seed: int = 0, return_logits: bool = False, use_graph: bool = True):
         if not input_ids.is_cuda:

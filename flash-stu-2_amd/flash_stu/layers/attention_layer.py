@@ -18,7 +18,7 @@ class AttentionLayer(nn.Module):
         self.mlp_norm = RMSNorm(config.n_embd, config.rms_norm_eps, dtype=config.torch_dtype)
         self.mlp = MLP(config, dtype=config.torch_dtype)
 
-    @torch.no_grad()
+    @_hip.inference
     def forward(self, x: torch.Tensor, past_key_value=None, use_cache: bool = True):
         a = self.attn_norm(x)
         if use_cache or past_key_value is not None:

@@ -31,7 +31,7 @@ class STULayer(nn.Module):
         self.mlp_norm = RMSNorm(config.n_embd, config.rms_norm_eps, dtype=config.torch_dtype)
         self.mlp = MLP(config, dtype=config.torch_dtype)
 
-    @torch.no_grad()
+    @_hip.inference
     def forward(self, x: torch.Tensor, past_key_value=None, use_cache: bool = False):
         """Returns x, or (x, state) when use_cache.  Unlike the reference, whose
         STU layers return None as their cache entry (stu_layer.py:118-119), the

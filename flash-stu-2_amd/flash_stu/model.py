@@ -131,7 +131,7 @@ class FlashSTU(nn.Module):
     def _head(self, x: torch.Tensor) -> torch.Tensor:
         return _hip.linear(x, self.lm_head.weight, self.lm_head.bias)
 
-    @torch.no_grad()
+    @_hip.inference
     def _run_layers(self, x, past_key_values, use_cache, hidden):
         cache = []
         for idx, layer in enumerate(self.layers):
@@ -145,7 +145,7 @@ class FlashSTU(nn.Module):
                 hidden.append(x.clone())
         return x, (tuple(cache) if use_cache else None)
 
-    @torch.no_grad()
+    @_hip.inference
     def forward(self, input_ids: Optional[torch.LongTensor] = None, attention_mask: Optional[torch.Tensor] = None,
                 past_key_values: Optional[Tuple] = None, labels: Optional[torch.LongTensor] = None,
                 use_cache: Optional[bool] = None, output_hidden_states: Optional[bool] = None,
@@ -208,7 +208,7 @@ class FlashSTU(nn.Module):
             self._engine = DecodeEngine(self)
         return self._engine
 
-    @torch.no_grad()
+    @_hip.inference
     def generate(self, input_ids: torch.LongTensor, max_length: int = 100, temperature: float = 1.0,
                  top_k: Optional[int] = None, top_p: Optional[float] = None, do_sample: bool = True,
                  use_cache: bool = True, seed: int = 0, return_logits: bool = False, **kwargs) -> torch.LongTensor:

@@ -56,7 +56,7 @@ class Attention(nn.Module):
         vr[:, :, pos % cap] = v[:, t - keep:].transpose(1, 2)
         return kr, vr, torch.full((B,), t, dtype=torch.int64)
 
-    @torch.no_grad()
+    @_hip.inference
     def forward(self, x: torch.Tensor, past_key_value=None, use_cache: bool = True):
         x = x.contiguous()
         B, T, d = x.shape

@@ -13,11 +13,11 @@ class RMSNorm(nn.Module):
         self.eps = eps
         self.weight = nn.Parameter(torch.ones(dim, dtype=dtype))
 
-    @torch.no_grad()
+    @_hip.inference
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         return _hip.add_rmsnorm(x.contiguous(), None, self.weight, self.eps)
 
-    @torch.no_grad()
+    @_hip.inference
     def add_then_norm(self, x: torch.Tensor, delta: torch.Tensor) -> torch.Tensor:
         """x += delta in place, returns norm(x)."""
         return _hip.add_rmsnorm(x, delta.contiguous(), self.weight, self.eps)

@@ -128,9 +128,9 @@ class STU(nn.Module):
     def filter_spectrum(self, n: int) -> torch.Tensor:
         """Spectra of the convolution filters for transform length n, (d,n,2) fp32 in approx mode, (K,n,2) in
         exact mode (the reference keeps its own phi_fft the same way, stu.py:43-53).  One length is kept."""
-        src = self.effective_filter() if self.use_approx else self.phi
         params = (self.phi, self.M_filters) if self.use_approx else (self.phi,)
-        return self._cached("spec", params, lambda: _hip.stu_fft_filter(src, n, single_branch=self.use_hankel_L), form=n)
+        return self._cached("spec", params, lambda: _hip.stu_fft_filter(self.effective_filter() if self.use_approx else params[0], n,
+                                                                       single_branch=self.use_hankel_L), form=n)
 
     def filter_taps(self, T: int) -> torch.Tensor:
         """The convolution filters as the Toeplitz product reads them for T positions, (d,2,S) (approx mode, bf16).  In the place
@@ -391,7 +391,7 @@ class STU(nn.Module):
             return plus if self.use_hankel_L else plus + minus
         return ApproxConvolveSum.apply(x_proj, phi_proj.to(x_proj.dtype))
 
-    @torch.no_grad()
+    @_hip.inference
     def forward(self, x: torch.Tensor, past_state=None, use_cache: bool = False):
         """x (B,T,d).  Without past_state the whole sequence is convolved from
         position 0 (the reference's forward).  With past_state, T must be 1 and

@@ -17,7 +17,7 @@ class MLP(nn.Module):
         self.up_proj = nn.Linear(self.hidden_size, self.intermediate_size, bias=config.bias, dtype=dtype)
         self.down_proj = nn.Linear(self.intermediate_size, self.hidden_size, bias=config.bias, dtype=dtype)
 
-    @torch.no_grad()
+    @_hip.inference
     def forward(self, x: torch.Tensor, residual: torch.Tensor = None):
         """x (..., d).  Up to 16 rows take the skinny MFMA kernels with the gate fused; more rows in bf16 take the
         matrix-core GEMM kernel with the gate as the epilogue of the gate/up pair.  With `residual` (same shape as x,
