@@ -677,6 +677,149 @@ int gemm_pp_launch(const void* A, long long lda, const void* W, const void* W2, 
   return 0;
 }
 
+// ---------------------------------------------------------------- 256 rows x 128 features in two alternating wave groups
+// Products whose 256 x 256 tiles leave half of the compute units idle, whole or in slices of K.  Waves 0-3 own rows 0..127, waves 4-7
+// rows 128..255, a wave 64 features x 64 rows; a k tile of 64 is one phase of 32 v_mfma_f32_16x16x32_bf16.  The groups run half
+// a phase apart as above.  Three stages of W | X0 | X1 (16 KB each); in its memory phase of k tile kt a group reads its 16 fragments
+// and requests its share of kt + 2 into the stage that both groups left a phase ago, and waits for its share of kt + 1.
+// What bounds it: 0.58 us a k tile in a nearly empty round, of which its products are 0.49; 0.65 to 0.9 in a full one (power, LDS).
+// us, before (256 x 256 or 128 x 128 tiles) / so: 4096 x 2048 x 2048 41.3 / 32.1, 2331 x 2304 x 768 17.2 / 13.7, 8192 x 768 x 768 17.3 / 13.7,
+// 1024 x 8192 x 4096 65.0 / 53.3; joined slices of K 2331 x 768 x 9216 44.9 / 41.3, 4096 x 768 x 9216 73.8 / 62.4, 1000 x 2048 x 24576 101.6 / 88.5.
+#define PH_STAGE 49152u
+#define PH_LDS (3 * PH_STAGE)
+template <int MODE>
+__global__ void __launch_bounds__(512)
+gemm_half_bf16_kernel(const bf16_t* __restrict__ A, long long lda, const bf16_t* __restrict__ W, const bf16_t* __restrict__ R, long long ldr,
+                      bf16_t* __restrict__ C, long long ldc, int M, int N, int K, int mt, int nt, int share, int ksplit) {
+  extern __shared__ __align__(16) unsigned char gm_smem[];
+  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int o = (int)(blockIdx.x & 7) * share + (int)(blockIdx.x >> 3);
+  if ((int)(blockIdx.x >> 3) >= share || o >= mt * nt * ksplit) return;
+  const int slice = o / (mt * nt), nk = K >> 6;       // MODE 3: slices of K outermost, any number of k tiles to each
+  o -= slice * (mt * nt);
+  const int kt0 = MODE == 3 ? (int)((long long)nk * slice / ksplit) : 0, kt1 = MODE == 3 ? (int)((long long)nk * (slice + 1) / ksplit) : nk;
+  const int per_panel = mt * GM_PANEL, panel = o / per_panel, in_panel = o - panel * per_panel;
+  const int pw = min(GM_PANEL, nt - panel * GM_PANEL);
+  const int m0 = in_panel / pw * 256, n0 = (panel * GM_PANEL + in_panel % pw) * 128;
+  const rsrc_t rs_w = make_rsrc(W + (size_t)n0 * K, (size_t)min(128, N - n0) * K * 2);
+  const rsrc_t rs_a = make_rsrc(A + (size_t)m0 * lda, ((size_t)(min(256, M - m0) - 1) * lda + K) * 2);
+  // ---- fills: a part is 128 rows of 128 bytes; a wave fills rows 16 wv .. + 15 of each with two instructions
+  unsigned wvoff[2], avoff[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int row = wv * 16 + j * 8 + (lane >> 3);
+    wvoff[j] = (unsigned)row * (unsigned)K * 2u + (unsigned)((lane & 7) ^ (((row >> 1) & 1) | ((row >> 2) & 6))) * 16u;
+    avoff[j] = (unsigned)row * (unsigned)lda * 2u + (unsigned)((lane & 7) ^ ((row >> 1) & 7)) * 16u;
+  }
+  const unsigned x1off = 128u * (unsigned)lda * 2u;
+  unsigned char* const fill0 = gm_smem + (unsigned)wv * 2048u;
+  auto fetch = [&](int kt, unsigned stage) __attribute__((always_inline)) {   // beyond the last k tile the addresses lie behind both descriptors
+    const unsigned so = (unsigned)min(kt, kt1 - 1) * 128u;
+    unsigned char* const l = fill0 + stage;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) buf_load16_to_lds(rs_w, wvoff[j], so, l + j * 1024);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) buf_load16_to_lds(rs_a, avoff[j], so, l + PP_PART + j * 1024);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) buf_load16_to_lds(rs_a, avoff[j] + x1off, so, l + 2 * PP_PART + j * 1024);
+  };
+  const int l16 = lane & 15, lq = lane >> 4, wf = wv & 1, wr = (wv >> 1) & 1, grp = wv >> 2;
+  unsigned fw_off[2], fx_off[2];
+#pragma unroll
+  for (int kk = 0; kk < 2; ++kk) {
+    const int rw = wf * 64 + 8 * (l16 >> 2) + (l16 & 3), rx = wr * 64 + l16, c = kk * 4 + lq;
+    fw_off[kk] = (unsigned)rw * 128u + (unsigned)((c ^ (((rw >> 1) & 1) | ((rw >> 2) & 6))) << 4);
+    fx_off[kk] = (unsigned)(1 + grp) * PP_PART + (unsigned)rx * 128u + (unsigned)((c ^ ((rx >> 1) & 7)) << 4);
+  }
+  const unsigned smem0 = lds_addr(gm_smem);
+  u32x4_t wa[8], xf[8];                                // (k step, feature tile), (k step, row tile)
+  floatx4_t acc[4][4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[i][j] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+  fetch(kt0, 0);
+  fetch(kt0 + 1, PH_STAGE);
+  asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  if (grp) __builtin_amdgcn_s_barrier();               // the second group runs half a phase later
+  unsigned cur = 0, two = 2 * PH_STAGE;                // stages of k tiles kt and kt + 2
+  __builtin_amdgcn_sched_barrier(0);
+  for (int kt = kt0; kt < kt1; ++kt) {
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      const unsigned a = smem0 + cur + fw_off[kk];
+      wa[4 * kk] = lds_read16<0>(a);
+      wa[4 * kk + 1] = lds_read16<512>(a);
+      wa[4 * kk + 2] = lds_read16<4096>(a);
+      wa[4 * kk + 3] = lds_read16<4096 + 512>(a);
+      lds_read_rows<4, 2048>(xf + 4 * kk, smem0 + cur + fx_off[kk]);
+    }
+    fetch(kt + 2, two);
+    asm volatile("s_waitcnt vmcnt(6) lgkmcnt(0)"
+                 : "+v"(xf[0]), "+v"(xf[1]), "+v"(xf[2]), "+v"(xf[3]), "+v"(xf[4]), "+v"(xf[5]), "+v"(xf[6]), "+v"(xf[7]),
+                   "+v"(wa[0]), "+v"(wa[1]), "+v"(wa[2]), "+v"(wa[3]), "+v"(wa[4]), "+v"(wa[5]), "+v"(wa[6]), "+v"(wa[7])::"memory");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, wa[4 * kk + i]), __builtin_bit_cast(bf16x8_t, xf[4 * kk + j]),
+                                                              acc[i][j], 0, 0, 0);
+    __builtin_amdgcn_s_setprio(0);
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    cur = cur == 2 * PH_STAGE ? 0 : cur + PH_STAGE;
+    two = two == 2 * PH_STAGE ? 0 : two + PH_STAGE;
+  }
+  if (!grp) __builtin_amdgcn_s_barrier();
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // the fills behind the last k tile
+  // lane l holds row l % 16 and, of two feature tiles, features 8*(l/16) .. + 7
+  if constexpr (MODE == 3) {
+    float* const part = (float*)C + (size_t)slice * M * N;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int m = m0 + grp * 128 + wr * 64 + j * 16 + l16, f = n0 + wf * 64 + (i >> 1) * 32 + 8 * lq + (i & 1) * 4;
+        if (m < M && f < N) *(floatx4_t*)(part + (size_t)m * N + f) = acc[i][j];
+      }
+  } else {
+    __builtin_amdgcn_s_barrier();                      // every wave has left the stages: rows of 256 bytes, chunks XOR-ed with the row
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        const int r = grp * 128 + wr * 64 + j * 16 + l16, c = wf * 8 + p * 4 + lq;
+        const floatx4_t a = acc[2 * p][j], b = acc[2 * p + 1][j];
+        *(uint4*)(gm_smem + r * 256 + ((c ^ (r & 15)) << 4)) = make_uint4(pack2_bf16(a[0], a[1]), pack2_bf16(a[2], a[3]), pack2_bf16(b[0], b[1]), pack2_bf16(b[2], b[3]));
+      }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int r = i * 32 + (tid >> 4), c = tid & 15, m = m0 + r, f = n0 + c * 8;
+      const u32x4_t v = *(const u32x4_t*)(gm_smem + r * 256 + ((c ^ (r & 15)) << 4));
+      if (m < M && f < N) store_feat8<MODE>(v, MODE == 2 ? R + (size_t)m * ldr + f : nullptr, C + (size_t)m * ldc + f, N - f);
+    }
+  }
+}
+
+template <int MODE>
+int gemm_half_launch(const void* A, long long lda, const void* W, const void* R, long long ldr, void* C, long long ldc, int M, int N, int K,
+                     hipStream_t s, int ksplit = 1) {
+  static fstu_lds_limit most;
+  if (const int rc = fstu_need_lds((const void*)gemm_half_bf16_kernel<MODE>, most, PH_LDS, "fstu_gemm_bf16")) return rc;
+  const int mt = (M + 255) / 256, nt = (N + 127) / 128, share = (int)(((long long)mt * nt * ksplit + 7) / 8);
+  hipLaunchKernelGGL((gemm_half_bf16_kernel<MODE>), dim3((unsigned)share * 8u), dim3(512), PH_LDS, s, (const bf16_t*)A, lda, (const bf16_t*)W,
+                     (const bf16_t*)R, ldr, (bf16_t*)C, ldc, M, N, K, mt, nt, share, ksplit);
+  return 0;
+}
+
 // ---------------------------------------------------------------- transposed activations
 // C[b][m, n] = sum_k A[b][k, m] W[n, k]: the activations come as a slab with the REDUCTION index slowest (k rows of
 // lda elements, m contiguous) — the time-major U+- of the exact-mode STU operator (flash_stu/modules/stu.py:107-120:
@@ -945,6 +1088,14 @@ bool pp_takes(int mode, int K, long long big, long long small) {
 }
 long long tiles_of(int side, int M, int N) { return (long long)((M + side - 1) / side) * (((long long)N + side - 1) / side); }
 
+// One round of 256 x 128 tiles where 128 x 128 ones would be more than one to a compute unit.  us, 256 x 128 / the others, either side of the
+// line, rows x features (256 x 128 tiles, 128 x 128 tiles): 2048 x 2304 (144, 288) K = 64 8.0 / 9.1, 256 8.3 / 11.0, 768 12.7 / 16.9, 2048 24.7 / 30.1,
+// 4096 42.0 / 50.6; 1024 x 8192 (256, 512) 8.1 / 8.6, 9.8 / 11.2, 16.7 / 19.0, 32.4 / 37.4, 53.3 / 65.0; 300 x 12000 (188, 282) K = 768 12.3 /
+// 15.2; 2048 x 2048 (128, 256) K = 768 12.2 / 12.1, 2048 27.0 / 22.8; 4096 x 2304 (288, 576) K = 768 24.1 / 20.1.
+bool half_takes(int M, int N) {
+  return (long long)((M + 255) / 256) * ((N + 127) / 128) <= gemm_cus() && tiles_of(128, M, N) > gemm_cus();
+}
+
 template <int MODE>
 int gemm_launch(const void* A, long long lda, const void* W, const void* W2, const void* R, long long ldr, void* C, long long ldc,
                 int M, int N, int K, hipStream_t s) {
@@ -952,6 +1103,9 @@ int gemm_launch(const void* A, long long lda, const void* W, const void* W2, con
   if (M <= 32) return gemm_launch_tile<TileRows32, MODE>(A, lda, W, W2, R, ldr, C, ldc, M, N, K, s);
   const int columns = MODE == 1 ? 2 * N : N;
   const long long small = tiles_of(128, M, columns);
+  if constexpr (MODE != 1) {
+    if (half_takes(M, N)) return gemm_half_launch<MODE>(A, lda, W, R, ldr, C, ldc, M, N, K, s);
+  }
   if (pp_takes(MODE, K, tiles_of(256, M, columns), small))
     return gemm_pp_launch<MODE>(A, lda, W, W2, R, ldr, C, ldc, M, N, K, s);
   // A grid that leaves one workgroup per compute unit anyway gains from the deeper pipeline when K is long (M=4096, N=768,
@@ -1009,10 +1163,15 @@ namespace {
 // 266 / 170 (L3); 8300 x 512 x 6144 75 / 60 (L3), 7800 x 1024 x 12288 225 / 161 (L2).  Where it stays as it was, with
 // the best slices of large tiles: 1000 x 2048 x 24576 105 / 91 (6), 6100 485 / 498 (4), 4096 x 768 x 9216 66 / 61 (4), 16000 180 / 230 (2), 2500 x 2048 x 2048 31 / 39 (2).  Slabs: 1 x 8192 x 1024 x 24576 451 / 309 (L2), 4 x 2048 454 / 303 (L2), 2 x
 // 2048 242 / 159 (L4), 1 x 4096 x 768 x 18432 142 / 111 (L4).
-struct SlicePlan { int count; bool large; };
-SlicePlan slice_plan(int M, int N, int K, int nb) {
+// Rows (not slabs) have 256 x 128 tiles between the two, in slices of any number of k tiles, where one round holds them all: before / with the
+// slices it picks, 2331 x 768 x 9216 44.9 / 41.3 (4), 4096 73.8 / 62.4 (2), 1800 40.4 / 36.4 (5), 3200 56.9 / 51.8 (3), 1000 x 2048 x 24576
+// 101.6 / 88.5 (4), 700 75.1 / 70.0 (5).  A k tile of 64 takes 0.55 us in a nearly empty round, 0.66 in a full one, and 0.9 through more than 128 of
+// them (4096 x 2048 x 24576 349 in one piece; 300 in two slices of large tiles), the joining launch 3 and 6 TB/s behind these.
+enum TileKind { SMALL, LARGE, HALF };
+struct SlicePlan { int count; TileKind on; };
+SlicePlan slice_plan(int M, int N, int K, int nb, bool rows) {
   const int before = fstu_gemm_bf16_slices(M, N, K, nb);
-  if (M < 256 || N % 4 != 0 || K % 64 != 0 || K < 2048) return {before, false};
+  if (M < 256 || N % 4 != 0 || K % 64 != 0 || K < 2048) return {before, SMALL};
   const long long cus = gemm_cus();
   const long long small = tiles_of(128, M, N) * nb, big = tiles_of(256, M, N) * nb;
   const int nkt = K / 64;
@@ -1027,27 +1186,41 @@ SlicePlan slice_plan(int M, int N, int K, int nb) {
     const long long rounds = (small * s + 2 * cus - 1) / (2 * cus);
     return rounds * (nkt / s) * (0.55 + (s == 1 ? 0.5 : 0.35) * (double)(small * s) / (double)(rounds * 2 * cus)) + join(s);
   };
-  double least = 0.95 * (before == 1 && 9 * ((big + cus - 1) / cus) * cus < 4 * small ? large(1) : little(before));
-  SlicePlan best = {before, false};
+  const bool whole_large = before == 1 && 9 * ((big + cus - 1) / cus) * cus < 4 * small;
+  double least = 0.95 * (whole_large ? large(1) : little(before));
+  SlicePlan best = {before, SMALL};
   for (int s = 2; s <= 32 && K / s >= 512 && big * s <= 2 * cus; ++s) {
     if (nkt % s != 0) continue;
     const double us = large(s);
-    if (us < least) { least = us; best = {s, true}; }
+    if (us < least) { least = us; best = {s, LARGE}; }
+  }
+  const long long halves = (long long)((M + 255) / 256) * ((N + 127) / 128);
+  if (!rows || best.on != SMALL || halves > cus) return best;
+  // (what the products that it is compared with take, a little closer than to rank them among each other)
+  const double full = (double)(small * before) / (double)cus;
+  least = 0.93 * (whole_large ? large(1) : small * before > cus ? 0.93 * little(before) : 4.0 + nkt / before * (0.43 + 0.12 * full * full) + join(before));
+  for (int s = half_takes(M, N) ? 1 : 2; s <= 32 && (s == 1 || nkt / s >= 16) && halves * s <= cus; ++s) {
+    const double f = (double)(halves * s) / (double)cus;
+    const int n = (nkt + s - 1) / s;
+    const double us = 5.0 + n * (0.55 + 0.11 * f + (n > 128 ? 0.25 * f * f * f * f : 0.0)) + (s == 1 ? 0.0 : 3.0 + 8e-6 / 6.0 * s * (double)M * N);
+    if (us < least) { least = us; best = {s, HALF}; }
   }
   return best;
 }
 
 }  // namespace
 
-extern "C" int fstu_gemm_bf16_row_slices(int M, int N, int K) { return slice_plan(M, N, K, 1).count; }
+extern "C" int fstu_gemm_bf16_row_slices(int M, int N, int K) { return slice_plan(M, N, K, 1, true).count; }
 extern "C" int fstu_gemm_bf16_slab_slices(int M, int N, int K, int nbatch) {
-  return M % 256 == 0 ? slice_plan(M, N, K, nbatch).count : fstu_gemm_bf16_slices(M, N, K, nbatch);
+  return M % 256 == 0 ? slice_plan(M, N, K, nbatch, false).count : fstu_gemm_bf16_slices(M, N, K, nbatch);
 }
 
-extern "C" int fstu_gemm_bf16_splitk(const void* A, int64_t lda, const void* W, float* partial, int M, int N, int K, int ksplit,
-                                     void* stream) {
+// planned: the slices are those that slice_plan picks, which need not be of one length
+static int gemm_splitk(const void* A, int64_t lda, const void* W, float* partial, int M, int N, int K, int ksplit, bool planned, void* stream) {
   FSTU_REQUIRE(A && W && partial, FSTU_ENULL, "fstu_gemm_bf16_splitk: null pointer");
-  FSTU_REQUIRE(ksplit >= 1 && ksplit <= 64 && K % (64 * ksplit) == 0, FSTU_ESHAPE,
+  const SlicePlan plan = slice_plan(M, N, K, 1, true);
+  const bool as_planned = plan.count == ksplit && M > 32, half = planned && as_planned && plan.on == HALF;
+  FSTU_REQUIRE(ksplit >= 1 && ksplit <= 64 && (half || K % (64 * ksplit) == 0), FSTU_ESHAPE,
                "fstu_gemm_bf16_splitk: K=%d must be a multiple of 64*ksplit (ksplit=%d, 1..64)", K, ksplit);
   FSTU_REQUIRE(M >= 1 && N >= 4 && N % 4 == 0 && lda >= K && lda % 8 == 0, FSTU_ESHAPE,
                "fstu_gemm_bf16_splitk: M=%d N=%d (N %% 4 == 0) lda=%lld", M, N, (long long)lda);
@@ -1056,9 +1229,9 @@ extern "C" int fstu_gemm_bf16_splitk(const void* A, int64_t lda, const void* W, 
   FSTU_REQUIRE(lda < GM_MAX_LD && K < GM_MAX_LD, FSTU_ESHAPE, "fstu_gemm_bf16_splitk: lda=%lld / K=%d beyond the 32-bit tile offsets",
                (long long)lda, K);
   int rc;
-  const SlicePlan plan = slice_plan(M, N, K, 1);
   if (M <= 32) rc = gemm_launch_tile<TileRows32, 3>(A, lda, W, nullptr, nullptr, 0, partial, N, M, N, K, (hipStream_t)stream, ksplit);
-  else if (plan.large && plan.count == ksplit)
+  else if (half) rc = gemm_half_launch<3>(A, lda, W, nullptr, 0, partial, N, M, N, K, (hipStream_t)stream, ksplit);
+  else if (as_planned && plan.on == LARGE)
     rc = gemm_pp_launch<3>(A, lda, W, nullptr, nullptr, 0, partial, N, M, N, K, (hipStream_t)stream, ksplit);
   else if ((long long)((M + 127) / 128) * ((N + 127) / 128) * ksplit <= gemm_cus())
     rc = gemm_launch_tile<TileDeep, 3>(A, lda, W, nullptr, nullptr, 0, partial, N, M, N, K, (hipStream_t)stream, ksplit);
@@ -1066,6 +1239,10 @@ extern "C" int fstu_gemm_bf16_splitk(const void* A, int64_t lda, const void* W, 
   if (rc) return rc;
   FSTU_CHECK_LAUNCH("fstu_gemm_bf16_splitk");
   return FSTU_OK;
+}
+extern "C" int fstu_gemm_bf16_splitk(const void* A, int64_t lda, const void* W, float* partial, int M, int N, int K, int ksplit,
+                                     void* stream) {
+  return gemm_splitk(A, lda, W, partial, M, N, K, ksplit, false, stream);
 }
 
 // fp32 slices (ns, nb, M, N) added in order -> C[b] = T(sum), or T(R[b] + T(sum)): bound by the slices' bytes
@@ -1115,7 +1292,7 @@ extern "C" int fstu_gemm_bf16_head_rows(int M, int N, int K) {
   const long long head = tiles / cus * cus / nt * 256;
   if (head <= 0 || head >= M) return 0;
   const long long left = (M - head + 127) / 128 * ((N + 127) / 128);
-  if (left <= (K < 2048 ? cus / 2 : cus) || slice_plan((int)(M - head), N, K, 1).large) return (int)head;
+  if (left <= (K < 2048 ? cus / 2 : cus) || slice_plan((int)(M - head), N, K, 1, true).on != SMALL) return (int)head;
   return 0;
 }
 
@@ -1140,7 +1317,7 @@ extern "C" int fstu_gemm_bf16_ws(const void* A, int64_t lda, const void* W, cons
   int rc;
   if (ksplit > 1) {
     FSTU_REQUIRE(mode != 1 && ldc % 4 == 0 && fstu_aligned(C, 8), FSTU_ESHAPE, "fstu_gemm_bf16_ws: slices in modes 0 and 2, ldc %% 4 == 0");
-    rc = fstu_gemm_bf16_splitk(A, lda, W, partial, M, N, K, ksplit, stream);
+    rc = gemm_splitk(A, lda, W, partial, M, N, K, ksplit, true, stream);
     if (rc) return rc;
     return fstu_join_slices(partial, ksplit, mode == 2 ? R : nullptr, ldr, 0, C, ldc, 0, 1, M, N, stream);
   }
@@ -1191,8 +1368,8 @@ extern "C" int fstu_gemm_bf16_ta_ws(const void* A, int64_t lda, int64_t batch_st
   int rc;
   if (ksplit > 1) {
     if ((rc = split_check("fstu_gemm_bf16_ta_ws", N, K, ksplit, partial))) return rc;
-    const SlicePlan plan = slice_plan(M, N, K, nbatch);
-    if (M % 256 == 0 && plan.large && plan.count == ksplit)
+    const SlicePlan plan = slice_plan(M, N, K, nbatch, false);
+    if (M % 256 == 0 && plan.on == LARGE && plan.count == ksplit)
       rc = gemm_pp_launch<3, true>(A, lda, W, nullptr, nullptr, 0, partial, N, M, N, K, s, ksplit * nbatch, batch_stride_a, 0, 0, nbatch);
     else rc = gemm_ta_launch_tile<TileSmall, 3>(A, lda, batch_stride_a, W, partial, 0, 0, C, 0, 0, M, N, K, nbatch, s, ksplit);
     if (rc) return rc;

@@ -453,8 +453,8 @@ int fstu_gemm_any(const void* A, int64_t sam, int64_t sak, const void* W, int64_
 int fstu_gemm_bf16_ta(const void* A, int64_t lda, int64_t batch_stride_a, const void* W, const void* R, int64_t ldr,
                       int64_t batch_stride_r, void* C, int64_t ldc, int64_t batch_stride_c, int M, int N, int K, int nbatch,
                       int mode, void* stream);
-/* Few output tiles and a long K: the same with K in ksplit slices (K % (64*ksplit) == 0, N % 4 == 0, modes 0 and 2), which a
- * second launch adds in order.  fstu_gemm_bf16_slices says how many pay (1: none; nbatch = 1 for fstu_gemm_bf16_ws); partial
+/* Few output tiles and a long K: the same with K in ksplit slices (K % (64*ksplit) == 0, or, in fstu_gemm_bf16_ws, as many as
+ * fstu_gemm_bf16_row_slices says; N % 4 == 0, modes 0 and 2), which a second launch adds in order.  fstu_gemm_bf16_slices says how many pay (1: none; nbatch = 1 for fstu_gemm_bf16_ws); partial
  * holds ksplit * nbatch * M * N floats, 16-byte aligned. */
 int fstu_gemm_bf16_slices(int M, int N, int K, int nbatch);
 /* The same for fstu_gemm_bf16_ws and fstu_gemm_bf16_splitk, and for fstu_gemm_bf16_ta_ws, whose slices also run on the large tiles. */

@@ -418,6 +418,28 @@ def test_gemm_bf16_large_tiles_one_behind_the_other(hip, M, N, K):
         assert bool(out[M:].isnan().all()) and bool(out[:, N:].isnan().all())
 
 
+@pytest.mark.parametrize("M,N,K,slices", [(2049, 2052, 64, 1), (300, 12289, 128, 1), (257, 16380, 192, 1), (4096, 1032, 832, 1), (1300, 516, 6208, None),
+                                          (4000, 772, 5696, None)])
+def test_gemm_bf16_tiles_of_256_rows_by_128_features(hip, M, N, K, slices):
+    """One round of them, whole with one, two, three and more k tiles, and in slices of unequal lengths: plain and residual, nothing read or
+    written behind the rows and the features."""
+    g = gen(M + K)
+    ns = hip.load().fstu_gemm_bf16_row_slices(M, N, K)
+    assert ns == slices if slices else (ns > 1 and (K // 64) % ns)
+    wide = torch.full((M + 1, K + 8), float("nan"), dtype=torch.bfloat16, device="cuda")
+    wide[:M, :K] = dev(torch.randn(M, K, generator=g).bfloat16())
+    A, W = wide[:M, :K], torch.full((N + 1, K), float("nan"), dtype=torch.bfloat16, device="cuda")[:N].copy_(torch.randn(N, K, generator=g))
+    out = torch.full((M + 1, N + 4 + N % 2), float("nan"), dtype=torch.bfloat16, device="cuda")
+    ref = torch.matmul(A.float(), W.float().t().contiguous())     # fp32 on the library: K * 2^-24 of the absolute sum like the kernel's
+    bound = (2 * K + ns) * 2.0 ** -24 * torch.matmul(A.float().abs(), W.float().abs().t().contiguous()) + 2.0 ** -8 * ref.abs()
+    y = hip.gemm(A, W, out=out[:M, :N])
+    assert bool(((y.float() - ref).abs() <= bound).all())
+    assert bool(out[M:].isnan().all()) and bool(out[:, N:].isnan().all())
+    if N % 4 == 0:
+        R = dev(torch.randn(M, N, generator=g).bfloat16())
+        assert torch.equal(hip.gemm(A, W, residual=R, out=R.clone()), (R.float() + y.float()).bfloat16())
+
+
 @pytest.mark.parametrize("K,M,N,slices", [(64, 128, 128, 1), (128, 256, 128, 1), (4160, 128, 384, None), (100, 128, 128, 1), (4131, 256, 128, None), (9280, 768, 768, 7), (2048, 2048, 2048, 1)])
 def test_gemm_bf16_tt(hip, K, M, N, slices):
     """Both operands with the reduction index slowest, whole and in slices of unequal lengths: fp32 sums of exact products stay within
