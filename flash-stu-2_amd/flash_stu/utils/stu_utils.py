@@ -233,7 +233,8 @@ class ApproxUnit(torch.autograd.Function):
     gradients are products: five launches forward and seven backward, none of them a library's, and one node for the host to
     go through (8 x 2048 x 768: as four nodes, two of them library products, the host took longer than the GPU).  phi_e holds the even
     rows of phi as the gradient of m_filters reads them.  Where the gradients are to be differentiated themselves
-    (create_graph=True) they are those of the composed operators."""
+    (create_graph=True) they are those of the composed operators.  No gradient needs the values of m_filters, which may therefore change
+    before the backward pass, as they may behind phi @ m_filters."""
 
     @staticmethod
     def takes(x, phi, m_inputs, m_filters) -> bool:
@@ -253,17 +254,25 @@ class ApproxUnit(torch.autograd.Function):
         x2 = _aligned(x.reshape(-1, x.shape[2]))
         u = _hip.gemm(x2, _hip.transpose(m_inputs[None])[0]).view(*x.shape[:2], m_inputs.shape[1])
         v, taps = _hip.stu_conv_taps_project(phi, m_filters, x.shape[1])
-        ctx.save_for_backward(x, phi, phi_e, m_inputs, m_filters, u, v)
+        ctx.save_for_backward(x, phi, phi_e, m_inputs, u, v)
+        ctx.m_filters = m_filters if ctx.needs_input_grad[4] else None
+        ctx.version = m_filters._version if ctx.needs_input_grad[4] else 0
         return _hip.stu_conv_mfma(u, taps)
 
     @staticmethod
     def backward(ctx, gy):
         from .. import _hip
-        x, phi, phi_e, m_inputs, m_filters, u, v = ctx.saved_tensors
+        x, phi, phi_e, m_inputs, u, v = ctx.saved_tensors
         want_x, _, _, want_i, want_f = ctx.needs_input_grad
         if torch.is_grad_enabled():
+            filt, m_filters = v, ctx.m_filters
+            if want_f:
+                if m_filters._version != ctx.version and m_filters.grad_fn is not None:
+                    raise RuntimeError("m_filters was modified in place by an operation that its gradient's own graph would run through")
+                now = phi[:v.shape[0]] @ m_filters
+                filt = v + (now - now.detach())          # the forward pass's values, on the way to m_filters
             wanted = [t for t, w in ((x, want_x), (m_inputs, want_i), (m_filters, want_f)) if w]
-            grads = iter(torch.autograd.grad(ApproxConvolveSum.apply(x @ m_inputs, phi @ m_filters), wanted, gy, create_graph=True))
+            grads = iter(torch.autograd.grad(ApproxConvolveSum.apply(x @ m_inputs, filt), wanted, gy, create_graph=True))
             return next(grads) if want_x else None, None, None, next(grads) if want_i else None, next(grads) if want_f else None
         gy, gf = _aligned(gy), None
         if want_f:

@@ -281,6 +281,33 @@ def test_training_step_as_one_node(B, T, d, monkeypatch):
     assert all(made)
 
 
+def test_filter_weights_may_change_before_the_backward_pass():
+    """No gradient of first order needs the values of M_filters: an update between the passes leaves the gradients those of the
+    forward pass's weights, bit for bit, and those with a graph of their own within three roundings to bf16 (2^-8 each)."""
+    from flash_stu import STU, FlashSTUConfig
+    B, T, d, L, K = 4, 64, 128, 128, 24
+    g = torch.Generator().manual_seed(5)
+    cfg = FlashSTUConfig(n_embd=d, n_heads=2, n_layers=2, seq_len=L, num_eigh=K, vocab_size=11, torch_dtype=torch.bfloat16)
+    stu = STU(cfg, torch.randn(L, K, generator=g).div(L ** 0.5).bfloat16().cuda(), 256).cuda()
+    mf = (torch.randn(K, d, generator=g) / K ** 0.5).cuda()
+    with torch.no_grad():
+        stu.M_inputs.copy_(torch.randn(d, d, generator=g) / d ** 0.5)
+    x, gy = (torch.randn(B, T, d, generator=g).bfloat16().cuda() for _ in range(2))
+    x.requires_grad_(True)
+    runs = []
+    for update, second in ((False, False), (True, False), (True, True)):
+        with torch.no_grad():
+            stu.M_filters.copy_(mf)
+        y = stu.forward_differentiable(x)
+        if update:
+            with torch.no_grad():
+                stu.M_filters.mul_(-3.0)
+        runs.append(torch.autograd.grad(y, (x, stu.M_inputs, stu.M_filters), gy, create_graph=second))
+    for want, got, graph in zip(*runs):
+        assert torch.equal(got, want)
+        assert float((graph.detach().float() - want.float()).norm()) <= 3 * 2.0 ** -8 * float(want.float().norm())
+
+
 @pytest.mark.parametrize("B,T,d", [(1, 128, 128), (3, 320, 256), (2, 97, 128)])
 def test_input_projection_gradients(B, T, d):
     """x @ M_inputs and its gradients on the matrix-core kernels (and, for rows they do not take, the library's product)
