@@ -33,6 +33,7 @@
 // branches 164 / 181); 4 x 4096 x 2048 210 / 210; 32 x 300 x 2048 106 / 104.
 #include "fstu_common.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace {
@@ -494,15 +495,18 @@ fft_filter_kernel(const T* __restrict__ filt, size_t f_ls, size_t f_cs, cpx* __r
 // Channel c of x at x[b*x_sb + c*x_sc]; the K outputs of a channel (K = 1: per-channel spectra spec[c]; K > 1: a shared
 // bank spec[k]) at y[b*y_sb + k*y_sk + c*y_sc] (and y2 likewise).
 // mode 0: y = T(T(plus) + T(minus));  mode 1: y = T(plus);  mode 2: y = T(plus), y2 = T(minus).
-// NT threads: as many columns as fill the longest transforms' workgroup or, for small grids, one wave or column.
+// NT threads: as many columns as fill the longest transforms' workgroup or, for small grids, one wave or column.  A workgroup takes the
+// filters of its slice of the bank, kper of them (bank_slice); the loop counts from 0, which keeps the registers of the whole bank's (4 x 8192
+// x 1024 2.95 ms; 3.00 from k0 to k1).
 template <typename T, int LOGN, int NT, bool SUM>
 __global__ void __launch_bounds__(NT, 4)
 fft_slab_kernel(const T* __restrict__ x, size_t x_sb, size_t x_sc, const cpx* __restrict__ spec, T* __restrict__ y,
                 T* __restrict__ y2, size_t y_sb, size_t y_sk, size_t y_sc, const cpx* __restrict__ tw, int Tn, int d, int K,
-                int xcd_remap) {
+                int kper, int xcd_remap) {
   extern __shared__ cpx fft_lds[];
   using W = Half<LOGN>;
   constexpr int N = W::N, COLS = NT / W::G;
+  const int k0 = blockIdx.z * kper, nk = min(K - k0, kper);   // the filters of this workgroup's slice
   int bx = blockIdx.x;
   if (xcd_remap) bx = (bx & 7) * (gridDim.x >> 3) + (bx >> 3);
   const int b = blockIdx.y, mycol = threadIdx.x / W::G, u = threadIdx.x % W::G, c = bx * COLS + mycol;
@@ -519,10 +523,10 @@ fft_slab_kernel(const T* __restrict__ x, size_t x_sb, size_t x_sc, const cpx* __
     else if (t < Tn) z[k].x = DT<T>::ld(xp + t);
   }
   fft_forward<LOGN, fine<T, TABLE>()>(col, tw, u, z, xs);
-  const cpx* sp = spec + (K == 1 ? (size_t)min(c, d - 1) * (2 * N) : 0) + 2 * u;
-  T* yp = y + (size_t)b * y_sb + (size_t)c * y_sc;
-  T* yp2 = y2 + (size_t)b * y_sb + (size_t)c * y_sc;
-  for (int k = 0; k < K; ++k, sp += 2 * N, yp += y_sk, yp2 += y_sk) {
+  const cpx* sp = spec + (size_t)(K == 1 ? min(c, d - 1) : k0) * (2 * N) + 2 * u;
+  T* yp = y + (size_t)b * y_sb + (size_t)k0 * y_sk + (size_t)c * y_sc;
+  T* yp2 = y2 + (size_t)b * y_sb + (size_t)k0 * y_sk + (size_t)c * y_sc;
+  for (int k = 0; k < nk; ++k, sp += 2 * N, yp += y_sk, yp2 += y_sk) {
     cpx v[16], e[8], o[8];
     float prev[8];
     product16<LOGN>(sp, xs, v);
@@ -1083,6 +1087,24 @@ extern "C" int fstu_stu_fft_filter(const void* filt, int64_t f_ls, int64_t f_cs,
   return FSTU_OK;
 }
 
+// Filters to a slice of a bank of time-major slabs, whose channels and rows alone make `waves` waves.  Below one round of the chip (1024
+// SIMDs of four waves) a transform is bound by its own chain of exchanges: it takes 2.3 + 0.7 times the waves on its SIMD (in us: 1.8 at
+// less than one, 2.8 at one, 5.2 at four, bf16), so slices that fill the SIMDs pay for their one forward transform beside the two inverse
+// ones of each filter; a round and more gains nothing (4 x 2000 x 768 398 / 407 in one / two slices, 3 x 6000 x 768 1419 / 1452).  24
+// filters, both branches, bf16, us with the whole bank to a workgroup / in slices: 1 x 64 x 256 68 / 7.8, 1 x 300 x 768 88 / 27, 4 x 250 x 1024
+// 102 / 58, 1 x 1000 x 1024 138 / 67, 3 x 700 x 768 161 / 134, 1 x 4000 x 256 142 / 73, 2 x 2000 x 512 143 / 126, 1 x 8000 x 256 216 / 176.
+static int bank_slice(int K, long long waves) {
+  if (waves >= 4096) return K;
+  int best = K;
+  long long least = -1;
+  for (int kper = (K + 65534) / 65535; kper <= K; ++kper) {
+    const long long w = waves * ((K + kper - 1) / kper), rest = w % 4096;
+    const long long cost = (2 * kper + 1) * (w / 4096 * 51 * 1024 + (rest ? 23 * 1024 + 7 * rest : 0));
+    if (least < 0 || cost < least) { least = cost; best = kper; }
+  }
+  return best;
+}
+
 static int conv_fft_launch(const char* name, const void* x, int64_t x_sb, int64_t x_st, int64_t x_sc, const float* spec,
                            void* y, void* y2, int64_t y_sb, int64_t y_st, int64_t y_sk, int64_t y_sc, const float* tw,
                            int B, int T_, int d, int K, int n, int mode, int dtype, void* stream) {
@@ -1115,12 +1137,13 @@ static int conv_fft_launch(const char* name, const void* x, int64_t x_sb, int64_
     const int g = n / 32, many = g >= 512 ? 1 : 512 / g, few = g >= 64 ? 1 : 64 / g;
     const bool narrow = (long long)((d + many - 1) / many) * B < 512;
     const int gx = narrow ? (d + few - 1) / few : (d + many - 1) / many;
-    dim3 grid(gx, B);
+    const int kper = bank_slice(K, (long long)gx * B * (narrow ? std::max(1, g / 64) : 8));
+    dim3 grid(gx, B, (K + kper - 1) / kper);
     const int remap = (gx % 8 == 0) ? 1 : 0;
     FSTU_DISPATCH_DTYPE(dtype, name,
                         FFT_LAUNCH(logn - 1, FFT_SLAB, grid, name, (const T*)x, (size_t)x_sb, (size_t)x_sc, (const cpx*)spec, (T*)y,
                                    mode == 2 ? (T*)y2 : (T*)nullptr, (size_t)y_sb, (size_t)y_sk, (size_t)y_sc, (const cpx*)tw, T_,
-                                   d, K, remap));
+                                   d, K, kper, remap));
     FSTU_CHECK_LAUNCH(name);
     return FSTU_OK;
   }

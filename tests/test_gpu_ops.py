@@ -676,6 +676,24 @@ def test_stu_conv_bank_in_slices(hip, dtype, B, T, d, K):
             assert torch.equal(a[..., :d], b.permute(0, 3, 1, 2)) and bool((a[..., d] == 9.0).all())
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("B,T,d,K", [(1, 33, 5, 3), (1, 300, 768, 24), (3, 700, 200, 23), (1, 1025, 256, 24), (2, 8191, 40, 7), (70, 100, 64, 24)])
+def test_stu_conv_bank_slabs_in_slices(hip, dtype, B, T, d, K):
+    """The filter bank into time-major slabs, one filter, several and all of them to a workgroup and a last slice that is shorter: the same
+    bits as each filter with its neighbour in a bank of their own; nothing is written beside."""
+    g = gen(T + K)
+    x, phi = dev(torch.randn(B, d, T, generator=g).to(dtype)), dev((torch.randn(T, K, generator=g) / math.sqrt(T)).to(dtype))
+    spec = hip.stu_fft_filter(phi, hip.fft_length(T))
+    u = [torch.full((B, K + 1, d, T), 9.0, dtype=dtype, device="cuda") for _ in range(2)]
+    hip.stu_conv_bank_fft(x.transpose(1, 2), spec, *(t[:, :K].permute(0, 3, 1, 2) for t in u))
+    for k in range(K - 1):
+        pair = [torch.empty(B, 2, d, T, dtype=dtype, device="cuda") for _ in u]
+        hip.stu_conv_bank_fft(x.transpose(1, 2), spec[k:k + 2], *(t.permute(0, 3, 1, 2) for t in pair))
+        for a, b in zip(u, pair):
+            assert torch.equal(a[:, k:k + 2], b)
+    assert all(bool((t[:, K] == 9.0).all()) for t in u)
+
+
 def test_stu_conv_fft_equals_direct_fp32(hip):
     """Both forms of the library on the same input: equal to fp32 round-off, and a delta returns the filter."""
     g = gen(21)
