@@ -14,6 +14,7 @@
 // Weights are given transposed (B^T (S,d_in), C^T (d_out,S)) so that every MFMA fragment is one 16-byte piece; both
 // travel through LDS so that the four waves of a workgroup share one fetch.
 #include "fstu_common.h"
+#include <algorithm>
 #include <type_traits>
 
 namespace {
@@ -64,18 +65,24 @@ __device__ __forceinline__ void store16(bf16_t* p, uint4 v) {
 // group of features for every row (340), the scans left out (322).  With whole lines of x to a load (half a line of twice as many
 // rows before) 327 / 322, state 128 304 / 298.
 //
+// Fewer blocks than compute units: a group of 64 output features takes 1.1 us, one behind the other (16 of the 38 us of a call on one block of
+// 1024 features, state 128), so as many workgroups as there are compute units for form the same U and states and a slice of the features
+// each; the first one publishes.  A second one on a compute unit loses more (three times).  us, one / slices: 128 x 1 x 1024, state 128, 37.9 / 22.5,
+// 3000 x 1 x 1024, 160, 45.8 / 30.2, 3000 x 3 x 1024, 128, 41.2 / 32.0, 4096 x 4 x 1024, 160, 48.1 / 40.4, 1000 x 8 x 512, 64, 20.7 / 17.7; where
+// there are no compute units for a second slice 4096 x 6 x 1024, 160, 47.5 / 52.4.
+//
 // PAST: the outputs leave past the L2s, where they are more than those hold (32 MB): what they would push out are the weights
 // that every workgroup fetches again, and the next kernel would not find them there.
 template <int NT, bool PAST>
 __global__ void __launch_bounds__(256, NT <= 10 ? 2 : 1)   // beyond S = 160 one workgroup fills the LDS anyway
 lds_seq_kernel(const bf16_t* x, const float* __restrict__ A, const bf16_t* BmT, const bf16_t* CmT, bf16_t* y, const float* __restrict__ h0,
                float* __restrict__ hnew, unsigned long long* __restrict__ etag, unsigned* __restrict__ status, unsigned tag,
-               int T, int Bt, int d_in, int d_out, int nblk) {
+               int T, int Bt, int d_in, int d_out, int nblk, int slices, int width) {
   constexpr int S = 16 * NT;
   extern __shared__ __align__(16) float Us[];       // LSQ_TB x S
   auto uslot = [](int row, int slot) { return slot ^ ((row >> 1) & 7); };   // 16-byte slot of a row (S/4 slots, a multiple of 8)
   // rows of the batch first: the blocks in front of a workgroup's are then long through when it asks for their states
-  const int blk = (int)(blockIdx.z * gridDim.y + blockIdx.y), b = blockIdx.x;
+  const int blk = (int)(blockIdx.z * gridDim.y + blockIdx.y), b = blockIdx.x / slices, slice = blockIdx.x % slices;
   if (blk >= nblk) return;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, r = lane & 15, g = lane >> 4;
   const int t0 = blk * LSQ_TB;
@@ -204,8 +211,8 @@ lds_seq_kernel(const bf16_t* x, const float* __restrict__ A, const bf16_t* BmT, 
       for (; p < nvalid; ++p) e = fmaf(a, e, *at(p));
     }
     const size_t rowbase = (size_t)b * nblk * S;
-    __hip_atomic_store(etag + rowbase + (size_t)blk * S + tid, ((unsigned long long)tag << 32) | __float_as_uint(e),
-                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (slice == 0) __hip_atomic_store(etag + rowbase + (size_t)blk * S + tid, ((unsigned long long)tag << 32) | __float_as_uint(e),
+                                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     // 2: the state that enters this block (every block in front of it is a full one)
     const double ad = (double)a;
     const float ap_full = (float)pow(ad, (double)LSQ_TB);
@@ -232,7 +239,7 @@ lds_seq_kernel(const bf16_t* x, const float* __restrict__ A, const bf16_t* BmT, 
         if (j0 + i < blk) h = fmaf(ap_full, h, __uint_as_float((unsigned)wv[i]));
     }
     if (timed_out) atomicOr(status, 1u);
-    if (blk == nblk - 1) {
+    if (blk == nblk - 1 && slice == 0) {
       const float ap = nvalid == LSQ_TB ? ap_full : (float)pow(ad, (double)nvalid);
       hnew[(size_t)b * S + tid] = fmaf(ap, h, e);
     }
@@ -281,6 +288,9 @@ lds_seq_kernel(const bf16_t* x, const float* __restrict__ A, const bf16_t* BmT, 
     // that lane (r, g) ends up with features 8g .. 8g+7 of position r, and lanes r and r ^ 8 swap pieces, so that
     // they hold the two halves of a line of 64 features.
     const int trow = t0 + 32 * w + (r & 7), fcol = 32 * (r >> 3) + 8 * g;
+    const int of = slice * width, dn = min(width, d_out - of);   // the features of this workgroup's slice
+    CmT += (size_t)of * S;
+    y += of;
     bf16_t* yr[4];                                           // position trow + 8 q
 #pragma unroll
     for (int q = 0; q < 4; ++q) yr[q] = y + ((size_t)min(trow + 8 * q, T - 1) * Bt + b) * d_out + fcol;
@@ -292,7 +302,7 @@ lds_seq_kernel(const bf16_t* x, const float* __restrict__ A, const bf16_t* BmT, 
     unsigned char* cst = (unsigned char*)Us;
     constexpr unsigned RS = S * 2u + 16u, cstage = 64u * RS;
     constexpr int PPR = S / 8;                               // 16-byte pieces per row; a stage's lie in memory one after the other
-    const int npiece = d_out * PPR;
+    const int npiece = dn * PPR;
     unsigned cdst[WPT];
 #pragma unroll
     for (int i = 0; i < WPT; ++i) {
@@ -348,16 +358,16 @@ lds_seq_kernel(const bf16_t* x, const float* __restrict__ A, const bf16_t* BmT, 
         for (int m = 0; m < 2; ++m) {
           const uint4 other = swap8(r < 8 ? pc[m][1] : pc[m][0]);
           const uint4 lo = r < 8 ? pc[m][0] : other, hi = r < 8 ? other : pc[m][1];
-          if (decltype(whole)::value || (o0 + fcol < d_out && trow + 16 * m < T)) store16<PAST>(yr[2 * m] + o0, lo);
-          if (decltype(whole)::value || (o0 + fcol < d_out && trow + 16 * m + 8 < T)) store16<PAST>(yr[2 * m + 1] + o0, hi);
+          if (decltype(whole)::value || (o0 + fcol < dn && trow + 16 * m < T)) store16<PAST>(yr[2 * m] + o0, lo);
+          if (decltype(whole)::value || (o0 + fcol < dn && trow + 16 * m + 8 < T)) store16<PAST>(yr[2 * m + 1] + o0, hi);
         }
         __syncthreads();
-        return (o0 += 64) < d_out;
+        return (o0 += 64) < dn;
       };
       while (pass(cb) && pass(ca)) {
       }
     };
-    if (nvalid == LSQ_TB && d_out % 64 == 0) outputs(std::true_type{});
+    if (nvalid == LSQ_TB && dn % 64 == 0) outputs(std::true_type{});
     else outputs(std::false_type{});
   }
 }
@@ -423,11 +433,18 @@ static int lds_sequence(float* h, const void* x, const float* A, const void* Bm,
   const size_t shm = (size_t)LSQ_TB * S * sizeof(float);
   hipStream_t s = (hipStream_t)stream;
   const unsigned ny = nblk < 32768 ? (unsigned)nblk : 32768u;
-  const dim3 grid((unsigned)Bt, ny, ((unsigned)nblk + ny - 1) / ny);
+  // Slices of the output features where there are fewer blocks than compute units (see the kernel); not where y is written over x, which the
+  // other slices of a block may still have to read.
+  const size_t xb = (size_t)T * Bt * d_in * sizeof(bf16_t), yb = (size_t)T * Bt * d_out * sizeof(bf16_t);
+  const bool apart = (const char*)y + yb <= (const char*)x || (const char*)x + xb <= (const char*)y;
+  const long long most_slices = fstu_cus() / ((long long)nblk * Bt);
+  const int groups = (d_out + 63) / 64, want = apart ? (int)std::min<long long>(std::max(most_slices, 1ll), groups) : 1;
+  const int width = 64 * ((groups + want - 1) / want), slices = (d_out + width - 1) / width;
+  const dim3 grid((unsigned)Bt * slices, ny, ((unsigned)nblk + ny - 1) / ny);
   const size_t nwords = (size_t)nblk * BtS;
   unsigned cgrid = (unsigned)((nwords + 255) / 256);
   if (cgrid > 1024u) cgrid = 1024u;
-  const bool past = (size_t)T * Bt * d_out * sizeof(bf16_t) > (size_t)32 << 20;
+  const bool past = yb > (size_t)32 << 20;
   int rc = FSTU_OK;
   auto run = [&](auto which) {                          // (a type for each kernel: a record of its own)
     constexpr auto kernel = decltype(which)::value;
@@ -436,7 +453,7 @@ static int lds_sequence(float* h, const void* x, const float* A, const void* Bm,
     hipLaunchKernelGGL(lds_seq_prepare_kernel, dim3(nt + cgrid), dim3(256), 0, s, etag, nwords, status, (const float*)h, h0, (int)BtS, (const bf16_t*)Bm,
                        (const bf16_t*)Cm, (bf16_t*)wt, d_in, S, d_out, nb, nt);
     hipLaunchKernelGGL(kernel, grid, dim3(256), shm, s, (const bf16_t*)x, A, (const bf16_t*)BmT, (const bf16_t*)CmT, (bf16_t*)y,
-                       (const float*)h0, h, etag, status, 1u, T, Bt, d_in, d_out, nblk);
+                       (const float*)h0, h, etag, status, 1u, T, Bt, d_in, d_out, nblk, slices, width);
   };
 #define LSQ_RUN(...) run(std::integral_constant<decltype(&lds_seq_kernel<__VA_ARGS__>), lds_seq_kernel<__VA_ARGS__>>{})
 #define LSQ_CASE(n) case 32 * n: past ? LSQ_RUN(2 * n, true) : LSQ_RUN(2 * n, false); break

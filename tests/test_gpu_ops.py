@@ -1810,6 +1810,25 @@ def test_lds_sequence_from_weights_as_they_lie(hip, T, Bt, din, S, dout):
     assert torch.equal(y1, y2) and torch.equal(h1, h2) and not torch.equal(h1, h0)
 
 
+@pytest.mark.parametrize("T,S,d", [(1, 32, 80), (128, 160, 1024), (260, 64, 208), (129, 256, 320)])
+def test_lds_sequence_in_slices_of_features(hip, T, S, d):
+    """A row alone, its features in slices, against the same row in a batch that fills the chip, whole: the same bits, also where y is
+    written over x."""
+    g, rows = gen(17), 300
+    A, h0 = dev(0.9 + 0.099 * torch.rand(S, generator=g)), dev(torch.randn(rows, S, generator=g))
+    Bm, Cm, x = (dev((torch.randn(*s, generator=g) / s[0] ** 0.5).bfloat16()) for s in ((d // 32 * 32, S), (S, d), (T, rows, d // 32 * 32)))
+    h = h0.clone()
+    y = hip.lds_steps(h, x, A, Bm, Cm, check_status=True)
+    for r in (0, rows - 1):
+        hr, xr = h0[r:r + 1].clone(), x[:, r:r + 1].contiguous()
+        around = torch.full((T * d + 8,), 7.0, dtype=torch.bfloat16, device="cuda")
+        yr = hip.lds_steps(hr, xr, A, Bm, Cm, out=around[4:-4].view(T, 1, d), check_status=True)
+        assert torch.equal(yr, y[:, r:r + 1]) and torch.equal(hr, h[r:r + 1])
+        assert bool((around[:4] == 7).all()) and bool((around[-4:] == 7).all())
+        if xr.shape == yr.shape:
+            assert torch.equal(hip.lds_steps(h0[r:r + 1].clone(), xr, A, Bm, Cm, out=xr, check_status=True), y[:, r:r + 1])
+
+
 def test_argument_errors_do_not_launch(hip):
     x = torch.zeros(17, 64, dtype=torch.bfloat16, device="cuda")
     W = torch.zeros(32, 64, dtype=torch.bfloat16, device="cuda")
