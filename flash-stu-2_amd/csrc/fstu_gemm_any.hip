@@ -101,20 +101,22 @@ gemm_any_split_kernel(const T* __restrict__ A, long long sam, long long sak, con
   }
 }
 
-// Many output tiles: a workgroup of 4 waves owns 128 rows x 128 features, a wave 64 x 64 on v_mfma_f32_32x32x2_f32; K runs
-// in tiles of 16 through two LDS buffers, the next tile's loads in flight while this one is multiplied.  A k step of a
-// wave is 4 LDS reads for 4 matrix instructions of 64 cycles.  Bound by the fp32 matrix rate.
-#define GA_B 128
+// Many output tiles: a workgroup of 4 waves owns B rows x B features, B = 128 or 64, a wave B/2 x B/2 on v_mfma_f32_32x32x2_f32; K runs
+// in tiles of 16 through two LDS buffers, the loads of the next two tiles in flight while one is multiplied; of one where the large tile
+// reads an operand element by element, whose registers would cost it a workgroup on the compute unit (1000 x 12288 x 3072 with both
+// so 811 us, two ahead 890).  A k step of a wave is B/32 LDS reads for (B/64)^2 matrix instructions of 64 cycles.  Bound by the fp32
+// matrix rate.  Both sizes add in the same order.  fp32, us, one ahead / two: 16384 x 2048 x 2048 1154 / 1084 (127 TFLOP/s), 1000 x 12288 x
+// 3072 675 / 612.
 #define GA_BK 16
 #define GA_LD (GA_BK + 1)
 
-// a thread's share (8 elements) of a 128 x 16 tile; threads run along the index whose stride is 1, so loads coalesce
-template <typename T, bool VEC>
-__device__ __forceinline__ void ga_fetch(float (&v)[8], const T* __restrict__ src, long long srow, long long sk, int row0,
+// a thread's share (B / 16 elements) of a B x 16 tile; threads run along the index whose stride is 1, so loads coalesce
+template <typename T, bool VEC, int B>
+__device__ __forceinline__ void ga_fetch(float (&v)[B / 16], const T* __restrict__ src, long long srow, long long sk, int row0,
                                          int nrows, int k0, int K) {
   if constexpr (VEC) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
+    for (int i = 0; i < B / 64; ++i) {
       const int r = (threadIdx.x >> 2) + 64 * i, k = k0 + 4 * (threadIdx.x & 3);
       const floatx4_t t = ga_load4<T, true>(src + (size_t)min(row0 + r, nrows - 1) * srow, 1, k, K);
 #pragma unroll
@@ -122,84 +124,106 @@ __device__ __forceinline__ void ga_fetch(float (&v)[8], const T* __restrict__ sr
     }
   } else {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+    for (int i = 0; i < B / 16; ++i) {
       const int idx = threadIdx.x + 256 * i;
-      const int r = sk == 1 ? idx / GA_BK : idx % GA_B, k = k0 + (sk == 1 ? idx % GA_BK : idx / GA_B);
+      const int r = sk == 1 ? idx / GA_BK : idx % B, k = k0 + (sk == 1 ? idx % GA_BK : idx / B);
       const float x = DT<T>::ld(src + (size_t)min(row0 + r, nrows - 1) * srow + (size_t)(k < K ? k : 0) * sk);
       v[i] = k < K ? x : 0.f;
     }
   }
 }
 
-template <bool VEC>
-__device__ __forceinline__ void ga_put(float (*dst)[GA_LD], const float (&v)[8], long long sk) {
+template <bool VEC, int B>
+__device__ __forceinline__ void ga_put(float (*dst)[GA_LD], const float (&v)[B / 16], long long sk) {
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
+  for (int i = 0; i < B / 16; ++i) {
     if constexpr (VEC) {
       dst[(threadIdx.x >> 2) + 64 * (i >> 2)][4 * (threadIdx.x & 3) + (i & 3)] = v[i];
     } else {
       const int idx = threadIdx.x + 256 * i;
       if (sk == 1) dst[idx / GA_BK][idx % GA_BK] = v[i];
-      else dst[idx % GA_B][idx / GA_B] = v[i];
+      else dst[idx % B][idx / B] = v[i];
     }
   }
 }
 
-template <typename T, bool VA, bool VW>
+template <typename T, bool VA, bool VW, int B>
 __global__ void __launch_bounds__(256)
 gemm_any_tile_kernel(const T* __restrict__ A, long long sam, long long sak, const T* __restrict__ W, long long swn, long long swk,
                      T* __restrict__ C, long long ldc, int M, int N, int K) {
-  __shared__ float xs[2][GA_B][GA_LD], ws[2][GA_B][GA_LD];
+  constexpr int Q = B / 64;
+  constexpr bool AHEAD = B == 64 || (VA && VW);        // two tiles ahead, or one
+  __shared__ float xs[2][B][GA_LD], ws[2][B][GA_LD];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int wm = 64 * (w & 1), wn = 64 * (w >> 1);
-  const int m0 = blockIdx.x * GA_B, n0 = blockIdx.y * GA_B;
+  const int wm = B / 2 * (w & 1), wn = B / 2 * (w >> 1);
+  const int m0 = blockIdx.x * B, n0 = blockIdx.y * B;
   const int l32 = lane & 31, lh = lane >> 5;
-  floatx16_t acc[2][2];
+  floatx16_t acc[Q][Q];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < Q; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int j = 0; j < Q; ++j)
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
-  float av[8], wv[8];
-  ga_fetch<T, VA>(av, A, sam, sak, m0, M, 0, K);
-  ga_fetch<T, VW>(wv, W, swn, swk, n0, N, 0, K);
-  ga_put<VA>(xs[0], av, sak);
-  ga_put<VW>(ws[0], wv, swk);
-  __syncthreads();
-  for (int k0 = 0, b = 0; k0 < K; k0 += GA_BK, b ^= 1) {
-    const bool more = k0 + GA_BK < K;
-    if (more) {
-      ga_fetch<T, VA>(av, A, sam, sak, m0, M, k0 + GA_BK, K);
-      ga_fetch<T, VW>(wv, W, swn, swk, n0, N, k0 + GA_BK, K);
-    }
+  struct Next { float a[B / 16], w[B / 16]; } n1, n2;
+  auto fetch = [&](Next& v, int k0) __attribute__((always_inline)) {
+    ga_fetch<T, VA, B>(v.a, A, sam, sak, m0, M, k0, K);
+    ga_fetch<T, VW, B>(v.w, W, swn, swk, n0, N, k0, K);
+  };
+  auto put = [&](int b, const Next& v) __attribute__((always_inline)) {
+    ga_put<VA, B>(xs[b], v.a, sak);
+    ga_put<VW, B>(ws[b], v.w, swk);
+  };
+  auto multiply = [&](int b) __attribute__((always_inline)) {
     // weights as the A operand (lane: feature l % 32, k = l / 32), activations as the B operand (lane: row l % 32)
 #pragma unroll
     for (int kk = 0; kk < GA_BK; kk += 2) {
-      float x[2], y[2];
+      float x[Q], y[Q];
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
+      for (int i = 0; i < Q; ++i) {
         x[i] = xs[b][wm + 32 * i + l32][kk + lh];
         y[i] = ws[b][wn + 32 * i + l32][kk + lh];
       }
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
+      for (int i = 0; i < Q; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(y[i], x[j], acc[i][j], 0, 0, 0);
+        for (int j = 0; j < Q; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(y[i], x[j], acc[i][j], 0, 0, 0);
     }
-    if (more) {      // the other buffer was last read before the barrier that ended the previous tile
-      ga_put<VA>(xs[b ^ 1], av, sak);
-      ga_put<VW>(ws[b ^ 1], wv, swk);
-    }
+  };
+  fetch(n1, 0);
+  if constexpr (AHEAD) {
+    fetch(n2, GA_BK);
+    put(0, n1);
+    fetch(n1, 2 * GA_BK);
     __syncthreads();
+    int k0 = 0;
+    auto pass = [&](int b, Next& v) __attribute__((always_inline)) {      // v: the tile behind this one
+      multiply(b);
+      put(b ^ 1, v);       // the other buffer was last read before the barrier that ended the previous tile
+      fetch(v, k0 + 3 * GA_BK);                                            // zeros from K on
+      __syncthreads();
+      return (k0 += GA_BK) < K;
+    };
+    while (pass(0, n2) && pass(1, n1)) {
+    }
+  } else {
+    put(0, n1);
+    __syncthreads();
+    for (int k0 = 0, b = 0; k0 < K; k0 += GA_BK, b ^= 1) {
+      const bool more = k0 + GA_BK < K;
+      if (more) fetch(n1, k0 + GA_BK);
+      multiply(b);
+      if (more) put(b ^ 1, n1);
+      __syncthreads();
+    }
   }
   // D: lane l holds row l % 32 and features 8*(e/4) + 4*(l/32) + e%4 of a 32 x 32 tile
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
+  for (int j = 0; j < Q; ++j) {
     const int m = m0 + wm + 32 * j + l32;
     if (m >= M) continue;
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < Q; ++i)
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
         const int f = n0 + wn + 32 * i + 8 * (e >> 2) + 4 * lh + (e & 3);
@@ -208,20 +232,25 @@ gemm_any_tile_kernel(const T* __restrict__ A, long long sam, long long sak, cons
   }
 }
 
-// 0: 16 x 16 tiles, 16 waves along K; 1: 32 x 32 tiles, 8 waves along K; 2: 128 x 128 tiles.  Rows or features that fill at
+// 0: 16 x 16 tiles, 16 waves along K; 1: 32 x 32 tiles, 8 waves along K; 2: 64 x 64 tiles; 3: 128 x 128 tiles.  Rows or features that fill at
 // most half of a large tile stay on 1 (bf16, us on 1 / 2: 17 x 50257 x 256 17 / 41, 64 x 50257 x 256 31 / 46, 100000 x 16 x 768
-// 68 / 227, 100000 x 64 x 256 54 / 89; 100 x 50257 x 768 143 / 128).  The large tile needs more
+// 68 / 227, 100000 x 64 x 256 54 / 89; 100 x 50257 x 768 143 / 128).  A large tile (2, 3) needs more
 // than one workgroup per compute unit before its matrix rate counts (192 tiles: 2000 x 1536 x 1536 141 us on 1, 158 on 2;
 // 512 tiles: 4096 x 2048 x 24 40 us on 1, 33 on 2; 1024: 16384 x 2048 x 2048 1885 on 1, 1153 on 2), the 32 x 32 tile half
 // the chip (16 tiles: 64 x 256 x 3072 13 us on 0, 27 on 1; 80: 300 x 256 x 3072 25 and 30; 256: 1000 x 256 x 3072 49 and 31).
 // One kernel of 64 x 64 tiles with no loads ahead took 228, 525, 500 us for the last three, 283 and 2860 for the first and
 // third, 23 us for 200 x 256 x 256 (now 8), and its sums in one chain were 2.5 to 4 times further from float64 than those
-// of the split kernels.
+// of the split kernels.  Of the two large tiles the one whose rounds over the compute units are shorter, four rounds of the smaller one
+// against 3.5 of the larger (LDS and the operands' second reading: 16384 x 2048 x 2048 1276 us on 2, 1084 on 3; 1024 tiles of 16384 x 1024 x 1024
+// 328 and 296; 378 of 8000 x 768 x 768 103 and 123; 320 of 2500 x 2048 x 2048 198 and 287; 314 of 20000 x 256 x 256 36 and 52).
 static int ga_pick(int M, int N) {
   const long long t128 = (long long)((M + 127) / 128) * ((N + 127) / 128);
   const long long t32 = (long long)((M + 31) / 32) * ((N + 31) / 32);
   if (t32 < 128) return 0;
-  return t128 > 256 && (std::min(M, N) > 64 || N > 65535 * 32) ? 2 : 1;
+  if (t128 <= 256 || (std::min(M, N) <= 64 && N <= 65535 * 32)) return 1;
+  const long long t64 = (long long)((M + 63) / 64) * ((N + 63) / 64), cus = fstu_cus();
+  const long long r128 = (t128 + cus - 1) / cus, r64 = (t64 + cus - 1) / cus;
+  return 115 * r64 < 400 * r128 && (N + 63) / 64 <= 65535 ? 2 : 3;
 }
 
 template <typename T, bool VA, bool VW>
@@ -236,9 +265,13 @@ static void ga_launch(const T* A, long long sam, long long sak, const T* W, long
       hipLaunchKernelGGL((gemm_any_split_kernel<T, VA, VW, 2, 2, 8, 2>), dim3((M + 31) / 32, (N + 31) / 32), dim3(512), 0, s, A, sam,
                          sak, W, swn, swk, C, ldc, M, N, K);
       break;
+    case 2:
+      hipLaunchKernelGGL((gemm_any_tile_kernel<T, VA, VW, 64>), dim3((M + 63) / 64, (N + 63) / 64), dim3(256), 0, s, A, sam, sak, W, swn, swk,
+                         C, ldc, M, N, K);
+      break;
     default:
-      hipLaunchKernelGGL((gemm_any_tile_kernel<T, VA, VW>), dim3((M + 127) / 128, (N + 127) / 128), dim3(256), 0, s, A, sam, sak, W,
-                         swn, swk, C, ldc, M, N, K);
+      hipLaunchKernelGGL((gemm_any_tile_kernel<T, VA, VW, 128>), dim3((M + 127) / 128, (N + 127) / 128), dim3(256), 0, s, A, sam, sak, W, swn,
+                         swk, C, ldc, M, N, K);
   }
 }
 
@@ -254,7 +287,7 @@ extern "C" int fstu_gemm_any(const void* A, int64_t sam, int64_t sak, const void
                    (swk > 0 || K == 1),
                FSTU_ESHAPE, "fstu_gemm_any: strides must be positive (sam=%lld sak=%lld swn=%lld swk=%lld)", (long long)sam,
                (long long)sak, (long long)swn, (long long)swk);
-  FSTU_REQUIRE(N <= 65535 * GA_B, FSTU_ESHAPE, "fstu_gemm_any: N=%d too large", N);
+  FSTU_REQUIRE(N <= 65535 * 128, FSTU_ESHAPE, "fstu_gemm_any: N=%d too large", N);
   // four elements per load: k contiguous, rows on 4-element boundaries, K a whole number of fours
   const size_t quad = dtype == FSTU_BF16 ? 8 : 16;
   const bool va = sak == 1 && K % 4 == 0 && (sam % 4 == 0 || M == 1) && fstu_aligned(A, quad);

@@ -198,6 +198,14 @@ def test_gemm_any_tiles(hip, dtype, M, N, K):
     assert torch.equal(hip.gemm_any(odd, Wd), got)
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("M,N", [(2049, 2111), (4033, 1985)])       # 64 x 64 tiles and 128 x 128
+@pytest.mark.parametrize("K", [1, 16, 31, 36, 64, 84])
+def test_gemm_any_large_tiles(hip, dtype, M, N, K):
+    """The two large tiles with fewer and more tiles of K than are requested ahead, to the same bounds."""
+    test_gemm_any_tiles(hip, dtype, M, N, K)
+
+
 @pytest.mark.parametrize("nb,M,N,K", [(1, 128, 64, 64), (3, 256, 132, 192), (2, 1024, 1024, 1536), (4, 512, 260, 2048),
                                       (1, 4096, 768, 3072)])
 def test_gemm_bf16_transposed_activations(hip, nb, M, N, K):
