@@ -310,23 +310,24 @@ class STU(nn.Module):
         return T >= FFT_MIN_T and _hip.fft_length(T) >= 8192 and (d // (16 // esz)) * B < 512
 
     def _convolve_time_major(self, xt: torch.Tensor, n: int) -> torch.Tensor:
-        """xt (B, d, T): the projected inputs as time-major slabs -> y (B, T, d)."""
-        yt = torch.empty_like(xt)
+        """xt (B, d, T): the projected inputs as time-major slabs, channels and rows of the batch at any strides -> y (B, T, d)."""
+        yt = xt.new_empty(xt.shape)
         _hip.stu_conv_fft_strided(xt.transpose(1, 2), self.filter_spectrum(n), yt.transpose(1, 2),
                                   single_branch=self.use_hankel_L)
         return _hip.transpose(yt)
 
     def _project_time_major(self, x: torch.Tensor) -> Optional[torch.Tensor]:
         """(x @ M_inputs) as time-major slabs (B, d_out, T), formed by the prompt GEMM with its operands swapped
-        (M_inputs^T as the rows, the sequence as the 'weights'), or None where that kernel does not take the shape."""
+        (M_inputs^T as the rows, the sequences as the 'weights'), or None where that kernel does not take the shape.  One product for
+        the whole batch, whose rows lie next to each other in a channel: one per row of the batch filled a part of the compute units each
+        (us a call, so / now: 7 x 2500 x 256 108 / 56, 8 x 5000 x 384 211 / 173, 3 x 6000 x 768 161 / 137)."""
         B, T, d = x.shape
-        w = self.m_inputs_t()
-        if not all(_hip.gemm_supported(w, x[b]) for b in range(B)) or T % 4 != 0:
+        w, x2 = self.m_inputs_t(), x.reshape(B * T, d)
+        if not _hip.gemm_supported(w, x2) or T % 4 != 0:
             return None
-        xt = torch.empty(B, w.shape[0], T, dtype=x.dtype, device=x.device)
-        for b in range(B):
-            _hip.gemm(w, x[b], out=xt[b])
-        return xt
+        xt = torch.empty(w.shape[0], B, T, dtype=x.dtype, device=x.device)
+        _hip.gemm(w, x2, out=xt.view(w.shape[0], B * T))
+        return xt.transpose(0, 1)
 
     def _exact_sequence(self, x: torch.Tensor) -> torch.Tensor:
         """use_approx=False: U+-[b,t,k,i] for the whole filter bank (one forward transform per channel, one

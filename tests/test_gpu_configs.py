@@ -73,6 +73,12 @@ def test_stu_forward_of_a_few_long_sequences_goes_time_major(dtype, B, T, d):
     assert float((y != y2).float().mean()) <= (0.0 if dtype == torch.float32 else 0.02)
 
 
+@pytest.mark.parametrize("B,T,d", [(5, 2052, 96), (3, 4092, 160), (9, 2500, 128)])
+def test_stu_forward_of_several_long_sequences_in_one_product(B, T, d):
+    """Rows of the batch that lie next to each other in a channel's slab, of lengths that are no whole tile, to the same bounds."""
+    test_stu_forward_of_a_few_long_sequences_goes_time_major(torch.bfloat16, B, T, d)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("T", [200, 384, 20])
 def test_c3_exact_mode_ragged_lengths_and_both_dtypes(dtype, T):
