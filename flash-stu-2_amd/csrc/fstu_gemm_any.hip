@@ -232,7 +232,7 @@ gemm_any_tile_kernel(const T* __restrict__ A, long long sam, long long sak, cons
   }
 }
 
-// 0: 16 x 16 tiles, 16 waves along K; 1: 32 x 32 tiles, 8 waves along K; 2: 64 x 64 tiles; 3: 128 x 128 tiles.  Rows or features that fill at
+// 0: 16 x 16 tiles, 16 waves along K; 1: 32 x 32 tiles, 8 waves along K; 4: the same with 64 rows; 2: 64 x 64 tiles; 3: 128 x 128 tiles.  Rows or features that fill at
 // most half of a large tile stay on 1 (bf16, us on 1 / 2: 17 x 50257 x 256 17 / 41, 64 x 50257 x 256 31 / 46, 100000 x 16 x 768
 // 68 / 227, 100000 x 64 x 256 54 / 89; 100 x 50257 x 768 143 / 128).  A large tile (2, 3) needs more
 // than one workgroup per compute unit before its matrix rate counts (192 tiles: 2000 x 1536 x 1536 141 us on 1, 158 on 2;
@@ -243,11 +243,15 @@ gemm_any_tile_kernel(const T* __restrict__ A, long long sam, long long sak, cons
 // of the split kernels.  Of the two large tiles the one whose rounds over the compute units are shorter, four rounds of the smaller one
 // against 3.5 of the larger (LDS and the operands' second reading: 16384 x 2048 x 2048 1276 us on 2, 1084 on 3; 1024 tiles of 16384 x 1024 x 1024
 // 328 and 296; 378 of 8000 x 768 x 768 103 and 123; 320 of 2500 x 2048 x 2048 198 and 287; 314 of 20000 x 256 x 256 36 and 52).
-static int ga_pick(int M, int N) {
+// Tiles of 64 rows fetch three quarters of the bytes to a matrix instruction and need a round of workgroups and more than a few trips of K
+// (4 / 1, fp32: 1000 x 1024 x 1024 28.0 / 32.2, 2000 x 1536 x 1536 106 / 131, 4000 x 512 x 512 31.8 / 32.4; 1000 x 768 x 768, 768 tiles of 32 x 32,
+// 22.3 / 19.7; 8000 x 384 x 384 36.8 / 36.2, 8000 x 256 x 256 20.8 / 18.9, 64 x 50257 x 256 32.3 / 28.2), and no rows that are mostly behind the end.
+static int ga_pick(int M, int N, int K) {
   const long long t128 = (long long)((M + 127) / 128) * ((N + 127) / 128);
   const long long t32 = (long long)((M + 31) / 32) * ((N + 31) / 32);
   if (t32 < 128) return 0;
-  if (t128 <= 256 || (std::min(M, N) <= 64 && N <= 65535 * 32)) return 1;
+  if (t128 <= 256 || (std::min(M, N) <= 64 && N <= 65535 * 32))
+    return t32 >= 1024 && K >= 512 && 16 * ((M + 63) / 64) * (long long)((N + 31) / 32) <= 9 * t32 ? 4 : 1;
   const long long t64 = (long long)((M + 63) / 64) * ((N + 63) / 64), cus = fstu_cus();
   const long long r128 = (t128 + cus - 1) / cus, r64 = (t64 + cus - 1) / cus;
   return 115 * r64 < 400 * r128 && (N + 63) / 64 <= 65535 ? 2 : 3;
@@ -256,13 +260,18 @@ static int ga_pick(int M, int N) {
 template <typename T, bool VA, bool VW>
 static void ga_launch(const T* A, long long sam, long long sak, const T* W, long long swn, long long swk, T* C, long long ldc,
                       int M, int N, int K, hipStream_t s) {
-  switch (ga_pick(M, N)) {
+  switch (ga_pick(M, N, K)) {
     case 0:
       hipLaunchKernelGGL((gemm_any_split_kernel<T, VA, VW, 1, 1, 16, 4>), dim3((M + 15) / 16, (N + 15) / 16), dim3(1024), 0, s, A, sam,
                          sak, W, swn, swk, C, ldc, M, N, K);
       break;
-    case 1:
-      hipLaunchKernelGGL((gemm_any_split_kernel<T, VA, VW, 2, 2, 8, 2>), dim3((M + 31) / 32, (N + 31) / 32), dim3(512), 0, s, A, sam,
+    case 1:        // one group of 16 k requested at a time: more waves on a compute unit cover a trip better than a second group (fp32, us, two / one:
+                   // 1000 x 512 x 512 12.2 / 10.9, 300 x 768 x 768 10.2 / 9.3, 2400 x 256 x 3072 73 / 67, 64 x 50257 x 256 33.0 / 28.2)
+      hipLaunchKernelGGL((gemm_any_split_kernel<T, VA, VW, 2, 2, 8, 1>), dim3((M + 31) / 32, (N + 31) / 32), dim3(512), 0, s, A, sam,
+                         sak, W, swn, swk, C, ldc, M, N, K);
+      break;
+    case 4:
+      hipLaunchKernelGGL((gemm_any_split_kernel<T, VA, VW, 4, 2, 8, 1>), dim3((M + 63) / 64, (N + 31) / 32), dim3(512), 0, s, A, sam,
                          sak, W, swn, swk, C, ldc, M, N, K);
       break;
     case 2:

@@ -206,6 +206,13 @@ def test_gemm_any_large_tiles(hip, dtype, M, N, K):
     test_gemm_any_tiles(hip, dtype, M, N, K)
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("M,N,K", [(1030, 1000, 512), (1030, 1000, 645), (63, 17000, 524), (1985, 545, 1028), (1000, 800, 700)])
+def test_gemm_any_tiles_of_64_rows(hip, dtype, M, N, K):
+    """64 x 32 tiles with the waves along K, ragged rows, features and K, the last size on 32 x 32 tiles, to the same bounds."""
+    test_gemm_any_tiles(hip, dtype, M, N, K)
+
+
 @pytest.mark.parametrize("nb,M,N,K", [(1, 128, 64, 64), (3, 256, 132, 192), (2, 1024, 1024, 1536), (4, 512, 260, 2048),
                                       (1, 4096, 768, 3072)])
 def test_gemm_bf16_transposed_activations(hip, nb, M, N, K):
