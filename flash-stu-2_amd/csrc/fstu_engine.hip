@@ -139,8 +139,8 @@ static inline int stu_pos(int pos) { return g_stu_parity >= 0 ? g_stu_parity : p
 
 // Where several greedy steps follow each other, the reduction of one step's packed maxima (token store, position advance) and
 // the next step's embedding + norm are one launch.  g_chain_prev: this step starts with that launch; g_chain_next:
-// this step's head leaves its maxima for the next step.
-static thread_local bool g_chain_prev = false, g_chain_next = false;
+// this step's head leaves its maxima for the next step.  g_chain_left: a head has left them and no launch has taken them yet.
+static thread_local bool g_chain_prev = false, g_chain_next = false, g_chain_left = false;
 static bool chain_ok(const fstu_model_desc* m, int do_sample) {
   return !do_sample && m->best && fstu_finish_embed_supported(m->B, m->d, m->emb, m->x, m->layers[0].norm1_w, m->h, m->dtype) &&
          (m->dtype == FSTU_BF16 ? fstu_head_argmax_fused_pick(m->h, m->d, m->emb, m->d, m->dtype)
@@ -292,10 +292,11 @@ static int decode_step_impl(const fstu_model_desc* m, const int64_t* tok_in, int
     return decode_step_wide(m, tok_in, tok_out, tok_stride, pos, temperature, top_k, top_p, do_sample, seed, step, dyn, stream);
   // x = embedding rows, h = norm(x) with the first layer's norm weight
   const bool chain = chain_ok(m, do_sample);
-  if (chain && g_chain_prev)      // (the token goes to where this step would read it: column 1 of the position still on the device)
+  if (chain && g_chain_prev) {    // (the token goes to where this step would read it: column 1 of the position still on the device)
     TIMED(PC_NORM, fstu_finish_embed_rmsnorm(m->best, dyn ? tok_out : const_cast<int64_t*>(tok_in), tok_stride, m->emb, m->x,
                                              m->layers[0].norm1_w, m->h, dyn, B, d, m->V, m->eps, dt, stream));
-  else
+    g_chain_left = false;
+  } else
     TIMED(PC_NORM, fstu_embed_rmsnorm(tok_in, tok_stride, m->emb, m->x, m->layers[0].norm1_w, m->h, B, d, m->V, m->eps, dt,
                                       stream, dyn));
   // The residual stream starts in m->x.  Where a layer has packed gate/up weights, its MLP norm runs as the
@@ -434,6 +435,7 @@ static int decode_step_impl(const fstu_model_desc* m, const int64_t* tok_in, int
       TIMED(PC_HEAD, fstu_head_argmax_dyn(m->h, d, m->emb, m->logits, m->V, B, m->V, d, temperature, m->best, tok_out, tok_stride, dyn,
                                           adv, dt, stream));
     }
+    g_chain_left = adv < 0;
   } else if (sample_spread_ok(m, do_sample, top_k)) {
     if (head_packed) TIMED(PC_HEAD, fstu_head_maxima_packed(m->h, d, m->wp_emb, m->logits, m->V, B, m->V, d, temperature, m->best, stream));
     else TIMED(PC_HEAD, fstu_head_maxima(m->h, d, m->emb, m->logits, m->V, B, m->V, d, temperature, m->best, dt, stream));
@@ -456,18 +458,21 @@ extern "C" int fstu_decode_step(const fstu_model_desc* m, const int64_t* tok_in,
 
 // n steps one behind the other on tokens (column 0 the position's own), one launch and one call from the host less a greedy step: 64
 // tokens of one row, 256-d, 4 layers, fp32 5.45 -> 5.12 ms (the host's 24 launches of a step take as long as the GPU's), 128 tokens of
-// 8 rows, 768-d, 12 layers 41.46 -> 41.26.
+// 8 rows, 768-d, 12 layers 41.46 -> 41.26.  Where a step is refused, the pick of the one in front of it is finished all the same: its
+// token is written, and no maxima stay behind for a later call to take with its own.
 extern "C" int fstu_decode_steps(const fstu_model_desc* m, int64_t* tokens, int64_t tok_stride, int pos, int n, float temperature, int top_k,
                                  float top_p, int do_sample, uint64_t seed, int step, void* stream) {
   FSTU_REQUIRE(tokens && n >= 0, FSTU_EARG, "fstu_decode_steps: null pointer or negative count");
   int rc = 0;
+  g_chain_left = false;
   for (int i = 0; i < n && rc == 0; ++i) {
     g_chain_prev = i > 0;
     g_chain_next = i + 1 < n;
     rc = decode_step_impl(m, tokens + i, tokens + i + 1, tok_stride, pos + i, temperature, top_k, top_p, do_sample, seed, step + i, nullptr,
                           stream);
+    if (rc && g_chain_left) fstu_argmax_finish_launch(m->best, tokens + i, tok_stride, m->B, nullptr, 1, stream);
   }
-  g_chain_prev = g_chain_next = false;
+  g_chain_prev = g_chain_next = g_chain_left = false;
   return rc;
 }
 

@@ -650,7 +650,8 @@ int fstu_decode_step(const fstu_model_desc* m, const int64_t* tok_in, int64_t* t
                      int pos, float temperature, int top_k, float top_p, int do_sample, uint64_t seed,
                      int step, void* stream);
 /* n such steps: the token at position pos + i is tokens[b*tok_stride + i], the next one is written behind it, the sampling stream's
- * index is step + i.  A greedy step's pick is finished in the launch that begins the next one. */
+ * index is step + i.  A greedy step's pick is finished in the launch that begins the next one; where a step is refused, the picks of those in
+ * front of it are written all the same. */
 int fstu_decode_steps(const fstu_model_desc* m, int64_t* tokens, int64_t tok_stride, int pos, int n, float temperature, int top_k,
                       float top_p, int do_sample, uint64_t seed, int step, void* stream);
 /* The same step without the pick: the state advances and m->logits holds the (B,V) logits; 1..16 rows. */

@@ -367,6 +367,35 @@ def test_greedy_steps_in_one_call(dtype, B, d):
         assert torch.equal(one, each), n
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_refused_steps_leave_no_pick_behind(dtype):
+    """A step behind the end of the history is refused: the picks of the steps in front of it are written all the same, and nothing of
+    them is left for the next call, which gives the tokens of a fresh descriptor."""
+    from flash_stu import FlashSTU, FlashSTUConfig, _hip
+    B, P, cap = 3, 9, 64
+    torch.manual_seed(4)
+    cfg = FlashSTUConfig(n_embd=64, n_heads=2, n_layers=2, seq_len=cap, window_size=cap, vocab_size=501, num_eigh=8, torch_dtype=dtype,
+                         stu_decode_mode="history")
+    model = FlashSTU(cfg).cuda().eval()
+    with torch.no_grad():
+        model.lm_head.weight.normal_(0.0, 1.0)
+    ids = torch.randint(0, 501, (B, P), generator=torch.Generator().manual_seed(4)).cuda()
+    want = model.generate(ids, max_length=cap, do_sample=False)
+    eng = model.decode_engine()
+    assert eng.desc.hist_cap == cap
+    for n, refused in ((cap - P + 1, True), (cap - P, False)):
+        tokens = torch.zeros(B, cap + 3, dtype=torch.int64, device="cuda")
+        tokens[:, :P + 1] = want[:, :P + 1]
+        how = (tokens, P, n, 1.0, None, None, False, 0, 1)
+        if refused:
+            with pytest.raises(_hip.FlashSTUHipError, match="history capacity"):
+                eng.steps(*how)
+        else:
+            eng.steps(*how)
+        assert torch.equal(tokens[:, :cap], want)
+        assert torch.equal(tokens[:, cap], eng.logits.float().argmax(-1)) and int(tokens[:, cap + 1:].abs().sum()) == 0
+
+
 def _teacher_forced(w, ocfg, tokens, P):
     logits, _ = O.model_forward(w, ocfg, tokens[:, :-1])
     return logits[:, P - 1:, :]          # predictions for positions P..end
