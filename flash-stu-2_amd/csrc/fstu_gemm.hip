@@ -1215,13 +1215,14 @@ extern "C" int fstu_gemm_bf16_slab_slices(int M, int N, int K, int nbatch) {
   return M % 256 == 0 ? slice_plan(M, N, K, nbatch, false).count : fstu_gemm_bf16_slices(M, N, K, nbatch);
 }
 
-// planned: the slices are those that slice_plan picks, which need not be of one length
-static int gemm_splitk(const void* A, int64_t lda, const void* W, float* partial, int M, int N, int K, int ksplit, bool planned, void* stream) {
+// slices as fstu_gemm_bf16_row_slices plans them, which need not be of one length, or any number that divides K's tiles of 64
+extern "C" int fstu_gemm_bf16_splitk(const void* A, int64_t lda, const void* W, float* partial, int M, int N, int K, int ksplit,
+                                     void* stream) {
   FSTU_REQUIRE(A && W && partial, FSTU_ENULL, "fstu_gemm_bf16_splitk: null pointer");
   const SlicePlan plan = slice_plan(M, N, K, 1, true);
-  const bool as_planned = plan.count == ksplit && M > 32, half = planned && as_planned && plan.on == HALF;
+  const bool as_planned = plan.count == ksplit && M > 32, half = as_planned && plan.on == HALF;
   FSTU_REQUIRE(ksplit >= 1 && ksplit <= 64 && (half || K % (64 * ksplit) == 0), FSTU_ESHAPE,
-               "fstu_gemm_bf16_splitk: K=%d must be a multiple of 64*ksplit (ksplit=%d, 1..64)", K, ksplit);
+               "fstu_gemm_bf16_splitk: K=%d must be a multiple of 64*ksplit (ksplit=%d, 1..64), or ksplit that of fstu_gemm_bf16_row_slices", K, ksplit);
   FSTU_REQUIRE(M >= 1 && N >= 4 && N % 4 == 0 && lda >= K && lda % 8 == 0, FSTU_ESHAPE,
                "fstu_gemm_bf16_splitk: M=%d N=%d (N %% 4 == 0) lda=%lld", M, N, (long long)lda);
   FSTU_REQUIRE(fstu_aligned(A, 16) && fstu_aligned(W, 16) && fstu_aligned(partial, 16), FSTU_EALIGN,
@@ -1239,10 +1240,6 @@ static int gemm_splitk(const void* A, int64_t lda, const void* W, float* partial
   if (rc) return rc;
   FSTU_CHECK_LAUNCH("fstu_gemm_bf16_splitk");
   return FSTU_OK;
-}
-extern "C" int fstu_gemm_bf16_splitk(const void* A, int64_t lda, const void* W, float* partial, int M, int N, int K, int ksplit,
-                                     void* stream) {
-  return gemm_splitk(A, lda, W, partial, M, N, K, ksplit, false, stream);
 }
 
 // fp32 slices (ns, nb, M, N) added in order -> C[b] = T(sum), or T(R[b] + T(sum)): bound by the slices' bytes
@@ -1317,7 +1314,7 @@ extern "C" int fstu_gemm_bf16_ws(const void* A, int64_t lda, const void* W, cons
   int rc;
   if (ksplit > 1) {
     FSTU_REQUIRE(mode != 1 && ldc % 4 == 0 && fstu_aligned(C, 8), FSTU_ESHAPE, "fstu_gemm_bf16_ws: slices in modes 0 and 2, ldc %% 4 == 0");
-    rc = gemm_splitk(A, lda, W, partial, M, N, K, ksplit, true, stream);
+    rc = fstu_gemm_bf16_splitk(A, lda, W, partial, M, N, K, ksplit, stream);
     if (rc) return rc;
     return fstu_join_slices(partial, ksplit, mode == 2 ? R : nullptr, ldr, 0, C, ldc, 0, 1, M, N, stream);
   }

@@ -474,10 +474,10 @@ def gemm_tt(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
 
 
 def gemm_splitk(x2: torch.Tensor, weight: torch.Tensor, ksplit: int, partial: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """fp32 partial sums (ksplit, M, N) of x2 (M,K) @ weight (N,K)^T over ksplit slices of K; add_rmsnorm with
-    delta_mode=1, nslices=ksplit folds them into the residual stream."""
+    """fp32 partial sums (ksplit, M, N) of x2 (M,K) @ weight (N,K)^T over ksplit slices of K, as many as fstu_gemm_bf16_row_slices
+    says or a number that divides K / 64; add_rmsnorm with delta_mode=1, nslices=ksplit folds them into the residual stream."""
     _dev(weight, partial)
-    if not gemm_supported(x2, weight) or not x2.is_cuda or x2.shape[1] % (64 * ksplit) != 0:
+    if not gemm_supported(x2, weight) or not x2.is_cuda:
         raise FlashSTUHipError(f"gemm_splitk: unsupported operands {tuple(x2.shape)} x {tuple(weight.shape)} / {ksplit}")
     M, K = x2.shape
     N = weight.shape[0]

@@ -430,7 +430,7 @@ int fstu_gemm_bf16(const void* A, int64_t lda, const void* W, const void* W2, co
 /* The same contraction cut into ksplit slices of K, for a long K with few output tiles (down_proj of a decode step over
  * 17..32 rows, flash_stu/modules/swiglu.py:28): partial (ksplit,M,N) fp32 receives the unrounded slice sums, which
  * fstu_add_rmsnorm (delta_mode 1, nslices = ksplit) adds into the residual stream as T(x + T(sum)).
- * K % (64*ksplit) == 0, ksplit 1..64. */
+ * ksplit 1..64: K % (64*ksplit) == 0, or what fstu_gemm_bf16_row_slices says, whose slices need not be of one length. */
 int fstu_gemm_bf16_splitk(const void* A, int64_t lda, const void* W, float* partial, int M, int N, int K, int ksplit,
                           void* stream);
 
@@ -454,8 +454,8 @@ int fstu_gemm_bf16_ta(const void* A, int64_t lda, int64_t batch_stride_a, const 
                       int64_t batch_stride_r, void* C, int64_t ldc, int64_t batch_stride_c, int M, int N, int K, int nbatch,
                       int mode, void* stream);
 /* Few output tiles and a long K: the same with K in ksplit slices (K % (64*ksplit) == 0, or, in fstu_gemm_bf16_ws, as many as
- * fstu_gemm_bf16_row_slices says; N % 4 == 0, modes 0 and 2), which a second launch adds in order.  fstu_gemm_bf16_slices says how many pay (1: none; nbatch = 1 for fstu_gemm_bf16_ws); partial
- * holds ksplit * nbatch * M * N floats, 16-byte aligned. */
+ * fstu_gemm_bf16_row_slices says; N % 4 == 0, modes 0 and 2), which a second launch adds in order.  fstu_gemm_bf16_slices says how
+ * many pay (1: none; nbatch = 1 for fstu_gemm_bf16_ws); partial holds ksplit * nbatch * M * N floats, 16-byte aligned. */
 int fstu_gemm_bf16_slices(int M, int N, int K, int nbatch);
 /* The same for fstu_gemm_bf16_ws and fstu_gemm_bf16_splitk, and for fstu_gemm_bf16_ta_ws, whose slices also run on the large tiles. */
 int fstu_gemm_bf16_row_slices(int M, int N, int K);

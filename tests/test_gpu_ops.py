@@ -455,6 +455,23 @@ def test_gemm_bf16_tiles_of_256_rows_by_128_features(hip, M, N, K, slices):
         assert torch.equal(hip.gemm(A, W, residual=R, out=R.clone()), (R.float() + y.float()).bfloat16())
 
 
+@pytest.mark.parametrize("M,N,K", [(1300, 516, 6208), (1800, 768, 9216), (700, 2048, 24576), (300, 256, 3072)])
+def test_gemm_splitk_takes_the_slices_that_row_slices_names(hip, M, N, K):
+    """The fp32 sums of as many slices as fstu_gemm_bf16_row_slices says, of unequal lengths too, and nothing behind them."""
+    g = gen(M)
+    ns = hip.load().fstu_gemm_bf16_row_slices(M, N, K)
+    assert ns > 1 and (M != 1300 or (K // 64) % ns)
+    A, W = (dev(torch.randn(n, K, generator=g).bfloat16()) for n in (M, N))
+    room = torch.full((ns * M * N + 8,), float("nan"), device="cuda")
+    hip.gemm_splitk(A, W, ns, partial=room[:ns * M * N].view(ns, M, N))
+    ref = torch.matmul(A.float(), W.float().t().contiguous())     # fp32 on the library: K * 2^-24 of the absolute sum like the kernel's
+    bound = (2 * K + ns) * 2.0 ** -24 * torch.matmul(A.float().abs(), W.float().abs().t().contiguous())
+    assert bool(((room[:ns * M * N].view(ns, M, N).sum(0) - ref).abs() <= bound).all())
+    assert bool(room[ns * M * N:].isnan().all())
+    with pytest.raises(hip.FlashSTUHipError):
+        hip.gemm_splitk(A, W, 5 if (K // 64) % 5 and ns != 5 else 7)
+
+
 @pytest.mark.parametrize("K,M,N,slices", [(64, 128, 128, 1), (128, 256, 128, 1), (4160, 128, 384, None), (100, 128, 128, 1), (4131, 256, 128, None), (9280, 768, 768, 7), (2048, 2048, 2048, 1)])
 def test_gemm_bf16_tt(hip, K, M, N, slices):
     """Both operands with the reduction index slowest, whole and in slices of unequal lengths: fp32 sums of exact products stay within
