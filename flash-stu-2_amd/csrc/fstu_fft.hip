@@ -1105,6 +1105,19 @@ static int bank_slice(int K, long long waves) {
   return best;
 }
 
+// Whether no byte between the first and the last one of y (strides b, t, k, c in elements) lies between those of x.  A bank whose slab is
+// written over x takes no slices: a workgroup that has all filters of its channels reads them before it writes, another slice's may not
+// have read them yet.
+static bool bank_apart(const void* x, const int64_t (&xs)[3], const void* y, const int64_t (&ys)[4], int B, int T_, int K, int d, int esz) {
+  if (!y) return true;
+  const int64_t xn[3] = {B, T_, d}, yn[4] = {B, T_, K, d};
+  int64_t x_lo = 0, x_hi = 1, y_lo = 0, y_hi = 1;
+  for (int i = 0; i < 3; ++i) (xs[i] < 0 ? x_lo : x_hi) += (xn[i] - 1) * xs[i];
+  for (int i = 0; i < 4; ++i) (ys[i] < 0 ? y_lo : y_hi) += (yn[i] - 1) * ys[i];
+  const char *const xb = (const char*)x, *const yb = (const char*)y;
+  return yb + y_hi * esz <= xb + x_lo * esz || xb + x_hi * esz <= yb + y_lo * esz;
+}
+
 static int conv_fft_launch(const char* name, const void* x, int64_t x_sb, int64_t x_st, int64_t x_sc, const float* spec,
                            void* y, void* y2, int64_t y_sb, int64_t y_st, int64_t y_sk, int64_t y_sc, const float* tw,
                            int B, int T_, int d, int K, int n, int mode, int dtype, void* stream) {
@@ -1132,12 +1145,14 @@ static int conv_fft_launch(const char* name, const void* x, int64_t x_sb, int64_
     FSTU_CHECK_LAUNCH(name);
     return FSTU_OK;
   }
+  const int64_t xs[3] = {x_sb, x_st, x_sc}, ys[4] = {y_sb, y_st, y_sk, y_sc};
+  const bool apart = K > 1 && bank_apart(x, xs, y, ys, B, T_, K, d, esz) && bank_apart(x, xs, y2, ys, B, T_, K, d, esz);
   if (x_st == 1 && y_st == 1) {
     // as many columns per workgroup as fill 512 threads, or, where that leaves compute units idle, one wave (or column)
     const int g = n / 32, many = g >= 512 ? 1 : 512 / g, few = g >= 64 ? 1 : 64 / g;
     const bool narrow = (long long)((d + many - 1) / many) * B < 512;
     const int gx = narrow ? (d + few - 1) / few : (d + many - 1) / many;
-    const int kper = bank_slice(K, (long long)gx * B * (narrow ? std::max(1, g / 64) : 8));
+    const int kper = apart ? bank_slice(K, (long long)gx * B * (narrow ? std::max(1, g / 64) : 8)) : K;
     dim3 grid(gx, B, (K + kper - 1) / kper);
     const int remap = (gx % 8 == 0) ? 1 : 0;
     FSTU_DISPATCH_DTYPE(dtype, name,
@@ -1151,7 +1166,7 @@ static int conv_fft_launch(const char* name, const void* x, int64_t x_sb, int64_
   // one / two slices: 4 x 1000 x 768, 384 workgroups, 396 / 409, 1 x 4096 x 512, 256 workgroups, 413 / 529)
   const int gx = (d + cols - 1) / cols;
   const long long groups = (long long)gx * B;
-  const int slices = groups >= 256 ? 1 : (int)(512 / groups), kper = slices >= K ? 1 : (K + slices - 1) / slices;
+  const int slices = groups >= 256 || !apart ? 1 : (int)(512 / groups), kper = slices >= K ? 1 : (K + slices - 1) / slices;
   dim3 grid(gx, B, (K + kper - 1) / kper);
   const int remap = (gx % 8 == 0) ? 1 : 0;
   FSTU_DISPATCH_DTYPE(dtype, name,

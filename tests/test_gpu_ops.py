@@ -694,7 +694,7 @@ def test_stu_conv_toeplitz_product(hip, B, T, d, L):
 @pytest.mark.parametrize("B,T,d,K", [(1, 40, 3, 2), (1, 64, 256, 24), (2, 100, 72, 7), (3, 300, 200, 24), (1, 1000, 256, 24), (40, 33, 256, 5)])
 def test_stu_conv_bank_in_slices(hip, dtype, B, T, d, K):
     """The filter bank into (B,T,K,d): one filter, several and all of them per workgroup, both branches and one, the same bits
-    as the slab kernel's, which runs through the bank in one go; nothing is written beside."""
+    as the slab kernel's; nothing is written beside."""
     g = gen(T + K)
     x, phi = dev(torch.randn(B, T, d, generator=g).to(dtype)), dev((torch.randn(T, K, generator=g) / math.sqrt(T)).to(dtype))
     spec = hip.stu_fft_filter(phi, hip.fft_length(T))
@@ -724,6 +724,28 @@ def test_stu_conv_bank_slabs_in_slices(hip, dtype, B, T, d, K):
         for a, b in zip(u, pair):
             assert torch.equal(a[:, k:k + 2], b)
     assert all(bool((t[:, K] == 9.0).all()) for t in u)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("slab", [True, False])
+@pytest.mark.parametrize("B,T,d,K,k", [(1, 300, 768, 24, 0), (2, 100, 40, 7, 3)])
+def test_stu_conv_bank_over_its_input(hip, dtype, slab, B, T, d, K, k):
+    """One filter's output, or that of its minus branch, written over x: the bits of outputs that lie apart."""
+    g = gen(k + T)
+    x, phi = dev(torch.randn(B, T, d, generator=g).to(dtype)), dev((torch.randn(T, K, generator=g) / math.sqrt(T)).to(dtype))
+    spec = hip.stu_fft_filter(phi, hip.fft_length(T))
+    def outputs():
+        if slab:
+            return [torch.empty(B, K, d, T, dtype=dtype, device="cuda").permute(0, 3, 1, 2) for _ in range(2)]
+        return [torch.empty(B, T, K, d, dtype=dtype, device="cuda") for _ in range(2)]
+    want = outputs()
+    hip.stu_conv_bank_fft(x.transpose(1, 2).contiguous().transpose(1, 2) if slab else x, spec, *want)
+    for place in (0, 1):
+        got = outputs()
+        over = got[place][:, :, k]
+        over.copy_(x)
+        hip.stu_conv_bank_fft(over, spec, *got)
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
 
 
 def test_stu_conv_fft_equals_direct_fp32(hip):
