@@ -714,9 +714,13 @@ def stu_conv_direct(xp: torch.Tensor, filt: torch.Tensor, single_branch: bool = 
 
 
 @functools.lru_cache(maxsize=256)
+def _fft_length(T: int) -> int:
+    return load().fstu_fft_length(T)
+
+
 def fft_length(T: int) -> int:
     """Smallest supported transform length (power of two, 64..16384) with n >= 2T; 0 if T is too long."""
-    return int(load().fstu_fft_length(int(T)))
+    return _fft_length(int(T))
 
 
 _twiddle_cache = {}

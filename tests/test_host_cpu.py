@@ -46,6 +46,18 @@ def test_argument_validation_happens_on_the_host():
     assert lib.fstu_embed(p, p, p, 1, 8, 4, 7, None) == -2                                   # unknown dtype
 
 
+def test_fft_length_goes_by_the_value():
+    """The number of positions as any whole number: arrays of no dimension, and a tensor that holds another one the next time."""
+    import numpy as np
+    from flash_stu import _hip
+    assert [_hip.fft_length(T) for T in (1, 33, 8192, 8193)] == [64, 128, 16384, 0]
+    assert _hip.fft_length(np.array(100)) == _hip.fft_length(np.int64(100)) == 256
+    T = torch.tensor(100)
+    assert _hip.fft_length(T) == 256
+    T.fill_(1000)
+    assert _hip.fft_length(T) == 2048
+
+
 def test_config_surface_matches_reference_defaults(tmp_path):
     from flash_stu import FlashSTUConfig
     c = FlashSTUConfig()
