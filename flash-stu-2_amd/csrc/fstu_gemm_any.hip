@@ -200,7 +200,7 @@ gemm_any_tile_kernel(const T* __restrict__ A, long long sam, long long sak, cons
     auto pass = [&](int b, Next& v) __attribute__((always_inline)) {      // v: the tile behind this one
       multiply(b);
       put(b ^ 1, v);       // the other buffer was last read before the barrier that ended the previous tile
-      fetch(v, k0 + 3 * GA_BK);                                            // zeros from K on
+      fetch(v, K - k0 > 3 * GA_BK ? k0 + 3 * GA_BK : K);                   // zeros from K on, and no sum beyond an int for the longest K
       __syncthreads();
       return (k0 += GA_BK) < K;
     };
