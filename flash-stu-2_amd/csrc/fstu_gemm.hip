@@ -1157,16 +1157,21 @@ namespace {
 // The same where the slices can also run on 256 x 256 tiles in the alternating-group kernel (rows, or slabs of whole tiles of them):
 // half the operands' bytes through the LDS for a product, and every compute unit at work where M and N leave it idle.  A k tile of
 // 64 takes those 1 us in a nearly empty round and 1.35 in a full one, which draws the matrix cores' power; 128 x 128 tiles 0.43 us alone on
-// a compute unit and, two to a unit, 0.55 to 0.9 in slices and up to 1.05 over a whole long K.  us before / with the slices it picks (L: large tiles), rows x features x K:
-// 1408 x 2048 x 24576 177 / 137 (L4), 1900 213 / 159 (L4), 2500 363 / 203 (L3), 3200 379 / 264 (L2), 4096 400 / 295 (L2), 5000 452 / 398
-// (L3); 5500 x 768 x 9216 99 / 81 (L3), 7000 125 / 95 (L3), 7700 145 / 121 (L2), 9000 139 / 119 (L2), 12000
-// 266 / 170 (L3); 8300 x 512 x 6144 75 / 60 (L3), 7800 x 1024 x 12288 225 / 161 (L2).  Where it stays as it was, with
-// the best slices of large tiles: 1000 x 2048 x 24576 105 / 91 (6), 6100 485 / 498 (4), 4096 x 768 x 9216 66 / 61 (4), 16000 180 / 230 (2), 2500 x 2048 x 2048 31 / 39 (2).  Slabs: 1 x 8192 x 1024 x 24576 451 / 309 (L2), 4 x 2048 454 / 303 (L2), 2 x
-// 2048 242 / 159 (L4), 1 x 4096 x 768 x 18432 142 / 111 (L4).
-// Rows (not slabs) have 256 x 128 tiles between the two, in slices of any number of k tiles, where one round holds them all: before / with the
-// slices it picks, 2331 x 768 x 9216 44.9 / 41.3 (4), 4096 73.8 / 62.4 (2), 1800 40.4 / 36.4 (5), 3200 56.9 / 51.8 (3), 1000 x 2048 x 24576
-// 101.6 / 88.5 (4), 700 75.1 / 70.0 (5).  A k tile of 64 takes 0.55 us in a nearly empty round, 0.66 in a full one, and 0.9 through more than 128 of
-// them (4096 x 2048 x 24576 349 in one piece; 300 in two slices of large tiles), the joining launch 3 and 6 TB/s behind these.
+// a compute unit and, two to a unit, 0.55 to 0.9 in slices and up to 1.05 over a whole long K.  us on small tiles / with the slices it picks
+// (L: large tiles), rows x features x K: 1408 x 2048 x 24576 151 / 119 (L4), 2500 257 / 186 (L3), 4096 391 / 277 (L2), 5500 x 768 x 9216
+// 95 / 75 (L3).  Slabs: 1 x 8192 x 1024 x 24576 451 / 309 (L2), 4 x 2048 454 / 303 (L2), 2 x 2048 242 / 159 (L4), 1 x 4096 x 768 x 18432 142
+// / 111 (L4); those of 129 to 144 large tiles in three slices / whole 3 x 6144 x 512 x 12288 220 / 231, 4 x 2816 x 768 x 9216 165 / 149.
+// Rows (not slabs) have 256 x 128 tiles between the two, in slices of any number of k tiles, where one round holds them all: without / with
+// the slices it picks, 2331 x 768 x 9216 43.4 / 40.2 (4), 4096 66.1 / 60.5 (2), 3200 54.8 / 50.4 (3), 1800 38.9 / 35.7 (5), 1000 x 2048 x 24576
+// 100 / 88 (4).  They are not asked for where slices on large tiles gain (400 x 4100 x 8192 47.9 in four of those, 41.2 in three of these).
+// A product whose whole runs on large or half tiles takes no slices where these do not gain: both sides' estimates there are fitted to 220
+// products of 256 to 12000 rows, 512 to 4096 features and K = 2048 to 24576 with every count on every tile (2 to 5 % off), and tried on 220
+// others.  A k tile costs the more the fuller the round is, large tiles from 32 and half ones from 96 of them on.  Slices on large tiles /
+// whole: on half tiles 7882 x 768 x 9216 108.9 / 92.2, 10660 130.7 / 112.3, 4963 x 1536 x 9216 120.2 / 108.7, at the line 8504 x 512 x 6144 59.3 /
+// 60.9, 2063 x 2048 x 6144 59.9 / 59.8; on large ones 4054 x 2304 x 6144 116.6 / 100.2, 5903 x 1536 x 6144 115.0 / 101.1, at the line 2119 x 4096 x
+// 12288 193.9 / 199.0, 12000 x 768 x 9216 168.6 / 165.5; beyond K = 12288, where the estimate of a long round is low, 3520 x 3072 x 24576 402 / 434.
+// Half tiles read the rows twice as often as large ones: where these are more than the memory-side cache holds beside the rest, slices stay
+// (200 MB of rows: 10660 x 768 x 9216, 197 MB, above; 12724 x 512 x 9216, 235 MB, 114.4 / 126.8, 10348 x 768 x 12288, 254 MB, 160 / 180).
 enum TileKind { SMALL, LARGE, HALF };
 struct SlicePlan { int count; TileKind on; };
 SlicePlan slice_plan(int M, int N, int K, int nb, bool rows) {
@@ -1186,25 +1191,42 @@ SlicePlan slice_plan(int M, int N, int K, int nb, bool rows) {
     const long long rounds = (small * s + 2 * cus - 1) / (2 * cus);
     return rounds * (nkt / s) * (0.55 + (s == 1 ? 0.5 : 0.35) * (double)(small * s) / (double)(rounds * 2 * cus)) + join(s);
   };
-  const bool whole_large = before == 1 && 9 * ((big + cus - 1) / cus) * cus < 4 * small;
-  double least = 0.95 * (whole_large ? large(1) : little(before));
+  const bool half_whole = rows && half_takes(M, N), large_whole = !half_whole && pp_takes(0, K, big, small);
+  double least = 0.95 * (!rows && before == 1 && 9 * ((big + cus - 1) / cus) * cus < 4 * small ? large(1) : little(before));
   SlicePlan best = {before, SMALL};
   for (int s = 2; s <= 32 && K / s >= 512 && big * s <= 2 * cus; ++s) {
     if (nkt % s != 0) continue;
     const double us = large(s);
     if (us < least) { least = us; best = {s, LARGE}; }
   }
+  if (!rows) return best;
   const long long halves = (long long)((M + 255) / 256) * ((N + 127) / 128);
-  if (!rows || best.on != SMALL || halves > cus) return best;
-  // (what the products that it is compared with take, a little closer than to rank them among each other)
-  const double full = (double)(small * before) / (double)cus;
-  least = 0.93 * (whole_large ? large(1) : small * before > cus ? 0.93 * little(before) : 4.0 + nkt / before * (0.43 + 0.12 * full * full) + join(before));
-  for (int s = half_takes(M, N) ? 1 : 2; s <= 32 && (s == 1 || nkt / s >= 16) && halves * s <= cus; ++s) {
-    const double f = (double)(halves * s) / (double)cus;
-    const int n = (nkt + s - 1) / s;
-    const double us = 5.0 + n * (0.55 + 0.11 * f + (n > 128 ? 0.25 * f * f * f * f : 0.0)) + (s == 1 ? 0.0 : 3.0 + 8e-6 / 6.0 * s * (double)M * N);
-    if (us < least) { least = us; best = {s, HALF}; }
+  if (best.on == SMALL && halves <= cus) {
+    // (what the products that it is compared with take, a little closer than to rank them among each other)
+    const double full = (double)(small * before) / (double)cus;
+    least = 0.93 * (small * before > cus ? 0.93 * little(before) : 4.0 + nkt / before * (0.43 + 0.12 * full * full) + join(before));
+    for (int s = half_whole ? 1 : 2; s <= 32 && (s == 1 || nkt / s >= 16) && halves * s <= cus; ++s) {
+      const double f = (double)(halves * s) / (double)cus;
+      const int n = (nkt + s - 1) / s;
+      const double us = 5.0 + n * (0.55 + 0.11 * f + (n > 128 ? 0.25 * f * f * f * f : 0.0)) + (s == 1 ? 0.0 : 3.0 + 8e-6 / 6.0 * s * (double)M * N);
+      if (us < least) { least = us; best = {s, HALF}; }
+    }
   }
+  if (best.on == SMALL || best.count == 1 || before > 1 || !(half_whole ? (long long)M * K <= 100 << 20 : large_whole)) return best;
+  const auto beyond = [](int n, int from, int over) { return std::min(1.0, std::max(0, n - from) / (double)over); };
+  const auto us = [&](TileKind on, int s) {
+    const double joined = s == 1 ? 0.0 : 7.0 + (on == LARGE ? 1e-6 : 0.8e-6) * s * (double)M * N;
+    const int n = (nkt + s - 1) / s;
+    if (on == HALF) {
+      const double f = (double)(halves * s) / (double)cus;
+      return 4.0 + n * (0.53 + 0.09 * f + f * f * f * f * (0.08 + 0.12 * beyond(n, 96, 288))) + joined;
+    }
+    const long long rounds = (big * s + cus - 1) / cus;
+    const double f = (double)(big * s) / (double)(rounds * cus);
+    return 5.0 + rounds * n * (0.9 + f * f * (0.36 + 0.19 * f * f * beyond(n, 32, 96))) + joined;
+  };
+  const TileKind whole = half_whole ? HALF : LARGE;
+  if (us(whole, 1) * (half_whole ? 1.02 : nkt <= 192 ? 0.94 : 0.97) <= us(best.on, best.count)) return {1, whole};
   return best;
 }
 
@@ -1289,7 +1311,9 @@ extern "C" int fstu_gemm_bf16_head_rows(int M, int N, int K) {
   const long long head = tiles / cus * cus / nt * 256;
   if (head <= 0 || head >= M) return 0;
   const long long left = (M - head + 127) / 128 * ((N + 127) / 128);
-  if (left <= (K < 2048 ? cus / 2 : cus) || slice_plan((int)(M - head), N, K, 1, true).on != SMALL) return (int)head;
+  const SlicePlan rest = slice_plan((int)(M - head), N, K, 1, true);
+  // (a rest that is whole on large tiles takes a round either way: 9587 x 6144 x 6144 498 split, 481 in one launch; 11157 x 2304 x 12288 485, 502)
+  if (left <= (K < 2048 ? cus / 2 : cus) || rest.on == HALF || (rest.on == LARGE && (rest.count > 1 || K >= 12288))) return (int)head;
   return 0;
 }
 

@@ -46,6 +46,17 @@ def test_argument_validation_happens_on_the_host():
     assert lib.fstu_embed(p, p, p, 1, 8, 4, 7, None) == -2                                   # unknown dtype
 
 
+def test_slices_of_k_are_measured_against_the_product_that_would_run():
+    """Products whose whole runs on 256 x 128 or 256 x 256 tiles take slices only where those gain (256 compute units)."""
+    from flash_stu import _hip
+    lib = _hip.load()
+    for M, N, K in ((7882, 768, 9216), (10660, 768, 9216), (4963, 1536, 9216), (4054, 2304, 6144), (5903, 1536, 6144), (12960, 768, 12288)):
+        assert lib.fstu_gemm_bf16_row_slices(M, N, K) == 1
+    for M, N, K, slices in ((5500, 768, 9216, 3), (4096, 2048, 24576, 2), (2119, 4096, 12288, 3), (3520, 3072, 24576, 3), (4096, 768, 9216, 2)):
+        assert lib.fstu_gemm_bf16_row_slices(M, N, K) == slices
+    assert lib.fstu_gemm_bf16_head_rows(9587, 6144, 6144) == 0 and lib.fstu_gemm_bf16_head_rows(22500, 768, 9216) > 0
+
+
 def test_fft_length_goes_by_the_value():
     """The number of positions as any whole number: arrays of no dimension, and a tensor that holds another one the next time."""
     import numpy as np
