@@ -713,7 +713,7 @@ gemm_half_bf16_kernel(const bf16_t* __restrict__ A, long long lda, const bf16_t*
   }
   const unsigned x1off = 128u * (unsigned)lda * 2u;
   unsigned char* const fill0 = gm_smem + (unsigned)wv * 2048u;
-  auto fetch = [&](int kt, unsigned stage) __attribute__((always_inline)) {   // beyond the last k tile the addresses lie behind both descriptors
+  auto fetch = [&](int kt, unsigned stage) __attribute__((always_inline)) {   // beyond the last k tile that one again, into a stage that nobody reads
     const unsigned so = (unsigned)min(kt, kt1 - 1) * 128u;
     unsigned char* const l = fill0 + stage;
 #pragma unroll
@@ -1076,17 +1076,17 @@ using TileK32 = GemmTile<2, 2, 4, 2, 32, 3>;     // 256 x 128, 4 waves, 72 KB, k
 // a round of small tiles, two to a compute unit.  A last round of small tiles costs 0.4 of a full one however few they are, and
 // their stores, a quarter of a line at a time, 0.2 more than the large tiles' do.  A round of large tiles, one to a compute
 // unit, takes 1.15 of them, and in mode 1, whose GELU covers only half of its round's products, 1.4 where K is long and 1.55
-// where it is short; from K = 4096 on and over several rounds 1.25.  us, large / small tiles.  Mode 0: 4096 x 2304 (144 large tiles, 576 small) K = 64 8.8 / 13.1, 768 17.8 / 25.9,
+// where it is short; where K is long and over three rounds, from K = 4096 on over two, 1.25.  us, large / small tiles.  Mode 0: 4096 x 2304 (144 large tiles, 576 small) K = 64 8.8 / 13.1, 768 17.8 / 25.9,
 // 2048 37.9 / 53.0; 2048 x 4096 (128, 512) 8.8 / 12.2, 17.8 / 19.6, 35.7 / 37.1; 8192 x 2304 (288, 1152) K = 768 38.5 / 42.9, 2048
 // 78.6 / 82.6; the line: 3840 x 2048 (120, 480) K = 256 10.7 / 11.4, 2048 39.0 / 35.4.  Mode 1: 4096 x 2 x 1152 (144, 576) K = 64
 // 9.4 / 9.8, 768 18.9 / 23.2, 2048 36.7 / 50.9; 8192 x 2 x 2304 (576, 2304) 21.6 / 22.3, 57.4 / 62.6, 128 / 144; the line: 8192
 // x 2 x 1152 (288, 1152) 15.7 / 14.2, 37.1 / 36.5, 81.6 / 80.6, 20000 x 2 x 512 (316, 1256) 15.7 / 14.2, 36.8 / 35.7, 80.5 / 81.1;
-// of a long K 583 x 2 x 24576 x 4096 (576, 1920) 244 / 257, 2842 x 2 x 3072 x 5120 (288, 1104) 185 / 195, 342 x 2 x 50256 x 12288 (786, 2358) 1032 /
+// of a long K 608 x 2 x 24576 x 2048 (576, 1920) 124 / 126, in a model's pass 128 / 138, x 4096 244 / 257, 2842 x 2 x 3072 x 5120 (288, 1104) 185 / 195, 342 x 2 x 50256 x 12288 (786, 2358) 1032 /
 // 1088, 263 rows of it at K = 6144 531 / 500, 970 x 2 x 4096 x 5120 (128, 512) 81 / 76.
 bool pp_takes(int mode, int K, long long big, long long small) {
   const long long cus = gemm_cus(), full = small / (2 * cus), rest = small % (2 * cus);
   const long long little = (mode == 1 ? 6 : 4) + 20 * full + (rest ? 8 + 6 * rest / cus : 0);
-  return (mode != 1 ? 23 : K >= 4096 && big > cus ? 25 : K >= 1024 ? 28 : 31) * ((big + cus - 1) / cus) < little;
+  return (mode != 1 ? 23 : K >= 1536 && big > (K < 4096 ? 2 : 1) * cus ? 25 : K >= 1024 ? 28 : 31) * ((big + cus - 1) / cus) < little;
 }
 long long tiles_of(int side, int M, int N) { return (long long)((M + side - 1) / side) * (((long long)N + side - 1) / side); }
 
