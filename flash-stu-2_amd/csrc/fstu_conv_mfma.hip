@@ -18,7 +18,7 @@
 // once, transposed 8 x 8 in registers, and a wave works on a channel by itself, so there are two barriers in all.  The result
 // replaces the channel's inputs in LDS and leaves the way it came.
 //
-// us, transforms -> this: 8 x 512 x 768 16 -> 10.1, 32 x 300 x 2048 100 -> 47.5, 8 x 2048 x 768 61 -> 41, 1 x 4096 x 2048 56 (with a
+// us, transforms -> this: 8 x 512 x 768 16 -> 10.1, 32 x 300 x 2048 100 -> 47.5, 8 x 2048 x 768 61 -> 42, 1 x 4096 x 2048 56 (with a
 // transpose) -> 43.6.  What bounds the longest two is the matrix cores: 2.36 and 2.62 M products of 16 x 16 x 32, which this card
 // issues every 20 cycles on random operands, are 19 and 21 us; the rows' way in and out, 5 and 2 us, is not hidden behind them,
 // because all workgroups that fit start together.  Blocks of 32 positions would save a sixth of the products, but the filter

@@ -683,8 +683,8 @@ int gemm_pp_launch(const void* A, long long lda, const void* W, const void* W2, 
 // a phase apart as above.  Three stages of W | X0 | X1 (16 KB each); in its memory phase of k tile kt a group reads its 16 fragments
 // and requests its share of kt + 2 into the stage that both groups left a phase ago, and waits for its share of kt + 1.
 // What bounds it: 0.58 us a k tile in a nearly empty round, of which its products are 0.49; 0.65 to 0.9 in a full one (power, LDS).
-// us, before (256 x 256 or 128 x 128 tiles) / so: 4096 x 2048 x 2048 41.3 / 32.1, 2331 x 2304 x 768 17.2 / 13.7, 8192 x 768 x 768 17.3 / 13.7,
-// 1024 x 8192 x 4096 65.0 / 53.3; joined slices of K 2331 x 768 x 9216 44.9 / 41.3, 4096 x 768 x 9216 73.8 / 62.4, 1000 x 2048 x 24576 101.6 / 88.5.
+// us, before (256 x 256 or 128 x 128 tiles) / so: 4096 x 2048 x 2048 36.6 / 30.4, 2331 x 2304 x 768 16.4 / 12.7, 8192 x 768 x 768 16.3 / 12.6,
+// 1024 x 8192 x 4096 65.9 / 53.5; joined slices of K 2331 x 768 x 9216 43.2 / 40.2, 4096 x 768 x 9216 65.8 / 60.3, 1000 x 2048 x 24576 102.6 / 88.5.
 #define PH_STAGE 49152u
 #define PH_LDS (3 * PH_STAGE)
 template <int MODE>

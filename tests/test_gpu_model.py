@@ -353,7 +353,8 @@ def test_input_projection_gradients_of_gradients():
 @pytest.mark.parametrize("B,d", [(1, 64), (3, 256), (16, 512)])
 def test_greedy_steps_in_one_call(dtype, B, d):
     """fstu_decode_steps, whose picks are finished in the launch that begins the next step, against a call per step: the same tokens, and
-    nothing left of one call's maxima for the next."""
+    nothing left of one call's maxima for the next; the last step's logits against those of one pass over all tokens, which knows
+    neither steps nor that launch."""
     from flash_stu import FlashSTU, FlashSTUConfig
     torch.manual_seed(B)
     cfg = FlashSTUConfig(n_embd=d, n_heads=2, n_layers=2, seq_len=64, window_size=16, vocab_size=501, num_eigh=8, torch_dtype=dtype)
@@ -365,6 +366,10 @@ def test_greedy_steps_in_one_call(dtype, B, d):
         one = model.generate(ids, max_length=9 + n, do_sample=False)
         each, _ = model.generate(ids, max_length=9 + n, do_sample=False, return_logits=True)
         assert torch.equal(one, each), n
+        if n > 1:
+            model.generate(ids, max_length=9 + n, do_sample=False)
+            got, ref = model.decode_engine().logits.float(), model(one[:, :-1], use_cache=False).logits[:, -1].float()
+            assert float((got - ref).abs().max()) <= (1e-4 if dtype == torch.float32 else 3e-2) * float(ref.abs().max()), n
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
