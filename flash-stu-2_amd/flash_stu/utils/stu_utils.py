@@ -254,7 +254,8 @@ class ApproxUnit(torch.autograd.Function):
         x2 = _aligned(x.reshape(-1, x.shape[2]))
         u = _hip.gemm(x2, _hip.transpose(m_inputs[None])[0]).view(*x.shape[:2], m_inputs.shape[1])
         v, taps = _hip.stu_conv_taps_project(phi, m_filters, x.shape[1])
-        ctx.save_for_backward(x, phi, phi_e, m_inputs, u, v)
+        of_inputs, of_filters = any(ctx.needs_input_grad[i] for i in (0, 3)), ctx.needs_input_grad[4]
+        ctx.save_for_backward(*((x, m_inputs) if of_inputs else (None, None)), *((phi, phi_e) if of_filters else (None, None)), u, v)
         ctx.m_filters = m_filters if ctx.needs_input_grad[4] else None
         ctx.version = m_filters._version if ctx.needs_input_grad[4] else 0
         return _hip.stu_conv_mfma(u, taps)
@@ -262,7 +263,7 @@ class ApproxUnit(torch.autograd.Function):
     @staticmethod
     def backward(ctx, gy):
         from .. import _hip
-        x, phi, phi_e, m_inputs, u, v = ctx.saved_tensors
+        x, m_inputs, phi, phi_e, u, v = ctx.saved_tensors        # (what the wanted ones need)
         want_x, _, _, want_i, want_f = ctx.needs_input_grad
         if torch.is_grad_enabled():
             filt, m_filters = v, ctx.m_filters
@@ -272,7 +273,8 @@ class ApproxUnit(torch.autograd.Function):
                 now = phi[:v.shape[0]] @ m_filters
                 filt = v + (now - now.detach())          # the forward pass's values, on the way to m_filters
             wanted = [t for t, w in ((x, want_x), (m_inputs, want_i), (m_filters, want_f)) if w]
-            grads = iter(torch.autograd.grad(ApproxConvolveSum.apply(x @ m_inputs, filt), wanted, gy, create_graph=True))
+            proj = x @ m_inputs if want_x or want_i else u
+            grads = iter(torch.autograd.grad(ApproxConvolveSum.apply(proj, filt), wanted, gy, create_graph=True))
             return next(grads) if want_x else None, None, None, next(grads) if want_i else None, next(grads) if want_f else None
         gy, gf = _aligned(gy), None
         if want_f:

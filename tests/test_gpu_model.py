@@ -308,6 +308,35 @@ def test_filter_weights_may_change_before_the_backward_pass():
         assert float((graph.detach().float() - want.float()).norm()) <= 3 * 2.0 ** -8 * float(want.float().norm())
 
 
+@pytest.mark.parametrize("second", [False, True])
+def test_what_no_gradient_needs_may_change_before_the_backward_pass(second):
+    """Where M_filters alone is trained its gradient needs neither x nor M_inputs, where it is frozen none needs phi: an update of them
+    between the passes leaves the gradients those of the forward pass, bit for bit."""
+    from flash_stu import STU, FlashSTUConfig
+    B, T, d, L, K = 4, 64, 128, 128, 24
+    g = torch.Generator().manual_seed(6)
+    cfg = FlashSTUConfig(n_embd=d, n_heads=2, n_layers=2, seq_len=L, num_eigh=K, vocab_size=11, torch_dtype=torch.bfloat16)
+    stu = STU(cfg, torch.randn(L, K, generator=g).div(L ** 0.5).bfloat16().cuda(), 256).cuda()
+    start = [torch.randn(p.shape, generator=g).div(p.shape[0] ** 0.5).bfloat16().cuda() for p in (stu.M_inputs, stu.M_filters)] + [stu.phi.clone()]
+    x0, gy = (torch.randn(B, T, d, generator=g).bfloat16().cuda() for _ in range(2))
+    for wanted, changed in (((2,), (0, 1)), ((0, 1), (3,)), ((1,), (3,))):
+        runs = []
+        for update in (False, True):
+            x = x0.clone()
+            leaves = (x, stu.M_inputs, stu.M_filters, stu.phi)
+            with torch.no_grad():
+                for t, v in zip(leaves[1:], start):
+                    t.copy_(v)
+            for i, t in enumerate(leaves[:3]):
+                t.requires_grad_(i in wanted)
+            y = stu.forward_differentiable(x)
+            with torch.no_grad():
+                for i in changed if update else ():
+                    leaves[i].mul_(-3.0)
+            runs.append(torch.autograd.grad(y, [leaves[i] for i in wanted], gy, create_graph=second))
+        assert all(torch.equal(a, b) for a, b in zip(*runs))
+
+
 @pytest.mark.parametrize("B,T,d", [(1, 128, 128), (3, 320, 256), (2, 97, 128)])
 def test_input_projection_gradients(B, T, d):
     """x @ M_inputs and its gradients on the matrix-core kernels (and, for rows they do not take, the library's product)
