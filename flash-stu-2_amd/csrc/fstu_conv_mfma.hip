@@ -288,7 +288,7 @@ conv_mfma_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ taps, 
 // are 6.4 us of a compute unit, 11 with the LDS reads in front of them; the latter bound it now.
 constexpr int cg_rows(int HB) { return 128 * HB + 256; }        // bytes of a channel of g: zeros behind it
 
-template <int NT>
+template <int NT, bool PROJECT>
 __global__ void __launch_bounds__(512, 4)
 conv_grad_mfma_kernel(const bf16_t* __restrict__ gy, const bf16_t* __restrict__ x, const bf16_t* __restrict__ f, bf16_t* __restrict__ gx,
                       float* __restrict__ part, const bf16_t* __restrict__ phi_e, int K, int P, int B, int T, int L, int d, int R) {
@@ -459,7 +459,7 @@ conv_grad_mfma_kernel(const bf16_t* __restrict__ gy, const bf16_t* __restrict__ 
         if (k0 + 16 * t < K && lag0 + 32 * step < P) ph[t][step] = *(const uint4*)(phi_e + (size_t)(k0 + 16 * t + col) * P + lag0 + 32 * step);
       }
   };
-  if (phi_e) rows_of_phi(0);
+  if constexpr (PROJECT) rows_of_phi(0);
   // lags of a channel -> channels of a lag, through the space of x and the taps
   float* const fl32 = (float*)xl;
   if (col < 8) {
@@ -469,7 +469,7 @@ conv_grad_mfma_kernel(const bf16_t* __restrict__ gy, const bf16_t* __restrict__ 
       for (int r = 0; r < 4; ++r) *(floatx4_t*)(fl32 + ch * (cap + 4) + (c + 8 * j) * 64 + 16 * r + 4 * g) = S[j][r];
   }
   __syncthreads();
-  if (phi_e) {
+  if constexpr (PROJECT) {
     // wave ch: an eighth of the lags; the waves' tiles of 2 x 16 filters x (8 channels, 8 remainders) meet in the space of g and the rings
     float* const red = (float*)gl;
     for (int k0 = 0; k0 < K; k0 += 32) {
@@ -750,17 +750,22 @@ int cg_launch(const char* name, const void* gy, const void* x, const void* filt,
   const long long units = (long long)((d + 63) / 64) * ((2 * B + R - 1) / R);
   FSTU_REQUIRE(units < 1 << 24, FSTU_ESHAPE, "%s: B=%d d=%d", name, B, d);
   const dim3 grid((unsigned)((units + 7) / 8 * 64));
-#define CG_GO(NT)                                                                                                                   \
+#define CG_GO(NT, PROJECT)                                                                                                          \
   do {                                                                                                                              \
     constexpr int lds__ = 16 * cm_region(8 * NT) + 8 * cg_rows(8 * NT) + 8 * 2048;                                                 \
     static fstu_lds_limit most;                                                                                                     \
-    const int rc__ = fstu_need_lds((const void*)conv_grad_mfma_kernel<NT>, most, lds__, name);                                      \
+    const int rc__ = fstu_need_lds((const void*)conv_grad_mfma_kernel<NT, PROJECT>, most, lds__, name);                             \
     if (rc__) return rc__;                                                                                                          \
-    hipLaunchKernelGGL((conv_grad_mfma_kernel<NT>), grid, dim3(512), lds__, s, (const bf16_t*)gy, (const bf16_t*)x, (const bf16_t*)filt, \
+    hipLaunchKernelGGL((conv_grad_mfma_kernel<NT, PROJECT>), grid, dim3(512), lds__, s, (const bf16_t*)gy, (const bf16_t*)x, (const bf16_t*)filt, \
                        (bf16_t*)gx, part, (const bf16_t*)phi_e, K, P, B, T, L, d, R);                                               \
   } while (0)
-  if (T <= 1024) CG_GO(1);
-  else CG_GO(2);
+  if (phi_e) {
+    if (T <= 1024) CG_GO(1, true);
+    else CG_GO(2, true);
+  } else {
+    if (T <= 1024) CG_GO(1, false);
+    else CG_GO(2, false);
+  }
 #undef CG_GO
   FSTU_CHECK_LAUNCH(name);
   return FSTU_OK;
