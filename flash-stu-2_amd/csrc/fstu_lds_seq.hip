@@ -73,7 +73,10 @@ __device__ __forceinline__ void store16(bf16_t* p, uint4 v) {
 //
 // PAST: the outputs leave past the L2s, where they are more than those hold (32 MB): what they would push out are the weights
 // that every workgroup fetches again, and the next kernel would not find them there.
-template <int NT, bool PAST>
+//
+// SLICED: the features may be in slices.  A kernel of its own for those in one only beyond S = 160, where a few more values that live through
+// the second product cost its LDS reads their overlap (4096 x 40 x 1024, state 256, 333 us; 316 so).
+template <int NT, bool PAST, bool SLICED>
 __global__ void __launch_bounds__(256, NT <= 10 ? 2 : 1)   // beyond S = 160 one workgroup fills the LDS anyway
 lds_seq_kernel(const bf16_t* x, const float* __restrict__ A, const bf16_t* BmT, const bf16_t* CmT, bf16_t* y, const float* __restrict__ h0,
                float* __restrict__ hnew, unsigned long long* __restrict__ etag, unsigned* __restrict__ status, unsigned tag,
@@ -82,7 +85,7 @@ lds_seq_kernel(const bf16_t* x, const float* __restrict__ A, const bf16_t* BmT, 
   extern __shared__ __align__(16) float Us[];       // LSQ_TB x S
   auto uslot = [](int row, int slot) { return slot ^ ((row >> 1) & 7); };   // 16-byte slot of a row (S/4 slots, a multiple of 8)
   // rows of the batch first: the blocks in front of a workgroup's are then long through when it asks for their states
-  const int blk = (int)(blockIdx.z * gridDim.y + blockIdx.y), b = blockIdx.x / slices, slice = blockIdx.x % slices;
+  const int blk = (int)(blockIdx.z * gridDim.y + blockIdx.y), b = SLICED ? blockIdx.x / slices : blockIdx.x, slice = SLICED ? blockIdx.x % slices : 0;
   if (blk >= nblk) return;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, r = lane & 15, g = lane >> 4;
   const int t0 = blk * LSQ_TB;
@@ -106,7 +109,10 @@ lds_seq_kernel(const bf16_t* x, const float* __restrict__ A, const bf16_t* BmT, 
 #pragma unroll
     for (int m = 0; m < 2; ++m) xr[m] = x + ((size_t)min(t0 + 32 * w + 16 * m + r, T - 1) * Bt + b) * d_in + g * 8;
     // A chunk of a row is a line.  The first eight lanes of a row's sixteen have its first half, the others the second, of rows 0..7 of a
-    // tile in one load and of rows 8..15 in another: whole lines; lanes r and r ^ 8 swap pieces in front of the products.
+    // tile in one load and of rows 8..15 in another: whole lines; lanes r and r ^ 8 swap pieces in front of the products.  Beyond S = 160,
+    // where the accumulators alone are most of the registers, the swaps cost more than the lines give (4096 x 40 x 1024, us, half lines / whole:
+    // state 256 333 / 341, 224 284 / 292, 192 255 / 261): there a load has its own k step's halves of sixteen lines.
+    constexpr bool LINES = NT <= 10;
     const bf16_t* xl[2][2];
 #pragma unroll
     for (int m = 0; m < 2; ++m)
@@ -135,12 +141,12 @@ lds_seq_kernel(const bf16_t* x, const float* __restrict__ A, const bf16_t* BmT, 
 #pragma unroll
         for (int i = 0; i < WPT; ++i) *(uintx4_t*)(wdst + stage + i * 4096) = v[i];
       };
-      auto xload = [&](int c, uintx4_t (&v)[2][2]) {            // both halves of both position tiles
+      auto xload = [&](int c, uintx4_t (&v)[2][2]) {            // both halves (or k steps) of both position tiles
         const int k0 = 64 * min(c, nk - 1);
 #pragma unroll
         for (int h = 0; h < 2; ++h)
 #pragma unroll
-          for (int m = 0; m < 2; ++m) v[h][m] = *(const uintx4_t*)(xl[m][h] + k0);
+          for (int m = 0; m < 2; ++m) v[h][m] = *(const uintx4_t*)(LINES ? xl[m][h] + k0 : xr[m] + k0 + 32 * h);
       };
       uintx4_t wa[WPT], wb[WPT], xa[2][2], xb[2][2], xc[2][2];
       wload(0, wa);
@@ -154,15 +160,20 @@ lds_seq_kernel(const bf16_t* x, const float* __restrict__ A, const bf16_t* BmT, 
       int c = 0;
       unsigned stage = 0;
       auto pass = [&](uintx4_t (&xs)[2][2], uintx4_t (&wn)[WPT]) __attribute__((always_inline)) { // chunk c; wn: the weights of chunk c + 1
-        uintx4_t x0[2], x1[2];
+        if constexpr (LINES) {
+          uintx4_t x0[2], x1[2];
 #pragma unroll
-        for (int m = 0; m < 2; ++m) {
-          const uintx4_t o = __builtin_bit_cast(uintx4_t, swap8(__builtin_bit_cast(uint4, r < 8 ? xs[1][m] : xs[0][m])));
-          x0[m] = r < 8 ? xs[0][m] : o;
-          x1[m] = r < 8 ? o : xs[1][m];
+          for (int m = 0; m < 2; ++m) {
+            const uintx4_t o = __builtin_bit_cast(uintx4_t, swap8(__builtin_bit_cast(uint4, r < 8 ? xs[1][m] : xs[0][m])));
+            x0[m] = r < 8 ? xs[0][m] : o;
+            x1[m] = r < 8 ? o : xs[1][m];
+          }
+          multiply(0, stage, x0);
+          multiply(1, stage, x1);
+        } else {
+          multiply(0, stage, xs[0]);
+          multiply(1, stage, xs[1]);
         }
-        multiply(0, stage, x0);
-        multiply(1, stage, x1);
         stage = wstage - stage;
         wstore(stage, wn);
         wload(c + 3, wn);
@@ -288,7 +299,7 @@ lds_seq_kernel(const bf16_t* x, const float* __restrict__ A, const bf16_t* BmT, 
     // that lane (r, g) ends up with features 8g .. 8g+7 of position r, and lanes r and r ^ 8 swap pieces, so that
     // they hold the two halves of a line of 64 features.
     const int trow = t0 + 32 * w + (r & 7), fcol = 32 * (r >> 3) + 8 * g;
-    const int of = slice * width, dn = min(width, d_out - of);   // the features of this workgroup's slice
+    const int of = SLICED ? slice * width : 0, dn = SLICED ? min(width, d_out - of) : d_out;   // the features of this workgroup's slice
     CmT += (size_t)of * S;
     y += of;
     bf16_t* yr[4];                                           // position trow + 8 q
@@ -456,7 +467,11 @@ static int lds_sequence(float* h, const void* x, const float* A, const void* Bm,
                        (const float*)h0, h, etag, status, 1u, T, Bt, d_in, d_out, nblk, slices, width);
   };
 #define LSQ_RUN(...) run(std::integral_constant<decltype(&lds_seq_kernel<__VA_ARGS__>), lds_seq_kernel<__VA_ARGS__>>{})
-#define LSQ_CASE(n) case 32 * n: past ? LSQ_RUN(2 * n, true) : LSQ_RUN(2 * n, false); break
+#define LSQ_CASE(n)                                                                                 \
+  case 32 * n:                                                                                      \
+    if (n > 5 && slices == 1) past ? LSQ_RUN(2 * n, true, n <= 5) : LSQ_RUN(2 * n, false, n <= 5);  \
+    else past ? LSQ_RUN(2 * n, true, true) : LSQ_RUN(2 * n, false, true);                           \
+    break
   switch (S) {
     LSQ_CASE(1); LSQ_CASE(2); LSQ_CASE(3); LSQ_CASE(4); LSQ_CASE(5); LSQ_CASE(6); LSQ_CASE(7); LSQ_CASE(8);
   }
