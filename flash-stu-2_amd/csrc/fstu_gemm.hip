@@ -1083,10 +1083,10 @@ using TileK32 = GemmTile<2, 2, 4, 2, 32, 3>;     // 256 x 128, 4 waves, 72 KB, k
 // x 2 x 1152 (288, 1152) 15.7 / 14.2, 37.1 / 36.5, 81.6 / 80.6, 20000 x 2 x 512 (316, 1256) 15.7 / 14.2, 36.8 / 35.7, 80.5 / 81.1;
 // of a long K 608 x 2 x 24576 x 2048 (576, 1920) 124 / 126, in a model's pass 128 / 138, x 4096 244 / 257, 2842 x 2 x 3072 x 5120 (288, 1104) 185 / 195, 342 x 2 x 50256 x 12288 (786, 2358) 1032 /
 // 1088, 263 rows of it at K = 6144 531 / 500, 970 x 2 x 4096 x 5120 (128, 512) 81 / 76.
-bool pp_takes(int mode, int K, long long big, long long small) {
+bool pp_takes(int mode, int K, long long big, long long small, bool slabs = false) {
   const long long cus = gemm_cus(), full = small / (2 * cus), rest = small % (2 * cus);
   const long long little = (mode == 1 ? 6 : 4) + 20 * full + (rest ? 8 + 6 * rest / cus : 0);
-  return (mode != 1 ? 23 : K >= 1536 && big > (K < 4096 ? 2 : 1) * cus ? 25 : K >= 1024 ? 28 : 31) * ((big + cus - 1) / cus) < little;
+  return (mode != 1 ? (slabs && K < 8192 ? 25 : 23) : K >= 1536 && big > (K < 4096 ? 2 : 1) * cus ? 25 : K >= 1024 ? 28 : 31) * ((big + cus - 1) / cus) < little;
 }
 long long tiles_of(int side, int M, int N) { return (long long)((M + side - 1) / side) * (((long long)N + side - 1) / side); }
 
@@ -1404,10 +1404,12 @@ extern "C" int fstu_gemm_bf16_ta_ws(const void* A, int64_t lda, int64_t batch_st
                                             nbatch, s)                                                                           \
              : gemm_ta_launch_tile<TILE, 2>(A, lda, batch_stride_a, W, R, ldr, batch_stride_r, C, ldc, batch_stride_c, M, N, K,  \
                                             nbatch, s))
-  // The line between the tiles is gemm_launch's.  Large / 128 x 128 tiles (or 256 x 256 tiles all in step, the form before), us,
+  // The line between the tiles is gemm_launch's, but that a round of large tiles, whose transposing reads cost the loop more, is 1.25 of the
+  // small ones' up to a K of 8192: us, large / small, 128 large tiles and just one round of small ones, 4 x 4096 x 512 x 1024 24.1 / 22.1,
+  // x 4096 68.3 / 67.0, x 12288 223 / 232; a few more, 1 x 5632 x 1536 x 1024 24.4 / 32.1.  Large / 128 x 128 tiles (or 256 x 256 tiles all in step, the form before), us,
   // K = 24 N: 4 x 8192 x 1024 (512 large tiles) 1155 / 1475, 2 x 8192 x 1024 (256) 547 / 833, 4 x 8192 x 768 (384) 758 / 880,
   // 4 x 8192 x 512 (256) 295 / 458, 4 x 2048 x 1024 (128) 432 / 453, 1 x 8192 x 1024 (128) 443 / 440, 1 x 4096 x 768 (48) 176 / 179.
-  if (M % 256 == 0 && pp_takes(0, K, tiles_of(256, M, N) * nbatch, tiles_of(128, M, N) * nbatch))
+  if (M % 256 == 0 && pp_takes(0, K, tiles_of(256, M, N) * nbatch, tiles_of(128, M, N) * nbatch, true))
     rc = mode == 0 ? gemm_pp_launch<0, true>(A, lda, W, nullptr, R, ldr, C, ldc, M, N, K, s, nbatch, batch_stride_a, batch_stride_c, batch_stride_r)
                    : gemm_pp_launch<2, true>(A, lda, W, nullptr, R, ldr, C, ldc, M, N, K, s, nbatch, batch_stride_a, batch_stride_c, batch_stride_r);
   else rc = TA_GO(TileSmall);
