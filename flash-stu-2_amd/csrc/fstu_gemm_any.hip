@@ -3,8 +3,8 @@
 // torch_dtype float32), bf16 shapes with K % 32 != 0 or unaligned rows, and operands with any pair of strides (the
 // (K*d, T) slabs of the exact-mode operator in fp32, flash_stu/modules/stu.py:107-120; phi @ M_filters, stu.py:88).
 // Accumulation in fp32 on the fp32 matrix instructions (bf16 inputs widen exactly), one rounding to the output dtype.
-// Every global access is bounds-checked, so any M, N, K >= 1 works.  Which kernel runs, and so the order of the sums,
-// depends on M, N and K alone: strides and alignment only choose how a tile is read.
+// Every global access is bounds-checked, so any M, N, K >= 1 works.  The order of the sums depends on M, N and K alone:
+// strides and alignment only choose how a tile is read and how much of it ahead.
 #include <algorithm>
 #include "fstu_common.h"
 
@@ -266,7 +266,16 @@ static void ga_launch(const T* A, long long sam, long long sak, const T* W, long
                          sak, W, swn, swk, C, ldc, M, N, K);
       break;
     case 1:        // one group of 16 k requested at a time: more waves on a compute unit cover a trip better than a second group (fp32, us, two / one:
-                   // 1000 x 512 x 512 12.2 / 10.9, 300 x 768 x 768 10.2 / 9.3, 2400 x 256 x 3072 73 / 67, 64 x 50257 x 256 33.0 / 28.2)
+                   // 1000 x 512 x 512 12.2 / 10.9, 300 x 768 x 768 10.2 / 9.3, 2400 x 256 x 3072 73 / 67, 64 x 50257 x 256 33.0 / 28.2),
+                   // but not where both operands are read element by element and no compute unit has a second workgroup (128 x 1024 x 18432
+                   // 135 / 145, 256 x 768 x 6144 49 / 51, with 520 workgroups 2080 x 256 x 6144 132 / 123)
+      if constexpr (!VA && !VW) {
+        if ((long long)((M + 31) / 32) * ((N + 31) / 32) <= fstu_cus()) {
+          hipLaunchKernelGGL((gemm_any_split_kernel<T, VA, VW, 2, 2, 8, 2>), dim3((M + 31) / 32, (N + 31) / 32), dim3(512), 0, s, A, sam,
+                             sak, W, swn, swk, C, ldc, M, N, K);
+          break;
+        }
+      }
       hipLaunchKernelGGL((gemm_any_split_kernel<T, VA, VW, 2, 2, 8, 1>), dim3((M + 31) / 32, (N + 31) / 32), dim3(512), 0, s, A, sam,
                          sak, W, swn, swk, C, ldc, M, N, K);
       break;

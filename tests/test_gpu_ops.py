@@ -213,6 +213,19 @@ def test_gemm_any_tiles_of_64_rows(hip, dtype, M, N, K):
     test_gemm_any_tiles(hip, dtype, M, N, K)
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("M,N,K", [(129, 833, 100), (250, 1000, 523), (256, 1024, 16), (257, 1024, 260)])
+def test_gemm_any_both_operands_element_by_element(hip, dtype, M, N, K):
+    """Up to a workgroup to each of 256 compute units (and one row more), both operands with k slowest: the bits of the same operands
+    row by row, which come with fewer loads ahead."""
+    g = gen(M)
+    x, W = dev(torch.randn(M, K, generator=g).to(dtype)), dev(torch.randn(N, K, generator=g).to(dtype))
+    want = hip.gemm_any(x, W)
+    out = torch.full((M + 1, N + 3), float("nan"), dtype=dtype, device="cuda")
+    assert torch.equal(hip.gemm_any(x.t().contiguous().t(), W.t().contiguous().t(), out=out[:M, :N]), want)
+    assert bool(torch.isnan(out[M:]).all()) and bool(torch.isnan(out[:, N:]).all())
+
+
 @pytest.mark.parametrize("nb,M,N,K", [(1, 128, 64, 64), (3, 256, 132, 192), (2, 1024, 1024, 1536), (4, 512, 260, 2048),
                                       (1, 4096, 768, 3072)])
 def test_gemm_bf16_transposed_activations(hip, nb, M, N, K):
